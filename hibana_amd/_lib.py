@@ -63,6 +63,8 @@ SIGNATURES = {
     "hb_w3_moe_layer_static": (_I, [_EX, _EX, _P, _P, _P, _P, _I, _I, _P, _P]),
     "hb_w3_moe_layer_e4m3": (_I, [_EX, _EX, _P, _P, _P, _P, _I, _I, _P, _P, _Z, _P]),
     "hb_w3_moe_layer_logits": (_I, [_EX, _EX, _P, _P, _P, _I, _I, _I, _P, _P, _P, _P, _Z, _P]),
+    "hb_w3_moe_layer_rows_workspace_bytes": (_Z, [_I, _I, _EX, _I, _I]),
+    "hb_w3_moe_layer_rows": (_I, [_EX, _EX, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _P, _Z, _P]),
     "hb_w3_moe_layer_budget": (_I, [_EX, _EX, _P, _P, _P, _I, _I, _I, _I, _I, _P, _I, _I, _I, _P, _P, _P, _P, _Z, _P]),
     "hb_w3_moe_layer_logits_e4m3": (_I, [_EX, _EX, _P, _P, _P, _I, _I, _I, _P, _P, _P, _P, _Z, _P]),
     "hb_moe_combine_pairs": (_I, [_P, _I, _P, _P, _P, _P, _P, _I, _I, _I, _I, _I, _P, _P]),
@@ -119,8 +121,14 @@ def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 
 
+# The current device and the raw handle of its current stream, without a `torch.cuda.Stream` object around it (0.1 us
+# against 2.9 us a call, and every kernel call asks). A call's tensors are on the GPU, so torch has initialised it.
+current_device = torch._C._cuda_getDevice
+raw_stream = torch._C._cuda_getCurrentRawStream
+
+
 def stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    return raw_stream(current_device())
 
 
 WORKSPACE_ZERO_BYTES = 1 << 20
@@ -134,8 +142,8 @@ def workspace(device: torch.device, need: int, kind: str = "moe") -> torch.Tenso
     another, so they can share it; calls on different streams get different buffers and share nothing. `kind` keeps
     apart calls that are in progress together on one stream (a latent block's workspace lives across several calls,
     among them a routed one)."""
-    index = device.index if device.index is not None else torch.cuda.current_device()
-    key = (index, torch.cuda.current_stream(device).cuda_stream, kind)
+    index = device.index if device.index is not None else current_device()
+    key = (index, raw_stream(index), kind)
     have = _workspaces.get(key)
     if have is None or have.numel() < need:
         have = torch.empty(max(need, 4096), dtype=torch.uint8, device=device)

@@ -721,6 +721,55 @@ __global__ __launch_bounds__(1024) void latent_router_kernel(RouterGemv g) {
   }
 }
 
+// The router's product of a routed layer for at most MOE_ROUTER_ROWS rows (the library product it replaces ran 8.4 - 8.7 us
+// at 1, 32 and 40 rows, hidden 2048, 512 experts, and another 2 us widened its BF16 result; this one TIMING): latency
+// bound (2 MB of weights), so sixteen columns a workgroup and K over its sixteen wavefronts, every load of a wavefront's
+// four steps in flight together; MT row tiles of sixteen share a weight fragment. Partial tiles through LDS, added in
+// wavefront order, rounded to BF16 once.
+template <int MT>
+__global__ __launch_bounds__(1024) void moe_router_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ x, uint16_t* __restrict__ logits, int e,
+                                                          int h, int m) {
+  extern __shared__ __align__(16) float part[];  // [16 wavefronts][MT][256]
+  constexpr int BATCH = 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, n0 = blockIdx.x * 16;
+  const int steps = h / 32, s0 = steps * wave / 16, s1 = steps * (wave + 1) / 16;
+  const uint16_t* wat = w + (int64_t)min(n0 + r16, e - 1) * h + 8 * (lane >> 4);
+  const uint16_t* xat[MT];
+  f32x4_t acc[MT];
+#pragma unroll
+  for (int t = 0; t < MT; t++) {
+    xat[t] = x + (int64_t)min(16 * t + r16, m - 1) * h + 8 * (lane >> 4);
+    acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  for (int s = s0; s < s1; s += BATCH) {
+    u32x4_t b[BATCH], a[BATCH][MT];
+#pragma unroll
+    for (int j = 0; j < BATCH; j++)
+      if (s + j < s1) {
+        b[j] = *reinterpret_cast<const u32x4_t*>(wat + 32 * (s + j));
+#pragma unroll
+        for (int t = 0; t < MT; t++) a[j][t] = *reinterpret_cast<const u32x4_t*>(xat[t] + 32 * (s + j));
+      }
+#pragma unroll
+    for (int j = 0; j < BATCH; j++)
+      if (s + j < s1) {
+#pragma unroll
+        for (int t = 0; t < MT; t++)
+          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[j][t]), __builtin_bit_cast(bf16x8_t, b[j]), acc[t], 0, 0, 0);
+      }
+  }
+#pragma unroll
+  for (int t = 0; t < MT; t++) *reinterpret_cast<f32x4_t*>(part + (wave * MT + t) * 256 + lane * 4) = acc[t];
+  __syncthreads();
+  for (int i = threadIdx.x; i < MT * 256; i += 1024) {
+    const int t = i >> 8, row = (i >> 4) & 15, n = n0 + (i & 15), at = t * 256 + ((row >> 2) * 16 + (i & 15)) * 4 + (row & 3);
+    float sum = 0.f;
+#pragma unroll
+    for (int v = 0; v < 16; v++) sum += part[v * MT * 256 + at];
+    if (16 * t + row < m && n < e) logits[(int64_t)(16 * t + row) * e + n] = bf16_of(sum);
+  }
+}
+
 // The last launch of a small latent block (nemotron_moe.cu's out kernel): out = bf16(shared + routed fc2^T) with
 // routed BF16 [m, latent]; sixteen output columns a workgroup, K split over its wavefronts (at most eight steps each).
 struct OutGemv {
@@ -898,8 +947,8 @@ static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, in
   if (m > ROUTE_FUSED_ROWS && pairs < PLAN_WIDE_PAIRS && g_route_plan_fused.load(std::memory_order_relaxed) != 2) {
     // a verify-sized call: the routing spread over the device, the plan by the workgroup that finishes last
     const int groups = (m + ROUTE_GROUP_ROWS - 1) / ROUTE_GROUP_ROWS;
-    // rows that name no expert twice: every row is real (a padded row repeats one id over its slots)
-    const int by_rows = !rp.slots && m <= PLAN_ROWS_MAX && rp.k <= 64 && g_route_plan_fused.load(std::memory_order_relaxed) != 1;
+    // rows that name no expert twice: every row is real, or a padded row names none (with `repeat` it names one over and over)
+    const int by_rows = (!rp.slots || (!rp.repeat && (rp.pad_id < e_lo || rp.pad_id >= e_lo + e_n))) && m <= PLAN_ROWS_MAX && rp.k <= 64 && g_route_plan_fused.load(std::memory_order_relaxed) != 1;
     HB_LAUNCH(moe_route_plan_kernel, dim3((unsigned)groups + plan_groups(job) - 1u), dim3(PLAN_THREADS), plan_lds, stream, rp.ids, (int)pairs, e_lo, e_n,
               shared_rows, ws.plan, ws.order, rp, m, groups, by_rows, slot_rows, (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows),
               job ? *job : QuantJob{});
@@ -918,17 +967,30 @@ static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, in
   return HB_OK;
 }
 
-int moe_launch_route_plan(const float* logits, int m, int e, int topk, int32_t* ids, float* weights, int e_lo, int e_n, int shared_rows,
+void moe_launch_router(const uint16_t* x, const uint16_t* w, int m, int e, int h, uint16_t* logits, hipStream_t stream) {
+  const dim3 grid((unsigned)((e + 15) / 16));
+  if (m <= 16) {
+    HB_LAUNCH(moe_router_kernel<1>, grid, dim3(1024), 16 * 1024, stream, w, x, logits, e, h, m);
+  } else if (m <= 32) {
+    HB_LAUNCH(moe_router_kernel<2>, grid, dim3(1024), 32 * 1024, stream, w, x, logits, e, h, m);
+  } else {
+    HB_LAUNCH(moe_router_kernel<4>, grid, dim3(1024), 64 * 1024, stream, w, x, logits, e, h, m);
+  }
+}
+
+int moe_launch_route_plan(const TopkRoute& route, int m, int topk, int32_t* ids, float* weights, int e_lo, int e_n, int shared_rows,
                           const MoeWorkspace& ws, hipStream_t stream, int slot_rows, const QuantJob* job) {
-  if (int err = moe_check_route(m, e, topk)) return err;
+  if (int err = moe_check_route(m, route.e, topk)) return err;
   RouteParams rp{};
-  rp.logits = logits;
-  rp.stride = e;
-  rp.e = e;
+  rp.logits = static_cast<const float*>(route.logits);
+  rp.half = route.half;
+  rp.stride = route.e;
+  rp.slots = route.slots;
+  rp.e = route.e;
   rp.k = topk;
-  rp.per = (e + 63) / 64;
-  rp.steps = 1;
-  rp.pad_id = e;
+  rp.per = (route.e + 63) / 64;
+  rp.steps = route.steps;
+  rp.pad_id = route.e;
   rp.ids = ids;
   rp.weights = weights;
   return launch_route_plan(rp, m, e_lo, e_n, shared_rows, ws, stream, slot_rows, job);

@@ -46,6 +46,7 @@ struct RouteParams {
   int e, k, per, latent;
   int pad_id;            // the id of a padded row's slots without `repeat` (the callers' default: e, "no expert")
   int sigmoid;           // the rule a kernel that serves both applies (route_any)
+  int half;              // softmax: `logits` points to BF16 values (read as FP32: the router's product as it was rounded)
   int32_t* ids;
   float* weights;
   uint16_t* lat;         // sigmoid: BF16 [m, latent], the row's latent columns
@@ -81,14 +82,27 @@ __device__ __forceinline__ int route_row(const RouteParams& p, int r, int lane, 
     }
   }
   const float* row = p.logits + (int64_t)(padded ? 0 : r) * p.stride;  // a padded row repeats row 0's first choice
+  const uint16_t* row16 = reinterpret_cast<const uint16_t*>(p.logits) + (int64_t)(padded ? 0 : r) * p.stride;
   float val[PER];   // the weight an expert would get before renormalization
   uint32_t key[PER];
   float lg[PER];    // the lane's logits: every load is asked for before the first is used
-  if (!THROUGH && PER == 8 && per == 8 && e == 512 && !((p.stride | (int64_t)(reinterpret_cast<uintptr_t>(p.logits) >> 2)) & 3)) {
+  if (!THROUGH && PER == 8 && per == 8 && e == 512 && !p.half && !((p.stride | (int64_t)(reinterpret_cast<uintptr_t>(p.logits) >> 2)) & 3)) {
     // the lane's eight logits are 32 consecutive bytes on a 16-byte boundary: two loads instead of eight
     const f32x4_t lo = *reinterpret_cast<const f32x4_t*>(row + first), hi = *reinterpret_cast<const f32x4_t*>(row + first + 4);
     lg[0] = lo.x, lg[1] = lo.y, lg[2] = lo.z, lg[3] = lo.w;
     if constexpr (PER >= 8) lg[4] = hi.x, lg[5] = hi.y, lg[6] = hi.z, lg[7] = hi.w;
+  } else if (!SIGMOID && p.half) {
+    if (PER == 8 && per == 8 && e == 512 && !(reinterpret_cast<uintptr_t>(row16) & 15)) {  // ... and one for eight BF16
+      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(row16 + first);
+#pragma unroll
+      for (int j = 0; j < 4; j++) {
+        lg[2 * j] = __uint_as_float(v[j] << 16);
+        lg[2 * j + 1] = __uint_as_float(v[j] & 0xffff0000u);
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < PER; j++) lg[j] = bf16_bits_to_f32(row16[min(first + j, e - 1)]);
+    }
   } else {
 #pragma unroll
     for (int j = 0; j < PER; j++) lg[j] = logit(row + min(first + j, e - 1));

@@ -541,8 +541,19 @@ struct BudgetRoute {
 // caller's arrays). `scratch`: room for the rows' candidates between the two launches (160 bytes a row).
 int moe_launch_budget_plan(const BudgetRoute& b, int m, int topk, int32_t* ids, float* weights, int e_lo, int e_n, int shared_rows,
                            const MoeWorkspace& ws, void* scratch, hipStream_t stream, int slot_rows = ROWS_PER_SLOT);
-int moe_launch_route_plan(const float* logits, int m, int e, int topk, int32_t* ids, float* weights, int e_lo, int e_n, int shared_rows,
+// The top-k routing of a routed call: logits FP32 or (`half`) BF16 [m, e]; row r is real iff slots[r / steps] != 0 (null:
+// every row), a padded row names no expert.
+struct TopkRoute {
+  const void* logits;
+  int half, e;
+  const int32_t* slots;
+  int steps;
+};
+int moe_launch_route_plan(const TopkRoute& route, int m, int topk, int32_t* ids, float* weights, int e_lo, int e_n, int shared_rows,
                           const MoeWorkspace& ws, hipStream_t stream, int slot_rows = ROWS_PER_SLOT, const QuantJob* job = nullptr);
+// The router's product of a call of at most MOE_ROUTER_ROWS rows: logits BF16 [m, e] = x [m, h] w[e, h]^T (h % 32 == 0).
+constexpr int MOE_ROUTER_ROWS = HB_ROUTER_MAX_ROWS;
+void moe_launch_router(const uint16_t* x, const uint16_t* w, int m, int e, int h, uint16_t* logits, hipStream_t stream);
 
 struct CombineParams {
   const void* pairs;      // [m * topk (+ m), h] FP32 or BF16

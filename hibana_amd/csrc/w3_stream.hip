@@ -1132,12 +1132,11 @@ int check_experts(const hb_w3_experts* ex) {
 
 // plan -> fc1 -> fc2 (-> combine, when `combine` is given): `out_pairs` receives fc2's per-pair outputs (the
 // workspace's y unless the caller wants the pairs themselves). One token's fc2 and combine are one launch.
-struct Routing {  // set: the chain routes `logits` [m, e] itself into the caller's ids / weights
-  const float* logits;
-  int e;
+struct Routing {  // set: the chain routes the logits itself into the caller's ids / weights
+  TopkRoute top;
   int32_t* ids;
   float* weights;
-  const BudgetRoute* budget = nullptr;  // ... under a budget, from BF16 logits (`logits` is then unused)
+  const BudgetRoute* budget = nullptr;  // ... under a budget (`top` is then unused)
 };
 
 int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void* x, const int32_t* ids, int m, int topk,
@@ -1159,9 +1158,9 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
                               : QuantJob{static_cast<const uint16_t*>(x), (int64_t)m * ex->hidden / 8, ws.xq, ws.xs, 0, 0};
   const QuantJob* job = e4m3 || split ? &xjob : nullptr;
   // one token from its logits, a slot a selection, and fc2 + combine as one launch after it: fc1 routes for itself
-  const bool route_in_fc1 = route && !route->budget && m == 1 && combine && !e4m3 && !split && !dense && topk <= 63 && slots == topk + shared_rows &&
+  const bool route_in_fc1 = route && !route->budget && !route->top.slots && m == 1 && combine && !e4m3 && !split && !dense && topk <= 63 && slots == topk + shared_rows &&
                             slots + (combine->gate_vec && combine->shared ? ONE_GATE_WAVES : 0) <= ONE_MAX_WAVES && g_tune.moe_one == 0 &&
-                            moe_check_route(m, route->e, topk) == HB_OK;
+                            moe_check_route(m, route->top.e, topk) == HB_OK;
   if (route_in_fc1) {
     // (nothing to launch here)
   } else if (route && route->budget) {
@@ -1171,8 +1170,7 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
     if (int e = moe_launch_budget_plan(*route->budget, m, topk, route->ids, route->weights, ex->base, ex->experts, shared_rows, ws, ws.y, stream, slot_rows))
       return e;
   } else if (route) {
-    if (int e = moe_launch_route_plan(route->logits, m, route->e, topk, route->ids, route->weights, ex->base, ex->experts, shared_rows, ws, stream,
-                                      slot_rows, job))
+    if (int e = moe_launch_route_plan(route->top, m, topk, route->ids, route->weights, ex->base, ex->experts, shared_rows, ws, stream, slot_rows, job))
       return e;
   } else if (int e = moe_launch_plan(ids, pairs, ex->base, ex->experts, shared_rows, ws, stream, slot_rows, job)) {
     return e;
@@ -1292,13 +1290,14 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
     if (int e = shape_stream(q, est, l1)) return e;
     q.a_stride = 0;  // every slot's row is the token's
     RouteParams rp{};
-    rp.logits = route->logits;
-    rp.stride = route->e;
-    rp.e = route->e;
+    rp.logits = static_cast<const float*>(route->top.logits);
+    rp.half = route->top.half;
+    rp.stride = route->top.e;
+    rp.e = route->top.e;
     rp.k = topk;
-    rp.per = (route->e + 63) / 64;
+    rp.per = (route->top.e + 63) / 64;
     rp.steps = 1;
-    rp.pad_id = route->e;
+    rp.pad_id = route->top.e;
     rp.ids = route->ids;
     rp.weights = route->weights;
     const dim3 grid((unsigned)((q.n_blocks + q.nbw - 1) / q.nbw), (unsigned)slots);
@@ -1511,7 +1510,7 @@ extern "C" int hb_w3_moe_layer_logits(const hb_w3_experts* routed, const hb_w3_e
                                       void* workspace, size_t workspace_bytes, void* stream) {
   if (!logits) return HB_ENULL;
   if (!aligned(logits, 4)) return HB_EINVAL;
-  const Routing route{logits, experts_total, ids, weights};
+  const Routing route{{logits, 0, experts_total, nullptr, 1}, ids, weights};
   return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, &route);
 }
 
@@ -1521,7 +1520,7 @@ extern "C" int hb_w3_moe_layer_budget(const hb_w3_experts* routed, const hb_w3_e
                                       size_t workspace_bytes, void* stream) {
   if (!logits) return HB_ENULL;
   const BudgetRoute b{static_cast<const uint16_t*>(logits), experts_total, keep, budget, steps, 0, per_request, min_cap, slots};
-  const Routing route{nullptr, experts_total, ids, weights, &b};
+  const Routing route{{}, ids, weights, &b};
   return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, &route);
 }
 
@@ -1530,6 +1529,57 @@ extern "C" int hb_w3_moe_layer_logits_e4m3(const hb_w3_experts* routed, const hb
                                            void* workspace, size_t workspace_bytes, void* stream) {
   if (!logits) return HB_ENULL;
   if (!aligned(logits, 4)) return HB_EINVAL;
-  const Routing route{logits, experts_total, ids, weights};
+  const Routing route{{logits, 0, experts_total, nullptr, 1}, ids, weights};
   return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, &route, true);
+}
+
+// The layer from its input rows: [workspace of the routed call][BF16 logits][ids][weights].
+namespace {
+struct LayerScratch {
+  size_t moe;  // the routed call's bytes
+  uint16_t* logits;
+  int32_t* ids;
+  float* weights;
+  size_t bytes;
+};
+LayerScratch layer_scratch(void* base, size_t moe, int m, int topk, int experts_total) {
+  LayerScratch l{moe, nullptr, nullptr, nullptr, 0};
+  size_t off = moe;
+  auto take = [&](size_t bytes) {
+    void* ptr = base ? static_cast<char*>(base) + off : nullptr;
+    off += (bytes + 255) & ~(size_t)255;
+    return ptr;
+  };
+  l.logits = static_cast<uint16_t*>(take((size_t)m * experts_total * 2));
+  l.ids = static_cast<int32_t*>(take((size_t)m * topk * 4));
+  l.weights = static_cast<float*>(take((size_t)m * topk * 4));
+  l.bytes = off;
+  return l;
+}
+}  // namespace
+
+extern "C" size_t hb_w3_moe_layer_rows_workspace_bytes(int m, int topk, const hb_w3_experts* routed, int shared, int experts_total) {
+  const size_t moe = hb_w3_moe_workspace_bytes(m, topk, routed, shared);
+  return moe && experts_total > 0 ? layer_scratch(nullptr, moe, m, topk, experts_total).bytes : 0;
+}
+
+extern "C" int hb_w3_moe_layer_rows(const hb_w3_experts* routed, const hb_w3_experts* shared, const float* gate_vec, const void* x, const void* router,
+                                    const void* logits, int experts_total, int m, int topk, int keep, int budget, const int32_t* slots, int steps,
+                                    int per_request, int min_cap, void* out, void* workspace, size_t workspace_bytes, void* stream) {
+  if (int e = check_experts(routed)) return e;
+  if (!x || !workspace || (!router && !logits)) return HB_ENULL;
+  if (m <= 0 || topk <= 0 || experts_total <= 0 || steps <= 0) return HB_EINVAL;
+  if (!aligned(x, 16) || !aligned(router, 16) || !aligned(logits, 2) || !aligned(slots, 4) || !aligned(workspace, 16)) return HB_EINVAL;
+  if (!logits && m > MOE_ROUTER_ROWS) return HB_EINVAL;
+  const size_t moe = hb_w3_moe_workspace_bytes(m, topk, routed, shared != nullptr);
+  const LayerScratch l = layer_scratch(workspace, moe, m, topk, experts_total);
+  if (!moe || workspace_bytes < l.bytes) return HB_EWORKSPACE;
+  const uint16_t* lg = static_cast<const uint16_t*>(logits);
+  if (!lg) {
+    moe_launch_router(static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(router), m, experts_total, routed->hidden, l.logits, as_stream(stream));
+    lg = l.logits;
+  }
+  const BudgetRoute b{lg, experts_total, keep, budget, steps, 0, per_request, min_cap, slots};
+  const Routing route{{lg, 1, experts_total, slots, steps}, l.ids, l.weights, budget > 0 ? &b : nullptr};
+  return moe_layer(routed, shared, gate_vec, x, l.ids, l.weights, m, topk, out, workspace, l.moe, stream, &route);
 }

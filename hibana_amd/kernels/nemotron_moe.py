@@ -48,8 +48,26 @@ class SmallWeights:
             if self.shared_up.in_features != self.hidden or (self.shared_down.out_features, self.shared_down.in_features) != (self.hidden, self.shared_up.out_features):
                 raise ValueError("shared_up [I, H] and shared_down [H, I] do not describe one expert")
         self._routed = None if self.experts is None else self.experts._struct()
+        self._struct = None
+        self._bytes = {}
 
     def struct(self) -> _lib.HbLatentWeights:
+        """The block as the library takes it: assembled once, and again when one of its tensors was replaced."""
+        up, down = self.shared_up, self.shared_down
+        key = (self.gate_fc1.data_ptr(), self.bias.data_ptr(), self.fc2.data_ptr(), None if up is None else (up.tiled.data_ptr(), up.scale2),
+               None if down is None else (down.tiled.data_ptr(), down.scale2))
+        if self._struct is None or self._struct[0] != key:
+            self._struct = key, self._assemble()
+            self._bytes.clear()
+        return self._struct[1]
+
+    def workspace_bytes(self, m: int, k: int) -> int:
+        need = self._bytes.get((m, k))
+        if need is None:
+            need = self._bytes[(m, k)] = _lib.lib().hb_latent_workspace_bytes(C.byref(self.struct()), m, k)
+        return need
+
+    def _assemble(self) -> _lib.HbLatentWeights:
         up, down = self.shared_up, self.shared_down
         return _lib.HbLatentWeights(
             _lib.ptr(self.gate_fc1), _lib.ptr(self.bias), _lib.ptr(self.fc2), None if self._routed is None else C.pointer(self._routed),
@@ -90,14 +108,14 @@ def router(x: torch.Tensor, weights: SmallWeights, bias: torch.Tensor | None, k:
         weights = SmallWeights(weights.gate_fc1, bias, weights.fc2, weights.experts, weights.shared_up, weights.shared_down)
     dev = x.device
     st = weights.struct()
-    need = _lib.lib().hb_latent_workspace_bytes(C.byref(st), m, k)
+    need = weights.workspace_bytes(m, k)
     if need == 0:
         raise ValueError("router: the block's shapes are not ones the kernels take")
     buffer = _lib.workspace(dev, need, "latent")  # the stream's own: a Workspace serves until the next `router` on this stream
-    fused = torch.empty((m, weights.experts_total + weights.latent), dtype=torch.float32, device=dev)
-    ids = torch.empty((m, k), dtype=torch.int32, device=dev)
-    wts = torch.empty((m, k), dtype=torch.float32, device=dev)
-    lat = torch.empty((m, weights.latent), dtype=torch.bfloat16, device=dev)
+    fused = x.new_empty((m, weights.experts_total + weights.latent), dtype=torch.float32)
+    ids = x.new_empty((m, k), dtype=torch.int32)
+    wts = x.new_empty((m, k), dtype=torch.float32)
+    lat = x.new_empty((m, weights.latent))
     sl = None if slots is None else slots.to(torch.int32).contiguous()
     xc = x.contiguous()
     _lib.check(_lib.lib().hb_latent_router(C.byref(st), _lib.ptr(xc), m, k, _lib.ptr(sl), steps, int(route), pad_id, _lib.ptr(fused), _lib.ptr(ids),

@@ -25,15 +25,18 @@ def nvfp4_linear(x: torch.Tensor, lin, prequantized=None, relu2: bool = False) -
     if x.dtype != torch.bfloat16 or x.ndim != 2 or x.shape[1] != lin.in_features:
         raise ValueError("nvfp4_linear: x must be BF16 [M, in_features]")
     _lib.need_gpu(x)
-    lin.tile()
-    m = x.shape[0]
-    y = torch.empty((m, lin.out_features), dtype=torch.bfloat16, device=x.device)
+    if lin.tiled is None or lin.scale2 is None:
+        lin.tile()
+    m, n, k = x.shape[0], lin.out_features, lin.in_features
+    y = x.new_empty((m, n))
     if m:
+        lib = _lib.lib()
         xc = x.contiguous()  # held until the launch is enqueued: a temporary's block could be handed out again before that
-        need = _lib.lib().hb_nvfp4_gemm_workspace_bytes(m, lin.out_features, lin.in_features)  # a few dozen rows: K shared among workgroups
+        need = lib.hb_nvfp4_gemm_workspace_bytes(m, n, k)  # a few dozen rows: K shared among workgroups
         ws = _lib.workspace(x.device, need, "gemm") if need else None
-        _lib.check(_lib.lib().hb_nvfp4_gemm_ws(_lib.ptr(xc), m, _lib.ptr(lin.tiled), lin.global_scale, lin.out_features, lin.in_features, int(relu2),
-                                               _lib.ptr(y), _lib.ptr(ws), need, _lib.stream()), "nvfp4_linear")
+        code = lib.hb_nvfp4_gemm_ws(xc.data_ptr(), m, lin.tiled.data_ptr(), lin.scale2, n, k, int(relu2), y.data_ptr(), _lib.ptr(ws), need, _lib.stream())
+        if code:
+            _lib.check(code, "nvfp4_linear")
     return y
 
 
@@ -80,8 +83,8 @@ def silu_mul_quant_groups(gate_up: torch.Tensor, pairs: int = 0, torch_chain: bo
     _lib.need_gpu(gate_up)
     gu = gate_up.contiguous()
     m = gu.shape[0]
-    q = torch.empty((m, half), dtype=torch.float8_e4m3fn, device=gu.device)
-    scales = torch.empty((m, half // 32), dtype=torch.float32, device=gu.device)
+    q = gu.new_empty((m, half), dtype=torch.float8_e4m3fn)
+    scales = gu.new_empty((m, half // 32), dtype=torch.float32)
     if m:
         _lib.check(_lib.lib().hb_silu_mul_quant_groups(_lib.ptr(gu), m, half, pairs, int(torch_chain), _lib.ptr(q), _lib.ptr(scales), _lib.stream()),
                    "silu_mul_quant_groups")

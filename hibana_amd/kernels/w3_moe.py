@@ -115,10 +115,33 @@ def tile(experts: W3Experts, release: bool = False) -> W3Experts:
 
 
 def _struct(experts: W3Experts) -> _lib.HbW3Experts:
-    tile(experts)
-    (n1, h), (h2, i) = experts.shape13, experts.shape2
-    return _lib.HbW3Experts(_lib.ptr(experts.tiled13), _lib.ptr(experts.row13), _lib.ptr(experts.tiled2), _lib.ptr(experts.row2),
-                            experts.lut, experts.fc2_lut, experts.experts, experts.base, h, i, h2, int(gated(experts)))
+    """The experts as the library takes them: built once, and again when a tensor or a number of `experts` was replaced."""
+    if experts.tiled13 is None or experts.tiled2 is None:
+        tile(experts)
+    key = (experts.tiled13.data_ptr(), experts.row13.data_ptr(), experts.tiled2.data_ptr(), experts.row2.data_ptr(), experts.lut,
+           experts.fc2_lut, experts.row13.shape[0], experts.base, experts.shape13, experts.shape2)
+    have = experts.__dict__.get("_packed")
+    if have is None or have[0] != key:
+        (n1, h), (h2, i) = experts.shape13, experts.shape2
+        have = key, _lib.HbW3Experts(*key[:8], h, i, h2, int(gated(experts)))
+        have[1].bytes_of = {}  # the workspace a call of (rows, k, ...) takes
+        experts._packed = have
+    return have[1]
+
+
+def _workspace_bytes(st: _lib.HbW3Experts, m: int, k: int, shared: bool, experts_total: int = 0) -> int:
+    """hb_w3_moe_workspace_bytes or, with `experts_total`, hb_w3_moe_layer_rows_workspace_bytes: asked once a size."""
+    key = (m, k, shared, experts_total)
+    need = st.bytes_of.get(key)
+    if need is None:
+        if len(st.bytes_of) >= 4096:
+            st.bytes_of.clear()
+        if experts_total:
+            need = _lib.lib().hb_w3_moe_layer_rows_workspace_bytes(m, k, C.byref(st), int(shared), experts_total)
+        else:
+            need = _lib.lib().hb_w3_moe_workspace_bytes(m, k, C.byref(st), int(shared))
+        st.bytes_of[key] = need
+    return need
 
 
 def _check_call(experts: W3Experts, x, ids, weights):
@@ -149,7 +172,7 @@ def w3_moe(experts: W3Experts, x: torch.Tensor, ids: torch.Tensor, weights: torc
     if m == 0:
         return out
     st = _struct(experts)
-    need = _lib.lib().hb_w3_moe_workspace_bytes(m, k, C.byref(st), 0)
+    need = _workspace_bytes(st, m, k, False)
     ws = _lib.workspace(x.device, need)
     ids32 = ids.to(torch.int32).contiguous()
     wt = weights.float().contiguous()
@@ -173,7 +196,7 @@ def moe_layer(experts: W3Experts, x: torch.Tensor, ids: torch.Tensor, weights: t
         return out
     st = _struct(experts)
     sh = _struct(shared) if shared is not None else None
-    need = _lib.lib().hb_w3_moe_workspace_bytes(m, k, C.byref(st), int(shared is not None))
+    need = _workspace_bytes(st, m, k, shared is not None)
     ws = _lib.workspace(x.device, need)
     ids32 = ids.to(torch.int32).contiguous()
     wt = weights.float().contiguous()
@@ -204,7 +227,7 @@ def moe_layer_logits(experts: W3Experts, x: torch.Tensor, logits: torch.Tensor, 
     if m:
         st = _struct(experts)
         sh = _struct(shared) if shared is not None else None
-        need = _lib.lib().hb_w3_moe_workspace_bytes(m, topk, C.byref(st), int(shared is not None))
+        need = _workspace_bytes(st, m, topk, shared is not None)
         ws = _lib.workspace(x.device, need)
         gv = None if gate_vec is None else gate_vec.float().contiguous()
         entry = _lib.lib().hb_w3_moe_layer_logits_e4m3 if e4m3 else _lib.lib().hb_w3_moe_layer_logits
@@ -238,7 +261,7 @@ def moe_layer_budget(experts: W3Experts, x: torch.Tensor, logits: torch.Tensor, 
     if m:
         st = _struct(experts)
         sh = _struct(shared) if shared is not None else None
-        need = _lib.lib().hb_w3_moe_workspace_bytes(m, topk, C.byref(st), int(shared is not None))
+        need = _workspace_bytes(st, m, topk, shared is not None)
         ws = _lib.workspace(x.device, need)
         gv = None if gate_vec is None else gate_vec.float().contiguous()
         sl = None if slots is None else slots.to(torch.int32).contiguous()
@@ -247,6 +270,42 @@ def moe_layer_budget(experts: W3Experts, x: torch.Tensor, logits: torch.Tensor, 
                                                      e_total, m, topk, keep, budget, _lib.ptr(sl), steps, per_request, min_cap, _lib.ptr(ids),
                                                      _lib.ptr(wt), _lib.ptr(out), _lib.ptr(ws), need, _lib.stream()), "moe_layer_budget")
     return (out, ids, wt) if return_routing else out
+
+
+ROUTER_ROWS = 64  # rows up to which the library makes the router's product itself (HB_ROUTER_MAX_ROWS)
+
+
+def moe_layer_rows(experts: W3Experts, x: torch.Tensor, router: torch.Tensor, topk: int, keep: int = 0, budget: int = 0,
+                   slots: torch.Tensor | None = None, steps: int = 1, per_request: int = 0, min_cap: int = 0, shared: W3Experts | None = None,
+                   gate_vec: torch.Tensor | None = None) -> torch.Tensor:
+    """The whole layer from its input rows: logits = bf16(x router^T) (router BF16 [E_total, hidden], contiguous; up to
+    ROUTER_ROWS rows in the library's own launch, beyond in a torch GEMM), then `moe_layer_budget` (`budget` > 0) or
+    softmax top-k routing and `moe_layer`, in one chain of launches; with `slots`, the padded rows of the graph name no
+    expert. Logits, ids and weights stay in the workspace (hibana/model/flashnext/moe.py:122-192)."""
+    m, e_total = x.shape[0], router.shape[0]
+    if x.dtype != torch.bfloat16 or x.ndim != 2 or x.shape[1] != experts.shape13[1]:
+        raise ValueError("moe_layer_rows: x must be BF16 [M, hidden]")
+    if router.dtype != torch.bfloat16 or router.ndim != 2 or router.shape[1] != x.shape[1] or not router.is_contiguous():
+        raise ValueError("moe_layer_rows: router must be BF16 [experts, hidden], contiguous")
+    if steps < 1 or m % steps or budget < 0 or (slots is not None and slots.numel() < m // steps):
+        raise ValueError("moe_layer_rows: whole requests of `steps` rows, a slot for every request")
+    if budget and not (20 <= e_total <= 1024 and 1 <= topk <= 20 and 0 <= keep <= 20):
+        raise ValueError("moe_layer_rows: under a budget 20 <= E <= 1024, topk and keep at most 20")
+    _lib.need_gpu(x, router, slots)
+    out = x.new_empty((m, experts.shape2[0]))
+    if m:
+        st = _struct(experts)
+        sh = None if shared is None else C.byref(_struct(shared))
+        need = _workspace_bytes(st, m, topk, shared is not None, e_total)
+        ws = _lib.workspace(x.device, need)
+        gv = None if gate_vec is None else gate_vec.float().contiguous()
+        sl = None if slots is None else slots.to(torch.int32).contiguous()
+        xc = x.contiguous()
+        logits = None if m <= ROUTER_ROWS else torch.mm(xc, router.T)
+        _lib.check(_lib.lib().hb_w3_moe_layer_rows(C.byref(st), sh, _lib.ptr(gv), xc.data_ptr(), router.data_ptr(), _lib.ptr(logits), e_total, m, topk, keep,
+                                                   budget, _lib.ptr(sl), steps, per_request, min_cap, out.data_ptr(), ws.data_ptr(), need, _lib.stream()),
+                   "moe_layer_rows")
+    return out
 
 
 # ------------------------------------------------------------------ offline: 3-bit experts from NVFP4 experts

@@ -140,14 +140,11 @@ class MoeLayer:
             pairs = w3_moe.w3_moe(self.w3, x, ids, weights, pairs=True, pairs_bf16=x.shape[0] >= w3_moe.WIDE_ROWS)
             shared = ops.nvfp4_linear(ops.silu_and_mul(ops.nvfp4_linear(x, self.shared_gate_up)), self.shared_down)
             return ops.moe_combine_pairs(pairs, ids, weights, shared, x, self.shared_gate_vec, self.w3.base, self.w3.experts)
-        slots, _ = self._padding(ctx)
-        if slots is None and not self.selects(ctx):  # routing, plan, both streams and the combine as one chain
-            logits = torch.mm(x, self.router.T).float()
-            return w3_moe.moe_layer_logits(self.w3, x, logits, self.topk, shared=self.shared, gate_vec=self.shared_gate_vec)
-        if self.selects(ctx) and self.budget:  # the selection's launches and the experts' as one chain
-            logits = torch.mm(x, self.router.T)
-            _, steps = self._padding(ctx)
-            return w3_moe.moe_layer_budget(self.w3, x, logits, self.topk, self.guarantee(x.shape[0], steps), self.budget, slots, steps,
-                                           per_request=self.per_request, min_cap=self.MIN_CAP, shared=self.shared, gate_vec=self.shared_gate_vec)
-        ids, weights = self.route(x, ctx)
-        return w3_moe.moe_layer(self.w3, x, ids, weights, shared=self.shared, gate_vec=self.shared_gate_vec)
+        # router product, routing (or the budgeted selection), plan, both streams and the combine as one chain
+        slots, steps = self._padding(ctx)
+        if not self.selects(ctx):
+            return w3_moe.moe_layer_rows(self.w3, x, self.router, self.topk, slots=slots, steps=steps, shared=self.shared, gate_vec=self.shared_gate_vec)
+        if not self.budget:  # each token's top `keep` alone, padded rows as any other
+            return w3_moe.moe_layer_rows(self.w3, x, self.router, self.keep, shared=self.shared, gate_vec=self.shared_gate_vec)
+        return w3_moe.moe_layer_rows(self.w3, x, self.router, self.topk, self.guarantee(x.shape[0], steps), self.budget, slots, steps,
+                                     per_request=self.per_request, min_cap=self.MIN_CAP, shared=self.shared, gate_vec=self.shared_gate_vec)

@@ -301,6 +301,20 @@ int hb_w3_moe_layer_budget(const hb_w3_experts* routed, const hb_w3_experts* sha
                            const int32_t* slots, int steps, int per_request, int min_cap, int32_t* ids, float* weights,
                            void* out, void* workspace, size_t workspace_bytes, void* stream);
 
+/* The layer from its input rows: x BF16 [m, hidden] -> the router's product (logits = bf16(x router^T), router BF16
+ * [experts_total, hidden], hidden % 32 == 0, at most HB_ROUTER_MAX_ROWS rows; or the caller's BF16 `logits`
+ * [m, experts_total], any m), the routing, then the chain of hb_w3_moe_layer. budget == 0: hb_route_softmax_topk's rule on
+ * those logits (slots / steps as there; a padded row names no expert); budget > 0: hb_route_budget's rule (keep,
+ * per_request, min_cap as there). Logits, ids and weights stay in the workspace
+ * (hb_w3_moe_layer_rows_workspace_bytes; its head as every routed call's).
+ * ref: MoeLayer.__call__, hibana/model/flashnext/moe.py:122-192. */
+#define HB_ROUTER_MAX_ROWS 64
+size_t hb_w3_moe_layer_rows_workspace_bytes(int m, int topk, const hb_w3_experts* routed, int shared, int experts_total);
+int hb_w3_moe_layer_rows(const hb_w3_experts* routed, const hb_w3_experts* shared, const float* gate_vec, const void* x,
+                         const void* router, const void* logits, int experts_total, int m, int topk, int keep,
+                         int budget, const int32_t* slots, int steps, int per_request, int min_cap, void* out,
+                         void* workspace, size_t workspace_bytes, void* stream);
+
 /* out = bf16( bf16(sum over the row's local slots of w * pairs) + g * shared ) from unsummed pair outputs (FP32 or,
  * pairs_bf16 != 0, BF16) [m * topk, h]; shared BF16 [m, h] or NULL; gate_vec float32 [h] or NULL (then g = 1; x
  * unused). ref: moe_combine_pairs, hibana/kernels/flashnext_fused.py:530-571; with shared == NULL it is

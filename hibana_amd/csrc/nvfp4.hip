@@ -2,13 +2,13 @@
 //
 // Tile layout: blocks of 64 output rows x 128 k, NVFP4_BLOCK_BYTES each, [rows/64][K/128]:
 //   bytes    0..4095  codes: four 128-bit loads per lane, load nt of lane l at (nt * 64 + l) * 16. Lane l = 16 q + r owns,
-//                     for the 16-row tile nt, the weights  row 64 nb + 16 nt + r,  k = 128 c + 16 b + 4 q + i
-//                     (b = 0..7 the 16-blocks of the chunk, i = 0..3): dword b / 2 of the load, its low half for even b,
-//                     high half for odd b, nibble i. That is the B operand of v_mfma_f32_16x16x16_bf16, one MFMA per
-//                     16-block, so the block scale multiplies the MFMA's FP32 result.
-//   bytes 4096..4607  scales: 32 B per row-in-tile r at 4096 + 32 r: byte 8 nt + b is the E4M3 scale of row
-//                     64 nb + 16 nt + r, block 8 c + b.
-// Codes expand with v_cvt_scalef32_pk_bf16_fp4 (two weights per instruction, exact).
+//                     for the 16-row tile nt, the weights of row 64 nb + 16 nt + r: dword s holds k = 128 c + 32 s + 8 q .. + 7,
+//                     nibble i the i-th. That is the lane's operand of v_mfma_f32_16x16x32_bf16 for the 32-k step s, eight
+//                     consecutive k of ONE 16-block (2 s + q / 2), so the activations' side is one 16-byte piece of a row
+//                     and an expansion has one block scale.
+//   bytes 4096..4607  scales: 16 B per row-in-tile r and block parity u at 4096 + 16 (2 r + u): byte 4 nt + s is the E4M3
+//                     scale of row 64 nb + 16 nt + r, block 8 c + 2 s + u - the sixteen scales of lane (q, r), u = q / 2.
+// Codes expand with v_cvt_scalef32_pk_{bf16,f32}_fp4 (two weights per instruction, exact).
 #include <string.h>
 
 #include <atomic>
@@ -21,7 +21,6 @@ namespace hb {
 
 constexpr int NVFP4_BLOCK_BYTES = 4608;
 constexpr int NVFP4_SCALE_OFFSET = 4096;
-typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4_t;
 typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
 
 __host__ __device__ inline int64_t swizzled_scale_offset(int64_t r, int c, int groups_pad) {
@@ -38,15 +37,10 @@ __global__ __launch_bounds__(256) void nvfp4_repack_codes_kernel(const uint8_t* 
   const int64_t nb = blk / chunks;
   const int c = (int)(blk % chunks);
   const int64_t n = nb * 64 + nt * 16 + r;
-  const uint8_t* src = weight + n * (chunks * 64) + c * 64;  // 64 bytes per chunk per row
+  const uint8_t* src = weight + n * (chunks * 64) + c * 64 + 4 * q;  // 64 bytes per chunk per row, 16 a step
   uint32_t d[4];
 #pragma unroll
-  for (int e = 0; e < 4; e++) {
-    // blocks 2e and 2e+1: bytes at k/2 = 8 b + 2 q, two bytes each (four nibbles)
-    const uint32_t lo = src[16 * e + 2 * q] | ((uint32_t)src[16 * e + 2 * q + 1] << 8);
-    const uint32_t hi = src[16 * e + 8 + 2 * q] | ((uint32_t)src[16 * e + 8 + 2 * q + 1] << 8);
-    d[e] = lo | (hi << 16);
-  }
+  for (int e = 0; e < 4; e++) d[e] = src[16 * e] | (uint32_t)src[16 * e + 1] << 8 | (uint32_t)src[16 * e + 2] << 16 | (uint32_t)src[16 * e + 3] << 24;
   *reinterpret_cast<u32x4_t*>(tiled + blk * NVFP4_BLOCK_BYTES + (nt * 64 + lane) * 16) = u32x4_t{d[0], d[1], d[2], d[3]};
 }
 
@@ -56,13 +50,13 @@ __global__ __launch_bounds__(256) void nvfp4_repack_scales_kernel(const uint8_t*
   const int64_t id = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (id >= blocks * 512) return;
   const int64_t blk = id >> 9;
-  const int within = (int)(id & 511), r = within >> 5, nt = (within >> 3) & 3, b = within & 7;
+  const int within = (int)(id & 511), r = within >> 5, u = (within >> 4) & 1, nt = (within >> 2) & 3, b = 2 * (within & 3) + u;
   const int64_t nb = blk / chunks;
   const int c = (int)(blk % chunks);
   const int64_t n = nb * 64 + nt * 16 + r;
   const int groups = chunks * 8, g = 8 * c + b;
   const uint8_t v = swizzled ? scales[swizzled_scale_offset(n, g, (groups + 3) / 4 * 4)] : scales[n * groups + g];
-  tiled[blk * NVFP4_BLOCK_BYTES + NVFP4_SCALE_OFFSET + 32 * r + 8 * nt + b] = v;
+  tiled[blk * NVFP4_BLOCK_BYTES + NVFP4_SCALE_OFFSET + within] = v;
 }
 
 __device__ __forceinline__ float e2m1_to_f32(uint32_t code) {
@@ -85,70 +79,70 @@ __global__ __launch_bounds__(256) void nvfp4_dequant_kernel(const uint8_t* __res
   const int64_t n = nb * 64 + nt * 16 + r;
   const u32x4_t d = *reinterpret_cast<const u32x4_t*>(base + (nt * 64 + lane) * 16);
   const uint32_t dw[4] = {d.x, d.y, d.z, d.w};
-  for (int b = 0; b < 8; b++) {
-    const float s = e4m3_to_f32(base[NVFP4_SCALE_OFFSET + 32 * r + 8 * nt + b]);
-    const uint32_t half = (dw[b >> 1] >> (16 * (b & 1))) & 0xffffu;
-    float* o = out + n * k + c * 128 + 16 * b + 4 * q;
+  for (int t = 0; t < 4; t++) {
+    const float s = e4m3_to_f32(base[NVFP4_SCALE_OFFSET + 16 * (2 * r + (q >> 1)) + 4 * nt + t]);
+    float* o = out + n * k + c * 128 + 32 * t + 8 * q;
 #pragma unroll
-    for (int i = 0; i < 4; i++) o[i] = __fmul_rn(__fmul_rn(e2m1_to_f32((half >> (4 * i)) & 15u), s), global_scale);
+    for (int i = 0; i < 8; i++) o[i] = __fmul_rn(__fmul_rn(e2m1_to_f32((dw[t] >> (4 * i)) & 15u), s), global_scale);
   }
 }
 
-struct Fp4Chunk {  // the weight side of a chunk: four 16-row tiles of codes, their block scales
-  u32x4_t w0, w1, w2, w3, s0, s1;
+struct Fp4Chunk {  // the weight side of a chunk: four 16-row tiles of codes (a dword a step), their block scales (a dword a tile, a byte a step)
+  u32x4_t w0, w1, w2, w3, sc;
+  __device__ __forceinline__ const u32x4_t& tile(int nt) const { return nt == 0 ? w0 : nt == 1 ? w1 : nt == 2 ? w2 : w3; }
 };
 
-struct Fp4Rows {  // the activation side: eight MFMA A fragments (one per 16-block), read from L2
-  u32x2_t a0, a1, a2, a3, a4, a5, a6, a7;
-};
-
-__device__ __forceinline__ void load_fp4_chunk(Fp4Chunk& ch, const uint8_t* blk, int lane, int r16) {
+__device__ __forceinline__ void load_fp4_chunk(Fp4Chunk& ch, const uint8_t* blk, int lane) {
   const u32x4_t* b = reinterpret_cast<const u32x4_t*>(blk);
   ch.w0 = __builtin_nontemporal_load(b + lane);
   ch.w1 = __builtin_nontemporal_load(b + 64 + lane);
   ch.w2 = __builtin_nontemporal_load(b + 128 + lane);
   ch.w3 = __builtin_nontemporal_load(b + 192 + lane);
-  ch.s0 = __builtin_nontemporal_load(b + 256 + 2 * r16);
-  ch.s1 = __builtin_nontemporal_load(b + 257 + 2 * r16);
+  ch.sc = __builtin_nontemporal_load(b + 256 + 2 * (lane & 15) + (lane >> 5));
 }
 
-// One 16-block: two conversions, one MFMA, the block scale folded into the accumulator.
-#define HB_FP4_BLOCK(codes, BYTE0, a_frag, scale_dword, SBYTE, acc)                                                                   \
-  {                                                                                                                                   \
-    u32x2_t packed;                                                                                                                   \
-    packed.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, 1.0f, BYTE0));                           \
-    packed.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, 1.0f, BYTE0 + 1));                       \
-    const f32x4_t part = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(bf16x4_t_s, a_frag), __builtin_bit_cast(bf16x4_t_s, packed), \
-                                                                   f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);                           \
-    const float s = __builtin_amdgcn_cvt_f32_fp8(scale_dword, SBYTE);                                                                 \
-    acc.x = fmaf(part.x, s, acc.x);                                                                                                   \
-    acc.y = fmaf(part.y, s, acc.y);                                                                                                   \
-    acc.z = fmaf(part.z, s, acc.z);                                                                                                   \
-    acc.w = fmaf(part.w, s, acc.w);                                                                                                   \
-  }
+// Byte S of a dword of E4M3 scales as FP32.
+template <int S>
+__device__ __forceinline__ float fp4_scale(uint32_t sc) { return __builtin_amdgcn_cvt_f32_fp8(sc, S); }
 
-typedef __attribute__((ext_vector_type(4))) short bf16x4_t_s;  // the 16x16x16 builtin takes its BF16 operands as 4 x i16
+// The eight weights of one code dword as they are (the block scale is folded into the sums) ...
+__device__ __forceinline__ bf16x8_t fp4_plain(uint32_t codes) {
+  u32x4_t b;
+  b.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, 1.0f, 0));
+  b.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, 1.0f, 1));
+  b.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, 1.0f, 2));
+  b.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, 1.0f, 3));
+  return __builtin_bit_cast(bf16x8_t, b);
+}
+// ... and times their block's scale: a product of a 2-bit and a 4-bit significand, exact in BF16.
+__device__ __forceinline__ bf16x8_t fp4_scaled(uint32_t codes, float s) {
+  const f32x2_pair_t a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(codes, 1.0f, 0), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(codes, 1.0f, 1);
+  const f32x2_pair_t c = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(codes, 1.0f, 2), d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(codes, 1.0f, 3);
+  return __builtin_bit_cast(bf16x8_t, u32x4_t{bf16_pair(a.x * s, a.y * s), bf16_pair(b.x * s, b.y * s), bf16_pair(c.x * s, c.y * s), bf16_pair(d.x * s, d.y * s)});
+}
 
-// Half of a 16-row tile of a chunk: 16-blocks 0 .. 3 (two code dwords, one scale dword, four activation fragments) or
-// 4 .. 7; the blocks of a chunk fold into the accumulator in ascending order either way.
-__device__ __forceinline__ void fp4_half_tile(uint32_t c01, uint32_t c23, uint32_t sc, const u32x2_t& a0, const u32x2_t& a1, const u32x2_t& a2,
-                                              const u32x2_t& a3, f32x4_t& acc) {
-  HB_FP4_BLOCK(c01, 0, a0, sc, 0, acc)
-  HB_FP4_BLOCK(c01, 2, a1, sc, 1, acc)
-  HB_FP4_BLOCK(c23, 0, a2, sc, 2, acc)
-  HB_FP4_BLOCK(c23, 2, a3, sc, 3, acc)
+__device__ __forceinline__ f32x4_t fp4_mfma(const u32x4_t& a, const bf16x8_t& b, const f32x4_t& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), b, c, 0, 0, 0);
+}
+__device__ __forceinline__ void fp4_fold(const f32x4_t& part, float s, f32x4_t& acc) {
+  acc.x = fmaf(part.x, s, acc.x);
+  acc.y = fmaf(part.y, s, acc.y);
+  acc.z = fmaf(part.z, s, acc.z);
+  acc.w = fmaf(part.w, s, acc.w);
 }
 
 // ------------------------------------------------------------------------------------------------ the weight ring
-// (ring.hpp) for NVFP4 blocks: four 16-byte loads a lane of codes, two 4-byte loads a lane of scales.
-struct Fp4Ring {
+// (ring.hpp) for NVFP4 blocks: four 16-byte loads a lane of codes, two 4-byte loads a lane of scales. U: the bit of q that
+// names the parity of the blocks whose scales the lane reads (1: its own weights' blocks; 0: see Fp4Few4Acts).
+template <int U>
+struct Fp4RingOf {
   typedef Fp4Chunk Chunk;
   static constexpr int BLOCK_BYTES = NVFP4_BLOCK_BYTES, LOADS = 6;
   static __device__ __forceinline__ void lanes(RingSource& src, int lane, int r16, uint32_t slot0, uint32_t& codes, uint32_t& scales) {
     src.codes = 16u * lane;
     src.scales = 4u * lane;
     codes = slot0 + 16u * lane;
-    scales = slot0 + 32u * r16;
+    scales = slot0 + 32u * r16 + 16u * ((lane >> (4 + U)) & 1);
   }
   static __device__ __forceinline__ void request(const RingSource& src, int chunk, lds_ptr_t slot) {
     const uint32_t at = (uint32_t)chunk * NVFP4_BLOCK_BYTES;
@@ -164,152 +158,228 @@ struct Fp4Ring {
   template <int BEHIND, int SLOT>
   static __device__ __forceinline__ void take(Chunk& ch, uint32_t codes, uint32_t scales) {
     asm volatile(
-        "s_waitcnt vmcnt(%8)\n\t"
-        "ds_read_b128 %0, %6 offset:%9\n\t"
-        "ds_read_b128 %1, %6 offset:%10\n\t"
-        "ds_read_b128 %2, %6 offset:%11\n\t"
-        "ds_read_b128 %3, %6 offset:%12\n\t"
-        "ds_read_b128 %4, %7 offset:%13\n\t"
-        "ds_read_b128 %5, %7 offset:%14\n\t"
+        "s_waitcnt vmcnt(%7)\n\t"
+        "ds_read_b128 %0, %5 offset:%8\n\t"
+        "ds_read_b128 %1, %5 offset:%9\n\t"
+        "ds_read_b128 %2, %5 offset:%10\n\t"
+        "ds_read_b128 %3, %5 offset:%11\n\t"
+        "ds_read_b128 %4, %6 offset:%12\n\t"
         "s_waitcnt lgkmcnt(0)"  // the slot is read: it may be given to another chunk
-        : "=&v"(ch.w0), "=&v"(ch.w1), "=&v"(ch.w2), "=&v"(ch.w3), "=&v"(ch.s0), "=&v"(ch.s1)
-        : "v"(codes), "v"(scales), "n"(BEHIND), "n"(SLOT * NVFP4_BLOCK_BYTES), "n"(SLOT * NVFP4_BLOCK_BYTES + 1024),
-          "n"(SLOT * NVFP4_BLOCK_BYTES + 2048), "n"(SLOT * NVFP4_BLOCK_BYTES + 3072), "n"(SLOT * NVFP4_BLOCK_BYTES + NVFP4_SCALE_OFFSET),
-          "n"(SLOT * NVFP4_BLOCK_BYTES + NVFP4_SCALE_OFFSET + 16)
+        : "=&v"(ch.w0), "=&v"(ch.w1), "=&v"(ch.w2), "=&v"(ch.w3), "=&v"(ch.sc)
+        : "v"(codes), "v"(scales), "n"(BEHIND), "n"(SLOT * NVFP4_BLOCK_BYTES), "n"(SLOT * NVFP4_BLOCK_BYTES + 1024), "n"(SLOT * NVFP4_BLOCK_BYTES + 2048),
+          "n"(SLOT * NVFP4_BLOCK_BYTES + 3072), "n"(SLOT * NVFP4_BLOCK_BYTES + NVFP4_SCALE_OFFSET)
         : "memory");
   }
 };
+typedef Fp4RingOf<1> Fp4Ring;
 constexpr int FP4_RING_BYTES = ring_bytes<Fp4Ring>();  // LDS per wavefront; its first 4 KB double as the K-split exchange
-
-// The stream's activations: lane (q, r16) feeds row r16, k 4 q .. 4 q + 3 of every 16-block. One chunk's fragments are
-// held; each half is asked for again (for the next chunk) as soon as its blocks are done.
-struct Fp4Acts {
-  static constexpr int LOADS = 8;
-  Fp4Rows held;
-  const uint16_t* at;
-  __device__ __forceinline__ void load_lo(const uint16_t* from) {
-    held.a0 = *reinterpret_cast<const u32x2_t*>(from);
-    held.a1 = *reinterpret_cast<const u32x2_t*>(from + 16);
-    held.a2 = *reinterpret_cast<const u32x2_t*>(from + 32);
-    held.a3 = *reinterpret_cast<const u32x2_t*>(from + 48);
-  }
-  __device__ __forceinline__ void load_hi(const uint16_t* from) {
-    held.a4 = *reinterpret_cast<const u32x2_t*>(from + 64);
-    held.a5 = *reinterpret_cast<const u32x2_t*>(from + 80);
-    held.a6 = *reinterpret_cast<const u32x2_t*>(from + 96);
-    held.a7 = *reinterpret_cast<const u32x2_t*>(from + 112);
-  }
-  template <int EPI>
-  __device__ __forceinline__ void start(const StreamParams& p, const Slot& sl, int, int c0, int, int lane) {
-    at = activation_row<EPI>(p, sl, lane & 15) + (int64_t)c0 * 128 + 4 * (lane >> 4);
-    load_lo(at);
-    load_hi(at);
-  }
-  template <int ODD, bool MORE2, bool MORE1>
-  __device__ __forceinline__ void step(const Fp4Chunk& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot&) {
-    const uint16_t* next = at + (int64_t)(i + 1) * 128;
-    fp4_half_tile(ch.w0.x, ch.w0.y, ch.s0.x, held.a0, held.a1, held.a2, held.a3, acc0);
-    fp4_half_tile(ch.w1.x, ch.w1.y, ch.s0.z, held.a0, held.a1, held.a2, held.a3, acc1);
-    fp4_half_tile(ch.w2.x, ch.w2.y, ch.s1.x, held.a0, held.a1, held.a2, held.a3, acc2);
-    fp4_half_tile(ch.w3.x, ch.w3.y, ch.s1.z, held.a0, held.a1, held.a2, held.a3, acc3);
-    if (MORE1) load_lo(next);
-    fp4_half_tile(ch.w0.z, ch.w0.w, ch.s0.y, held.a4, held.a5, held.a6, held.a7, acc0);
-    fp4_half_tile(ch.w1.z, ch.w1.w, ch.s0.w, held.a4, held.a5, held.a6, held.a7, acc1);
-    fp4_half_tile(ch.w2.z, ch.w2.w, ch.s1.y, held.a4, held.a5, held.a6, held.a7, acc2);
-    fp4_half_tile(ch.w3.z, ch.w3.w, ch.s1.w, held.a4, held.a5, held.a6, held.a7, acc3);
-    if (MORE1) load_hi(next);
-  }
-};
 
 // ---------------------------------------------------------------------------------------- slots of one to eight rows
 //
-// With at most eight rows in the slot the sixteen MFMA rows carry two 16-blocks at once: A row 8 p + i holds row i of
-// the slot over the k of block 2 j + p only (zero over the other block's), so one v_mfma_f32_16x16x32_bf16 does the
-// blocks 2 j and 2 j + 1 of a tile (one code dword: four conversions) and leaves block 2 j + p's partial sums in its
-// output rows 8 p .. 8 p + 7. Half the MFMAs, scale conversions and folds of the sixteen-row body, and four 8-byte
-// activation loads a chunk instead of eight. Lane (q, r16) ends up with block parity q / 2 of slot rows 4 (q % 2) ..
-// + 3: the two parities are added across the lanes after the last chunk, which leaves the sixteen-row layout.
-constexpr int FP4_FEW_ROWS = 8;
+// With few rows in the slot the sixteen MFMA rows carry several 16-blocks at once, so that a block scale is folded into
+// the sums of many weights' products instead of being multiplied into every weight, and the activations are one or two
+// 16-byte loads a lane and chunk.
+//
+// Up to eight rows: A row 8 u + i holds row i of the slot over the lanes of block parity u only (q / 2 == u; zero over
+// the others), so step s leaves block 2 s + u's partial sums in its output rows 8 u .. 8 u + 7: lane (q, r16) ends up with
+// parity q / 2 of slot rows 4 (q % 2) .. + 3 - the parity of its own weights' scales. Sixteen scale conversions and 64
+// multiply-adds a chunk.
+//
+// Up to four rows: two steps 2 t, 2 t + 1 chain into one result. A row 4 j + i holds row i over the blocks 4 t + j only:
+// step 2 t + j / 2 and the lanes of parity j % 2. Lane (q, r16) ends up with block 4 t + q of the slot's four rows: its
+// scale is the byte 2 t + q / 2 of parity q % 2 (the ring hands the lane that parity's). Eight conversions and 32
+// multiply-adds a chunk.
+//
+// The blocks' sums are added across the lanes after the last chunk, which leaves the sixteen-row layout.
+constexpr int FP4_FEW_ROWS = 8, FP4_FEWER_ROWS = 4;
 
-struct Fp4Pieces {  // the lane's four 8-byte pieces of a chunk, one per block pair
-  u32x2_t p0, p1, p2, p3;
-};
-
-struct Fp4FewActs {
+struct Fp4Few8Acts {
   static constexpr int LOADS = 4;
-  Fp4Pieces even, odd;  // of the next even and the next odd chunk
-  bool upper;           // this lane's A row belongs to the odd blocks (p = 1)
-  uint32_t shift;       // 8 * (q / 2): where this lane's OUTPUT rows find their block's scale in a scale dword
-  const uint16_t* at;   // the lane's piece of block pair 0 of the wavefront's first chunk
-  __device__ __forceinline__ void load(Fp4Pieces& to, int i) const {
-    const uint16_t* from = at + (int64_t)i * 128;
-    to.p0 = *reinterpret_cast<const u32x2_t*>(from);
-    to.p1 = *reinterpret_cast<const u32x2_t*>(from + 32);
-    to.p2 = *reinterpret_cast<const u32x2_t*>(from + 64);
-    to.p3 = *reinterpret_cast<const u32x2_t*>(from + 96);
+  u32x4_t even[4], odd[4];  // the lane's piece of each step of the next even and the next odd chunk
+  bool mine;                // this lane's weights belong to its A row's parity
+  const uint16_t* at;       // the lane's piece of step 0 of the wavefront's first chunk
+  __device__ __forceinline__ void load(u32x4_t (&to)[4], int i) const {
+#pragma unroll
+    for (int s = 0; s < 4; s++) to[s] = *reinterpret_cast<const u32x4_t*>(at + (int64_t)i * 128 + 32 * s);
   }
   template <int EPI>
   __device__ __forceinline__ void start(const StreamParams& p, const Slot& sl, int, int c0, int n, int lane) {
     const int q = lane >> 4, r16 = lane & 15;
-    upper = r16 >= 8;
-    shift = 8 * (q >> 1);
-    at = activation_row<EPI>(p, sl, r16 & 7) + (int64_t)c0 * 128 + (upper ? 16 : 0) + 4 * q;
+    mine = (r16 >> 3) == (q >> 1);
+    at = activation_row<EPI>(p, sl, r16 & 7) + (int64_t)c0 * 128 + 8 * q;
     load(even, 0);
     if (n > 1) load(odd, 1);
   }
-  // MFMA j's A operand: the lane's piece in its own block's half, zero in the other
-  __device__ __forceinline__ u32x4_t operand(const u32x2_t& piece) const {
-    u32x4_t a;  // word by word: a select between two vectors built from the same piece is compiled through memory
-    a.x = upper ? 0u : piece.x;
-    a.y = upper ? 0u : piece.y;
-    a.z = upper ? piece.x : 0u;
-    a.w = upper ? piece.y : 0u;
-    return a;
+  template <int S>
+  __device__ __forceinline__ void one(uint32_t codes, uint32_t sc, const u32x4_t& a, f32x4_t& acc) const {
+    fp4_fold(fp4_mfma(a, fp4_plain(codes), f32x4_t{0.f, 0.f, 0.f, 0.f}), fp4_scale<S>(sc), acc);
   }
-  // One tile over one block pair: the pair's code dword, the scale dword holding its two scales in bytes BYTE, BYTE + 1.
-  template <int BYTE>
-  __device__ __forceinline__ void pair(uint32_t codes, uint32_t sc, const u32x4_t& a, f32x4_t& acc) const {
-    u32x4_t b;
-    b.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, 1.0f, 0));
-    b.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, 1.0f, 1));
-    b.z = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, 1.0f, 2));
-    b.w = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(codes, 1.0f, 3));
-    const f32x4_t part = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b),
-                                                                 f32x4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-    const float s = __builtin_amdgcn_cvt_f32_fp8(sc >> shift, BYTE);  // the scale of block BYTE + q / 2 of the dword
-    acc.x = fmaf(part.x, s, acc.x);
-    acc.y = fmaf(part.y, s, acc.y);
-    acc.z = fmaf(part.z, s, acc.z);
-    acc.w = fmaf(part.w, s, acc.w);
-  }
-  __device__ __forceinline__ void tile(const u32x4_t& w, uint32_t sc_lo, uint32_t sc_hi, const u32x4_t& a0, const u32x4_t& a1, const u32x4_t& a2,
-                                       const u32x4_t& a3, f32x4_t& acc) const {
-    pair<0>(w.x, sc_lo, a0, acc);
-    pair<2>(w.y, sc_lo, a1, acc);
-    pair<0>(w.z, sc_hi, a2, acc);
-    pair<2>(w.w, sc_hi, a3, acc);
+  __device__ __forceinline__ void tile(const u32x4_t& w, uint32_t sc, const u32x4_t (&a)[4], f32x4_t& acc) const {
+    one<0>(w.x, sc, a[0], acc);
+    one<1>(w.y, sc, a[1], acc);
+    one<2>(w.z, sc, a[2], acc);
+    one<3>(w.w, sc, a[3], acc);
   }
   template <int ODD, bool MORE2, bool MORE1>
   __device__ __forceinline__ void step(const Fp4Chunk& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot&) {
-    Fp4Pieces& held = ODD ? odd : even;
-    const u32x4_t a0 = operand(held.p0), a1 = operand(held.p1), a2 = operand(held.p2), a3 = operand(held.p3);
-    tile(ch.w0, ch.s0.x, ch.s0.y, a0, a1, a2, a3, acc0);
+    u32x4_t a[4];
+#pragma unroll
+    for (int s = 0; s < 4; s++) {  // word by word: a select between two vectors is compiled through memory
+      const u32x4_t& held = ODD ? odd[s] : even[s];
+      a[s] = u32x4_t{mine ? held.x : 0u, mine ? held.y : 0u, mine ? held.z : 0u, mine ? held.w : 0u};
+    }
+    tile(ch.w0, ch.sc.x, a, acc0);
     __builtin_amdgcn_sched_barrier(0);  // a tile at a time: interleaving the four costs more registers than there are
-    tile(ch.w1, ch.s0.z, ch.s0.w, a0, a1, a2, a3, acc1);
+    tile(ch.w1, ch.sc.y, a, acc1);
     __builtin_amdgcn_sched_barrier(0);
-    tile(ch.w2, ch.s1.x, ch.s1.y, a0, a1, a2, a3, acc2);
+    tile(ch.w2, ch.sc.z, a, acc2);
     __builtin_amdgcn_sched_barrier(0);
-    tile(ch.w3, ch.s1.z, ch.s1.w, a0, a1, a2, a3, acc3);
-    if (MORE2) load(held, i + 2);
+    tile(ch.w3, ch.sc.w, a, acc3);
+    if (MORE2) {
+      if (ODD) load(odd, i + 2); else load(even, i + 2);
+    }
   }
 };
 
-__device__ __forceinline__ void add_parities(f32x4_t& acc) {
-  acc.x += __shfl_xor(acc.x, 32);
-  acc.y += __shfl_xor(acc.y, 32);
-  acc.z += __shfl_xor(acc.z, 32);
-  acc.w += __shfl_xor(acc.w, 32);
+struct Fp4Few4Acts {
+  static constexpr int LOADS = 2;
+  u32x4_t even[2], odd[2];  // the lane's piece of the pairs of steps of the next even and the next odd chunk
+  bool first, second;       // the step of a pair this lane's A row takes its block from (neither: the block's other lanes)
+  uint32_t shift;           // 8 * (q / 2)
+  const uint16_t* at;       // the lane's piece of pair 0 of the wavefront's first chunk
+  __device__ __forceinline__ void load(u32x4_t (&to)[2], int i) const {
+    to[0] = *reinterpret_cast<const u32x4_t*>(at + (int64_t)i * 128);
+    to[1] = *reinterpret_cast<const u32x4_t*>(at + (int64_t)i * 128 + 64);
+  }
+  template <int EPI>
+  __device__ __forceinline__ void start(const StreamParams& p, const Slot& sl, int, int c0, int n, int lane) {
+    const int q = lane >> 4, r16 = lane & 15, j = r16 >> 2;
+    const bool mine = (j & 1) == (q >> 1);
+    first = mine && j < 2;
+    second = mine && j >= 2;
+    shift = 8 * (q >> 1);
+    at = activation_row<EPI>(p, sl, r16 & 3) + (int64_t)c0 * 128 + 32 * (j >> 1) + 8 * q;
+    load(even, 0);
+    if (n > 1) load(odd, 1);
+  }
+  static __device__ __forceinline__ u32x4_t masked(const u32x4_t& v, bool keep) { return u32x4_t{keep ? v.x : 0u, keep ? v.y : 0u, keep ? v.z : 0u, keep ? v.w : 0u}; }
+  __device__ __forceinline__ void tile(const u32x4_t& w, uint32_t sc, const u32x4_t (&a)[4], f32x4_t& acc) const {
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    const uint32_t mine = sc >> shift;
+    fp4_fold(fp4_mfma(a[1], fp4_plain(w.y), fp4_mfma(a[0], fp4_plain(w.x), zero)), fp4_scale<0>(mine), acc);
+    fp4_fold(fp4_mfma(a[3], fp4_plain(w.w), fp4_mfma(a[2], fp4_plain(w.z), zero)), fp4_scale<2>(mine), acc);
+  }
+  template <int ODD, bool MORE2, bool MORE1>
+  __device__ __forceinline__ void step(const Fp4Chunk& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot&) {
+    u32x4_t a[4];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      a[2 * t] = masked(ODD ? odd[t] : even[t], first);
+      a[2 * t + 1] = masked(ODD ? odd[t] : even[t], second);
+    }
+    tile(ch.w0, ch.sc.x, a, acc0);
+    tile(ch.w1, ch.sc.y, a, acc1);
+    tile(ch.w2, ch.sc.z, a, acc2);
+    tile(ch.w3, ch.sc.w, a, acc3);
+    if (MORE2) {
+      if (ODD) load(odd, i + 2); else load(even, i + 2);
+    }
+  }
+};
+
+__device__ __forceinline__ void add_lanes(f32x4_t& acc, int distance) {
+  acc.x += __shfl_xor(acc.x, distance);
+  acc.y += __shfl_xor(acc.y, distance);
+  acc.z += __shfl_xor(acc.z, distance);
+  acc.w += __shfl_xor(acc.w, distance);
 }
+
+// ------------------------------------------------------------------------------------------------ slots of more rows
+//
+// MT 16-row tiles of activations against every weight, which is expanded once, its block scale multiplied in, and used MT
+// times. Lane (q, r16) feeds row 16 t + r16 of tile t, k 8 q .. + 7 of a step: a chunk's 4 x MT pieces rest in registers, and
+// each is asked for again, for the next chunk, as soon as its products are issued - straight from the L2: a wavefront
+// shares them with nobody and meets no barrier. The requests of a wavefront come back in order, so the next weights are
+// asked for BEHIND those pieces (a piece that waited behind weights from memory would wait for them too): a block is on
+// its way for the whole of the chunk before it.
+template <int MT>
+struct Fp4Wide {
+  f32x4_t acc[MT][4];
+  u32x4_t a[4][MT];
+  uint32_t at[MT];  // the lane's piece of step 0 of the wavefront's first chunk: byte offset from the matrix (the launch keeps it under 4 GiB)
+  const uint8_t* x;
+  __device__ __forceinline__ u32x4_t piece(int t, int i, int s) const { return *reinterpret_cast<const u32x4_t*>(x + (size_t)i * 256 + 64 * s + at[t]); }
+  template <int EPI>
+  __device__ __forceinline__ void start(const StreamParams& p, const Slot& sl, int c0, int lane) {
+    x = reinterpret_cast<const uint8_t*>(p.a) + (size_t)c0 * 256;
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+      at[t] = (uint32_t)(activation_row_index<EPI>(p, sl, 16 * t + (lane & 15)) * p.a_stride) * 2 + 16 * (lane >> 4);
+#pragma unroll
+      for (int nt = 0; nt < 4; nt++) acc[t][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int s = 0; s < 4; s++)
+#pragma unroll
+      for (int t = 0; t < MT; t++) a[s][t] = piece(t, 0, s);
+  }
+  template <int J>  // fragment J = 4 * step + tile of a chunk
+  static __device__ __forceinline__ bf16x8_t fragment(const Fp4Chunk& ch) { return fp4_scaled(ch.tile(J & 3)[J >> 2], fp4_scale<(J >> 2)>(ch.sc[J & 3])); }
+  // The products of fragment J, and beside them, an instruction or a few behind each product, the expansion of the next
+  // fragment: a product holds the matrix core for sixteen cycles and the issue port for about seven of them.
+  template <int J>
+  __device__ __forceinline__ void fragments(const Fp4Chunk& ch, int i, bool more, bf16x8_t b) {
+    if constexpr (J < 16) {
+      constexpr int S = J >> 2, NT = J & 3;
+      bf16x8_t next{};
+      if constexpr (J < 15) next = fragment<J + 1>(ch);
+#pragma unroll
+      for (int t = 0; t < MT; t++) acc[t][NT] = fp4_mfma(a[S][t], b, acc[t][NT]);
+#pragma unroll
+      for (int t = 0; t < MT; t++) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, (17 + MT - 1) / MT, 0);
+      }
+      if (NT == 3) {
+        u32x4_t held = __builtin_bit_cast(u32x4_t, next);
+        asm volatile("" : "+v"(held));  // expanded here, beside the products, not behind the branch
+        next = __builtin_bit_cast(bf16x8_t, held);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (NT == 3 && more) {  // uniform
+#pragma unroll
+        for (int t = 0; t < MT; t++) a[S][t] = piece(t, i + 1, S);
+      }
+      fragments<J + 1>(ch, i, more, next);
+    }
+  }
+  // One loop body for every chunk: the ring's slot by its parity, what is still to come by uniform branches.
+  template <int EPI>
+  __device__ __forceinline__ void run(const StreamParams& p, const Slot& sl, int nb, int c0, int c1, int lane, uint8_t* ring) {
+    const int n = c1 - c0;
+    RingSource src;
+    src.row = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(sl.w + (int64_t)nb * p.chunks * NVFP4_BLOCK_BYTES), 0, p.chunks * NVFP4_BLOCK_BYTES, 0x00020000);
+    const lds_ptr_t slot0 = (lds_ptr_t)ring;
+    uint32_t codes, scales;
+    Fp4Ring::lanes(src, lane, lane & 15, (uint32_t)(uintptr_t)slot0, codes, scales);
+    Fp4Ring::request(src, c0, slot0);
+    asm volatile("" ::: "memory");
+    start<EPI>(p, sl, c0, lane);
+    asm volatile("" ::: "memory");
+    if (n > 1) Fp4Ring::request(src, c0 + 1, slot0 + NVFP4_BLOCK_BYTES);
+    for (int i = 0; i < n; i++) {
+      const uint32_t slot = (i & 1) * NVFP4_BLOCK_BYTES;
+      Fp4Chunk ch;
+      if (i + 1 < n) {
+        Fp4Ring::take<4 * MT + Fp4Ring::LOADS, 0>(ch, codes + slot, scales + slot);
+      } else {
+        Fp4Ring::take<4 * MT, 0>(ch, codes + slot, scales + slot);
+      }
+      fragments<0>(ch, i, i + 1 < n, fragment<0>(ch));
+      if (i + 2 < n) Fp4Ring::request(src, c0 + i + 2, slot0 + slot);
+    }
+  }
+};
 
 // y = x Wq^T, dense or grouped by the expert plan: one wavefront per (64-row block, K range, slot of 16 activation rows),
 // the same launch shape, slot table, weight ring, K-split exchange and epilogues as the W3 stream.
@@ -325,14 +395,27 @@ __device__ __forceinline__ void nvfp4_workgroup(const StreamParams& p, int slot,
   f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0, acc2 = acc0, acc3 = acc0;
   if (active) {  // at least one chunk: the launch keeps ks <= chunks
     uint8_t* ring = rings + wave * FP4_RING_BYTES;
-    if (sl.rows <= FP4_FEW_ROWS && !p.no_few) {  // uniform over the workgroup
-      stream_block<EPI, Fp4FewActs, Fp4Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
-      add_parities(acc0);  // lanes q = 0, 1 now hold slot rows 0 .. 7 as the epilogue expects them; q = 2, 3 stand for rows past the slot's end
-      add_parities(acc1);
-      add_parities(acc2);
-      add_parities(acc3);
+    if (sl.rows <= FP4_FEWER_ROWS && !p.no_few) {  // uniform over the workgroup
+      stream_block<EPI, Fp4Few4Acts, Fp4RingOf<0>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+      for (int d = 16; d <= 32; d *= 2) {  // the four blocks' sums: lane q = 0 now holds the slot's rows as the epilogue expects them
+        add_lanes(acc0, d);
+        add_lanes(acc1, d);
+        add_lanes(acc2, d);
+        add_lanes(acc3, d);
+      }
+    } else if (sl.rows <= FP4_FEW_ROWS && !p.no_few) {
+      stream_block<EPI, Fp4Few8Acts, Fp4Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+      add_lanes(acc0, 32);  // the two parities': lanes q = 0, 1 hold slot rows 0 .. 7
+      add_lanes(acc1, 32);
+      add_lanes(acc2, 32);
+      add_lanes(acc3, 32);
     } else {
-      stream_block<EPI, Fp4Acts, Fp4Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+      Fp4Wide<1> wide;
+      wide.run<EPI>(p, sl, nb, share.c0, share.c1, lane, ring);
+      acc0 = wide.acc[0][0];
+      acc1 = wide.acc[0][1];
+      acc2 = wide.acc[0][2];
+      acc3 = wide.acc[0][3];
     }
   }
   finish_block<EPI, false, FP4_RING_BYTES / 4>(p, sl, RowScales{}, nb, active, ks, nbi, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3);
@@ -342,6 +425,31 @@ template <int EPI>
 __global__ __launch_bounds__(1024) void nvfp4_stream_kernel(StreamParams p) {
   extern __shared__ __align__(16) uint8_t rings[];
   nvfp4_workgroup<EPI>(p, blockIdx.y, blockIdx.x, rings);
+}
+
+// Dense calls of seventeen to ninety-six rows: slots of up to 16 MT rows. A workgroup's wavefronts split K and / or take
+// neighbouring blocks as the stream's do; the splits' partial tiles meet in LDS, sixteen rows at a time.
+constexpr int FP4_WIDE_TILES = 6;
+template <int EPI, int MT>
+__global__ __launch_bounds__(512, 2) void nvfp4_wide_kernel(StreamParams p) {
+  extern __shared__ __align__(16) uint8_t rings[];
+  const Slot sl = slot_of<EPI>(p, blockIdx.y);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const WaveShare share = wave_share(p, wave);
+  const int nb = blockIdx.x * p.nbw + share.nbi;
+  const bool active = nb < p.n_blocks;
+  Fp4Wide<MT> wide;
+  if (active) wide.template run<EPI>(p, sl, nb, share.c0, share.c1, lane, rings + wave * FP4_RING_BYTES);
+#pragma unroll
+  for (int t = 0; t < MT; t++) {
+    Slot part = sl;
+    part.p0 += 16 * t;
+    part.rows = min(16, sl.rows - 16 * t);
+    if (t && p.ks > 1) __syncthreads();  // the exchange areas have been read
+    __builtin_amdgcn_sched_barrier(0);
+    finish_block<EPI, false, FP4_RING_BYTES / 4>(p, part, RowScales{}, nb, active, share.ks, share.nbi, reinterpret_cast<float*>(rings), wide.acc[t][0],
+                                                 wide.acc[t][1], wide.acc[t][2], wide.acc[t][3]);
+  }
 }
 
 // Two matrices of different geometry in one launch (the routed experts' layer beside the shared expert's, which reads
@@ -386,6 +494,35 @@ static int launch_nvfp4(StreamParams& p, int64_t slots, int64_t busy_slots, hipS
   return HB_OK;
 }
 
+// The wide kernel: slots of 16 MT rows, MT the fewest tiles that hold the call's rows in as few slots as can be.
+static bool wide_serves(int m) { return m > ROWS_PER_SLOT && m <= 16 * FP4_WIDE_TILES; }
+template <int EPI>
+static int launch_wide(StreamParams& p, hipStream_t stream) {
+  const int mt = (p.m + 15) / 16;
+  p.ks = 4;
+  p.nbw = 1;
+  if (g_nvfp4_ksplit) {
+    p.ks = g_nvfp4_ksplit;
+    p.nbw = g_nvfp4_nbw ? g_nvfp4_nbw.load() : 1;
+  }
+  while (p.ks > p.chunks) p.ks /= 2;
+  if (p.ks * p.nbw > 8) return HB_EINVAL;
+  set_split(p);
+  p.slot_rows = 16 * mt;
+  const dim3 grid((unsigned)((p.n_blocks + p.nbw - 1) / p.nbw), 1);
+  const int waves = p.ks * p.nbw;
+  auto launch = [&](auto kernel) { HB_LAUNCH(kernel, grid, dim3(64 * waves), (size_t)waves * FP4_RING_BYTES, stream, p); };
+  switch (mt) {
+    case 2: launch(nvfp4_wide_kernel<EPI, 2>); break;
+    case 3: launch(nvfp4_wide_kernel<EPI, 3>); break;
+    case 4: launch(nvfp4_wide_kernel<EPI, 4>); break;
+    case 5: launch(nvfp4_wide_kernel<EPI, 5>); break;
+    case 6: launch(nvfp4_wide_kernel<EPI, 6>); break;
+    default: return HB_EINVAL;
+  }
+  return HB_OK;
+}
+
 // `a` over its plan's slots beside the dense `b` in one launch (nvfp4_twin_kernel).
 template <int EPI_A, int EPI_B>
 static int launch_twin(StreamParams& a, int64_t slots_a, int64_t busy_a, StreamParams& b, int64_t slots_b, hipStream_t stream) {
@@ -406,40 +543,14 @@ static int launch_twin(StreamParams& a, int64_t slots_a, int64_t busy_a, StreamP
 }
 
 // ------------------------------------------------------------------------------ the prefill kernel's NVFP4 format
-__device__ __forceinline__ uint32_t scaled_pair(uint32_t codes, int byte, float scale) {
-  typedef __attribute__((ext_vector_type(2))) float f32x2_t;
-  f32x2_t w;
-  switch (byte) {  // the byte selector is an immediate of the instruction
-    case 0: w = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(codes, 1.0f, 0); break;
-    case 1: w = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(codes, 1.0f, 1); break;
-    case 2: w = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(codes, 1.0f, 2); break;
-    default: w = __builtin_amdgcn_cvt_scalef32_pk_f32_fp4(codes, 1.0f, 3); break;
-  }
-  typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_v;
-  const bf16x2_v packed = {(__bf16)(w.x * scale), (__bf16)(w.y * scale)};
-  return __builtin_bit_cast(uint32_t, packed);
-}
-
 struct TileNvfp4 {
   typedef Fp4Chunk Chunk;
   static constexpr int BLOCK_BYTES = NVFP4_BLOCK_BYTES;
-  static constexpr bool SPLIT_A = true, PER_ROW = false;
-  static __device__ __forceinline__ void load(Chunk& ch, const uint8_t* blk, int lane, int r16) { load_fp4_chunk(ch, blk, lane, r16); }
-  // k-step s = blocks 2 s, 2 s + 1: dword s of the tile's codes (low half the even block), scale bytes 2 s, 2 s + 1 of
-  // the tile's eight
+  static constexpr bool PER_ROW = false;
+  static __device__ __forceinline__ void load(Chunk& ch, const uint8_t* blk, int lane, int) { load_fp4_chunk(ch, blk, lane); }
   static __device__ __forceinline__ bf16x8_t fragment(const Chunk& ch, int nt, int s, const Slot&) {
-    const u32x4_t w = nt == 0 ? ch.w0 : nt == 1 ? ch.w1 : nt == 2 ? ch.w2 : ch.w3;
-    const u32x4_t sc4 = nt < 2 ? ch.s0 : ch.s1;
-    const uint32_t sd = (nt & 1) ? (s < 2 ? sc4.z : sc4.w) : (s < 2 ? sc4.x : sc4.y);
-    const float s_even = (s & 1) ? __builtin_amdgcn_cvt_f32_fp8(sd, 2) : __builtin_amdgcn_cvt_f32_fp8(sd, 0);
-    const float s_odd = (s & 1) ? __builtin_amdgcn_cvt_f32_fp8(sd, 3) : __builtin_amdgcn_cvt_f32_fp8(sd, 1);
-    const uint32_t codes = w[s];
-    u32x4_t packed;
-    packed.x = scaled_pair(codes, 0, s_even);
-    packed.y = scaled_pair(codes, 1, s_even);
-    packed.z = scaled_pair(codes, 2, s_odd);
-    packed.w = scaled_pair(codes, 3, s_odd);
-    return __builtin_bit_cast(bf16x8_t, packed);
+    const uint32_t sc = ch.sc[nt];
+    return fp4_scaled(ch.tile(nt)[s], s == 0 ? fp4_scale<0>(sc) : s == 1 ? fp4_scale<1>(sc) : s == 2 ? fp4_scale<2>(sc) : fp4_scale<3>(sc));
   }
 };
 
@@ -497,6 +608,10 @@ static int nvfp4_gemm(const void* x, int m, const void* tiled, float global_scal
   if (m <= 0 || n <= 0 || k <= 0 || n % 64 || k % 128) return HB_EINVAL;
   if (!aligned(x, 16) || !aligned(tiled, 16) || !aligned(y, 2) || !aligned(workspace, 16)) return HB_EINVAL;
   StreamParams p = dense_params(tiled, global_scale, n, k, x, m, y);
+  if (wide_serves(m) && tile_takes(m, k) && g_nvfp4_tile == 0 && !g_nvfp4_tile_ks) {
+    if (int e = relu2 ? launch_wide<EPI_DENSE_RELU2>(p, stream) : launch_wide<EPI_DENSE>(p, stream)) return e;
+    return launch_status();
+  }
   // between the weight stream's sixteen rows a pass and a call that fills the device with 128-row tiles: tiles whose K
   // is shared among workgroups
   int ks = workspace && m > TILE_SPLIT_ROWS ? tile_split(m, p.n_blocks, p.chunks) : 1;

@@ -11,9 +11,7 @@
 //     accumulators for 8 x 4 tiles in registers; the FP32 matrix / row scale is applied in the epilogue.
 //
 // A format provides: Chunk (the registers of one 64-row x 128-k block), BLOCK_BYTES, load(), fragment() (the scaled B
-// operand of 16-row tile nt and 32-k step s), SPLIT_A (how the lane's eight k of a step lie: NVFP4's tile layout gives
-// lane q the k 4q..4q+3 of both 16-blocks of the step, so its A fragment is two 8-byte reads; W3's gives it 8q..8q+7),
-// and PER_ROW (FP32 scale per output row, else one per matrix).
+// operand of 16-row tile nt and 32-k step s: lane (q, r) the eight k 8q..8q+7 of row r) and PER_ROW (FP32 scale per output row, else one per matrix).
 #pragma once
 
 #include <algorithm>
@@ -25,11 +23,7 @@ namespace hb {
 
 constexpr int TILE_ROWS = 128;
 constexpr int TILE_MT = TILE_ROWS / 16;
-// A 16-row tile of an activation buffer is 4 KB and 16 bytes of padding: with the tiles a multiple of 512 bytes apart
-// the compiler pairs the 8-byte reads of neighbouring tiles into one instruction and then moves registers to put a
-// fragment's two halves side by side (a quarter of the loop's VALU instructions); off that grid every half is its own
-// read, straight into its place.
-constexpr int TILE_PITCH = 16 * 256 + 16;
+constexpr int TILE_PITCH = 16 * 256;            // bytes of a 16-row tile of an activation buffer
 constexpr int TILE_BUF = TILE_MT * TILE_PITCH;  // bytes of one activation buffer
 constexpr int TILE_DENSE_ROWS = 24;        // average rows an expert from which the tile kernel serves a routed call
 typedef __attribute__((ext_vector_type(2))) uint32_t tile_u32x2_t;
@@ -109,21 +103,12 @@ __device__ __forceinline__ void tile_slot(const StreamParams& p, const Slot& sl,
 #pragma unroll
       for (int nt = 0; nt < 4; nt++) b[nt] = Fmt::fragment(w, nt, s, sl);
       // lane (q, r16) of tile t: row 16 t + r16; its eight k of the step as the format's tile layout owns them
-      const int half = (q & 1) << 3;
-      const int slot_lo = ((4 * s + (q >> 1)) ^ r16) << 4, slot_hi = ((4 * s + 2 + (q >> 1)) ^ r16) << 4;
       const int slot_one = ((4 * s + q) ^ r16) << 4;
 #pragma unroll
       for (int t = 0; t < MT; t++) {
         if (FULL || t < tiles) {
           const uint8_t* row = buf + t * TILE_PITCH + r16 * 256;
-          u32x4_t a;
-          if (Fmt::SPLIT_A) {
-            const tile_u32x2_t lo = *reinterpret_cast<const tile_u32x2_t*>(row + half + slot_lo);
-            const tile_u32x2_t hi = *reinterpret_cast<const tile_u32x2_t*>(row + half + slot_hi);
-            a = u32x4_t{lo.x, lo.y, hi.x, hi.y};
-          } else {
-            a = *reinterpret_cast<const u32x4_t*>(row + slot_one);
-          }
+          const u32x4_t a = *reinterpret_cast<const u32x4_t*>(row + slot_one);
           const bf16x8_t af = __builtin_bit_cast(bf16x8_t, a);
 #pragma unroll
           for (int nt = 0; nt < 4; nt++) acc[t][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[nt], af, acc[t][nt], 0, 0, 0);

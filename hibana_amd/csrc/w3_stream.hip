@@ -945,7 +945,7 @@ __global__ __launch_bounds__(1024) void w3_fc2_combine_one_kernel(StreamParams p
 struct TileW3 {
   typedef hb::Chunk Chunk;
   static constexpr int BLOCK_BYTES = W3_BLOCK_BYTES;
-  static constexpr bool SPLIT_A = false, PER_ROW = true;
+  static constexpr bool PER_ROW = true;
   static __device__ __forceinline__ void load(Chunk& ch, const uint8_t* blk, int lane, int r16) { load_chunk(ch, blk, lane, r16); }
   // The B operand of 16-row tile nt, 32-group s, scaled by the group's E4M3 scale (a 4-bit level times a 4-bit scale:
   // exact in BF16); the FP32 row scale stays in the epilogue.

@@ -13,6 +13,7 @@
 
 #include <atomic>
 
+#include "panel_kernel.hpp"
 #include "ring.hpp"
 #include "stream_common.hpp"
 #include "tile_kernel.hpp"
@@ -154,6 +155,21 @@ struct Fp4RingOf {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(src.row, slot + NVFP4_SCALE_OFFSET, 4, src.scales, at + NVFP4_SCALE_OFFSET, 0, 2);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(src.row, slot + NVFP4_SCALE_OFFSET, 4, src.scales, at + NVFP4_SCALE_OFFSET, 256, 2);
     __builtin_amdgcn_sched_barrier(0);  // asked for here, not wherever the scheduler would sink it below the arithmetic
+  }
+  // the reads of a block from slot 0, and (after a wait) their values
+  static __device__ __forceinline__ void ask(Chunk& ch, uint32_t codes, uint32_t scales) {
+    ask_lds<0>(ch.w0, codes);
+    ask_lds<1024>(ch.w1, codes);
+    ask_lds<2048>(ch.w2, codes);
+    ask_lds<3072>(ch.w3, codes);
+    ask_lds<NVFP4_SCALE_OFFSET>(ch.sc, scales);
+  }
+  static __device__ __forceinline__ void have(Chunk& ch) {
+    pin(ch.w0);
+    pin(ch.w1);
+    pin(ch.w2);
+    pin(ch.w3);
+    pin(ch.sc);
   }
   template <int BEHIND, int SLOT>
   static __device__ __forceinline__ void take(Chunk& ch, uint32_t codes, uint32_t scales) {
@@ -427,31 +443,6 @@ __global__ __launch_bounds__(1024) void nvfp4_stream_kernel(StreamParams p) {
   nvfp4_workgroup<EPI>(p, blockIdx.y, blockIdx.x, rings);
 }
 
-// Dense calls of seventeen to ninety-six rows: slots of up to 16 MT rows. A workgroup's wavefronts split K and / or take
-// neighbouring blocks as the stream's do; the splits' partial tiles meet in LDS, sixteen rows at a time.
-constexpr int FP4_WIDE_TILES = 6;
-template <int EPI, int MT>
-__global__ __launch_bounds__(512, 2) void nvfp4_wide_kernel(StreamParams p) {
-  extern __shared__ __align__(16) uint8_t rings[];
-  const Slot sl = slot_of<EPI>(p, blockIdx.y);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const WaveShare share = wave_share(p, wave);
-  const int nb = blockIdx.x * p.nbw + share.nbi;
-  const bool active = nb < p.n_blocks;
-  Fp4Wide<MT> wide;
-  if (active) wide.template run<EPI>(p, sl, nb, share.c0, share.c1, lane, rings + wave * FP4_RING_BYTES);
-#pragma unroll
-  for (int t = 0; t < MT; t++) {
-    Slot part = sl;
-    part.p0 += 16 * t;
-    part.rows = min(16, sl.rows - 16 * t);
-    if (t && p.ks > 1) __syncthreads();  // the exchange areas have been read
-    __builtin_amdgcn_sched_barrier(0);
-    finish_block<EPI, false, FP4_RING_BYTES / 4>(p, part, RowScales{}, nb, active, share.ks, share.nbi, reinterpret_cast<float*>(rings), wide.acc[t][0],
-                                                 wide.acc[t][1], wide.acc[t][2], wide.acc[t][3]);
-  }
-}
-
 // Two matrices of different geometry in one launch (the routed experts' layer beside the shared expert's, which reads
 // other activations): the first `first` workgroups are (slot, block group) of the dense `b`, slot-major - every one of
 // them has a whole K range to stream, so they start first - the rest of the planned `a`. Should the two shapes differ
@@ -494,35 +485,6 @@ static int launch_nvfp4(StreamParams& p, int64_t slots, int64_t busy_slots, hipS
   return HB_OK;
 }
 
-// The wide kernel: slots of 16 MT rows, MT the fewest tiles that hold the call's rows in as few slots as can be.
-static bool wide_serves(int m) { return m > ROWS_PER_SLOT && m <= 16 * FP4_WIDE_TILES; }
-template <int EPI>
-static int launch_wide(StreamParams& p, hipStream_t stream) {
-  const int mt = (p.m + 15) / 16;
-  p.ks = 4;
-  p.nbw = 1;
-  if (g_nvfp4_ksplit) {
-    p.ks = g_nvfp4_ksplit;
-    p.nbw = g_nvfp4_nbw ? g_nvfp4_nbw.load() : 1;
-  }
-  while (p.ks > p.chunks) p.ks /= 2;
-  if (p.ks * p.nbw > 8) return HB_EINVAL;
-  set_split(p);
-  p.slot_rows = 16 * mt;
-  const dim3 grid((unsigned)((p.n_blocks + p.nbw - 1) / p.nbw), 1);
-  const int waves = p.ks * p.nbw;
-  auto launch = [&](auto kernel) { HB_LAUNCH(kernel, grid, dim3(64 * waves), (size_t)waves * FP4_RING_BYTES, stream, p); };
-  switch (mt) {
-    case 2: launch(nvfp4_wide_kernel<EPI, 2>); break;
-    case 3: launch(nvfp4_wide_kernel<EPI, 3>); break;
-    case 4: launch(nvfp4_wide_kernel<EPI, 4>); break;
-    case 5: launch(nvfp4_wide_kernel<EPI, 5>); break;
-    case 6: launch(nvfp4_wide_kernel<EPI, 6>); break;
-    default: return HB_EINVAL;
-  }
-  return HB_OK;
-}
-
 // `a` over its plan's slots beside the dense `b` in one launch (nvfp4_twin_kernel).
 template <int EPI_A, int EPI_B>
 static int launch_twin(StreamParams& a, int64_t slots_a, int64_t busy_a, StreamParams& b, int64_t slots_b, hipStream_t stream) {
@@ -545,6 +507,31 @@ static int launch_twin(StreamParams& a, int64_t slots_a, int64_t busy_a, StreamP
 // ------------------------------------------------------------------------------ the prefill kernel's NVFP4 format
 struct TileNvfp4 {
   typedef Fp4Chunk Chunk;
+  typedef Fp4Ring Ring;
+  struct Part {  // a fragment being expanded: its eight codes and their block's scale
+    uint32_t codes;
+    float scale;
+  };
+  template <int NT, int S>
+  static __device__ __forceinline__ Part open(const Chunk& ch, const Slot&) {
+    return Part{ch.tile(NT)[S], fp4_scale<S>(ch.sc[NT])};
+  }
+#define HB_FP4_CVT "v_cvt_scalef32_pk_f32_fp4"
+  template <int K, bool AFTER_VALU>  // a product, then values 2 K, 2 K + 1 of the part
+  static __device__ __forceinline__ void product_pair(f32x4_t& acc, const u32x4_t& w, const u32x4_t& a, const Part& part, uint32_t& out) {
+    if constexpr (K == 0 && AFTER_VALU) HB_PANEL_PRODUCT_PAIR("s_nop 1\n\t", HB_FP4_CVT, "", acc, out, w, part.codes, part.scale, a);
+    if constexpr (K == 0 && !AFTER_VALU) HB_PANEL_PRODUCT_PAIR("", HB_FP4_CVT, "", acc, out, w, part.codes, part.scale, a);
+    if constexpr (K == 1) HB_PANEL_PRODUCT_PAIR("", HB_FP4_CVT, " op_sel:[1,0,0]", acc, out, w, part.codes, part.scale, a);
+    if constexpr (K == 2) HB_PANEL_PRODUCT_PAIR("", HB_FP4_CVT, " op_sel:[0,1,0]", acc, out, w, part.codes, part.scale, a);
+    if constexpr (K == 3) HB_PANEL_PRODUCT_PAIR("", HB_FP4_CVT, " op_sel:[1,1,0]", acc, out, w, part.codes, part.scale, a);
+  }
+  template <int K>
+  static __device__ __forceinline__ void pair_alone(const Part& part, uint32_t& out) {
+    if constexpr (K == 0) HB_PANEL_PAIR_ALONE(HB_FP4_CVT, "", out, part.codes, part.scale);
+    if constexpr (K == 1) HB_PANEL_PAIR_ALONE(HB_FP4_CVT, " op_sel:[1,0,0]", out, part.codes, part.scale);
+    if constexpr (K == 2) HB_PANEL_PAIR_ALONE(HB_FP4_CVT, " op_sel:[0,1,0]", out, part.codes, part.scale);
+    if constexpr (K == 3) HB_PANEL_PAIR_ALONE(HB_FP4_CVT, " op_sel:[1,1,0]", out, part.codes, part.scale);
+  }
   static constexpr int BLOCK_BYTES = NVFP4_BLOCK_BYTES;
   static constexpr bool PER_ROW = false;
   static __device__ __forceinline__ void load(Chunk& ch, const uint8_t* blk, int lane, int) { load_fp4_chunk(ch, blk, lane); }
@@ -553,6 +540,45 @@ struct TileNvfp4 {
     return fp4_scaled(ch.tile(nt)[s], s == 0 ? fp4_scale<0>(sc) : s == 1 ? fp4_scale<1>(sc) : s == 2 ? fp4_scale<2>(sc) : fp4_scale<3>(sc));
   }
 };
+
+template <int EPI>
+static int launch_panel(StreamParams& p, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  PanelPlan q = plan_panel<TileNvfp4>(p.m, p.n_blocks, p.chunks, workspace ? workspace_bytes : 0);
+  if (g_nvfp4_ksplit) {
+    q.ks = g_nvfp4_ksplit;
+    q.nbw = g_nvfp4_nbw ? g_nvfp4_nbw.load() : 1;
+    q.mt = ((p.m + (p.m + 127) / 128 - 1) / ((p.m + 127) / 128) + 15) / 16;
+    q.groups = (p.n_blocks + q.nbw - 1) / q.nbw;
+    q.tiles = q.full = (int64_t)q.groups * ((p.m + 16 * q.mt - 1) / (16 * q.mt));
+    q.kz = 1;
+    if (g_nvfp4_tile_ks > 1) q.kz = g_nvfp4_tile_ks, q.full = 0;
+  }
+  const size_t lds = panel_lds_bytes<TileNvfp4>(q.mt, q.ks, q.nbw);
+  const int64_t grid = q.full + (q.tiles - q.full) * q.kz;
+  if (q.us > 1e29 || q.ks * q.nbw > PANEL_WAVES || q.ks > p.chunks / q.kz || (q.ks & (q.ks - 1)) || q.nbw < panel_least_blocks(q.mt) || lds > PANEL_LDS || grid > 0x7fffffff || panel_room(q) > workspace_bytes) return HB_EINVAL;
+  p.ks = q.ks;
+  p.nbw = q.nbw;
+  set_split(p);
+  p.slot_rows = 16 * q.mt;
+  p.a_bytes = (uint32_t)((int64_t)p.m * p.a_stride * 2);
+  p.panel_groups = q.groups;
+  p.panel_full = (int)q.full;
+  p.panel_kz = q.kz;
+  p.tile_tickets = static_cast<uint32_t*>(workspace) + PLAN_HEADER;
+  p.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + PANEL_TICKET_BYTES);
+  auto launch = [&](auto kernel) { HB_LAUNCH(kernel, dim3((unsigned)grid), dim3(64 * q.ks * q.nbw), lds, stream, p); };
+  switch (q.mt) {
+    case 1: launch(panel_kernel<TileNvfp4, EPI, 1>); break;
+    case 2: launch(panel_kernel<TileNvfp4, EPI, 2>); break;
+    case 3: launch(panel_kernel<TileNvfp4, EPI, 3>); break;
+    case 4: launch(panel_kernel<TileNvfp4, EPI, 4>); break;
+    case 5: launch(panel_kernel<TileNvfp4, EPI, 5>); break;
+    case 6: launch(panel_kernel<TileNvfp4, EPI, 6>); break;
+    case 7: launch(panel_kernel<TileNvfp4, EPI, 7>); break;
+    default: launch(panel_kernel<TileNvfp4, EPI, 8>); break;
+  }
+  return HB_OK;
+}
 
 static inline unsigned grid_for(int64_t threads) { return (unsigned)((threads + 255) / 256); }
 
@@ -608,8 +634,8 @@ static int nvfp4_gemm(const void* x, int m, const void* tiled, float global_scal
   if (m <= 0 || n <= 0 || k <= 0 || n % 64 || k % 128) return HB_EINVAL;
   if (!aligned(x, 16) || !aligned(tiled, 16) || !aligned(y, 2) || !aligned(workspace, 16)) return HB_EINVAL;
   StreamParams p = dense_params(tiled, global_scale, n, k, x, m, y);
-  if (wide_serves(m) && tile_takes(m, k) && g_nvfp4_tile == 0 && !g_nvfp4_tile_ks) {
-    if (int e = relu2 ? launch_wide<EPI_DENSE_RELU2>(p, stream) : launch_wide<EPI_DENSE>(p, stream)) return e;
+  if (m > ROWS_PER_SLOT && tile_takes(m, k) && tile_writes(y, false) && g_nvfp4_tile == 0 && (g_nvfp4_ksplit || !g_nvfp4_tile_ks)) {
+    if (int e = relu2 ? launch_panel<EPI_DENSE_RELU2>(p, workspace, workspace_bytes, stream) : launch_panel<EPI_DENSE>(p, workspace, workspace_bytes, stream)) return e;
     return launch_status();
   }
   // between the weight stream's sixteen rows a pass and a call that fills the device with 128-row tiles: tiles whose K
@@ -642,6 +668,11 @@ extern "C" size_t hb_nvfp4_gemm_workspace_bytes(int m, int n, int k) {
   if (m <= TILE_SPLIT_ROWS || n <= 0 || k <= 0 || n % 64 || k % 128) return 0;
   const int want = g_nvfp4_tile_ks ? std::min(g_nvfp4_tile_ks.load(), k / 128) : tile_split(m, n / 64, k / 128);
   return tile_partial_bytes(m, n / 64, want);
+}
+
+extern "C" size_t hb_nvfp4_gemm_room_bytes(int m, int n, int k) {
+  if (m <= ROWS_PER_SLOT || n <= 0 || k <= 0 || n % 64 || k % 128) return 0;
+  return panel_room(plan_panel<TileNvfp4>(m, n / 64, k / 128, ~(size_t)0));
 }
 
 extern "C" int hb_nvfp4_gemm_ws(const void* x, int m, const void* tiled, float global_scale, int n, int k, int relu2, void* y, void* workspace,
@@ -714,8 +745,8 @@ int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, i
   StreamParams p, f2;
   expert_params(ex, x, m, topk, ws, out_pairs, pairs_bf16, p, f2);
   if (dense) {
-    if (int e = ex->gated ? launch_tile<TileNvfp4, EPI_FC1_GATED>(p, slots, m, stream) : launch_tile<TileNvfp4, EPI_FC1_RELU2>(p, slots, m, stream)) return e;
-    if (int e = launch_tile<TileNvfp4, EPI_FC2>(f2, slots, pairs, stream)) return e;
+    if (int e = ex->gated ? launch_panel_routed<TileNvfp4, EPI_FC1_GATED>(p, slots, m, stream) : launch_panel_routed<TileNvfp4, EPI_FC1_RELU2>(p, slots, m, stream)) return e;
+    if (int e = launch_panel_routed<TileNvfp4, EPI_FC2>(f2, slots, pairs, stream)) return e;
     return launch_status();
   }
   if (int e = ex->gated ? launch_nvfp4<EPI_FC1_GATED>(p, slots, est, stream) : launch_nvfp4<EPI_FC1_RELU2>(p, slots, est, stream)) return e;

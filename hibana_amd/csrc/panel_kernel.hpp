@@ -1,0 +1,517 @@
+// Dense contractions against packed weights on the matrix cores, shared by the weight formats: a slot of up to 128
+// activation rows against `nbw` neighbouring 64-row weight blocks, K split `ks` ways among the wavefronts of ONE workgroup.
+//
+// A wavefront owns a 64-row block over its split of K and 16 MT activation rows: MT x 4 accumulator tiles. It expands each
+// weight once, in registers (Fmt::fragment: scaled BF16, exact), and uses it for MT products. The activations of a
+// half chunk (64 k) lie in LDS, one copy a split, shared by the split's nbw wavefronts: brought by LDS-direct loads as 1 KB
+// pieces of eight rows x 128 contiguous bytes (reading fragments straight from the L2 instead, sixteen rows x 64 bytes a load,
+// runs at 11 B/clk a compute unit: 65 us against PANEL77 at 77 rows, 25600 x 5120), two buffers, a barrier a half chunk. The
+// weights of the next chunk wait in a slot of LDS of the wavefront's own.
+//
+// What bounds it is the issue port and the matrix core together: a product holds the core for 16 cycles and the port for
+// about 7, a vector instruction the port for 4.6, and a fragment (eight weights a lane) costs 17 (NVFP4) to 24 (W3) of them.
+// So the expansion of the NEXT fragment stands between the products of this one, an instruction or a few behind each
+// (two wavefronts a SIMD with two vector instructions a product run at the matrix core's full rate; the same work in
+// phases at 88 % of it). A fragment of activations is asked for again, for the next 32-k step, as soon as its last product
+// is issued (one set of registers), and the barrier of a half chunk stands after the first quarter of that half's LAST
+// step, when its fragments are in registers anyway: the next half's first ones are asked for beside the rest of it.
+#pragma once
+
+#include "ring.hpp"
+#include "stream_common.hpp"
+
+namespace hb {
+
+constexpr int PANEL_HALF = 64;       // k of a half chunk
+constexpr int PANEL_WAVES = 8;       // at most, a workgroup
+constexpr int PANEL_LDS = 160 * 1024;
+
+// The fewest blocks of a workgroup whose splits' activations fit the LDS beside the weights (PANEL_WAVES wavefronts).
+constexpr int panel_least_blocks(int mt) { return mt <= 4 ? 1 : mt <= 6 ? 2 : 4; }
+
+// A workgroup's part of the launch: its run of blocks, and where several workgroups share a tile's K (kz > 1), which
+// share is its own and the tile's number among those.
+struct PanelShare {
+  int group, z, kz, shared_tile;
+};
+// A wavefront's: its block of the run, its split and the chunks c0 .. c0 + chunks - 1 of it, and the most chunks a split of
+// the workgroup has.
+struct PanelWave {
+  int ks, nbi, c0, chunks, most;
+};
+__device__ __forceinline__ PanelWave panel_wave(const StreamParams& p, const PanelShare& part, int wave) {
+  PanelWave w;
+  w.nbi = (wave * p.ks_inv) >> 16;
+  w.ks = wave - w.nbi * p.ks;
+  const int z0 = part.kz > 1 ? part.z * p.chunks / part.kz : 0, z1 = part.kz > 1 ? (part.z + 1) * p.chunks / part.kz : p.chunks;
+  const int base = ((z1 - z0) * p.ks_inv) >> 16, rem = z1 - z0 - base * p.ks;  // p.ks is a power of two: ks_inv is exact
+  w.c0 = z0 + w.ks * base + min(w.ks, rem);
+  w.chunks = base + (w.ks < rem ? 1 : 0);
+  w.most = base + (rem ? 1 : 0);
+  return w;
+}
+
+// Sixteen bytes a lane past the caches. The wait state behind the store is its own: a vector instruction right after it may
+// overwrite the data registers before the last lanes are read, and the compiler, which guards its own stores, does not know
+// this statement for one.
+__device__ __forceinline__ void store_through16(f32x4_t* at, const f32x4_t& v) { asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(at), "v"(v) : "memory"); }
+template <int N>
+__device__ __forceinline__ void wait_vm(void) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+__device__ __forceinline__ void wait_lds(void) { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
+template <class T>
+__device__ __forceinline__ void pin(T& v) { asm volatile("" : "+v"(v)); }
+template <int OFFSET>
+__device__ __forceinline__ void ask_lds(u32x4_t& v, uint32_t at) { asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(v) : "v"(at), "n"(OFFSET) : "memory"); }
+
+// acc += w a^T, in place (the builtin lets the compiler move an accumulator to other registers at every product, a third
+// more of them in all). The statement hides a matrix instruction from the compiler's wait-state bookkeeping: AFTER_VALU
+// stands where the operand w may have been written by the vector instruction before it (two wait states), and products_done
+// between the last product and the first other use of an accumulator.
+template <bool AFTER_VALU>
+__device__ __forceinline__ void product(f32x4_t& acc, const u32x4_t& w, const u32x4_t& a) {
+  if constexpr (AFTER_VALU) {
+    asm volatile("s_nop 1\n\tv_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(w), "v"(a));
+  } else {
+    asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc) : "v"(w), "v"(a));
+  }
+}
+// ... and behind it the expansion of one pair of weights: convert (two values of the packed dword `from`), times the scale,
+// rounded (exactly) into a BF16 pair. One statement, because the compiler guards the seams between its own instructions and
+// ours with a wait state each; the two FP32 values live in v64, v65, which a statement cannot name otherwise.
+#define HB_PANEL_PAIR(CONVERT, SELECT) CONVERT " v[64:65], %3, 1.0" SELECT "\n\tv_mul_f32 v64, v64, %4\n\tv_mul_f32 v65, v65, %4\n\tv_cvt_pk_bf16_f32 %1, v64, v65"
+#define HB_PANEL_PRODUCT_PAIR(NOP, CONVERT, SELECT, acc, out, w, from, scale, a)                                                          \
+  asm volatile(NOP "v_mfma_f32_16x16x32_bf16 %0, %2, %5, %0\n\t" HB_PANEL_PAIR(CONVERT, SELECT)                                           \
+               : "+v"(acc), "=&v"(out)                                                                                                   \
+               : "v"(w), "v"(from), "v"(scale), "v"(a)                                                                                   \
+               : "v64", "v65")
+#define HB_PANEL_PAIR_ALONE(CONVERT, SELECT, out, from, scale) \
+  asm volatile(CONVERT " v[64:65], %1, 1.0" SELECT "\n\tv_mul_f32 v64, v64, %2\n\tv_mul_f32 v65, v65, %2\n\tv_cvt_pk_bf16_f32 %0, v64, v65" : "=&v"(out) : "v"(from), "v"(scale) : "v64", "v65")
+__device__ __forceinline__ void products_done(void) { asm volatile("s_nop 15\n\ts_nop 7" ::: "memory"); }
+
+template <class Fmt, int EPI, int MT>
+struct Panel {
+  typedef typename Fmt::Ring Ring;
+  typedef typename Fmt::Chunk Chunk;
+  static constexpr int BUF = MT * 16 * PANEL_HALF * 2;  // bytes of one split's half chunk of activations
+  static constexpr int PIECES = MT * 2;                 // its 1 KB pieces ...
+  static constexpr int HELD = (PIECES + panel_least_blocks(MT) - 1) / panel_least_blocks(MT);  // ... those a wavefront brings at most
+
+  f32x4_t acc[MT][4];
+  u32x4_t now[MT];  // the activations' fragments of the step in hand
+
+  // The products of fragment J = 4 * step + tile of a chunk, and between them the expansion of fragment J + 1, a pair of
+  // its values behind every MT / 4 products. The empty statements hold that order: left to itself the compiler puts the
+  // expansion behind the products (fewer registers), where nothing runs beside it.
+  // FRESH: the activations' fragments may still be on their way (asked for in order, nothing behind them). NEXT >= 0: the
+  // LDS offset of the next step's, from `at`.
+  template <int J, bool FRESH, int NEXT>
+  __device__ __forceinline__ bf16x8_t group(const Chunk& ch, const Slot& sl, bf16x8_t b, uint32_t at) {
+    u32x4_t w = __builtin_bit_cast(u32x4_t, b);
+    typename Fmt::Part part;
+    uint32_t out[4] = {0u, 0u, 0u, 0u};
+    products<J, FRESH, NEXT, 0>(ch, sl, w, at, part, out);
+    return __builtin_bit_cast(bf16x8_t, u32x4_t{out[0], out[1], out[2], out[3]});
+  }
+  template <int J, bool FRESH, int NEXT, int T>
+  __device__ __forceinline__ void products(const Chunk& ch, const Slot& sl, u32x4_t& w, uint32_t at, typename Fmt::Part& part, uint32_t (&out)[4]) {
+    constexpr int NT = J & 3;
+    if constexpr (T < MT) {
+      if constexpr (FRESH) {
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(MT - 1 - T) : "memory");
+        pin(now[T]);
+      }
+      constexpr int K = (4 * T + MT - 1) / MT;  // the pairs are dealt out evenly: pair K goes behind product K MT / 4
+      constexpr bool FIRST = J < 15 && K < 4 && K * MT / 4 == T;
+      if constexpr (J < 15 && T == 0) part = Fmt::template open<((J + 1) & 3), ((J + 1) >> 2)>(ch, sl);
+      if constexpr (FIRST) {
+        Fmt::template product_pair<K, T == 0>(acc[T][NT], w, now[T], part, out[K]);
+      } else {
+        product<T == 0>(acc[T][NT], w, now[T]);
+      }
+      if constexpr (FIRST && K + 1 < 4 && (K + 1) * MT / 4 == T) Fmt::template pair_alone<(K + 1) & 3>(part, out[(K + 1) & 3]);
+      if constexpr (FIRST && MT == 1) {
+        Fmt::template pair_alone<2>(part, out[2]);
+        Fmt::template pair_alone<3>(part, out[3]);
+      }
+      if constexpr (NEXT >= 0) ask_lds<NEXT + T * 2048>(now[T], at);
+      products<J, FRESH, NEXT, T + 1>(ch, sl, w, at, part, out);
+    }
+  }
+  static __device__ __forceinline__ bf16x8_t whole(const Chunk& ch, const Slot& sl) {  // fragment 0 of a chunk
+    typename Fmt::Part part = Fmt::template open<0, 0>(ch, sl);
+    uint32_t out[4];
+    Fmt::template pair_alone<0>(part, out[0]);
+    Fmt::template pair_alone<1>(part, out[1]);
+    Fmt::template pair_alone<2>(part, out[2]);
+    Fmt::template pair_alone<3>(part, out[3]);
+    return __builtin_bit_cast(bf16x8_t, u32x4_t{out[0], out[1], out[2], out[3]});
+  }
+
+  template <int T = 0>
+  __device__ __forceinline__ void ask_first(uint32_t at) {
+    if constexpr (T < MT) {
+      ask_lds<T * 2048>(now[T], at);
+      ask_first<T + 1>(at);
+    }
+  }
+
+  __device__ __forceinline__ void run(const StreamParams& p, const Slot& sl, uint8_t* lds, const PanelShare& part) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), q = lane >> 4, r16 = lane & 15;
+    const PanelWave share = panel_wave(p, part, wave);
+    const int nb = part.group * p.nbw + share.nbi;
+    const bool active = nb < p.n_blocks;
+    const int mine = 2 * share.chunks, halves = 2 * share.most;  // this split's half chunks; the longest split's, which all wavefronts walk
+    uint8_t* abuf = lds + share.ks * 2 * BUF;
+    uint8_t* slot = lds + p.ks * 2 * BUF + wave * Fmt::BLOCK_BYTES;
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+      for (int nt = 0; nt < 4; nt++) acc[t][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    RingSource w;
+    w.row = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(sl.w + (int64_t)(active ? nb : 0) * p.chunks * Fmt::BLOCK_BYTES), 0, p.chunks * Fmt::BLOCK_BYTES, 0x00020000);
+    uint32_t codes, scales;
+    Ring::lanes(w, lane, r16, (uint32_t)(uintptr_t)(lds_ptr_t)slot, codes, scales);
+    Ring::request(w, share.c0, (lds_ptr_t)slot);
+    // The split's pieces, dealt to its wavefronts in turn: piece j is rows 8 j .. 8 j + 7, lane l lands at its byte 16 l, the
+    // 16-byte column (l & 7) of row 8 j + l / 8 - which holds the row's column (l & 7) ^ (row / 2 & 7), so that the sixteen
+    // rows of a fragment read lie in sixteen different 16-byte columns of the LDS.
+    const __amdgpu_buffer_rsrc_t arow = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p.a), 0, (int)p.a_bytes, 0x00020000);
+    uint32_t piece[HELD];
+#pragma unroll
+    for (int j = 0; j < HELD; j++) {
+      const int id = j * p.nbw + share.nbi;
+      if (id < PIECES) {
+        const int row = 8 * id + (lane >> 3);
+        piece[j] = (uint32_t)(activation_row_index<EPI>(p, sl, row) * p.a_stride) * 2 + (uint32_t)(((lane & 7) ^ ((row >> 1) & 7)) << 4);
+      }
+    }
+    auto bring = [&](int h) {
+#pragma unroll
+      for (int j = 0; j < HELD; j++) {
+        const int id = j * p.nbw + share.nbi;
+        if (id < PIECES)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(arow, (lds_ptr_t)(abuf + (h & 1) * BUF + id * 1024), 16, piece[j], (uint32_t)(share.c0 * 256 + h * (PANEL_HALF * 2)), 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    const uint32_t at0 = (uint32_t)(uintptr_t)(lds_ptr_t)abuf + r16 * 128 + ((q ^ (r16 >> 1)) << 4), at1 = at0 ^ 64;
+    bring(0);
+    bring(1);
+    wait_vm<0>();
+    __builtin_amdgcn_s_barrier();
+    Chunk ch;
+    Ring::ask(ch, codes, scales);
+    ask_first(at0);
+    wait_lds();
+    Ring::have(ch);
+    if (mine > 2) Ring::request(w, share.c0 + 1, (lds_ptr_t)slot);
+    for (int h = 0; h < halves; h += 2) {
+      if (h < mine) {
+        bf16x8_t b = whole(ch, sl);
+        b = group<0, true, -1>(ch, sl, b, 0);
+        b = group<1, false, -1>(ch, sl, b, 0);
+        b = group<2, false, -1>(ch, sl, b, 0);
+        b = group<3, false, 0>(ch, sl, b, at1);
+        b = group<4, true, -1>(ch, sl, b, 0);
+        if (h + 2 < mine) wait_vm<Ring::LOADS>(); else wait_vm<0>();  // the half after this one has landed; what was asked for behind it are the next weights
+        __builtin_amdgcn_s_barrier();
+        if (h + 2 < mine) bring(h + 2);
+        b = group<5, false, -1>(ch, sl, b, 0);
+        b = group<6, false, -1>(ch, sl, b, 0);
+        b = group<7, false, BUF>(ch, sl, b, at0);
+        b = group<8, true, -1>(ch, sl, b, 0);
+        b = group<9, false, -1>(ch, sl, b, 0);
+        b = group<10, false, -1>(ch, sl, b, 0);
+        b = group<11, false, BUF>(ch, sl, b, at1);
+        b = group<12, true, -1>(ch, sl, b, 0);
+        wait_vm<0>();
+        __builtin_amdgcn_s_barrier();
+        if (h + 3 < mine) bring(h + 3);
+        b = group<13, false, -1>(ch, sl, b, 0);
+        b = group<14, false, -1>(ch, sl, b, 0);
+        Chunk after;
+        Ring::ask(after, codes, scales);
+        group<15, false, 0>(ch, sl, b, at0);
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(MT) : "memory");  // the weights; the fragments' own waits follow
+        Ring::have(after);
+        ch = after;
+        if (h + 4 < mine) Ring::request(w, share.c0 + (h >> 1) + 2, (lds_ptr_t)slot);
+      } else {
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_s_barrier();
+      }
+    }
+    wait_lds();
+    products_done();
+#pragma unroll
+    for (int t = 0; t < MT; t++)
+#pragma unroll
+      for (int nt = 0; nt < 4; nt++) pin(acc[t][nt]);
+    finish(p, sl, lds, part, nb, active, share.ks, share.nbi, lane);
+  }
+
+  // The four neighbouring output columns of one lane and tile (gated: the pair's up and gate tiles).
+  static __device__ __forceinline__ void emit(const StreamParams& p, const Slot& sl, int nb, int t, int nt, int lane, const f32x4_t& v0, const f32x4_t& v1) {
+    typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
+    const int q = lane >> 4, i = 16 * t + (lane & 15);
+    if (i >= sl.rows) return;
+    const int64_t pos = sl.p0 + i;
+    auto scale = [&](int r, int tile) { return Fmt::PER_ROW ? sl.rs[nb * 64 + 16 * tile + 4 * q + r] : sl.scalar; };
+    if (EPI == EPI_FC1_GATED) {  // nt: the pair
+      float h[4];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {
+        const uint32_t ug = bf16_pair(v0[r] * scale(r, 2 * nt), v1[r] * scale(r, 2 * nt + 1));  // up and gate rounded to BF16 ...
+        h[r] = silu(pair_hi(ug)) * pair_lo(ug);                                                // ... and their product, rounded below
+      }
+      *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(p.out) + pos * p.out_stride + nb * 32 + 16 * nt + 4 * q) = u32x2_t{bf16_pair(h[0], h[1]), bf16_pair(h[2], h[3])};
+      return;
+    }
+    const int64_t at = (EPI == EPI_FC2 ? (int64_t)p.order[pos] : pos) * p.out_stride + nb * 64 + 16 * nt + 4 * q;
+    float y[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) y[r] = v0[r] * scale(r, nt);
+    if (EPI == EPI_FC1_RELU2 || EPI == EPI_DENSE_RELU2) {  // bf16(relu(bf16(y))^2), two values a conversion
+      const uint32_t u01 = bf16_pair(y[0], y[1]), u23 = bf16_pair(y[2], y[3]);
+      // relu on the bits: a negative value (and -0) is a negative integer; a NaN stays one, as torch's relu leaves it
+      const float h0 = __int_as_float(max((int)(u01 << 16), 0)), h1 = __int_as_float(max((int)(u01 & 0xffff0000u), 0));
+      const float h2 = __int_as_float(max((int)(u23 << 16), 0)), h3 = __int_as_float(max((int)(u23 & 0xffff0000u), 0));
+      y[0] = h0 * h0, y[1] = h1 * h1, y[2] = h2 * h2, y[3] = h3 * h3;
+    }
+    if (EPI != EPI_FC2 || p.out_bf16) {
+      *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(p.out) + at) = u32x2_t{bf16_pair(y[0], y[1]), bf16_pair(y[2], y[3])};
+    } else {
+      *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.out) + at) = f32x4_t{y[0], y[1], y[2], y[3]};
+    }
+  }
+
+  // What becomes of a K-complete (over this workgroup's share) result: stored, or left in memory for the workgroup that
+  // arrives last.
+  static __device__ __forceinline__ void deliver(const StreamParams& p, const Slot& sl, const PanelShare& part, int nb, int nbi, int t, int nt, int lane, const f32x4_t& v0,
+                                                 const f32x4_t& v1) {
+    if (part.kz > 1) {
+      store_through16(partial_at(p, part, part.z, nbi, t, nt) + lane, v0);
+    } else {
+      emit(p, sl, nb, t, nt, lane, v0, v1);
+    }
+  }
+  static __device__ __forceinline__ f32x4_t* partial_at(const StreamParams& p, const PanelShare& part, int z, int nbi, int t, int nt) {
+    return reinterpret_cast<f32x4_t*>(p.partial) + ((((int64_t)part.shared_tile * part.kz + z) * p.nbw + nbi) * (MT * 4) + t * 4 + nt) * 64;
+  }
+
+  // The K splits' tiles meet in LDS, two row tiles at a time, and are added in split order; each split's wavefront takes
+  // every ks-th of the results. Where further workgroups share the tile's K, all leave their results in memory (written
+  // through and waited for) and draw a ticket; the last one adds them in the order of the shares: the same sum whichever
+  // it is. The tickets lie at a fixed place in the workspace and are zero again when the launch ends.
+  __device__ __forceinline__ void finish(const StreamParams& p, const Slot& sl, uint8_t* lds, const PanelShare& part, int nb, bool active, int ks, int nbi, int lane) {
+    constexpr bool GATED = EPI == EPI_FC1_GATED;
+    if (p.ks == 1) {
+      if (active) {
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+          if (16 * t < sl.rows) {
+#pragma unroll
+            for (int nt = 0; nt < (GATED ? 2 : 4); nt++) deliver(p, sl, part, nb, nbi, t, nt, lane, acc[t][GATED ? 2 * nt : nt], acc[t][GATED ? 2 * nt + 1 : nt]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    } else {
+      f32x4_t* all = reinterpret_cast<f32x4_t*>(lds);
+      f32x4_t* mine = all + (nbi * p.ks + ks) * 512 + lane;
+      const f32x4_t* first = all + nbi * p.ks * 512 + lane;
+#pragma unroll
+      for (int t0 = 0; t0 < MT; t0 += 2) {
+        __syncthreads();  // the memory is free: the last fragments, or the tiles before these, have been read
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+          if (t0 + (u >> 2) < MT) mine[u * 64] = acc[t0 + (u >> 2) < MT ? t0 + (u >> 2) : 0][u & 3];
+        __syncthreads();
+        if (active) {
+          for (int u = ks; u < (GATED ? 4 : 8); u += p.ks) {
+            const int t = t0 + (GATED ? u >> 1 : u >> 2), nt = GATED ? u & 1 : u & 3, from = GATED ? 2 * u : u;
+            if (t >= MT || 16 * t >= sl.rows) continue;
+            f32x4_t v0 = first[from * 64], v1 = v0;
+            if (GATED) v1 = first[(from + 1) * 64];
+            for (int s = 1; s < p.ks; s++) {
+              v0 += first[s * 512 + from * 64];
+              if (GATED) v1 += first[s * 512 + (from + 1) * 64];
+            }
+            deliver(p, sl, part, nb, nbi, t, nt, lane, v0, v1);
+          }
+        }
+      }
+    }
+    if (GATED || part.kz == 1) return;  // (calls that share K among workgroups are dense)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's results are in memory before the count
+    __syncthreads();
+    int* last = reinterpret_cast<int*>(lds);
+    if (threadIdx.x == 0) {
+      unsigned int* ticket = p.tile_tickets + part.shared_tile;
+      *last = atomicAdd(ticket, 1u) == (unsigned)part.kz - 1u;
+      if (*last) *ticket = 0u;
+    }
+    __syncthreads();
+    if (!*last || !active) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // drop what this compute die's L2 holds of the others' results
+    constexpr int BATCH = 4;  // results whose shares are asked for together, a share ahead of the one being added
+    const int count = (MT * 4 - ks + p.ks - 1) / p.ks;  // what this wavefront delivered: results ks, ks + p.ks, ...
+    auto unit = [&](int i) { return i * p.ks + ks; };
+    for (int i0 = 0; i0 < count; i0 += BATCH) {
+      f32x4_t sum[BATCH], more[BATCH];
+      auto load = [&](f32x4_t (&to)[BATCH], int z) {
+#pragma unroll
+        for (int j = 0; j < BATCH; j++) to[j] = partial_at(p, part, z, nbi, 0, unit(min(i0 + j, count - 1)))[lane];
+      };
+      load(sum, 0);
+      load(more, 1);
+      for (int z = 1; z < part.kz; z++) {
+        f32x4_t then[BATCH];
+        if (z + 1 < part.kz) load(then, z + 1);
+#pragma unroll
+        for (int j = 0; j < BATCH; j++) {
+          sum[j] += more[j];
+          more[j] = then[j];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < BATCH; j++) {
+        const int u = unit(i0 + j);
+        if (i0 + j < count && 16 * (u >> 2) < sl.rows) emit(p, sl, nb, u >> 2, u & 3, lane, sum[j], sum[j]);
+      }
+    }
+  }
+};
+
+// Dense calls: every slot has up to 16 MT rows. Tile by tile, a slot's blocks one after the other (they share its
+// activations); the tiles past p.panel_full have their K shared by p.panel_kz workgroups each.
+template <class Fmt, int EPI, int MT>
+__global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_kernel(StreamParams p) {
+  extern __shared__ __align__(16) uint8_t panel_lds[];
+  int tile = blockIdx.x;
+  PanelShare part{0, 0, 1, 0};
+  if (tile >= p.panel_full) {
+    const int r = tile - p.panel_full;
+    part.shared_tile = r / p.panel_kz;
+    part.z = r - part.shared_tile * p.panel_kz;
+    part.kz = p.panel_kz;
+    tile = p.panel_full + part.shared_tile;
+  }
+  const int slot = tile / p.panel_groups;
+  part.group = tile - slot * p.panel_groups;
+  const Slot sl = slot_of<EPI>(p, slot);
+  if (sl.rows <= 0) return;
+  Panel<Fmt, EPI, MT> panel;
+  panel.run(p, sl, panel_lds, part);
+}
+
+template <class Fmt>
+inline size_t panel_lds_bytes(int mt, int ks, int nbw) {
+  const size_t loop = (size_t)ks * 2 * mt * 2048 + (size_t)ks * nbw * Fmt::BLOCK_BYTES, exchange = ks > 1 ? (size_t)ks * nbw * 8192 : 0;
+  return loop > exchange ? loop : exchange;
+}
+
+
+// Routed calls: a plan's slots of up to 128 rows, as many row tiles as the slot's rows need.
+template <class Fmt, int EPI>
+__global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_routed_kernel(StreamParams p) {
+  extern __shared__ __align__(16) uint8_t panel_lds[];
+  const int slot = blockIdx.x / p.panel_groups;
+  const PanelShare part{(int)blockIdx.x - slot * p.panel_groups, 0, 1, 0};
+  const Slot sl = slot_of<EPI>(p, slot);
+  if (sl.rows <= 0) return;  // a slot the plan did not fill: the whole workgroup leaves
+  auto run = [&](auto panel) { panel.run(p, sl, panel_lds, part); };
+  switch ((sl.rows + 15) >> 4) {
+    case 1: run(Panel<Fmt, EPI, 1>{}); break;
+    case 2: run(Panel<Fmt, EPI, 2>{}); break;
+    case 3: run(Panel<Fmt, EPI, 3>{}); break;
+    case 4: run(Panel<Fmt, EPI, 4>{}); break;
+    case 5: run(Panel<Fmt, EPI, 5>{}); break;
+    case 6: run(Panel<Fmt, EPI, 6>{}); break;
+    case 7: run(Panel<Fmt, EPI, 7>{}); break;
+    default: run(Panel<Fmt, EPI, 8>{}); break;
+  }
+}
+
+// How a dense call is cut: row tiles a slot, the shape of a workgroup, the tiles whose K is shared and among how many.
+struct PanelPlan {
+  int mt, slots, ks, nbw, groups, kz;
+  int64_t full, tiles;
+  double us;  // the estimate it was chosen by
+};
+// The tickets of the tiles whose K is shared: a fixed place at the head of the workspace, whatever the call's shape, so that
+// no other call's partial results are ever found there; the partial results follow.
+constexpr size_t PANEL_TICKET_BYTES = 4096;
+constexpr int64_t PANEL_SHARED_TILES = PANEL_TICKET_BYTES / 4 - PLAN_HEADER;
+inline size_t panel_room(const PanelPlan& q) { return q.kz > 1 ? PANEL_TICKET_BYTES + (size_t)(q.tiles - q.full) * q.kz * q.nbw * q.mt * 4 * 64 * sizeof(f32x4_t) : 0; }
+
+// The cut with the least estimated time, by a model fitted to 3 300 measured (size, cut) pairs (MI355X, us; 1024 .. 25600
+// columns, K 512 .. 5120, 17 .. 2048 rows; the cut it takes is within 2.4 % of the best measured one on average): a chunk of
+// a wavefront takes 1.45 + 0.16 mt with two wavefronts a SIMD and 0.7 + 0.1 mt alone; a workgroup's start and end 4.6;
+// eight-wavefront workgroups run one a compute unit, four-wavefront ones two where their LDS allows; the last arriver of
+// a shared tile reads its partial results at about 46 GB/s and the handing over costs 5.3. `room`: bytes of the workspace.
+template <class Fmt>
+inline PanelPlan search_panel(int m, int n_blocks, int chunks, size_t room) {
+  static const struct { int ks, nbw; } shapes[] = {{1, 4}, {1, 8}, {2, 2}, {2, 4}, {4, 1}, {4, 2}, {8, 1}};
+  PanelPlan best{};
+  best.us = 1e30;
+  const int least = (m + 127) / 128;
+  for (int slots = least; slots <= least + 1; slots++) {
+    const int mt = ((m + slots - 1) / slots + 15) / 16;
+    const double pair = 1.45 + 0.16 * mt, alone = 0.7 + 0.105 * mt;
+    for (auto& shape : shapes) {
+      const size_t lds = panel_lds_bytes<Fmt>(mt, shape.ks, shape.nbw);
+      if (lds > PANEL_LDS || shape.nbw < panel_least_blocks(mt) || shape.ks > chunks) continue;
+      const bool wide = shape.ks * shape.nbw == 8;
+      const int64_t groups = (n_blocks + shape.nbw - 1) / shape.nbw, tiles = groups * ((m + 16 * mt - 1) / (16 * mt));
+      const int64_t resident = !wide && 2 * lds <= PANEL_LDS ? 512 : 256;
+      auto rounds = [&](int64_t workgroups, int c) {  // us of that many workgroups of c chunks a wavefront
+        const int64_t whole = workgroups / resident, rest = workgroups - whole * resident;
+        const double busy = wide || resident == 512 ? pair : alone;
+        return whole * (c * busy + 4.6) + (rest ? c * (wide || rest > 256 ? pair : alone) + 4.6 : 0);
+      };
+      for (int kz = 1; kz <= 16 && (kz == 1 || chunks / kz >= shape.ks); kz++) {
+        const int64_t full = kz == 1 ? tiles : tiles / resident * resident, rest = tiles - full;
+        if (kz > 1 && (!rest || rest > PANEL_SHARED_TILES)) continue;
+        PanelPlan q{mt, slots, shape.ks, shape.nbw, (int)groups, kz, full, tiles, 0};
+        if (panel_room(q) > room) continue;
+        q.us = rounds(full, (chunks + shape.ks - 1) / shape.ks);
+        if (rest) q.us += rounds(rest * kz, ((chunks + kz - 1) / kz + shape.ks - 1) / shape.ks) + (kz > 1 ? 5.3 + kz * (double)mt * shape.nbw * 4096 / 46e3 : 0);
+        if (q.us < best.us * (kz > 1 ? 0.97 : 1.0)) best = q;
+      }
+    }
+  }
+  return best;
+}
+
+// ... kept for the sizes a thread asks for again and again (the search takes microseconds).
+template <class Fmt>
+inline const PanelPlan& plan_panel(int m, int n_blocks, int chunks, size_t room) {
+  struct Entry {
+    int m, n_blocks, chunks;
+    size_t room;
+    PanelPlan plan;
+  };
+  static thread_local Entry kept[64];
+  Entry& e = kept[((unsigned)m * 31u + (unsigned)n_blocks * 7u + (unsigned)chunks + (room ? 13u : 0u)) & 63u];
+  if (e.m != m || e.n_blocks != n_blocks || e.chunks != chunks || e.room != room) e = Entry{m, n_blocks, chunks, room, search_panel<Fmt>(m, n_blocks, chunks, room)};
+  return e.plan;
+}
+
+// Over a plan's slots of PANEL_SLOT_ROWS rows; `a_rows`: rows of the activation matrix. Four wavefronts a workgroup on four
+// blocks, two workgroups a compute unit: one's start and end lie beside the other's products.
+constexpr int PANEL_SLOT_ROWS = 128;
+template <class Fmt, int EPI>
+static int launch_panel_routed(StreamParams& p, int64_t slots, int64_t a_rows, hipStream_t stream) {
+  p.ks = 1;
+  p.nbw = 4;
+  set_split(p);
+  p.slot_rows = PANEL_SLOT_ROWS;
+  p.panel_groups = (p.n_blocks + p.nbw - 1) / p.nbw;
+  p.a_bytes = (uint32_t)(a_rows * p.a_stride * 2);
+  if (a_rows * p.a_stride * 2 > 0xffffffffll || slots * p.panel_groups > 0x7fffffff) return HB_EINVAL;
+  HB_LAUNCH((panel_routed_kernel<Fmt, EPI>), dim3((unsigned)(slots * p.panel_groups)), dim3(64 * p.ks * p.nbw), panel_lds_bytes<Fmt>(PANEL_SLOT_ROWS / 16, p.ks, p.nbw), stream, p);
+  return HB_OK;
+}
+
+}  // namespace hb

@@ -55,6 +55,8 @@ struct StreamParams {
   float* partial;         // tile kernel with K shared among workgroups: their partial tiles (see tile_kernel.hpp)
   int tile_ks, tile_mt;   // ... the workgroups a tile (1: none), the 16-row tiles a partial region holds
   uint32_t* tile_tickets; // ... and the tiles' arrival counters (one a tile, in the caller's workspace: zero between calls)
+  uint32_t a_bytes;       // panel kernel: bytes of the activation matrix (under 4 GiB)
+  int panel_groups, panel_full, panel_kz;  // panel kernel: runs of blocks a slot; the tiles below panel_full are a workgroup's each, the others' K is shared by panel_kz
   int64_t* trace;         // measurement hook (hb_debug_trace): a record a workgroup, else null
   int64_t trace_records;  // ... and the records it holds
   int32_t* done;          // fc1 and fc2 in one launch: the slots' arrival counters (plan_done), else null

@@ -17,6 +17,7 @@
 #include <algorithm>
 #include <atomic>
 
+#include "panel_kernel.hpp"
 #include "stream_common.hpp"
 
 namespace hb {
@@ -55,10 +56,6 @@ __device__ __forceinline__ void stage_tile(const StreamParams& p, const uint32_t
 // and runs the epilogue. The counters (p.tile_tickets, one a tile) lie at the head of the caller's workspace, ahead of
 // the partial tiles: zero when the caller hands the workspace over, put back to zero by every last arriver, so calls in
 // flight together on workspaces of their own share nothing.
-
-__device__ __forceinline__ void store_through16(f32x4_t* at, const f32x4_t& v) {
-  asm volatile("global_store_dwordx4 %0, %1, off sc1" ::"v"(at), "v"(v) : "memory");
-}
 
 template <int N>
 __device__ __forceinline__ void wait_but(void) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }

@@ -433,6 +433,7 @@ int hb_nvfp4_gemm(const void* x, int m, const void* tiled, float global_scale, i
  * in one fixed order: the result does not depend on the schedule. hb_nvfp4_gemm_workspace_bytes: what a call of this
  * shape uses (0: none, the call is hb_nvfp4_gemm's); the tiles' arrival counters lie at its head (zero before the first
  * use, see "Workspaces" above). No counterpart in the reference (cuBLASLt / FlashInfer own their workspaces there). */
+size_t hb_nvfp4_gemm_room_bytes(int m, int n, int k);
 size_t hb_nvfp4_gemm_workspace_bytes(int m, int n, int k);
 int hb_nvfp4_gemm_ws(const void* x, int m, const void* tiled, float global_scale, int n, int k, int relu2, void* y,
                      void* workspace, size_t workspace_bytes, void* stream);

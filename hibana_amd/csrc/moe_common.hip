@@ -721,52 +721,40 @@ __global__ __launch_bounds__(1024) void latent_router_kernel(RouterGemv g) {
   }
 }
 
-// The router's product of a routed layer for at most MOE_ROUTER_ROWS rows (the library product it replaces ran 8.4 - 8.7 us
-// at 1, 32 and 40 rows, hidden 2048, 512 experts, and another 2 us widened its BF16 result; this one TIMING): latency
-// bound (2 MB of weights), so sixteen columns a workgroup and K over its sixteen wavefronts, every load of a wavefront's
-// four steps in flight together; MT row tiles of sixteen share a weight fragment. Partial tiles through LDS, added in
-// wavefront order, rounded to BF16 once.
-template <int MT>
+// The router's product of a routed layer for at most MOE_ROUTER_ROWS rows: latency bound (2 MB of weights), so sixteen
+// columns and sixteen rows a workgroup and K over its sixteen wavefronts, every load of a wavefront's four steps in flight
+// together. Partial tiles through LDS, added in wavefront order, rounded to BF16 once. At hidden 2048, 512 experts the
+// library product it replaces took 8.4 - 8.7 us at 1, 32 and 40 rows, and another 2 us widened its BF16 result; the row
+// tiles on one workgroup (sharing a weight fragment) 4.7, 7.9 and 9.6 us, on workgroups of their own 5.0, 5.8 and 6.0.
 __global__ __launch_bounds__(1024) void moe_router_kernel(const uint16_t* __restrict__ w, const uint16_t* __restrict__ x, uint16_t* __restrict__ logits, int e,
                                                           int h, int m) {
-  extern __shared__ __align__(16) float part[];  // [16 wavefronts][MT][256]
+  __shared__ __align__(16) float part[16 * 256];
   constexpr int BATCH = 4;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, n0 = blockIdx.x * 16;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, n0 = blockIdx.x * 16, m0 = blockIdx.y * 16;
   const int steps = h / 32, s0 = steps * wave / 16, s1 = steps * (wave + 1) / 16;
   const uint16_t* wat = w + (int64_t)min(n0 + r16, e - 1) * h + 8 * (lane >> 4);
-  const uint16_t* xat[MT];
-  f32x4_t acc[MT];
-#pragma unroll
-  for (int t = 0; t < MT; t++) {
-    xat[t] = x + (int64_t)min(16 * t + r16, m - 1) * h + 8 * (lane >> 4);
-    acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  }
+  const uint16_t* xat = x + (int64_t)min(m0 + r16, m - 1) * h + 8 * (lane >> 4);
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
   for (int s = s0; s < s1; s += BATCH) {
-    u32x4_t b[BATCH], a[BATCH][MT];
+    u32x4_t b[BATCH], a[BATCH];
 #pragma unroll
     for (int j = 0; j < BATCH; j++)
       if (s + j < s1) {
         b[j] = *reinterpret_cast<const u32x4_t*>(wat + 32 * (s + j));
-#pragma unroll
-        for (int t = 0; t < MT; t++) a[j][t] = *reinterpret_cast<const u32x4_t*>(xat[t] + 32 * (s + j));
+        a[j] = *reinterpret_cast<const u32x4_t*>(xat + 32 * (s + j));
       }
 #pragma unroll
     for (int j = 0; j < BATCH; j++)
-      if (s + j < s1) {
-#pragma unroll
-        for (int t = 0; t < MT; t++)
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[j][t]), __builtin_bit_cast(bf16x8_t, b[j]), acc[t], 0, 0, 0);
-      }
+      if (s + j < s1) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[j]), __builtin_bit_cast(bf16x8_t, b[j]), acc, 0, 0, 0);
   }
-#pragma unroll
-  for (int t = 0; t < MT; t++) *reinterpret_cast<f32x4_t*>(part + (wave * MT + t) * 256 + lane * 4) = acc[t];
+  *reinterpret_cast<f32x4_t*>(part + wave * 256 + lane * 4) = acc;
   __syncthreads();
-  for (int i = threadIdx.x; i < MT * 256; i += 1024) {
-    const int t = i >> 8, row = (i >> 4) & 15, n = n0 + (i & 15), at = t * 256 + ((row >> 2) * 16 + (i & 15)) * 4 + (row & 3);
+  if (threadIdx.x < 256) {
+    const int row = threadIdx.x >> 4, n = n0 + (threadIdx.x & 15), at = ((row >> 2) * 16 + (threadIdx.x & 15)) * 4 + (row & 3);
     float sum = 0.f;
 #pragma unroll
-    for (int v = 0; v < 16; v++) sum += part[v * MT * 256 + at];
-    if (16 * t + row < m && n < e) logits[(int64_t)(16 * t + row) * e + n] = bf16_of(sum);
+    for (int v = 0; v < 16; v++) sum += part[v * 256 + at];
+    if (m0 + row < m && n < e) logits[(int64_t)(m0 + row) * e + n] = bf16_of(sum);
   }
 }
 
@@ -968,14 +956,7 @@ static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, in
 }
 
 void moe_launch_router(const uint16_t* x, const uint16_t* w, int m, int e, int h, uint16_t* logits, hipStream_t stream) {
-  const dim3 grid((unsigned)((e + 15) / 16));
-  if (m <= 16) {
-    HB_LAUNCH(moe_router_kernel<1>, grid, dim3(1024), 16 * 1024, stream, w, x, logits, e, h, m);
-  } else if (m <= 32) {
-    HB_LAUNCH(moe_router_kernel<2>, grid, dim3(1024), 32 * 1024, stream, w, x, logits, e, h, m);
-  } else {
-    HB_LAUNCH(moe_router_kernel<4>, grid, dim3(1024), 64 * 1024, stream, w, x, logits, e, h, m);
-  }
+  HB_LAUNCH(moe_router_kernel, dim3((unsigned)((e + 15) / 16), (unsigned)((m + 15) / 16)), dim3(1024), 0, stream, w, x, logits, e, h, m);
 }
 
 int moe_launch_route_plan(const TopkRoute& route, int m, int topk, int32_t* ids, float* weights, int e_lo, int e_n, int shared_rows,

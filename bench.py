@@ -103,7 +103,7 @@ MFMA_BF16_PEAK_TFLOPS = 2500.0
 def latent_prefill(args) -> dict:
     """BASELINE config 4 (not the headline line; `--config 4`): the NVFP4 latent-MoE layer on a prefill chunk of 2048
     tokens - hidden 4096 projected to latent 1024, 512 ReLU^2 experts of intermediate 2688, top-22 by sigmoid scores.
-    A step is the whole block (fused router|fc1_latent GEMM, routing, plan, the two expert GEMMs on the MFMA tile kernel,
+    A step is the whole block (fused router|fc1_latent GEMM, routing, plan, the two expert GEMMs on the panel kernel,
     combine, fc2_latent GEMM); the roofline entry is the fc1 expert GEMM against the dense BF16 MFMA peak."""
     import torch
 
@@ -159,7 +159,7 @@ def latent_prefill(args) -> dict:
         "config": {"workload": "BASELINE config 4: NVFP4 latent-MoE layer, 2048 tokens, hidden 4096 -> latent 1024, 512 experts x inter 2688, "
                                "ReLU^2, top-22 sigmoid routing of N(0,1) logits, no shared expert",
                    "timed_as": "replays of one HIP graph of all steps; value and ms_per_step are the median replay"},
-        "roofline": {"bound": "mfma", "kernel": "tile_kernel<TileNvfp4, fc1 relu2>", "achieved": gemm_flops / (fc1_ms * 1e-3) / 1e12,
+        "roofline": {"bound": "mfma", "kernel": "panel_tile_kernel<TileNvfp4, fc1 relu2>", "achieved": gemm_flops / (fc1_ms * 1e-3) / 1e12,
                      "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": gemm_flops / (fc1_ms * 1e-3) / 1e12 / MFMA_BF16_PEAK_TFLOPS,
                      "traffic": None, "launch_flops": gemm_flops, "launch_ms": fc1_ms, "peak_measured": mfma_tflops,
                      "frac_of_measured": gemm_flops / (fc1_ms * 1e-3) / 1e12 / mfma_tflops,
@@ -324,7 +324,7 @@ def dense_decode(args) -> dict:
                                                 _lib.stream()), "nvfp4 gemm")
                 return yr
 
-            return run, "tile_kernel<TileNvfp4, dense>, K shared among workgroups" if need else "nvfp4_stream_kernel<dense>"
+            return run, "panel_kernel<TileNvfp4, dense>" if rows > 16 else "nvfp4_stream_kernel<dense>"
 
         step, kernel = call(m)
         what = f"BASELINE config 1: NVFP4 dense linear {n} x {k}, M = {m} (codes and block scales random, global scale 1/448)"

@@ -16,7 +16,6 @@
 #include "panel_kernel.hpp"
 #include "ring.hpp"
 #include "stream_common.hpp"
-#include "tile_kernel.hpp"
 
 namespace hb {
 
@@ -92,15 +91,6 @@ struct Fp4Chunk {  // the weight side of a chunk: four 16-row tiles of codes (a 
   u32x4_t w0, w1, w2, w3, sc;
   __device__ __forceinline__ const u32x4_t& tile(int nt) const { return nt == 0 ? w0 : nt == 1 ? w1 : nt == 2 ? w2 : w3; }
 };
-
-__device__ __forceinline__ void load_fp4_chunk(Fp4Chunk& ch, const uint8_t* blk, int lane) {
-  const u32x4_t* b = reinterpret_cast<const u32x4_t*>(blk);
-  ch.w0 = __builtin_nontemporal_load(b + lane);
-  ch.w1 = __builtin_nontemporal_load(b + 64 + lane);
-  ch.w2 = __builtin_nontemporal_load(b + 128 + lane);
-  ch.w3 = __builtin_nontemporal_load(b + 192 + lane);
-  ch.sc = __builtin_nontemporal_load(b + 256 + 2 * (lane & 15) + (lane >> 5));
-}
 
 // Byte S of a dword of E4M3 scales as FP32.
 template <int S>
@@ -461,7 +451,7 @@ __global__ __launch_bounds__(1024) void nvfp4_twin_kernel(StreamParams a, Stream
   }
 }
 
-// experiments (hb_tune): the stream's workgroup shape ("nvfp4_ksplit", "nvfp4_nbw"); "nvfp4_tile": 1 forces the tile kernel, 2 the stream
+// experiments (hb_tune): the stream's workgroup shape ("nvfp4_ksplit", "nvfp4_nbw"); "nvfp4_tile": 1 forces the panel kernel, 2 the stream
 static std::atomic<int> g_nvfp4_ksplit{0}, g_nvfp4_nbw{0}, g_nvfp4_tile{0}, g_nvfp4_few{0}, g_nvfp4_tile_ks{0};  // "nvfp4_few": 2 switches off the body for slots of at most eight rows; "nvfp4_tile_ks": the workgroups that share a tile's K
 
 static int shape_nvfp4(StreamParams& p, int64_t busy_slots) {
@@ -504,7 +494,7 @@ static int launch_twin(StreamParams& a, int64_t slots_a, int64_t busy_a, StreamP
   return HB_OK;
 }
 
-// ------------------------------------------------------------------------------ the prefill kernel's NVFP4 format
+// ------------------------------------------------------------------------------ the panel kernel's NVFP4 format
 struct TileNvfp4 {
   typedef Fp4Chunk Chunk;
   typedef Fp4Ring Ring;
@@ -534,51 +524,9 @@ struct TileNvfp4 {
   }
   static constexpr int BLOCK_BYTES = NVFP4_BLOCK_BYTES;
   static constexpr bool PER_ROW = false;
-  static __device__ __forceinline__ void load(Chunk& ch, const uint8_t* blk, int lane, int) { load_fp4_chunk(ch, blk, lane); }
-  static __device__ __forceinline__ bf16x8_t fragment(const Chunk& ch, int nt, int s, const Slot&) {
-    const uint32_t sc = ch.sc[nt];
-    return fp4_scaled(ch.tile(nt)[s], s == 0 ? fp4_scale<0>(sc) : s == 1 ? fp4_scale<1>(sc) : s == 2 ? fp4_scale<2>(sc) : fp4_scale<3>(sc));
-  }
+  static constexpr float EXPAND_US = 0.f;  // (the estimate's own constants are this format's)
+  static constexpr int BESIDE_TILES = 0;
 };
-
-template <int EPI>
-static int launch_panel(StreamParams& p, void* workspace, size_t workspace_bytes, hipStream_t stream) {
-  PanelPlan q = plan_panel<TileNvfp4>(p.m, p.n_blocks, p.chunks, workspace ? workspace_bytes : 0);
-  if (g_nvfp4_ksplit) {
-    q.ks = g_nvfp4_ksplit;
-    q.nbw = g_nvfp4_nbw ? g_nvfp4_nbw.load() : 1;
-    q.mt = ((p.m + (p.m + 127) / 128 - 1) / ((p.m + 127) / 128) + 15) / 16;
-    q.groups = (p.n_blocks + q.nbw - 1) / q.nbw;
-    q.tiles = q.full = (int64_t)q.groups * ((p.m + 16 * q.mt - 1) / (16 * q.mt));
-    q.kz = 1;
-    if (g_nvfp4_tile_ks > 1) q.kz = g_nvfp4_tile_ks, q.full = 0;
-  }
-  const size_t lds = panel_lds_bytes<TileNvfp4>(q.mt, q.ks, q.nbw);
-  const int64_t grid = q.full + (q.tiles - q.full) * q.kz;
-  if (q.us > 1e29 || q.ks * q.nbw > PANEL_WAVES || q.ks > p.chunks / q.kz || (q.ks & (q.ks - 1)) || q.nbw < panel_least_blocks(q.mt) || lds > PANEL_LDS || grid > 0x7fffffff || panel_room(q) > workspace_bytes) return HB_EINVAL;
-  p.ks = q.ks;
-  p.nbw = q.nbw;
-  set_split(p);
-  p.slot_rows = 16 * q.mt;
-  p.a_bytes = (uint32_t)((int64_t)p.m * p.a_stride * 2);
-  p.panel_groups = q.groups;
-  p.panel_full = (int)q.full;
-  p.panel_kz = q.kz;
-  p.tile_tickets = static_cast<uint32_t*>(workspace) + PLAN_HEADER;
-  p.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + PANEL_TICKET_BYTES);
-  auto launch = [&](auto kernel) { HB_LAUNCH(kernel, dim3((unsigned)grid), dim3(64 * q.ks * q.nbw), lds, stream, p); };
-  switch (q.mt) {
-    case 1: launch(panel_kernel<TileNvfp4, EPI, 1>); break;
-    case 2: launch(panel_kernel<TileNvfp4, EPI, 2>); break;
-    case 3: launch(panel_kernel<TileNvfp4, EPI, 3>); break;
-    case 4: launch(panel_kernel<TileNvfp4, EPI, 4>); break;
-    case 5: launch(panel_kernel<TileNvfp4, EPI, 5>); break;
-    case 6: launch(panel_kernel<TileNvfp4, EPI, 6>); break;
-    case 7: launch(panel_kernel<TileNvfp4, EPI, 7>); break;
-    default: launch(panel_kernel<TileNvfp4, EPI, 8>); break;
-  }
-  return HB_OK;
-}
 
 static inline unsigned grid_for(int64_t threads) { return (unsigned)((threads + 255) / 256); }
 
@@ -634,24 +582,12 @@ static int nvfp4_gemm(const void* x, int m, const void* tiled, float global_scal
   if (m <= 0 || n <= 0 || k <= 0 || n % 64 || k % 128) return HB_EINVAL;
   if (!aligned(x, 16) || !aligned(tiled, 16) || !aligned(y, 2) || !aligned(workspace, 16)) return HB_EINVAL;
   StreamParams p = dense_params(tiled, global_scale, n, k, x, m, y);
-  if (m > ROWS_PER_SLOT && tile_takes(m, k) && tile_writes(y, false) && g_nvfp4_tile == 0 && (g_nvfp4_ksplit || !g_nvfp4_tile_ks)) {
-    if (int e = relu2 ? launch_panel<EPI_DENSE_RELU2>(p, workspace, workspace_bytes, stream) : launch_panel<EPI_DENSE>(p, workspace, workspace_bytes, stream)) return e;
-    return launch_status();
-  }
-  // between the weight stream's sixteen rows a pass and a call that fills the device with 128-row tiles: tiles whose K
-  // is shared among workgroups
-  int ks = workspace && m > TILE_SPLIT_ROWS ? tile_split(m, p.n_blocks, p.chunks) : 1;
-  if (g_nvfp4_tile_ks && workspace) ks = std::min(g_nvfp4_tile_ks.load(), p.chunks);
-  if (tile_partial_bytes(m, p.n_blocks, ks) > workspace_bytes || tile_ticket_bytes(m, p.n_blocks) > HB_WORKSPACE_ZERO_BYTES) ks = 1;
-  if (tile_takes(m, k) && tile_writes(y, false) && (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && (ks > 1 || tile_serves_dense(m, p.n_blocks))))) {
-    const int64_t tile_slots = (m + TILE_ROWS - 1) / TILE_ROWS;
-    if (ks > 1) {
-      p.tile_ks = ks;
-      p.tile_mt = tile_partial_mt(m);
-      p.tile_tickets = static_cast<uint32_t*>(workspace) + PLAN_HEADER;
-      p.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + tile_ticket_bytes(m, p.n_blocks));
-    }
-    if (int e = relu2 ? launch_tile<TileNvfp4, EPI_DENSE_RELU2>(p, tile_slots, m, stream) : launch_tile<TileNvfp4, EPI_DENSE>(p, tile_slots, m, stream)) return e;
+  // the weight stream would pass over the matrix once for every sixteen rows; the panel kernel expands it once for 128
+  if (panel_takes(m, k) && panel_writes(y, false) && (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && m > ROWS_PER_SLOT))) {
+    const PanelForce force{g_nvfp4_ksplit, g_nvfp4_nbw, g_nvfp4_tile_ks};
+    if (int e = relu2 ? launch_panel<TileNvfp4, EPI_DENSE_RELU2>(p, workspace, workspace_bytes, force, stream)
+                      : launch_panel<TileNvfp4, EPI_DENSE>(p, workspace, workspace_bytes, force, stream))
+      return e;
     return launch_status();
   }
   const int64_t slots = (m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT;
@@ -664,10 +600,15 @@ extern "C" int hb_nvfp4_gemm(const void* x, int m, const void* tiled, float glob
   return nvfp4_gemm(x, m, tiled, global_scale, n, k, relu2, y, nullptr, 0, as_stream(stream));
 }
 
+// What the entry point has asked of its callers since it was added: room for every tile of four blocks (128 rows) to have
+// its K shared by about four hundred workgroups in all. A call takes the best cut that fits (hb_nvfp4_gemm_room_bytes: the
+// best of all).
 extern "C" size_t hb_nvfp4_gemm_workspace_bytes(int m, int n, int k) {
-  if (m <= TILE_SPLIT_ROWS || n <= 0 || k <= 0 || n % 64 || k % 128) return 0;
-  const int want = g_nvfp4_tile_ks ? std::min(g_nvfp4_tile_ks.load(), k / 128) : tile_split(m, n / 64, k / 128);
-  return tile_partial_bytes(m, n / 64, want);
+  if (m <= 20 || n <= 0 || k <= 0 || n % 64 || k % 128) return 0;
+  const int64_t tiles = (int64_t)((n / 64 + 3) / 4) * ((m + 127) / 128), chunks = k / 128;
+  const int64_t ks = g_nvfp4_tile_ks ? std::min<int64_t>(g_nvfp4_tile_ks, chunks) : tiles >= 200 ? 1 : std::max<int64_t>(1, std::min<int64_t>(chunks / 4, 400 / tiles));
+  const int mt = (std::min(m, 128) + 15) / 16;
+  return ks > 1 ? (((size_t)(PLAN_HEADER + tiles) * sizeof(uint32_t) + 255) & ~(size_t)255) + (size_t)tiles * ks * 4 * mt * 4 * 64 * sizeof(f32x4_t) : 0;
 }
 
 extern "C" size_t hb_nvfp4_gemm_room_bytes(int m, int n, int k) {
@@ -733,11 +674,13 @@ int64_t busy_slots(int64_t pairs, int experts, int64_t slots) { return pairs < 2
 int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, int m, int topk, const MoeWorkspace& ws, void* out_pairs,
                 int pairs_bf16, hipStream_t stream) {
   const int64_t pairs = (int64_t)m * topk;
-  // a dense contraction once an expert sees a few dozen rows: slots of 128 rows on the MFMA tile kernel; below that the
-  // 16-row slots of the weight stream
-  const bool dense = tile_takes(m, ex->hidden) && tile_takes(pairs, ex->inter) && tile_writes(out_pairs, !pairs_bf16) &&
-                     (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && pairs >= (int64_t)ex->experts * TILE_DENSE_ROWS));
-  const int slot_rows = dense ? TILE_ROWS : ROWS_PER_SLOT;
+  // A dense contraction once an expert sees about ten rows: slots of 128 rows on the panel kernel; below that the 16-row
+  // slots of the weight stream. Measured, stream and panel, the whole latent block in us: 512 experts (1024, 2688) 8 rows an
+  // expert 384 and 388, 12 rows 474 and 403, 24 rows 748 and 455; 256 experts (768, 1536) 8 rows 121 and 123, 10 rows 131 and
+  // 126, 24 rows 212 and 146; 128 experts (512, 1024) 10 rows 71 and 72, 24 rows 82 and 72.
+  const bool dense = panel_takes(m, ex->hidden) && panel_takes(pairs, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
+                     (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && pairs >= 10ll * ex->experts));
+  const int slot_rows = dense ? PANEL_SLOT_ROWS : ROWS_PER_SLOT;
   const int64_t slots = moe_max_slots(pairs, ex->experts, 0, slot_rows);
   if (slots > 65535) return HB_EINVAL;
   if (int e = moe_launch_plan(ids, pairs, ex->base, ex->experts, 0, ws, stream, slot_rows)) return e;

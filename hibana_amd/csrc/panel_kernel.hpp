@@ -17,6 +17,8 @@
 // step, when its fragments are in registers anyway: the next half's first ones are asked for beside the rest of it.
 #pragma once
 
+#include <algorithm>
+
 #include "ring.hpp"
 #include "stream_common.hpp"
 
@@ -347,7 +349,7 @@ struct Panel {
     __syncthreads();
     int* last = reinterpret_cast<int*>(lds);
     if (threadIdx.x == 0) {
-      unsigned int* ticket = p.tile_tickets + part.shared_tile;
+      unsigned int* ticket = p.panel_tickets + part.shared_tile;
       *last = atomicAdd(ticket, 1u) == (unsigned)part.kz - 1u;
       if (*last) *ticket = 0u;
     }
@@ -414,7 +416,7 @@ inline size_t panel_lds_bytes(int mt, int ks, int nbw) {
 
 // Routed calls: a plan's slots of up to 128 rows, as many row tiles as the slot's rows need.
 template <class Fmt, int EPI>
-__global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_routed_kernel(StreamParams p) {
+__global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_tile_kernel(StreamParams p) {
   extern __shared__ __align__(16) uint8_t panel_lds[];
   const int slot = blockIdx.x / p.panel_groups;
   const PanelShare part{(int)blockIdx.x - slot * p.panel_groups, 0, 1, 0};
@@ -458,7 +460,7 @@ inline PanelPlan search_panel(int m, int n_blocks, int chunks, size_t room) {
   const int least = (m + 127) / 128;
   for (int slots = least; slots <= least + 1; slots++) {
     const int mt = ((m + slots - 1) / slots + 15) / 16;
-    const double pair = 1.45 + 0.16 * mt, alone = 0.7 + 0.105 * mt;
+    const double pair = 1.45 + Fmt::EXPAND_US + 0.16 * mt, alone = 0.7 + 0.5 * Fmt::EXPAND_US + 0.105 * mt;
     for (auto& shape : shapes) {
       const size_t lds = panel_lds_bytes<Fmt>(mt, shape.ks, shape.nbw);
       if (lds > PANEL_LDS || shape.nbw < panel_least_blocks(mt) || shape.ks > chunks) continue;
@@ -466,6 +468,7 @@ inline PanelPlan search_panel(int m, int n_blocks, int chunks, size_t room) {
       const int64_t groups = (n_blocks + shape.nbw - 1) / shape.nbw, tiles = groups * ((m + 16 * mt - 1) / (16 * mt));
       const int64_t resident = !wide && 2 * lds <= PANEL_LDS ? 512 : 256;
       auto rounds = [&](int64_t workgroups, int c) {  // us of that many workgroups of c chunks a wavefront
+        if (wide && mt <= Fmt::BESIDE_TILES && 2 * lds <= PANEL_LDS && workgroups > 256) return workgroups / 256.0 * (c * pair + 4.6);  // the next ones start beside those at work
         const int64_t whole = workgroups / resident, rest = workgroups - whole * resident;
         const double busy = wide || resident == 512 ? pair : alone;
         return whole * (c * busy + 4.6) + (rest ? c * (wide || rest > 256 ? pair : alone) + 4.6 : 0);
@@ -498,6 +501,63 @@ inline const PanelPlan& plan_panel(int m, int n_blocks, int chunks, size_t room)
   return e.plan;
 }
 
+// Whether an activation matrix of `rows` rows is one the panel kernel takes: it addresses the matrix with 32-bit byte
+// offsets ...
+inline bool panel_takes(int64_t rows, int64_t a_stride) { return rows * a_stride * 2 <= 0xffffffffll; }
+// ... and writes four neighbouring output columns with one store: 8 bytes of BF16, 16 of FP32.
+inline bool panel_writes(const void* out, bool f32) { return aligned(out, f32 ? 16 : 8); }
+
+// hb_tune's cut of a dense call, where it fits (0: the estimate's): K splits and blocks of a workgroup, workgroups a tile.
+struct PanelForce {
+  int ks, nbw, kz;
+};
+
+// A dense call of p.m rows; `workspace`: room for shared tiles' partial results, or null (no tile's K is shared).
+template <class Fmt, int EPI>
+static int launch_panel(StreamParams& p, void* workspace, size_t workspace_bytes, const PanelForce& force, hipStream_t stream) {
+  const size_t room = workspace ? workspace_bytes : 0;
+  PanelPlan q = plan_panel<Fmt>(p.m, p.n_blocks, p.chunks, room);
+  if (force.ks || force.kz) {
+    PanelPlan f = q;
+    if (force.ks) {
+      f.ks = force.ks;
+      f.nbw = std::max(1, force.nbw);
+    }
+    f.groups = (p.n_blocks + f.nbw - 1) / f.nbw;
+    f.tiles = (int64_t)f.groups * ((p.m + 16 * f.mt - 1) / (16 * f.mt));
+    f.kz = std::max(1, std::min(force.kz, p.chunks / f.ks));
+    f.full = f.kz > 1 ? 0 : f.tiles;
+    if (f.ks * f.nbw <= PANEL_WAVES && !(f.ks & (f.ks - 1)) && f.ks <= p.chunks / f.kz && f.nbw >= panel_least_blocks(f.mt) && panel_lds_bytes<Fmt>(f.mt, f.ks, f.nbw) <= PANEL_LDS &&
+        panel_room(f) <= room && (f.kz == 1 || f.tiles <= PANEL_SHARED_TILES))
+      q = f;
+  }
+  const size_t lds = panel_lds_bytes<Fmt>(q.mt, q.ks, q.nbw);
+  const int64_t grid = q.full + (q.tiles - q.full) * q.kz;
+  if (q.us > 1e29 || grid > 0x7fffffff) return HB_EINVAL;
+  p.ks = q.ks;
+  p.nbw = q.nbw;
+  set_split(p);
+  p.slot_rows = 16 * q.mt;
+  p.a_bytes = (uint32_t)((int64_t)p.m * p.a_stride * 2);
+  p.panel_groups = q.groups;
+  p.panel_full = (int)q.full;
+  p.panel_kz = q.kz;
+  p.panel_tickets = static_cast<uint32_t*>(workspace) + PLAN_HEADER;
+  p.partial = reinterpret_cast<float*>(static_cast<char*>(workspace) + PANEL_TICKET_BYTES);
+  auto launch = [&](auto kernel) { HB_LAUNCH(kernel, dim3((unsigned)grid), dim3(64 * q.ks * q.nbw), lds, stream, p); };
+  switch (q.mt) {
+    case 1: launch(panel_kernel<Fmt, EPI, 1>); break;
+    case 2: launch(panel_kernel<Fmt, EPI, 2>); break;
+    case 3: launch(panel_kernel<Fmt, EPI, 3>); break;
+    case 4: launch(panel_kernel<Fmt, EPI, 4>); break;
+    case 5: launch(panel_kernel<Fmt, EPI, 5>); break;
+    case 6: launch(panel_kernel<Fmt, EPI, 6>); break;
+    case 7: launch(panel_kernel<Fmt, EPI, 7>); break;
+    default: launch(panel_kernel<Fmt, EPI, 8>); break;
+  }
+  return HB_OK;
+}
+
 // Over a plan's slots of PANEL_SLOT_ROWS rows; `a_rows`: rows of the activation matrix. Four wavefronts a workgroup on four
 // blocks, two workgroups a compute unit: one's start and end lie beside the other's products.
 constexpr int PANEL_SLOT_ROWS = 128;
@@ -509,8 +569,8 @@ static int launch_panel_routed(StreamParams& p, int64_t slots, int64_t a_rows, h
   p.slot_rows = PANEL_SLOT_ROWS;
   p.panel_groups = (p.n_blocks + p.nbw - 1) / p.nbw;
   p.a_bytes = (uint32_t)(a_rows * p.a_stride * 2);
-  if (a_rows * p.a_stride * 2 > 0xffffffffll || slots * p.panel_groups > 0x7fffffff) return HB_EINVAL;
-  HB_LAUNCH((panel_routed_kernel<Fmt, EPI>), dim3((unsigned)(slots * p.panel_groups)), dim3(64 * p.ks * p.nbw), panel_lds_bytes<Fmt>(PANEL_SLOT_ROWS / 16, p.ks, p.nbw), stream, p);
+  if (!panel_takes(a_rows, p.a_stride) || slots * p.panel_groups > 0x7fffffff) return HB_EINVAL;
+  HB_LAUNCH((panel_tile_kernel<Fmt, EPI>), dim3((unsigned)(slots * p.panel_groups)), dim3(64 * p.ks * p.nbw), panel_lds_bytes<Fmt>(PANEL_SLOT_ROWS / 16, p.ks, p.nbw), stream, p);
   return HB_OK;
 }
 

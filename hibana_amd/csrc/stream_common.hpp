@@ -52,9 +52,8 @@ struct StreamParams {
   int ks, nbw;            // wavefronts per workgroup = ks (K splits) * nbw (64-row blocks)
   int ks_inv, chunks_base, chunks_rem;  // set_split(): ceil(65536 / ks), chunks / ks, chunks % ks
   int no_few;             // W3 stream: slots of at most four rows take the sixteen-row body too
-  float* partial;         // tile kernel with K shared among workgroups: their partial tiles (see tile_kernel.hpp)
-  int tile_ks, tile_mt;   // ... the workgroups a tile (1: none), the 16-row tiles a partial region holds
-  uint32_t* tile_tickets; // ... and the tiles' arrival counters (one a tile, in the caller's workspace: zero between calls)
+  float* partial;         // panel kernel, K shared among workgroups: their partial results ...
+  uint32_t* panel_tickets; // ... and the shared tiles' arrival counters (in the caller's workspace: zero between calls)
   uint32_t a_bytes;       // panel kernel: bytes of the activation matrix (under 4 GiB)
   int panel_groups, panel_full, panel_kz;  // panel kernel: runs of blocks a slot; the tiles below panel_full are a workgroup's each, the others' K is shared by panel_kz
   int64_t* trace;         // measurement hook (hb_debug_trace): a record a workgroup, else null
@@ -642,7 +641,7 @@ int64_t* moe_trace_buffer(int64_t* records);  // hb_debug_trace's buffer and its
 // least four chunks per wavefront; what is left of a 4-wavefront workgroup takes neighbouring 64-row blocks.
 void pick_shape(int n_blocks, int chunks, int64_t slots, int want, int* ks, int* nbw);
 
-// hb_tune keys of the NVFP4 kernels ("nvfp4_tile": 1 forces the tile kernel, 2 the stream, 0 the built-in choice).
+// hb_tune keys of the NVFP4 kernels ("nvfp4_tile": 1 forces the panel kernel, 2 the stream, 0 the built-in choice).
 int nvfp4_tune(const char* key, int value);
 // hb_tune keys of the kernels shared by the routed calls ("route_plan": 2 keeps routing and plan in separate launches).
 int moe_tune(const char* key, int value);

@@ -13,19 +13,18 @@
 // LDS in a fixed order) and/or take neighbouring 64-row blocks. No atomics on floating point anywhere: results are
 // bitwise repeatable.
 //
-// Calls with many rows per weight block (prefill) go to the 128-row MFMA tile kernel of tile_kernel.hpp instead, through
-// the TileW3 policy below; the entry points choose (tile_serves_dense for a dense call, pairs per expert for a routed
-// one), and hb_tune("w3_tile", 1 | 2) forces one or the other.
+// Calls of more than sixteen rows, and routed ones with many rows an expert (prefill), go to the panel kernel of
+// panel_kernel.hpp instead, through the TileW3 policies below; hb_tune("w3_tile", 1 | 2) forces one or the other.
 #include <string.h>
 
 #include <algorithm>
 #include <atomic>
 #include <mutex>
 
+#include "panel_kernel.hpp"
 #include "ring.hpp"
 #include "route.hpp"
 #include "stream_common.hpp"
-#include "tile_kernel.hpp"
 #include "w3_layout.hpp"
 
 namespace hb {
@@ -144,6 +143,19 @@ struct W3RingOf<AUX, 3> {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(src.row, slot, 4, src.scales, at, W3_SCALE_OFFSET, AUX);
     __builtin_amdgcn_sched_barrier(0);  // asked for here, not wherever the scheduler would sink it below the arithmetic
   }
+  // the reads of a block from slot 0, and (after a wait) their values
+  static __device__ __forceinline__ void ask(Chunk& ch, uint32_t codes, uint32_t scales) {
+    ask_lds<0>(ch.w0, codes);
+    ask_lds<1024>(ch.w1, codes);
+    ask_lds<2048>(ch.w2, codes);
+    ask_lds<W3_SCALE_OFFSET>(ch.sc, scales);
+  }
+  static __device__ __forceinline__ void have(Chunk& ch) {
+    pin(ch.w0);
+    pin(ch.w1);
+    pin(ch.w2);
+    pin(ch.sc);
+  }
   template <int BEHIND, int SLOT>  // BEHIND: requests that may stay outstanding
   static __device__ __forceinline__ void take(Chunk& ch, uint32_t codes, uint32_t scales) {
     asm volatile(
@@ -177,6 +189,16 @@ struct W3RingOf<AUX, 2> {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(src.row, slot, 16, src.codes, at, 1024, AUX);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(src.row, slot, 4, src.scales, at, W2_SCALE_OFFSET, AUX);
     __builtin_amdgcn_sched_barrier(0);
+  }
+  static __device__ __forceinline__ void ask(Chunk& ch, uint32_t codes, uint32_t scales) {
+    ask_lds<0>(ch.w0, codes);
+    ask_lds<1024>(ch.w1, codes);
+    ask_lds<W2_SCALE_OFFSET>(ch.sc, scales);
+  }
+  static __device__ __forceinline__ void have(Chunk& ch) {
+    pin(ch.w0);
+    pin(ch.w1);
+    pin(ch.sc);
   }
   template <int BEHIND, int SLOT>
   static __device__ __forceinline__ void take(Chunk& ch, uint32_t codes, uint32_t scales) {
@@ -941,37 +963,53 @@ __global__ __launch_bounds__(1024) void w3_fc2_combine_one_kernel(StreamParams p
   if (PARTS == 1 || q / (4 / PARTS) == part) c.out[nb * 64 + lane] = f32_to_bf16_bits(v);  // lane (q, r16) is column 16 q + r16
 }
 
-// ------------------------------------------------------------------------------------ the prefill kernel's W3 format
+// ---------------------------------------------------------------------------------- the panel kernel's W3 formats
+// A fragment's eight weights: two selectors and two permutes give their E4M3 codebook bytes, which are expanded times the
+// group's E4M3 scale (a 4-bit significand times a 4-bit one: exact in BF16); the FP32 row scale stays in the epilogue.
+template <int BITS>
 struct TileW3 {
-  typedef hb::Chunk Chunk;
-  static constexpr int BLOCK_BYTES = W3_BLOCK_BYTES;
+  typedef W3RingOf<2, BITS> Ring;
+  typedef typename Ring::Chunk Chunk;
+  static constexpr int BLOCK_BYTES = Ring::BLOCK_BYTES;
   static constexpr bool PER_ROW = true;
-  static __device__ __forceinline__ void load(Chunk& ch, const uint8_t* blk, int lane, int r16) { load_chunk(ch, blk, lane, r16); }
-  // The B operand of 16-row tile nt, 32-group s, scaled by the group's E4M3 scale (a 4-bit level times a 4-bit scale:
-  // exact in BF16); the FP32 row scale stays in the epilogue.
-  static __device__ __forceinline__ bf16x8_t fragment(const Chunk& ch, int nt, int s, const Slot& sl) {
-    typedef __attribute__((ext_vector_type(2))) float f32x2_t;
-    typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_v;
-    const uint32_t q0 = nt == 0 ? ch.w0.x : nt == 1 ? ch.w0.w : nt == 2 ? ch.w1.z : ch.w2.y;
-    const uint32_t q1 = nt == 0 ? ch.w0.y : nt == 1 ? ch.w1.x : nt == 2 ? ch.w1.w : ch.w2.z;
-    const uint32_t q2 = nt == 0 ? ch.w0.z : nt == 1 ? ch.w1.y : nt == 2 ? ch.w2.x : ch.w2.w;
-    const uint32_t scales = nt == 0 ? ch.sc.x : nt == 1 ? ch.sc.y : nt == 2 ? ch.sc.z : ch.sc.w;
+  // For search_panel: a chunk of a pair of wavefronts takes this much longer than NVFP4's; and up to this many row tiles the
+  // registers of two eight-wavefront workgroups fit a compute unit (the pair of them is 10 % faster than whole rounds say).
+  static constexpr float EXPAND_US = 0.45f;
+  static constexpr int BESIDE_TILES = 3;
+  struct Part {
+    uint32_t lo, hi;  // codebook bytes of weights 0 .. 3 and 4 .. 7
+    float scale;
+  };
+  template <int NT, int S>
+  static __device__ __forceinline__ Part open(const Chunk& ch, const Slot& sl) {
     uint32_t sel[8];
-    w3_selectors(q0, q1, q2, sel);  // the six the step does not use fold away
-    const uint32_t f0 = __builtin_amdgcn_perm(sl.lut_hi, sl.lut_lo, sel[2 * s]);
-    const uint32_t f1 = __builtin_amdgcn_perm(sl.lut_hi, sl.lut_lo, sel[2 * s + 1]);
-    const float g = s == 0 ? __builtin_amdgcn_cvt_f32_fp8(scales, 0) : s == 1 ? __builtin_amdgcn_cvt_f32_fp8(scales, 1)
-                  : s == 2 ? __builtin_amdgcn_cvt_f32_fp8(scales, 2) : __builtin_amdgcn_cvt_f32_fp8(scales, 3);
-    const f32x2_t a = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(f0, 1.0f, false), b = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(f0, 1.0f, true);
-    const f32x2_t c = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(f1, 1.0f, false), d = __builtin_amdgcn_cvt_scalef32_pk_f32_fp8(f1, 1.0f, true);
-    u32x4_t packed;
-    packed.x = __builtin_bit_cast(uint32_t, bf16x2_v{(__bf16)(a.x * g), (__bf16)(a.y * g)});
-    packed.y = __builtin_bit_cast(uint32_t, bf16x2_v{(__bf16)(b.x * g), (__bf16)(b.y * g)});
-    packed.z = __builtin_bit_cast(uint32_t, bf16x2_v{(__bf16)(c.x * g), (__bf16)(c.y * g)});
-    packed.w = __builtin_bit_cast(uint32_t, bf16x2_v{(__bf16)(d.x * g), (__bf16)(d.y * g)});
-    return __builtin_bit_cast(bf16x8_t, packed);
+    chunk_selectors<NT>(ch, sel);  // the six the step does not use fold away
+    return Part{__builtin_amdgcn_perm(sl.lut_hi, sl.lut_lo, sel[2 * S]), __builtin_amdgcn_perm(sl.lut_hi, sl.lut_lo, sel[2 * S + 1]),
+                __builtin_amdgcn_cvt_f32_fp8(chunk_scales<NT>(ch), S)};
+  }
+#define HB_W3_CVT "v_cvt_scalef32_pk_f32_fp8"
+  template <int K, bool AFTER_VALU>  // a product, then values 2 K, 2 K + 1 of the part
+  static __device__ __forceinline__ void product_pair(f32x4_t& acc, const u32x4_t& w, const u32x4_t& a, const Part& part, uint32_t& out) {
+    if constexpr (K == 0 && AFTER_VALU) HB_PANEL_PRODUCT_PAIR("s_nop 1\n\t", HB_W3_CVT, "", acc, out, w, part.lo, part.scale, a);
+    if constexpr (K == 0 && !AFTER_VALU) HB_PANEL_PRODUCT_PAIR("", HB_W3_CVT, "", acc, out, w, part.lo, part.scale, a);
+    if constexpr (K == 1) HB_PANEL_PRODUCT_PAIR("", HB_W3_CVT, " op_sel:[1,0,0]", acc, out, w, part.lo, part.scale, a);
+    if constexpr (K == 2) HB_PANEL_PRODUCT_PAIR("", HB_W3_CVT, "", acc, out, w, part.hi, part.scale, a);
+    if constexpr (K == 3) HB_PANEL_PRODUCT_PAIR("", HB_W3_CVT, " op_sel:[1,0,0]", acc, out, w, part.hi, part.scale, a);
+  }
+  template <int K>
+  static __device__ __forceinline__ void pair_alone(const Part& part, uint32_t& out) {
+    if constexpr (K == 0) HB_PANEL_PAIR_ALONE(HB_W3_CVT, "", out, part.lo, part.scale);
+    if constexpr (K == 1) HB_PANEL_PAIR_ALONE(HB_W3_CVT, " op_sel:[1,0,0]", out, part.lo, part.scale);
+    if constexpr (K == 2) HB_PANEL_PAIR_ALONE(HB_W3_CVT, "", out, part.hi, part.scale);
+    if constexpr (K == 3) HB_PANEL_PAIR_ALONE(HB_W3_CVT, " op_sel:[1,0,0]", out, part.hi, part.scale);
   }
 };
+
+// A dense call: the stream's passes (one a sixteen rows) run side by side while their blocks do not fill the device, and the
+// few rows of a second pass are nearly free. Measured, stream and panel: 5120 x 5120 (80 blocks) 48 rows 10.9 and 15.0 us,
+// 77 rows 16.9 and 17.4, 128 rows 23.7 and 19.4; 8192 x 2048 32 rows 7.6 and 8.8, 48 rows 9.8 and 9.0; 51200 x 2048 17 rows
+// 20.6 and 20.3, 48 rows 30.7 and 22.8; 51200 x 5120 128 rows 195 and 70.
+constexpr int PANEL_W3_ROWS = 20, PANEL_W3_BLOCKS = 384;
 
 // ---------------------------------------------------------------------------------------------------- host side
 struct Tuning {  // hb_tune's knobs: relaxed atomics, so a knob set from one thread while another launches is a plain race-free read
@@ -1066,9 +1104,9 @@ extern "C" int hb_w3_gemm(const void* x, int m, const void* tiled, const float* 
   p.m = m;
   p.out = y;
   p.out_stride = n;
-  // (the MFMA tile kernel reads three-bit tiles; a two-bit matrix is served by the stream at every size)
-  if (bits == 3 && tile_takes(m, k) && tile_writes(y, false) && (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && tile_serves_dense(m, p.n_blocks)))) {
-    if (int e = launch_tile<TileW3, EPI_DENSE>(p, (m + TILE_ROWS - 1) / TILE_ROWS, m, as_stream(stream))) return e;
+  if (panel_takes(m, k) && panel_writes(y, false) && (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && m > PANEL_W3_ROWS && (int64_t)p.n_blocks * ((m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT) >= PANEL_W3_BLOCKS))) {
+    const PanelForce force{g_tune.w3_ksplit, g_tune.w3_nbw, 0};
+    if (int e = bits == 2 ? launch_panel<TileW3<2>, EPI_DENSE>(p, nullptr, 0, force, as_stream(stream)) : launch_panel<TileW3<3>, EPI_DENSE>(p, nullptr, 0, force, as_stream(stream))) return e;
     return launch_status();
   }
   const int64_t slots = (m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT;
@@ -1144,11 +1182,17 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
                 bool e4m3 = false, const CombineParams* combine = nullptr) {
   const int64_t pairs = (int64_t)m * topk;
   const int shared_rows = shared ? m : 0;
-  // a dense contraction once an expert sees a few dozen rows: slots of 128 rows on the MFMA tile kernel
-  // (E4M3 activations: the stream only)
-  const bool dense = !e4m3 && tile_takes(m, ex->hidden) && tile_takes(pairs + shared_rows, ex->inter) && tile_writes(out_pairs, !pairs_bf16) &&
-                     (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && pairs >= (int64_t)ex->experts * 2 * TILE_DENSE_ROWS));  // the pre-scaled expansion costs more here than the stream's
-  const int slot_rows = dense ? TILE_ROWS : ROWS_PER_SLOT;
+  // A dense contraction once an expert sees a few dozen rows: slots of 128 rows on the panel kernel (E4M3 activations: the
+  // stream only). The stream pays for a pass a sixteen rows, the panel for an expansion the few rows do not amortise and for
+  // a last round of workgroups that a small call does not fill. Measured, stream and panel, the whole layer in us: 512
+  // experts (2048, 512) 12 rows an expert 235 and 267, 16 rows 288 and 277, 30 rows 439 and 311 (skewed routing 16 rows 248
+  // and 208); 256 experts (2560, 768) 12 rows 224 and 235, 16 rows 292 and 250; 128 experts (2048, 512) 20 rows (0.98 M
+  // pairs x blocks) 111 and 120, 24 rows (1.2 M) 123 and 123; 128 experts (1024, 256) 24 rows (0.3 M) 70 and 83, 48 rows 98
+  // and 100, 96 rows 132 and 100.
+  const int64_t expert_blocks = (int64_t)((ex->gated ? 2 : 1) * ex->inter / W3_BLOCK_ROWS) * (ex->hidden / W3_CHUNK) + (int64_t)(ex->hidden_out / W3_BLOCK_ROWS) * (ex->inter / W3_CHUNK);
+  const bool dense = !e4m3 && panel_takes(m, ex->hidden) && panel_takes(pairs + shared_rows, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
+                     (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && (pairs >= 48ll * ex->experts || (pairs >= 16ll * ex->experts && pairs * expert_blocks >= 1000000))));
+  const int slot_rows = dense ? PANEL_SLOT_ROWS : ROWS_PER_SLOT;
   const int64_t slots = moe_max_slots(pairs, ex->experts, shared_rows, slot_rows);
   if (slots > 65535) return HB_EINVAL;
   // E4M3 activations: x is rounded by further workgroups of the plan's launch, h in fc1's epilogue
@@ -1221,8 +1265,8 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   f2.out_stride = ex->hidden_out;
   f2.out_bf16 = pairs_bf16;
   if (dense) {
-    if (int e = ex->gated ? launch_tile<TileW3, EPI_FC1_GATED>(p, slots, m, stream) : launch_tile<TileW3, EPI_FC1_RELU2>(p, slots, m, stream)) return e;
-    if (int e = launch_tile<TileW3, EPI_FC2>(f2, slots, pairs + shared_rows, stream)) return e;
+    if (int e = ex->gated ? launch_panel_routed<TileW3<3>, EPI_FC1_GATED>(p, slots, m, stream) : launch_panel_routed<TileW3<3>, EPI_FC1_RELU2>(p, slots, m, stream)) return e;
+    if (int e = launch_panel_routed<TileW3<3>, EPI_FC2>(f2, slots, pairs + shared_rows, stream)) return e;
     if (combine) moe_launch_combine(*combine, stream);
     return launch_status();
   }

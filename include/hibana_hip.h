@@ -72,7 +72,7 @@ int hb_workspace_status(const void* workspace, int32_t* status, int wait, void* 
 
 /* Tuning knobs for experiments and tests; value 0 restores the built-in choice. "w3_ksplit" / "w3_nbw",
  * "moe_fc1_ksplit" / "moe_fc1_nbw", "moe_fc2_ksplit" / "moe_fc2_nbw", "nvfp4_ksplit" / "nvfp4_nbw": K splits and 64-row
- * blocks per workgroup (their product at most 16); "w3_tile" / "nvfp4_tile": 1 forces the MFMA tile kernel, 2 the weight
+ * blocks per workgroup (their product at most 16); "w3_tile" / "nvfp4_tile": 1 forces the panel kernel, 2 the weight
  * stream; "w3_few" / "nvfp4_few": 2 switches off the stream's body for slots of few rows (W3: at most four, NVFP4: at
  * most eight); "moe_one": 2 switches off the single launch that does one token's fc2 and combine; "moe_fused": 2 runs a
  * routed call's fc1 and fc2 as two launches; "moe_lag": the slots fc2 lags fc1 by in their common launch; "moe_split":
@@ -427,12 +427,12 @@ int hb_nvfp4_dequant(const void* tiled, float global_scale, int64_t rows, int k,
 int hb_nvfp4_gemm(const void* x, int m, const void* tiled, float global_scale, int n, int k, int relu2, void* y,
                   void* stream);
 
-/* The same product with room for partial sums: calls of a few dozen rows (17 .. about 250), too many for the weight
- * stream's sixteen rows a pass over the matrix and too few to fill the device with 128-row tiles, share K among the
- * workgroups of a tile; their partial tiles meet in `workspace` and whichever workgroup of a tile finishes last adds them
- * in one fixed order: the result does not depend on the schedule. hb_nvfp4_gemm_workspace_bytes: what a call of this
- * shape uses (0: none, the call is hb_nvfp4_gemm's); the tiles' arrival counters lie at its head (zero before the first
- * use, see "Workspaces" above). No counterpart in the reference (cuBLASLt / FlashInfer own their workspaces there). */
+/* The same product with room for partial sums: calls of more than sixteen rows whose tiles do not fill the device share
+ * the K of some tiles among workgroups; their partial results meet in `workspace` and whichever workgroup of a tile
+ * finishes last adds them in one fixed order: the result does not depend on the schedule. hb_nvfp4_gemm_room_bytes: what
+ * the fastest cut of a call of this shape needs (0: none); hb_nvfp4_gemm_workspace_bytes: the room asked of callers since
+ * the entry point was added (a call takes the fastest cut that fits what it is given). The tiles' arrival counters lie at
+ * its head (zero before the first use, see "Workspaces" above). No counterpart in the reference (cuBLASLt / FlashInfer own their workspaces there). */
 size_t hb_nvfp4_gemm_room_bytes(int m, int n, int k);
 size_t hb_nvfp4_gemm_workspace_bytes(int m, int n, int k);
 int hb_nvfp4_gemm_ws(const void* x, int m, const void* tiled, float global_scale, int n, int k, int relu2, void* y,

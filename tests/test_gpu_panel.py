@@ -1,0 +1,83 @@
+"""The panel kernel (more than sixteen rows a weight block) at the edges of its cuts: one row more or less than whole row
+tiles and slots, a single 64-row block and a single chunk of K, row tiles that only wide workgroups hold, K shared inside a
+workgroup and among workgroups, calls of several shapes over one workspace."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import layers, nvfp4_format as onv, w3_format as ow3
+from tests.test_gpu_nvfp4 import _linear, _matrix
+from tests.util import MAX_REL, NORM_REL, errors, random_w3, to_device_w3
+
+pytestmark = pytest.mark.gpu
+ROWS = [17, 32, 33, 64, 65, 80, 96, 97, 112, 113, 128, 129, 257]
+
+
+@pytest.mark.parametrize("n,k", [(64, 128), (192, 640), (576, 1280)])
+def test_nvfp4_rows_around_whole_tiles(n, k):
+    """Every call on one workspace, whose head the calls before it (other shapes, other cuts) have used and left zero."""
+    from hibana_amd.kernels import ops
+    packed, scales = _matrix(n, k, n + k, hi=8.0)
+    lin = _linear(packed, scales, alpha=0.3, inv=1.0)
+    dense = onv.unpack_fp4(packed, scales)
+    for m in ROWS + ROWS[::-1]:
+        x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).bfloat16()
+        mx, nr = errors(ops.nvfp4_linear(x.cuda(), lin), layers.nvfp4_dense_ref(x, dense, np.float32(0.3)))
+        assert mx < MAX_REL and nr < NORM_REL, (m, mx, nr)
+
+
+@pytest.mark.parametrize("codebook", ["lloyd", "lloyd2"])  # three-bit and two-bit tiles
+@pytest.mark.parametrize("n,k", [(128, 128), (640, 640), (384, 1280)])
+def test_w3_rows_around_whole_tiles(n, k, codebook):
+    from hibana_amd import _lib
+    from hibana_amd.kernels import w3
+    packed, *_ = random_w3(n, k, 7, codebook)
+    dev = to_device_w3(packed)
+    dense = ow3.dequantize(packed)
+    assert _lib.lib().hb_tune(b"w3_tile", 1) == 0  # (these matrices are too small for the kernel to be the faster one)
+    try:
+        for m in [1, 16] + [m for m in ROWS if m <= w3.MAX_ROWS]:
+            x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).bfloat16()
+            got = w3.w3_linear(x.cuda(), dev)
+            mx, nr = errors(got, layers.dense_ref(x, dense))
+            assert mx < MAX_REL and nr < NORM_REL, (m, mx, nr)
+            assert torch.equal(w3.w3_linear(x.cuda(), dev), got), m
+    finally:
+        _lib.lib().hb_tune(b"w3_tile", 0)
+
+
+@pytest.mark.parametrize("m", [20, 21, 48, 77, 128])
+def test_w3_calls_the_library_gives_to_the_panel(m):
+    """n large enough for the built-in choice (24576 rows: 384 blocks) against the weight stream's product of the same call."""
+    from hibana_amd import _lib
+    from hibana_amd.kernels import w3
+    packed, *_ = random_w3(24576, 256, 3, "lloyd")
+    dev = to_device_w3(packed)
+    x = torch.randn(m, 256, generator=torch.Generator().manual_seed(m)).bfloat16().cuda()
+    got = w3.w3_linear(x, dev)
+    assert _lib.lib().hb_tune(b"w3_tile", 2) == 0
+    try:
+        stream = w3.w3_linear(x, dev)
+    finally:
+        _lib.lib().hb_tune(b"w3_tile", 0)
+    mx, nr = errors(got, stream)
+    assert mx < MAX_REL and nr < NORM_REL, (mx, nr)
+
+
+def test_nvfp4_calls_of_several_shapes_share_a_workspace():
+    """Shared tiles' counters lie at a fixed place of the workspace: calls whose tiles number differently, one after the
+    other on a stream, never take another's partial results for counters (a result nobody adds up is never stored)."""
+    from hibana_amd.kernels import ops
+    shapes = [(5120, 2688), (1024, 512), (2688, 1024), (64, 128), (4096, 1280)]
+    mats = []
+    for i, (n, k) in enumerate(shapes):
+        packed, scales = _matrix(n, k, i, hi=8.0)
+        mats.append((_linear(packed, scales, alpha=0.3, inv=1.0), torch.from_numpy(onv.unpack_fp4(packed, scales)).cuda()))
+    for m in (33, 200, 64, 512, 77, 333):
+        for (n, k), (lin, dense) in zip(shapes, mats):
+            x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).bfloat16().cuda()
+            junk = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")  # what the result's memory may hold before
+            del junk
+            got = ops.nvfp4_linear(x, lin)
+            mx, nr = errors(got, ((x.float() @ dense.T) * 0.3).bfloat16())
+            assert mx < MAX_REL and nr < NORM_REL, (m, n, k, mx, nr)

@@ -199,20 +199,26 @@ constexpr int FP4_RING_BYTES = ring_bytes<Fp4Ring>();  // LDS per wavefront; its
 // The blocks' sums are added across the lanes after the last chunk, which leaves the sixteen-row layout.
 constexpr int FP4_FEW_ROWS = 8, FP4_FEWER_ROWS = 4;
 
+// What a lane reads whose weights are not of its A row's parity: zeros, from here. That spares sixteen selects a chunk and
+// half of the activations' way through the L1 (eight rows, 25600 x 5120: 17.1 us, with the selects 19.3).
+__device__ const u32x4_t fp4_zero_piece[16] = {};
+
 struct Fp4Few8Acts {
   static constexpr int LOADS = 4;
   u32x4_t even[4], odd[4];  // the lane's piece of each step of the next even and the next odd chunk
-  bool mine;                // this lane's weights belong to its A row's parity
-  const uint16_t* at;       // the lane's piece of step 0 of the wavefront's first chunk
+  const uint16_t* at;       // the lane's piece of step 0 of the wavefront's first chunk ...
+  uint32_t stride;          // ... and the elements to the next chunk's (0: the zeros)
   __device__ __forceinline__ void load(u32x4_t (&to)[4], int i) const {
+    const uint16_t* from = at + i * stride;
 #pragma unroll
-    for (int s = 0; s < 4; s++) to[s] = *reinterpret_cast<const u32x4_t*>(at + (int64_t)i * 128 + 32 * s);
+    for (int s = 0; s < 4; s++) to[s] = *(const __attribute__((address_space(1))) u32x4_t*)(from + 32 * s);  // (said to be global: the compiler cannot tell of the two)
   }
   template <int EPI>
   __device__ __forceinline__ void start(const StreamParams& p, const Slot& sl, int, int c0, int n, int lane) {
     const int q = lane >> 4, r16 = lane & 15;
-    mine = (r16 >> 3) == (q >> 1);
-    at = activation_row<EPI>(p, sl, r16 & 7) + (int64_t)c0 * 128 + 8 * q;
+    const bool mine = (r16 >> 3) == (q >> 1);
+    at = mine ? activation_row<EPI>(p, sl, r16 & 7) + (int64_t)c0 * 128 + 8 * q : reinterpret_cast<const uint16_t*>(fp4_zero_piece);
+    stride = mine ? 128 : 0;
     load(even, 0);
     if (n > 1) load(odd, 1);
   }
@@ -228,12 +234,7 @@ struct Fp4Few8Acts {
   }
   template <int ODD, bool MORE2, bool MORE1>
   __device__ __forceinline__ void step(const Fp4Chunk& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot&) {
-    u32x4_t a[4];
-#pragma unroll
-    for (int s = 0; s < 4; s++) {  // word by word: a select between two vectors is compiled through memory
-      const u32x4_t& held = ODD ? odd[s] : even[s];
-      a[s] = u32x4_t{mine ? held.x : 0u, mine ? held.y : 0u, mine ? held.z : 0u, mine ? held.w : 0u};
-    }
+    const u32x4_t(&a)[4] = ODD ? odd : even;
     tile(ch.w0, ch.sc.x, a, acc0);
     __builtin_amdgcn_sched_barrier(0);  // a tile at a time: interleaving the four costs more registers than there are
     tile(ch.w1, ch.sc.y, a, acc1);

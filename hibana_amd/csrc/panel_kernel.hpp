@@ -414,12 +414,15 @@ inline size_t panel_lds_bytes(int mt, int ks, int nbw) {
 }
 
 
-// Routed calls: a plan's slots of up to 128 rows, as many row tiles as the slot's rows need.
+// Routed calls: a plan's slots of up to 128 rows, as many row tiles as the slot's rows need. Workgroups go to the eight
+// compute dies in turn: all of a slot's take the same place in that turn, so that its activations come into one L2 once
+// (2048 rows, 22 of 512 experts, (1024, 2688): the latent block 811 -> 782 us; 1543 rows of the three-bit layer 285 -> 276).
 template <class Fmt, int EPI>
 __global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_tile_kernel(StreamParams p) {
   extern __shared__ __align__(16) uint8_t panel_lds[];
-  const int slot = blockIdx.x / p.panel_groups;
-  const PanelShare part{(int)blockIdx.x - slot * p.panel_groups, 0, 1, 0};
+  const int die = blockIdx.x & 7, local = blockIdx.x >> 3, round = local / p.panel_groups, slot = 8 * round + die;
+  if (slot >= p.panel_full) return;
+  const PanelShare part{local - round * p.panel_groups, 0, 1, 0};
   const Slot sl = slot_of<EPI>(p, slot);
   if (sl.rows <= 0) return;  // a slot the plan did not fill: the whole workgroup leaves
   auto run = [&](auto panel) { panel.run(p, sl, panel_lds, part); };
@@ -569,8 +572,10 @@ static int launch_panel_routed(StreamParams& p, int64_t slots, int64_t a_rows, h
   p.slot_rows = PANEL_SLOT_ROWS;
   p.panel_groups = (p.n_blocks + p.nbw - 1) / p.nbw;
   p.a_bytes = (uint32_t)(a_rows * p.a_stride * 2);
-  if (!panel_takes(a_rows, p.a_stride) || slots * p.panel_groups > 0x7fffffff) return HB_EINVAL;
-  HB_LAUNCH((panel_tile_kernel<Fmt, EPI>), dim3((unsigned)(slots * p.panel_groups)), dim3(64 * p.ks * p.nbw), panel_lds_bytes<Fmt>(PANEL_SLOT_ROWS / 16, p.ks, p.nbw), stream, p);
+  p.panel_full = (int)slots;
+  const int64_t grid = (slots + 7) / 8 * 8 * p.panel_groups;
+  if (!panel_takes(a_rows, p.a_stride) || grid > 0x7fffffff) return HB_EINVAL;
+  HB_LAUNCH((panel_tile_kernel<Fmt, EPI>), dim3((unsigned)grid), dim3(64 * p.ks * p.nbw), panel_lds_bytes<Fmt>(PANEL_SLOT_ROWS / 16, p.ks, p.nbw), stream, p);
   return HB_OK;
 }
 

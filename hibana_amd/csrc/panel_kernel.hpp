@@ -27,6 +27,7 @@ namespace hb {
 constexpr int PANEL_HALF = 64;       // k of a half chunk
 constexpr int PANEL_WAVES = 8;       // at most, a workgroup
 constexpr int PANEL_LDS = 160 * 1024;
+constexpr int PANEL_MT = 8;          // row tiles of a slot, at most
 
 // The fewest blocks of a workgroup whose splits' activations fit the LDS beside the weights (PANEL_WAVES wavefronts).
 constexpr int panel_least_blocks(int mt) { return mt <= 4 ? 1 : mt <= 6 ? 2 : 4; }
@@ -385,8 +386,7 @@ struct Panel {
   }
 };
 
-// Dense calls: every slot has up to 16 MT rows. Tile by tile, a slot's blocks one after the other (they share its
-// activations); the tiles past p.panel_full have their K shared by p.panel_kz workgroups each.
+// Dense calls: every slot has up to 16 MT rows. The tiles past p.panel_full have their K shared by p.panel_kz workgroups each.
 template <class Fmt, int EPI, int MT>
 __global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_kernel(StreamParams p) {
   extern __shared__ __align__(16) uint8_t panel_lds[];
@@ -399,8 +399,12 @@ __global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_kernel(StreamParams
     part.kz = p.panel_kz;
     tile = p.panel_full + part.shared_tile;
   }
-  const int slot = tile / p.panel_groups;
-  part.group = tile - slot * p.panel_groups;
+  // Workgroups go to the eight compute dies in turn; a die's take neighbouring runs of blocks, all slots of a run one after
+  // the other, so that a run's weights come into one L2 once (25600 x 5120: 2048 rows 476 -> 453 us, 512 rows 133 -> 122).
+  const int even = p.panel_full & ~7;
+  if (tile < even) tile = (tile & 7) * (even >> 3) + (tile >> 3);
+  part.group = tile / p.panel_slots;
+  const int slot = tile - part.group * p.panel_slots;
   const Slot sl = slot_of<EPI>(p, slot);
   if (sl.rows <= 0) return;
   Panel<Fmt, EPI, MT> panel;
@@ -454,15 +458,21 @@ inline size_t panel_room(const PanelPlan& q) { return q.kz > 1 ? PANEL_TICKET_BY
 // columns, K 512 .. 5120, 17 .. 2048 rows; the cut it takes is within 2.4 % of the best measured one on average): a chunk of
 // a wavefront takes 1.45 + 0.16 mt with two wavefronts a SIMD and 0.7 + 0.1 mt alone; a workgroup's start and end 4.6;
 // eight-wavefront workgroups run one a compute unit, four-wavefront ones two where their LDS allows; the last arriver of
-// a shared tile reads its partial results at about 46 GB/s and the handing over costs 5.3. `room`: bytes of the workspace.
+// a shared tile reads its partial results at about 46 GB/s and the handing over costs 5.3; all shared tiles' results together
+// are written and read at about 2 TB/s (left out, 1024 rows of 25600 x 5120 shared 288 tiles five ways: 318 us, 243
+// without). `room`: bytes of the workspace.
 template <class Fmt>
 inline PanelPlan search_panel(int m, int n_blocks, int chunks, size_t room) {
   static const struct { int ks, nbw; } shapes[] = {{1, 4}, {1, 8}, {2, 2}, {2, 4}, {4, 1}, {4, 2}, {8, 1}};
   PanelPlan best{};
   best.us = 1e30;
   const int least = (m + 127) / 128;
-  for (int slots = least; slots <= least + 1; slots++) {
-    const int mt = ((m + slots - 1) / slots + 15) / 16;
+  // A call that fills the device takes the fewest slots its rows allow, or one more (the rows dealt out evenly); a smaller
+  // one may be faster in many slots of few row tiles (1024 x 512, 1024 rows: 14.7 us in eight slots, 7.1 in more; 4096 x 1024, 512 rows 18.6 and 10.2).
+  const bool small = (int64_t)n_blocks * least <= 512;
+  for (int mt = PANEL_MT; mt >= 1; mt--) {
+    const int slots = (m + 16 * mt - 1) / (16 * mt);
+    if (mt != ((m + least - 1) / least + 15) / 16 && mt != ((m + least) / (least + 1) + 15) / 16 && !(small && slots > least)) continue;
     const double pair = 1.45 + Fmt::EXPAND_US + 0.16 * mt, alone = 0.7 + 0.5 * Fmt::EXPAND_US + 0.105 * mt;
     for (auto& shape : shapes) {
       const size_t lds = panel_lds_bytes<Fmt>(mt, shape.ks, shape.nbw);
@@ -482,7 +492,8 @@ inline PanelPlan search_panel(int m, int n_blocks, int chunks, size_t room) {
         PanelPlan q{mt, slots, shape.ks, shape.nbw, (int)groups, kz, full, tiles, 0};
         if (panel_room(q) > room) continue;
         q.us = rounds(full, (chunks + shape.ks - 1) / shape.ks);
-        if (rest) q.us += rounds(rest * kz, ((chunks + kz - 1) / kz + shape.ks - 1) / shape.ks) + (kz > 1 ? 5.3 + kz * (double)mt * shape.nbw * 4096 / 46e3 : 0);
+        const double shared_tile = kz > 1 ? kz * (double)mt * shape.nbw * 4096 : 0;  // bytes of partial results
+        if (rest) q.us += rounds(rest * kz, ((chunks + kz - 1) / kz + shape.ks - 1) / shape.ks) + (kz > 1 ? 5.3 + shared_tile / 46e3 + rest * shared_tile / 2e6 : 0);
         if (q.us < best.us * (kz > 1 ? 0.97 : 1.0)) best = q;
       }
     }
@@ -543,6 +554,7 @@ static int launch_panel(StreamParams& p, void* workspace, size_t workspace_bytes
   p.slot_rows = 16 * q.mt;
   p.a_bytes = (uint32_t)((int64_t)p.m * p.a_stride * 2);
   p.panel_groups = q.groups;
+  p.panel_slots = (int)(q.tiles / q.groups);
   p.panel_full = (int)q.full;
   p.panel_kz = q.kz;
   p.panel_tickets = static_cast<uint32_t*>(workspace) + PLAN_HEADER;

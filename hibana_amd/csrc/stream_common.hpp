@@ -55,7 +55,7 @@ struct StreamParams {
   float* partial;         // panel kernel, K shared among workgroups: their partial results ...
   uint32_t* panel_tickets; // ... and the shared tiles' arrival counters (in the caller's workspace: zero between calls)
   uint32_t a_bytes;       // panel kernel: bytes of the activation matrix (under 4 GiB)
-  int panel_groups, panel_full, panel_kz;  // panel kernel: runs of blocks a slot; the tiles below panel_full are a workgroup's each, the others' K is shared by panel_kz (routed calls: panel_full slots)
+  int panel_groups, panel_slots, panel_full, panel_kz;  // panel kernel: runs of blocks a slot; the dense call's slots; the tiles below panel_full are a workgroup's each, the others' K is shared by panel_kz (routed calls: panel_full slots)
   int64_t* trace;         // measurement hook (hb_debug_trace): a record a workgroup, else null
   int64_t trace_records;  // ... and the records it holds
   int32_t* done;          // fc1 and fc2 in one launch: the slots' arrival counters (plan_done), else null

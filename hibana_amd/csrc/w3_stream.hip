@@ -336,16 +336,16 @@ __device__ __forceinline__ void compute_tile_few8(const C& w, const long a[4], c
   acc.w = fmaf(part.w, xs.w * s, acc.w);
 }
 
-template <class C>
+template <int T0 = 0, int T1 = 4, class C>  // the 16-row tiles T0 .. T1 - 1 of the block
 __device__ __forceinline__ void compute_few8(const C& ch, long a, const f32x4_t& xs, int grp, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2,
                                              f32x4_t& acc3, uint32_t lut_lo, uint32_t lut_hi, uint32_t q8) {
   long rows[4];  // MFMA j's A operand: the lane's codes in its own group, zero in the others
 #pragma unroll
   for (int j = 0; j < 4; j++) rows[j] = grp == j ? a : 0L;
-  compute_tile_few8<0>(ch, rows, xs, acc0, lut_lo, lut_hi, q8);
-  compute_tile_few8<1>(ch, rows, xs, acc1, lut_lo, lut_hi, q8);
-  compute_tile_few8<2>(ch, rows, xs, acc2, lut_lo, lut_hi, q8);
-  compute_tile_few8<3>(ch, rows, xs, acc3, lut_lo, lut_hi, q8);
+  if (T0 <= 0 && 0 < T1) compute_tile_few8<0>(ch, rows, xs, acc0, lut_lo, lut_hi, q8);
+  if (T0 <= 1 && 1 < T1) compute_tile_few8<1>(ch, rows, xs, acc1, lut_lo, lut_hi, q8);
+  if (T0 <= 2 && 2 < T1) compute_tile_few8<2>(ch, rows, xs, acc2, lut_lo, lut_hi, q8);
+  if (T0 <= 3 && 3 < T1) compute_tile_few8<3>(ch, rows, xs, acc3, lut_lo, lut_hi, q8);
 }
 
 // `a`: the lane's sixteen activation bytes of the chunk (row r16 % 4 of the slot, the k range of group r16 / 4 that this
@@ -439,6 +439,16 @@ struct FewActs8 {  // E4M3 activations: eight codes a lane and chunk, and the sc
   template <int ODD, bool MORE2, bool MORE1, class C>
   __device__ __forceinline__ void step(const C& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot& sl) {
     compute_few8(ch, held[ODD], scale[ODD], grp, acc0, acc1, acc2, acc3, sl.lut_lo, sl.lut_hi, q8);
+    if (MORE2) load(ODD, i + 2);
+  }
+};
+
+// FewActs8 over the 16-row tiles T0 .. T1 - 1 of the block only (the other accumulators stay zero).
+template <int T0, int T1>
+struct FewActs8Part : FewActs8 {
+  template <int ODD, bool MORE2, bool MORE1, class C>
+  __device__ __forceinline__ void step(const C& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot& sl) {
+    compute_few8<T0, T1>(ch, held[ODD], scale[ODD], grp, acc0, acc1, acc2, acc3, sl.lut_lo, sl.lut_hi, q8);
     if (MORE2) load(ODD, i + 2);
   }
 };
@@ -616,7 +626,7 @@ struct FullActs8 {
 template <int EPI, bool QUANT = false, bool SCALED = false, bool PLANES = false>  // SCALED: the sums are of the two-plane activations and take their row's scale; PLANES: registers 2, 3 hold the lower plane of rows 0, 1
 __device__ __forceinline__ void finish_few(const StreamParams& p, const Slot& sl, int row0, float scale, int nb, bool active, int wave, int ks,
                                            int nbi, float* partial, const f32x4_t& acc0, const f32x4_t& acc1, const f32x4_t& acc2,
-                                           const f32x4_t& acc3, const FewPairs& pairs = FewPairs{}, const FewScales& xs = FewScales{}) {
+                                           const f32x4_t& acc3, const FewPairs& pairs = FewPairs{}, const FewScales& xs = FewScales{}, int t0 = 0, int t1 = 4) {
   constexpr int STRIDE = RING_BYTES / 4;
   const int lane = threadIdx.x & 63, q = lane >> 4, r16 = lane & 15;
   float* mine = partial + wave * STRIDE;
@@ -633,7 +643,7 @@ __device__ __forceinline__ void finish_few(const StreamParams& p, const Slot& sl
   } else {
     __builtin_amdgcn_wave_barrier();  // the lanes of one wavefront: its LDS operations execute in program order
   }
-  if (!active) return;
+  if (!active || q < t0 || q >= t1) return;  // (fewer than all four tiles: dense calls, which exchange nothing between lanes below)
   const float* first = partial + nbi * p.ks * STRIDE + r16;
   const int rows = min(PLANES ? PLANE_ROWS : FEW_ROWS, sl.rows - row0);
   for (int r = ks; r < rows; r += p.ks) {
@@ -737,6 +747,40 @@ __global__ __launch_bounds__(1024) void w3_stream_kernel(StreamParams p) {
   const Slot sl = slot_of<EPI>(p, blockIdx.y);
   if (sl.rows <= 0) return;  // a slot the plan did not fill: the whole workgroup leaves
   stream_workgroup<EPI, A8, SPLIT, W3RingOf<2, BITS>>(p, sl, blockIdx.x, rings);
+}
+
+// A dense call of at most four rows whose blocks are fewer than half the compute units: PARTS workgroups a 64-row block,
+// each its 4 / PARTS 16-row tiles (of the block's loads it asks only for those with its tiles' dwords, and the ones that two
+// parts need come from the L2 the second time: a block's workgroups are on one die). The sums and their order are those of
+// the one workgroup. What bounds the undivided launch is the expansion on a third of the device.
+template <bool A8, int T0, int T1>
+__device__ __forceinline__ void part_block(const StreamParams& p, const Slot& sl, int nb, const WaveShare& share, int lane, int wave, uint8_t* rings) {
+  f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0, acc2 = acc0, acc3 = acc0;
+  const float scale = sl.rs[nb * 64 + lane];
+  uint8_t* ring = rings + wave * RING_BYTES;
+  if constexpr (A8) {
+    stream_block<EPI_DENSE, FewActs8Part<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+  } else {
+    stream_block<EPI_DENSE, FewActsPart<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+  }
+  finish_few<EPI_DENSE>(p, sl, 0, scale, nb, true, wave, share.ks, 0, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3, FewPairs{}, FewScales{}, T0, T1);
+}
+template <bool A8, int PARTS>
+__global__ __launch_bounds__(1024) void w3_part_kernel(StreamParams p) {
+  extern __shared__ __align__(16) uint8_t rings[];
+  const int die = blockIdx.x & 7, local = blockIdx.x >> 3, part = local % PARTS, nb = local / PARTS * 8 + die;
+  if (nb >= p.n_blocks) return;
+  const Slot sl = slot_of<EPI_DENSE>(p, 0);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const WaveShare share = wave_share(p, wave);
+  if constexpr (PARTS == 2) {
+    if (part == 0) part_block<A8, 0, 2>(p, sl, nb, share, lane, wave, rings); else part_block<A8, 2, 4>(p, sl, nb, share, lane, wave, rings);
+  } else {
+    if (part == 0) part_block<A8, 0, 1>(p, sl, nb, share, lane, wave, rings);
+    else if (part == 1) part_block<A8, 1, 2>(p, sl, nb, share, lane, wave, rings);
+    else if (part == 2) part_block<A8, 2, 3>(p, sl, nb, share, lane, wave, rings);
+    else part_block<A8, 3, 4>(p, sl, nb, share, lane, wave, rings);
+  }
 }
 
 // One token from its router logits: fc1 with the routing inside it, so that the call has no launch for routing and plan.
@@ -1007,9 +1051,9 @@ struct TileW3 {
 
 // A dense call: the stream's passes (one a sixteen rows) run side by side while their blocks do not fill the device, and the
 // few rows of a second pass are nearly free. Measured, stream and panel: 5120 x 5120 (80 blocks) 48 rows 10.9 and 15.0 us,
-// 77 rows 16.9 and 17.4, 128 rows 23.7 and 19.4; 8192 x 2048 32 rows 7.6 and 8.8, 48 rows 9.8 and 9.0; 51200 x 2048 17 rows
+// 64 rows 16.3 and 14.2, 128 rows 22.6 and 16.8; 8192 x 2048 32 rows 7.6 and 8.8, 48 rows 9.8 and 9.0; 51200 x 2048 17 rows
 // 20.6 and 20.3, 48 rows 30.7 and 22.8; 51200 x 5120 128 rows 195 and 70.
-constexpr int PANEL_W3_ROWS = 20, PANEL_W3_BLOCKS = 384;
+constexpr int PANEL_W3_ROWS = 20, PANEL_W3_BLOCKS = 300;
 
 // ---------------------------------------------------------------------------------------------------- host side
 struct Tuning {  // hb_tune's knobs: relaxed atomics, so a knob set from one thread while another launches is a plain race-free read
@@ -1037,9 +1081,26 @@ static int shape_stream(StreamParams& p, int64_t busy_slots, Launch want) {
   return HB_OK;
 }
 
+// Blocks up to which a dense call of at most four rows gives a block's tiles to two workgroups (up to half of them: to
+// four). 5120 x 5120 at one row 7.7 -> 6.4 us; the dense block at four rows (its down projection is 5120 x 25600) 50.5 -> 46.7.
+constexpr int PARTS_BLOCKS = 128;
 template <int EPI>
 static int launch_stream(StreamParams& p, int64_t slots, int64_t busy_slots, Launch want, hipStream_t stream, int bits = 3) {
   if (int e = shape_stream(p, busy_slots, want)) return e;
+  if constexpr (EPI == EPI_DENSE) {
+    if (bits == 3 && p.m <= FEW_ROWS && p.n_blocks <= PARTS_BLOCKS && !want.ks && !want.nbw && !p.no_few && !p.a2) {
+      p.nbw = 1;
+      const int parts = p.n_blocks <= PARTS_BLOCKS / 2 ? 4 : 2;
+      const dim3 blocks((unsigned)((p.n_blocks + 7) / 8 * 8 * parts));
+      auto launch = [&](auto kernel) { HB_LAUNCH(kernel, blocks, dim3(64 * p.ks), (size_t)p.ks * RING_BYTES, stream, p); };
+      if (p.aq) {
+        parts == 4 ? launch(w3_part_kernel<true, 4>) : launch(w3_part_kernel<true, 2>);
+      } else {
+        parts == 4 ? launch(w3_part_kernel<false, 4>) : launch(w3_part_kernel<false, 2>);
+      }
+      return HB_OK;
+    }
+  }
   const dim3 grid((unsigned)((p.n_blocks + p.nbw - 1) / p.nbw), (unsigned)slots);
   const int waves = p.ks * p.nbw;
   const size_t lds = (size_t)waves * RING_BYTES;

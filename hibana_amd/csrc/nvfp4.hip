@@ -614,7 +614,7 @@ extern "C" size_t hb_nvfp4_gemm_workspace_bytes(int m, int n, int k) {
 
 extern "C" size_t hb_nvfp4_gemm_room_bytes(int m, int n, int k) {
   if (m <= ROWS_PER_SLOT || n <= 0 || k <= 0 || n % 64 || k % 128) return 0;
-  return panel_room(plan_panel<TileNvfp4>(m, n / 64, k / 128, ~(size_t)0));
+  return panel_room(plan_panel<TileNvfp4>(m, n / 64, k / 128, PANEL_ANY_ROOM));
 }
 
 extern "C" int hb_nvfp4_gemm_ws(const void* x, int m, const void* tiled, float global_scale, int n, int k, int relu2, void* y, void* workspace,

@@ -501,7 +501,9 @@ inline PanelPlan search_panel(int m, int n_blocks, int chunks, size_t room) {
   return best;
 }
 
-// ... kept for the sizes a thread asks for again and again (the search takes microseconds).
+// ... kept for the sizes a thread asks for again and again (the search takes microseconds; the best cut of all and the one
+// for a smaller room have places of their own).
+constexpr size_t PANEL_ANY_ROOM = ~(size_t)0;
 template <class Fmt>
 inline const PanelPlan& plan_panel(int m, int n_blocks, int chunks, size_t room) {
   struct Entry {
@@ -510,7 +512,7 @@ inline const PanelPlan& plan_panel(int m, int n_blocks, int chunks, size_t room)
     PanelPlan plan;
   };
   static thread_local Entry kept[64];
-  Entry& e = kept[((unsigned)m * 31u + (unsigned)n_blocks * 7u + (unsigned)chunks + (room ? 13u : 0u)) & 63u];
+  Entry& e = kept[((unsigned)m * 31u + (unsigned)n_blocks * 7u + (unsigned)chunks + (room == PANEL_ANY_ROOM ? 13u : room ? 29u : 0u)) & 63u];
   if (e.m != m || e.n_blocks != n_blocks || e.chunks != chunks || e.room != room) e = Entry{m, n_blocks, chunks, room, search_panel<Fmt>(m, n_blocks, chunks, room)};
   return e.plan;
 }
@@ -530,7 +532,8 @@ struct PanelForce {
 template <class Fmt, int EPI>
 static int launch_panel(StreamParams& p, void* workspace, size_t workspace_bytes, const PanelForce& force, hipStream_t stream) {
   const size_t room = workspace ? workspace_bytes : 0;
-  PanelPlan q = plan_panel<Fmt>(p.m, p.n_blocks, p.chunks, room);
+  PanelPlan q = plan_panel<Fmt>(p.m, p.n_blocks, p.chunks, room ? PANEL_ANY_ROOM : 0);
+  if (panel_room(q) > room) q = plan_panel<Fmt>(p.m, p.n_blocks, p.chunks, room);
   if (force.ks || force.kz) {
     PanelPlan f = q;
     if (force.ks) {

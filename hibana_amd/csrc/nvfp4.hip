@@ -303,65 +303,60 @@ __device__ __forceinline__ void add_lanes(f32x4_t& acc, int distance) {
 
 // ------------------------------------------------------------------------------------------------ slots of more rows
 //
-// MT 16-row tiles of activations against every weight, which is expanded once, its block scale multiplied in, and used MT
-// times. Lane (q, r16) feeds row 16 t + r16 of tile t, k 8 q .. + 7 of a step: a chunk's 4 x MT pieces rest in registers, and
-// each is asked for again, for the next chunk, as soon as its products are issued - straight from the L2: a wavefront
-// shares them with nobody and meets no barrier. The requests of a wavefront come back in order, so the next weights are
-// asked for BEHIND those pieces (a piece that waited behind weights from memory would wait for them too): a block is on
-// its way for the whole of the chunk before it.
-template <int MT>
-struct Fp4Wide {
-  f32x4_t acc[MT][4];
-  u32x4_t a[4][MT];
-  uint32_t at[MT];  // the lane's piece of step 0 of the wavefront's first chunk: byte offset from the matrix (the launch keeps it under 4 GiB)
-  const uint8_t* x;
-  __device__ __forceinline__ u32x4_t piece(int t, int i, int s) const { return *reinterpret_cast<const u32x4_t*>(x + (size_t)i * 256 + 64 * s + at[t]); }
-  template <int EPI>
+// Nine to sixteen rows: every weight is expanded with its block scale multiplied in. Lane (q, r16) feeds row r16, k 8 q ..
+// + 7 of a step: a chunk's four pieces rest in registers, and each is asked for again, for the next chunk, as soon as its
+// products are issued - straight from the L2: a wavefront shares them with nobody and meets no barrier. The requests of a
+// wavefront come back in order, so the next weights are asked for BEHIND those pieces (a piece that waited behind weights
+// from memory would wait for them too): a block is on its way for the whole of the chunk before it.
+//
+// The body serves matrices past 4 GiB too, which the panel kernel does not take: a lane's 32-bit byte offset counts from the
+// slot's first row (a uniform base: 2048 x 2048 at nine rows 8.6 us against 9.0 with a pointer a lane), and where the
+// slot's rows are gathered, which may lie anywhere, the lane holds a whole pointer.
+template <int EPI>
+struct Fp4Full {
+  f32x4_t acc[4];
+  u32x4_t a[4];
+  const uint8_t* x;  // step 0 of the wavefront's first chunk: of the slot's first row (the same for all lanes) or, gathered, the lane's own piece ...
+  uint32_t at;       // ... and from there to the lane's piece
+  __device__ __forceinline__ u32x4_t piece(int i, int s) const { return *reinterpret_cast<const u32x4_t*>(x + (size_t)i * 256 + 64 * s + at); }
   __device__ __forceinline__ void start(const StreamParams& p, const Slot& sl, int c0, int lane) {
-    x = reinterpret_cast<const uint8_t*>(p.a) + (size_t)c0 * 256;
-#pragma unroll
-    for (int t = 0; t < MT; t++) {
-      at[t] = (uint32_t)(activation_row_index<EPI>(p, sl, 16 * t + (lane & 15)) * p.a_stride) * 2 + 16 * (lane >> 4);
-#pragma unroll
-      for (int nt = 0; nt < 4; nt++) acc[t][nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int r16 = lane & 15;
+    if constexpr (epi_gathers(EPI)) {
+      x = reinterpret_cast<const uint8_t*>(activation_row<EPI>(p, sl, r16) + (int64_t)c0 * 128 + 8 * (lane >> 4));
+      at = 0;
+    } else {
+      x = reinterpret_cast<const uint8_t*>(p.a + (int64_t)sl.p0 * p.a_stride + (int64_t)c0 * 128);
+      at = (uint32_t)(min(r16, sl.rows - 1) * p.a_stride) * 2 + 16 * (lane >> 4);
     }
 #pragma unroll
-    for (int s = 0; s < 4; s++)
+    for (int nt = 0; nt < 4; nt++) acc[nt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int t = 0; t < MT; t++) a[s][t] = piece(t, 0, s);
+    for (int s = 0; s < 4; s++) a[s] = piece(0, s);
   }
   template <int J>  // fragment J = 4 * step + tile of a chunk
   static __device__ __forceinline__ bf16x8_t fragment(const Fp4Chunk& ch) { return fp4_scaled(ch.tile(J & 3)[J >> 2], fp4_scale<(J >> 2)>(ch.sc[J & 3])); }
-  // The products of fragment J, and beside them, an instruction or a few behind each product, the expansion of the next
-  // fragment: a product holds the matrix core for sixteen cycles and the issue port for about seven of them.
+  // The product of fragment J, and behind it the expansion of the next fragment: a product holds the matrix core for
+  // sixteen cycles and the issue port for about seven of them.
   template <int J>
   __device__ __forceinline__ void fragments(const Fp4Chunk& ch, int i, bool more, bf16x8_t b) {
     if constexpr (J < 16) {
       constexpr int S = J >> 2, NT = J & 3;
       bf16x8_t next{};
       if constexpr (J < 15) next = fragment<J + 1>(ch);
-#pragma unroll
-      for (int t = 0; t < MT; t++) acc[t][NT] = fp4_mfma(a[S][t], b, acc[t][NT]);
-#pragma unroll
-      for (int t = 0; t < MT; t++) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, (17 + MT - 1) / MT, 0);
-      }
+      acc[NT] = fp4_mfma(a[S], b, acc[NT]);
+      __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x002, 17, 0);
       if (NT == 3) {
         u32x4_t held = __builtin_bit_cast(u32x4_t, next);
-        asm volatile("" : "+v"(held));  // expanded here, beside the products, not behind the branch
+        asm volatile("" : "+v"(held));  // expanded here, beside the product, not behind the branch
         next = __builtin_bit_cast(bf16x8_t, held);
       }
       __builtin_amdgcn_sched_barrier(0);
-      if (NT == 3 && more) {  // uniform
-#pragma unroll
-        for (int t = 0; t < MT; t++) a[S][t] = piece(t, i + 1, S);
-      }
+      if (NT == 3 && more) a[S] = piece(i + 1, S);  // uniform
       fragments<J + 1>(ch, i, more, next);
     }
   }
   // One loop body for every chunk: the ring's slot by its parity, what is still to come by uniform branches.
-  template <int EPI>
   __device__ __forceinline__ void run(const StreamParams& p, const Slot& sl, int nb, int c0, int c1, int lane, uint8_t* ring) {
     const int n = c1 - c0;
     RingSource src;
@@ -371,16 +366,16 @@ struct Fp4Wide {
     Fp4Ring::lanes(src, lane, lane & 15, (uint32_t)(uintptr_t)slot0, codes, scales);
     Fp4Ring::request(src, c0, slot0);
     asm volatile("" ::: "memory");
-    start<EPI>(p, sl, c0, lane);
+    start(p, sl, c0, lane);
     asm volatile("" ::: "memory");
     if (n > 1) Fp4Ring::request(src, c0 + 1, slot0 + NVFP4_BLOCK_BYTES);
     for (int i = 0; i < n; i++) {
       const uint32_t slot = (i & 1) * NVFP4_BLOCK_BYTES;
       Fp4Chunk ch;
       if (i + 1 < n) {
-        Fp4Ring::take<4 * MT + Fp4Ring::LOADS, 0>(ch, codes + slot, scales + slot);
+        Fp4Ring::take<4 + Fp4Ring::LOADS, 0>(ch, codes + slot, scales + slot);
       } else {
-        Fp4Ring::take<4 * MT, 0>(ch, codes + slot, scales + slot);
+        Fp4Ring::take<4, 0>(ch, codes + slot, scales + slot);
       }
       fragments<0>(ch, i, i + 1 < n, fragment<0>(ch));
       if (i + 2 < n) Fp4Ring::request(src, c0 + i + 2, slot0 + slot);
@@ -417,12 +412,12 @@ __device__ __forceinline__ void nvfp4_workgroup(const StreamParams& p, int slot,
       add_lanes(acc2, 32);
       add_lanes(acc3, 32);
     } else {
-      Fp4Wide<1> wide;
-      wide.run<EPI>(p, sl, nb, share.c0, share.c1, lane, ring);
-      acc0 = wide.acc[0][0];
-      acc1 = wide.acc[0][1];
-      acc2 = wide.acc[0][2];
-      acc3 = wide.acc[0][3];
+      Fp4Full<EPI> full;
+      full.run(p, sl, nb, share.c0, share.c1, lane, ring);
+      acc0 = full.acc[0];
+      acc1 = full.acc[1];
+      acc2 = full.acc[2];
+      acc3 = full.acc[3];
     }
   }
   finish_block<EPI, false, FP4_RING_BYTES / 4>(p, sl, RowScales{}, nb, active, ks, nbi, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3);

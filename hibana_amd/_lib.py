@@ -59,6 +59,8 @@ SIGNATURES = {
     "hb_w3_gemm_e4m3": (_I, [_P, _P, _I, _P, _P, _L, _I, _I, _I, _P, _P]),
     "hb_w3_moe_workspace_bytes": (_Z, [_I, _I, _EX, _I]),
     "hb_w3_moe": (_I, [_EX, _P, _P, _P, _I, _I, _I, _P, _P, _Z, _P]),
+    "hb_w3_moe_among": (_I, [_EX, _I, _P, _P, _P, _I, _I, _I, _P, _P, _Z, _P]),
+    "hb_w3_moe_layer_among": (_I, [_EX, _I, _EX, _P, _P, _P, _P, _I, _I, _P, _P, _Z, _P]),
     "hb_w3_moe_layer": (_I, [_EX, _EX, _P, _P, _P, _P, _I, _I, _P, _P, _Z, _P]),
     "hb_w3_moe_layer_static": (_I, [_EX, _EX, _P, _P, _P, _P, _I, _I, _P, _P]),
     "hb_w3_moe_layer_e4m3": (_I, [_EX, _EX, _P, _P, _P, _P, _I, _I, _P, _P, _Z, _P]),
@@ -87,6 +89,7 @@ SIGNATURES = {
     "hb_nvfp4_gemm_ws": (_I, [_P, _I, _P, _F, _I, _I, _I, _P, _P, _Z, _P]),
     "hb_nvfp4_moe_workspace_bytes": (_Z, [_I, _I, _EX4]),
     "hb_nvfp4_moe": (_I, [_EX4, _P, _P, _P, _I, _I, _I, _P, _P, _Z, _P]),
+    "hb_nvfp4_moe_among": (_I, [_EX4, _I, _P, _P, _P, _I, _I, _I, _P, _P, _Z, _P]),
     "hb_latent_workspace_bytes": (_Z, [_LW, _I, _I]),
     "hb_latent_router": (_I, [_LW, _P, _I, _I, _P, _I, _I, _I, _P, _P, _P, _P, _P, _Z, _P]),
     "hb_latent_block": (_I, [_LW, _P, _P, _P, _P, _I, _I, _I, _P, _P, _Z, _P]),

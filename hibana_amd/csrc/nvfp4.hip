@@ -668,14 +668,18 @@ int64_t busy_slots(int64_t pairs, int experts, int64_t slots) { return pairs < 2
 
 // plan -> fc1 -> fc2: `out_pairs` receives fc2's per-pair outputs.
 int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, int m, int topk, const MoeWorkspace& ws, void* out_pairs,
-                int pairs_bf16, hipStream_t stream) {
-  const int64_t pairs = (int64_t)m * topk;
+                int pairs_bf16, hipStream_t stream, int experts_total) {
+  const int64_t pairs = (int64_t)m * topk, named = experts_named(experts_total, ex->base, ex->experts);
   // A dense contraction once an expert sees about ten rows: slots of 128 rows on the panel kernel; below that the 16-row
   // slots of the weight stream. Measured, stream and panel, the whole latent block in us: 512 experts (1024, 2688) 8 rows an
   // expert 384 and 388, 12 rows 474 and 403, 24 rows 748 and 455; 256 experts (768, 1536) 8 rows 121 and 123, 10 rows 131 and
-  // 126, 24 rows 212 and 146; 128 experts (512, 1024) 10 rows 71 and 72, 24 rows 82 and 72.
+  // 126, 24 rows 212 and 146; 128 experts (512, 1024) 10 rows 71 and 72, 24 rows 82 and 72. A range of the experts sees its
+  // share of the pairs only, and the stream's launches, sized for all of them, lose a little earlier: 64 of 512 experts
+  // (1024, 2688), the summed experts alone, 4 rows an expert 59 and 68, 8 rows 86 and 76; 256 of 512 8 rows 196 and 198, 11 rows
+  // 218 and 204; 32 of 256 (768, 1536) 8 rows 39 and 40, 16 rows 50 and 44.
+  const int64_t rows_min = ex->experts < named ? 8 : 10;
   const bool dense = panel_takes(m, ex->hidden) && panel_takes(pairs, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
-                     (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && pairs >= 10ll * ex->experts));
+                     (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && pairs >= rows_min * named));
   const int slot_rows = dense ? PANEL_SLOT_ROWS : ROWS_PER_SLOT;
   const int64_t slots = moe_max_slots(pairs, ex->experts, 0, slot_rows);
   if (slots > 65535) return HB_EINVAL;
@@ -754,6 +758,11 @@ extern "C" size_t hb_nvfp4_moe_workspace_bytes(int m, int topk, const hb_nvfp4_e
 
 extern "C" int hb_nvfp4_moe(const hb_nvfp4_experts* routed, const void* x, const int32_t* ids, const float* weights, int m, int topk, int mode,
                             void* out, void* workspace, size_t workspace_bytes, void* stream) {
+  return hb_nvfp4_moe_among(routed, 0, x, ids, weights, m, topk, mode, out, workspace, workspace_bytes, stream);
+}
+
+extern "C" int hb_nvfp4_moe_among(const hb_nvfp4_experts* routed, int experts_total, const void* x, const int32_t* ids, const float* weights, int m,
+                                  int topk, int mode, void* out, void* workspace, size_t workspace_bytes, void* stream) {
   if (int e = check_experts(routed)) return e;
   if (!x || !ids || !weights || !out || !workspace) return HB_ENULL;
   if (m <= 0 || topk <= 0 || mode < HB_MOE_SUM || mode > HB_MOE_PAIRS_BF16) return HB_EINVAL;
@@ -765,7 +774,7 @@ extern "C" int hb_nvfp4_moe(const hb_nvfp4_experts* routed, const void* x, const
   // a summed prefill-sized call keeps its pair outputs in BF16: half the traffic of its widest tensor, as the reference's
   // layer does from the same size (hibana/model/flashnext/moe.py:186)
   const bool narrow = sum && m >= MOE_WIDE_ROWS;
-  if (int e = run_experts(routed, x, ids, m, topk, ws, pairs_out, mode == HB_MOE_PAIRS_BF16 || narrow, as_stream(stream))) return e;
+  if (int e = run_experts(routed, x, ids, m, topk, ws, pairs_out, mode == HB_MOE_PAIRS_BF16 || narrow, as_stream(stream), experts_total)) return e;
   if (sum) {
     CombineParams c{};
     c.pairs = ws.y;

@@ -3,6 +3,7 @@
 // LDS, and the host-side helpers of a routed call (workspace, plan launch, combine launch).
 #pragma once
 
+#include <algorithm>
 #include <hip/hip_ext.h>
 
 #include "common.hpp"
@@ -533,6 +534,10 @@ void moe_launch_quant_rows(const uint16_t* x, int64_t m, int k, uint8_t* q, floa
 int moe_check_route(int m, int e, int k);  // HB_EINVAL for a row the routing wavefront cannot hold
 
 // A routed call whose experts are chosen under a budget (route_budget.hpp): BF16 logits [m, e] and the rule's settings.
+// The experts a routed call's ids are drawn from, as far as is known: what the caller says (0: nothing), at least up to
+// the end of the range held here. Its pairs spread over these, so the range sees experts / experts_named of them, and the
+// rows an expert that choose a call's kernels are pairs / experts_named.
+inline int64_t experts_named(int experts_total, int base, int experts) { return std::max<int64_t>(experts_total, (int64_t)base + experts); }
 struct BudgetRoute {
   const uint16_t* logits;
   int e, keep, budget, steps, repeat, per_request, min_cap;

@@ -1239,9 +1239,9 @@ struct Routing {  // set: the chain routes the logits itself into the caller's i
 };
 
 int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void* x, const int32_t* ids, int m, int topk,
-                const MoeWorkspace& ws, void* out_pairs, int pairs_bf16, hipStream_t stream, const Routing* route = nullptr,
+                const MoeWorkspace& ws, void* out_pairs, int pairs_bf16, hipStream_t stream, int experts_total, const Routing* route = nullptr,
                 bool e4m3 = false, const CombineParams* combine = nullptr) {
-  const int64_t pairs = (int64_t)m * topk;
+  const int64_t pairs = (int64_t)m * topk, named = experts_named(experts_total, ex->base, ex->experts);
   const int shared_rows = shared ? m : 0;
   // A dense contraction once an expert sees a few dozen rows: slots of 128 rows on the panel kernel (E4M3 activations: the
   // stream only). The stream pays for a pass a sixteen rows, the panel for an expansion the few rows do not amortise and for
@@ -1249,10 +1249,11 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   // experts (2048, 512) 12 rows an expert 235 and 267, 16 rows 288 and 277, 30 rows 439 and 311 (skewed routing 16 rows 248
   // and 208); 256 experts (2560, 768) 12 rows 224 and 235, 16 rows 292 and 250; 128 experts (2048, 512) 20 rows (0.98 M
   // pairs x blocks) 111 and 120, 24 rows (1.2 M) 123 and 123; 128 experts (1024, 256) 24 rows (0.3 M) 70 and 83, 48 rows 98
-  // and 100, 96 rows 132 and 100.
+  // and 100, 96 rows 132 and 100. A range of the experts sees its share of the pairs only: 64 of 512 (2048, 512), the summed
+  // experts alone, 5 rows an expert 44 and 53, 16 rows 72 and 72, 31 rows 98 and 90; 256 of 512 12 rows 116 and 138, 20 rows 179 and 157.
   const int64_t expert_blocks = (int64_t)((ex->gated ? 2 : 1) * ex->inter / W3_BLOCK_ROWS) * (ex->hidden / W3_CHUNK) + (int64_t)(ex->hidden_out / W3_BLOCK_ROWS) * (ex->inter / W3_CHUNK);
   const bool dense = !e4m3 && panel_takes(m, ex->hidden) && panel_takes(pairs + shared_rows, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
-                     (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && (pairs >= 48ll * ex->experts || (pairs >= 16ll * ex->experts && pairs * expert_blocks >= 1000000))));
+                     (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && (pairs >= 48 * named || (pairs >= 16 * named && pairs * expert_blocks >= 1000000))));
   const int slot_rows = dense ? PANEL_SLOT_ROWS : ROWS_PER_SLOT;
   const int64_t slots = moe_max_slots(pairs, ex->experts, shared_rows, slot_rows);
   if (slots > 65535) return HB_EINVAL;
@@ -1465,6 +1466,11 @@ extern "C" int hb_debug_workspace_layout(int m, int topk, const hb_w3_experts* r
 
 extern "C" int hb_w3_moe(const hb_w3_experts* routed, const void* x, const int32_t* ids, const float* weights, int m, int topk, int mode,
                          void* out, void* workspace, size_t workspace_bytes, void* stream) {
+  return hb_w3_moe_among(routed, 0, x, ids, weights, m, topk, mode, out, workspace, workspace_bytes, stream);
+}
+
+extern "C" int hb_w3_moe_among(const hb_w3_experts* routed, int experts_total, const void* x, const int32_t* ids, const float* weights, int m, int topk,
+                               int mode, void* out, void* workspace, size_t workspace_bytes, void* stream) {
   if (int e = check_experts(routed)) return e;
   if (!x || !ids || !weights || !out || !workspace) return HB_ENULL;
   const bool e4m3 = (mode & HB_MOE_E4M3) != 0;
@@ -1486,13 +1492,13 @@ extern "C" int hb_w3_moe(const hb_w3_experts* routed, const void* x, const int32
   c.topk = topk;
   c.h = routed->hidden_out;
   c.out = static_cast<uint16_t*>(out);
-  return run_experts(routed, nullptr, x, ids, m, topk, ws, pairs_out, mode == HB_MOE_PAIRS_BF16 || narrow, as_stream(stream), nullptr, e4m3,
+  return run_experts(routed, nullptr, x, ids, m, topk, ws, pairs_out, mode == HB_MOE_PAIRS_BF16 || narrow, as_stream(stream), experts_total, nullptr, e4m3,
                      mode == HB_MOE_SUM ? &c : nullptr);
 }
 
 static int moe_layer(const hb_w3_experts* routed, const hb_w3_experts* shared, const float* gate_vec, const void* x, const int32_t* ids,
                      const float* weights, int m, int topk, void* out, void* workspace, size_t workspace_bytes, void* stream,
-                     const Routing* route, bool e4m3 = false) {
+                     int experts_total, const Routing* route, bool e4m3 = false) {
   if (int e = check_experts(routed)) return e;
   if (shared) {
     if (int e = check_experts(shared)) return e;
@@ -1528,19 +1534,25 @@ static int moe_layer(const hb_w3_experts* routed, const hb_w3_experts* shared, c
   c.topk = topk;
   c.h = routed->hidden_out;
   c.out = static_cast<uint16_t*>(out);
-  return run_experts(routed, shared, x, ids, m, topk, ws, ws.y, narrow, as_stream(stream), route, e4m3, &c);
+  return run_experts(routed, shared, x, ids, m, topk, ws, ws.y, narrow, as_stream(stream), experts_total, route, e4m3, &c);
 }
 
 extern "C" int hb_w3_moe_layer(const hb_w3_experts* routed, const hb_w3_experts* shared, const float* gate_vec, const void* x,
                                const int32_t* ids, const float* weights, int m, int topk, void* out, void* workspace,
                                size_t workspace_bytes, void* stream) {
-  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, nullptr);
+  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, 0, nullptr);
+}
+
+extern "C" int hb_w3_moe_layer_among(const hb_w3_experts* routed, int experts_total, const hb_w3_experts* shared, const float* gate_vec, const void* x,
+                                     const int32_t* ids, const float* weights, int m, int topk, void* out, void* workspace,
+                                     size_t workspace_bytes, void* stream) {
+  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, experts_total, nullptr);
 }
 
 extern "C" int hb_w3_moe_layer_e4m3(const hb_w3_experts* routed, const hb_w3_experts* shared, const float* gate_vec, const void* x,
                                     const int32_t* ids, const float* weights, int m, int topk, void* out, void* workspace,
                                     size_t workspace_bytes, void* stream) {
-  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, nullptr, true);
+  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, 0, nullptr, true);
 }
 
 // ------------------------------------------------------------------------------- the entry point that allocates nothing
@@ -1578,7 +1590,7 @@ extern "C" int hb_w3_moe_layer_static(const hb_w3_experts* routed, const hb_w3_e
     return HB_ESCRATCH;
   void* ptr = scratch_of_current_device();
   if (!ptr) return HB_ELAUNCH;
-  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, ptr, HB_STATIC_SCRATCH_BYTES, stream, nullptr);
+  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, ptr, HB_STATIC_SCRATCH_BYTES, stream, 0, nullptr);
 }
 
 // ------------------------------------------------------------------------------------- a workspace's head words
@@ -1616,7 +1628,7 @@ extern "C" int hb_w3_moe_layer_logits(const hb_w3_experts* routed, const hb_w3_e
   if (!logits) return HB_ENULL;
   if (!aligned(logits, 4)) return HB_EINVAL;
   const Routing route{{logits, 0, experts_total, nullptr, 1}, ids, weights};
-  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, &route);
+  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, experts_total, &route);
 }
 
 extern "C" int hb_w3_moe_layer_budget(const hb_w3_experts* routed, const hb_w3_experts* shared, const float* gate_vec, const void* x,
@@ -1626,7 +1638,7 @@ extern "C" int hb_w3_moe_layer_budget(const hb_w3_experts* routed, const hb_w3_e
   if (!logits) return HB_ENULL;
   const BudgetRoute b{static_cast<const uint16_t*>(logits), experts_total, keep, budget, steps, 0, per_request, min_cap, slots};
   const Routing route{{}, ids, weights, &b};
-  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, &route);
+  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, experts_total, &route);
 }
 
 extern "C" int hb_w3_moe_layer_logits_e4m3(const hb_w3_experts* routed, const hb_w3_experts* shared, const float* gate_vec, const void* x,
@@ -1635,7 +1647,7 @@ extern "C" int hb_w3_moe_layer_logits_e4m3(const hb_w3_experts* routed, const hb
   if (!logits) return HB_ENULL;
   if (!aligned(logits, 4)) return HB_EINVAL;
   const Routing route{{logits, 0, experts_total, nullptr, 1}, ids, weights};
-  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, &route, true);
+  return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, experts_total, &route, true);
 }
 
 // The layer from its input rows: [workspace of the routed call][BF16 logits][ids][weights].
@@ -1686,5 +1698,5 @@ extern "C" int hb_w3_moe_layer_rows(const hb_w3_experts* routed, const hb_w3_exp
   }
   const BudgetRoute b{lg, experts_total, keep, budget, steps, 0, per_request, min_cap, slots};
   const Routing route{{lg, 1, experts_total, slots, steps}, l.ids, l.weights, budget > 0 ? &b : nullptr};
-  return moe_layer(routed, shared, gate_vec, x, l.ids, l.weights, m, topk, out, workspace, l.moe, stream, &route);
+  return moe_layer(routed, shared, gate_vec, x, l.ids, l.weights, m, topk, out, workspace, l.moe, stream, experts_total, &route);
 }

@@ -66,9 +66,12 @@ class B12xExperts:
         return _lib.HbNvfp4Experts(_lib.ptr(self.tiled1), _lib.ptr(self.alpha1), _lib.ptr(self.tiled2), _lib.ptr(self.alpha2),
                                    self.experts, self.base, self.k, self.n, self.out_features, int(self.gated))
 
-    def __call__(self, x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, pairs: bool = False) -> torch.Tensor:
+    def __call__(self, x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, pairs: bool = False,
+                 experts_total: int = 0) -> torch.Tensor:
         """BF16 x [M, K], ids / weights [M, k] -> BF16 [M, K_out], the weighted routed sum in selection order
-        (hibana/kernels/b12x_moe.py:58-68). With `pairs`, the FP32 outputs per (row, k) pair [M * k, K_out], unsummed."""
+        (hibana/kernels/b12x_moe.py:58-68). With `pairs`, the FP32 outputs per (row, k) pair [M * k, K_out], unsummed.
+        `experts_total`: how many experts the ids are drawn from where these are a range of them (0: not known); it only
+        chooses between kernels, by the pairs the range can expect."""
         if x.dtype != torch.bfloat16 or x.ndim != 2 or x.shape[1] != self.k:
             raise ValueError("B12xExperts: x must be BF16 [M, K]")
         if ids.ndim != 2 or ids.shape[0] != x.shape[0] or weights.shape != ids.shape:
@@ -85,6 +88,6 @@ class B12xExperts:
         ids32 = ids.to(torch.int32).contiguous()
         wt = weights.float().contiguous()
         xc = x.contiguous()
-        _lib.check(_lib.lib().hb_nvfp4_moe(C.byref(st), _lib.ptr(xc), _lib.ptr(ids32), _lib.ptr(wt), m, topk, int(pairs),
-                                           _lib.ptr(out), _lib.ptr(ws), need, _lib.stream()), "nvfp4 experts")
+        _lib.check(_lib.lib().hb_nvfp4_moe_among(C.byref(st), experts_total, _lib.ptr(xc), _lib.ptr(ids32), _lib.ptr(wt), m, topk, int(pairs),
+                                                 _lib.ptr(out), _lib.ptr(ws), need, _lib.stream()), "nvfp4 experts")
         return out

@@ -170,4 +170,4 @@ def w3_block(x: torch.Tensor, ws: Workspace, lat: torch.Tensor, ids: torch.Tenso
     shared expert's down -> BF16 [M, H] (hibana/kernels/nemotron_moe.py:63-68)."""
     from hibana_amd.kernels.w3_moe import w3_moe
     shared_up(x, ws, weights)
-    return out(x, ws, w3_moe(experts, lat, ids, wts), weights)
+    return out(x, ws, w3_moe(experts, lat, ids, wts, experts_total=weights.experts_total), weights)

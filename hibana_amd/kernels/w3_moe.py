@@ -156,13 +156,15 @@ MOE_E4M3 = 16  # hb_w3_moe mode flag: activations through the reference's E4M3 r
 
 
 def w3_moe(experts: W3Experts, x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, pairs: bool = False,
-           pairs_bf16: bool = False, e4m3: bool = False) -> torch.Tensor:
+           pairs_bf16: bool = False, e4m3: bool = False, experts_total: int = 0) -> torch.Tensor:
     """Routed experts for x [M, H] BF16 with the router's ids [M, k] and weights [M, k] -> BF16 [M, H_out], the
     weighted sum in selection order (no shared expert). An id outside this object's range base .. base + E - 1 (another
     rank's expert, or the "no expert" id 512) adds nothing. With `pairs`, the FP32 (`pairs_bf16`: BF16) output of each
     (row, k) pair [M * k, H_out], unsummed; rows of skipped pairs are unspecified
     (hibana/kernels/w3_moe.py:158-179). `e4m3`: x and h are rounded to E4M3 per (row, 32-group) before their products, as
-    the reference kernel does (its torch statement: hibana/kernels/w3_moe.py:193-214); default: weight-only."""
+    the reference kernel does (its torch statement: hibana/kernels/w3_moe.py:193-214); default: weight-only.
+    `experts_total`: how many experts the ids are drawn from where this object holds a range of them (0: not known); it
+    only chooses between kernels, by the pairs the range can expect."""
     _check_call(experts, x, ids, weights)
     m, k = ids.shape
     h_out = experts.shape2[0]
@@ -178,17 +180,17 @@ def w3_moe(experts: W3Experts, x: torch.Tensor, ids: torch.Tensor, weights: torc
     wt = weights.float().contiguous()
     mode |= MOE_E4M3 if e4m3 else 0
     xc = x.contiguous()  # converted operands keep a name until the launch is enqueued
-    _lib.check(_lib.lib().hb_w3_moe(C.byref(st), _lib.ptr(xc), _lib.ptr(ids32), _lib.ptr(wt), m, k, mode, _lib.ptr(out),
-                                    _lib.ptr(ws), need, _lib.stream()), "w3_moe")
+    _lib.check(_lib.lib().hb_w3_moe_among(C.byref(st), experts_total, _lib.ptr(xc), _lib.ptr(ids32), _lib.ptr(wt), m, k, mode, _lib.ptr(out),
+                                          _lib.ptr(ws), need, _lib.stream()), "w3_moe")
     return out
 
 
 def moe_layer(experts: W3Experts, x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor, shared: W3Experts | None = None,
-              gate_vec: torch.Tensor | None = None, e4m3: bool = False) -> torch.Tensor:
+              gate_vec: torch.Tensor | None = None, e4m3: bool = False, experts_total: int = 0) -> torch.Tensor:
     """The MoE layer on 3-bit weights in one chain of launches: routed sum + the shared expert (`shared`: a one-expert
     W3Experts of the same geometry) combined as bf16(bf16(routed) + g * bf16(shared)), g = sigmoid(x . gate_vec) or 1
     (hibana/model/flashnext/moe.py:177-192). `e4m3`: x and h of every expert are rounded to E4M3 per (row, 32-group)
-    before their products, as in `w3_moe`."""
+    before their products, as in `w3_moe`; `experts_total` as there."""
     _check_call(experts, x, ids, weights)
     m, k = ids.shape
     out = torch.empty((m, experts.shape2[0]), dtype=torch.bfloat16, device=x.device)
@@ -201,10 +203,11 @@ def moe_layer(experts: W3Experts, x: torch.Tensor, ids: torch.Tensor, weights: t
     ids32 = ids.to(torch.int32).contiguous()
     wt = weights.float().contiguous()
     gv = None if gate_vec is None else gate_vec.float().contiguous()
-    entry = _lib.lib().hb_w3_moe_layer_e4m3 if e4m3 else _lib.lib().hb_w3_moe_layer
     xc = x.contiguous()
-    _lib.check(entry(C.byref(st), C.byref(sh) if sh is not None else None, _lib.ptr(gv), _lib.ptr(xc),
-                     _lib.ptr(ids32), _lib.ptr(wt), m, k, _lib.ptr(out), _lib.ptr(ws), need, _lib.stream()), "moe_layer")
+    args = (C.byref(sh) if sh is not None else None, _lib.ptr(gv), _lib.ptr(xc), _lib.ptr(ids32), _lib.ptr(wt), m, k, _lib.ptr(out), _lib.ptr(ws), need,
+            _lib.stream())
+    code = _lib.lib().hb_w3_moe_layer_e4m3(C.byref(st), *args) if e4m3 else _lib.lib().hb_w3_moe_layer_among(C.byref(st), experts_total, *args)
+    _lib.check(code, "moe_layer")
     return out
 
 

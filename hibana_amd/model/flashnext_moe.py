@@ -119,7 +119,7 @@ class MoeLayer:
 
     def routed(self, x: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor) -> torch.Tensor:
         """The routed experts' weighted sum (this rank's part) for x [M, H] -> BF16 [M, H]."""
-        return w3_moe.w3_moe(self.w3, x, ids, weights)
+        return w3_moe.w3_moe(self.w3, x, ids, weights, experts_total=self.experts)
 
     def shared_on_linears(self, m: int) -> bool:
         """Whether a call of `m` rows runs the shared expert on its own linears: the reference does, and takes their 3-bit
@@ -137,7 +137,7 @@ class MoeLayer:
             # the reference's own chain: the experts' unsummed pair outputs (BF16 from WIDE_ROWS rows), the shared expert
             # on its linears (silu(gate) * up in between), the combine over both
             ids, weights = self.route(x, ctx)
-            pairs = w3_moe.w3_moe(self.w3, x, ids, weights, pairs=True, pairs_bf16=x.shape[0] >= w3_moe.WIDE_ROWS)
+            pairs = w3_moe.w3_moe(self.w3, x, ids, weights, pairs=True, pairs_bf16=x.shape[0] >= w3_moe.WIDE_ROWS, experts_total=self.experts)
             shared = ops.nvfp4_linear(ops.silu_and_mul(ops.nvfp4_linear(x, self.shared_gate_up)), self.shared_down)
             return ops.moe_combine_pairs(pairs, ids, weights, shared, x, self.shared_gate_vec, self.w3.base, self.w3.experts)
         # router product, routing (or the budgeted selection), plan, both streams and the combine as one chain

@@ -120,7 +120,7 @@ class NemotronMoe:
         self.hidden = gate_fc1.shape[1]
         self.w3 = experts if isinstance(experts, W3Experts) else None
         self.b12x = experts if isinstance(experts, B12xExperts) else None
-        self.experts_op = (lambda lat, ids, w: w3_moe(self.w3, lat, ids, w)) if self.w3 is not None else experts
+        self.experts_op = (lambda lat, ids, w: w3_moe(self.w3, lat, ids, w, experts_total=self.experts)) if self.w3 is not None else experts
         self._small = None
 
     def small_weights(self) -> small_block.SmallWeights:
@@ -163,6 +163,8 @@ class NemotronMoe:
         return route_topk(fused, self.bias, self.topk, self.latent, slots, steps, repeat)
 
     def routed(self, latent: torch.Tensor, ids: torch.Tensor, weights: torch.Tensor) -> torch.Tensor:
+        if type(self.experts_op) is B12xExperts:  # these may be a rank's range of the experts the ids name
+            return self.experts_op(latent, ids, weights, experts_total=self.experts)
         return self.experts_op(latent, ids, weights)
 
     def shared(self, x: torch.Tensor) -> torch.Tensor:

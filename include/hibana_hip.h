@@ -237,6 +237,13 @@ int hb_debug_workspace_layout(int m, int topk, const hb_w3_experts* routed, int 
 int hb_w3_moe(const hb_w3_experts* routed, const void* x, const int32_t* ids, const float* weights, int m, int topk,
               int mode, void* out, void* workspace, size_t workspace_bytes, void* stream);
 
+/* hb_w3_moe where the experts held here are a range of those the ids name: `experts_total` of them in all (0: not known; then
+ * taken as base + experts). The same results to rounding; the number only chooses between kernels, by the pairs that the
+ * range can expect (without it a rank that holds the first experts is taken to hold all).
+ * No counterpart in the reference (its kernels do not change with the pairs an expert). */
+int hb_w3_moe_among(const hb_w3_experts* routed, int experts_total, const void* x, const int32_t* ids, const float* weights,
+                    int m, int topk, int mode, void* out, void* workspace, size_t workspace_bytes, void* stream);
+
 /* The whole MoE layer on 3-bit weights: routed sum + shared expert (a one-expert hb_w3_experts, may be NULL) +
  * combine: out = bf16( bf16(routed) + g * bf16(shared) ), g = sigmoid(x . gate_vec) or 1 when gate_vec is NULL
  * (float32 [hidden]).
@@ -245,6 +252,11 @@ int hb_w3_moe(const hb_w3_experts* routed, const void* x, const int32_t* ids, co
 int hb_w3_moe_layer(const hb_w3_experts* routed, const hb_w3_experts* shared, const float* gate_vec, const void* x,
                     const int32_t* ids, const float* weights, int m, int topk, void* out, void* workspace,
                     size_t workspace_bytes, void* stream);
+
+/* ... of a range of `experts_total` experts, as in hb_w3_moe_among (the forms from logits or rows know the total). */
+int hb_w3_moe_layer_among(const hb_w3_experts* routed, int experts_total, const hb_w3_experts* shared, const float* gate_vec,
+                          const void* x, const int32_t* ids, const float* weights, int m, int topk, void* out,
+                          void* workspace, size_t workspace_bytes, void* stream);
 
 /* hb_w3_moe_layer for callers that cannot allocate device memory or carry a workspace (code under HIP graph capture,
  * tight serving loops, harnesses that forbid hipMalloc): the same chain of launches and the same bits, with the plan, the
@@ -461,6 +473,10 @@ size_t hb_nvfp4_moe_workspace_bytes(int m, int topk, const hb_nvfp4_experts* rou
  * tests/nemotron_reference.py:568-593. */
 int hb_nvfp4_moe(const hb_nvfp4_experts* routed, const void* x, const int32_t* ids, const float* weights, int m,
                  int topk, int mode, void* out, void* workspace, size_t workspace_bytes, void* stream);
+
+/* ... of a range of `experts_total` experts, as in hb_w3_moe_among. */
+int hb_nvfp4_moe_among(const hb_nvfp4_experts* routed, int experts_total, const void* x, const int32_t* ids, const float* weights,
+                       int m, int topk, int mode, void* out, void* workspace, size_t workspace_bytes, void* stream);
 
 /* ------------------------------------------------------------------------------------------------------------------
  * The latent-MoE block of a decode / verify call (at most HB_LATENT_MAX_ROWS rows), the native surface of the

@@ -571,20 +571,32 @@ extern "C" int hb_nvfp4_dequant(const void* tiled, float global_scale, int64_t r
   return launch_status();
 }
 
-// `workspace`: room for partial tiles (hb_nvfp4_gemm_workspace_bytes), or null: no call shares K among workgroups.
+// The weight stream passes over the matrix once for every sixteen rows; the panel kernel expands it once for 128, and is the
+// faster one past sixteen rows except where K is long, the blocks are few and its cut gives no tile's K to several
+// workgroups: the stream splits K sixteen ways in a workgroup where the panel has eight, and its passes run side by side as
+// long as all of them fit the device at once. Measured, stream and panel, us: 2048 x 5120 17 rows 13.2 and 15.4, 64 rows 13.0
+// and 15.2; 5120 x 5120 (80 blocks) 48 rows (240 workgroups) 13.8 and 15.7, 64 rows (320) 22.3 and 13.6; 512 x 3072 (24 chunks)
+// 33 rows 10.0 and 10.9, 64 rows 11.2 and 10.8; 512 x 12800 17 rows 23.2 and, with K shared, 13.4, without 33.2.
+constexpr int STREAM_LONG_CHUNKS = 32, STREAM_PASSES_WORKGROUPS = 256;
+static bool stream_serves(int m, int n_blocks, int chunks, const PanelPlan& cut) {
+  return cut.kz == 1 && chunks >= STREAM_LONG_CHUNKS && (int64_t)n_blocks * ((m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT) <= STREAM_PASSES_WORKGROUPS;
+}
+static PanelForce nvfp4_force() { return PanelForce{g_nvfp4_ksplit, g_nvfp4_nbw, g_nvfp4_tile_ks}; }
+
+// `workspace`: room for partial tiles (hb_nvfp4_gemm_room_bytes), or null: no call shares K among workgroups.
 static int nvfp4_gemm(const void* x, int m, const void* tiled, float global_scale, int n, int k, int relu2, void* y, void* workspace, size_t workspace_bytes,
                       hipStream_t stream) {
   if (!x || !tiled || !y) return HB_ENULL;
   if (m <= 0 || n <= 0 || k <= 0 || n % 64 || k % 128) return HB_EINVAL;
   if (!aligned(x, 16) || !aligned(tiled, 16) || !aligned(y, 2) || !aligned(workspace, 16)) return HB_EINVAL;
   StreamParams p = dense_params(tiled, global_scale, n, k, x, m, y);
-  // the weight stream would pass over the matrix once for every sixteen rows; the panel kernel expands it once for 128
   if (panel_takes(m, k) && panel_writes(y, false) && (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && m > ROWS_PER_SLOT))) {
-    const PanelForce force{g_nvfp4_ksplit, g_nvfp4_nbw, g_nvfp4_tile_ks};
-    if (int e = relu2 ? launch_panel<TileNvfp4, EPI_DENSE_RELU2>(p, workspace, workspace_bytes, force, stream)
-                      : launch_panel<TileNvfp4, EPI_DENSE>(p, workspace, workspace_bytes, force, stream))
-      return e;
-    return launch_status();
+    const PanelForce force = nvfp4_force();
+    const PanelPlan cut = cut_panel<TileNvfp4>(m, p.n_blocks, p.chunks, workspace ? workspace_bytes : 0, force);
+    if (g_nvfp4_tile == 1 || force.ks || force.kz || !stream_serves(m, p.n_blocks, p.chunks, cut)) {
+      if (int e = relu2 ? launch_panel<TileNvfp4, EPI_DENSE_RELU2>(p, cut, workspace, stream) : launch_panel<TileNvfp4, EPI_DENSE>(p, cut, workspace, stream)) return e;
+      return launch_status();
+    }
   }
   const int64_t slots = (m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT;
   if (slots > 65535) return HB_EINVAL;

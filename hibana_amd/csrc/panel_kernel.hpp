@@ -528,26 +528,31 @@ struct PanelForce {
   int ks, nbw, kz;
 };
 
-// A dense call of p.m rows; `workspace`: room for shared tiles' partial results, or null (no tile's K is shared).
-template <class Fmt, int EPI>
-static int launch_panel(StreamParams& p, void* workspace, size_t workspace_bytes, const PanelForce& force, hipStream_t stream) {
-  const size_t room = workspace ? workspace_bytes : 0;
-  PanelPlan q = plan_panel<Fmt>(p.m, p.n_blocks, p.chunks, room ? PANEL_ANY_ROOM : 0);
-  if (panel_room(q) > room) q = plan_panel<Fmt>(p.m, p.n_blocks, p.chunks, room);
+// The cut of a dense call that has `room` bytes for shared tiles' partial results (0: no tile's K is shared).
+template <class Fmt>
+static PanelPlan cut_panel(int m, int n_blocks, int chunks, size_t room, const PanelForce& force) {
+  PanelPlan q = plan_panel<Fmt>(m, n_blocks, chunks, room ? PANEL_ANY_ROOM : 0);
+  if (panel_room(q) > room) q = plan_panel<Fmt>(m, n_blocks, chunks, room);
   if (force.ks || force.kz) {
     PanelPlan f = q;
     if (force.ks) {
       f.ks = force.ks;
       f.nbw = std::max(1, force.nbw);
     }
-    f.groups = (p.n_blocks + f.nbw - 1) / f.nbw;
-    f.tiles = (int64_t)f.groups * ((p.m + 16 * f.mt - 1) / (16 * f.mt));
-    f.kz = std::max(1, std::min(force.kz, p.chunks / f.ks));
+    f.groups = (n_blocks + f.nbw - 1) / f.nbw;
+    f.tiles = (int64_t)f.groups * ((m + 16 * f.mt - 1) / (16 * f.mt));
+    f.kz = std::max(1, std::min(force.kz, chunks / f.ks));
     f.full = f.kz > 1 ? 0 : f.tiles;
-    if (f.ks * f.nbw <= PANEL_WAVES && !(f.ks & (f.ks - 1)) && f.ks <= p.chunks / f.kz && f.nbw >= panel_least_blocks(f.mt) && panel_lds_bytes<Fmt>(f.mt, f.ks, f.nbw) <= PANEL_LDS &&
+    if (f.ks * f.nbw <= PANEL_WAVES && !(f.ks & (f.ks - 1)) && f.ks <= chunks / f.kz && f.nbw >= panel_least_blocks(f.mt) && panel_lds_bytes<Fmt>(f.mt, f.ks, f.nbw) <= PANEL_LDS &&
         panel_room(f) <= room && (f.kz == 1 || f.tiles <= PANEL_SHARED_TILES))
       q = f;
   }
+  return q;
+}
+
+// A dense call of p.m rows by the cut `q`; `workspace`: the room that the cut asks for (panel_room).
+template <class Fmt, int EPI>
+static int launch_panel(StreamParams& p, const PanelPlan& q, void* workspace, hipStream_t stream) {
   const size_t lds = panel_lds_bytes<Fmt>(q.mt, q.ks, q.nbw);
   const int64_t grid = q.full + (q.tiles - q.full) * q.kz;
   if (q.us > 1e29 || grid > 0x7fffffff) return HB_EINVAL;

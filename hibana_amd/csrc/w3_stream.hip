@@ -1167,7 +1167,9 @@ extern "C" int hb_w3_gemm(const void* x, int m, const void* tiled, const float* 
   p.out_stride = n;
   if (panel_takes(m, k) && panel_writes(y, false) && (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && m > PANEL_W3_ROWS && (int64_t)p.n_blocks * ((m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT) >= PANEL_W3_BLOCKS))) {
     const PanelForce force{g_tune.w3_ksplit, g_tune.w3_nbw, 0};
-    if (int e = bits == 2 ? launch_panel<TileW3<2>, EPI_DENSE>(p, nullptr, 0, force, as_stream(stream)) : launch_panel<TileW3<3>, EPI_DENSE>(p, nullptr, 0, force, as_stream(stream))) return e;
+    if (int e = bits == 2 ? launch_panel<TileW3<2>, EPI_DENSE>(p, cut_panel<TileW3<2>>(m, p.n_blocks, p.chunks, 0, force), nullptr, as_stream(stream))
+                          : launch_panel<TileW3<3>, EPI_DENSE>(p, cut_panel<TileW3<3>>(m, p.n_blocks, p.chunks, 0, force), nullptr, as_stream(stream)))
+      return e;
     return launch_status();
   }
   const int64_t slots = (m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT;

@@ -51,6 +51,14 @@ class SmallWeights:
         self._struct = None
         self._bytes = {}
 
+    def __getstate__(self):
+        """A copy or a pickle takes the tensors, not the structures of their addresses."""
+        return dict(self.__dict__, _routed=None, _struct=None, _bytes={})
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._routed = None if self.experts is None else self.experts._struct()
+
     def struct(self) -> _lib.HbLatentWeights:
         """The block as the library takes it: assembled once, and again when one of its tensors was replaced."""
         up, down = self.shared_up, self.shared_down

@@ -48,6 +48,10 @@ class W3Experts:
             self.shape13 = (self.planes13.shape[1] * 32, self.planes13.shape[2] * w3.CHUNK)
             self.shape2 = (self.planes2.shape[1] * 32, self.planes2.shape[2] * w3.CHUNK)
 
+    def __getstate__(self):
+        """A copy or a pickle takes the tensors, not the structure of their addresses that `_struct` keeps here."""
+        return {k: v for k, v in self.__dict__.items() if k != "_packed"}
+
     @property
     def experts(self) -> int:
         return self.row13.shape[0]

@@ -294,10 +294,12 @@ def moe_layer_rows(experts: W3Experts, x: torch.Tensor, router: torch.Tensor, to
         raise ValueError("moe_layer_rows: x must be BF16 [M, hidden]")
     if router.dtype != torch.bfloat16 or router.ndim != 2 or router.shape[1] != x.shape[1] or not router.is_contiguous():
         raise ValueError("moe_layer_rows: router must be BF16 [experts, hidden], contiguous")
-    if steps < 1 or m % steps or budget < 0 or (slots is not None and slots.numel() < m // steps):
-        raise ValueError("moe_layer_rows: whole requests of `steps` rows, a slot for every request")
-    if budget and not (20 <= e_total <= 1024 and 1 <= topk <= 20 and 0 <= keep <= 20):
-        raise ValueError("moe_layer_rows: under a budget 20 <= E <= 1024, topk and keep at most 20")
+    if slots is None and not budget:
+        steps = 1  # every row is real: the requests mean nothing
+    if steps < 1 or budget < 0 or (slots is not None and slots.numel() < -(-m // steps)):
+        raise ValueError("moe_layer_rows: a slot for every `steps` rows")
+    if budget and not (20 <= e_total <= 1024 and 1 <= topk <= 20 and 0 <= keep <= 20 and m % steps == 0):
+        raise ValueError("moe_layer_rows: under a budget 20 <= E <= 1024, topk and keep at most 20, whole requests of `steps` rows")
     _lib.need_gpu(x, router, slots)
     out = x.new_empty((m, experts.shape2[0]))
     if m:

@@ -37,3 +37,22 @@ def test_layer_from_rows_is_the_chain_on_its_logits(e, hidden, m):
     ids, weights = ops.route_topk(logits, 6, slots)
     got = w3_moe.moe_layer_rows(ex, x, router, 6, slots=slots, shared=shared, gate_vec=gate)
     assert torch.equal(got, w3_moe.moe_layer(ex, x, ids, weights, shared=shared, gate_vec=gate))
+
+
+@pytest.mark.parametrize("m", [10, 70])  # the router's product in the library and handed in
+def test_verify_forwards_that_are_no_whole_requests(m):
+    """Without slots the requests' length means nothing; with them the last request may be cut short."""
+    from types import SimpleNamespace
+
+    from hibana_amd.kernels import ops, w3_moe
+    from hibana_amd.model.flashnext_moe import MoeLayer
+    ex, shared, x, router, gate = _setup(30, 1152, m, 900)
+    layer = MoeLayer(router, gate, ex, 6, shared=shared)
+    assert torch.equal(layer(x, SimpleNamespace(mode="verify", seq_slots=None, verify_steps=4)), layer(x))
+    slots = torch.ones(-(-m // 4), dtype=torch.int32, device="cuda")
+    slots[1] = 0
+    ids, weights = ops.route_topk(torch.mm(x, router.T), 6, slots, 4)
+    got = layer(x, SimpleNamespace(mode="verify", seq_slots=slots, verify_steps=4))
+    assert torch.equal(got, w3_moe.moe_layer(ex, x, ids, weights, shared=shared, gate_vec=gate))
+    with pytest.raises(ValueError):
+        layer(x, SimpleNamespace(mode="verify", seq_slots=slots[1:], verify_steps=4))

@@ -1688,7 +1688,7 @@ extern "C" int hb_w3_moe_layer_rows(const hb_w3_experts* routed, const hb_w3_exp
   if (int e = check_experts(routed)) return e;
   if (!x || !workspace || (!router && !logits)) return HB_ENULL;
   if (m <= 0 || topk <= 0 || experts_total <= 0 || steps <= 0) return HB_EINVAL;
-  if (!aligned(x, 16) || !aligned(router, 16) || !aligned(logits, 2) || !aligned(slots, 4) || !aligned(workspace, 16)) return HB_EINVAL;
+  if (!aligned(x, 16) || (!logits && !aligned(router, 16)) || !aligned(logits, 2) || !aligned(slots, 4) || !aligned(workspace, 16)) return HB_EINVAL;
   if (!logits && m > MOE_ROUTER_ROWS) return HB_EINVAL;
   const size_t moe = hb_w3_moe_workspace_bytes(m, topk, routed, shared != nullptr);
   const LayerScratch l = layer_scratch(workspace, moe, m, topk, experts_total);

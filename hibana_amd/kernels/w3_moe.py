@@ -310,7 +310,7 @@ def moe_layer_rows(experts: W3Experts, x: torch.Tensor, router: torch.Tensor, to
         gv = None if gate_vec is None else gate_vec.float().contiguous()
         sl = None if slots is None else slots.to(torch.int32).contiguous()
         xc = x.contiguous()
-        logits = None if m <= ROUTER_ROWS else torch.mm(xc, router.T)
+        logits = None if m <= ROUTER_ROWS and router.data_ptr() % 16 == 0 else torch.mm(xc, router.T)  # (the library's product reads 16 bytes a lane; a slice of a larger tensor may start anywhere)
         _lib.check(_lib.lib().hb_w3_moe_layer_rows(C.byref(st), sh, _lib.ptr(gv), xc.data_ptr(), router.data_ptr(), _lib.ptr(logits), e_total, m, topk, keep,
                                                    budget, _lib.ptr(sl), steps, per_request, min_cap, out.data_ptr(), ws.data_ptr(), need, _lib.stream()),
                    "moe_layer_rows")

@@ -56,3 +56,13 @@ def test_verify_forwards_that_are_no_whole_requests(m):
     assert torch.equal(got, w3_moe.moe_layer(ex, x, ids, weights, shared=shared, gate_vec=gate))
     with pytest.raises(ValueError):
         layer(x, SimpleNamespace(mode="verify", seq_slots=slots[1:], verify_steps=4))
+
+
+@pytest.mark.parametrize("m", [3, 70])
+def test_a_router_off_the_vector_boundary(m):
+    """A router sliced out of a larger tensor need not start on a 16-byte boundary."""
+    from hibana_amd.model.flashnext_moe import MoeLayer
+    ex, shared, x, router, gate = _setup(30, 256, m, 700)
+    slice_ = torch.cat([router.new_zeros(4), router.flatten()])[4:].view_as(router)
+    assert slice_.data_ptr() % 16 == 8 and slice_.is_contiguous()
+    assert torch.equal(MoeLayer(slice_, gate, ex, 6, shared=shared)(x), MoeLayer(router, gate, ex, 6, shared=shared)(x))

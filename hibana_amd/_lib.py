@@ -126,13 +126,10 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 # The current device and the raw handle of its current stream, without a `torch.cuda.Stream` object around it (0.1 us
-# against 2.9 us a call, and every kernel call asks). A call's tensors are on the GPU, so torch has initialised it.
-current_device = torch._C._cuda_getDevice
-raw_stream = torch._C._cuda_getCurrentRawStream
-
-
+# against 2.9 us a call, and every kernel call asks). A call's tensors are on the GPU, so torch has initialised it. Looked up
+# at the call: a torch without a GPU backend has neither, and the package is imported there too (its host side runs on the CPU).
 def stream() -> int:
-    return raw_stream(current_device())
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 WORKSPACE_ZERO_BYTES = 1 << 20
@@ -146,8 +143,8 @@ def workspace(device: torch.device, need: int, kind: str = "moe") -> torch.Tenso
     another, so they can share it; calls on different streams get different buffers and share nothing. `kind` keeps
     apart calls that are in progress together on one stream (a latent block's workspace lives across several calls,
     among them a routed one)."""
-    index = device.index if device.index is not None else current_device()
-    key = (index, raw_stream(index), kind)
+    index = device.index if device.index is not None else torch._C._cuda_getDevice()
+    key = (index, torch._C._cuda_getCurrentRawStream(index), kind)
     have = _workspaces.get(key)
     if have is None or have.numel() < need:
         have = torch.empty(max(need, 4096), dtype=torch.uint8, device=device)

@@ -608,9 +608,9 @@ extern "C" int hb_nvfp4_gemm(const void* x, int m, const void* tiled, float glob
   return nvfp4_gemm(x, m, tiled, global_scale, n, k, relu2, y, nullptr, 0, as_stream(stream));
 }
 
-// What the entry point has asked of its callers since it was added: room for every tile of four blocks (128 rows) to have
-// its K shared by about four hundred workgroups in all. A call takes the best cut that fits (hb_nvfp4_gemm_room_bytes: the
-// best of all).
+// Kept for callers built against it: room for every tile of four blocks (128 rows) to have its K shared by about four hundred
+// workgroups in all, which no cut needs any more; a call takes the best cut that fits what it is given. New callers ask
+// hb_nvfp4_gemm_room_bytes, which is what the best cut uses.
 extern "C" size_t hb_nvfp4_gemm_workspace_bytes(int m, int n, int k) {
   if (m <= 20 || n <= 0 || k <= 0 || n % 64 || k % 128) return 0;
   const int64_t tiles = (int64_t)((n / 64 + 3) / 4) * ((m + 127) / 128), chunks = k / 128;
@@ -621,7 +621,7 @@ extern "C" size_t hb_nvfp4_gemm_workspace_bytes(int m, int n, int k) {
 
 extern "C" size_t hb_nvfp4_gemm_room_bytes(int m, int n, int k) {
   if (m <= ROWS_PER_SLOT || n <= 0 || k <= 0 || n % 64 || k % 128) return 0;
-  return panel_room(plan_panel<TileNvfp4>(m, n / 64, k / 128, PANEL_ANY_ROOM));
+  return panel_room(cut_panel<TileNvfp4>(m, n / 64, k / 128, PANEL_ANY_ROOM, nvfp4_force()));
 }
 
 extern "C" int hb_nvfp4_gemm_ws(const void* x, int m, const void* tiled, float global_scale, int n, int k, int relu2, void* y, void* workspace,

@@ -1652,7 +1652,7 @@ extern "C" int hb_w3_moe_layer_logits_e4m3(const hb_w3_experts* routed, const hb
   return moe_layer(routed, shared, gate_vec, x, ids, weights, m, topk, out, workspace, workspace_bytes, stream, experts_total, &route, true);
 }
 
-// The layer from its input rows: [workspace of the routed call][BF16 logits][ids][weights].
+// The layer from its input rows: [workspace of the routed call][BF16 logits, where the call makes them][ids][weights].
 namespace {
 struct LayerScratch {
   size_t moe;  // the routed call's bytes
@@ -1669,7 +1669,7 @@ LayerScratch layer_scratch(void* base, size_t moe, int m, int topk, int experts_
     off += (bytes + 255) & ~(size_t)255;
     return ptr;
   };
-  l.logits = static_cast<uint16_t*>(take((size_t)m * experts_total * 2));
+  l.logits = static_cast<uint16_t*>(take(m <= MOE_ROUTER_ROWS ? (size_t)m * experts_total * 2 : 0));
   l.ids = static_cast<int32_t*>(take((size_t)m * topk * 4));
   l.weights = static_cast<float*>(take((size_t)m * topk * 4));
   l.bytes = off;

@@ -32,7 +32,7 @@ def nvfp4_linear(x: torch.Tensor, lin, prequantized=None, relu2: bool = False) -
     if m:
         lib = _lib.lib()
         xc = x.contiguous()  # held until the launch is enqueued: a temporary's block could be handed out again before that
-        need = max(lib.hb_nvfp4_gemm_room_bytes(m, n, k), lib.hb_nvfp4_gemm_workspace_bytes(m, n, k)) if m > 16 else 0  # K shared among workgroups
+        need = lib.hb_nvfp4_gemm_room_bytes(m, n, k) if m > 16 else 0  # where K is shared among workgroups
         ws = _lib.workspace(x.device, need, "gemm") if need else None
         code = lib.hb_nvfp4_gemm_ws(xc.data_ptr(), m, lin.tiled.data_ptr(), lin.scale2, n, k, int(relu2), y.data_ptr(), _lib.ptr(ws), need, _lib.stream())
         if code:

@@ -442,9 +442,10 @@ int hb_nvfp4_gemm(const void* x, int m, const void* tiled, float global_scale, i
 /* The same product with room for partial sums: calls of more than sixteen rows whose tiles do not fill the device share
  * the K of some tiles among workgroups; their partial results meet in `workspace` and whichever workgroup of a tile
  * finishes last adds them in one fixed order: the result does not depend on the schedule. hb_nvfp4_gemm_room_bytes: what
- * the fastest cut of a call of this shape needs (0: none); hb_nvfp4_gemm_workspace_bytes: the room asked of callers since
- * the entry point was added (a call takes the fastest cut that fits what it is given). The tiles' arrival counters lie at
- * its head (zero before the first use, see "Workspaces" above). No counterpart in the reference (cuBLASLt / FlashInfer own their workspaces there). */
+ * the fastest cut of a call of this shape uses (0: none). hb_nvfp4_gemm_workspace_bytes: an older, mostly larger answer, 0 up
+ * to twenty rows, kept for callers built against it; a call takes the fastest cut that fits what it is given. The tiles'
+ * arrival counters lie at its head (zero before the first use, see "Workspaces" above). No counterpart in the reference
+ * (cuBLASLt / FlashInfer own their workspaces there). */
 size_t hb_nvfp4_gemm_room_bytes(int m, int n, int k);
 size_t hb_nvfp4_gemm_workspace_bytes(int m, int n, int k);
 int hb_nvfp4_gemm_ws(const void* x, int m, const void* tiled, float global_scale, int n, int k, int relu2, void* y,

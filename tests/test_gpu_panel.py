@@ -81,3 +81,14 @@ def test_nvfp4_calls_of_several_shapes_share_a_workspace():
             got = ops.nvfp4_linear(x, lin)
             mx, nr = errors(got, ((x.float() @ dense.T) * 0.3).bfloat16())
             assert mx < MAX_REL and nr < NORM_REL, (m, n, k, mx, nr)
+
+
+@pytest.mark.parametrize("m,n,k", [(64, 25600, 1280), (64, 512, 12800)])  # a cut that shares no K, one that does
+def test_nvfp4_linear_holds_the_room_its_cut_uses(m, n, k, monkeypatch):
+    from hibana_amd import _lib, synthetic
+    from hibana_amd.kernels import ops
+    asked, real = [], _lib.workspace
+    monkeypatch.setattr(_lib, "workspace", lambda device, need, kind="moe": asked.append(need) or real(device, need, kind))
+    ops.nvfp4_linear(torch.zeros(m, k, dtype=torch.bfloat16, device="cuda"), synthetic.nvfp4_linear(n, k, 1))
+    room = _lib.lib().hb_nvfp4_gemm_room_bytes(m, n, k)
+    assert asked == ([room] if room else []) and (room > 0) == (k == 12800)

@@ -48,19 +48,25 @@ def test_w3_rows_around_whole_tiles(n, k, codebook):
 
 @pytest.mark.parametrize("m", [20, 21, 48, 77, 128])
 def test_w3_calls_the_library_gives_to_the_panel(m):
-    """n large enough for the built-in choice (24576 rows: 384 blocks) against the weight stream's product of the same call."""
+    """n large enough for the built-in choice (24576 rows: 384 blocks), which is the panel kernel from 21 rows and the weight
+    stream at 20: the two scale and add in different orders, so the bits say which one ran. Either way the product of the
+    dequantized matrix."""
     from hibana_amd import _lib
     from hibana_amd.kernels import w3
     packed, *_ = random_w3(24576, 256, 3, "lloyd")
     dev = to_device_w3(packed)
-    x = torch.randn(m, 256, generator=torch.Generator().manual_seed(m)).bfloat16().cuda()
-    got = w3.w3_linear(x, dev)
-    assert _lib.lib().hb_tune(b"w3_tile", 2) == 0
-    try:
-        stream = w3.w3_linear(x, dev)
-    finally:
-        _lib.lib().hb_tune(b"w3_tile", 0)
-    mx, nr = errors(got, stream)
+    x = torch.randn(m, 256, generator=torch.Generator().manual_seed(m)).bfloat16()
+    results = []
+    for tile in (0, 1, 2):
+        assert _lib.lib().hb_tune(b"w3_tile", tile) == 0
+        try:
+            results.append(w3.w3_linear(x.cuda(), dev))
+        finally:
+            _lib.lib().hb_tune(b"w3_tile", 0)
+    got, panel, stream = results
+    assert not torch.equal(panel, stream)
+    assert torch.equal(got, panel if m > 20 else stream)
+    mx, nr = errors(got, layers.dense_ref(x, ow3.dequantize(packed)))
     assert mx < MAX_REL and nr < NORM_REL, (mx, nr)
 
 

@@ -4,11 +4,11 @@
                  logits; 32 tokens with Zipf(1.1) routing. Oracle: the C restatement (oracle/c/w3_oracle.c), which
                  unpacks the experts a call names from the checkpoint layout.
   config 1       NVFP4 dense 25600 x 5120 at M = 64 (and 1, 8): (x unpack^T) * s2 (tests/nemotron_reference.py:236-254
-                 of the reference), on the weight stream and on the tile kernel.
+                 of the reference), on the weight stream and on the panel kernel.
   config 4       NVFP4 latent-MoE block, 2048 tokens, hidden 4096 -> latent 1024, 512 ReLU^2 experts of intermediate
                  2688, top-22: a token's output depends on its own 22 experts only, so the oracle
                  (tests/nemotron_reference.py:568-593 restated) is evaluated on a seeded sample of token rows; through
-                 the tile kernel, the library's own choice and the weight stream.
+                 the panel kernel, the library's own choice and the weight stream.
 
 The 512-expert plan, the slot table at well over a hundred distinct experts, the three-launch plan of 45 056 pairs and
 the stream / tile switch-over run here at the sizes they are built for.
@@ -156,18 +156,23 @@ def test_nvfp4_dense_partial_tiles_do_not_depend_on_what_the_workspace_held(nvfp
     n, k, m = 25600, 5120, 64
     lib = _lib.lib()
     x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).bfloat16().cuda()
-    need = lib.hb_nvfp4_gemm_workspace_bytes(m, n, k)
-    assert need > 0
-    ws = torch.empty(need // 4, dtype=torch.float32, device="cuda")
-    y = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
-    first = None
-    for _ in range(12):
-        ws.fill_(float("nan"))
-        _lib.check(lib.hb_workspace_reset(_lib.ptr(ws), need, _lib.stream()), "reset")  # the head (the tiles' arrival counters) starts at zero
-        _lib.check(lib.hb_nvfp4_gemm_ws(_lib.ptr(x), m, _lib.ptr(lin.tiled), lin.global_scale, n, k, 0, _lib.ptr(y), _lib.ptr(ws), need, _lib.stream()), "gemm")
-        if first is None:
-            first = y.clone()
-        assert torch.equal(y, first)
+    assert lib.hb_tune(b"nvfp4_tile_ks", 4) == 0  # (the library's own cut of this call shares no tile's K)
+    try:
+        need = lib.hb_nvfp4_gemm_room_bytes(m, n, k)
+        assert need > 100 * 4 * 4 * 4 * 64 * 16  # more than one share of a hundred tiles of a row tile each
+        ws = torch.empty(need // 4, dtype=torch.float32, device="cuda")
+        y = torch.empty(m, n, dtype=torch.bfloat16, device="cuda")
+        first = None
+        for _ in range(12):
+            ws.fill_(float("nan"))
+            _lib.check(lib.hb_workspace_reset(_lib.ptr(ws), need, _lib.stream()), "reset")  # the head (the tiles' arrival counters) starts at zero
+            _lib.check(lib.hb_nvfp4_gemm_ws(_lib.ptr(x), m, _lib.ptr(lin.tiled), lin.global_scale, n, k, 0, _lib.ptr(y), _lib.ptr(ws), need, _lib.stream()), "gemm")
+            if first is None:
+                first = y.clone()
+            assert torch.equal(y, first)
+    finally:
+        lib.hb_tune(b"nvfp4_tile_ks", 0)
+    assert not bool(ws[1 << 18:].isnan().all())  # (behind the head: partial tiles)
     assert lib.hb_tune(b"nvfp4_tile", 2) == 0
     try:
         stream = ops.nvfp4_linear(x, lin)

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(params=["auto", "tile", "stream", "stream16"], autouse=True)
 def kernel_choice(request):
-    """Every case runs with the library's own choice between the 128-row tile kernel and the 16-row weight stream, with
+    """Every case runs with the library's own choice between the panel kernel and the 16-row weight stream, with
     each of them forced, and with the stream's body for slots of at most eight rows switched off (so those slots take the
     sixteen-row body)."""
     from hibana_amd import _lib
@@ -113,7 +113,7 @@ def test_tiles_whose_k_is_shared_among_workgroups(m, ks):
     lib = _lib.lib()
     assert lib.hb_tune(b"nvfp4_tile_ks", ks) == 0
     try:
-        assert (lib.hb_nvfp4_gemm_workspace_bytes(m, n, k) > 0) == (m > 20)  # up to twenty rows the weight stream serves
+        assert (lib.hb_nvfp4_gemm_workspace_bytes(m, n, k) > 0) == (m > 20)  # (the older size: nothing up to twenty rows)
         got = [ops.nvfp4_linear(x.cuda(), lin, relu2=bool(ks & 1)) for _ in range(3)]
     finally:
         lib.hb_tune(b"nvfp4_tile_ks", 0)

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(params=["auto", "tile", "stream", "stream16"], autouse=True)
 def kernel_choice(request):
-    """Every case runs with the library's own choice between the 128-row tile kernel and the 16-row weight stream, with
+    """Every case runs with the library's own choice between the panel kernel and the 16-row weight stream, with
     each of them forced, and with the stream's body for slots of at most eight rows switched off (so those slots take the
     sixteen-row body)."""
     from hibana_amd import _lib

@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 ROWS = [17, 32, 33, 64, 65, 80, 96, 97, 112, 113, 128, 129, 257]
 
 
-@pytest.mark.parametrize("n,k", [(64, 128), (192, 640), (576, 1280)])
+@pytest.mark.parametrize("n,k", [(64, 128), (192, 640), (576, 1280), (320, 6400)])  # the last: K shared among workgroups up to 200 rows
 def test_nvfp4_rows_around_whole_tiles(n, k):
     """Every call on one workspace, whose head the calls before it (other shapes, other cuts) have used and left zero."""
     from hibana_amd.kernels import ops
@@ -73,13 +73,16 @@ def test_w3_calls_the_library_gives_to_the_panel(m):
 def test_nvfp4_calls_of_several_shapes_share_a_workspace():
     """Shared tiles' counters lie at a fixed place of the workspace: calls whose tiles number differently, one after the
     other on a stream, never take another's partial results for counters (a result nobody adds up is never stored)."""
+    from hibana_amd import _lib
     from hibana_amd.kernels import ops
-    shapes = [(5120, 2688), (1024, 512), (2688, 1024), (64, 128), (4096, 1280)]
+    shapes = [(5120, 2688), (512, 12800), (1024, 512), (320, 6400), (2688, 1024), (64, 128), (4096, 1280), (1024, 12800)]
+    rows = (33, 200, 64, 512, 77, 333)
+    assert sum(_lib.lib().hb_nvfp4_gemm_room_bytes(m, n, k) > 0 for m in rows for n, k in shapes) >= 12  # calls that share K, among calls that do not
     mats = []
     for i, (n, k) in enumerate(shapes):
         packed, scales = _matrix(n, k, i, hi=8.0)
         mats.append((_linear(packed, scales, alpha=0.3, inv=1.0), torch.from_numpy(onv.unpack_fp4(packed, scales)).cuda()))
-    for m in (33, 200, 64, 512, 77, 333):
+    for m in rows:
         for (n, k), (lin, dense) in zip(shapes, mats):
             x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).bfloat16().cuda()
             junk = torch.full((m, n), float("nan"), dtype=torch.bfloat16, device="cuda")  # what the result's memory may hold before

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(params=["auto", "tile", "stream", "stream16"], autouse=True)
 def kernel_choice(request):
-    """Every case runs with the library's own choice between the 128-row MFMA tile kernel and the 16-row weight stream,
+    """Every case runs with the library's own choice between the panel kernel and the 16-row weight stream,
     with each of them forced, and with the stream's body for slots of at most four rows switched off (so those slots
     take the sixteen-row body, as they do when the activation matrix is too large for a buffer descriptor)."""
     from hibana_amd import _lib
@@ -62,7 +62,7 @@ def test_two_bit_linear_matches_the_oracle(m, n, k, kernel_choice):
     assert torch.equal(w3.w3_linear(x.cuda(), dev), got)
     wide = w3.tile(to_device_w3(packed), widen=True)
     assert wide.tile_bits == 3
-    if kernel_choice.startswith("stream"):  # the same sums from either layout (the MFMA tile kernel, which serves only three-bit tiles, adds in another order)
+    if kernel_choice.startswith("stream"):  # the same sums from either layout (the panel kernel adds in another order)
         assert torch.equal(w3.w3_linear(x.cuda(), wide), got)
     else:
         mx, nr = errors(w3.w3_linear(x.cuda(), wide), want)

@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.fixture(params=["auto", "tile", "stream", "stream16", "apart", "planes"], autouse=True)
 def kernel_choice(request):
-    """Every case runs with the library's own choice between the 128-row MFMA tile kernel and the 16-row weight stream,
+    """Every case runs with the library's own choice between the panel kernel and the 16-row weight stream,
     with each of them forced, with the stream's body for slots of at most four rows switched off (so those slots
     take the sixteen-row body, as they do when the activation matrix is too large for a buffer descriptor), with fc1
     and fc2 of a call in launches of their own instead of one ("apart"), and with fc1's slots of at most four rows on the

@@ -132,7 +132,7 @@ def test_plan_of_a_prefill_sized_call_three_launches():
     torch.cuda.synchronize()
     st = w3_moe._struct(ex)
     head, entries, slots, order = _read_plan(_lib.workspace(x.device, 0), st, m, topk, False)
-    assert entries[:slots, 2].max() == 128  # the MFMA tile kernel's slots
+    assert entries[:slots, 2].max() == 128  # the panel kernel's slots
     _check_plan(head, entries, slots, order, ids.numpy(), topk, 0, 32, 0, slot_rows=128)
 
 
@@ -181,7 +181,7 @@ def test_a_wait_that_gives_up_is_reported_and_reset_restores_service(small):
     _lib.workspace_reset(None)
 
 
-def test_two_streams_with_workspaces_of_their_own_share_nothing():
+def test_two_streams_with_workspaces_of_their_own_share_nothing(request):
     """Two verify-sized layer calls from logits (routing and plan in one launch: the arrival counter; fc1 and fc2 in one
     launch: the slots' counters) on two ordinary streams at once, and two NVFP4 products of 64 rows (tiles that share K:
     the tiles' counters), many iterations: every result is the serial call's, bit for bit."""
@@ -198,7 +198,9 @@ def test_two_streams_with_workspaces_of_their_own_share_nothing():
         logits = torch.randn(32, 64, generator=g).cuda()
         xd = torch.randn(64, 1024, generator=g).bfloat16().cuda()
         cases.append((x, logits, xd))
-    assert _lib.lib().hb_nvfp4_gemm_workspace_bytes(64, 2048, 1024) > 0
+    assert _lib.lib().hb_tune(b"nvfp4_tile_ks", 3) == 0  # (the library's own cut of this product shares no tile's K)
+    request.addfinalizer(lambda: _lib.lib().hb_tune(b"nvfp4_tile_ks", 0))
+    assert _lib.lib().hb_nvfp4_gemm_room_bytes(64, 2048, 1024) > 0
     serial = [(w3_moe.moe_layer_logits(ex, x, lg, 8, shared=sh).clone(), ops.nvfp4_linear(xd, lin).clone()) for x, lg, xd in cases]
     torch.cuda.synchronize()
     streams = [torch.cuda.Stream(), torch.cuda.Stream()]  # default priority both

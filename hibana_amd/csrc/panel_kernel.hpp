@@ -5,7 +5,7 @@
 // weight once, in registers (Fmt::fragment: scaled BF16, exact), and uses it for MT products. The activations of a
 // half chunk (64 k) lie in LDS, one copy a split, shared by the split's nbw wavefronts: brought by LDS-direct loads as 1 KB
 // pieces of eight rows x 128 contiguous bytes (reading fragments straight from the L2 instead, sixteen rows x 64 bytes a load,
-// runs at 11 B/clk a compute unit: 65 us against PANEL77 at 77 rows, 25600 x 5120), two buffers, a barrier a half chunk. The
+// runs at 11 B/clk a compute unit: 65 us against 32 at 77 rows, 25600 x 5120), two buffers, a barrier a half chunk. The
 // weights of the next chunk wait in a slot of LDS of the wavefront's own.
 //
 // What bounds it is the issue port and the matrix core together: a product holds the core for 16 cycles and the port for
@@ -29,7 +29,9 @@ constexpr int PANEL_WAVES = 8;       // at most, a workgroup
 constexpr int PANEL_LDS = 160 * 1024;
 constexpr int PANEL_MT = 8;          // row tiles of a slot, at most
 
-// The fewest blocks of a workgroup whose splits' activations fit the LDS beside the weights (PANEL_WAVES wavefronts).
+// The fewest blocks of a workgroup. A split's half chunk of activations is 2 mt pieces, brought by the split's wavefronts, one a
+// block, each of which holds its pieces' addresses in registers: eight at most, and four from seven row tiles on, where the
+// accumulators take most of them. (Whether a cut fits the LDS is panel_lds_bytes' to say.)
 constexpr int panel_least_blocks(int mt) { return mt <= 4 ? 1 : mt <= 6 ? 2 : 4; }
 
 // A workgroup's part of the launch: its run of blocks, and where several workgroups share a tile's K (kz > 1), which
@@ -400,7 +402,7 @@ __global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_kernel(StreamParams
     tile = p.panel_full + part.shared_tile;
   }
   // Workgroups go to the eight compute dies in turn; a die's take neighbouring runs of blocks, all slots of a run one after
-  // the other, so that a run's weights come into one L2 once (25600 x 5120: 2048 rows 476 -> 453 us, 512 rows 133 -> 122).
+  // the other, so that a run's weights come into one L2 once (25600 x 5120, four matrices in turn: 2048 rows 436 -> 422 us, 512 rows 142 -> 126).
   const int even = p.panel_full & ~7;
   if (tile < even) tile = (tile & 7) * (even >> 3) + (tile >> 3);
   part.group = tile / p.panel_slots;
@@ -562,7 +564,7 @@ static int launch_panel(StreamParams& p, const PanelPlan& q, void* workspace, hi
   p.slot_rows = 16 * q.mt;
   p.a_bytes = (uint32_t)((int64_t)p.m * p.a_stride * 2);
   p.panel_groups = q.groups;
-  p.panel_slots = (int)(q.tiles / q.groups);
+  p.panel_slots = q.slots;
   p.panel_full = (int)q.full;
   p.panel_kz = q.kz;
   p.panel_tickets = static_cast<uint32_t*>(workspace) + PLAN_HEADER;

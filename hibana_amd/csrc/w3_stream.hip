@@ -61,14 +61,6 @@ struct Rows {  // the activation side: four MFMA A fragments (one per 32-group),
   u32x4_t a0, a1, a2, a3;
 };
 
-__device__ __forceinline__ void load_chunk(Chunk& ch, const uint8_t* blk, int lane, int r16) {
-  const u32x4_t* b = reinterpret_cast<const u32x4_t*>(blk);
-  ch.w0 = __builtin_nontemporal_load(b + lane);
-  ch.w1 = __builtin_nontemporal_load(b + 64 + lane);
-  ch.w2 = __builtin_nontemporal_load(b + 128 + lane);
-  ch.sc = __builtin_nontemporal_load(b + 192 + r16);
-}
-
 __device__ __forceinline__ void load_rows(Rows& ch, const uint16_t* arow) {
   ch.a0 = *reinterpret_cast<const u32x4_t*>(arow);
   ch.a1 = *reinterpret_cast<const u32x4_t*>(arow + 32);

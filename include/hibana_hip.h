@@ -11,7 +11,10 @@
  * last workgroup plans a routed call; of the tiles whose K several workgroups share) and a fault word. The caller
  * hands a workspace over with its first min(bytes, HB_WORKSPACE_ZERO_BYTES) bytes ZERO, once, before its first use
  * (hipMemsetAsync, or hb_workspace_reset); every call that completes leaves the counters zero again, so one workspace
- * serves any number of calls one after the other. The library keeps no counters of its own: calls that are in flight
+ * serves any number of calls of its kind one after the other. The kinds: the routed calls (hb_w3_moe*, hb_nvfp4_moe*), the
+ * latent block's (hb_latent_*), the dense product (hb_nvfp4_gemm_ws); each may keep its data where another kind has its
+ * counters, so a workspace that goes from one kind to another takes hb_workspace_reset in between. (The `workspace` of
+ * hb_route_budget and hb_route_budget_sigmoid is plain scratch, without counters.) The library keeps no counters of its own: calls that are in flight
  * together (different streams, or graphs replayed side by side) must each have a workspace of their own and then share
  * nothing; two calls in flight on ONE workspace race on everything in it. A call that was aborted midway (a reset
  * device, a killed launch) may leave a counter standing: hb_workspace_reset puts the workspace back in service.
@@ -40,7 +43,7 @@ enum {
   HB_ESCRATCH = -5    /* hb_w3_moe_layer_static: the call needs more scratch than HB_STATIC_SCRATCH_BYTES */
 };
 
-/* Library version (major * 1000 + minor). */
+/* Library version (major * 1000 + minor): the minor one counts up with entry points and with the bytes of a tile layout. */
 int hb_version(void);
 const char* hb_error_string(int code);
 
@@ -418,7 +421,9 @@ int hb_route_budget_sigmoid(const float* fused, int64_t stride, const float* bia
 /* ------------------------------------------------------------------------------------------------------------------
  * NVFP4 format: E2M1 codes two per byte (element 2i in the low nibble), one E4M3 scale per 16 weights, one FP32
  * global scale. ref: hibana/weights/modelopt.py:57-81,150-156.
- * Tile layout: blocks of 64 rows x 128 k, 4608 bytes each: { 4 x 64 lanes x 16 B of codes, 64 rows x 8 scale bytes }.
+ * Tile layout: blocks of 64 rows x 128 k, 4608 bytes each: { 4 x 64 lanes x 16 B of codes, 64 rows x 8 scale bytes }. The
+ * order of the bytes inside a block belongs to the library that wrote them (it changed in 1.6): tile layouts are made from the
+ * checkpoint's tensors at load time and not kept in files.
  * ---------------------------------------------------------------------------------------------------------------- */
 size_t hb_nvfp4_tiled_bytes(int64_t rows, int k);
 

@@ -252,30 +252,31 @@ struct Panel {
     for (int t = 0; t < MT; t++)
 #pragma unroll
       for (int nt = 0; nt < 4; nt++) pin(acc[t][nt]);
-    finish(p, sl, lds, part, nb, active, share.ks, share.nbi, lane);
+    if (p.ks == 1 && part.kz == 1 && !((reinterpret_cast<uintptr_t>(p.out) | (uintptr_t)(p.out_stride * 2)) & 15)) {
+      if (active) store_rows(p, sl, slot, nb, lane);
+    } else {
+      finish(p, sl, lds, part, nb, active, share.ks, share.nbi, lane);
+    }
   }
 
-  // The four neighbouring output columns of one lane and tile (gated: the pair's up and gate tiles).
-  static __device__ __forceinline__ void emit(const StreamParams& p, const Slot& sl, int nb, int t, int nt, int lane, const f32x4_t& v0, const f32x4_t& v1) {
-    typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
-    const int q = lane >> 4, i = 16 * t + (lane & 15);
-    if (i >= sl.rows) return;
-    const int64_t pos = sl.p0 + i;
-    auto scale = [&](int r, int tile) { return Fmt::PER_ROW ? sl.rs[nb * 64 + 16 * tile + 4 * q + r] : sl.scalar; };
-    if (EPI == EPI_FC1_GATED) {  // nt: the pair
-      float h[4];
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        const uint32_t ug = bf16_pair(v0[r] * scale(r, 2 * nt), v1[r] * scale(r, 2 * nt + 1));  // up and gate rounded to BF16 ...
-        h[r] = silu(pair_hi(ug)) * pair_lo(ug);                                                // ... and their product, rounded below
-      }
-      *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(p.out) + pos * p.out_stride + nb * 32 + 16 * nt + 4 * q) = u32x2_t{bf16_pair(h[0], h[1]), bf16_pair(h[2], h[3])};
-      return;
-    }
-    const int64_t at = (EPI == EPI_FC2 ? (int64_t)p.order[pos] : pos) * p.out_stride + nb * 64 + 16 * nt + 4 * q;
+  typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
+  static constexpr bool GATED = EPI == EPI_FC1_GATED;
+  // The FP32 scales of a lane's output columns: one a column of each 16-row tile, or the matrix's one.
+  static __device__ __forceinline__ f32x4_t column_scales(const Slot& sl, int nb, int tile, int q) {
+    typedef f32x4_t __attribute__((aligned(4))) loose_f32x4_t;  // row scales start on any float
+    return Fmt::PER_ROW ? *reinterpret_cast<const loose_f32x4_t*>(sl.rs + nb * 64 + 16 * tile + 4 * q) : f32x4_t{sl.scalar, sl.scalar, sl.scalar, sl.scalar};
+  }
+  // Four neighbouring output columns as BF16 (gated: v0 / s0 the up tile, v1 / s1 the gate tile).
+  static __device__ __forceinline__ u32x2_t rounded(const f32x4_t& v0, const f32x4_t& v1, const f32x4_t& s0, const f32x4_t& s1) {
     float y[4];
 #pragma unroll
-    for (int r = 0; r < 4; r++) y[r] = v0[r] * scale(r, nt);
+    for (int r = 0; r < 4; r++) {
+      y[r] = v0[r] * s0[r];
+      if (GATED) {
+        const uint32_t ug = bf16_pair(y[r], v1[r] * s1[r]);  // up and gate rounded to BF16 ...
+        y[r] = silu(pair_hi(ug)) * pair_lo(ug);              // ... and their product, rounded below
+      }
+    }
     if (EPI == EPI_FC1_RELU2 || EPI == EPI_DENSE_RELU2) {  // bf16(relu(bf16(y))^2), two values a conversion
       const uint32_t u01 = bf16_pair(y[0], y[1]), u23 = bf16_pair(y[2], y[3]);
       // relu on the bits: a negative value (and -0) is a negative integer; a NaN stays one, as torch's relu leaves it
@@ -283,10 +284,74 @@ struct Panel {
       const float h2 = __int_as_float(max((int)(u23 << 16), 0)), h3 = __int_as_float(max((int)(u23 & 0xffff0000u), 0));
       y[0] = h0 * h0, y[1] = h1 * h1, y[2] = h2 * h2, y[3] = h3 * h3;
     }
+    return u32x2_t{bf16_pair(y[0], y[1]), bf16_pair(y[2], y[3])};
+  }
+
+  // One lane's four neighbouring output columns of a tile (gated: of pair `nt` of tiles), stored as they are.
+  static __device__ __forceinline__ void emit(const StreamParams& p, const Slot& sl, int nb, int t, int nt, int lane, const f32x4_t& v0, const f32x4_t& v1) {
+    const int q = lane >> 4, i = 16 * t + (lane & 15);
+    if (i >= sl.rows) return;
+    const int64_t pos = sl.p0 + i;
+    const f32x4_t s0 = column_scales(sl, nb, GATED ? 2 * nt : nt, q), s1 = GATED ? column_scales(sl, nb, 2 * nt + 1, q) : s0;
+    const int64_t at = (EPI == EPI_FC2 ? (int64_t)p.order[pos] : pos) * p.out_stride + nb * (GATED ? 32 : 64) + 16 * nt + 4 * q;
     if (EPI != EPI_FC2 || p.out_bf16) {
-      *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(p.out) + at) = u32x2_t{bf16_pair(y[0], y[1]), bf16_pair(y[2], y[3])};
+      *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(p.out) + at) = rounded(v0, v1, s0, s1);
     } else {
-      *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.out) + at) = f32x4_t{y[0], y[1], y[2], y[3]};
+      *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.out) + at) = v0 * s0;
+    }
+  }
+
+  // All of a wavefront's results where it holds them K-complete, as whole rows: a lane's four columns of sixteen rows are 32
+  // bytes a row and store, so a row tile goes through the wavefront's own (by now empty) slot of LDS and leaves as 128 (gated:
+  // 64) contiguous bytes a row; what the stores need from memory (the rows' places, the column scales) is asked for once, ahead
+  // of the first. Before, the last row tiles of a slot of 128 stood behind eight round trips to `order`: 11.9 us of a workgroup's
+  // 23.9 (fc2 of the three-bit layer, 1543 rows), 14.6 of 68.6 (the latent block's, 2048). A row of LDS is 144 bytes: sixteen rows' columns start in different banks.
+  static constexpr int LINE = 144;
+  static_assert(16 * LINE <= Fmt::BLOCK_BYTES && LINE % 16 == 0 && Fmt::BLOCK_BYTES % 16 == 0, "a row tile in the slot of a weight block");
+  __device__ __forceinline__ void store_rows(const StreamParams& p, const Slot& sl, uint8_t* slot, int nb, int lane) {
+    constexpr int PER_ROW = GATED ? 4 : 8, ROWS = 64 / PER_ROW, PASSES = 16 / ROWS;  // lanes a row, rows a store, stores a row tile
+    const int q = lane >> 4, r16 = lane & 15, line = lane / PER_ROW, part = lane % PER_ROW;
+    f32x4_t scale[4];
+#pragma unroll
+    for (int nt = 0; nt < 4; nt++) scale[nt] = column_scales(sl, nb, nt, q);
+    int row[MT * PASSES];
+#pragma unroll
+    for (int j = 0; j < MT * PASSES; j++) {
+      row[j] = sl.p0 + min(ROWS * j + line, sl.rows - 1);
+      if (EPI == EPI_FC2) row[j] = p.order[row[j]];
+    }
+    const bool wide = EPI == EPI_FC2 && !p.out_bf16;  // FP32: two tiles' columns are a row of LDS
+    uint8_t* out = static_cast<uint8_t*>(p.out) + (int64_t)nb * (GATED ? 64 : wide ? 256 : 128) + 16 * part;
+    const int64_t pitch = p.out_stride * (wide ? 4 : 2);
+    uint8_t* write = slot + r16 * LINE;
+    const uint8_t* read = slot + line * LINE + 16 * part;
+    auto leave = [&](int t, int offset) {
+      asm volatile("" ::: "memory");  // the lanes read what other lanes of the wavefront wrote: LDS serves a wavefront in order
+#pragma unroll
+      for (int u = 0; u < PASSES; u++) {
+        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(read + u * ROWS * LINE);
+        if (16 * t + ROWS * u + line < sl.rows) *reinterpret_cast<u32x4_t*>(out + row[PASSES * t + u] * pitch + offset) = v;
+      }
+      asm volatile("" ::: "memory");
+    };
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+      if (16 * t >= sl.rows) break;
+      if (wide) {
+#pragma unroll
+        for (int nt = 0; nt < 4; nt += 2) {
+          *reinterpret_cast<f32x4_t*>(write + 16 * q) = acc[t][nt] * scale[nt];
+          *reinterpret_cast<f32x4_t*>(write + 64 + 16 * q) = acc[t][nt + 1] * scale[nt + 1];
+          leave(t, 64 * nt);
+        }
+      } else {
+#pragma unroll
+        for (int nt = 0; nt < (GATED ? 2 : 4); nt++) {
+          const int a = GATED ? 2 * nt : nt, b = GATED ? 2 * nt + 1 : nt;
+          *reinterpret_cast<u32x2_t*>(write + 32 * nt + 8 * q) = rounded(acc[t][a], acc[t][b], scale[a], scale[b]);
+        }
+        leave(t, 0);
+      }
     }
   }
 
@@ -309,7 +374,6 @@ struct Panel {
   // through and waited for) and draw a ticket; the last one adds them in the order of the shares: the same sum whichever
   // it is. The tickets lie at a fixed place in the workspace and are zero again when the launch ends.
   __device__ __forceinline__ void finish(const StreamParams& p, const Slot& sl, uint8_t* lds, const PanelShare& part, int nb, bool active, int ks, int nbi, int lane) {
-    constexpr bool GATED = EPI == EPI_FC1_GATED;
     if (p.ks == 1) {
       if (active) {
 #pragma unroll

@@ -101,3 +101,37 @@ def test_nvfp4_linear_holds_the_room_its_cut_uses(m, n, k, monkeypatch):
     ops.nvfp4_linear(torch.zeros(m, k, dtype=torch.bfloat16, device="cuda"), synthetic.nvfp4_linear(n, k, 1))
     room = _lib.lib().hb_nvfp4_gemm_room_bytes(m, n, k)
     assert asked == ([room] if room else []) and (room > 0) == (k == 12800)
+
+
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("mode,shift", [(1, 0), (2, 0), (2, 4)])  # FP32 and BF16 pair outputs; BF16 ones that start off a 16-byte boundary (shift: elements)
+def test_routed_slots_around_whole_row_tiles(gated, mode, shift):
+    """An expert a row count: every number of row tiles of a slot, a row more or less, two slots, none; the rows leave as whole
+    lines where the output allows, else four columns at a time."""
+    import ctypes as C
+    from hibana_amd import _lib
+    from hibana_amd.kernels import w3_moe
+    from tests.util import oracle_expert_getter, random_experts
+    counts = [1, 15, 16, 17, 33, 48, 0, 64, 65, 81, 97, 112, 127, 128, 129, 250]
+    hidden, inter, m = 256, 384, sum(counts)
+    ex, per = random_experts(len(counts), hidden, inter, gated, 5)
+    w3_moe.tile(ex)
+    g = torch.Generator().manual_seed(m)
+    ids = torch.repeat_interleave(torch.arange(len(counts)), torch.tensor(counts))[torch.randperm(m, generator=g)].to(torch.int32)[:, None]
+    x = torch.randn(m, hidden, generator=g).bfloat16()
+    want = layers.routed_experts_ref(x, ids.numpy(), oracle_expert_getter(per, gated, inter), gated, e_n=len(counts))
+    lib, st = _lib.lib(), w3_moe._struct(ex)
+    dtype = torch.float32 if mode == 1 else torch.bfloat16
+    guard = 64
+    out = torch.full((m * hidden + shift + guard,), 7.0, dtype=dtype, device="cuda")
+    need = w3_moe._workspace_bytes(st, m, 1, False)
+    xd, idd, wd = x.cuda(), ids.cuda(), torch.ones(m, 1, device="cuda")
+    assert lib.hb_tune(b"w3_tile", 1) == 0
+    try:
+        _lib.check(lib.hb_w3_moe_among(C.byref(st), 0, _lib.ptr(xd), _lib.ptr(idd), _lib.ptr(wd), m, 1, mode, C.c_void_p(out.data_ptr() + shift * out.element_size()),
+                                       _lib.ptr(_lib.workspace(xd.device, need)), need, _lib.stream()), "w3_moe")
+    finally:
+        lib.hb_tune(b"w3_tile", 0)
+    mx, nr = errors(out[shift:shift + m * hidden].view(m, hidden), want)
+    assert mx < MAX_REL and nr < NORM_REL, (mx, nr)
+    assert bool((out[:shift] == 7).all()) and bool((out[shift + m * hidden:] == 7).all())

@@ -472,6 +472,22 @@ __global__ __launch_bounds__(PLAN_THREADS) void moe_plan_kernel(const int32_t* i
   plan_work<WIDE>(ids, pairs, e_lo, e_n, shared_rows, plan, order, slot_rows, slot_cap, wide, groups, phase, blockIdx.x, lds);
 }
 
+// For launches whose last workgroup plans. "No rows" into every entry of the slot table and the slots' arrival counters at
+// zero, word `first` and every `step`-th after it - with stores that go through to memory and are waited for, so the words
+// are there, and in no L2 as modified lines, before anyone's ticket: the planner's own stores to the entries it fills come
+// after its ticket and are the only modified copies.
+__device__ __forceinline__ void clear_plan(int32_t* plan, int slot_cap, int first, int step) {
+  int32_t* done = plan_done(plan, slot_cap);
+  for (int i = first; i < 5 * slot_cap; i += step) store_through(i < 4 * slot_cap ? plan + PLAN_HEADER + i : done + (i - 4 * slot_cap) * DONE_PITCH, 0);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+// One thread a workgroup draws a ticket: whether it is the last of `groups`, which puts the counter back for the next call.
+__device__ __forceinline__ int last_to_arrive(int32_t* plan, int groups) {
+  const bool last = atomicAdd(reinterpret_cast<unsigned*>(plan + PLAN_TICKET), 1u) == (unsigned)groups - 1u;
+  if (last) store_through(plan + PLAN_TICKET, 0);  // every other workgroup of this launch has drawn
+  return last;
+}
+
 // Routing and plan of a verify-sized call in ONE launch: `route_groups` workgroups route ROUTE_GROUP_ROWS rows each (a
 // row a wavefront, spread over the device, as the routing launch does), and the one that finishes last plans - it
 // learns that it is the last from an arrival counter in the call's own workspace (plan[PLAN_TICKET]: zero when the
@@ -498,23 +514,11 @@ __global__ __launch_bounds__(PLAN_THREADS) void moe_route_plan_kernel(const int3
     route_any(route, r, threadIdx.x & 63);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this row's ids (write-through stores) have reached memory before the ticket is drawn
   } else if (by_rows && wave >= ROUTE_GROUP_ROWS) {
-    // Meanwhile the wavefronts that route nothing put "no rows" into every entry of the slot table and zero the slots'
-    // arrival counters, a word a thread over the launch's routing workgroups - with stores that go through to memory
-    // and are waited for, so the words are there, and in no L2 as modified lines, before anyone's ticket: the planner's
-    // own stores to the entries it fills come after its ticket and are the only modified copies.
-    constexpr int IDLE = PLAN_THREADS - 64 * ROUTE_GROUP_ROWS;
-    int32_t* done = plan_done(plan, slot_cap);
-    for (int i = blockIdx.x * IDLE + (int)threadIdx.x - 64 * ROUTE_GROUP_ROWS; i < 5 * slot_cap; i += route_groups * IDLE)
-      store_through(i < 4 * slot_cap ? plan + PLAN_HEADER + i : done + (i - 4 * slot_cap) * DONE_PITCH, 0);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    constexpr int IDLE = PLAN_THREADS - 64 * ROUTE_GROUP_ROWS;  // meanwhile, the wavefronts that route nothing
+    clear_plan(plan, slot_cap, blockIdx.x * IDLE + (int)threadIdx.x - 64 * ROUTE_GROUP_ROWS, route_groups * IDLE);
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    unsigned* ticket = reinterpret_cast<unsigned*>(plan + PLAN_TICKET);
-    const unsigned drawn = atomicAdd(ticket, 1u);
-    last = drawn == (unsigned)route_groups - 1u;
-    if (last) store_through(plan + PLAN_TICKET, 0);  // every other workgroup of this launch has drawn: the counter is zero for the next call
-  }
+  if (threadIdx.x == 0) last = last_to_arrive(plan, route_groups);
   __syncthreads();
   if (!last) return;  // the last arriver: every row's ids are in memory, and the plan reads them from there (load_through)
   if (by_rows) {
@@ -524,20 +528,37 @@ __global__ __launch_bounds__(PLAN_THREADS) void moe_route_plan_kernel(const int3
   }
 }
 
-// Budgeted selection and the plan of its ids in one launch: the selection is one workgroup's work already, and so is
-// the plan of a decode or verify call; the ids go through to memory and are waited for before the plan reads them back
-// past the L2, as in the routing launch above. `PLAN`: false leaves the plan to launches of its own (a call of more
-// pairs than one workgroup plans).
+// Budgeted selection and the plan of its ids in one launch: its workgroups rank `group_rows` rows each (a row a
+// wavefront), and the last of them to finish selects and plans, as in the routing launch above: candidates and ids go through
+// to memory, are waited for ahead of the ticket or the plan, and are read past the L2. (A rank launch of its own before it:
+// 5.0 + 13.0 us at 40 rows of 512 experts, the whole layer 50.4 us and 48.7 so.) `PLAN`: false leaves the plan to launches of its own (a call of more pairs than
+// one workgroup plans). `by_rows`: no row names an expert twice and they are at most PLAN_ROWS_MAX; each group ranks one.
 template <int PER, bool PLAN>
 __global__ __launch_bounds__(PLAN_THREADS) void moe_budget_plan_kernel(BudgetParams q, int copies_n, int e_lo, int e_n, int shared_rows,
-                                                                       int32_t* __restrict__ plan, int32_t* __restrict__ order, int slot_rows,
-                                                                       int slot_cap) {
+                                                                       int32_t* __restrict__ plan, int32_t* __restrict__ order, int group_rows, int by_rows,
+                                                                       int slot_rows, int slot_cap) {
   extern __shared__ int lds[];
-  budget_pick<PER, false>(q, copies_n, reinterpret_cast<float*>(lds));
+  __shared__ int last;
+  const int wave = threadIdx.x >> 6, r = blockIdx.x * group_rows + wave;
+  if (wave < group_rows && r < q.r) {
+    rank_row<PER, true>(q, r, threadIdx.x & 63);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  } else if (by_rows) {
+    clear_plan(plan, slot_cap, blockIdx.x * (PLAN_THREADS - 64) + (int)threadIdx.x - 64, gridDim.x * (PLAN_THREADS - 64));
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) last = last_to_arrive(plan, gridDim.x);
+  __syncthreads();
+  if (!last) return;
+  budget_pick<PER, false, true>(q, copies_n, reinterpret_cast<float*>(lds));
   if (!PLAN) return;
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's ids have reached memory
   __syncthreads();                                    // ... and everyone's; the selection's use of the LDS is over
-  plan_work<false>(q.ids, q.r * q.k, e_lo, e_n, shared_rows, plan, order, slot_rows, slot_cap, nullptr, 1, 0, 0, lds);
+  if (by_rows) {
+    plan_by_rows(q.ids, q.r, q.k, e_lo, e_n, shared_rows, plan, order, slot_rows, slot_cap, lds, true);
+  } else {
+    plan_work<false>(q.ids, q.r * q.k, e_lo, e_n, shared_rows, plan, order, slot_rows, slot_cap, nullptr, 1, 0, 0, lds);
+  }
 }
 
 // ---------------------------------------------------------------------------------------------------- combine
@@ -652,27 +673,6 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(CombineParams p) {
   }
 }
 
-// ------------------------------------------------------------------ the latent block's BF16 projections (M <= 16)
-//
-// y[i, n] = sum_k x[i, k] w[n, k] for at most sixteen rows of x, on the BF16 matrix cores with nothing staged: a
-// wavefront takes sixteen weight rows over `steps` K steps of 32 from k0; lane (q, r16) holds k = 32 s + 8 q .. + 7 of
-// weight row n0 + r16 (the B operand) and of activation row r16 (A; rows past m read row m - 1 and are never stored).
-// Register i of lane (q, r16) of the result is y[4 q + i][n0 + r16]. Up to eight steps are in flight at a time.
-struct GemvFrags {
-  u32x4_t v[8];
-};
-__device__ __forceinline__ void gemv16_load(GemvFrags& f, const uint16_t* __restrict__ base, int64_t ld, int row, int k0, int steps, int lane) {
-  const uint16_t* at = base + row * ld + k0 + 8 * (lane >> 4);
-#pragma unroll
-  for (int j = 0; j < 8; j++)
-    if (j < steps) f.v[j] = *reinterpret_cast<const u32x4_t*>(at + 32 * j);
-}
-__device__ __forceinline__ void gemv16_mfma(f32x4_t& acc, const GemvFrags& a, const GemvFrags& b, int steps) {
-#pragma unroll
-  for (int j = 0; j < 8; j++)
-    if (j < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a.v[j]), __builtin_bit_cast(bf16x8_t, b.v[j]), acc, 0, 0, 0);
-}
-__device__ __forceinline__ f32x4_t gemv16_wave(const uint16_t* __restrict__ w, int64_t ldw, int n0, int n, const uint16_t* __restrict__ x, int64_t ldx, int m,
 // A long call's sum of BF16 pairs alone: sixteen bytes of a pair a thread and load instead of four. combine_span's chain, operation
 // for operation: the same bits. Bound by the pairs' traffic (5 TB/s). Measured alone, before and now: 1024 rows of 22 pairs, 1024
 // columns, 12.7 and 10.8 us, 2048 rows 24.6 and 19.2. (With the shared expert's gate, whose dot product is half a row's loads,
@@ -704,6 +704,27 @@ __global__ __launch_bounds__(256) void moe_combine_wide_kernel(CombineParams p) 
   *reinterpret_cast<u32x4_t*>(p.out + (int64_t)r * p.h + c) = out;
 }
 
+// ------------------------------------------------------------------ the latent block's BF16 projections (M <= 16)
+//
+// y[i, n] = sum_k x[i, k] w[n, k] for at most sixteen rows of x, on the BF16 matrix cores with nothing staged: a
+// wavefront takes sixteen weight rows over `steps` K steps of 32 from k0; lane (q, r16) holds k = 32 s + 8 q .. + 7 of
+// weight row n0 + r16 (the B operand) and of activation row r16 (A; rows past m read row m - 1 and are never stored).
+// Register i of lane (q, r16) of the result is y[4 q + i][n0 + r16]. Up to eight steps are in flight at a time.
+struct GemvFrags {
+  u32x4_t v[8];
+};
+__device__ __forceinline__ void gemv16_load(GemvFrags& f, const uint16_t* __restrict__ base, int64_t ld, int row, int k0, int steps, int lane) {
+  const uint16_t* at = base + row * ld + k0 + 8 * (lane >> 4);
+#pragma unroll
+  for (int j = 0; j < 8; j++)
+    if (j < steps) f.v[j] = *reinterpret_cast<const u32x4_t*>(at + 32 * j);
+}
+__device__ __forceinline__ void gemv16_mfma(f32x4_t& acc, const GemvFrags& a, const GemvFrags& b, int steps) {
+#pragma unroll
+  for (int j = 0; j < 8; j++)
+    if (j < steps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a.v[j]), __builtin_bit_cast(bf16x8_t, b.v[j]), acc, 0, 0, 0);
+}
+__device__ __forceinline__ f32x4_t gemv16_wave(const uint16_t* __restrict__ w, int64_t ldw, int n0, int n, const uint16_t* __restrict__ x, int64_t ldx, int m,
                                                int k0, int steps, int lane) {
   const int r16 = lane & 15, wrow = min(n0 + r16, n - 1), xrow = min(r16, m - 1);
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
@@ -938,10 +959,10 @@ static unsigned plan_groups(const QuantJob* job) {
 }
 
 int moe_launch_plan(const int32_t* ids, int64_t pairs, int e_lo, int e_n, int shared_rows, const MoeWorkspace& ws, hipStream_t stream, int slot_rows,
-                    const QuantJob* job) {
+                    const QuantJob* job, int distinct) {
   const size_t plan_lds = ((size_t)(PLAN_WAVES + 1) * e_n + 3 * (PLAN_WAVES + 1)) * sizeof(int);
   if (plan_lds > 64 * 1024 || e_n > PLAN_THREADS || pairs > 0x3fffffff) return HB_EINVAL;
-  const int slot_cap = (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows);
+  const int slot_cap = (int)moe_max_slots(pairs, distinct ? distinct : e_n, shared_rows, slot_rows);
   if (pairs >= PLAN_WIDE_PAIRS) {  // a share of about a thousand pairs a workgroup
     const int groups = (int)std::min<int64_t>(PLAN_WIDE_GROUPS, pairs / 1024);
     if (job) moe_launch_quant_groups(*job, stream);
@@ -1008,6 +1029,7 @@ int moe_launch_route_plan(const TopkRoute& route, int m, int topk, int32_t* ids,
   return launch_route_plan(rp, m, e_lo, e_n, shared_rows, ws, stream, slot_rows, job);
 }
 
+constexpr int BUDGET_SPREAD_ROWS = 256;  // about the compute units
 int moe_launch_budget_plan(const BudgetRoute& b, int m, int topk, int32_t* ids, float* weights, int e_lo, int e_n, int shared_rows,
                            const MoeWorkspace& ws, void* scratch, hipStream_t stream, int slot_rows) {
   static_assert(BUDGET_THREADS == PLAN_THREADS, "the selection and the plan share a workgroup");
@@ -1029,33 +1051,22 @@ int moe_launch_budget_plan(const BudgetRoute& b, int m, int topk, int32_t* ids, 
   q.share = q.prob;
   q.ids = ids, q.weights = weights;
   const bool small = b.e <= 512;
-  if (small) {
-    HB_LAUNCH((route_rank_kernel<8>), dim3((unsigned)m), dim3(64), 0, stream, q);
-  } else {
-    HB_LAUNCH((route_rank_kernel<16>), dim3((unsigned)m), dim3(64), 0, stream, q);
-  }
   const int copies_n = small ? BUDGET_WAVES : BUDGET_WAVES / 2;
   const size_t pick_lds = (size_t)copies_n * b.e * sizeof(float);
-  const int slot_cap = (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows);
-  if (pairs < PLAN_WIDE_PAIRS) {
-    const size_t lds = std::max(pick_lds, plan_lds);
-    if (small) {
-      HB_LAUNCH((moe_budget_plan_kernel<8, true>), dim3(1), dim3(PLAN_THREADS), lds, stream, q, copies_n, e_lo, e_n, shared_rows, ws.plan, ws.order, slot_rows,
-                slot_cap);
-    } else {
-      HB_LAUNCH((moe_budget_plan_kernel<16, true>), dim3(1), dim3(PLAN_THREADS), lds, stream, q, copies_n, e_lo, e_n, shared_rows, ws.plan, ws.order, slot_rows,
-                slot_cap);
-    }
+  const int distinct = (int)budget_distinct(b, m, e_n), slot_cap = (int)moe_max_slots(pairs, distinct, shared_rows, slot_rows);
+  const bool plan = pairs < PLAN_WIDE_PAIRS, by_rows = plan && !b.repeat && m <= PLAN_ROWS_MAX && topk <= 64;
+  const int group_rows = m <= BUDGET_SPREAD_ROWS ? 1 : PLAN_WAVES;  // a row a workgroup while that spreads them over the device
+  const dim3 grid((unsigned)((m + group_rows - 1) / group_rows));
+  const size_t lds = plan ? std::max(pick_lds, plan_lds) : pick_lds;
+  auto launch = [&](auto kernel) {
+    HB_LAUNCH(kernel, grid, dim3(PLAN_THREADS), lds, stream, q, copies_n, e_lo, e_n, shared_rows, ws.plan, ws.order, group_rows, (int)by_rows, slot_rows, slot_cap);
+  };
+  if (plan) {
+    small ? launch(moe_budget_plan_kernel<8, true>) : launch(moe_budget_plan_kernel<16, true>);
     return HB_OK;
   }
-  if (small) {
-    HB_LAUNCH((moe_budget_plan_kernel<8, false>), dim3(1), dim3(PLAN_THREADS), pick_lds, stream, q, copies_n, e_lo, e_n, shared_rows, ws.plan, ws.order,
-              slot_rows, slot_cap);
-  } else {
-    HB_LAUNCH((moe_budget_plan_kernel<16, false>), dim3(1), dim3(PLAN_THREADS), pick_lds, stream, q, copies_n, e_lo, e_n, shared_rows, ws.plan, ws.order,
-              slot_rows, slot_cap);
-  }
-  return moe_launch_plan(ids, pairs, e_lo, e_n, shared_rows, ws, stream, slot_rows, nullptr);
+  small ? launch(moe_budget_plan_kernel<8, false>) : launch(moe_budget_plan_kernel<16, false>);
+  return moe_launch_plan(ids, pairs, e_lo, e_n, shared_rows, ws, stream, slot_rows, nullptr, distinct);
 }
 
 int latent_launch_router(const LatentRouter& r, hipStream_t stream) {
@@ -1100,6 +1111,12 @@ int latent_launch_out(const uint16_t* fc2, const uint16_t* routed, const uint16_
 }
 
 void moe_launch_combine(const CombineParams& c, hipStream_t stream) {
+  // the wide form from the size that its comment measures (a summed call's pairs are FP32 below), where the addresses allow it
+  if (c.pairs_bf16 && !c.shared && c.m >= MOE_WIDE_ROWS && c.h % 8 == 0 && aligned(c.pairs, 16) && aligned(c.out, 16)) {
+    const int threads = std::min(256, (c.h / 8 + 63) / 64 * 64);
+    HB_LAUNCH(moe_combine_wide_kernel<12>, dim3((unsigned)c.m, (unsigned)((c.h / 8 + threads - 1) / threads)), dim3((unsigned)threads), 0, stream, c);
+    return;
+  }
   const dim3 grid((unsigned)c.m, (unsigned)((c.h + COMBINE_SPAN - 1) / COMBINE_SPAN));
   if (c.topk <= 8 || (c.topk > 12 && c.m > 64)) {  // a long call is bound by its traffic: fewer registers, more wavefronts
     HB_LAUNCH(moe_combine_kernel<8>, grid, dim3(256), 0, stream, c);
@@ -1111,12 +1128,6 @@ void moe_launch_combine(const CombineParams& c, hipStream_t stream) {
 }
 
 }  // namespace hb
-  // the wide form from the size that its comment measures (a summed call's pairs are FP32 below), where the addresses allow it
-  if (c.pairs_bf16 && !c.shared && c.m >= MOE_WIDE_ROWS && c.h % 8 == 0 && aligned(c.pairs, 16) && aligned(c.out, 16)) {
-    const int threads = std::min(256, (c.h / 8 + 63) / 64 * 64);
-    HB_LAUNCH(moe_combine_wide_kernel<12>, dim3((unsigned)c.m, (unsigned)((c.h / 8 + threads - 1) / threads)), dim3((unsigned)threads), 0, stream, c);
-    return;
-  }
 
 using namespace hb;
 

@@ -1,7 +1,9 @@
-// Budgeted expert selection (device code shared by the routing launches and the routed layer's chain): a cap on the distinct experts one decode or verify forward reads, chosen for all its rows
+// Budgeted expert selection (device code shared by the routing launches and the routed layer's chain): a cap on the distinct experts one
+// decode or verify forward reads, chosen for all its rows
 // (route_budget, hibana/kernels/flashnext_fused.py:322-502 of the reference; the rule row by row:
 // tests/unit/test_moe_selection.py:19-58; the latent MoE's form with its own ranking, hibana/model/nemotron/moe.py:
-// 124-313). Two launches, no atomics on floating-point data, no host synchronization:
+// 124-313). Two steps (two launches, or one whose last workgroup takes the second: moe_budget_plan_kernel), no atomics on
+// floating-point data, no host synchronization:
 //   1. rank: a wavefront a row finds the row's candidates, best first, with the weight each would carry: the 20 largest
 //      BF16 logits (an exact tie to the lower expert; -0 equals +0) and their softmax probabilities over all experts,
 //      or the top k of sigmoid + bias with the plain sigmoids (the routing kernel itself, which also writes each
@@ -48,9 +50,10 @@ __device__ __forceinline__ float bf16_order_value(uint32_t o) {
 
 // Lane l holds columns l, l + 64, ... as keys (value order above 65535 - column): distinct, every real one above 0, so
 // the wave-wide maximum names the largest logit left and, among equal logits, the lowest expert.
-template <int PER>
-__global__ __launch_bounds__(64) void route_rank_kernel(BudgetParams q) {
-  const int t = blockIdx.x, lane = threadIdx.x, e = q.e;
+// THROUGH: the candidates are read by another workgroup of the same launch.
+template <int PER, bool THROUGH>
+__device__ __forceinline__ void rank_row(const BudgetParams& q, int t, int lane) {
+  const int e = q.e;
   const uint16_t* row = q.logits + (int64_t)t * e;
   uint32_t key[PER], raw[PER];
   float val[PER];
@@ -98,9 +101,19 @@ __global__ __launch_bounds__(64) void route_rank_kernel(BudgetParams q) {
   }
   const float mine = expf(mine_v - mx) / sum;
   if (lane < BUDGET_CANDIDATES) {
-    q.cand[(int64_t)t * BUDGET_CANDIDATES + lane] = mine_id;
-    q.prob[(int64_t)t * BUDGET_CANDIDATES + lane] = mine;
+    const int64_t at = (int64_t)t * BUDGET_CANDIDATES + lane;
+    if (THROUGH) {
+      store_through(&q.cand[at], mine_id);
+      store_through(&q.prob[at], mine);
+    } else {
+      q.cand[at] = mine_id;
+      q.prob[at] = mine;
+    }
   }
+}
+template <int PER>
+__global__ __launch_bounds__(64) void route_rank_kernel(BudgetParams q) {
+  rank_row<PER, false>(q, blockIdx.x, threadIdx.x);
 }
 
 // One workgroup (BUDGET_THREADS threads; `copies`: copies_n * e floats of its dynamic LDS). Scores: wavefront w adds the rows t = w (mod copies) into a copy of its own, in row order, and the
@@ -109,7 +122,7 @@ __global__ __launch_bounds__(64) void route_rank_kernel(BudgetParams q) {
 // ballot a register. The rows: two a wavefront at a time, one in each half. IN_ORDER: a row's weights are divided by
 // the sum of the taken ones added in rank order, as the routing kernel adds a row's top k (a row that keeps all of its
 // top k gets that kernel's weights bit for bit); otherwise by a butterfly sum.
-template <int PER, bool IN_ORDER>
+template <int PER, bool IN_ORDER, bool THROUGH = false>
 __device__ __forceinline__ void budget_pick(const BudgetParams& q, int copies_n, float* copies) {
   __shared__ uint32_t keys[BUDGET_THREADS];
   __shared__ uint8_t core[BUDGET_THREADS], core_fallback[BUDGET_THREADS], chosen[BUDGET_THREADS];
@@ -120,17 +133,19 @@ __device__ __forceinline__ void budget_pick(const BudgetParams& q, int copies_n,
   constexpr int PAIRS = BUDGET_BATCH / 2;
   int cd[PAIRS];
   float pv[PAIRS];
+  auto candidate = [&](int64_t at) -> int { if constexpr (THROUGH) return load_through(&q.cand[at]); else return q.cand[at]; };
+  auto value = [&](const float* from, int64_t at) -> float { if constexpr (THROUGH) return load_through(&from[at]); else return from[at]; };
   auto request = [&](int t0) {
 #pragma unroll
     for (int b = 0; b < PAIRS; b++) {
       const int t = t0 + 2 * BUDGET_WAVES * b + half;
       const bool live = t < r && hl < cands;
-      cd[b] = live ? q.cand[(int64_t)t * cands + hl] : 0;
-      pv[b] = live ? q.prob[(int64_t)t * cands + hl] : 0.f;
+      cd[b] = live ? candidate((int64_t)t * cands + hl) : 0;
+      pv[b] = live ? value(q.prob, (int64_t)t * cands + hl) : 0.f;
     }
   };
   request(2 * wave);
-  const int first = q.repeat ? q.cand[0] : e;  // a padded row's slots under `repeat`: row 0's first candidate
+  const int first = q.repeat ? candidate(0) : e;  // a padded row's slots under `repeat`: row 0's first candidate
   for (int i = tid; i < copies_n * e; i += BUDGET_THREADS) copies[i] = 0.f;
   core[tid] = 0;
   core_fallback[tid] = 0;
@@ -153,8 +168,8 @@ __device__ __forceinline__ void budget_pick(const BudgetParams& q, int copies_n,
       for (int b = 0; b < BUDGET_BATCH; b++) {
         const int t = t0 + b * copies_n;
         real[b] = real_row(t) && lane < cands;
-        sc[b] = real[b] ? q.cand[(int64_t)t * cands + lane] : 0;
-        sp[b] = real[b] ? q.share[(int64_t)t * cands + lane] : 0.f;
+        sc[b] = real[b] ? candidate((int64_t)t * cands + lane) : 0;
+        sp[b] = real[b] ? value(q.share, (int64_t)t * cands + lane) : 0.f;
       }
 #pragma unroll
       for (int b = 0; b < BUDGET_BATCH; b++) {  // a row's candidates are distinct experts: no two lanes meet

@@ -523,9 +523,10 @@ struct MoeWorkspace {
 int64_t moe_max_slots(int64_t pairs, int experts, int shared_rows, int slot_rows = ROWS_PER_SLOT);
 MoeWorkspace moe_carve(void* base, int m, int topk, int experts, int inter, int hidden_out, int shared, int hidden = 0);  // hidden: also the E4M3 activation buffers
 // Enqueue the plan kernel; HB_EINVAL if the expert count does not fit its LDS.
-// A rounding job rides in the plan's launch (further workgroups beside the one that plans).
+// A rounding job rides in the plan's launch (further workgroups beside the one that plans). `distinct`: the most experts of
+// the range that the ids can name (0: all).
 int moe_launch_plan(const int32_t* ids, int64_t pairs, int e_lo, int e_n, int shared_rows, const MoeWorkspace& ws, hipStream_t stream,
-                    int slot_rows = ROWS_PER_SLOT, const QuantJob* job = nullptr);
+                    int slot_rows = ROWS_PER_SLOT, const QuantJob* job = nullptr, int distinct = 0);
 void moe_launch_quant_groups(const QuantJob& job, hipStream_t stream);  // the rounding alone
 void moe_launch_quant_rows(const uint16_t* x, int64_t m, int k, uint8_t* q, float* scales, hipStream_t stream);  // one scale a row
 
@@ -543,6 +544,13 @@ struct BudgetRoute {
   int e, keep, budget, steps, repeat, per_request, min_cap;
   const int32_t* slots;  // or null: every row is real
 };
+// The cap on distinct experts of a call whose requests are all real (padded ones only lower it), and the most a selection can
+// name: its set is the rows' guaranteed experts filled up to the cap, and a slot left over names no expert. (With `repeat` it
+// names a row's first candidate, in the set or not: no bound then.)
+inline int64_t budget_cap(const BudgetRoute& b, int m) { return b.per_request > 0 ? std::min<int64_t>(b.budget, std::max<int64_t>(b.min_cap, (int64_t)b.per_request * (m / b.steps))) : b.budget; }
+inline int64_t budget_distinct(const BudgetRoute& b, int m, int experts) {
+  return b.repeat ? experts : std::min<int64_t>(experts, std::max<int64_t>({1, budget_cap(b, m), (int64_t)b.keep * m}));
+}
 // Rank, then the selection and the plan of its ids in one workgroup's launch (the selection leaves ids / weights in the
 // caller's arrays). `scratch`: room for the rows' candidates between the two launches (160 bytes a row).
 int moe_launch_budget_plan(const BudgetRoute& b, int m, int topk, int32_t* ids, float* weights, int e_lo, int e_n, int shared_rows,

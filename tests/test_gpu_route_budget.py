@@ -272,3 +272,24 @@ def test_sigmoid_form_graph_replay():
         eager = call(f.cuda(), s.cuda())
         assert all(torch.equal(a.view(torch.int32) if a.dtype == torch.float32 else a, b.view(torch.int32) if b.dtype == torch.float32 else b)
                    for a, b in zip(out, eager))
+
+
+@pytest.mark.parametrize("experts", [48, 600])  # eight and sixteen logits a lane
+@pytest.mark.parametrize("m,steps", [(1, 1), (17, 1), (64, 8), (65, 1), (256, 4), (257, 1), (832, 8)])  # rows of a row plan, of a workgroup each, of sixteen a workgroup, of the shared plan
+def test_layer_selects_and_plans_in_one_launch(experts, m, steps):
+    """`moe_layer_budget` ranks, selects and plans in one launch whose last workgroup to arrive takes the last two; its slot table
+    ends behind the experts the selection can name (here the guaranteed ones, above and below the cap)."""
+    from hibana_amd import synthetic
+    from hibana_amd.kernels import ops, w3_moe
+    from tests.util import MAX_REL, NORM_REL, errors
+    ex, shared = synthetic.w3_experts(experts, 256, 128, True, 3), synthetic.w3_experts(1, 256, 128, True, 4)
+    g = torch.Generator().manual_seed(m)
+    x, logits = torch.randn(m, 256, generator=g).bfloat16().cuda(), (torch.randn(m, experts, generator=g) * 2).bfloat16().cuda()
+    slots = (torch.arange(m // steps) % 5 != 3).to(torch.int32).cuda()
+    for keep, budget, per_request in [(1, 24, 0), (3, 16, 2), (2, 0, 0), (0, 9, 0)]:
+        ids, wts = ops.route_budget(logits, 10, keep, budget, slots, steps, repeat=False, per_request=per_request, min_cap=6)
+        for _ in range(2):
+            got, got_ids, got_w = w3_moe.moe_layer_budget(ex, x, logits, 10, keep, budget, slots, steps, per_request=per_request, min_cap=6, shared=shared, return_routing=True)
+            assert torch.equal(got_ids, ids) and torch.equal(got_w, wts)
+            mx, nr = errors(got, w3_moe.moe_layer(ex, x, ids, wts, shared=shared))
+            assert mx < MAX_REL and nr < NORM_REL, (keep, budget, mx, nr)

@@ -533,6 +533,14 @@ using namespace hb;
 static StreamParams dense_params(const void* tiled, float scale, int n, int k, const void* x, int m, void* y) {
   StreamParams p{};
   p.w = static_cast<const uint8_t*>(tiled);
+  template <int K, bool AFTER_VALU>  // a product, then the first half of that
+  static __device__ __forceinline__ void product_first(f32x4_t& acc, const u32x4_t& w, const u32x4_t& a, const Part& part, panel_two_t& two) {
+    if constexpr (K == 0 && AFTER_VALU) HB_PANEL_PRODUCT_FIRST("s_nop 1\n\t", HB_FP4_CVT, "", acc, two, w, part.codes, part.scale, a);
+    if constexpr (K == 0 && !AFTER_VALU) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, "", acc, two, w, part.codes, part.scale, a);
+    if constexpr (K == 1) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, " op_sel:[1,0,0]", acc, two, w, part.codes, part.scale, a);
+    if constexpr (K == 2) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, " op_sel:[0,1,0]", acc, two, w, part.codes, part.scale, a);
+    if constexpr (K == 3) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, " op_sel:[1,1,0]", acc, two, w, part.codes, part.scale, a);
+  }
   p.scalar = scale;
   p.n_blocks = n / 64;
   p.chunks = k / 128;

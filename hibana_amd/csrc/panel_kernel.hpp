@@ -91,6 +91,18 @@ __device__ __forceinline__ void product(f32x4_t& acc, const u32x4_t& w, const u3
                : "v64", "v65")
 #define HB_PANEL_PAIR_ALONE(CONVERT, SELECT, out, from, scale) \
   asm volatile(CONVERT " v[64:65], %1, 1.0" SELECT "\n\tv_mul_f32 v64, v64, %2\n\tv_mul_f32 v65, v65, %2\n\tv_cvt_pk_bf16_f32 %0, v64, v65" : "=&v"(out) : "v"(from), "v"(scale) : "v64", "v65")
+// The same in two halves, behind a product each: convert and the first value's scale, then the second's and the rounding.
+// `two`: what is between them, bound to the fixed registers.
+#define HB_PANEL_PRODUCT_FIRST(NOP, CONVERT, SELECT, acc, two, w, from, scale, a)                            \
+  asm volatile(NOP "v_mfma_f32_16x16x32_bf16 %0, %2, %5, %0\n\t" CONVERT " v[64:65], %3, 1.0" SELECT "\n\tv_mul_f32 v64, v64, %4" \
+               : "+v"(acc), "=&{v[64:65]}"(two)                                                              \
+               : "v"(w), "v"(from), "v"(scale), "v"(a))
+typedef __attribute__((ext_vector_type(2))) float panel_two_t;
+__device__ __forceinline__ void product_second(f32x4_t& acc, const u32x4_t& w, const u32x4_t& a, panel_two_t& two, float scale, uint32_t& out) {
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %3, %5, %0\n\tv_mul_f32 v65, v65, %4\n\tv_cvt_pk_bf16_f32 %2, v64, v65"
+               : "+v"(acc), "+{v[64:65]}"(two), "=&v"(out)
+               : "v"(w), "v"(scale), "v"(a));
+}
 __device__ __forceinline__ void products_done(void) { asm volatile("s_nop 15\n\ts_nop 7" ::: "memory"); }
 
 template <class Fmt, int EPI, int MT>
@@ -104,8 +116,13 @@ struct Panel {
   f32x4_t acc[MT][4];
   u32x4_t now[MT];  // the activations' fragments of the step in hand
 
+  // From this many row tiles the products and not the expansion bound a fragment, and a product hides two vector instructions
+  // beside it but not four: the pairs are dealt out in halves. Two wavefronts a SIMD, cycles a fragment (the products alone 16
+  // each): eight tiles 150.8 with whole pairs and 136.5 with halves, seven 136.7 and 128.8, six 125.1 and 120.5, five 113.9 and 122.1.
+  static constexpr int HALVES_FROM = 6;
+
   // The products of fragment J = 4 * step + tile of a chunk, and between them the expansion of fragment J + 1, a pair of
-  // its values behind every MT / 4 products. The empty statements hold that order: left to itself the compiler puts the
+  // its values behind every MT / 4 products (or half a pair behind every MT / 8). The empty statements hold that order: left to itself the compiler puts the
   // expansion behind the products (fewer registers), where nothing runs beside it.
   // FRESH: the activations' fragments may still be on their way (asked for in order, nothing behind them). NEXT >= 0: the
   // LDS offset of the next step's, from `at`.
@@ -114,32 +131,48 @@ struct Panel {
     u32x4_t w = __builtin_bit_cast(u32x4_t, b);
     typename Fmt::Part part;
     uint32_t out[4] = {0u, 0u, 0u, 0u};
-    products<J, FRESH, NEXT, 0>(ch, sl, w, at, part, out);
+    panel_two_t two = {0.f, 0.f};
+    products<J, FRESH, NEXT, 0>(ch, sl, w, at, part, out, two);
     return __builtin_bit_cast(bf16x8_t, u32x4_t{out[0], out[1], out[2], out[3]});
   }
   template <int J, bool FRESH, int NEXT, int T>
-  __device__ __forceinline__ void products(const Chunk& ch, const Slot& sl, u32x4_t& w, uint32_t at, typename Fmt::Part& part, uint32_t (&out)[4]) {
+  __device__ __forceinline__ void products(const Chunk& ch, const Slot& sl, u32x4_t& w, uint32_t at, typename Fmt::Part& part, uint32_t (&out)[4],
+                                           panel_two_t& two) {
     constexpr int NT = J & 3;
     if constexpr (T < MT) {
       if constexpr (FRESH) {
         asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(MT - 1 - T) : "memory");
         pin(now[T]);
       }
-      constexpr int K = (4 * T + MT - 1) / MT;  // the pairs are dealt out evenly: pair K goes behind product K MT / 4
-      constexpr bool FIRST = J < 15 && K < 4 && K * MT / 4 == T;
       if constexpr (J < 15 && T == 0) part = Fmt::template open<((J + 1) & 3), ((J + 1) >> 2)>(ch, sl);
-      if constexpr (FIRST) {
-        Fmt::template product_pair<K, T == 0>(acc[T][NT], w, now[T], part, out[K]);
+      if constexpr (MT >= HALVES_FROM) {  // halves of pairs: half I goes behind product I MT / 8
+        constexpr int I = (8 * T + MT - 1) / MT;
+        static_assert(I * MT / 8 == T && I < 8, "a half for every product");
+        if constexpr (J >= 15) {
+          product<T == 0>(acc[T][NT], w, now[T]);
+        } else if constexpr (I & 1) {
+          product_second(acc[T][NT], w, now[T], two, part.scale, out[I >> 1]);
+        } else if constexpr ((I + 1) * MT / 8 == T) {
+          Fmt::template product_pair<(I >> 1), T == 0>(acc[T][NT], w, now[T], part, out[I >> 1]);
+        } else {
+          Fmt::template product_first<(I >> 1), T == 0>(acc[T][NT], w, now[T], part, two);
+        }
       } else {
-        product<T == 0>(acc[T][NT], w, now[T]);
-      }
-      if constexpr (FIRST && K + 1 < 4 && (K + 1) * MT / 4 == T) Fmt::template pair_alone<(K + 1) & 3>(part, out[(K + 1) & 3]);
-      if constexpr (FIRST && MT == 1) {
-        Fmt::template pair_alone<2>(part, out[2]);
-        Fmt::template pair_alone<3>(part, out[3]);
+        constexpr int K = (4 * T + MT - 1) / MT;  // the pairs are dealt out evenly: pair K goes behind product K MT / 4
+        constexpr bool FIRST = J < 15 && K < 4 && K * MT / 4 == T;
+        if constexpr (FIRST) {
+          Fmt::template product_pair<K, T == 0>(acc[T][NT], w, now[T], part, out[K]);
+        } else {
+          product<T == 0>(acc[T][NT], w, now[T]);
+        }
+        if constexpr (FIRST && K + 1 < 4 && (K + 1) * MT / 4 == T) Fmt::template pair_alone<(K + 1) & 3>(part, out[(K + 1) & 3]);
+        if constexpr (FIRST && MT == 1) {
+          Fmt::template pair_alone<2>(part, out[2]);
+          Fmt::template pair_alone<3>(part, out[3]);
+        }
       }
       if constexpr (NEXT >= 0) ask_lds<NEXT + T * 2048>(now[T], at);
-      products<J, FRESH, NEXT, T + 1>(ch, sl, w, at, part, out);
+      products<J, FRESH, NEXT, T + 1>(ch, sl, w, at, part, out, two);
     }
   }
   static __device__ __forceinline__ bf16x8_t whole(const Chunk& ch, const Slot& sl) {  // fragment 0 of a chunk

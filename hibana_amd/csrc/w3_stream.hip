@@ -1032,6 +1032,14 @@ struct TileW3 {
     if constexpr (K == 2) HB_PANEL_PRODUCT_PAIR("", HB_W3_CVT, "", acc, out, w, part.hi, part.scale, a);
     if constexpr (K == 3) HB_PANEL_PRODUCT_PAIR("", HB_W3_CVT, " op_sel:[1,0,0]", acc, out, w, part.hi, part.scale, a);
   }
+  template <int K, bool AFTER_VALU>  // a product, then the first half of that
+  static __device__ __forceinline__ void product_first(f32x4_t& acc, const u32x4_t& w, const u32x4_t& a, const Part& part, panel_two_t& two) {
+    if constexpr (K == 0 && AFTER_VALU) HB_PANEL_PRODUCT_FIRST("s_nop 1\n\t", HB_W3_CVT, "", acc, two, w, part.lo, part.scale, a);
+    if constexpr (K == 0 && !AFTER_VALU) HB_PANEL_PRODUCT_FIRST("", HB_W3_CVT, "", acc, two, w, part.lo, part.scale, a);
+    if constexpr (K == 1) HB_PANEL_PRODUCT_FIRST("", HB_W3_CVT, " op_sel:[1,0,0]", acc, two, w, part.lo, part.scale, a);
+    if constexpr (K == 2) HB_PANEL_PRODUCT_FIRST("", HB_W3_CVT, "", acc, two, w, part.hi, part.scale, a);
+    if constexpr (K == 3) HB_PANEL_PRODUCT_FIRST("", HB_W3_CVT, " op_sel:[1,0,0]", acc, two, w, part.hi, part.scale, a);
+  }
   template <int K>
   static __device__ __forceinline__ void pair_alone(const Part& part, uint32_t& out) {
     if constexpr (K == 0) HB_PANEL_PAIR_ALONE(HB_W3_CVT, "", out, part.lo, part.scale);

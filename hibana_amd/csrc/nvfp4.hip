@@ -462,9 +462,31 @@ static int shape_nvfp4(StreamParams& p, int64_t busy_slots) {
   return HB_OK;
 }
 
+// The shape of a dense call of one slot: K split eight ways as far as there are chunks, since a wavefront's start and the
+// exchange cost about as much as two or three of them. Measured, a replayed graph of calls, the general rule and this one (us,
+// blocks x chunks): twelve rows 16 x 12 10.8 and 5.4, 160 x 12 12.0 and 6.0, 400 x 16 12.5 and 10.9, 640 x 4 8.3 and 6.8, 800 x 8
+// 13.2 and 10.9; eight rows 80 x 12 8.2 and 5.6, 400 x 16 10.4 and 9.5, 640 x 12 13.2 and 10.8; one row 80 x 4 4.9 and 4.4. With
+// few rows and many blocks short of K the launch is bound by its traffic, and fewer wavefronts are better: 640 x 7 one row 7.0 by the
+// general rule and 7.8 split four ways, 520 x 8 8.4, split eight ways 9.0, four ways 8.2; and from 768 blocks eight wavefronts
+// on four blocks: 800 x 40 one row 27.6 and 25.8, 800 x 16 14.3 and 13.1, eight rows 15.6 and 15.5.
+static void shape_nvfp4_dense(StreamParams& p) {
+  const bool few = p.m <= FP4_FEW_ROWS && !p.no_few;
+  int most = 8;
+  if (few && p.n_blocks >= 768) {
+    if (p.chunks >= 12) p.ks = 2, p.nbw = 4;
+    most = 0;
+  } else if (few && p.n_blocks > 300 && p.chunks < 12) {
+    most = p.chunks >= 8 ? 4 : 0;
+  }
+  while (p.ks < most && 2 * p.ks <= p.chunks) p.ks *= 2;
+  if (p.ks >= 4) p.nbw = 1;
+  set_split(p);
+}
+
 template <int EPI>
 static int launch_nvfp4(StreamParams& p, int64_t slots, int64_t busy_slots, hipStream_t stream) {
   if (int e = shape_nvfp4(p, busy_slots)) return e;
+  if (epi_dense(EPI) && slots == 1 && !g_nvfp4_ksplit) shape_nvfp4_dense(p);
   const dim3 grid((unsigned)((p.n_blocks + p.nbw - 1) / p.nbw), (unsigned)slots);
   const int waves = p.ks * p.nbw;
   HB_LAUNCH(nvfp4_stream_kernel<EPI>, grid, dim3(64 * waves), (size_t)waves * FP4_RING_BYTES, stream, p);
@@ -511,6 +533,14 @@ struct TileNvfp4 {
     if constexpr (K == 2) HB_PANEL_PRODUCT_PAIR("", HB_FP4_CVT, " op_sel:[0,1,0]", acc, out, w, part.codes, part.scale, a);
     if constexpr (K == 3) HB_PANEL_PRODUCT_PAIR("", HB_FP4_CVT, " op_sel:[1,1,0]", acc, out, w, part.codes, part.scale, a);
   }
+  template <int K, bool AFTER_VALU>  // a product, then the first half of that
+  static __device__ __forceinline__ void product_first(f32x4_t& acc, const u32x4_t& w, const u32x4_t& a, const Part& part, panel_two_t& two) {
+    if constexpr (K == 0 && AFTER_VALU) HB_PANEL_PRODUCT_FIRST("s_nop 1\n\t", HB_FP4_CVT, "", acc, two, w, part.codes, part.scale, a);
+    if constexpr (K == 0 && !AFTER_VALU) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, "", acc, two, w, part.codes, part.scale, a);
+    if constexpr (K == 1) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, " op_sel:[1,0,0]", acc, two, w, part.codes, part.scale, a);
+    if constexpr (K == 2) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, " op_sel:[0,1,0]", acc, two, w, part.codes, part.scale, a);
+    if constexpr (K == 3) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, " op_sel:[1,1,0]", acc, two, w, part.codes, part.scale, a);
+  }
   template <int K>
   static __device__ __forceinline__ void pair_alone(const Part& part, uint32_t& out) {
     if constexpr (K == 0) HB_PANEL_PAIR_ALONE(HB_FP4_CVT, "", out, part.codes, part.scale);
@@ -533,14 +563,6 @@ using namespace hb;
 static StreamParams dense_params(const void* tiled, float scale, int n, int k, const void* x, int m, void* y) {
   StreamParams p{};
   p.w = static_cast<const uint8_t*>(tiled);
-  template <int K, bool AFTER_VALU>  // a product, then the first half of that
-  static __device__ __forceinline__ void product_first(f32x4_t& acc, const u32x4_t& w, const u32x4_t& a, const Part& part, panel_two_t& two) {
-    if constexpr (K == 0 && AFTER_VALU) HB_PANEL_PRODUCT_FIRST("s_nop 1\n\t", HB_FP4_CVT, "", acc, two, w, part.codes, part.scale, a);
-    if constexpr (K == 0 && !AFTER_VALU) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, "", acc, two, w, part.codes, part.scale, a);
-    if constexpr (K == 1) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, " op_sel:[1,0,0]", acc, two, w, part.codes, part.scale, a);
-    if constexpr (K == 2) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, " op_sel:[0,1,0]", acc, two, w, part.codes, part.scale, a);
-    if constexpr (K == 3) HB_PANEL_PRODUCT_FIRST("", HB_FP4_CVT, " op_sel:[1,1,0]", acc, two, w, part.codes, part.scale, a);
-  }
   p.scalar = scale;
   p.n_blocks = n / 64;
   p.chunks = k / 128;

@@ -444,8 +444,8 @@ __device__ __forceinline__ void plan_work(const int32_t* ids, int pairs, int e_l
   }
 }
 
-// With `route.logits` set the workgroup first routes the route_rows rows itself (softmax top-k, a row a wavefront at a
-// time) into route.ids / route.weights, which `ids` then names.
+// With `route.logits` set the workgroup first routes the route_rows rows itself (a row a wavefront: at most
+// ROUTE_FUSED_ROWS) into route.ids / route.weights, which `ids` then names; `by_rows`: none of them names an expert twice.
 //
 // With `job.lanes` set the launch has further workgroups, which round the job's activations to E4M3 and plan nothing.
 //
@@ -456,18 +456,22 @@ __device__ __forceinline__ void plan_work(const int32_t* ids, int pairs, int e_l
 template <bool WIDE>
 __global__ __launch_bounds__(PLAN_THREADS) void moe_plan_kernel(const int32_t* ids, int pairs, int e_lo, int e_n, int shared_rows,
                                                                 int32_t* __restrict__ plan, int32_t* __restrict__ order, RouteParams route,
-                                                                int route_rows, int slot_rows, int slot_cap, int32_t* __restrict__ wide, int groups,
-                                                                int phase, QuantJob job) {
+                                                                int route_rows, int by_rows, int slot_rows, int slot_cap, int32_t* __restrict__ wide,
+                                                                int groups, int phase, QuantJob job) {
   extern __shared__ int lds[];
   if (!WIDE && blockIdx.x > 0) {  // the workgroups beside the plan's: the activation rounding
     quant_job_share(job, blockIdx.x - 1, reinterpret_cast<float*>(lds));
     return;
   }
-  if (route.logits) {
-    for (int r = threadIdx.x >> 6; r < route_rows; r += PLAN_WAVES) {
-      route_any(route, r, threadIdx.x & 63);
-    }
+  if (!WIDE && route.logits) {
+    // (a loop over the rows keeps what no row changes in registers, and spills: latent block of four rows 83.8 us, without 82.0)
+    const int r = threadIdx.x >> 6;
+    if (r < route_rows) route_any(route, r, threadIdx.x & 63);
     __syncthreads();
+  }
+  if (!WIDE && by_rows) {
+    plan_by_rows(ids, route_rows, route.k, e_lo, e_n, shared_rows, plan, order, slot_rows, slot_cap, lds);
+    return;
   }
   plan_work<WIDE>(ids, pairs, e_lo, e_n, shared_rows, plan, order, slot_rows, slot_cap, wide, groups, phase, blockIdx.x, lds);
 }
@@ -968,11 +972,11 @@ int moe_launch_plan(const int32_t* ids, int64_t pairs, int e_lo, int e_n, int sh
     if (job) moe_launch_quant_groups(*job, stream);
     for (int phase = 1; phase <= 3; phase++)
       HB_LAUNCH(moe_plan_kernel<true>, dim3(phase == 2 ? 1 : groups), dim3(PLAN_THREADS), plan_lds, stream, ids, (int)pairs, e_lo, e_n, shared_rows, ws.plan,
-                ws.order, RouteParams{}, 0, slot_rows, slot_cap, ws.plan_wide, groups, phase, QuantJob{});
+                ws.order, RouteParams{}, 0, 0, slot_rows, slot_cap, ws.plan_wide, groups, phase, QuantJob{});
     return HB_OK;
   }
   HB_LAUNCH(moe_plan_kernel<false>, dim3(plan_groups(job)), dim3(PLAN_THREADS), plan_lds, stream, ids, (int)pairs, e_lo, e_n, shared_rows, ws.plan, ws.order,
-            RouteParams{}, 0, slot_rows, slot_cap, ws.plan_wide, 1, 0, job ? *job : QuantJob{});
+            RouteParams{}, 0, 0, slot_rows, slot_cap, ws.plan_wide, 1, 0, job ? *job : QuantJob{});
   return HB_OK;
 }
 
@@ -984,11 +988,11 @@ static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, in
   const int64_t pairs = (int64_t)m * rp.k;
   const size_t plan_lds = ((size_t)(PLAN_WAVES + 1) * e_n + 3 * (PLAN_WAVES + 1)) * sizeof(int);
   if (plan_lds > 64 * 1024 || e_n > PLAN_THREADS || pairs > 0x3fffffff) return HB_EINVAL;
+  // rows that name no expert twice: every row is real, or a padded row names none (with `repeat` it names one over and over)
+  const int by_rows = (!rp.slots || (!rp.repeat && (rp.pad_id < e_lo || rp.pad_id >= e_lo + e_n))) && m <= PLAN_ROWS_MAX && rp.k <= 64 && g_route_plan_fused.load(std::memory_order_relaxed) != 1;
   if (m > ROUTE_FUSED_ROWS && pairs < PLAN_WIDE_PAIRS && g_route_plan_fused.load(std::memory_order_relaxed) != 2) {
     // a verify-sized call: the routing spread over the device, the plan by the workgroup that finishes last
     const int groups = (m + ROUTE_GROUP_ROWS - 1) / ROUTE_GROUP_ROWS;
-    // rows that name no expert twice: every row is real, or a padded row names none (with `repeat` it names one over and over)
-    const int by_rows = (!rp.slots || (!rp.repeat && (rp.pad_id < e_lo || rp.pad_id >= e_lo + e_n))) && m <= PLAN_ROWS_MAX && rp.k <= 64 && g_route_plan_fused.load(std::memory_order_relaxed) != 1;
     HB_LAUNCH(moe_route_plan_kernel, dim3((unsigned)groups + plan_groups(job) - 1u), dim3(PLAN_THREADS), plan_lds, stream, rp.ids, (int)pairs, e_lo, e_n,
               shared_rows, ws.plan, ws.order, rp, m, groups, by_rows, slot_rows, (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows),
               job ? *job : QuantJob{});
@@ -1002,8 +1006,9 @@ static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, in
     }
     return moe_launch_plan(rp.ids, pairs, e_lo, e_n, shared_rows, ws, stream, slot_rows, job);
   }
+  static_assert(ROUTE_FUSED_ROWS <= PLAN_WAVES, "a wavefront a row");
   HB_LAUNCH(moe_plan_kernel<false>, dim3(plan_groups(job)), dim3(PLAN_THREADS), plan_lds, stream, rp.ids, (int)pairs, e_lo, e_n, shared_rows, ws.plan, ws.order,
-            rp, m, slot_rows, (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows), ws.plan_wide, 1, 0, job ? *job : QuantJob{});
+            rp, m, by_rows && pairs > 64, slot_rows, (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows), ws.plan_wide, 1, 0, job ? *job : QuantJob{});  // (up to 64 pairs one wavefront plans)
   return HB_OK;
 }
 

@@ -492,7 +492,7 @@ __device__ __forceinline__ int last_to_arrive(int32_t* plan, int groups) {
   return last;
 }
 
-// Routing and plan of a verify-sized call in ONE launch: `route_groups` workgroups route ROUTE_GROUP_ROWS rows each (a
+// Routing and plan of a verify-sized call in ONE launch: `route_groups` workgroups route `group_rows` rows each (a
 // row a wavefront, spread over the device, as the routing launch does), and the one that finishes last plans - it
 // learns that it is the last from an arrival counter in the call's own workspace (plan[PLAN_TICKET]: zero when the
 // caller hands the workspace over, put back to zero by every last arriver, as the split-K counters of the reference's
@@ -501,11 +501,9 @@ __device__ __forceinline__ int last_to_arrive(int32_t* plan, int groups) {
 // the plan reads ids past its own L2 (store_through / load_through): no cache write-back, no invalidate. Nobody
 // waits: a workgroup that is not the last leaves. `by_rows`: the rows name no expert twice and are at most
 // PLAN_ROWS_MAX (plan_by_rows). Workgroups past the routing ones round the job's activations, as in moe_plan_kernel.
-constexpr int ROUTE_GROUP_ROWS = 1;
-
 __global__ __launch_bounds__(PLAN_THREADS) void moe_route_plan_kernel(const int32_t* ids, int pairs, int e_lo, int e_n, int shared_rows,
                                                                       int32_t* __restrict__ plan, int32_t* __restrict__ order, RouteParams route,
-                                                                      int route_rows, int route_groups, int by_rows, int slot_rows, int slot_cap,
+                                                                      int route_rows, int route_groups, int group_rows, int by_rows, int slot_rows, int slot_cap,
                                                                       QuantJob job) {
   extern __shared__ int lds[];
   __shared__ int last;
@@ -513,13 +511,13 @@ __global__ __launch_bounds__(PLAN_THREADS) void moe_route_plan_kernel(const int3
     quant_job_share(job, blockIdx.x - route_groups, reinterpret_cast<float*>(lds));
     return;
   }
-  const int wave = threadIdx.x >> 6, r = blockIdx.x * ROUTE_GROUP_ROWS + wave;
-  if (wave < ROUTE_GROUP_ROWS && r < route_rows) {
+  const int wave = threadIdx.x >> 6, r = blockIdx.x * group_rows + wave;
+  if (wave < group_rows && r < route_rows) {
     route_any(route, r, threadIdx.x & 63);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this row's ids (write-through stores) have reached memory before the ticket is drawn
-  } else if (by_rows && wave >= ROUTE_GROUP_ROWS) {
-    constexpr int IDLE = PLAN_THREADS - 64 * ROUTE_GROUP_ROWS;  // meanwhile, the wavefronts that route nothing
-    clear_plan(plan, slot_cap, blockIdx.x * IDLE + (int)threadIdx.x - 64 * ROUTE_GROUP_ROWS, route_groups * IDLE);
+  } else if (by_rows) {  // (one row a group) meanwhile, the wavefronts that route nothing
+    constexpr int IDLE = PLAN_THREADS - 64;
+    clear_plan(plan, slot_cap, blockIdx.x * IDLE + (int)threadIdx.x - 64, route_groups * IDLE);
   }
   __syncthreads();
   if (threadIdx.x == 0) last = last_to_arrive(plan, route_groups);
@@ -982,6 +980,10 @@ int moe_launch_plan(const int32_t* ids, int64_t pairs, int e_lo, int e_n, int sh
 
 int moe_check_route(int m, int e, int k) { return m <= 0 || e <= 0 || k <= 0 || k > e || k > 64 || e > 64 * ROUTE_PER_LANE ? HB_EINVAL : HB_OK; }
 
+// From more rows than compute units a workgroup routes several: each is a full one, of which a compute unit holds two, and all
+// draw tickets from one counter (800 rows of 512 experts, the whole layer 272.0 us with a row each, 263.7 with eight, 265.3 with
+// sixteen; 400 rows 169.7, 167.5, 168.9; at 200 rows and fewer no gain).
+constexpr int ROUTE_GROUP_ROWS = 8, ROUTE_SPREAD_ROWS = 256;
 // Routing by `rp` (either rule) and the plan of its ids, in as few launches as the size allows.
 static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, int shared_rows, const MoeWorkspace& ws, hipStream_t stream, int slot_rows,
                              const QuantJob* job) {
@@ -992,9 +994,9 @@ static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, in
   const int by_rows = (!rp.slots || (!rp.repeat && (rp.pad_id < e_lo || rp.pad_id >= e_lo + e_n))) && m <= PLAN_ROWS_MAX && rp.k <= 64 && g_route_plan_fused.load(std::memory_order_relaxed) != 1;
   if (m > ROUTE_FUSED_ROWS && pairs < PLAN_WIDE_PAIRS && g_route_plan_fused.load(std::memory_order_relaxed) != 2) {
     // a verify-sized call: the routing spread over the device, the plan by the workgroup that finishes last
-    const int groups = (m + ROUTE_GROUP_ROWS - 1) / ROUTE_GROUP_ROWS;
+    const int group_rows = m <= ROUTE_SPREAD_ROWS ? 1 : ROUTE_GROUP_ROWS, groups = (m + group_rows - 1) / group_rows;
     HB_LAUNCH(moe_route_plan_kernel, dim3((unsigned)groups + plan_groups(job) - 1u), dim3(PLAN_THREADS), plan_lds, stream, rp.ids, (int)pairs, e_lo, e_n,
-              shared_rows, ws.plan, ws.order, rp, m, groups, by_rows, slot_rows, (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows),
+              shared_rows, ws.plan, ws.order, rp, m, groups, group_rows, by_rows, slot_rows, (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows),
               job ? *job : QuantJob{});
     return HB_OK;
   }

@@ -66,3 +66,18 @@ def test_a_router_off_the_vector_boundary(m):
     slice_ = torch.cat([router.new_zeros(4), router.flatten()])[4:].view_as(router)
     assert slice_.data_ptr() % 16 == 8 and slice_.is_contiguous()
     assert torch.equal(MoeLayer(slice_, gate, ex, 6, shared=shared)(x), MoeLayer(router, gate, ex, 6, shared=shared)(x))
+
+
+@pytest.mark.parametrize("m", [256, 257, 263, 640])
+def test_layer_routes_several_rows_a_workgroup(m):
+    """From more rows than compute units the routing launch gives a workgroup eight rows; the last one to arrive plans."""
+    from hibana_amd import synthetic
+    from hibana_amd.kernels import ops, w3_moe
+    ex = synthetic.w3_experts(48, 256, 128, True, 3)
+    g = torch.Generator().manual_seed(m)
+    x, logits = torch.randn(m, 256, generator=g).bfloat16().cuda(), (torch.randn(m, 48, generator=g) * 2).cuda()
+    ids, wts = ops.route_topk(logits, 6)
+    want = w3_moe.moe_layer(ex, x, ids, wts)
+    for _ in range(2):
+        got, got_ids, got_w = w3_moe.moe_layer_logits(ex, x, logits, 6, return_routing=True)
+        assert torch.equal(got_ids, ids) and torch.equal(got_w, wts) and torch.equal(got, want)

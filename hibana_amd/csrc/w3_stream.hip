@@ -608,6 +608,50 @@ struct FullActs8 {
   }
 };
 
+// The sixteen-row bodies over the 16-row tiles T0 .. T1 - 1 of the block only (the other accumulators stay zero).
+template <int T0, int T1>
+struct FullActsPart : FullActs {
+  template <int HALF, class C>
+  static __device__ __forceinline__ void half(const C& ch, const u32x4_t& a_lo, const u32x4_t& a_hi, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot& sl) {
+    if (T0 <= 0 && 0 < T1) compute_half_tile<HALF, 0>(ch, a_lo, a_hi, acc0, sl.lut_lo, sl.lut_hi);
+    if (T0 <= 1 && 1 < T1) compute_half_tile<HALF, 1>(ch, a_lo, a_hi, acc1, sl.lut_lo, sl.lut_hi);
+    if (T0 <= 2 && 2 < T1) compute_half_tile<HALF, 2>(ch, a_lo, a_hi, acc2, sl.lut_lo, sl.lut_hi);
+    if (T0 <= 3 && 3 < T1) compute_half_tile<HALF, 3>(ch, a_lo, a_hi, acc3, sl.lut_lo, sl.lut_hi);
+  }
+  template <int ODD, bool MORE2, bool MORE1, class C>
+  __device__ __forceinline__ void step(const C& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot& sl) {
+    const uint16_t* next = at + (int64_t)(i + 1) * 128;
+    half<0>(ch, held.a0, held.a1, acc0, acc1, acc2, acc3, sl);
+    if (MORE1) {
+      held.a0 = *reinterpret_cast<const u32x4_t*>(next);
+      held.a1 = *reinterpret_cast<const u32x4_t*>(next + 32);
+    }
+    half<1>(ch, held.a2, held.a3, acc0, acc1, acc2, acc3, sl);
+    if (MORE1) {
+      held.a2 = *reinterpret_cast<const u32x4_t*>(next + 64);
+      held.a3 = *reinterpret_cast<const u32x4_t*>(next + 96);
+    }
+  }
+};
+template <int T0, int T1>
+struct FullActs8Part : FullActs8 {
+  static constexpr int LOADS = 8;  // at least: with a tile or two between them the compiler makes one load of a row's two scale pairs (twelve waited for too little)
+  template <int HALF, class C>
+  __device__ __forceinline__ void half(const C& ch, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot& sl) const {
+    if (T0 <= 0 && 0 < T1) half_tile<HALF, 0>(ch, acc0, sl.lut_lo, sl.lut_hi);
+    if (T0 <= 1 && 1 < T1) half_tile<HALF, 1>(ch, acc1, sl.lut_lo, sl.lut_hi);
+    if (T0 <= 2 && 2 < T1) half_tile<HALF, 2>(ch, acc2, sl.lut_lo, sl.lut_hi);
+    if (T0 <= 3 && 3 < T1) half_tile<HALF, 3>(ch, acc3, sl.lut_lo, sl.lut_hi);
+  }
+  template <int ODD, bool MORE2, bool MORE1, class C>
+  __device__ __forceinline__ void step(const C& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot& sl) {
+    half<0>(ch, acc0, acc1, acc2, acc3, sl);
+    if (MORE1) load_half(0, i + 1);
+    half<1>(ch, acc0, acc1, acc2, acc3, sl);
+    if (MORE1) load_half(1, i + 1);
+  }
+};
+
 // The end of a 64-row block for a slot of at most four rows. Lane (g, r16) of each of the block's K splits holds, in
 // register r of accumulator t, group g's part of (tile t, slot row r, column r16): sixteen values a lane, each to be
 // added over the four groups and the splits. They go to LDS, and the workgroup's 64 x ks lanes share the 16 x 16
@@ -741,23 +785,48 @@ __global__ __launch_bounds__(1024) void w3_stream_kernel(StreamParams p) {
   stream_workgroup<EPI, A8, SPLIT, W3RingOf<2, BITS>>(p, sl, blockIdx.x, rings);
 }
 
-// A dense call of at most four rows whose blocks are fewer than half the compute units: PARTS workgroups a 64-row block,
+// A dense call of one slot whose blocks are fewer than half the compute units: PARTS workgroups a 64-row block,
 // each its 4 / PARTS 16-row tiles (of the block's loads it asks only for those with its tiles' dwords, and the ones that two
 // parts need come from the L2 the second time: a block's workgroups are on one die). The sums and their order are those of
 // the one workgroup. What bounds the undivided launch is the expansion on a third of the device.
-template <bool A8, int T0, int T1>
+template <bool A8, bool FEW, int T0, int T1>
 __device__ __forceinline__ void part_block(const StreamParams& p, const Slot& sl, int nb, const WaveShare& share, int lane, int wave, uint8_t* rings) {
   f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0, acc2 = acc0, acc3 = acc0;
-  const float scale = sl.rs[nb * 64 + lane];
   uint8_t* ring = rings + wave * RING_BYTES;
-  if constexpr (A8) {
-    stream_block<EPI_DENSE, FewActs8Part<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+  if constexpr (FEW) {
+    const float scale = sl.rs[nb * 64 + lane];
+    if constexpr (A8) {
+      stream_block<EPI_DENSE, FewActs8Part<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+    } else {
+      stream_block<EPI_DENSE, FewActsPart<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+    }
+    finish_few<EPI_DENSE>(p, sl, 0, scale, nb, true, wave, share.ks, 0, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3, FewPairs{}, FewScales{}, T0, T1);
   } else {
-    stream_block<EPI_DENSE, FewActsPart<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+    if constexpr (A8) {
+      stream_block<EPI_DENSE, FullActs8Part<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+    } else {
+      stream_block<EPI_DENSE, FullActsPart<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+    }
+    // finish_block for these tiles: the splits' sums through LDS, added in split order, an accumulator register a split and turn
+    const RowScales rs = row_scales<true>(sl, nb, lane & 15);
+    const f32x4_t all[4] = {acc0, acc1, acc2, acc3};
+    float* first = reinterpret_cast<float*>(rings);
+    float* mine = first + wave * (RING_BYTES / 4);
+#pragma unroll
+    for (int t = T0; t < T1; t++)
+#pragma unroll
+      for (int r = 0; r < 4; r++) mine[(t * 4 + r) * 64 + lane] = all[t][r];
+    __syncthreads();
+    for (int idx = 4 * T0 + share.ks; idx < 4 * T1; idx += p.ks) {
+      const int t = idx >> 2, r = idx & 3;
+      if (r >= sl.rows) continue;
+      float v = 0.f;
+      for (int s = 0; s < p.ks; s++) v += first[s * (RING_BYTES / 4) + idx * 64 + lane];
+      emit<EPI_DENSE, true>(p, sl, rs, nb, t, r, lane >> 4, lane & 15, v, 0.f);
+    }
   }
-  finish_few<EPI_DENSE>(p, sl, 0, scale, nb, true, wave, share.ks, 0, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3, FewPairs{}, FewScales{}, T0, T1);
 }
-template <bool A8, int PARTS>
+template <bool A8, bool FEW, int PARTS>
 __global__ __launch_bounds__(1024) void w3_part_kernel(StreamParams p) {
   extern __shared__ __align__(16) uint8_t rings[];
   const int die = blockIdx.x & 7, local = blockIdx.x >> 3, part = local % PARTS, nb = local / PARTS * 8 + die;
@@ -766,12 +835,12 @@ __global__ __launch_bounds__(1024) void w3_part_kernel(StreamParams p) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const WaveShare share = wave_share(p, wave);
   if constexpr (PARTS == 2) {
-    if (part == 0) part_block<A8, 0, 2>(p, sl, nb, share, lane, wave, rings); else part_block<A8, 2, 4>(p, sl, nb, share, lane, wave, rings);
+    if (part == 0) part_block<A8, FEW, 0, 2>(p, sl, nb, share, lane, wave, rings); else part_block<A8, FEW, 2, 4>(p, sl, nb, share, lane, wave, rings);
   } else {
-    if (part == 0) part_block<A8, 0, 1>(p, sl, nb, share, lane, wave, rings);
-    else if (part == 1) part_block<A8, 1, 2>(p, sl, nb, share, lane, wave, rings);
-    else if (part == 2) part_block<A8, 2, 3>(p, sl, nb, share, lane, wave, rings);
-    else part_block<A8, 3, 4>(p, sl, nb, share, lane, wave, rings);
+    if (part == 0) part_block<A8, FEW, 0, 1>(p, sl, nb, share, lane, wave, rings);
+    else if (part == 1) part_block<A8, FEW, 1, 2>(p, sl, nb, share, lane, wave, rings);
+    else if (part == 2) part_block<A8, FEW, 2, 3>(p, sl, nb, share, lane, wave, rings);
+    else part_block<A8, FEW, 3, 4>(p, sl, nb, share, lane, wave, rings);
   }
 }
 
@@ -1109,26 +1178,36 @@ static void shape_dense(StreamParams& p) {
   set_split(p);
 }
 
-// Blocks up to which a dense call of at most four rows gives a block's tiles to two workgroups (up to half of them: to
-// four). 5120 x 5120 at one row 7.7 -> 6.4 us; the dense block at four rows (its down projection is 5120 x 25600) 50.5 -> 46.7.
+// Blocks up to which a dense call of one slot gives a block's tiles to two workgroups (up to half of them: to four).
+// 5120 x 5120 at one row 7.7 -> 6.4 us; the dense block at four rows (its down projection is 5120 x 25600) 50.5 -> 46.7. Five to
+// sixteen rows, replayed graphs, eight rows: 1024 x 4096 7.8 -> 5.5 us, 4096 x 5120 9.5 -> 6.6, 8192 x 5120 9.9 -> 7.5; the dense
+// block of ten rows (4096, 8192), whose down projection takes E4M3 activations, 31.2 -> 24.8.
 constexpr int PARTS_BLOCKS = 128;
 template <int EPI>
 static int launch_stream(StreamParams& p, int64_t slots, int64_t busy_slots, Launch want, hipStream_t stream, int bits = 3) {
   if (int e = shape_stream(p, busy_slots, want)) return e;
   if constexpr (EPI == EPI_DENSE) {
-    if (bits == 3 && p.m <= FEW_ROWS && p.n_blocks <= PARTS_BLOCKS && !want.ks && !want.nbw && !p.no_few && !p.a2) {
+    const bool chosen = slots == 1 && !want.ks && !want.nbw && !p.a2, few = p.m <= FEW_ROWS;
+    const bool parted = bits == 3 && p.n_blocks <= PARTS_BLOCKS && !(few && p.no_few);
+    if (chosen && !p.aq && !(parted && few)) shape_dense(p);
+    if (chosen && parted) {
       p.nbw = 1;
       const int parts = p.n_blocks <= PARTS_BLOCKS / 2 ? 4 : 2;
       const dim3 blocks((unsigned)((p.n_blocks + 7) / 8 * 8 * parts));
       auto launch = [&](auto kernel) { HB_LAUNCH(kernel, blocks, dim3(64 * p.ks), (size_t)p.ks * RING_BYTES, stream, p); };
-      if (p.aq) {
-        parts == 4 ? launch(w3_part_kernel<true, 4>) : launch(w3_part_kernel<true, 2>);
+      if (few) {
+        if (p.aq) {
+          parts == 4 ? launch(w3_part_kernel<true, true, 4>) : launch(w3_part_kernel<true, true, 2>);
+        } else {
+          parts == 4 ? launch(w3_part_kernel<false, true, 4>) : launch(w3_part_kernel<false, true, 2>);
+        }
+      } else if (p.aq) {
+        parts == 4 ? launch(w3_part_kernel<true, false, 4>) : launch(w3_part_kernel<true, false, 2>);
       } else {
-        parts == 4 ? launch(w3_part_kernel<false, 4>) : launch(w3_part_kernel<false, 2>);
+        parts == 4 ? launch(w3_part_kernel<false, false, 4>) : launch(w3_part_kernel<false, false, 2>);
       }
       return HB_OK;
     }
-    if (slots == 1 && !p.aq && !p.a2 && !want.ks && !want.nbw) shape_dense(p);
   }
   const dim3 grid((unsigned)((p.n_blocks + p.nbw - 1) / p.nbw), (unsigned)slots);
   const int waves = p.ks * p.nbw;

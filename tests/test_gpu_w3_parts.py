@@ -30,3 +30,20 @@ def test_parts_of_a_block_against_the_product_and_the_sixteen_row_body(n, k):
             _lib.lib().hb_tune(b"w3_few", 0)
         mx, nr = errors(got, full)
         assert mx < MAX_REL and nr < NORM_REL, (m, mx, nr)
+
+
+@pytest.mark.parametrize("n", [64, 1152, 4096, 4160, 8192])  # one, 18 and 64 blocks in four parts, 65 and 128 in two
+@pytest.mark.parametrize("k", [128, 640, 2048, 5120])  # one chunk of K, fewer and more chunks than splits
+def test_parts_of_a_block_on_the_sixteen_row_bodies(n, k):
+    from hibana_amd import synthetic
+    from hibana_amd.kernels import w3
+    mat = synthetic.w3_matrix(n, k, n + k)
+    dense = w3.dequantize(mat).double()
+    for m in (5, 7, 8, 13, 16):
+        x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).bfloat16().cuda()
+        q, s = w3.quant_groups(x)
+        for _ in range(3):  # a read of the ring ahead of its data would not be wrong every time
+            mx, nr = errors(w3.w3_linear(x, mat), x.double() @ dense.T)
+            assert mx < MAX_REL and nr < NORM_REL, (m, mx, nr)
+            mx, nr = errors(w3.w3_linear(q, mat, s), (q.double().reshape(m, -1, 32) * s.double()[:, :, None]).reshape(m, k) @ dense.T)
+            assert mx < MAX_REL and nr < NORM_REL, (m, mx, nr)

@@ -32,7 +32,7 @@ def test_parts_of_a_block_against_the_product_and_the_sixteen_row_body(n, k):
         assert mx < MAX_REL and nr < NORM_REL, (m, mx, nr)
 
 
-@pytest.mark.parametrize("n", [64, 1152, 4096, 4160, 8192])  # one, 18 and 64 blocks in four parts, 65 and 128 in two
+@pytest.mark.parametrize("n", [128, 1152, 4096, 4224, 8192])  # 2, 18 and 64 blocks in four parts, 66 and 128 in two
 @pytest.mark.parametrize("k", [128, 640, 2048, 5120])  # one chunk of K, fewer and more chunks than splits
 def test_parts_of_a_block_on_the_sixteen_row_bodies(n, k):
     from hibana_amd import synthetic

@@ -300,7 +300,7 @@ def dense_decode(args) -> dict:
         def step(i: int):
             return w3.w3_linear(x, mats[i % args.layers])
 
-        kernel = "w3_part_kernel (w3_stream_kernel<dense>, a block on two workgroups)" if bits == 3 and m <= 4 else "w3_stream_kernel<dense>"
+        kernel = "w3_part_kernel (w3_stream_kernel<dense>, a block on two workgroups)" if bits == 3 and m <= 16 else "w3_stream_kernel<dense>"
         what = f"BASELINE config 0: w3 dense linear {n} x {k}, M = {m}, {book} codebook" + (" (two-bit tiles)" if bits == 2 else "")
     else:
         n, k = 25600, 5120

@@ -1366,10 +1366,12 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
                      (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && (pairs >= 48 * named || (pairs >= 16 * named && pairs * expert_blocks >= 1000000))));
   const int slot_rows = dense ? PANEL_SLOT_ROWS : ROWS_PER_SLOT;
   // Under a budget the table ends behind the experts the selection can name: the launches' grids reach over all of it, and a
-  // workgroup without rows is not free (40 rows of 10, a cap of 60 of 512 experts: 53.5 us before, 53.2 so).
+  // workgroup without rows is not free (40 rows of 10, a cap of 60 of 512 experts: 53.5 us before, 53.2 so). What a call of
+  // these pairs is refused for, and how its launches split K, go by the whole table: the bits of the same ids without a budget.
+  const int64_t whole = moe_max_slots(pairs, ex->experts, shared_rows, slot_rows);
+  if (whole > 65535) return HB_EINVAL;
   const int64_t distinct = route && route->budget ? budget_distinct(*route->budget, m, ex->experts) : ex->experts;
   const int64_t slots = moe_max_slots(pairs, (int)distinct, shared_rows, slot_rows);
-  if (slots > 65535) return HB_EINVAL;
   // E4M3 activations: x is rounded by further workgroups of the plan's launch, h in fc1's epilogue
   // weight-only on the stream: x also in its two-plane form, for the slots of at most two rows (fc1 on the FP8 matrix cores)
   const bool split = !e4m3 && !dense && g_tune.moe_split == 1 && g_tune.w3_few != 2;
@@ -1395,10 +1397,7 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
     return e;
   }
   const int n1 = ex->gated ? 2 * ex->inter : ex->inter;
-  // Rough number of busy slots. Under a budget about the cap's experts, some with more rows than a slot (40 rows of 10, a cap of
-  // 60: the shapes for 75 busy slots instead of 203, 53.2 -> 50.5 us).
-  int64_t est = pairs < 2 * ex->experts ? (pairs + 1) / 2 + (shared_rows + 15) / 16 : slots;
-  if (route && route->budget && !route->budget->repeat) est = std::max<int64_t>(1, std::min(est, budget_cap(*route->budget, m) + pairs / 32 + (shared_rows + 15) / 16));
+  const int64_t est = pairs < 2 * ex->experts ? (pairs + 1) / 2 + (shared_rows + 15) / 16 : whole;  // rough number of busy slots
   StreamParams p{};
   p.w = static_cast<const uint8_t*>(ex->fc1);
   p.expert_bytes = (int64_t)hb_w3_tiled_bytes(n1, ex->hidden, 3);

@@ -250,9 +250,8 @@ def moe_layer_budget(experts: W3Experts, x: torch.Tensor, logits: torch.Tensor, 
                      gate_vec: torch.Tensor | None = None, return_routing: bool = False):
     """`moe_layer` from the router's BF16 logits [M, E_total] under a budget: `ops.route_budget`'s selection (slots left
     over name no expert) runs in the same chain, as one launch that also plans the call
-    (hibana/model/flashnext/moe.py:122-135,177-192). The ids and weights are `route_budget`'s, bit for bit, and the
-    output that of `moe_layer` on them, whose sums over K a larger call may split otherwise (its launches are shaped for
-    the cap's experts). With `return_routing`, also the ids and weights it used."""
+    (hibana/model/flashnext/moe.py:122-135,177-192). The bits of `route_budget` followed by `moe_layer`. With
+    `return_routing`, also the ids and weights it used."""
     if x.dtype != torch.bfloat16 or x.ndim != 2 or x.shape[1] != experts.shape13[1]:
         raise ValueError("moe_layer_budget: x must be BF16 [M, hidden]")
     if logits.ndim != 2 or logits.shape[0] != x.shape[0] or logits.dtype != torch.bfloat16:

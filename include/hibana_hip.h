@@ -308,9 +308,8 @@ int hb_w3_moe_layer_logits_e4m3(const hb_w3_experts* routed, const hb_w3_experts
  * id experts_total at weight 0, which the experts skip), written to ids / weights (caller's buffers), then the chain of
  * hb_w3_moe_layer. One launch ahead of the experts': its workgroups rank the rows, and the last to arrive selects and also
  * plans (up to 8191 pairs; beyond, the plan's own launches follow). Weight-only arithmetic. topk and keep at most
- * HB_ROUTE_CANDIDATES, 20 <= experts_total <= 1024, m a multiple of steps. The ids and weights are hb_route_budget's, bit for
- * bit; the output is that of hb_w3_moe_layer on them, up to the order of the sums over K (the launches are shaped for the
- * cap's experts).
+ * HB_ROUTE_CANDIDATES, 20 <= experts_total <= 1024, m a multiple of steps. The same ids, weights and output as
+ * hb_route_budget followed by hb_w3_moe_layer, bit for bit.
  * ref: MoeLayer.__call__ with the budgeted branch of its route step, hibana/model/flashnext/moe.py:122-135,177-192. */
 int hb_w3_moe_layer_budget(const hb_w3_experts* routed, const hb_w3_experts* shared, const float* gate_vec,
                            const void* x, const void* logits, int experts_total, int m, int topk, int keep, int budget,

@@ -183,7 +183,7 @@ def test_layer_from_logits_is_route_then_layer(gated, m):
 
 @pytest.mark.parametrize("m,steps", [(1, 1), (5, 5), (12, 3), (32, 8), (200, 1)])
 def test_layer_under_a_budget_is_route_budget_then_layer(m, steps):
-    """`moe_layer_budget`: the selection's second launch also plans the call; ids, weights and output are the bits of
+    """`moe_layer_budget`: the selection's launch also plans the call; ids, weights and output are the bits of
     `ops.route_budget` followed by `moe_layer`, with padded requests, a cap per request, and a call of more pairs
     than one workgroup plans (the plan's own launches then follow)."""
     from hibana_amd.kernels import ops, w3_moe

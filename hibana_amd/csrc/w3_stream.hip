@@ -1154,9 +1154,10 @@ static int shape_stream(StreamParams& p, int64_t busy_slots, Launch want) {
 // expansion of a chunk more with each row, and no shape beats a launch whose workgroups all start at once. Measured, a replayed
 // graph of calls, the general rule and this one (us, blocks x chunks): twelve rows, K split eight ways: 40 x 12 8.9 and 5.0,
 // 160 x 12 8.9 and 5.2, 640 x 24 17.8 and 16.9, 400 x 7 9.4 and 7.0; four rows, at least four: 160 x 4 5.2 and 3.5, 400 x 7 6.9
-// and 5.4, 640 x 12 9.5 and 8.3. From BIG_BLOCKS runs of blocks a workgroup, 200 to 250 workgroups of eight wavefronts or 400 to
-// 500 of four: four rows 800 x 40 26.0 and 23.1, 800 x 24 16.7 and 15.8 (eight wavefronts: 16.8), 1000 x 24 18.1 and 17.0; twelve
-// rows 800 x 24 21.9 and 20.4, 1000 x 24 24.4 and 21.6, two-bit 800 x 16 15.0 and 13.9 (640 x 40 in runs of four: 22.2 instead of 20.2).
+// and 5.4, 640 x 12 9.5 and 8.3. From BIG_BLOCKS, past four rows, runs of four blocks a workgroup, 200 to 250 workgroups of eight
+// wavefronts: twelve rows 800 x 24 21.9 and 20.4, 1000 x 24 24.4 and 21.6, two-bit 800 x 16 15.0 and 13.9 (640 x 40 in runs of
+// four: 22.2 instead of 20.2). Up to four rows the general rule stays there: in runs four rows of 768 x 40 took 1.15 times as
+// long, of 1200 x 40 1.39, of 1600 x 24 1.11, and only 800 and 1000 blocks gained (up to 7 %).
 constexpr int BIG_BLOCKS = 768;
 static void shape_dense(StreamParams& p) {
   const bool few = p.m <= FEW_ROWS && !p.no_few;
@@ -1164,10 +1165,7 @@ static void shape_dense(StreamParams& p) {
     while (p.ks < most && 2 * p.ks <= p.chunks) p.ks *= 2;
     p.nbw = p.ks >= 4 ? 1 : p.nbw;
   };
-  if (p.n_blocks >= BIG_BLOCKS && few && p.chunks >= 8) {
-    p.ks = 2;
-    p.nbw = p.chunks < 32 ? 2 : 4;
-  } else if (p.n_blocks >= BIG_BLOCKS && !few && p.chunks >= 12 && p.chunks < 32) {
+  if (p.n_blocks >= BIG_BLOCKS && !few && p.chunks >= 12 && p.chunks < 32) {
     p.ks = 2;
     p.nbw = 4;
   } else if (!few) {

@@ -48,3 +48,28 @@ def test_nvfp4_shapes(blocks, chunks):
     n, k = blocks * 64, chunks * 128
     lin = synthetic.nvfp4_linear(n, k, 3)
     _check(lin, lambda x: ops.nvfp4_linear(x, lin), n, k)
+
+
+def _general_split(blocks, chunks, want):
+    """How many ways the rule for any launch splits K: until there are `want` wavefronts, four chunks each at least."""
+    ks = 1
+    while ks < 16 and blocks * ks < want and chunks // (2 * ks) >= 4:
+        ks *= 2
+    return ks
+
+
+# sizes that keep the general rule's split
+@pytest.mark.parametrize("rows,blocks,chunks", [(1, 768, 16), (4, 800, 40), (4, 1200, 12), (2, 2374, 9)])
+@pytest.mark.parametrize("codebook", ["lloyd", "lloyd2"])
+def test_w3_shapes_that_split_k_as_any_launch(rows, blocks, chunks, codebook):
+    from hibana_amd import _lib, synthetic
+    from hibana_amd.kernels import w3
+    mat = synthetic.w3_matrix(blocks * 64, chunks * 128, 3, codebook=codebook)
+    x = torch.randn(rows, chunks * 128, generator=torch.Generator().manual_seed(rows)).bfloat16().cuda()
+    got = w3.w3_linear(x, mat)
+    try:
+        assert _lib.lib().hb_tune(b"w3_ksplit", _general_split(blocks, chunks, 8192)) == 0
+        want = w3.w3_linear(x, mat)
+    finally:
+        _lib.lib().hb_tune(b"w3_ksplit", 0)
+    assert torch.equal(got, want)

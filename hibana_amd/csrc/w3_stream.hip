@@ -1151,27 +1151,31 @@ static int shape_stream(StreamParams& p, int64_t busy_slots, Launch want) {
 }
 
 // The shape of a dense call of one slot. A wavefront's start and the exchange cost about as much as two chunks of its K, the
-// expansion of a chunk more with each row, and no shape beats a launch whose workgroups all start at once. Measured, a replayed
-// graph of calls, the general rule and this one (us, blocks x chunks): twelve rows, K split eight ways: 40 x 12 8.9 and 5.0,
-// 160 x 12 8.9 and 5.2, 640 x 24 17.8 and 16.9, 400 x 7 9.4 and 7.0; four rows, at least four: 160 x 4 5.2 and 3.5, 400 x 7 6.9
-// and 5.4, 640 x 12 9.5 and 8.3. From BIG_BLOCKS, past four rows, runs of four blocks a workgroup, 200 to 250 workgroups of eight
-// wavefronts: twelve rows 800 x 24 21.9 and 20.4, 1000 x 24 24.4 and 21.6, two-bit 800 x 16 15.0 and 13.9 (640 x 40 in runs of
-// four: 22.2 instead of 20.2). Up to four rows the general rule stays there: in runs four rows of 768 x 40 took 1.15 times as
-// long, of 1200 x 40 1.39, of 1600 x 24 1.11, and only 800 and 1000 blocks gained (up to 7 %).
-constexpr int BIG_BLOCKS = 768;
+// expansion of a chunk more with each row. Measured, replayed graphs of calls on cycled weights, the general rule and this one
+// (us, blocks x chunks): twelve rows, K split eight ways: 40 x 12 8.9 and 5.0, 160 x 12 8.9 and 5.2, 640 x 24 17.8 and 16.9,
+// 400 x 7 9.4 and 7.0; up to four rows, at least four: 160 x 4 5.2 and 3.5, 400 x 7 6.9 and 5.4, 640 x 12 9.5 and 8.3. The general rule
+// stays where its workgroups fit the device better:
+// - up to four rows of 257 to 512 blocks, from eight chunks: two blocks a workgroup all start at once, and four ways
+//   took 1.00 to 1.12 times as long (one row of 300 x 10: 1.08, 512 x 10 1.07, 400 x 12 0.99);
+// - past three blocks a compute unit: four ways or eight of 2374 x 4 and 2374 x 8 chunks at twelve rows took 1.21 and 1.16 times as
+//   long (1200 x 8 0.93). From twelve rows one form gains there: up to four blocks a compute unit, some have four of them
+//   whichever way they are dealt out, and runs of four start a quarter of the workgroups: sixteen rows of 800 x 16 0.94, 1024 x 16 0.95, two-bit
+//   1000 x 20 0.95; twelve rows 0.94 to 1.04, two-bit 0.95 to 1.00. With fewer rows it is even (eight rows 0.98 to 1.05), and with fewer
+//   blocks or more the runs leave units idle: 768 x 24 1.14, 1200 x 24 1.42.
+constexpr int COMPUTE_UNITS = 256, RUN_ROWS = 12;
 static void shape_dense(StreamParams& p) {
   const bool few = p.m <= FEW_ROWS && !p.no_few;
   auto split = [&](int most) {  // at least as many ways as the general rule
     while (p.ks < most && 2 * p.ks <= p.chunks) p.ks *= 2;
     p.nbw = p.ks >= 4 ? 1 : p.nbw;
   };
-  if (p.n_blocks >= BIG_BLOCKS && !few && p.chunks >= 12 && p.chunks < 32) {
+  if (few) {
+    if (p.n_blocks < 3 * COMPUTE_UNITS && (p.n_blocks <= COMPUTE_UNITS || p.n_blocks > 2 * COMPUTE_UNITS || p.chunks < 8)) split(4);
+  } else if (p.n_blocks <= 3 * COMPUTE_UNITS) {
+    split(8);
+  } else if (p.n_blocks <= 4 * COMPUTE_UNITS && p.m >= RUN_ROWS && p.chunks >= 12 && p.chunks < 32) {
     p.ks = 2;
     p.nbw = 4;
-  } else if (!few) {
-    split(8);
-  } else if (p.n_blocks < BIG_BLOCKS) {
-    split(4);
   }
   set_split(p);
 }

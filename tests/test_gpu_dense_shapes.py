@@ -59,7 +59,8 @@ def _general_split(blocks, chunks, want):
 
 
 # sizes that keep the general rule's split
-@pytest.mark.parametrize("rows,blocks,chunks", [(1, 768, 16), (4, 800, 40), (4, 1200, 12), (2, 2374, 9)])
+@pytest.mark.parametrize("rows,blocks,chunks", [(1, 768, 16), (4, 800, 40), (4, 1200, 12), (2, 2374, 9), (1, 258, 8), (4, 512, 14), (16, 770, 8), (8, 800, 16),
+                                                (12, 1026, 16), (16, 2374, 4)])
 @pytest.mark.parametrize("codebook", ["lloyd", "lloyd2"])
 def test_w3_shapes_that_split_k_as_any_launch(rows, blocks, chunks, codebook):
     from hibana_amd import _lib, synthetic

@@ -463,20 +463,28 @@ static int shape_nvfp4(StreamParams& p, int64_t busy_slots) {
 }
 
 // The shape of a dense call of one slot: K split eight ways as far as there are chunks, since a wavefront's start and the
-// exchange cost about as much as two or three of them. Measured, a replayed graph of calls, the general rule and this one (us,
-// blocks x chunks): twelve rows 16 x 12 10.8 and 5.4, 160 x 12 12.0 and 6.0, 400 x 16 12.5 and 10.9, 640 x 4 8.3 and 6.8, 800 x 8
-// 13.2 and 10.9; eight rows 80 x 12 8.2 and 5.6, 400 x 16 10.4 and 9.5, 640 x 12 13.2 and 10.8; one row 80 x 4 4.9 and 4.4. With
-// few rows and many blocks short of K the launch is bound by its traffic, and fewer wavefronts are better: 640 x 7 one row 7.0 by the
-// general rule and 7.8 split four ways, 520 x 8 8.4, split eight ways 9.0, four ways 8.2; and from 768 blocks eight wavefronts
-// on four blocks: 800 x 40 one row 27.6 and 25.8, 800 x 16 14.3 and 13.1, eight rows 15.6 and 15.5.
+// exchange cost about as much as two or three of them. Measured, replayed graphs of calls on cycled weights, the general rule and
+// this one (us, blocks x chunks): twelve rows 16 x 12 10.8 and 5.4, 160 x 12 12.0 and 6.0, 400 x 16 12.5 and 10.9, 640 x 4 8.3 and
+// 6.8, 800 x 8 13.2 and 10.9; eight rows 80 x 12 8.2 and 5.6, 400 x 16 10.4 and 9.5, 640 x 12 13.2 and 10.8; one row 80 x 4 4.9 and
+// 4.4. With few rows and many blocks short of K the launch is bound by its traffic, and fewer wavefronts are better:
+// - 257 to 512 blocks, where the general rule's workgroups of two blocks all start at once: its shape up to two rows below sixteen
+//   chunks (the splits took 0.95 to 1.11 times as long: 302 x 10 1.11, 400 x 8 1.07, 300 x 12 1.06) and, past 300 blocks, up to
+//   eight rows below twelve (0.96 to 1.06);
+// - 513 to 767 blocks: its shape below eight chunks (640 x 7 one row 7.0, split four ways 7.8), four ways below twelve (520 x 8
+//   one row by the general rule 8.4, split eight ways 9.0, four ways 8.2);
+// - from three blocks a compute unit its shape: four blocks a workgroup took 1.21 times as long at 768 x 40 and eight rows, 1200 x
+//   40 1.38, 2374 x 24 1.12, and gained at 800 blocks alone (one row up to 11 %).
 static void shape_nvfp4_dense(StreamParams& p) {
-  const bool few = p.m <= FP4_FEW_ROWS && !p.no_few;
+  constexpr int COMPUTE_UNITS = 256;
   int most = 8;
-  if (few && p.n_blocks >= 768) {
-    if (p.chunks >= 12) p.ks = 2, p.nbw = 4;
-    most = 0;
-  } else if (few && p.n_blocks > 300 && p.chunks < 12) {
-    most = p.chunks >= 8 ? 4 : 0;
+  if (p.m <= FP4_FEW_ROWS && !p.no_few && p.n_blocks > COMPUTE_UNITS) {
+    if (p.n_blocks <= 2 * COMPUTE_UNITS) {
+      if (p.chunks < (p.m <= 2 ? 16 : p.n_blocks > 300 ? 12 : 0)) return;
+    } else if (p.n_blocks < 3 * COMPUTE_UNITS && p.chunks >= 8) {
+      most = p.chunks < 12 ? 4 : 8;
+    } else {
+      return;
+    }
   }
   while (p.ks < most && 2 * p.ks <= p.chunks) p.ks *= 2;
   if (p.ks >= 4) p.nbw = 1;

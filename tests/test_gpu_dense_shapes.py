@@ -74,3 +74,18 @@ def test_w3_shapes_that_split_k_as_any_launch(rows, blocks, chunks, codebook):
     finally:
         _lib.lib().hb_tune(b"w3_ksplit", 0)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("rows,blocks,chunks", [(1, 258, 12), (2, 400, 8), (1, 512, 15), (8, 302, 10), (4, 514, 7), (4, 768, 40), (8, 1200, 12), (1, 2374, 24)])
+def test_nvfp4_shapes_that_split_k_as_any_launch(rows, blocks, chunks):
+    from hibana_amd import _lib, synthetic
+    from hibana_amd.kernels import ops
+    lin = synthetic.nvfp4_linear(blocks * 64, chunks * 128, 3)
+    x = torch.randn(rows, chunks * 128, generator=torch.Generator().manual_seed(rows)).bfloat16().cuda()
+    got = ops.nvfp4_linear(x, lin)
+    try:
+        assert _lib.lib().hb_tune(b"nvfp4_ksplit", _general_split(blocks, chunks, 4096)) == 0
+        want = ops.nvfp4_linear(x, lin)
+    finally:
+        _lib.lib().hb_tune(b"nvfp4_ksplit", 0)
+    assert torch.equal(got, want)

@@ -1036,6 +1036,12 @@ int moe_launch_route_plan(const TopkRoute& route, int m, int topk, int32_t* ids,
   return launch_route_plan(rp, m, e_lo, e_n, shared_rows, ws, stream, slot_rows, job);
 }
 
+int moe_check_budget(const BudgetRoute& b, int m, int topk) {
+  const bool refused = b.e < BUDGET_CANDIDATES || b.e > BUDGET_THREADS || topk > BUDGET_CANDIDATES || b.keep < 0 || b.keep > BUDGET_CANDIDATES || b.budget < 0 ||
+                       b.steps <= 0 || m % b.steps || b.per_request < 0 || b.min_cap < 0 || !aligned(b.logits, 2) || !aligned(b.slots, 4);
+  return refused ? HB_EINVAL : HB_OK;
+}
+
 constexpr int BUDGET_SPREAD_ROWS = 256;  // about the compute units
 int moe_launch_budget_plan(const BudgetRoute& b, int m, int topk, int32_t* ids, float* weights, int e_lo, int e_n, int shared_rows,
                            const MoeWorkspace& ws, void* scratch, hipStream_t stream, int slot_rows) {
@@ -1044,9 +1050,8 @@ int moe_launch_budget_plan(const BudgetRoute& b, int m, int topk, int32_t* ids, 
   const size_t plan_lds = ((size_t)(PLAN_WAVES + 1) * e_n + 3 * (PLAN_WAVES + 1)) * sizeof(int);
   if (plan_lds > 64 * 1024 || e_n > PLAN_THREADS || pairs > 0x3fffffff) return HB_EINVAL;
   if (!b.logits || !scratch) return HB_ENULL;
-  if (b.e < BUDGET_CANDIDATES || b.e > BUDGET_THREADS || topk > BUDGET_CANDIDATES || b.keep < 0 || b.keep > BUDGET_CANDIDATES || b.budget < 0 ||
-      b.steps <= 0 || m % b.steps || b.per_request < 0 || b.min_cap < 0 || !aligned(b.logits, 2) || !aligned(b.slots, 4) || !aligned(scratch, 4))
-    return HB_EINVAL;
+  if (!aligned(scratch, 4)) return HB_EINVAL;
+  if (int e = moe_check_budget(b, m, topk)) return e;
   BudgetParams q{};
   q.logits = b.logits;
   q.slots = b.slots;

@@ -534,16 +534,17 @@ void moe_launch_quant_rows(const uint16_t* x, int64_t m, int k, uint8_t* q, floa
 // for up to a few dozen rows, two beyond.
 int moe_check_route(int m, int e, int k);  // HB_EINVAL for a row the routing wavefront cannot hold
 
-// A routed call whose experts are chosen under a budget (route_budget.hpp): BF16 logits [m, e] and the rule's settings.
 // The experts a routed call's ids are drawn from, as far as is known: what the caller says (0: nothing), at least up to
 // the end of the range held here. Its pairs spread over these, so the range sees experts / experts_named of them, and the
 // rows an expert that choose a call's kernels are pairs / experts_named.
 inline int64_t experts_named(int experts_total, int base, int experts) { return std::max<int64_t>(experts_total, (int64_t)base + experts); }
+// A routed call whose experts are chosen under a budget (route_budget.hpp): BF16 logits [m, e] and the rule's settings.
 struct BudgetRoute {
   const uint16_t* logits;
   int e, keep, budget, steps, repeat, per_request, min_cap;
   const int32_t* slots;  // or null: every row is real
 };
+int moe_check_budget(const BudgetRoute& b, int m, int topk);  // HB_EINVAL for settings the selection does not take; ahead of the two below
 // The cap on distinct experts of a call whose requests are all real (padded ones only lower it), and the most a selection can
 // name: its set is the rows' guaranteed experts filled up to the cap, and a slot left over names no expert. (With `repeat` it
 // names a row's first candidate, in the set or not: no bound then.)

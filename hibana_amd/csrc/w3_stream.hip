@@ -1372,6 +1372,9 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   // these pairs is refused for, and how its launches split K, go by the whole table: the bits of the same ids without a budget.
   const int64_t whole = moe_max_slots(pairs, ex->experts, shared_rows, slot_rows);
   if (whole > 65535) return HB_EINVAL;
+  if (route && route->budget) {
+    if (int e = moe_check_budget(*route->budget, m, topk)) return e;
+  }
   const int64_t distinct = route && route->budget ? budget_distinct(*route->budget, m, ex->experts) : ex->experts;
   const int64_t slots = moe_max_slots(pairs, (int)distinct, shared_rows, slot_rows);
   // E4M3 activations: x is rounded by further workgroups of the plan's launch, h in fc1's epilogue

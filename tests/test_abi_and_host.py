@@ -107,6 +107,18 @@ def test_validation_without_a_gpu():
         _lib.check(_lib.HB_ELAUNCH, "x")
 
 
+@pytest.mark.parametrize("change", [dict(steps=0), dict(steps=-1), dict(steps=3), dict(per_request=-1), dict(min_cap=-1), dict(keep=21), dict(budget=-1), dict(topk=21),
+                                    dict(experts_total=19)])
+def test_a_budget_that_is_refused_is_refused_before_anything_is_made_of_it(change):
+    """`hb_w3_moe_layer_budget` returns HB_EINVAL for settings that `hb_route_budget` refuses, a row count per request of zero
+    among them: the bound on the experts a selection can name divides by it."""
+    lib = _lib.lib()
+    ex = _lib.HbW3Experts(256, 256, 256, 256, 0, 0, 8, 0, 256, 128, 256, 1)  # (no call below reads through the pointers)
+    it = dict(experts_total=512, m=4, topk=10, keep=4, budget=64, steps=1, per_request=12, min_cap=16) | change
+    assert lib.hb_w3_moe_layer_budget(C.byref(ex), None, None, 256, 256, it["experts_total"], it["m"], it["topk"], it["keep"], it["budget"], None, it["steps"],
+                                      it["per_request"], it["min_cap"], 256, 256, 256, 256, 1 << 30, None) == _lib.HB_EINVAL
+
+
 def test_host_logic_mirrors_the_reference_interface(monkeypatch):
     from hibana_amd.kernels import ops, w3, w3_moe
     from hibana_amd.weights import modelopt

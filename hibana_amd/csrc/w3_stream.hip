@@ -540,7 +540,7 @@ struct FullActs {  // up to sixteen rows: lane (q, r16) feeds row r16, k 8 q .. 
 // accumulator registers hold (rows 4 q .. 4 q + 3). Both are asked for again by halves, as FullActs does.
 struct FullActs8 {
   typedef __attribute__((ext_vector_type(2))) float f32x2_t;
-  static constexpr int LOADS = 12;
+  static constexpr int LOADS = 8;  // four of codes and at least four of scales: of a row's two scale pairs, asked for side by side, the compiler makes one load
   long a[4];            // the lane's codes of groups 0..3
   f32x2_t xs_lo[4];     // activation scales of rows 4 q + r at groups 0, 1
   f32x2_t xs_hi[4];     // ... at groups 2, 3
@@ -570,7 +570,6 @@ struct FullActs8 {
     load_half(0, 0);
     load_half(1, 0);
   }
-  // groups 2 HALF and 2 HALF + 1 of the four tiles
   // groups 2 HALF and 2 HALF + 1 of tile NT
   template <int HALF, int NT, class C>
   __device__ __forceinline__ void half_tile(const C& ch, f32x4_t& acc, uint32_t lut_lo, uint32_t lut_hi) const {
@@ -591,6 +590,7 @@ struct FullActs8 {
       acc.w = fmaf(part.w, (jj ? xs[3].y : xs[3].x) * ws, acc.w);
     }
   }
+  // ... of the four tiles
   template <int HALF, class C>
   __device__ __forceinline__ void half_chunk(const C& ch, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, uint32_t lut_lo,
                                              uint32_t lut_hi) const {
@@ -635,7 +635,6 @@ struct FullActsPart : FullActs {
 };
 template <int T0, int T1>
 struct FullActs8Part : FullActs8 {
-  static constexpr int LOADS = 8;  // at least: with a tile or two between them the compiler makes one load of a row's two scale pairs (twelve waited for too little)
   template <int HALF, class C>
   __device__ __forceinline__ void half(const C& ch, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot& sl) const {
     if (T0 <= 0 && 0 < T1) half_tile<HALF, 0>(ch, acc0, sl.lut_lo, sl.lut_hi);

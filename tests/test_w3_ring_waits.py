@@ -1,0 +1,66 @@
+"""The weight ring's waits in the machine code of the built library (no kernel runs): a wait ahead of a block's reads may leave
+outstanding at most the next block's loads into LDS, or the block that is read has not landed. How many requests that is
+counts the activation loads a body says it makes, and the compiler may make one load of two."""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from hibana_amd import _lib
+
+OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
+REQUEST = re.compile(r"(buffer|global|flat)_(load|store|atomic)")  # (a spill is none: nothing may rest on one)
+
+
+def _kernels(folder):
+    """(name, [(address, instruction)]) of every three-bit stream kernel of the library."""
+    shutil.copy(_lib.LIBRARY, folder / "lib.so")
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=folder, check=True, capture_output=True)
+    for part in sorted(p for p in os.listdir(folder) if "gfx950" in p):
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", part], cwd=folder, check=True, capture_output=True, text=True).stdout
+        for name, code in re.findall(r"^[0-9a-f]+ <(\S+)>:\n((?:.+\n)*)", text, re.M):
+            if re.search(r"w3_(stream|part|fc\w+)_kernel", name):
+                yield name, [(int(at, 16), ins) for ins, at in re.findall(r"^\s+(\S.*?)\s*// ([0-9A-F]+):", code, re.M)]
+
+
+def _most_left_in_flight(code):
+    """For every wait of a ring's take: how many loads into LDS stand among the last requests that it leaves outstanding, over
+    all ways there, and how many loads a block has (as many as the take has reads)."""
+    place = {at: i for i, (at, _) in enumerate(code)}
+    before = [[] for _ in code]
+    for i, (at, ins) in enumerate(code):
+        if ins.startswith(("s_branch", "s_cbranch")):
+            words = int(ins.split()[1])
+            before[place[at + 4 + 4 * (words - 65536 if words >= 32768 else words)]].append(i)
+        if not ins.startswith(("s_branch", "s_endpgm", "s_setpc")) and i + 1 < len(code):
+            before[i + 1].append(i)
+    for i, (_, ins) in enumerate(code[:-1]):
+        wait = re.fullmatch(r"s_waitcnt vmcnt\((\d+)\)", ins)
+        if not wait or wait.group(1) == "0" or not code[i + 1][1].startswith("ds_read_b128"):
+            continue
+        reads = next(j for j in range(1, 9) if not code[i + 1 + j][1].startswith("ds_read_b128"))
+        most, seen, todo = 0, set(), [(j, int(wait.group(1)), 0) for j in before[i]]
+        while todo:
+            state = todo.pop()
+            if state in seen:
+                continue
+            seen.add(state)
+            j, left, into_lds = state
+            if REQUEST.match(code[j][1]):
+                left, into_lds = left - 1, into_lds + code[j][1].endswith(" lds")
+                most = max(most, into_lds)
+            if left:
+                todo += [(h, left, into_lds) for h in before[j]]
+        yield most, reads
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
+def test_a_wait_leaves_the_next_block_outstanding_and_no_more(tmp_path):
+    checked = 0
+    for name, code in _kernels(tmp_path):
+        takes = list(_most_left_in_flight(code))
+        assert takes and all(most <= reads for most, reads in takes), (name, takes)
+        checked += 1
+    assert checked >= 20, checked

@@ -97,6 +97,31 @@ def test_moe_combine_of_a_routed_sum_and_the_gated_shared_expert():
     assert (got.view(torch.int16) != want.view(torch.int16)).float().mean() < 0.02
 
 
+# 1024 rows: the wide form's first; topk: one batch of twelve, its edge, a remainder, a third batch; columns: less than a wavefront's, a workgroup's
+# 2048 and its neighbours, more than one; off: pairs that start on an 8-byte boundary only, and 2052 columns: the narrow form
+@pytest.mark.parametrize("m,topk,h,off", [(1024, 1, 8, 0), (1024, 12, 2040, 0), (1025, 13, 2048, 0), (1024, 22, 2056, 0), (1031, 25, 520, 0), (1024, 3, 4104, 0),
+                                          (1024, 13, 2048, 4), (1024, 13, 2052, 0)])
+def test_moe_combine_of_many_rows_of_bf16_pairs(m, topk, h, off):
+    """A long call's sum of BF16 pairs gives the bits of the same pairs in FP32 and of the rows taken in short calls; an id
+    outside the range drops its pair, whatever the pair holds, in the last slots of a batch as in the first."""
+    from hibana_amd.kernels import ops
+    g = torch.Generator(device="cuda").manual_seed(m + topk + h)
+    e_lo, e_n = 3, 9
+    ids = torch.randint(0, 16, (m, topk), generator=g, device="cuda", dtype=torch.int32)  # a quarter of them outside
+    ids[5], ids[6] = -1, e_lo + e_n  # rows of which nothing is left
+    weights = torch.rand(m, topk, generator=g, device="cuda")
+    y = torch.empty(m * topk * h + off, dtype=torch.bfloat16, device="cuda")[off:].view(m * topk, h)
+    y.copy_(torch.randn(m * topk, h, generator=g, device="cuda"))
+    dropped = ((ids < e_lo) | (ids >= e_lo + e_n)).view(-1)
+    y[dropped] = float("nan")
+    got = ops.moe_combine_pairs(y, ids, weights, None, None, None, e_lo, e_n)
+    assert torch.isfinite(got).all() and not got[5:7].any()
+    assert torch.equal(got, ops.moe_combine_pairs(y.float(), ids, weights, None, None, None, e_lo, e_n))
+    half = m // 2
+    parts = [ops.moe_combine_pairs(y[r0 * topk:r1 * topk], ids[r0:r1], weights[r0:r1], None, None, None, e_lo, e_n) for r0, r1 in ((0, half), (half, m))]
+    assert torch.equal(got, torch.cat(parts))
+
+
 def test_relu2_in_place():
     from hibana_amd.model import nemotron_moe
     g = torch.Generator().manual_seed(9)

@@ -503,8 +503,8 @@ __device__ __forceinline__ int last_to_arrive(int32_t* plan, int groups) {
 // PLAN_ROWS_MAX (plan_by_rows). Workgroups past the routing ones round the job's activations, as in moe_plan_kernel.
 __global__ __launch_bounds__(PLAN_THREADS) void moe_route_plan_kernel(const int32_t* ids, int pairs, int e_lo, int e_n, int shared_rows,
                                                                       int32_t* __restrict__ plan, int32_t* __restrict__ order, RouteParams route,
-                                                                      int route_rows, int route_groups, int group_rows, int by_rows, int slot_rows, int slot_cap,
-                                                                      QuantJob job) {
+                                                                      int route_rows, int route_groups, int group_rows, int by_rows, int slot_rows,
+                                                                      int slot_cap, QuantJob job) {
   extern __shared__ int lds[];
   __shared__ int last;
   if ((int)blockIdx.x >= route_groups) {
@@ -533,8 +533,9 @@ __global__ __launch_bounds__(PLAN_THREADS) void moe_route_plan_kernel(const int3
 // Budgeted selection and the plan of its ids in one launch: its workgroups rank `group_rows` rows each (a row a
 // wavefront), and the last of them to finish selects and plans, as in the routing launch above: candidates and ids go through
 // to memory, are waited for ahead of the ticket or the plan, and are read past the L2. (A rank launch of its own before it:
-// 5.0 + 13.0 us at 40 rows of 512 experts, the whole layer 50.4 us and 48.7 so.) `PLAN`: false leaves the plan to launches of its own (a call of more pairs than
-// one workgroup plans). `by_rows`: no row names an expert twice and they are at most PLAN_ROWS_MAX; each group ranks one.
+// 5.0 + 13.0 us at 40 rows of 512 experts, the whole layer 50.4 us and 48.7 so.) `PLAN`: false leaves the plan to launches of
+// its own (a call of more pairs than one workgroup plans). `by_rows`: no row names an expert twice and they are at most
+// PLAN_ROWS_MAX; each group ranks one.
 template <int PER, bool PLAN>
 __global__ __launch_bounds__(PLAN_THREADS) void moe_budget_plan_kernel(BudgetParams q, int copies_n, int e_lo, int e_n, int shared_rows,
                                                                        int32_t* __restrict__ plan, int32_t* __restrict__ order, int group_rows, int by_rows,
@@ -991,7 +992,8 @@ static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, in
   const size_t plan_lds = ((size_t)(PLAN_WAVES + 1) * e_n + 3 * (PLAN_WAVES + 1)) * sizeof(int);
   if (plan_lds > 64 * 1024 || e_n > PLAN_THREADS || pairs > 0x3fffffff) return HB_EINVAL;
   // rows that name no expert twice: every row is real, or a padded row names none (with `repeat` it names one over and over)
-  const int by_rows = (!rp.slots || (!rp.repeat && (rp.pad_id < e_lo || rp.pad_id >= e_lo + e_n))) && m <= PLAN_ROWS_MAX && rp.k <= 64 && g_route_plan_fused.load(std::memory_order_relaxed) != 1;
+  const bool distinct = !rp.slots || (!rp.repeat && (rp.pad_id < e_lo || rp.pad_id >= e_lo + e_n));
+  const int by_rows = distinct && m <= PLAN_ROWS_MAX && rp.k <= 64 && g_route_plan_fused.load(std::memory_order_relaxed) != 1;
   if (m > ROUTE_FUSED_ROWS && pairs < PLAN_WIDE_PAIRS && g_route_plan_fused.load(std::memory_order_relaxed) != 2) {
     // a verify-sized call: the routing spread over the device, the plan by the workgroup that finishes last
     const int group_rows = m <= ROUTE_SPREAD_ROWS ? 1 : ROUTE_GROUP_ROWS, groups = (m + group_rows - 1) / group_rows;
@@ -1010,7 +1012,8 @@ static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, in
   }
   static_assert(ROUTE_FUSED_ROWS <= PLAN_WAVES, "a wavefront a row");
   HB_LAUNCH(moe_plan_kernel<false>, dim3(plan_groups(job)), dim3(PLAN_THREADS), plan_lds, stream, rp.ids, (int)pairs, e_lo, e_n, shared_rows, ws.plan, ws.order,
-            rp, m, by_rows && pairs > 64, slot_rows, (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows), ws.plan_wide, 1, 0, job ? *job : QuantJob{});  // (up to 64 pairs one wavefront plans)
+            rp, m, by_rows && pairs > 64 /* up to 64 pairs one wavefront plans */, slot_rows, (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows),
+            ws.plan_wide, 1, 0, job ? *job : QuantJob{});
   return HB_OK;
 }
 
@@ -1071,7 +1074,8 @@ int moe_launch_budget_plan(const BudgetRoute& b, int m, int topk, int32_t* ids, 
   const dim3 grid((unsigned)((m + group_rows - 1) / group_rows));
   const size_t lds = plan ? std::max(pick_lds, plan_lds) : pick_lds;
   auto launch = [&](auto kernel) {
-    HB_LAUNCH(kernel, grid, dim3(PLAN_THREADS), lds, stream, q, copies_n, e_lo, e_n, shared_rows, ws.plan, ws.order, group_rows, (int)by_rows, slot_rows, slot_cap);
+    HB_LAUNCH(kernel, grid, dim3(PLAN_THREADS), lds, stream, q, copies_n, e_lo, e_n, shared_rows, ws.plan, ws.order, group_rows, (int)by_rows, slot_rows,
+              slot_cap);
   };
   if (plan) {
     small ? launch(moe_budget_plan_kernel<8, true>) : launch(moe_budget_plan_kernel<16, true>);

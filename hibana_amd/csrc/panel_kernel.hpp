@@ -122,8 +122,8 @@ struct Panel {
   static constexpr int HALVES_FROM = 6;
 
   // The products of fragment J = 4 * step + tile of a chunk, and between them the expansion of fragment J + 1, a pair of
-  // its values behind every MT / 4 products (or half a pair behind every MT / 8). The empty statements hold that order: left to itself the compiler puts the
-  // expansion behind the products (fewer registers), where nothing runs beside it.
+  // its values behind every MT / 4 products (or half a pair behind every MT / 8). The empty statements hold that order: left to
+  // itself the compiler puts the expansion behind the products (fewer registers), where nothing runs beside it.
   // FRESH: the activations' fragments may still be on their way (asked for in order, nothing behind them). NEXT >= 0: the
   // LDS offset of the next step's, from `at`.
   template <int J, bool FRESH, int NEXT>
@@ -338,7 +338,8 @@ struct Panel {
   // bytes a row and store, so a row tile goes through the wavefront's own (by now empty) slot of LDS and leaves as 128 (gated:
   // 64) contiguous bytes a row; what the stores need from memory (the rows' places, the column scales) is asked for once, ahead
   // of the first. Before, the last row tiles of a slot of 128 stood behind eight round trips to `order`: 11.9 us of a workgroup's
-  // 23.9 (fc2 of the three-bit layer, 1543 rows), 14.6 of 68.6 (the latent block's, 2048). A row of LDS is 144 bytes: sixteen rows' columns start in different banks.
+  // 23.9 (fc2 of the three-bit layer, 1543 rows), 14.6 of 68.6 (the latent block's, 2048). A row of LDS is 144 bytes: sixteen
+  // rows' columns start in different banks.
   static constexpr int LINE = 144;
   static_assert(16 * LINE <= Fmt::BLOCK_BYTES && LINE % 16 == 0 && Fmt::BLOCK_BYTES % 16 == 0, "a row tile in the slot of a weight block");
   __device__ __forceinline__ void store_rows(const StreamParams& p, const Slot& sl, uint8_t* slot, int nb, int lane) {

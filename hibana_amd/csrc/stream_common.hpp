@@ -548,12 +548,15 @@ int moe_check_budget(const BudgetRoute& b, int m, int topk);  // HB_EINVAL for s
 // The cap on distinct experts of a call whose requests are all real (padded ones only lower it), and the most a selection can
 // name: its set is the rows' guaranteed experts filled up to the cap, and a slot left over names no expert. (With `repeat` it
 // names a row's first candidate, in the set or not: no bound then.)
-inline int64_t budget_cap(const BudgetRoute& b, int m) { return b.per_request > 0 ? std::min<int64_t>(b.budget, std::max<int64_t>(b.min_cap, (int64_t)b.per_request * (m / b.steps))) : b.budget; }
+inline int64_t budget_cap(const BudgetRoute& b, int m) {
+  return b.per_request > 0 ? std::min<int64_t>(b.budget, std::max<int64_t>(b.min_cap, (int64_t)b.per_request * (m / b.steps))) : b.budget;
+}
 inline int64_t budget_distinct(const BudgetRoute& b, int m, int experts) {
   return b.repeat ? experts : std::min<int64_t>(experts, std::max<int64_t>({1, budget_cap(b, m), (int64_t)b.keep * m}));
 }
-// Rank, then the selection and the plan of its ids in one workgroup's launch (the selection leaves ids / weights in the
-// caller's arrays). `scratch`: room for the rows' candidates between the two launches (160 bytes a row).
+// The ranking of the rows, the selection and the plan of its ids in one launch, whose last workgroup takes the second and the
+// third (beyond 8191 pairs the plan's own launches follow); the selection leaves ids / weights in the caller's arrays.
+// `scratch`: room for the rows' candidates in between (160 bytes a row).
 int moe_launch_budget_plan(const BudgetRoute& b, int m, int topk, int32_t* ids, float* weights, int e_lo, int e_n, int shared_rows,
                            const MoeWorkspace& ws, void* scratch, hipStream_t stream, int slot_rows = ROWS_PER_SLOT);
 // The top-k routing of a routed call: logits FP32 or (`half`) BF16 [m, e]; row r is real iff slots[r / steps] != 0 (null:

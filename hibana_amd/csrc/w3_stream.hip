@@ -612,7 +612,8 @@ struct FullActs8 {
 template <int T0, int T1>
 struct FullActsPart : FullActs {
   template <int HALF, class C>
-  static __device__ __forceinline__ void half(const C& ch, const u32x4_t& a_lo, const u32x4_t& a_hi, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot& sl) {
+  static __device__ __forceinline__ void half(const C& ch, const u32x4_t& a_lo, const u32x4_t& a_hi, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3,
+                                              const Slot& sl) {
     if (T0 <= 0 && 0 < T1) compute_half_tile<HALF, 0>(ch, a_lo, a_hi, acc0, sl.lut_lo, sl.lut_hi);
     if (T0 <= 1 && 1 < T1) compute_half_tile<HALF, 1>(ch, a_lo, a_hi, acc1, sl.lut_lo, sl.lut_hi);
     if (T0 <= 2 && 2 < T1) compute_half_tile<HALF, 2>(ch, a_lo, a_hi, acc2, sl.lut_lo, sl.lut_hi);
@@ -799,7 +800,8 @@ __device__ __forceinline__ void part_block(const StreamParams& p, const Slot& sl
     } else {
       stream_block<EPI_DENSE, FewActsPart<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
     }
-    finish_few<EPI_DENSE>(p, sl, 0, scale, nb, true, wave, share.ks, 0, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3, FewPairs{}, FewScales{}, T0, T1);
+    finish_few<EPI_DENSE>(p, sl, 0, scale, nb, true, wave, share.ks, 0, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3, FewPairs{}, FewScales{},
+                          T0, T1);
   } else {
     if constexpr (A8) {
       stream_block<EPI_DENSE, FullActs8Part<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
@@ -1158,9 +1160,10 @@ static int shape_stream(StreamParams& p, int64_t busy_slots, Launch want) {
 //   took 1.00 to 1.12 times as long (one row of 300 x 10: 1.08, 512 x 10 1.07, 400 x 12 0.99);
 // - past three blocks a compute unit: four ways or eight of 2374 x 4 and 2374 x 8 chunks at twelve rows took 1.21 and 1.16 times as
 //   long (1200 x 8 0.93). From twelve rows one form gains there: up to four blocks a compute unit, some have four of them
-//   whichever way they are dealt out, and runs of four start a quarter of the workgroups: sixteen rows of 800 x 16 0.94, 1024 x 16 0.95, two-bit
-//   1000 x 20 0.95; twelve rows 0.94 to 1.04, two-bit 0.95 to 1.00. With fewer rows it is even (eight rows 0.98 to 1.05), and with fewer
-//   blocks or more the runs leave units idle: 768 x 24 1.14, 1200 x 24 1.42.
+//   whichever way they are dealt out, and runs of four start a quarter of the workgroups: sixteen rows of 800 x 16 0.94,
+//   1024 x 16 0.95, two-bit 1000 x 20 0.95; twelve and thirteen rows 0.96 to 1.01, two-bit 0.95 to 1.01 (770 to 1024 blocks,
+//   12 to 31 chunks). With fewer rows it is even (eight rows 0.98 to 1.05), and with fewer blocks or more the runs leave units
+//   idle: 768 x 24 1.14, 1200 x 24 1.42.
 constexpr int COMPUTE_UNITS = 256, RUN_ROWS = 12;
 static void shape_dense(StreamParams& p) {
   const bool few = p.m <= FEW_ROWS && !p.no_few;

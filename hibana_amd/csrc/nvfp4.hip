@@ -560,6 +560,9 @@ struct TileNvfp4 {
   static constexpr bool PER_ROW = false;
   static constexpr float EXPAND_US = 0.f;  // (the estimate's own constants are this format's)
   static constexpr int BESIDE_TILES = 0;
+  static constexpr int LIGHT_ROWS = 0;  // (an expansion takes the scale along at the price of the stream's)
+  template <int EPI>
+  static __device__ __forceinline__ void light(const StreamParams&, const Slot&, int, uint8_t*) {}
 };
 
 static inline unsigned grid_for(int64_t threads) { return (unsigned)((threads + 255) / 256); }

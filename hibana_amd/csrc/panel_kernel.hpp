@@ -529,6 +529,7 @@ __global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_tile_kernel(StreamP
   const PanelShare part{local - round * p.panel_groups, 0, 1, 0};
   const Slot sl = slot_of<EPI>(p, slot);
   if (sl.rows <= 0) return;  // a slot the plan did not fill: the whole workgroup leaves
+  if (sl.rows <= Fmt::LIGHT_ROWS) return Fmt::template light<EPI>(p, sl, part.group, panel_lds);
   auto run = [&](auto panel) { panel.run(p, sl, panel_lds, part); };
   switch ((sl.rows + 15) >> 4) {
     case 1: run(Panel<Fmt, EPI, 1>{}); break;
@@ -681,6 +682,12 @@ static int launch_panel(StreamParams& p, const PanelPlan& q, void* workspace, hi
   return HB_OK;
 }
 
+// The LDS of a routed call's workgroup: the panel's, or the weight rings of its light slots.
+template <class Fmt>
+inline size_t panel_routed_lds(int mt, int nbw) {
+  return std::max(panel_lds_bytes<Fmt>(mt, 1, nbw), Fmt::LIGHT_ROWS > 0 ? (size_t)nbw * ring_bytes<typename Fmt::Ring>() : 0);
+}
+
 // Over a plan's slots of PANEL_SLOT_ROWS rows; `a_rows`: rows of the activation matrix. Four wavefronts a workgroup on four
 // blocks, two workgroups a compute unit: one's start and end lie beside the other's products.
 constexpr int PANEL_SLOT_ROWS = 128;
@@ -695,7 +702,7 @@ static int launch_panel_routed(StreamParams& p, int64_t slots, int64_t a_rows, h
   p.panel_full = (int)slots;
   const int64_t grid = (slots + 7) / 8 * 8 * p.panel_groups;
   if (!panel_takes(a_rows, p.a_stride) || grid > 0x7fffffff) return HB_EINVAL;
-  HB_LAUNCH((panel_tile_kernel<Fmt, EPI>), dim3((unsigned)grid), dim3(64 * p.ks * p.nbw), panel_lds_bytes<Fmt>(PANEL_SLOT_ROWS / 16, p.ks, p.nbw), stream, p);
+  HB_LAUNCH((panel_tile_kernel<Fmt, EPI>), dim3((unsigned)grid), dim3(64 * p.ks * p.nbw), panel_routed_lds<Fmt>(PANEL_SLOT_ROWS / 16, p.nbw), stream, p);
   return HB_OK;
 }
 

@@ -1082,6 +1082,19 @@ struct TileW3 {
   // registers of two eight-wavefront workgroups fit a compute unit (the pair of them is 10 % faster than whole rounds say).
   static constexpr float EXPAND_US = 0.45f;
   static constexpr int BESIDE_TILES = 3;
+  // A routed call's slots of at most this many rows run on the weight stream's bodies, a wavefront a block over all of K. With
+  // one product a fragment the panel's expansion to scaled BF16 (four conversions, eight multiplications and four roundings a
+  // fragment) bounds the slot: 100 to 107 cycles a fragment and SIMD, two wavefronts. The stream's bodies convert
+  // without the scale and fold it into the FP32 sums (four conversions, four multiply-adds; up to four rows one): 84. Skewed
+  // routing of 10 of 512 experts (2048, 512), where 218 of 377 slots are such: the layer of 1024 rows 205 -> 187 us, 1543
+  // 251 -> 234, 2048 296 -> 271; even routing at the same sizes unchanged. A ring of four slots with the activations as far
+  // ahead gave nothing: what the wavefronts wait for is each other's issue slots.
+  static constexpr int LIGHT_ROWS = ROWS_PER_SLOT;
+  template <int EPI>
+  static __device__ __forceinline__ void light(const StreamParams& p, const Slot& sl, int group, uint8_t* lds) {
+    static_assert(BITS == 3 || epi_dense(EPI), "routed experts are three-bit");
+    if constexpr (BITS == 3) stream_workgroup<EPI, false, false, Ring>(p, sl, group, lds);
+  }
   struct Part {
     uint32_t lo, hi;  // codebook bytes of weights 0 .. 3 and 4 .. 7
     float scale;

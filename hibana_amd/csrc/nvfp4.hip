@@ -560,6 +560,7 @@ struct TileNvfp4 {
   static constexpr bool PER_ROW = false;
   static constexpr float EXPAND_US = 0.f;  // (the estimate's own constants are this format's)
   static constexpr int BESIDE_TILES = 0;
+  static constexpr int LOW_ROWS = 24, MIDDLE_ROWS = 46;  // panel_height's lines
   static constexpr int LIGHT_ROWS = 0;  // (an expansion takes the scale along at the price of the stream's)
   template <int EPI>
   static __device__ __forceinline__ void light(const StreamParams&, const Slot&, int, uint8_t*) {}
@@ -723,17 +724,16 @@ int64_t busy_slots(int64_t pairs, int experts, int64_t slots) { return pairs < 2
 int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, int m, int topk, const MoeWorkspace& ws, void* out_pairs,
                 int pairs_bf16, hipStream_t stream, int experts_total) {
   const int64_t pairs = (int64_t)m * topk, named = experts_named(experts_total, ex->base, ex->experts);
-  // A dense contraction once an expert sees about ten rows: slots of 128 rows on the panel kernel; below that the 16-row
-  // slots of the weight stream. Measured, stream and panel, the whole latent block in us: 512 experts (1024, 2688) 8 rows an
-  // expert 384 and 388, 12 rows 474 and 403, 24 rows 748 and 455; 256 experts (768, 1536) 8 rows 121 and 123, 10 rows 131 and
-  // 126, 24 rows 212 and 146; 128 experts (512, 1024) 10 rows 71 and 72, 24 rows 82 and 72. A range of the experts sees its
-  // share of the pairs only, and the stream's launches, sized for all of them, lose a little earlier: 64 of 512 experts
-  // (1024, 2688), the summed experts alone, 4 rows an expert 59 and 68, 8 rows 86 and 76; 256 of 512 8 rows 196 and 198, 11 rows
-  // 218 and 204; 32 of 256 (768, 1536) 8 rows 39 and 40, 16 rows 50 and 44.
-  const int64_t rows_min = ex->experts < named ? 8 : 10;
+  // A dense contraction once an expert sees seven rows: the panel kernel; below that the 16-row slots of the weight stream. Measured,
+  // stream and panel, the two launches in us: 160 experts (512, 1536) 6 rows an expert 41.8 and 44.8, 8 rows 45.4 and 45.2, 14 rows 50.0
+  // and 46.6; 300 experts (640, 1280) 6 rows 67 and 66, 8 rows 75 and 68; 400 experts (896, 2048) 6 rows 170 and 177, 8 rows 190 and 178, 11 rows
+  // 224 and 194; the whole latent block of 512 experts (1024, 2688) 6 rows 344 and 326, 8 rows 380 and 341. A range of the experts sees its
+  // share of the pairs only, and its few slots fill the device a little later: 64 of 512 experts
+  // (1024, 2688), the summed experts alone, on slots of 128 rows 4 rows an expert 59 and 68, 8 rows 86 and 76.
+  const int64_t rows_min = ex->experts < named ? 8 : 7;
   const bool dense = panel_takes(m, ex->hidden) && panel_takes(pairs, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
                      (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && pairs >= rows_min * named));
-  const int slot_rows = dense ? PANEL_SLOT_ROWS : ROWS_PER_SLOT;
+  const int tiles = panel_height<TileNvfp4>(pairs, named), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
   const int64_t slots = moe_max_slots(pairs, ex->experts, 0, slot_rows);
   if (slots > 65535) return HB_EINVAL;
   if (int e = moe_launch_plan(ids, pairs, ex->base, ex->experts, 0, ws, stream, slot_rows)) return e;
@@ -741,8 +741,8 @@ int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, i
   StreamParams p, f2;
   expert_params(ex, x, m, topk, ws, out_pairs, pairs_bf16, p, f2);
   if (dense) {
-    if (int e = ex->gated ? launch_panel_routed<TileNvfp4, EPI_FC1_GATED>(p, slots, m, stream) : launch_panel_routed<TileNvfp4, EPI_FC1_RELU2>(p, slots, m, stream)) return e;
-    if (int e = launch_panel_routed<TileNvfp4, EPI_FC2>(f2, slots, pairs, stream)) return e;
+    if (int e = ex->gated ? launch_panel_routed<TileNvfp4, EPI_FC1_GATED>(p, tiles, slots, m, stream) : launch_panel_routed<TileNvfp4, EPI_FC1_RELU2>(p, tiles, slots, m, stream)) return e;
+    if (int e = launch_panel_routed<TileNvfp4, EPI_FC2>(f2, tiles, slots, pairs, stream)) return e;
     return launch_status();
   }
   if (int e = ex->gated ? launch_nvfp4<EPI_FC1_GATED>(p, slots, est, stream) : launch_nvfp4<EPI_FC1_RELU2>(p, slots, est, stream)) return e;

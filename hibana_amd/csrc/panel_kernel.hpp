@@ -518,11 +518,22 @@ inline size_t panel_lds_bytes(int mt, int ks, int nbw) {
 }
 
 
-// Routed calls: a plan's slots of up to 128 rows, as many row tiles as the slot's rows need. Workgroups go to the eight
-// compute dies in turn: all of a slot's take the same place in that turn, so that its activations come into one L2 once
+template <class Fmt, int EPI, int MT>  // as many row tiles as the slot's rows need, MT at most
+__device__ __forceinline__ void panel_tiles(const StreamParams& p, const Slot& sl, uint8_t* lds, const PanelShare& part) {
+  if constexpr (MT > 1) {
+    if ((sl.rows + 15) >> 4 < MT) return panel_tiles<Fmt, EPI, MT - 1>(p, sl, lds, part);
+  }
+  Panel<Fmt, EPI, MT> panel;
+  panel.run(p, sl, lds, part);
+}
+
+// Routed calls: a plan's slots of up to 16 MOST rows. Workgroups go to the eight compute dies in turn: all of a slot's take
+// the same place in that turn, so that its activations come into one L2 once
 // (2048 rows, 22 of 512 experts, (1024, 2688): the latent block 811 -> 782 us; 1543 rows of the three-bit layer 285 -> 276).
-template <class Fmt, int EPI>
-__global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_tile_kernel(StreamParams p) {
+// A compute unit holds as many workgroups as the registers of the highest slot leave room for: four with slots of 48 rows, three
+// with 80, two with 128 (the choice: panel_height).
+template <class Fmt, int EPI, int MOST>
+__global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void panel_tile_kernel(StreamParams p) {
   extern __shared__ __align__(16) uint8_t panel_lds[];
   const int die = blockIdx.x & 7, local = blockIdx.x >> 3, round = local / p.panel_groups, slot = 8 * round + die;
   if (slot >= p.panel_full) return;
@@ -530,17 +541,7 @@ __global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_tile_kernel(StreamP
   const Slot sl = slot_of<EPI>(p, slot);
   if (sl.rows <= 0) return;  // a slot the plan did not fill: the whole workgroup leaves
   if (sl.rows <= Fmt::LIGHT_ROWS) return Fmt::template light<EPI>(p, sl, part.group, panel_lds);
-  auto run = [&](auto panel) { panel.run(p, sl, panel_lds, part); };
-  switch ((sl.rows + 15) >> 4) {
-    case 1: run(Panel<Fmt, EPI, 1>{}); break;
-    case 2: run(Panel<Fmt, EPI, 2>{}); break;
-    case 3: run(Panel<Fmt, EPI, 3>{}); break;
-    case 4: run(Panel<Fmt, EPI, 4>{}); break;
-    case 5: run(Panel<Fmt, EPI, 5>{}); break;
-    case 6: run(Panel<Fmt, EPI, 6>{}); break;
-    case 7: run(Panel<Fmt, EPI, 7>{}); break;
-    default: run(Panel<Fmt, EPI, 8>{}); break;
-  }
+  panel_tiles<Fmt, EPI, MOST>(p, sl, panel_lds, part);
 }
 
 // How a dense call is cut: row tiles a slot, the shape of a workgroup, the tiles whose K is shared and among how many.
@@ -688,21 +689,35 @@ inline size_t panel_routed_lds(int mt, int nbw) {
   return std::max(panel_lds_bytes<Fmt>(mt, 1, nbw), Fmt::LIGHT_ROWS > 0 ? (size_t)nbw * ring_bytes<typename Fmt::Ring>() : 0);
 }
 
-// Over a plan's slots of PANEL_SLOT_ROWS rows; `a_rows`: rows of the activation matrix. Four wavefronts a workgroup on four
-// blocks, two workgroups a compute unit: one's start and end lie beside the other's products.
-constexpr int PANEL_SLOT_ROWS = 128;
+// The row tiles of a routed call's slots, by its rows an expert. Higher slots expand an expert's weights for more rows at a
+// time; lower ones leave registers for more workgroups on a compute unit, and with few rows a product it is their starts, ends and
+// waits, not the expansion, that want something beside them. Measured at 48, 80 and 128 rows a slot, the summed experts' launches or the
+// whole block in us: NVFP4, 512 experts (1024, 2688) 8 rows an expert 341, 347 and 380, 18 rows 385, 399, 422, 24 rows 412, 414, 442,
+// 32 rows 475, 436, 464, 52 rows 617, 535, 526; 256 experts (768, 1536) 14 rows 116, 118, 133, 40 rows 165, 151, 160, 64 rows 207, 188, 182.
+// Three-bit, 512 experts (2048, 512), even routing 14 rows 223, 234, 252, 24 rows 262, 265, 277, 40 rows 324, 313, 321, 52 rows
+// 421, 351, 366; skewed 14 rows 176, 171, 174, 24 rows 232, 217, 224, 52 rows 395, 351, 343; 180 experts (1664, 384) 64 rows 158, 135, 143, 90
+// rows 184, 179, 167.
+constexpr int PANEL_SLOT_TILES = 8;  // at most
+template <class Fmt>
+inline int panel_height(int64_t pairs, int64_t named) {
+  return pairs < Fmt::LOW_ROWS * named ? 3 : pairs < Fmt::MIDDLE_ROWS * named ? 5 : PANEL_SLOT_TILES;
+}
+
+// Over a plan's slots of 16 `tiles` rows; `a_rows`: rows of the activation matrix. Four wavefronts a workgroup on four
+// blocks, two to four workgroups a compute unit: one's start and end lie beside the others' products.
 template <class Fmt, int EPI>
-static int launch_panel_routed(StreamParams& p, int64_t slots, int64_t a_rows, hipStream_t stream) {
+static int launch_panel_routed(StreamParams& p, int tiles, int64_t slots, int64_t a_rows, hipStream_t stream) {
   p.ks = 1;
   p.nbw = 4;
   set_split(p);
-  p.slot_rows = PANEL_SLOT_ROWS;
+  p.slot_rows = 16 * tiles;
   p.panel_groups = (p.n_blocks + p.nbw - 1) / p.nbw;
   p.a_bytes = (uint32_t)(a_rows * p.a_stride * 2);
   p.panel_full = (int)slots;
   const int64_t grid = (slots + 7) / 8 * 8 * p.panel_groups;
   if (!panel_takes(a_rows, p.a_stride) || grid > 0x7fffffff) return HB_EINVAL;
-  HB_LAUNCH((panel_tile_kernel<Fmt, EPI>), dim3((unsigned)grid), dim3(64 * p.ks * p.nbw), panel_routed_lds<Fmt>(PANEL_SLOT_ROWS / 16, p.nbw), stream, p);
+  auto launch = [&](auto kernel) { HB_LAUNCH(kernel, dim3((unsigned)grid), dim3(64 * p.ks * p.nbw), panel_routed_lds<Fmt>(tiles, p.nbw), stream, p); };
+  tiles == 3 ? launch(panel_tile_kernel<Fmt, EPI, 3>) : tiles == 5 ? launch(panel_tile_kernel<Fmt, EPI, 5>) : launch(panel_tile_kernel<Fmt, EPI, PANEL_SLOT_TILES>);
   return HB_OK;
 }
 

@@ -1089,6 +1089,7 @@ struct TileW3 {
   // routing of 10 of 512 experts (2048, 512), where 218 of 377 slots are such: the layer of 1024 rows 205 -> 187 us, 1543
   // 251 -> 234, 2048 296 -> 271; even routing at the same sizes unchanged. A ring of four slots with the activations as far
   // ahead gave nothing: what the wavefronts wait for is each other's issue slots.
+  static constexpr int LOW_ROWS = 22, MIDDLE_ROWS = 60;  // panel_height's lines
   static constexpr int LIGHT_ROWS = ROWS_PER_SLOT;
   template <int EPI>
   static __device__ __forceinline__ void light(const StreamParams& p, const Slot& sl, int group, uint8_t* lds) {
@@ -1368,20 +1369,21 @@ struct Routing {  // set: the chain routes the logits itself into the caller's i
 int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void* x, const int32_t* ids, int m, int topk,
                 const MoeWorkspace& ws, void* out_pairs, int pairs_bf16, hipStream_t stream, int experts_total, const Routing* route = nullptr,
                 bool e4m3 = false, const CombineParams* combine = nullptr) {
-  const int64_t pairs = (int64_t)m * topk, named = experts_named(experts_total, ex->base, ex->experts);
+  const int64_t pairs = (int64_t)m * topk, named = experts_named(experts_total, ex->base, ex->experts), local = pairs * ex->experts / named;
   const int shared_rows = shared ? m : 0;
-  // A dense contraction once an expert sees a few dozen rows: slots of 128 rows on the panel kernel (E4M3 activations: the
-  // stream only). The stream pays for a pass a sixteen rows, the panel for an expansion the few rows do not amortise and for
-  // a last round of workgroups that a small call does not fill. Measured, stream and panel, the whole layer in us: 512
-  // experts (2048, 512) 12 rows an expert 235 and 267, 16 rows 288 and 277, 30 rows 439 and 311 (skewed routing 16 rows 248
-  // and 208); 256 experts (2560, 768) 12 rows 224 and 235, 16 rows 292 and 250; 128 experts (2048, 512) 20 rows (0.98 M
-  // pairs x blocks) 111 and 120, 24 rows (1.2 M) 123 and 123; 128 experts (1024, 256) 24 rows (0.3 M) 70 and 83, 48 rows 98
-  // and 100, 96 rows 132 and 100. A range of the experts sees its share of the pairs only: 64 of 512 (2048, 512), the summed
-  // experts alone, 5 rows an expert 44 and 53, 16 rows 72 and 72, 31 rows 98 and 90; 256 of 512 12 rows 116 and 138, 20 rows 179 and 157.
+  // A dense contraction once an expert sees ten rows or more: the panel kernel's higher slots (E4M3 activations: the stream only).
+  // The stream pays for a pass a sixteen rows, the panel for two launches where the stream has one, which a call of few
+  // experts does not fill. The lines lie where neither even nor skewed routing loses. Measured, stream and panel (at its better
+  // height), the whole layer in us: 512 experts (2048, 512) 8 rows an expert 191 and 196 (skewed 152 and 131), 11 rows 215 and
+  // 211 (189 and 157), 14 rows 253 and 223 (225 and 176); 256 experts (2560, 768) 11 rows 210 and 192; 180 experts (1664, 384) 13 rows
+  // (0.55 M pairs x blocks) 88 and 88, 16 rows (0.67 M) 98 and 90; 300 experts (1280, 384) 13 rows 95 and 94, 16 rows 111 and 99; 96 experts (2560,
+  // 768) 13 rows (0.9 M) 100 and 107, 16 rows 128 and 119; 64 experts (2048, 512) 25 rows (0.6 M) 76 and 83; 128 experts (1024, 256)
+  // 24 rows 63 and 66, 32 rows 70 and 69, 40 rows 77 and 73. A range of the experts sees its share of the pairs only.
   const int64_t expert_blocks = (int64_t)((ex->gated ? 2 : 1) * ex->inter / W3_BLOCK_ROWS) * (ex->hidden / W3_CHUNK) + (int64_t)(ex->hidden_out / W3_BLOCK_ROWS) * (ex->inter / W3_CHUNK);
   const bool dense = !e4m3 && panel_takes(m, ex->hidden) && panel_takes(pairs + shared_rows, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
-                     (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && (pairs >= 48 * named || (pairs >= 16 * named && pairs * expert_blocks >= 1000000))));
-  const int slot_rows = dense ? PANEL_SLOT_ROWS : ROWS_PER_SLOT;
+                     (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && (pairs >= (ex->experts < named ? 48 : 32) * named || (pairs >= 16 * named && local * expert_blocks >= 650000) ||
+                                                                                        (pairs >= 10 * named && local * expert_blocks >= 1400000))));
+  const int tiles = panel_height<TileW3<3>>(pairs, named), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
   // Under a budget the table ends behind the experts the selection can name: the launches' grids reach over all of it, and a
   // workgroup without rows is not free (40 rows of 10, a cap of 60 of 512 experts: 53.5 us before, 53.2 so). What a call of
   // these pairs is refused for, and how its launches split K, go by the whole table: the bits of the same ids without a budget.
@@ -1462,8 +1464,8 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   f2.out_stride = ex->hidden_out;
   f2.out_bf16 = pairs_bf16;
   if (dense) {
-    if (int e = ex->gated ? launch_panel_routed<TileW3<3>, EPI_FC1_GATED>(p, slots, m, stream) : launch_panel_routed<TileW3<3>, EPI_FC1_RELU2>(p, slots, m, stream)) return e;
-    if (int e = launch_panel_routed<TileW3<3>, EPI_FC2>(f2, slots, pairs + shared_rows, stream)) return e;
+    if (int e = ex->gated ? launch_panel_routed<TileW3<3>, EPI_FC1_GATED>(p, tiles, slots, m, stream) : launch_panel_routed<TileW3<3>, EPI_FC1_RELU2>(p, tiles, slots, m, stream)) return e;
+    if (int e = launch_panel_routed<TileW3<3>, EPI_FC2>(f2, tiles, slots, pairs + shared_rows, stream)) return e;
     if (combine) moe_launch_combine(*combine, stream);
     return launch_status();
   }

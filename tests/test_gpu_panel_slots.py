@@ -1,9 +1,10 @@
 """Routed calls on the panel kernel, slot by slot: the weight stream's bodies for a slot's few rows (one to four, five to
-sixteen), the panel's from seventeen, at every number of K chunks around the stream's two-deep ring."""
+sixteen), the panel's from seventeen, at every number of K chunks around the stream's two-deep ring; slots of 48, 80 and 128
+rows, which the rows an expert choose; and the lines that give a call to the panel kernel."""
 import pytest
 import torch
 
-from oracle import layers
+from oracle import layers, nvfp4_format as onv
 from tests.util import MAX_REL, NORM_REL, errors, oracle_expert_getter, random_experts
 
 pytestmark = pytest.mark.gpu
@@ -17,21 +18,71 @@ def _call(counts, seed):
     return m, ids, g
 
 
+TOTALS = [0, 31, 100]  # experts that the ids are said to name: 59, 46 and 14 rows an expert
+MORE = [300]            # ... and with one expert more 69
+
+
+@pytest.mark.parametrize("total,more", [(t, []) for t in TOTALS] + [(0, MORE)])
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("hidden,inter", [(128, 256), (256, 384), (384, 128), (640, 512)])  # 1, 2, 3, 5 chunks of fc1; 2, 3, 1, 4 of fc2
-def test_w3_slots_of_every_height(hidden, inter, gated):
+def test_w3_slots_of_every_height(hidden, inter, gated, total, more):
     from hibana_amd import _lib
     from hibana_amd.kernels import w3_moe
-    ex, per = random_experts(len(COUNTS), hidden, inter, gated, 9)
-    m, ids, g = _call(COUNTS, hidden)
+    counts = COUNTS + more
+    ex, per = random_experts(len(counts), hidden, inter, gated, 9)
+    m, ids, g = _call(counts, hidden)
     x = torch.randn(m, hidden, generator=g).bfloat16()
-    want = layers.routed_experts_ref(x, ids.numpy(), oracle_expert_getter(per, gated, inter), gated, e_n=len(COUNTS))
+    want = layers.routed_experts_ref(x, ids.numpy(), oracle_expert_getter(per, gated, inter), gated, e_n=len(counts))
+    ones = torch.ones(m, 1, device="cuda")
     assert _lib.lib().hb_tune(b"w3_tile", 1) == 0
     try:
-        got = w3_moe.w3_moe(ex, x.cuda(), ids.cuda(), torch.ones(m, 1, device="cuda"))
-        again = w3_moe.w3_moe(ex, x.cuda(), ids.cuda(), torch.ones(m, 1, device="cuda"))
+        got, again = (w3_moe.w3_moe(ex, x.cuda(), ids.cuda(), ones, experts_total=total) for _ in range(2))
     finally:
         _lib.lib().hb_tune(b"w3_tile", 0)
     mx, nr = errors(got, want)
     assert mx < MAX_REL and nr < NORM_REL, (mx, nr)
     assert torch.equal(got, again)
+
+
+@pytest.mark.parametrize("total,more", [(t, []) for t in TOTALS] + [(0, MORE)])
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("hidden,inter", [(128, 256), (384, 128)])
+def test_nvfp4_slots_of_every_height(hidden, inter, gated, total, more):
+    from hibana_amd import _lib
+    from tests.test_gpu_nvfp4_moe import _experts
+    counts = COUNTS + more
+    ex, (w1, s1, g1, w2, s2, g2) = _experts(len(counts), hidden, inter, gated, 4)
+    m, ids, g = _call(counts, inter)
+    x = torch.randn(m, hidden, generator=g).bfloat16()
+
+    def get(i):
+        return onv.unpack_fp4(w1[i], s1[i]) * g1[i], onv.unpack_fp4(w2[i], s2[i]) * g2[i]
+
+    want = layers.routed_experts_ref(x, ids.numpy(), get, gated, e_n=len(counts))
+    assert _lib.lib().hb_tune(b"nvfp4_tile", 1) == 0
+    try:
+        got = ex(x.cuda(), ids.cuda(), torch.ones(m, 1, device="cuda"), experts_total=total)
+    finally:
+        _lib.lib().hb_tune(b"nvfp4_tile", 0)
+    mx, nr = errors(got, want)
+    assert mx < MAX_REL and nr < NORM_REL, (mx, nr)
+
+
+@pytest.mark.parametrize("m,panel", [(255, False), (256, True)])  # 16 rows an expert of 64, 0.79 M pairs x blocks
+def test_w3_calls_from_sixteen_rows_an_expert(m, panel):
+    """The two kernels add in different orders, so the bits say which one ran."""
+    from hibana_amd import _lib, synthetic
+    from hibana_amd.kernels import w3_moe
+    ex = synthetic.w3_experts(64, 2048, 1024, True, 3)  # 768 blocks an expert
+    g = torch.Generator().manual_seed(m)
+    ids = torch.stack([torch.randperm(64, generator=g)[:4] for _ in range(m)]).to(torch.int32).cuda()
+    x, weights = torch.randn(m, 2048, generator=g).bfloat16().cuda(), torch.rand(m, 4, generator=g).cuda()
+    results = []
+    for tile in (0, 1, 2):
+        assert _lib.lib().hb_tune(b"w3_tile", tile) == 0
+        try:
+            results.append(w3_moe.w3_moe(ex, x, ids, weights))
+        finally:
+            _lib.lib().hb_tune(b"w3_tile", 0)
+    got, by_panel, by_stream = results
+    assert not torch.equal(by_panel, by_stream) and torch.equal(got, by_panel if panel else by_stream)

@@ -124,7 +124,7 @@ def latent_prefill(args) -> dict:
         block(x)
     torch.cuda.synchronize()
     hip = Hip()
-    names = ["route", "plan count", "plan scan", "plan place", "fc1", "fc2", "combine"]  # 45 056 pairs: the plan is three launches
+    names = ["route", "plan count", "plan place", "fc1", "fc2", "combine"]  # 45 056 pairs: the plan is two launches
     per_kernel = {n: [] for n in names}
     for rep in range(4):
         evs = hip.events(2 * len(names))

@@ -92,38 +92,27 @@ __device__ __forceinline__ Scan2 block_exclusive_scan2(Scan2 v, int* scratch, Sc
 // Exclusive scan of three integers per thread over the workgroup at once; `total` receives the three sums.
 __device__ __forceinline__ Scan3 block_exclusive_scan3(Scan3 v, int* scratch /* 3 * (PLAN_WAVES + 1) ints */, Scan3* total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  Scan3 inc = v;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int oa = __shfl_up(inc.a, d), ob = __shfl_up(inc.b, d), oc = __shfl_up(inc.c, d);
-    if (lane >= d) {
-      inc.a += oa;
-      inc.b += ob;
-      inc.c += oc;
-    }
-  }
+  const Scan3 inc{wave_inclusive_sum(v.a), wave_inclusive_sum(v.b), wave_inclusive_sum(v.c)};
   __syncthreads();  // scratch may still be read from a previous scan
   if (lane == 63) {
     scratch[wave] = inc.a;
-    scratch[PLAN_WAVES + 1 + wave] = inc.b;
-    scratch[2 * (PLAN_WAVES + 1) + wave] = inc.c;
+    scratch[PLAN_WAVES + wave] = inc.b;
+    scratch[2 * PLAN_WAVES + wave] = inc.c;
   }
   __syncthreads();
-  if (threadIdx.x < 3) {
-    int* row = scratch + threadIdx.x * (PLAN_WAVES + 1);
-    int run = 0;
-    for (int wv = 0; wv < PLAN_WAVES; wv++) {
-      const int c = row[wv];
-      row[wv] = run;
-      run += c;
-    }
-    row[PLAN_WAVES] = run;
+  Scan3 before{0, 0, 0}, all{0, 0, 0};
+#pragma unroll
+  for (int w = 0; w < PLAN_WAVES; w++) {  // the same address in every lane: broadcast reads
+    const int a = scratch[w], b = scratch[PLAN_WAVES + w], c = scratch[2 * PLAN_WAVES + w];
+    before.a += w < wave ? a : 0;
+    before.b += w < wave ? b : 0;
+    before.c += w < wave ? c : 0;
+    all.a += a;
+    all.b += b;
+    all.c += c;
   }
-  __syncthreads();
-  total->a = scratch[PLAN_WAVES];
-  total->b = scratch[2 * PLAN_WAVES + 1];
-  total->c = scratch[3 * PLAN_WAVES + 2];
-  return Scan3{scratch[wave] + inc.a - v.a, scratch[PLAN_WAVES + 1 + wave] + inc.b - v.b, scratch[2 * (PLAN_WAVES + 1) + wave] + inc.c - v.c};
+  *total = all;
+  return Scan3{before.a + inc.a - v.a, before.b + inc.b - v.b, before.c + inc.c - v.c};
 }
 
 // The plan of at most 64 pairs (a decode step), by one wavefront, a pair a lane: no counters per expert, no scan over
@@ -449,8 +438,8 @@ __device__ __forceinline__ void plan_work(const int32_t* ids, int pairs, int e_l
 //
 // With `job.lanes` set the launch has further workgroups, which round the job's activations to E4M3 and plan nothing.
 //
-// Many pairs (a prefill chunk) are shared among `groups` workgroups in three launches of this kernel, `wide` [groups, e_n]
-// between them: phase 1, each group counts its share of the pairs per expert; phase 2, one workgroup adds the groups'
+// Many pairs (a prefill chunk) are counted by `groups` workgroups into `wide` [groups, e_n] (phase 1; moe_place_kernel does the rest),
+// and very many, or ones with a rounding job, shared among them in three launches of this kernel, `wide` between them: phase 1, each group counts its share of the pairs per expert; phase 2, one workgroup adds the groups'
 // counts, writes the slot table and turns `wide` into the first sorted position of each group's run of each expert;
 // phase 3, each group places its share. Phase 0 is all of it in one workgroup.
 template <bool WIDE>
@@ -474,6 +463,125 @@ __global__ __launch_bounds__(PLAN_THREADS) void moe_plan_kernel(const int32_t* i
     return;
   }
   plan_work<WIDE>(ids, pairs, e_lo, e_n, shared_rows, plan, order, slot_rows, slot_cap, wide, groups, phase, blockIdx.x, lds);
+}
+
+// The plan of more pairs than one workgroup places quickly, by workgroups that each place a share of `share` pairs (a multiple
+// of 64, one pair a thread) and share nothing: every one of them learns all experts' counts, and how many of those are
+// ahead of its share, for itself. Writes exactly what plan_work writes. TABLE: from the counts of the shares `wide`
+// [gridDim.x, e_n] that a launch ahead of it has made (moe_plan_kernel, phase 1); else from all ids, read by each workgroup.
+// What bounds it is latency: one trip to memory for the ids or counts, a histogram in LDS, the scan over the experts, the
+// stores. One workgroup that plans behind the routing in its launch took 15.0 us for both at 128 rows of ten, 21.8 at 512 (a
+// routing launch and this one 5.4 + 5.9 and 6.2 + 7.2); alone 14.4 us at 5632 pairs; count, scan and place as three launches 19.2 us at
+// 15430 pairs, 19.8 at 45056 (count and this 12.2 and 14.7).
+constexpr int PLACE_SHARE = 256, PLACE_TABLE_SHARE = PLAN_THREADS;
+template <bool TABLE>
+__global__ __launch_bounds__(PLAN_THREADS) void moe_place_kernel(const int32_t* __restrict__ ids, int pairs, int e_lo, int e_n, int shared_rows,
+                                                                 int32_t* __restrict__ plan, int32_t* __restrict__ order, int slot_rows, int slot_cap,
+                                                                 const int32_t* __restrict__ wide) {
+  constexpr int SHARE = TABLE ? PLACE_TABLE_SHARE : PLACE_SHARE, TILES = SHARE / 64;
+  extern __shared__ int lds[];
+  int* run = lds;                                      // [TILES][e_n]: pairs of expert e in tile w of the share, then the tile's first position
+  int* total = run + TILES * e_n;                      // [e_n] (from all ids) pairs of expert e ...
+  int* ahead = total + e_n;                            // [e_n] ... and those ahead of the share
+  int* scratch = TABLE ? total : ahead + e_n;          // [3 * (PLAN_WAVES + 1)]
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, group = blockIdx.x, groups = gridDim.x, lo = group * SHARE;
+  auto local = [&](int i) {
+    const int e = i < pairs ? ids[i] - e_lo : -1;
+    return e >= 0 && e < e_n ? e : -1;
+  };
+  const int mine = threadIdx.x < SHARE ? local(lo + threadIdx.x) : -1;
+  const int e = threadIdx.x;  // one thread an expert: the launch keeps e_n <= PLAN_THREADS
+  int count = 0, before = 0;
+  if (TABLE) {
+    constexpr int BATCH = 16;  // asked for together, without a condition
+    for (int g0 = 0; g0 < groups; g0 += BATCH) {
+      int of_group[BATCH];
+#pragma unroll
+      for (int j = 0; j < BATCH; j++) of_group[j] = wide[min(g0 + j, groups - 1) * e_n + min(e, e_n - 1)];
+#pragma unroll
+      for (int j = 0; j < BATCH; j++) {
+        count += g0 + j < groups ? of_group[j] : 0;
+        before += g0 + j < group ? of_group[j] : 0;
+      }
+    }
+    if (e >= e_n) count = 0;
+  }
+  for (int i = threadIdx.x; i < (TABLE ? TILES : TILES + 2) * e_n; i += PLAN_THREADS) lds[i] = 0;
+  __syncthreads();
+  if (!TABLE) {
+    for (int i0 = threadIdx.x; i0 < pairs; i0 += PLAN_THREADS * PLAN_BATCH) {
+      int of[PLAN_BATCH];
+#pragma unroll
+      for (int j = 0; j < PLAN_BATCH; j++) of[j] = local(i0 + j * PLAN_THREADS);
+#pragma unroll
+      for (int j = 0; j < PLAN_BATCH; j++)
+        if (of[j] >= 0) {
+          atomicAdd(&total[of[j]], 1);
+          if (i0 + j * PLAN_THREADS < lo) atomicAdd(&ahead[of[j]], 1);
+        }
+    }
+  }
+  // the lanes of a tile that name the same expert, by ballots over the id's bits
+  int rank = 0;
+  if (wave < TILES) {
+    int id_bits = 1;
+    while ((1 << id_bits) < e_n) id_bits++;
+    uint64_t same = __ballot(mine >= 0);
+    for (int b = 0; b < id_bits; b++) {
+      const uint64_t m = __ballot((mine >> b) & 1);
+      same &= ((mine >> b) & 1) ? m : ~m;
+    }
+    rank = __popcll(same & ((1ull << lane) - 1ull));
+    if (mine >= 0 && rank == 0) run[wave * e_n + mine] = __popcll(same);
+  }
+  __syncthreads();
+  if (!TABLE && e < e_n) count = total[e], before = ahead[e];
+  const int my_slots = (count + slot_rows - 1) / slot_rows, shared_slots = (shared_rows + slot_rows - 1) / slot_rows;
+  const bool heavy = 4 * count > slot_rows;
+  Scan3 tot;  // as in plan_work
+  const Scan3 at = block_exclusive_scan3(Scan3{count, (heavy ? my_slots : 0) | (count > 0 ? 1 << 16 : 0), heavy ? 0 : my_slots}, scratch, &tot);
+  const int kept = tot.a, heavy_slots = tot.b & 0xffff, slots = shared_slots + heavy_slots + tot.c;
+  if (e < e_n) {
+    int first = at.a + before;
+#pragma unroll
+    for (int w = 0; w < TILES; w++) {
+      const int c = run[w * e_n + e];
+      run[w * e_n + e] = first;
+      first += c;
+    }
+  }
+  __syncthreads();
+  if (mine >= 0) order[run[wave * e_n + mine] + rank] = lo + threadIdx.x;
+  // what is written once, dealt out to the workgroups
+  if (e < e_n && e % groups == group) {
+    const int my_slot = shared_slots + (heavy ? (at.b & 0xffff) : heavy_slots + at.c);
+    for (int s = 0; s < my_slots; s++) {
+      int32_t* entry = plan + PLAN_HEADER + 4 * (my_slot + s);
+      entry[0] = e;
+      entry[1] = at.a + s * slot_rows;
+      entry[2] = min(slot_rows, count - s * slot_rows);
+      entry[3] = 0;
+    }
+  }
+  const int first = group * PLAN_THREADS + threadIdx.x, step = groups * PLAN_THREADS;
+  for (int s = first; s < shared_slots; s += step) {
+    int32_t* entry = plan + PLAN_HEADER + 4 * s;
+    entry[0] = -1;
+    entry[1] = kept + s * slot_rows;
+    entry[2] = min(slot_rows, shared_rows - s * slot_rows);
+    entry[3] = 0;
+  }
+  for (int r = first; r < shared_rows; r += step) order[kept + r] = pairs + r;
+  for (int s = slots + first; s < slot_cap; s += step) {
+    int32_t* entry = plan + PLAN_HEADER + 4 * s;
+    entry[0] = entry[1] = entry[2] = entry[3] = 0;
+  }
+  for (int s = first; s < slot_cap; s += step) plan_done(plan, slot_cap)[s * DONE_PITCH] = 0;
+  if (first == 0) {
+    plan[0] = slots;
+    plan[1] = tot.b >> 16;
+    plan[2] = kept;
+  }
 }
 
 // For launches whose last workgroup plans. "No rows" into every entry of the slot table and the slots' arrival counters at
@@ -956,6 +1064,9 @@ int moe_tune(const char* key, int value) {
   return HB_OK;
 }
 
+// From this many pairs: the layer of 65 and 80 rows of ten took 66.5 and 71.8 us with one workgroup, 67.1 and 72.5 in shares, of 128
+// rows 80.8 and 77.9, of 256 rows 113.6 and 108.8; a latent block of 64 rows of 22 283 and 278.
+constexpr int64_t PLACE_PAIRS = 1024;
 static unsigned plan_groups(const QuantJob* job) {
   if (!job) return 1u;
   return 1u + (job->split_rows ? (unsigned)job->split_rows : (unsigned)((job->lanes + PLAN_THREADS - 1) / PLAN_THREADS));
@@ -966,6 +1077,22 @@ int moe_launch_plan(const int32_t* ids, int64_t pairs, int e_lo, int e_n, int sh
   const size_t plan_lds = ((size_t)(PLAN_WAVES + 1) * e_n + 3 * (PLAN_WAVES + 1)) * sizeof(int);
   if (plan_lds > 64 * 1024 || e_n > PLAN_THREADS || pairs > 0x3fffffff) return HB_EINVAL;
   const int slot_cap = (int)moe_max_slots(pairs, distinct ? distinct : e_n, shared_rows, slot_rows);
+  if (!job && pairs >= PLACE_PAIRS && pairs <= PLACE_TABLE_SHARE * PLAN_WIDE_GROUPS) {
+    auto place = [&](auto kernel, int share, int tiles) {
+      const size_t lds = ((size_t)tiles * e_n + 3 * (PLAN_WAVES + 1)) * sizeof(int);
+      HB_LAUNCH(kernel, dim3((unsigned)((pairs + share - 1) / share)), dim3(PLAN_THREADS), lds, stream, ids, (int)pairs, e_lo, e_n, shared_rows, ws.plan,
+                ws.order, slot_rows, slot_cap, ws.plan_wide);
+    };
+    if (pairs < PLAN_WIDE_PAIRS) {
+      place(moe_place_kernel<false>, PLACE_SHARE, PLACE_SHARE / 64 + 2);
+    } else {
+      const int groups = (int)((pairs + PLACE_TABLE_SHARE - 1) / PLACE_TABLE_SHARE);  // the counting workgroups' shares are the placing ones'
+      HB_LAUNCH(moe_plan_kernel<true>, dim3(groups), dim3(PLAN_THREADS), plan_lds, stream, ids, (int)pairs, e_lo, e_n, shared_rows, ws.plan, ws.order,
+                RouteParams{}, 0, 0, slot_rows, slot_cap, ws.plan_wide, groups, 1, QuantJob{});
+      place(moe_place_kernel<true>, PLACE_TABLE_SHARE, PLACE_TABLE_SHARE / 64);
+    }
+    return HB_OK;
+  }
   if (pairs >= PLAN_WIDE_PAIRS) {  // a share of about a thousand pairs a workgroup
     const int groups = (int)std::min<int64_t>(PLAN_WIDE_GROUPS, pairs / 1024);
     if (job) moe_launch_quant_groups(*job, stream);
@@ -994,7 +1121,8 @@ static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, in
   // rows that name no expert twice: every row is real, or a padded row names none (with `repeat` it names one over and over)
   const bool distinct = !rp.slots || (!rp.repeat && (rp.pad_id < e_lo || rp.pad_id >= e_lo + e_n));
   const int by_rows = distinct && m <= PLAN_ROWS_MAX && rp.k <= 64 && g_route_plan_fused.load(std::memory_order_relaxed) != 1;
-  if (m > ROUTE_FUSED_ROWS && pairs < PLAN_WIDE_PAIRS && g_route_plan_fused.load(std::memory_order_relaxed) != 2) {
+  const bool apart = !job && m > PLAN_ROWS_MAX && pairs >= PLACE_PAIRS && g_route_plan_fused.load(std::memory_order_relaxed) == 0;
+  if (m > ROUTE_FUSED_ROWS && pairs < PLAN_WIDE_PAIRS && g_route_plan_fused.load(std::memory_order_relaxed) != 2 && !apart) {
     // a verify-sized call: the routing spread over the device, the plan by the workgroup that finishes last
     const int group_rows = m <= ROUTE_SPREAD_ROWS ? 1 : ROUTE_GROUP_ROWS, groups = (m + group_rows - 1) / group_rows;
     HB_LAUNCH(moe_route_plan_kernel, dim3((unsigned)groups + plan_groups(job) - 1u), dim3(PLAN_THREADS), plan_lds, stream, rp.ids, (int)pairs, e_lo, e_n,
@@ -1069,7 +1197,7 @@ int moe_launch_budget_plan(const BudgetRoute& b, int m, int topk, int32_t* ids, 
   const int copies_n = small ? BUDGET_WAVES : BUDGET_WAVES / 2;
   const size_t pick_lds = (size_t)copies_n * b.e * sizeof(float);
   const int distinct = (int)budget_distinct(b, m, e_n), slot_cap = (int)moe_max_slots(pairs, distinct, shared_rows, slot_rows);
-  const bool plan = pairs < PLAN_WIDE_PAIRS, by_rows = plan && !b.repeat && m <= PLAN_ROWS_MAX && topk <= 64;
+  const bool plan = m <= PLAN_ROWS_MAX || pairs < PLACE_PAIRS, by_rows = plan && !b.repeat && m <= PLAN_ROWS_MAX && topk <= 64;
   const int group_rows = m <= BUDGET_SPREAD_ROWS ? 1 : PLAN_WAVES;  // a row a workgroup while that spreads them over the device
   const dim3 grid((unsigned)((m + group_rows - 1) / group_rows));
   const size_t lds = plan ? std::max(pick_lds, plan_lds) : pick_lds;

@@ -50,18 +50,6 @@ struct Scan3 {
   int a, b, c;
 };
 
-// Inclusive prefix sum over the wavefront's lanes without LDS: shifts within rows of sixteen lanes, then the rows' last
-// lanes broadcast to the rows after them (DPP).
-__device__ __forceinline__ int wave_inclusive_sum(int x) {
-  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
-  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
-  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
-  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
-  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
-  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
-  return x;
-}
-
 // Exclusive scan over the workgroup of two words a thread whose four 16-bit halves are sums of their own (none reaches
 // 65536, so no carry crosses a half): one DPP scan a word in each wavefront, the wavefronts' totals through LDS, one
 // barrier. `total` receives the two sums. scratch: 2 * PLAN_WAVES ints, not in use by anyone before the call's barrier.

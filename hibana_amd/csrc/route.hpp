@@ -9,10 +9,8 @@ namespace hb {
 // Top-k routing, one wavefront per row: softmax over all experts, top-k, renormalized
 // (hibana/kernels/flashnext_fused.py:278-319 of the reference), or sigmoid scores chosen by score + bias with the plain
 // scores as weights (hibana/model/nemotron/moe.py:57-121). Lane l holds experts l * per .. l * per + per - 1 in
-// registers as order-preserving 32-bit keys, so a selection round is one wave-wide integer maximum (DPP within rows of
-// 16, four scalar reads across them) and a ballot: among equal scores the lowest lane, then the lowest register,
-// wins - the lowest expert id. Up to eight registers a lane are sorted once and a round looks at their heads; with
-// sixteen a round scans them.
+// registers as order-preserving 32-bit keys; among equal scores the lowest lane, then the lowest register, wins - the lowest
+// expert id (top_ranked).
 constexpr int ROUTE_PER_LANE = 16;
 
 __device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
@@ -25,16 +23,125 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t x) {
   return max(max(a, b), max(c, d));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
-  return v;
+// The largest of a value over the wavefront (NaN only if all are), in every lane.
+__device__ __forceinline__ float wave_max(float x) {
+  x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0xB1, 0xF, 0xF, false)));
+  x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x4E, 0xF, 0xF, false)));
+  x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x141, 0xF, 0xF, false)));
+  x = fmaxf(x, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x140, 0xF, 0xF, false)));
+  const int bits = __builtin_bit_cast(int, x);
+  const float a = __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 0)), b = __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 16));
+  const float c = __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 32)), d = __builtin_bit_cast(float, __builtin_amdgcn_readlane(bits, 48));
+  return fmaxf(fmaxf(a, b), fmaxf(c, d));
 }
 
 // Key of a score: larger score <=> larger key, every real key above 0 (the key of an empty register).
 __device__ __forceinline__ uint32_t score_key(float v) {
   const int32_t bits = __builtin_bit_cast(int32_t, v);
   return (uint32_t)(bits ^ ((bits >> 31) & 0x7fffffff)) ^ 0x80000000u;
+}
+
+// Inclusive prefix sum over the wavefront's lanes without LDS: shifts within rows of sixteen lanes, then the rows' last
+// lanes broadcast to the rows after them (DPP).
+__device__ __forceinline__ int wave_inclusive_sum(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xF, 0xF, false);  // row_shr:1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xF, 0xF, false);  // row_shr:2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xF, 0xF, false);  // row_shr:4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xF, 0xF, false);  // row_shr:8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xA, 0xF, false);  // row_bcast:15 into rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xC, 0xF, false);  // row_bcast:31 into rows 2 and 3
+  return x;
+}
+
+// The k largest of a wavefront's keys (0: no key), largest first, one a lane: lane s < k gets selection s's key and its tag, the
+// lane's place of it (lane * per + register). Equal keys in ascending lane, then register.
+//
+// A threshold that at least k lanes' largest keys reach, found by cutting the interval in four a step; the keys that reach it, some
+// k + k / 4 of them, go to a lane each (ds_permute), every lane counts the ones ahead of its own, and they go to the lanes their ranks
+// name. Before, a round a selection (wave-wide maximum, ballot, a lane's list moving up) on lists sorted in each lane and sums and maxima through the LDS:
+// one token of the three-bit layer (top 10 of 512) 19.8 us, 19.2 so; the latent block's one token (top 22 of 512) 47.4 and 46.0, four 81.6
+// and 79.7.
+// Rounds, without the sort, remain for rows where more than 63 keys reach the threshold: many equal scores, or the best experts
+// side by side in a few lanes.
+constexpr int TOP_SLACK = 3;  // lanes that may reach the threshold beyond k
+template <int PER>
+__device__ __forceinline__ void top_ranked(uint32_t (&key)[PER], int per, int k, int lane, uint32_t& out_key, int& out_tag) {
+  uint32_t head = key[0];
+#pragma unroll
+  for (int j = 1; j < PER; j++) head = max(head, key[j]);
+  const uint32_t most = wave_max_u32(head), least = ~wave_max_u32(~head);
+  uint32_t lo = max(least, 1u), hi = most;  // at least k lanes reach lo (or all that hold a key do); fewer than k reach hi, unless it is the threshold
+  if (__popcll(__ballot(head >= hi)) >= k) lo = hi;
+  while (hi - lo > 1u) {  // three places of the interval a step, their ballots side by side
+    const uint32_t part = max((hi - lo) >> 2, 1u);
+    const uint32_t at1 = lo + part, at2 = min(at1, hi - part) + part, at3 = min(at2, hi - part) + part;
+    const int reach1 = __popcll(__ballot(head >= at1)), reach2 = __popcll(__ballot(head >= at2)), reach3 = __popcll(__ballot(head >= at3));
+    const bool over1 = reach1 >= k, over2 = reach2 >= k, over3 = reach3 >= k;
+    const int reach = over3 ? reach3 : over2 ? reach2 : over1 ? reach1 : 64;
+    hi = over3 ? hi : over2 ? at3 : over1 ? at2 : at1;
+    lo = over3 ? at3 : over2 ? at2 : over1 ? at1 : lo;
+    if (reach <= k + TOP_SLACK) break;
+  }
+  int count = 0;
+#pragma unroll
+  for (int j = 0; j < PER; j++) count += key[j] >= lo ? 1 : 0;
+  const int upto = wave_inclusive_sum(count), all = __builtin_amdgcn_readlane(upto, 63);
+  out_key = 0u;
+  out_tag = 0;
+  if (all <= 63) {  // uniform; (all >= k, or every key there is)
+    int at = upto - count;
+    uint32_t mine = 0u;
+    int tag = 0;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {  // lane 63 takes what goes nowhere; a lane that nothing is sent to gets zero
+      const bool take = key[j] >= lo;
+      const int to = 4 * (take ? at : 63);
+      mine |= (uint32_t)__builtin_amdgcn_ds_permute(to, (int)key[j]);
+      tag |= __builtin_amdgcn_ds_permute(to, lane * per + j);
+      at += take ? 1 : 0;
+    }
+    if (lane >= all) mine = 0u;
+    auto deal = [&](bool ties) {
+      int rank = 0;
+      for (int c0 = 0; c0 < all; c0 += 4) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+          const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, min(c0 + c, 63));
+          rank += other > mine ? 1 : 0;
+          if (ties) rank += other == mine && c0 + c < lane ? 1 : 0;
+        }
+      }
+      const int to = 4 * (lane < all && rank < k ? rank : 63);
+      out_key = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)mine);
+      out_tag = __builtin_amdgcn_ds_permute(to, tag);
+      return __popcll(__ballot(lane < all && rank < k)) == __popcll(__ballot(lane < k && out_key != 0u));  // a rank for every key, a key for every rank
+    };
+    if (!deal(false)) deal(true);  // equal keys had one rank between them
+    if (lane >= k) out_key = 0u, out_tag = 0;
+    return;
+  }
+  for (int s = 0; s < k; s++) {
+    uint32_t best = 0;
+    int at = 0;
+#pragma unroll
+    for (int j = 0; j < PER; j++)
+      if (key[j] > best) {  // ascending index within the lane: the first of equals stays
+        best = key[j];
+        at = j;
+      }
+    const uint32_t top = wave_max_u32(best);
+    const int winner = __builtin_ctzll(__ballot(best == top));
+    const int wj = __builtin_amdgcn_readlane(at, winner);
+    if (lane == s) {
+      out_key = top;
+      out_tag = winner * per + wj;
+    }
+    if (lane == winner) {
+#pragma unroll
+      for (int j = 0; j < PER; j++)
+        if (j == wj) key[j] = 0u;
+    }
+  }
 }
 
 struct RouteParams {
@@ -124,8 +231,7 @@ __device__ __forceinline__ int route_row(const RouteParams& p, int r, int lane, 
       val[j] = j < per && first + j < e ? lg[j] : -INFINITY;
       mx = fmaxf(mx, val[j]);
     }
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) mx = fmaxf(mx, __shfl_xor(mx, d));
+    mx = wave_max(mx);
     float sum = 0.f;
 #pragma unroll
     for (int j = 0; j < PER; j++) {
@@ -140,82 +246,18 @@ __device__ __forceinline__ int route_row(const RouteParams& p, int r, int lane, 
     }
   }
   float total = 0.f, mine = 0.f;
-  int mine_id = 0;
-  if constexpr (PER == 8) {
-    // The lane's registers in descending order once (adjacent exchanges on a strictly larger right neighbour only, so
-    // equal keys keep ascending index), their indices as nibbles of one register: a round is then the wave-wide
-    // maximum of the heads and the winner's list moving up by one.
-    uint32_t at[PER];
-#pragma unroll
-    for (int j = 0; j < PER; j++) at[j] = j;
-#pragma unroll
-    for (int pass = 0; pass < PER; pass++) {
-#pragma unroll
-      for (int j = pass & 1; j + 1 < PER; j += 2) {
-        const bool swap = key[j + 1] > key[j];
-        const uint32_t ka = key[j], kb = key[j + 1], ia = at[j], ib = at[j + 1];
-        key[j] = swap ? kb : ka;
-        key[j + 1] = swap ? ka : kb;
-        at[j] = swap ? ib : ia;
-        at[j + 1] = swap ? ia : ib;
-      }
-    }
-    uint32_t order = 0;
-#pragma unroll
-    for (int j = 0; j < PER; j++) order |= at[j] << (4 * j);
-    uint32_t mine_key = 0;
-    for (int s = 0; s < p.k; s++) {
-      const uint32_t top = wave_max_u32(key[0]);
-      const int winner = __builtin_ctzll(__ballot(key[0] == top));
-      const int wj = __builtin_amdgcn_readlane((int)order, winner) & 15;
-      if (lane == s) {
-        mine_key = top;
-        mine_id = winner * per + wj;
-      }
-      if (lane == winner) {
-#pragma unroll
-        for (int j = 0; j + 1 < PER; j++) key[j] = key[j + 1];
-        key[PER - 1] = 0u;
-        order >>= 4;
-      }
-    }
-    if (lane < p.k) {
-      if (SIGMOID) {  // the key is score + bias: the plain score is made again from the logit
-        mine = 1.0f / (1.0f + expf(-logit(row + mine_id)));
-      } else {        // the key is the probability's own bits
-        const uint32_t u = mine_key ^ 0x80000000u;
-        mine = __builtin_bit_cast(float, u ^ (uint32_t)(((int32_t)u >> 31) & 0x7fffffff));
-      }
-    }
-    for (int s = 0; s < p.k; s++) total += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine), s));  // in rank order
-  } else {
-    for (int s = 0; s < p.k; s++) {
-      uint32_t best = 0;
-      int at = 0;
-      float bv = 0.f;
-#pragma unroll
-      for (int j = 0; j < PER; j++)
-        if (key[j] > best) {  // ascending index within the lane: the first of equals stays
-          best = key[j];
-          at = j;
-          bv = val[j];
-        }
-      const uint32_t top = wave_max_u32(best);
-      const int winner = __builtin_ctzll(__ballot(best == top));
-      const int wj = __builtin_amdgcn_readlane(at, winner);
-      const float wv = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, bv), winner));
-      total += wv;
-      if (lane == s) {
-        mine = wv;
-        mine_id = winner * per + wj;
-      }
-      if (lane == winner) {
-#pragma unroll
-        for (int j = 0; j < PER; j++)
-          if (j == wj) key[j] = 0u;
-      }
+  int mine_id;
+  uint32_t mine_key;
+  top_ranked(key, per, p.k, lane, mine_key, mine_id);
+  if (lane < p.k) {
+    if (SIGMOID) {  // the key is score + bias: the plain score is made again from the logit
+      mine = 1.0f / (1.0f + expf(-logit(row + mine_id)));
+    } else {        // the key is the probability's own bits
+      const uint32_t u = mine_key ^ 0x80000000u;
+      mine = __builtin_bit_cast(float, u ^ (uint32_t)(((int32_t)u >> 31) & 0x7fffffff));
     }
   }
+  for (int s = 0; s < p.k; s++) total += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, mine), s));  // in rank order
   int id = mine_id;
   float w = SIGMOID ? mine / (total + 1e-20f) : mine / total;
   if (padded) {

@@ -66,39 +66,19 @@ __device__ __forceinline__ void rank_row(const BudgetParams& q, int t, int lane)
     key[j] = col < e ? (bf16_order(h) << 16) | (uint32_t)(0xffff - col) : 0u;
     val[j] = col < e ? __uint_as_float(h << 16) : -INFINITY;
   }
-  // the lane's keys in descending order once: a round is the wave-wide maximum of the heads, and the winner's list
-  // moves up by one
+  uint32_t head = key[0];
 #pragma unroll
-  for (int pass = 0; pass < PER; pass++) {
+  for (int j = 1; j < PER; j++) head = max(head, key[j]);
+  const float mx = bf16_order_value(wave_max_u32(head) >> 16);  // the row's maximum: the softmax denominator over all experts
+  float sum = 0.f;
 #pragma unroll
-    for (int j = pass & 1; j + 1 < PER; j += 2) {
-      const uint32_t hi = max(key[j], key[j + 1]), lo = min(key[j], key[j + 1]);
-      key[j] = hi;
-      key[j + 1] = lo;
-    }
-  }
-  float mx = -INFINITY, sum = 0.f, mine_v = 0.f;
-  int mine_id = 0;
-  for (int c = 0; c < BUDGET_CANDIDATES; c++) {
-    const uint32_t top = wave_max_u32(key[0]);
-    const int col = 0xffff - (int)(top & 0xffffu);
-    const float v = bf16_order_value(top >> 16);
-    if (c == 0) {  // the row's maximum: the softmax denominator over all experts
-      mx = v;
-#pragma unroll
-      for (int j = 0; j < PER; j++) sum += j * 64 + lane < e ? expf(val[j] - mx) : 0.f;
-      sum = wave_sum(sum);
-    }
-    if (lane == c) {
-      mine_v = v;
-      mine_id = col;
-    }
-    if (lane == (col & 63)) {
-#pragma unroll
-      for (int j = 0; j + 1 < PER; j++) key[j] = key[j + 1];
-      key[PER - 1] = 0u;
-    }
-  }
+  for (int j = 0; j < PER; j++) sum += j * 64 + lane < e ? expf(val[j] - mx) : 0.f;
+  sum = wave_sum(sum);
+  uint32_t mine_key;
+  int place;
+  top_ranked(key, PER, BUDGET_CANDIDATES, lane, mine_key, place);
+  const int mine_id = 0xffff - (int)(mine_key & 0xffffu);
+  const float mine_v = bf16_order_value(mine_key >> 16);
   const float mine = expf(mine_v - mx) / sum;
   if (lane < BUDGET_CANDIDATES) {
     const int64_t at = (int64_t)t * BUDGET_CANDIDATES + lane;
@@ -118,7 +98,7 @@ __global__ __launch_bounds__(64) void route_rank_kernel(BudgetParams q) {
 
 // One workgroup (BUDGET_THREADS threads; `copies`: copies_n * e floats of its dynamic LDS). Scores: wavefront w adds the rows t = w (mod copies) into a copy of its own, in row order, and the
 // copies are added in wavefront order (the same bits on every run). The set: wavefront 0 holds every expert's key in
-// registers (column j * 64 + lane, as above) and finds the need-th largest by bisection on its bits, each step one
+// registers (column j * 64 + lane, as above) and finds the need-th largest by bisection, each step one
 // ballot a register. The rows: two a wavefront at a time, one in each half. IN_ORDER: a row's weights are divided by
 // the sum of the taken ones added in rank order, as the routing kernel adds a row's top k (a row that keeps all of its
 // top k gets that kernel's weights bit for bit); otherwise by a butterfly sum.
@@ -219,16 +199,20 @@ __device__ __forceinline__ void budget_pick(const BudgetParams& q, int copies_n,
     if (need > 0 && contenders <= need) {
       at = 0u;
     } else if (need > 0) {
-      // the need-th largest key: the largest value that `need` keys reach, a bit at a time from the top; a value that
-      // exactly `need` keys reach ends the search (the keys at or above it are the answer)
+      // the need-th largest key: the largest value that `need` keys reach, by bisection from within a factor 2^16 of the largest
+      // key where that many lie there; a value that exactly `need` keys reach ends the search (the keys at or above it are the answer)
+      uint32_t most = kk[0];
+#pragma unroll
+      for (int j = 1; j < PER; j++) most = max(most, kk[j]);
+      uint32_t over = wave_max_u32(most) + 1u, trial = over > (16u << 23) ? over - (16u << 23) : 1u;
       at = 0u;
-      for (int bit = 30; bit >= 0; bit--) {
-        const uint32_t trial = at | (1u << bit);
+      while (over - at > 1u) {
         int n = 0;
 #pragma unroll
         for (int j = 0; j < PER; j++) n += __popcll(__ballot(kk[j] >= trial));
-        if (n >= need) at = trial;
+        if (n >= need) at = trial; else over = trial;
         if (n == need) break;
+        trial = at + ((over - at) >> 1);
       }
       // `at` may now lie below the need-th largest key, between it and the next one: nothing equals it then
       int above = 0;
@@ -271,8 +255,7 @@ __device__ __forceinline__ void budget_pick(const BudgetParams& q, int copies_n,
           }
         total = half ? upper : lower;
       } else {
-#pragma unroll
-        for (int d = 16; d >= 1; d >>= 1) total += __shfl_xor(total, d);  // stays within the half
+        total = half_wave_sum(total);
       }
       total += q.eps;
       const int used = real ? min(__popc(mask), q.k) : 0;

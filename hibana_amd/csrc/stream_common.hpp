@@ -174,6 +174,25 @@ __device__ __forceinline__ void store_out(const StreamParams& p, const Slot& sl,
   }
 }
 
+// A value's sum over the wavefront's lanes (over each half of them), in every lane: the additions of the butterfly that adds lane ^ 32,
+// then ^ 16, ... ^ 1, so its bits, without its six trips through the LDS (120 cycles each): two lane swaps and, as behind
+// the exchange at distance 2 d the values repeat every 2 d lanes, rotations within rows of sixteen for ^ 8 ... ^ 1.
+__device__ __forceinline__ float rotations_sum(float x) {
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x128, 0xF, 0xF, false));
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x124, 0xF, 0xF, false));
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x122, 0xF, 0xF, false));
+  x += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x121, 0xF, 0xF, false));
+  return x;
+}
+__device__ __forceinline__ float half_wave_sum(float x) {
+  const auto rows = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
+  return rotations_sum(__uint_as_float(rows[0]) + __uint_as_float(rows[1]));
+}
+__device__ __forceinline__ float wave_sum(float x) {
+  const auto halves = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, x), false, false);
+  return half_wave_sum(__uint_as_float(halves[0]) + __uint_as_float(halves[1]));
+}
+
 // The largest of a value over the sixteen lanes of a DPP row, in each of them. Lanes that are switched off
 // contribute 0 (the values are magnitudes).
 __device__ __forceinline__ float row16_max(float x) {
@@ -628,8 +647,7 @@ __device__ __forceinline__ void combine_gate_partial(const uint16_t* x, const fl
     for (int j = 0; j < 8; j++)
       if (i0 + 256 * j < hx) dot += xv[j] * gv[j];
   }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) dot += __shfl_xor(dot, d);
+  dot = wave_sum(dot);
   if ((t & 63) == 0) red[t >> 6] = dot;
 }
 __device__ __forceinline__ float combine_gate_value(const float* red) {

@@ -1,0 +1,53 @@
+"""The selection of a row's top k from one wavefront's registers: the forms that its threshold does not separate from one
+another - equal scores inside the selection and across its end, all scores equal, the best experts side by side in a few lanes
+(more than 63 keys at the threshold) - and expert counts that leave registers and lanes empty."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rows(kind, e, g):
+    m = 24
+    x = torch.randn(m, e, generator=g)
+    if kind == "coarse":      # many equal scores, some of them across the selection's end
+        return (x * 2).round() / 2
+    if kind == "equal":
+        return torch.zeros(m, e)
+    if kind == "clustered":   # the best experts next to one another
+        return x * 0.01 - (torch.arange(e) - e // 3).abs() * 0.05
+    if kind == "pairs":       # every score twice, in lanes far apart
+        half = x[:, :(e + 1) // 2]
+        return torch.cat([half, half], 1)[:, :e]
+    if kind == "wide":        # probabilities over the whole range of the type
+        return x * 40
+    return x
+
+
+@pytest.mark.parametrize("kind", ["plain", "coarse", "equal", "clustered", "pairs", "wide"])
+@pytest.mark.parametrize("e,k", [(8, 8), (40, 30), (64, 12), (100, 60), (130, 7), (512, 10), (512, 22), (512, 62), (512, 64), (700, 12), (1024, 40)])
+def test_softmax_and_sigmoid_rows(kind, e, k):
+    from hibana_amd.kernels import ops
+    from hibana_amd.model import nemotron_moe
+    g = torch.Generator().manual_seed(e * 64 + k)
+    logits = _rows(kind, e, g).float().cuda()
+    # the rule on the scores the device computed: descending, equal ones to the lower expert
+    ids, weights = ops.route_topk(logits, k)
+    prob = torch.softmax(logits.double(), -1)
+    order = torch.argsort(prob, dim=-1, descending=True, stable=True)[:, :k]
+    same = ids.long() == order
+    assert bool((same | ((prob.gather(1, ids.long()) - prob.gather(1, order)).abs() <= 1e-6 * prob.gather(1, order) + 1e-37)).all())
+    if kind in ("coarse", "equal", "pairs"):  # equal logits are equal scores, bit for bit
+        assert torch.equal(ids.long(), torch.argsort(logits, dim=-1, descending=True, stable=True)[:, :k])
+    want = prob.gather(1, ids.long())
+    assert torch.allclose(weights.double(), want / want.sum(-1, keepdim=True), rtol=1e-5, atol=1e-30)
+    bias = torch.zeros(e, device="cuda")
+    ids, weights, _ = nemotron_moe.route_topk(torch.cat([logits, logits[:, :1]], 1), bias, k, 1)
+    score = torch.sigmoid(logits.double())
+    assert all(len(set(row)) == k for row in ids.tolist())
+    picked = score.gather(1, ids.long())
+    assert bool((picked[:, :-1] >= picked[:, 1:] - 1e-6).all())
+    assert bool((picked[:, -1:] >= torch.topk(score, k, -1)[0][:, -1:] - 1e-6).all())
+    if kind in ("coarse", "equal", "pairs"):
+        assert torch.equal(ids.long(), torch.argsort(logits, dim=-1, descending=True, stable=True)[:, :k])
+    assert torch.allclose(weights.double(), picked / (picked.sum(-1, keepdim=True) + 1e-20), rtol=1e-5)

@@ -774,8 +774,8 @@ __global__ __launch_bounds__(256) void moe_combine_kernel(CombineParams p) {
 
 // A long call's sum of BF16 pairs alone: sixteen bytes of a pair a thread and load instead of four. combine_span's chain, operation
 // for operation: the same bits. Bound by the pairs' traffic (5 TB/s). Measured alone, before and now: 1024 rows of 22 pairs, 1024
-// columns, 12.7 and 10.8 us, 2048 rows 24.6 and 19.2. (With the shared expert's gate, whose dot product is half a row's loads,
-// it was no faster; FP32 pairs took 41.6 us instead of 31.1 at 1543 rows of 10, 2048 columns.)
+// columns, 12.7 and 10.8 us, 2048 rows 24.6 and 19.2; with the ids and weights asked for ahead of the pairs 9.0 and 15.7. (A row's ids
+// and weights one at a time, behind its pairs, were a trip to memory each.)
 template <int B>
 __global__ __launch_bounds__(256) void moe_combine_wide_kernel(CombineParams p) {
   const int r = blockIdx.x, c = (blockIdx.y * blockDim.x + threadIdx.x) * 8;
@@ -785,22 +785,91 @@ __global__ __launch_bounds__(256) void moe_combine_wide_kernel(CombineParams p) 
 #pragma unroll
   for (int i = 0; i < 8; i++) v[i] = 0.f;
   for (int s0 = 0; s0 < p.topk; s0 += B) {
+    int e[B];
+    float w[B];
     u32x4_t y[B];
+#pragma unroll
+    for (int j = 0; j < B; j++) {  // all asked for together
+      e[j] = p.ids[r * p.topk + min(s0 + j, p.topk - 1)];
+      w[j] = p.weights[r * p.topk + min(s0 + j, p.topk - 1)];
+    }
 #pragma unroll
     for (int j = 0; j < B; j++) y[j] = *reinterpret_cast<const u32x4_t*>(at + (int64_t)min(s0 + j, p.topk - 1) * p.h);
 #pragma unroll
     for (int j = 0; j < B; j++) {
-      const int s = min(s0 + j, p.topk - 1), local = p.ids[r * p.topk + s] - p.e_lo;
+      const int local = e[j] - p.e_lo;
       const bool keep = s0 + j < p.topk && local >= 0 && local < p.e_n;
-      const float w = keep ? p.weights[r * p.topk + s] : 0.f;
+      const float weight = keep ? w[j] : 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; i++) v[i] = fmaf(w, keep ? (i & 1 ? pair_hi(y[j][i >> 1]) : pair_lo(y[j][i >> 1])) : 0.f, v[i]);
+      for (int i = 0; i < 8; i++) v[i] = fmaf(weight, keep ? (i & 1 ? pair_hi(y[j][i >> 1]) : pair_lo(y[j][i >> 1])) : 0.f, v[i]);
     }
   }
   u32x4_t out;
 #pragma unroll
   for (int i = 0; i < 8; i += 2) out[i / 2] = (uint32_t)f32_to_bf16_bits(v[i]) | ((uint32_t)f32_to_bf16_bits(v[i + 1]) << 16);
   *reinterpret_cast<u32x4_t*>(p.out + (int64_t)r * p.h + c) = out;
+}
+
+constexpr int64_t COMBINE_ROW_VALUES = 1 << 20;
+// A row a workgroup, sixteen bytes of a pair a thread and load, the gate's dot product once a row: combine_span's chain and dot
+// product, operation for operation: the same bits. There every span of 512 columns makes the dot product again, whose loads (12 KB
+// at 2048 columns) are as many as the span's own. Measured alone, rows of ten
+// pairs, 2048 columns, in spans and so, us: BF16 1024 rows 17.4 and 11.2, 1543 rows 24.2 and 15.6, 2048 rows 30.6 and 19.1; FP32 256 rows 7.4 and 8.2,
+// 512 rows 12.2 and 10.8, 1000 rows 19.4 and 17.0; 500 rows of six, 1280 columns, 6.8 and 7.9.
+template <int B, bool BF16>
+__global__ __launch_bounds__(256) void moe_combine_row_kernel(CombineParams p) {
+  constexpr int V = BF16 ? 8 : 4;  // columns a load
+  __shared__ float red[4];
+  const int r = blockIdx.x;
+  const uint8_t* pairs = static_cast<const uint8_t*>(p.pairs) + (int64_t)r * p.topk * p.h * (BF16 ? 2 : 4);
+  const uint8_t* shared = static_cast<const uint8_t*>(p.shared) + (int64_t)r * p.shared_stride * (BF16 ? 2 : 4);
+  float g = 1.0f;
+  for (int c0 = 0; c0 < p.h; c0 += 256 * V) {
+    const int c = c0 + V * threadIdx.x;
+    const bool in = c < p.h;  // h is a multiple of 8
+    const int at = in ? c * (BF16 ? 2 : 4) : 0;
+    float v[V];
+#pragma unroll
+    for (int i = 0; i < V; i++) v[i] = 0.f;
+    const u32x4_t sh = *reinterpret_cast<const u32x4_t*>(shared + at);
+    for (int s0 = 0; s0 < p.topk; s0 += B) {
+      int e[B];
+      float w[B];
+      u32x4_t y[B];
+#pragma unroll
+      for (int j = 0; j < B; j++) {
+        e[j] = p.ids[r * p.topk + min(s0 + j, p.topk - 1)];
+        w[j] = p.weights[r * p.topk + min(s0 + j, p.topk - 1)];
+      }
+#pragma unroll
+      for (int j = 0; j < B; j++) y[j] = *reinterpret_cast<const u32x4_t*>(pairs + (int64_t)min(s0 + j, p.topk - 1) * p.h * (BF16 ? 2 : 4) + at);
+      if (c0 == 0 && s0 == 0 && p.gate_vec) {  // uniform; behind the first loads, so that everything is on its way together
+        combine_gate_partial(p.x, p.gate_vec, p.hx, r, threadIdx.x, red);
+        __syncthreads();
+        g = combine_gate_value(red);
+      }
+#pragma unroll
+      for (int j = 0; j < B; j++) {
+        const int local = e[j] - p.e_lo;
+        const bool keep = s0 + j < p.topk && local >= 0 && local < p.e_n;
+        const float weight = keep ? w[j] : 0.f;
+#pragma unroll
+        for (int i = 0; i < V; i++) v[i] = fmaf(weight, !keep ? 0.f : !BF16 ? __uint_as_float(y[j][i & 3]) : i & 1 ? pair_hi(y[j][i >> 1]) : pair_lo(y[j][i >> 1]), v[i]);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < V; i++) v[i] = combine_shared(v[i], g, !BF16 ? __uint_as_float(sh[i & 3]) : i & 1 ? pair_hi(sh[i >> 1]) : pair_lo(sh[i >> 1]));
+    uint32_t out[V / 2];
+#pragma unroll
+    for (int i = 0; i < V; i += 2) out[i / 2] = (uint32_t)f32_to_bf16_bits(v[i]) | ((uint32_t)f32_to_bf16_bits(v[i + 1]) << 16);
+    if (in) {
+      if constexpr (BF16) {
+        *reinterpret_cast<u32x4_t*>(p.out + (int64_t)r * p.h + c) = u32x4_t{out[0], out[1], out[2], out[3]};
+      } else {
+        *reinterpret_cast<uint2*>(p.out + (int64_t)r * p.h + c) = make_uint2(out[0], out[1]);
+      }
+    }
+  }
 }
 
 // ------------------------------------------------------------------ the latent block's BF16 projections (M <= 16)
@@ -1247,6 +1316,17 @@ void moe_launch_combine(const CombineParams& c, hipStream_t stream) {
   if (c.pairs_bf16 && !c.shared && c.m >= MOE_WIDE_ROWS && c.h % 8 == 0 && aligned(c.pairs, 16) && aligned(c.out, 16)) {
     const int threads = std::min(256, (c.h / 8 + 63) / 64 * 64);
     HB_LAUNCH(moe_combine_wide_kernel<12>, dim3((unsigned)c.m, (unsigned)((c.h / 8 + threads - 1) / threads)), dim3((unsigned)threads), 0, stream, c);
+    return;
+  }
+  // ... and with a shared expert a row a workgroup, FP32 pairs from the size where the dot products' loads, not one workgroup's
+  // trips to memory, are what takes time
+  if (c.shared && (c.pairs_bf16 ? c.m >= MOE_WIDE_ROWS : (int64_t)c.m * c.h >= COMBINE_ROW_VALUES) && c.h % 8 == 0 && c.shared_stride % 8 == 0 && (c.pairs_bf16 != 0) == (c.shared_f32 == 0) &&
+      aligned(c.pairs, 16) && aligned(c.shared, 16) && aligned(c.out, 16)) {
+    if (c.pairs_bf16) {
+      HB_LAUNCH((moe_combine_row_kernel<12, true>), dim3((unsigned)c.m), dim3(256), 0, stream, c);
+    } else {
+      HB_LAUNCH((moe_combine_row_kernel<12, false>), dim3((unsigned)c.m), dim3(256), 0, stream, c);
+    }
     return;
   }
   const dim3 grid((unsigned)c.m, (unsigned)((c.h + COMBINE_SPAN - 1) / COMBINE_SPAN));

@@ -47,11 +47,13 @@ def silu_and_mul(gate_up: torch.Tensor, pairs: int = 0) -> torch.Tensor:
         raise ValueError("silu_and_mul: BF16 [..., 2 * half], half even (and a multiple of an even `pairs`)")
     _lib.need_gpu(gate_up)
     half = gate_up.shape[-1] // 2
-    flat = gate_up.reshape(-1, 2 * half).contiguous()
-    out = torch.empty((flat.shape[0], half), dtype=torch.bfloat16, device=gate_up.device)
+    flat = (gate_up if gate_up.ndim == 2 else gate_up.reshape(-1, 2 * half)).contiguous()
+    out = flat.new_empty((flat.shape[0], half))
     if flat.shape[0]:
-        _lib.check(_lib.lib().hb_silu_and_mul(_lib.ptr(flat), flat.shape[0], half, pairs, _lib.ptr(out), _lib.stream()), "silu_and_mul")
-    return out.reshape(*gate_up.shape[:-1], half)
+        code = _lib.lib().hb_silu_and_mul(flat.data_ptr(), flat.shape[0], half, pairs, out.data_ptr(), _lib.stream())
+        if code:
+            _lib.check(code, "silu_and_mul")
+    return out if gate_up.ndim == 2 else out.reshape(*gate_up.shape[:-1], half)
 
 
 def silu_mul(gate_up: torch.Tensor, pairs: int = 0) -> torch.Tensor:
@@ -86,8 +88,9 @@ def silu_mul_quant_groups(gate_up: torch.Tensor, pairs: int = 0, torch_chain: bo
     q = gu.new_empty((m, half), dtype=torch.float8_e4m3fn)
     scales = gu.new_empty((m, half // 32), dtype=torch.float32)
     if m:
-        _lib.check(_lib.lib().hb_silu_mul_quant_groups(_lib.ptr(gu), m, half, pairs, int(torch_chain), _lib.ptr(q), _lib.ptr(scales), _lib.stream()),
-                   "silu_mul_quant_groups")
+        code = _lib.lib().hb_silu_mul_quant_groups(gu.data_ptr(), m, half, pairs, int(torch_chain), q.data_ptr(), scales.data_ptr(), _lib.stream())
+        if code:
+            _lib.check(code, "silu_mul_quant_groups")
     return q, scales
 
 

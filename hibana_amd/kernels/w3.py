@@ -353,8 +353,10 @@ def w3_linear(x: torch.Tensor, w3: W3Weight, x_scale: torch.Tensor | None = None
             raise ValueError("w3_linear: x_scale must have 1, M or M * K/32 elements")
         scale = x_scale if x_scale.dtype == torch.float32 and x_scale.shape == (m, groups) and x_scale.is_contiguous() else \
             x_scale.float().reshape(-1, groups if x_scale.numel() == m * groups else 1).expand(m, groups).contiguous()
-        _lib.check(_lib.lib().hb_w3_gemm_e4m3(_lib.ptr(x), _lib.ptr(scale), m, _lib.ptr(w3.tiled), _lib.ptr(w3.row_scale), w3.lut,
-                                              w3.out_features, k, w3.tile_bits, _lib.ptr(y), _lib.stream()), "w3_linear")
+        code = _lib.lib().hb_w3_gemm_e4m3(x.data_ptr(), scale.data_ptr(), m, w3.tiled.data_ptr(), w3.row_scale.data_ptr(), w3.lut, w3.out_features, k,
+                                          w3.tile_bits, y.data_ptr(), _lib.stream())
+        if code:
+            _lib.check(code, "w3_linear")
         return y
     code = _lib.lib().hb_w3_gemm(x.data_ptr(), m, w3.tiled.data_ptr(), w3.row_scale.data_ptr(), w3.lut, w3.out_features, k, w3.tile_bits, y.data_ptr(),
                                  _lib.stream())

@@ -198,6 +198,6 @@ class NemotronMoe:
         routed = self.routed(latent, ids, weights)
         if self.shared_up is None:
             return torch.mm(routed, self.fc2.T)
-        return torch.addmm(self.shared(x), routed, self.fc2.T)
+        return self.shared(x).addmm_(routed, self.fc2.T)  # in place: out of place torch copies the shared part first, a launch of its own
 
     __call__ = forward

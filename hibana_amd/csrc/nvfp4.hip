@@ -178,6 +178,47 @@ struct Fp4RingOf {
   }
 };
 typedef Fp4RingOf<1> Fp4Ring;
+// A ring that brings in only the codes of the 16-row tiles T0 .. T1 - 1 (a load a tile) and the scales. The Chunk's other
+// registers stay unset and unread.
+template <int U, int T0, int T1>
+struct Fp4RingPart : Fp4RingOf<U> {
+  typedef Fp4Chunk Chunk;
+  static constexpr int TILES = T1 - T0, LOADS = TILES + 2;
+  static_assert(0 <= T0 && T1 <= 4 && (TILES == 1 || TILES == 2), "a tile or a pair of tiles");
+  static __device__ __forceinline__ void request(const RingSource& src, int chunk, lds_ptr_t slot) {
+    const uint32_t at = (uint32_t)chunk * NVFP4_BLOCK_BYTES;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src.row, slot, 16, src.codes, at, 1024 * T0, 2);
+    if (TILES == 2) __builtin_amdgcn_raw_ptr_buffer_load_lds(src.row, slot, 16, src.codes, at, 1024 * (T1 - 1), 2);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src.row, slot + NVFP4_SCALE_OFFSET, 4, src.scales, at + NVFP4_SCALE_OFFSET, 0, 2);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(src.row, slot + NVFP4_SCALE_OFFSET, 4, src.scales, at + NVFP4_SCALE_OFFSET, 256, 2);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  static __device__ __forceinline__ u32x4_t& load_of(Chunk& ch, int t) { return t == 0 ? ch.w0 : t == 1 ? ch.w1 : t == 2 ? ch.w2 : ch.w3; }
+  template <int BEHIND, int SLOT>
+  static __device__ __forceinline__ void take(Chunk& ch, uint32_t codes, uint32_t scales) {
+    if (TILES == 2) {
+      asm volatile(
+          "s_waitcnt vmcnt(%5)\n\t"
+          "ds_read_b128 %0, %3 offset:%6\n\t"
+          "ds_read_b128 %1, %3 offset:%7\n\t"
+          "ds_read_b128 %2, %4 offset:%8\n\t"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&v"(load_of(ch, T0)), "=&v"(load_of(ch, T1 - 1)), "=&v"(ch.sc)
+          : "v"(codes), "v"(scales), "n"(BEHIND), "n"(SLOT * NVFP4_BLOCK_BYTES + 1024 * T0), "n"(SLOT * NVFP4_BLOCK_BYTES + 1024 * (T1 - 1)),
+            "n"(SLOT * NVFP4_BLOCK_BYTES + NVFP4_SCALE_OFFSET)
+          : "memory");
+    } else {
+      asm volatile(
+          "s_waitcnt vmcnt(%4)\n\t"
+          "ds_read_b128 %0, %2 offset:%5\n\t"
+          "ds_read_b128 %1, %3 offset:%6\n\t"
+          "s_waitcnt lgkmcnt(0)"
+          : "=&v"(load_of(ch, T0)), "=&v"(ch.sc)
+          : "v"(codes), "v"(scales), "n"(BEHIND), "n"(SLOT * NVFP4_BLOCK_BYTES + 1024 * T0), "n"(SLOT * NVFP4_BLOCK_BYTES + NVFP4_SCALE_OFFSET)
+          : "memory");
+    }
+  }
+};
 constexpr int FP4_RING_BYTES = ring_bytes<Fp4Ring>();  // LDS per wavefront; its first 4 KB double as the K-split exchange
 
 // ---------------------------------------------------------------------------------------- slots of one to eight rows
@@ -203,6 +244,7 @@ constexpr int FP4_FEW_ROWS = 8, FP4_FEWER_ROWS = 4;
 // half of the activations' way through the L1 (eight rows, 25600 x 5120: 17.1 us, with the selects 19.3).
 __device__ const u32x4_t fp4_zero_piece[16] = {};
 
+template <int T0 = 0, int T1 = 4>  // the 16-row tiles T0 .. T1 - 1 of the block (the other accumulators stay zero)
 struct Fp4Few8Acts {
   static constexpr int LOADS = 4;
   u32x4_t even[4], odd[4];  // the lane's piece of each step of the next even and the next odd chunk
@@ -235,19 +277,20 @@ struct Fp4Few8Acts {
   template <int ODD, bool MORE2, bool MORE1>
   __device__ __forceinline__ void step(const Fp4Chunk& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot&) {
     const u32x4_t(&a)[4] = ODD ? odd : even;
-    tile(ch.w0, ch.sc.x, a, acc0);
+    if (T0 <= 0 && 0 < T1) tile(ch.w0, ch.sc.x, a, acc0);
     __builtin_amdgcn_sched_barrier(0);  // a tile at a time: interleaving the four costs more registers than there are
-    tile(ch.w1, ch.sc.y, a, acc1);
+    if (T0 <= 1 && 1 < T1) tile(ch.w1, ch.sc.y, a, acc1);
     __builtin_amdgcn_sched_barrier(0);
-    tile(ch.w2, ch.sc.z, a, acc2);
+    if (T0 <= 2 && 2 < T1) tile(ch.w2, ch.sc.z, a, acc2);
     __builtin_amdgcn_sched_barrier(0);
-    tile(ch.w3, ch.sc.w, a, acc3);
+    if (T0 <= 3 && 3 < T1) tile(ch.w3, ch.sc.w, a, acc3);
     if (MORE2) {
       if (ODD) load(odd, i + 2); else load(even, i + 2);
     }
   }
 };
 
+template <int T0 = 0, int T1 = 4>
 struct Fp4Few4Acts {
   static constexpr int LOADS = 2;
   u32x4_t even[2], odd[2];  // the lane's piece of the pairs of steps of the next even and the next odd chunk
@@ -284,10 +327,10 @@ struct Fp4Few4Acts {
       a[2 * t] = masked(ODD ? odd[t] : even[t], first);
       a[2 * t + 1] = masked(ODD ? odd[t] : even[t], second);
     }
-    tile(ch.w0, ch.sc.x, a, acc0);
-    tile(ch.w1, ch.sc.y, a, acc1);
-    tile(ch.w2, ch.sc.z, a, acc2);
-    tile(ch.w3, ch.sc.w, a, acc3);
+    if (T0 <= 0 && 0 < T1) tile(ch.w0, ch.sc.x, a, acc0);
+    if (T0 <= 1 && 1 < T1) tile(ch.w1, ch.sc.y, a, acc1);
+    if (T0 <= 2 && 2 < T1) tile(ch.w2, ch.sc.z, a, acc2);
+    if (T0 <= 3 && 3 < T1) tile(ch.w3, ch.sc.w, a, acc3);
     if (MORE2) {
       if (ODD) load(odd, i + 2); else load(even, i + 2);
     }
@@ -312,8 +355,9 @@ __device__ __forceinline__ void add_lanes(f32x4_t& acc, int distance) {
 // The body serves matrices past 4 GiB too, which the panel kernel does not take: a lane's 32-bit byte offset counts from the
 // slot's first row (a uniform base: 2048 x 2048 at nine rows 8.6 us against 9.0 with a pointer a lane), and where the
 // slot's rows are gathered, which may lie anywhere, the lane holds a whole pointer.
-template <int EPI>
+template <int EPI, int T0 = 0, int T1 = 4, class Ring = Fp4Ring>  // the 16-row tiles T0 .. T1 - 1 of the block
 struct Fp4Full {
+  static constexpr int TILES = T1 - T0;
   f32x4_t acc[4];
   u32x4_t a[4];
   const uint8_t* x;  // step 0 of the wavefront's first chunk: of the slot's first row (the same for all lanes) or, gathered, the lane's own piece ...
@@ -333,26 +377,29 @@ struct Fp4Full {
 #pragma unroll
     for (int s = 0; s < 4; s++) a[s] = piece(0, s);
   }
-  template <int J>  // fragment J = 4 * step + tile of a chunk
-  static __device__ __forceinline__ bf16x8_t fragment(const Fp4Chunk& ch) { return fp4_scaled(ch.tile(J & 3)[J >> 2], fp4_scale<(J >> 2)>(ch.sc[J & 3])); }
+  template <int J>  // fragment J = TILES * step + tile - T0 of a chunk
+  static __device__ __forceinline__ bf16x8_t fragment(const Fp4Chunk& ch) {
+    constexpr int S = J / TILES, NT = T0 + J % TILES;
+    return fp4_scaled(ch.tile(NT)[S], fp4_scale<S>(ch.sc[NT]));
+  }
   // The product of fragment J, and behind it the expansion of the next fragment: a product holds the matrix core for
   // sixteen cycles and the issue port for about seven of them.
   template <int J>
   __device__ __forceinline__ void fragments(const Fp4Chunk& ch, int i, bool more, bf16x8_t b) {
-    if constexpr (J < 16) {
-      constexpr int S = J >> 2, NT = J & 3;
+    if constexpr (J < 4 * TILES) {
+      constexpr int S = J / TILES, NT = T0 + J % TILES;
       bf16x8_t next{};
-      if constexpr (J < 15) next = fragment<J + 1>(ch);
+      if constexpr (J + 1 < 4 * TILES) next = fragment<J + 1>(ch);
       acc[NT] = fp4_mfma(a[S], b, acc[NT]);
       __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x002, 17, 0);
-      if (NT == 3) {
+      if (NT == T1 - 1) {
         u32x4_t held = __builtin_bit_cast(u32x4_t, next);
         asm volatile("" : "+v"(held));  // expanded here, beside the product, not behind the branch
         next = __builtin_bit_cast(bf16x8_t, held);
       }
       __builtin_amdgcn_sched_barrier(0);
-      if (NT == 3 && more) a[S] = piece(i + 1, S);  // uniform
+      if (NT == T1 - 1 && more) a[S] = piece(i + 1, S);  // uniform
       fragments<J + 1>(ch, i, more, next);
     }
   }
@@ -363,22 +410,22 @@ struct Fp4Full {
     src.row = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(sl.w + (int64_t)nb * p.chunks * NVFP4_BLOCK_BYTES), 0, p.chunks * NVFP4_BLOCK_BYTES, 0x00020000);
     const lds_ptr_t slot0 = (lds_ptr_t)ring;
     uint32_t codes, scales;
-    Fp4Ring::lanes(src, lane, lane & 15, (uint32_t)(uintptr_t)slot0, codes, scales);
-    Fp4Ring::request(src, c0, slot0);
+    Ring::lanes(src, lane, lane & 15, (uint32_t)(uintptr_t)slot0, codes, scales);
+    Ring::request(src, c0, slot0);
     asm volatile("" ::: "memory");
     start(p, sl, c0, lane);
     asm volatile("" ::: "memory");
-    if (n > 1) Fp4Ring::request(src, c0 + 1, slot0 + NVFP4_BLOCK_BYTES);
+    if (n > 1) Ring::request(src, c0 + 1, slot0 + NVFP4_BLOCK_BYTES);
     for (int i = 0; i < n; i++) {
       const uint32_t slot = (i & 1) * NVFP4_BLOCK_BYTES;
       Fp4Chunk ch;
       if (i + 1 < n) {
-        Fp4Ring::take<4 + Fp4Ring::LOADS, 0>(ch, codes + slot, scales + slot);
+        Ring::template take<4 + Ring::LOADS, 0>(ch, codes + slot, scales + slot);
       } else {
-        Fp4Ring::take<4, 0>(ch, codes + slot, scales + slot);
+        Ring::template take<4, 0>(ch, codes + slot, scales + slot);
       }
       fragments<0>(ch, i, i + 1 < n, fragment<0>(ch));
-      if (i + 2 < n) Fp4Ring::request(src, c0 + i + 2, slot0 + slot);
+      if (i + 2 < n) Ring::request(src, c0 + i + 2, slot0 + slot);
     }
   }
 };
@@ -398,7 +445,7 @@ __device__ __forceinline__ void nvfp4_workgroup(const StreamParams& p, int slot,
   if (active) {  // at least one chunk: the launch keeps ks <= chunks
     uint8_t* ring = rings + wave * FP4_RING_BYTES;
     if (sl.rows <= FP4_FEWER_ROWS && !p.no_few) {  // uniform over the workgroup
-      stream_block<EPI, Fp4Few4Acts, Fp4RingOf<0>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+      stream_block<EPI, Fp4Few4Acts<>, Fp4RingOf<0>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
       for (int d = 16; d <= 32; d *= 2) {  // the four blocks' sums: lane q = 0 now holds the slot's rows as the epilogue expects them
         add_lanes(acc0, d);
         add_lanes(acc1, d);
@@ -406,7 +453,7 @@ __device__ __forceinline__ void nvfp4_workgroup(const StreamParams& p, int slot,
         add_lanes(acc3, d);
       }
     } else if (sl.rows <= FP4_FEW_ROWS && !p.no_few) {
-      stream_block<EPI, Fp4Few8Acts, Fp4Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+      stream_block<EPI, Fp4Few8Acts<>, Fp4Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
       add_lanes(acc0, 32);  // the two parities': lanes q = 0, 1 hold slot rows 0 .. 7
       add_lanes(acc1, 32);
       add_lanes(acc2, 32);
@@ -427,6 +474,69 @@ template <int EPI>
 __global__ __launch_bounds__(1024) void nvfp4_stream_kernel(StreamParams p) {
   extern __shared__ __align__(16) uint8_t rings[];
   nvfp4_workgroup<EPI>(p, blockIdx.y, blockIdx.x, rings);
+}
+
+// A dense call of a few slots whose blocks are fewer than half the compute units: PARTS workgroups a 64-row block and slot, each
+// its 4 / PARTS 16-row tiles and only those tiles' codes. The sums and their order are those of the one workgroup. What bounds the
+// undivided launch is the expansion on a part of the device, and a small one the loads of a whole block ahead of the first product.
+// Traced, one workgroup a block and so, us: one row 1024 x 1024 4.5 and 3.4, 4096 x 2048 5.9 and 4.4, 2048 x 5120 8.1 and 5.5, 8192 x
+// 5120 9.0 and 7.0; eight rows 1024 x 4096 8.3 and 6.0, 8192 x 1024 5.5 and 4.4, 4096 x 5120 10.2 and 7.1; twelve rows, K split eight ways
+// and sixteen, 2048 x 5120 13.3, 8.6 and 8.0, 8192 x 5120 14.2, 10.8 and 9.8; 33 rows 2048 x 5120 13.0, 10.2 and 9.5. In two up to 256 blocks it
+// gained up to two rows only (12288 x 5120 four rows 10.2 and 11.2).
+template <int EPI, int T0, int T1>
+__device__ __forceinline__ void nvfp4_part_block(const StreamParams& p, const Slot& sl, int nb, const WaveShare& share, int lane, int wave, uint8_t* rings) {
+  f32x4_t acc[4];
+#pragma unroll
+  for (int t = 0; t < 4; t++) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  uint8_t* ring = rings + wave * FP4_RING_BYTES;
+  if (sl.rows <= FP4_FEWER_ROWS && !p.no_few) {  // uniform over the workgroup
+    stream_block<EPI, Fp4Few4Acts<T0, T1>, Fp4RingPart<0, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc[0], acc[1], acc[2], acc[3]);
+    for (int d = 16; d <= 32; d *= 2)
+#pragma unroll
+      for (int t = T0; t < T1; t++) add_lanes(acc[t], d);
+  } else if (sl.rows <= FP4_FEW_ROWS && !p.no_few) {
+    stream_block<EPI, Fp4Few8Acts<T0, T1>, Fp4RingPart<1, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc[0], acc[1], acc[2], acc[3]);
+#pragma unroll
+    for (int t = T0; t < T1; t++) add_lanes(acc[t], 32);
+  } else {
+    Fp4Full<EPI, T0, T1, Fp4RingPart<1, T0, T1>> full;
+    full.run(p, sl, nb, share.c0, share.c1, lane, ring);
+#pragma unroll
+    for (int t = T0; t < T1; t++) acc[t] = full.acc[t];
+  }
+  // finish_block for these tiles: the splits' sums through LDS, added in split order, an accumulator register a split and turn
+  constexpr int STRIDE = FP4_RING_BYTES / 4;
+  float* first = reinterpret_cast<float*>(rings);
+  float* mine = first + wave * STRIDE;
+#pragma unroll
+  for (int t = T0; t < T1; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) mine[(t * 4 + r) * 64 + lane] = acc[t][r];
+  __syncthreads();
+  for (int idx = 4 * T0 + share.ks; idx < 4 * T1; idx += p.ks) {
+    const int t = idx >> 2, r = idx & 3;
+    if (r >= sl.rows) continue;
+    float v = 0.f;
+    for (int s = 0; s < p.ks; s++) v += first[s * STRIDE + idx * 64 + lane];
+    emit<EPI, false>(p, sl, RowScales{}, nb, t, r, lane >> 4, lane & 15, v, 0.f);
+  }
+}
+template <int EPI, int PARTS>
+__global__ __launch_bounds__(1024) void nvfp4_part_kernel(StreamParams p) {
+  extern __shared__ __align__(16) uint8_t rings[];
+  const int die = blockIdx.x & 7, local = blockIdx.x >> 3, part = local % PARTS, nb = local / PARTS * 8 + die;  // a block's workgroups on one die
+  if (nb >= p.n_blocks) return;
+  const Slot sl = slot_of<EPI>(p, blockIdx.y);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const WaveShare share = wave_share(p, wave);
+  if constexpr (PARTS == 2) {
+    if (part == 0) nvfp4_part_block<EPI, 0, 2>(p, sl, nb, share, lane, wave, rings); else nvfp4_part_block<EPI, 2, 4>(p, sl, nb, share, lane, wave, rings);
+  } else {
+    if (part == 0) nvfp4_part_block<EPI, 0, 1>(p, sl, nb, share, lane, wave, rings);
+    else if (part == 1) nvfp4_part_block<EPI, 1, 2>(p, sl, nb, share, lane, wave, rings);
+    else if (part == 2) nvfp4_part_block<EPI, 2, 3>(p, sl, nb, share, lane, wave, rings);
+    else nvfp4_part_block<EPI, 3, 4>(p, sl, nb, share, lane, wave, rings);
+  }
 }
 
 // Two matrices of different geometry in one launch (the routed experts' layer beside the shared expert's, which reads
@@ -491,10 +601,25 @@ static void shape_nvfp4_dense(StreamParams& p) {
   set_split(p);
 }
 
+// Blocks, times slots of sixteen rows, up to which a dense call gives a block's tiles to two workgroups (up to half of them: to four).
+constexpr int FP4_PARTS_BLOCKS = 128;
 template <int EPI>
 static int launch_nvfp4(StreamParams& p, int64_t slots, int64_t busy_slots, hipStream_t stream) {
   if (int e = shape_nvfp4(p, busy_slots)) return e;
   if (epi_dense(EPI) && slots == 1 && !g_nvfp4_ksplit) shape_nvfp4_dense(p);
+  if constexpr (epi_dense(EPI)) {
+    if (!g_nvfp4_ksplit && p.n_blocks * slots <= FP4_PARTS_BLOCKS) {
+      p.nbw = 1;
+      const int most = p.m > FP4_FEW_ROWS && p.chunks >= 24 ? 16 : 8;  // a wavefront's start and the exchange against the expansion of nine rows and more
+      while (p.ks < most && 2 * p.ks <= p.chunks) p.ks *= 2;
+      set_split(p);
+      const bool four = p.n_blocks * slots <= FP4_PARTS_BLOCKS / 2;
+      const dim3 grid((unsigned)((p.n_blocks + 7) / 8 * 8 * (four ? 4 : 2)), (unsigned)slots);
+      auto launch = [&](auto kernel) { HB_LAUNCH(kernel, grid, dim3(64 * p.ks), (size_t)p.ks * FP4_RING_BYTES, stream, p); };
+      four ? launch(nvfp4_part_kernel<EPI, 4>) : launch(nvfp4_part_kernel<EPI, 2>);
+      return HB_OK;
+    }
+  }
   const dim3 grid((unsigned)((p.n_blocks + p.nbw - 1) / p.nbw), (unsigned)slots);
   const int waves = p.ks * p.nbw;
   HB_LAUNCH(nvfp4_stream_kernel<EPI>, grid, dim3(64 * waves), (size_t)waves * FP4_RING_BYTES, stream, p);

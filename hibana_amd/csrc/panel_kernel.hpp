@@ -27,7 +27,7 @@ namespace hb {
 constexpr int PANEL_HALF = 64;       // k of a half chunk
 constexpr int PANEL_WAVES = 8;       // at most, a workgroup
 constexpr int PANEL_LDS = 160 * 1024;
-constexpr int PANEL_MT = 8;          // row tiles of a slot, at most
+constexpr int PANEL_MT = 8;          // row tiles of a dense call's slot, at most
 
 // The fewest blocks of a workgroup. A split's half chunk of activations is 2 mt pieces, brought by the split's wavefronts, one a
 // block, each of which holds its pieces' addresses in registers: eight at most, and four from seven row tiles on, where the
@@ -122,8 +122,8 @@ struct Panel {
   static constexpr int HALVES_FROM = 6;
 
   // The products of fragment J = 4 * step + tile of a chunk, and between them the expansion of fragment J + 1, a pair of
-  // its values behind every MT / 4 products (or half a pair behind every MT / 8). The empty statements hold that order: left to
-  // itself the compiler puts the expansion behind the products (fewer registers), where nothing runs beside it.
+  // its values behind every MT / 4 products (or half a pair behind every MT / 8; the last of nine
+  // has none). The empty statements hold that order: left to itself the compiler puts the expansion behind the products (fewer registers), where nothing runs beside it.
   // FRESH: the activations' fragments may still be on their way (asked for in order, nothing behind them). NEXT >= 0: the
   // LDS offset of the next step's, from `at`.
   template <int J, bool FRESH, int NEXT>
@@ -147,8 +147,8 @@ struct Panel {
       if constexpr (J < 15 && T == 0) part = Fmt::template open<((J + 1) & 3), ((J + 1) >> 2)>(ch, sl);
       if constexpr (MT >= HALVES_FROM) {  // halves of pairs: half I goes behind product I MT / 8
         constexpr int I = (8 * T + MT - 1) / MT;
-        static_assert(I * MT / 8 == T && I < 8, "a half for every product");
-        if constexpr (J >= 15) {
+        static_assert(I == 8 || I * MT / 8 == T, "a half for every product, up to the eighth");
+        if constexpr (J >= 15 || I == 8) {
           product<T == 0>(acc[T][NT], w, now[T]);
         } else if constexpr (I & 1) {
           product_second(acc[T][NT], w, now[T], two, part.scale, out[I >> 1]);
@@ -531,7 +531,7 @@ __device__ __forceinline__ void panel_tiles(const StreamParams& p, const Slot& s
 // the same place in that turn, so that its activations come into one L2 once
 // (2048 rows, 22 of 512 experts, (1024, 2688): the latent block 811 -> 782 us; 1543 rows of the three-bit layer 285 -> 276).
 // A compute unit holds as many workgroups as the registers of the highest slot leave room for: four with slots of 48 rows, three
-// with 80, two with 128 (the choice: panel_height).
+// with 80, two with 128 and 144 (the choice: panel_height).
 template <class Fmt, int EPI, int MOST>
 __global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void panel_tile_kernel(StreamParams p) {
   extern __shared__ __align__(16) uint8_t panel_lds[];
@@ -697,10 +697,16 @@ inline size_t panel_routed_lds(int mt, int nbw) {
 // Three-bit, 512 experts (2048, 512), even routing 14 rows 223, 234, 252, 24 rows 262, 265, 277, 40 rows 324, 313, 321, 52 rows
 // 421, 351, 366; skewed 14 rows 176, 171, 174, 24 rows 232, 217, 224, 52 rows 395, 351, 343; 180 experts (1664, 384) 64 rows 158, 135, 143, 90
 // rows 184, 179, 167.
-constexpr int PANEL_SLOT_TILES = 8;  // at most
+// 128 and 144 rows a slot, both two workgroups a compute unit: the higher one is for the experts just past 128 rows, whose last
+// rows cost a second expansion of all their weights. NVFP4, 512 experts (1024, 2688) 60 rows an expert 550 and 552, 73 rows 625 and 609, 88
+// rows 713 and 698, 172 rows 1199 and 1172; 200 experts (768, 1536) 56 rows 148.5 and 149.7, 66 rows 159.7 and 160.9, 77 rows 169.4 and
+// 168.4, 126 rows 214.0 and 214.7. Three-bit, 200 experts (2048, 512), even routing 75 rows 186.3 and 187.6, 90 rows 204.7 and
+// 205.6, 118 rows 237 and 235, 130 rows 275 and 249, 150 rows 316 and 303; skewed 90 rows 224 and 217, 130 rows 279 and 275.
+constexpr int PANEL_SLOT_TILES = 9;      // at most
+constexpr int PANEL_REFUSED_ROWS = 128;  // calls of more than 65535 slots are refused; of higher slots, as many rows as of these
 template <class Fmt>
 inline int panel_height(int64_t pairs, int64_t named) {
-  return pairs < Fmt::LOW_ROWS * named ? 3 : pairs < Fmt::MIDDLE_ROWS * named ? 5 : PANEL_SLOT_TILES;
+  return pairs < Fmt::LOW_ROWS * named ? 3 : pairs < Fmt::MIDDLE_ROWS * named ? 5 : pairs < Fmt::HIGH_ROWS * named ? 8 : PANEL_SLOT_TILES;
 }
 
 // Over a plan's slots of 16 `tiles` rows; `a_rows`: rows of the activation matrix. Four wavefronts a workgroup on four
@@ -717,7 +723,7 @@ static int launch_panel_routed(StreamParams& p, int tiles, int64_t slots, int64_
   const int64_t grid = (slots + 7) / 8 * 8 * p.panel_groups;
   if (!panel_takes(a_rows, p.a_stride) || grid > 0x7fffffff) return HB_EINVAL;
   auto launch = [&](auto kernel) { HB_LAUNCH(kernel, dim3((unsigned)grid), dim3(64 * p.ks * p.nbw), panel_routed_lds<Fmt>(tiles, p.nbw), stream, p); };
-  tiles == 3 ? launch(panel_tile_kernel<Fmt, EPI, 3>) : tiles == 5 ? launch(panel_tile_kernel<Fmt, EPI, 5>) : launch(panel_tile_kernel<Fmt, EPI, PANEL_SLOT_TILES>);
+  tiles == 3 ? launch(panel_tile_kernel<Fmt, EPI, 3>) : tiles == 5 ? launch(panel_tile_kernel<Fmt, EPI, 5>) : tiles == 8 ? launch(panel_tile_kernel<Fmt, EPI, 8>) : launch(panel_tile_kernel<Fmt, EPI, PANEL_SLOT_TILES>);
   return HB_OK;
 }
 

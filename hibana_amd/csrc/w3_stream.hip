@@ -1089,7 +1089,7 @@ struct TileW3 {
   // routing of 10 of 512 experts (2048, 512), where 218 of 377 slots are such: the layer of 1024 rows 205 -> 187 us, 1543
   // 251 -> 234, 2048 296 -> 271; even routing at the same sizes unchanged. A ring of four slots with the activations as far
   // ahead gave nothing: what the wavefronts wait for is each other's issue slots.
-  static constexpr int LOW_ROWS = 22, MIDDLE_ROWS = 60;  // panel_height's lines
+  static constexpr int LOW_ROWS = 22, MIDDLE_ROWS = 60, HIGH_ROWS = 88;  // panel_height's lines
   static constexpr int LIGHT_ROWS = ROWS_PER_SLOT;
   template <int EPI>
   static __device__ __forceinline__ void light(const StreamParams& p, const Slot& sl, int group, uint8_t* lds) {
@@ -1387,7 +1387,7 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   // Under a budget the table ends behind the experts the selection can name: the launches' grids reach over all of it, and a
   // workgroup without rows is not free (40 rows of 10, a cap of 60 of 512 experts: 53.5 us before, 53.2 so). What a call of
   // these pairs is refused for, and how its launches split K, go by the whole table: the bits of the same ids without a budget.
-  const int64_t whole = moe_max_slots(pairs, ex->experts, shared_rows, slot_rows);
+  const int64_t whole = moe_max_slots(pairs, ex->experts, shared_rows, std::min(slot_rows, PANEL_REFUSED_ROWS));
   if (whole > 65535) return HB_EINVAL;
   if (route && route->budget) {
     if (int e = moe_check_budget(*route->budget, m, topk)) return e;

@@ -1,6 +1,6 @@
 """Routed calls on the panel kernel, slot by slot: the weight stream's bodies for a slot's few rows (one to four, five to
-sixteen), the panel's from seventeen, at every number of K chunks around the stream's two-deep ring; slots of 48, 80 and 128
-rows, which the rows an expert choose; and the lines that give a call to the panel kernel."""
+sixteen), the panel's from seventeen, at every number of K chunks around the stream's two-deep ring; slots of 48, 80, 128 and
+144 rows, which the rows an expert choose; and the lines that give a call to the panel kernel."""
 import pytest
 import torch
 
@@ -18,11 +18,11 @@ def _call(counts, seed):
     return m, ids, g
 
 
-TOTALS = [0, 31, 100]  # experts that the ids are said to name: 59, 46 and 14 rows an expert
-MORE = [300]            # ... and with one expert more 69
+TOTALS = [0, 31, 100]  # experts that the ids are said to name: 56, 43 and 13 rows an expert
+MORE, MOST = [300], [900]  # ... and with one expert more 65 and 89
 
 
-@pytest.mark.parametrize("total,more", [(t, []) for t in TOTALS] + [(0, MORE)])
+@pytest.mark.parametrize("total,more", [(t, []) for t in TOTALS] + [(0, MORE), (0, MOST)])
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("hidden,inter", [(128, 256), (256, 384), (384, 128), (640, 512)])  # 1, 2, 3, 5 chunks of fc1; 2, 3, 1, 4 of fc2
 def test_w3_slots_of_every_height(hidden, inter, gated, total, more):
@@ -44,7 +44,7 @@ def test_w3_slots_of_every_height(hidden, inter, gated, total, more):
     assert torch.equal(got, again)
 
 
-@pytest.mark.parametrize("total,more", [(t, []) for t in TOTALS] + [(0, MORE)])
+@pytest.mark.parametrize("total,more", [(t, []) for t in TOTALS] + [(0, MORE), (0, MOST)])
 @pytest.mark.parametrize("gated", [True, False])
 @pytest.mark.parametrize("hidden,inter", [(128, 256), (384, 128)])
 def test_nvfp4_slots_of_every_height(hidden, inter, gated, total, more):

@@ -702,11 +702,12 @@ inline size_t panel_routed_lds(int mt, int nbw) {
 // rows 713 and 698, 172 rows 1199 and 1172; 200 experts (768, 1536) 56 rows 148.5 and 149.7, 66 rows 159.7 and 160.9, 77 rows 169.4 and
 // 168.4, 126 rows 214.0 and 214.7. Three-bit, 200 experts (2048, 512), even routing 75 rows 186.3 and 187.6, 90 rows 204.7 and
 // 205.6, 118 rows 237 and 235, 130 rows 275 and 249, 150 rows 316 and 303; skewed 90 rows 224 and 217, 130 rows 279 and 275.
+// From 256 rows an expert, with two and more full slots each, 128 again: the higher ones are measured to 172 rows.
 constexpr int PANEL_SLOT_TILES = 9;      // at most
 constexpr int PANEL_REFUSED_ROWS = 128;  // calls of more than 65535 slots are refused; of higher slots, as many rows as of these
 template <class Fmt>
 inline int panel_height(int64_t pairs, int64_t named) {
-  return pairs < Fmt::LOW_ROWS * named ? 3 : pairs < Fmt::MIDDLE_ROWS * named ? 5 : pairs < Fmt::HIGH_ROWS * named ? 8 : PANEL_SLOT_TILES;
+  return pairs < Fmt::LOW_ROWS * named ? 3 : pairs < Fmt::MIDDLE_ROWS * named ? 5 : pairs < Fmt::HIGH_ROWS * named || pairs >= 256 * named ? 8 : PANEL_SLOT_TILES;
 }
 
 // Over a plan's slots of 16 `tiles` rows; `a_rows`: rows of the activation matrix. Four wavefronts a workgroup on four

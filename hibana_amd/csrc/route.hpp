@@ -56,90 +56,125 @@ __device__ __forceinline__ int wave_inclusive_sum(int x) {
 // The k largest of a wavefront's keys (0: no key), largest first, one a lane: lane s < k gets selection s's key and its tag, the
 // lane's place of it (lane * per + register). Equal keys in ascending lane, then register.
 //
-// A threshold that at least k lanes' largest keys reach, found by cutting the interval in four a step; the keys that reach it, some
-// k + k / 4 of them, go to a lane each (ds_permute), every lane counts the ones ahead of its own, and they go to the lanes their ranks
-// name. Before, a round a selection (wave-wide maximum, ballot, a lane's list moving up) on lists sorted in each lane and sums and maxima through the LDS:
-// one token of the three-bit layer (top 10 of 512) 19.8 us, 19.2 so; the latent block's one token (top 22 of 512) 47.4 and 46.0, four 81.6
-// and 79.7.
-// Rounds, without the sort, remain for rows where more than 63 keys reach the threshold: many equal scores, or the best experts
-// side by side in a few lanes.
-constexpr int TOP_SLACK = 3;  // lanes that may reach the threshold beyond k
-template <int PER>
+// A threshold that at least k lanes' largest keys reach, found by cutting the interval in four a step; where more than 63 keys
+// reach it (rows of more than some 36 selections), raised until 63 or fewer do. Those go to a lane each (ds_permute), every lane
+// counts the ones ahead of its own, and they go to the lanes their ranks name. TIES: equal keys are common (softmax scores of BF16
+// logits: six rows in ten tie inside or at the end of the top 10 of 512), and the count goes by key and lane at once; else by the
+// keys alone, and again where two lanes get one rank. What bounds it is one wavefront's chain of dependent instructions. The routing
+// launch of 64 rows of 512 softmax scores, us, by rounds on sorted lists and so: top 10 4.7 and 4.1, top 22 6.3 and 4.9, top 40 8.8 and
+// 6.2, top 56 11.0 and 7.1; scores of BF16 logits counted by the keys alone first, 4.7 and 6.0 at 10 and 22, so 4.1 and 4.9. One token of the three-bit
+// layer (top 10 of 512) 19.8 us by rounds, 19.2 so; the latent block's one token (top 22) 47.4 and 46.0.
+// Rounds, a selection each, remain for more than TOP_SEARCH selections, which leave the threshold too little room between k and 63
+// keys (ties among 64 rows of BF16 logits: at 60 selections 14.4 us with the search in vain ahead of the rounds, 11.5 without), and for rows
+// of many equal scores at it.
+constexpr int TOP_SLACK = 3;    // lanes that may reach the threshold beyond k
+constexpr int TOP_SEARCH = 56;  // selections, at most, that the threshold serves
+template <bool TIES, int PER>
 __device__ __forceinline__ void top_ranked(uint32_t (&key)[PER], int per, int k, int lane, uint32_t& out_key, int& out_tag) {
-  uint32_t head = key[0];
-#pragma unroll
-  for (int j = 1; j < PER; j++) head = max(head, key[j]);
-  const uint32_t most = wave_max_u32(head), least = ~wave_max_u32(~head);
-  uint32_t lo = max(least, 1u), hi = most;  // at least k lanes reach lo (or all that hold a key do); fewer than k reach hi, unless it is the threshold
-  if (__popcll(__ballot(head >= hi)) >= k) lo = hi;
-  while (hi - lo > 1u) {  // three places of the interval a step, their ballots side by side
-    const uint32_t part = max((hi - lo) >> 2, 1u);
-    const uint32_t at1 = lo + part, at2 = min(at1, hi - part) + part, at3 = min(at2, hi - part) + part;
-    const int reach1 = __popcll(__ballot(head >= at1)), reach2 = __popcll(__ballot(head >= at2)), reach3 = __popcll(__ballot(head >= at3));
-    const bool over1 = reach1 >= k, over2 = reach2 >= k, over3 = reach3 >= k;
-    const int reach = over3 ? reach3 : over2 ? reach2 : over1 ? reach1 : 64;
-    hi = over3 ? hi : over2 ? at3 : over1 ? at2 : at1;
-    lo = over3 ? at3 : over2 ? at2 : over1 ? at1 : lo;
-    if (reach <= k + TOP_SLACK) break;
-  }
-  int count = 0;
-#pragma unroll
-  for (int j = 0; j < PER; j++) count += key[j] >= lo ? 1 : 0;
-  const int upto = wave_inclusive_sum(count), all = __builtin_amdgcn_readlane(upto, 63);
   out_key = 0u;
   out_tag = 0;
-  if (all <= 63) {  // uniform; (all >= k, or every key there is)
-    int at = upto - count;
-    uint32_t mine = 0u;
-    int tag = 0;
+  if (__builtin_expect(k <= TOP_SEARCH, 1)) {  // uniform
+    uint32_t head = key[0];
 #pragma unroll
-    for (int j = 0; j < PER; j++) {  // lane 63 takes what goes nowhere; a lane that nothing is sent to gets zero
-      const bool take = key[j] >= lo;
-      const int to = 4 * (take ? at : 63);
-      mine |= (uint32_t)__builtin_amdgcn_ds_permute(to, (int)key[j]);
-      tag |= __builtin_amdgcn_ds_permute(to, lane * per + j);
-      at += take ? 1 : 0;
+    for (int j = 1; j < PER; j++) head = max(head, key[j]);
+    const uint32_t most = wave_max_u32(head), least = ~wave_max_u32(~head);
+    uint32_t lo = max(least, 1u), hi = most;  // at least k lanes reach lo (or all that hold a key do); fewer than k reach hi, unless it is the threshold
+    if (__popcll(__ballot(head >= hi)) >= k) lo = hi;
+    while (hi - lo > 1u) {  // three places of the interval a step, their ballots side by side
+      const uint32_t part = max((hi - lo) >> 2, 1u);
+      const uint32_t at1 = lo + part, at2 = min(at1, hi - part) + part, at3 = min(at2, hi - part) + part;
+      const int reach1 = __popcll(__ballot(head >= at1)), reach2 = __popcll(__ballot(head >= at2)), reach3 = __popcll(__ballot(head >= at3));
+      const bool over1 = reach1 >= k, over2 = reach2 >= k, over3 = reach3 >= k;
+      const int reach = over3 ? reach3 : over2 ? reach2 : over1 ? reach1 : 64;
+      hi = over3 ? hi : over2 ? at3 : over1 ? at2 : at1;
+      lo = over3 ? at3 : over2 ? at2 : over1 ? at1 : lo;
+      if (reach <= k + TOP_SLACK) break;
     }
-    if (lane >= all) mine = 0u;
-    auto deal = [&](bool ties) {
-      int rank = 0;
-      for (int c0 = 0; c0 < all; c0 += 4) {
+    auto reaching = [&] {
+      int n = 0;
 #pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, min(c0 + c, 63));
-          rank += other > mine ? 1 : 0;
-          if (ties) rank += other == mine && c0 + c < lane ? 1 : 0;
-        }
-      }
-      const int to = 4 * (lane < all && rank < k ? rank : 63);
-      out_key = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)mine);
-      out_tag = __builtin_amdgcn_ds_permute(to, tag);
-      return __popcll(__ballot(lane < all && rank < k)) == __popcll(__ballot(lane < k && out_key != 0u));  // a rank for every key, a key for every rank
+      for (int j = 0; j < PER; j++) n += key[j] >= lo ? 1 : 0;
+      return n;
     };
-    if (!deal(false)) deal(true);  // equal keys had one rank between them
-    if (lane >= k) out_key = 0u, out_tag = 0;
-    return;
-  }
-  for (int s = 0; s < k; s++) {
-    uint32_t best = 0;
-    int at = 0;
+    int count = reaching(), upto = wave_inclusive_sum(count), all = __builtin_amdgcn_readlane(upto, 63);
+    if (__builtin_expect(all > 63, 0)) {  // uniform
+      uint32_t over = most;
+      while (over - lo > 1u && all > 63) {
+        const uint32_t mid = lo + ((over - lo) >> 1);
+        int n = 0;
 #pragma unroll
-    for (int j = 0; j < PER; j++)
-      if (key[j] > best) {  // ascending index within the lane: the first of equals stays
-        best = key[j];
-        at = j;
+        for (int j = 0; j < PER; j++) n += __popcll(__ballot(key[j] >= mid));
+        if (n >= k) lo = mid, all = n; else over = mid;
       }
-    const uint32_t top = wave_max_u32(best);
-    const int winner = __builtin_ctzll(__ballot(best == top));
-    const int wj = __builtin_amdgcn_readlane(at, winner);
+      count = reaching();
+      upto = wave_inclusive_sum(count);
+    }
+    if (__builtin_expect(all <= 63, 1)) {  // (all >= k, or every key there is)
+      int at = upto - count;
+      uint32_t mine = 0u;
+      int tag = 0;
+#pragma unroll
+      for (int j = 0; j < PER; j++) {  // lane 63 takes what goes nowhere; a lane that nothing is sent to gets zero
+        const bool take = key[j] >= lo;
+        const int to = 4 * (take ? at : 63);
+        mine |= (uint32_t)__builtin_amdgcn_ds_permute(to, (int)key[j]);
+        tag |= __builtin_amdgcn_ds_permute(to, lane * per + j);
+        at += take ? 1 : 0;
+      }
+      if (lane >= all) mine = 0u;
+      const uint32_t under = mine - 1u;  // a lower lane's equal key is ahead: it exceeds the key less one (no key here is 0)
+      auto deal = [&](bool ties) {
+        int rank = 0;
+        for (int c0 = 0; c0 < all; c0 += 4) {
+#pragma unroll
+          for (int c = 0; c < 4; c++) {
+            const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, min(c0 + c, 63));
+            rank += other > (ties && __builtin_amdgcn_inverse_ballot_w64(~1ull << min(c0 + c, 63)) ? under : mine) ? 1 : 0;
+          }
+        }
+        const int to = 4 * (lane < all && rank < k ? rank : 63);
+        out_key = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)mine);
+        out_tag = __builtin_amdgcn_ds_permute(to, tag);
+        return TIES || __popcll(__ballot(lane < all && rank < k)) == __popcll(__ballot(lane < k && out_key != 0u));  // a rank for every key, a key for every rank
+      };
+      if (__builtin_expect(!deal(TIES), 0)) deal(true);  // equal keys had one rank between them
+      if (lane >= k) out_key = 0u, out_tag = 0;
+      return;
+    }
+  }
+  // The lane's keys in descending order once (adjacent exchanges on a strictly larger right neighbour only, so equal keys keep
+  // their order), their registers as nibbles of one word: a round looks at the heads, and the winner's list moves up by one.
+  uint32_t from[PER];
+#pragma unroll
+  for (int j = 0; j < PER; j++) from[j] = j;
+#pragma unroll
+  for (int pass = 0; pass < PER; pass++) {
+#pragma unroll
+    for (int j = pass & 1; j + 1 < PER; j += 2) {
+      const bool swap = key[j + 1] > key[j];
+      const uint32_t ka = key[j], kb = key[j + 1], fa = from[j], fb = from[j + 1];
+      key[j] = swap ? kb : ka;
+      key[j + 1] = swap ? ka : kb;
+      from[j] = swap ? fb : fa;
+      from[j + 1] = swap ? fa : fb;
+    }
+  }
+  uint64_t order = 0;
+#pragma unroll
+  for (int j = 0; j < PER; j++) order |= (uint64_t)from[j] << (4 * j);
+  for (int s = 0; s < k; s++) {
+    const uint32_t top = wave_max_u32(key[0]);
+    const int winner = __builtin_ctzll(__ballot(key[0] == top));
+    const int from_register = __builtin_amdgcn_readlane((int)order, winner) & 15;
     if (lane == s) {
       out_key = top;
-      out_tag = winner * per + wj;
+      out_tag = winner * per + from_register;
     }
     if (lane == winner) {
 #pragma unroll
-      for (int j = 0; j < PER; j++)
-        if (j == wj) key[j] = 0u;
+      for (int j = 0; j + 1 < PER; j++) key[j] = key[j + 1];
+      key[PER - 1] = 0u;
+      order >>= 4;
     }
   }
 }
@@ -248,7 +283,7 @@ __device__ __forceinline__ int route_row(const RouteParams& p, int r, int lane, 
   float total = 0.f, mine = 0.f;
   int mine_id;
   uint32_t mine_key;
-  top_ranked(key, per, p.k, lane, mine_key, mine_id);
+  top_ranked<!SIGMOID>(key, per, p.k, lane, mine_key, mine_id);
   if (lane < p.k) {
     if (SIGMOID) {  // the key is score + bias: the plain score is made again from the logit
       mine = 1.0f / (1.0f + expf(-logit(row + mine_id)));

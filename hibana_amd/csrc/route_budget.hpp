@@ -76,7 +76,7 @@ __device__ __forceinline__ void rank_row(const BudgetParams& q, int t, int lane)
   sum = wave_sum(sum);
   uint32_t mine_key;
   int place;
-  top_ranked(key, PER, BUDGET_CANDIDATES, lane, mine_key, place);
+  top_ranked<false>(key, PER, BUDGET_CANDIDATES, lane, mine_key, place);
   const int mine_id = 0xffff - (int)(mine_key & 0xffffu);
   const float mine_v = bf16_order_value(mine_key >> 16);
   const float mine = expf(mine_v - mx) / sum;

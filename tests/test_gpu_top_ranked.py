@@ -51,3 +51,51 @@ def test_softmax_and_sigmoid_rows(kind, e, k):
     if kind in ("coarse", "equal", "pairs"):
         assert torch.equal(ids.long(), torch.argsort(logits, dim=-1, descending=True, stable=True)[:, :k])
     assert torch.allclose(weights.double(), picked / (picked.sum(-1, keepdim=True) + 1e-20), rtol=1e-5)
+
+
+@pytest.mark.parametrize("kind", ["plain", "coarse", "clustered", "pairs", "bf16"])
+@pytest.mark.parametrize("e,k", [(512, 36), (512, 41), (512, 48), (512, 56), (512, 57), (1024, 48), (1024, 56), (1024, 57), (1024, 64)])
+def test_more_selections_than_the_lanes_largest_keys_separate(kind, e, k):
+    """Past some 36 selections the lanes' largest keys let more than 63 keys through: the threshold is raised, and past 56 rounds
+    on sorted lists take over (with eight registers a lane and with sixteen)."""
+    from hibana_amd.kernels import ops
+    g = torch.Generator().manual_seed(e + k)
+    logits = (torch.randn(24, e, generator=g).bfloat16() if kind == "bf16" else _rows(kind, e, g)).float().cuda()
+    ids, weights = ops.route_topk(logits, k)
+    prob = torch.softmax(logits.double(), -1)
+    order = torch.argsort(logits, dim=-1, descending=True, stable=True)[:, :k]
+    same = ids.long() == order
+    if kind in ("coarse", "pairs", "bf16"):  # logits apart by more than a rounding of the scores, or equal
+        assert bool(same.all())
+    assert all(len(set(row)) == k for row in ids.tolist())
+    assert bool((same | ((prob.gather(1, ids.long()) - prob.gather(1, order)).abs() <= 1e-6 * prob.gather(1, order) + 1e-37)).all())
+    want = prob.gather(1, ids.long())
+    assert torch.allclose(weights.double(), want / want.sum(-1, keepdim=True), rtol=1e-5, atol=1e-30)
+
+
+@pytest.mark.parametrize("bf16", [False, True])
+def test_forty_eight_selections_take_no_rounds(bf16):
+    """The routing launch at 48 selections against 32: 1.2 times as long by the threshold (a round a selection behind a search in
+    vain made it 2.1 to 2.9)."""
+    from hibana_amd.kernels import ops
+    logits = torch.randn(64, 512, generator=torch.Generator().manual_seed(2))
+    logits = (logits.bfloat16().float() if bf16 else logits).cuda()
+
+    def shortest(k, calls=50):
+        ops.route_topk(logits, k)
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(calls):
+                ops.route_topk(logits, k)
+        times = []
+        for _ in range(20):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            graph.replay()
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end))
+        return min(times)
+
+    assert shortest(48) < 1.7 * shortest(32)

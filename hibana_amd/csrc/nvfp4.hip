@@ -858,9 +858,9 @@ int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, i
   const int64_t rows_min = ex->experts < named ? 8 : 7;
   const bool dense = panel_takes(m, ex->hidden) && panel_takes(pairs, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
                      (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && pairs >= rows_min * named));
-  const int tiles = panel_height<TileNvfp4>(pairs, named), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
+  const int tiles = panel_height<TileNvfp4>(pairs, named, ex->experts, 0), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
   const int64_t slots = moe_max_slots(pairs, ex->experts, 0, slot_rows);
-  if (moe_max_slots(pairs, ex->experts, 0, std::min(slot_rows, PANEL_REFUSED_ROWS)) > 65535) return HB_EINVAL;
+  if (moe_max_slots(pairs, ex->experts, 0, std::min(slot_rows, PANEL_REFUSED_ROWS)) > PANEL_MAX_SLOTS) return HB_EINVAL;
   if (int e = moe_launch_plan(ids, pairs, ex->base, ex->experts, 0, ws, stream, slot_rows)) return e;
   const int64_t est = busy_slots(pairs, ex->experts, slots);
   StreamParams p, f2;

@@ -704,10 +704,13 @@ inline size_t panel_routed_lds(int mt, int nbw) {
 // 205.6, 118 rows 237 and 235, 130 rows 275 and 249, 150 rows 316 and 303; skewed 90 rows 224 and 217, 130 rows 279 and 275.
 // From 256 rows an expert, with two and more full slots each, 128 again: the higher ones are measured to 172 rows.
 constexpr int PANEL_SLOT_TILES = 9;      // at most
-constexpr int PANEL_REFUSED_ROWS = 128;  // calls of more than 65535 slots are refused; of higher slots, as many rows as of these
+constexpr int PANEL_REFUSED_ROWS = 128;  // calls of more than PANEL_MAX_SLOTS slots are refused; of higher slots, as many rows as of these
+constexpr int64_t PANEL_MAX_SLOTS = 65535;
 template <class Fmt>
-inline int panel_height(int64_t pairs, int64_t named) {
-  return pairs < Fmt::LOW_ROWS * named ? 3 : pairs < Fmt::MIDDLE_ROWS * named ? 5 : pairs < Fmt::HIGH_ROWS * named || pairs >= 256 * named ? 8 : PANEL_SLOT_TILES;
+inline int panel_height(int64_t pairs, int64_t named, int experts, int shared_rows) {
+  const int tiles = pairs < Fmt::LOW_ROWS * named ? 3 : pairs < Fmt::MIDDLE_ROWS * named ? 5 : pairs < Fmt::HIGH_ROWS * named || pairs >= 256 * named ? 8 : PANEL_SLOT_TILES;
+  // the ids may all lie here, whatever share of the experts this is: a call that low slots would have refused takes higher ones
+  return tiles < 8 && moe_max_slots(pairs, experts, shared_rows, 16 * tiles) > PANEL_MAX_SLOTS ? 8 : tiles;
 }
 
 // Over a plan's slots of 16 `tiles` rows; `a_rows`: rows of the activation matrix. Four wavefronts a workgroup on four

@@ -1383,12 +1383,12 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   const bool dense = !e4m3 && panel_takes(m, ex->hidden) && panel_takes(pairs + shared_rows, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
                      (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && (pairs >= (ex->experts < named ? 48 : 32) * named || (pairs >= 16 * named && local * expert_blocks >= 650000) ||
                                                                                         (pairs >= 10 * named && local * expert_blocks >= 1400000))));
-  const int tiles = panel_height<TileW3<3>>(pairs, named), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
+  const int tiles = panel_height<TileW3<3>>(pairs, named, ex->experts, shared_rows), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
   // Under a budget the table ends behind the experts the selection can name: the launches' grids reach over all of it, and a
   // workgroup without rows is not free (40 rows of 10, a cap of 60 of 512 experts: 53.5 us before, 53.2 so). What a call of
   // these pairs is refused for, and how its launches split K, go by the whole table: the bits of the same ids without a budget.
   const int64_t whole = moe_max_slots(pairs, ex->experts, shared_rows, std::min(slot_rows, PANEL_REFUSED_ROWS));
-  if (whole > 65535) return HB_EINVAL;
+  if (whole > PANEL_MAX_SLOTS) return HB_EINVAL;
   if (route && route->budget) {
     if (int e = moe_check_budget(*route->budget, m, topk)) return e;
   }

@@ -86,3 +86,23 @@ def test_w3_calls_from_sixteen_rows_an_expert(m, panel):
             _lib.lib().hb_tune(b"w3_tile", 0)
     got, by_panel, by_stream = results
     assert not torch.equal(by_panel, by_stream) and torch.equal(got, by_panel if panel else by_stream)
+
+
+@pytest.mark.parametrize("fmt", ["w3", "nvfp4"])
+def test_low_slots_refuse_nothing(fmt):
+    """Ids that all lie in a small share of the experts: 3.3 million pairs are more slots of 48 rows than a call may have, and fewer
+    of 128."""
+    from hibana_amd import _lib, synthetic
+    from hibana_amd.kernels import w3_moe
+    m, topk, named = 51200, 64, 200000
+    ex = synthetic.w3_experts(64, 128, 128, True, 3) if fmt == "w3" else synthetic.nvfp4_experts(64, 128, 128, 3)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    ids = torch.rand(m, 64, device="cuda", generator=g).argsort(1).to(torch.int32)
+    x, weights = torch.randn(m, 128, device="cuda", generator=g).bfloat16(), torch.rand(m, topk, device="cuda", generator=g)
+    call = (lambda total: w3_moe.w3_moe(ex, x, ids, weights, experts_total=total)) if fmt == "w3" else (lambda total: ex(x, ids, weights, experts_total=total))
+    key = b"w3_tile" if fmt == "w3" else b"nvfp4_tile"
+    assert _lib.lib().hb_tune(key, 1) == 0  # the panel kernel for both
+    try:
+        assert torch.equal(call(named), call(0))
+    finally:
+        _lib.lib().hb_tune(key, 0)

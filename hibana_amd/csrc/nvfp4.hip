@@ -685,7 +685,7 @@ struct TileNvfp4 {
   static constexpr bool PER_ROW = false;
   static constexpr float EXPAND_US = 0.f;  // (the estimate's own constants are this format's)
   static constexpr int BESIDE_TILES = 0;
-  static constexpr int LOW_ROWS = 24, MIDDLE_ROWS = 46, HIGH_ROWS = 70;  // panel_height's lines
+  static constexpr int LOW_ROWS = 24, MIDDLE_ROWS = 46, MIDDLE_ROWS_LARGE = 46, HIGH_ROWS = 70;  // panel_height's lines
   static constexpr int LIGHT_ROWS = 0;  // (an expansion takes the scale along at the price of the stream's)
   template <int EPI>
   static __device__ __forceinline__ void light(const StreamParams&, const Slot&, int, uint8_t*) {}
@@ -858,7 +858,7 @@ int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, i
   const int64_t rows_min = ex->experts < named ? 8 : 7;
   const bool dense = panel_takes(m, ex->hidden) && panel_takes(pairs, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
                      (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && pairs >= rows_min * named));
-  const int tiles = panel_height<TileNvfp4>(pairs, named, ex->experts, 0), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
+  const int tiles = panel_height<TileNvfp4>(pairs, named, ex->experts, 0, (ex->gated ? 2 : 1) * ex->inter / 64), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
   const int64_t slots = moe_max_slots(pairs, ex->experts, 0, slot_rows);
   if (moe_max_slots(pairs, ex->experts, 0, std::min(slot_rows, PANEL_REFUSED_ROWS)) > PANEL_MAX_SLOTS) return HB_EINVAL;
   if (int e = moe_launch_plan(ids, pairs, ex->base, ex->experts, 0, ws, stream, slot_rows)) return e;

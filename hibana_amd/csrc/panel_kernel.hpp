@@ -699,16 +699,30 @@ inline size_t panel_routed_lds(int mt, int nbw) {
 // rows 184, 179, 167.
 // 128 and 144 rows a slot, both two workgroups a compute unit: the higher one is for the experts just past 128 rows, whose last
 // rows cost a second expansion of all their weights. NVFP4, 512 experts (1024, 2688) 60 rows an expert 550 and 552, 73 rows 625 and 609, 88
-// rows 713 and 698, 172 rows 1199 and 1172; 200 experts (768, 1536) 56 rows 148.5 and 149.7, 66 rows 159.7 and 160.9, 77 rows 169.4 and
-// 168.4, 126 rows 214.0 and 214.7. Three-bit, 200 experts (2048, 512), even routing 75 rows 186.3 and 187.6, 90 rows 204.7 and
-// 205.6, 118 rows 237 and 235, 130 rows 275 and 249, 150 rows 316 and 303; skewed 90 rows 224 and 217, 130 rows 279 and 275.
-// From 256 rows an expert, with two and more full slots each, 128 again: the higher ones are measured to 172 rows.
+// rows 713 and 698, 172 rows 1199 and 1172; 128 experts (1024, 2688) 256 rows 416 and 386, 400 rows 633 and 597, 1408 rows 1998 and
+// 1928; blocks of 130 to 400 rows an expert, seventeen sizes, 0.956 to 1.022 times as long with the higher ones, 0.977 on average.
+// Three-bit, 200 experts (2048, 512), even routing 75 rows 186.3 and 187.6, 90 rows 204.7 and 205.6, 130 rows 275 and 249, 150 rows 316 and
+// 303, skewed 90 rows 224 and 217; 64 experts 352 rows 204 and 192, 1000 rows 495 and 480, 1408 rows 696 and 678; 96 experts (2560, 768) 512
+// rows 626 and 631, 400 rows 530 and 493.
+// Where slots of 128 rows all run at once (two workgroups on each of 256 compute units), higher ones only make each of them longer, but
+// for the experts that one of them holds: fourteen shapes of both formats, 145 to 1000 rows an expert, 1.02 times as long with the
+// higher ones on average (64 experts (1024, 256) 330 rows 85.2 and 87.5; 32 experts (2048, 512) 290 rows 110.5 and 114.4), 0.97 past one round.
+// And more, lower slots start more workgroups: the three-bit format's 80 rows serve up to 60 rows an expert there (128 experts (2048,
+// 512) 56 rows 99 and, of 128 rows, 102, 64 rows 115 and 102) and up to 72 elsewhere (512 experts (2048, 512), even and skewed, 68 rows 332, 346
+// and 380, 396, 76 rows 379, 365; 180 experts (1664, 384) 72 rows 110, 119 and 117, 122; 256 experts (2560, 768) 72 rows 317, 319 and 350, 364).
 constexpr int PANEL_SLOT_TILES = 9;      // at most
-constexpr int PANEL_REFUSED_ROWS = 128;  // calls of more than PANEL_MAX_SLOTS slots are refused; of higher slots, as many rows as of these
+constexpr int PANEL_REFUSED_ROWS = 128;  // calls of more than MAX_SLOTS slots are refused; of higher slots, as many rows as of these
 constexpr int64_t PANEL_MAX_SLOTS = 65535;
+// pairs / named: the rows an expert; `experts` of the `named` are here, whose fc1 has n_blocks blocks.
 template <class Fmt>
-inline int panel_height(int64_t pairs, int64_t named, int experts, int shared_rows) {
-  const int tiles = pairs < Fmt::LOW_ROWS * named ? 3 : pairs < Fmt::MIDDLE_ROWS * named ? 5 : pairs < Fmt::HIGH_ROWS * named || pairs >= 256 * named ? 8 : PANEL_SLOT_TILES;
+inline int panel_height(int64_t pairs, int64_t named, int experts, int shared_rows, int n_blocks) {
+  constexpr int AT_ONCE = 2 * 256;  // workgroups of 128-row slots, one a slot and four blocks
+  const int64_t rows = pairs * experts / named + shared_rows, slots = rows / 128 + experts / 2;  // (half a slot an expert is not full)
+  const bool at_once = slots * ((n_blocks + 3) / 4) <= AT_ONCE;
+  const int tiles = pairs < Fmt::LOW_ROWS * named                                            ? 3
+                    : pairs < (at_once ? Fmt::MIDDLE_ROWS : Fmt::MIDDLE_ROWS_LARGE) * named  ? 5
+                    : pairs < Fmt::HIGH_ROWS * named || (at_once && pairs > 144 * named)     ? 8
+                                                                                             : PANEL_SLOT_TILES;
   // the ids may all lie here, whatever share of the experts this is: a call that low slots would have refused takes higher ones
   return tiles < 8 && moe_max_slots(pairs, experts, shared_rows, 16 * tiles) > PANEL_MAX_SLOTS ? 8 : tiles;
 }

@@ -1089,7 +1089,7 @@ struct TileW3 {
   // routing of 10 of 512 experts (2048, 512), where 218 of 377 slots are such: the layer of 1024 rows 205 -> 187 us, 1543
   // 251 -> 234, 2048 296 -> 271; even routing at the same sizes unchanged. A ring of four slots with the activations as far
   // ahead gave nothing: what the wavefronts wait for is each other's issue slots.
-  static constexpr int LOW_ROWS = 22, MIDDLE_ROWS = 60, HIGH_ROWS = 88;  // panel_height's lines
+  static constexpr int LOW_ROWS = 22, MIDDLE_ROWS = 60, MIDDLE_ROWS_LARGE = 72, HIGH_ROWS = 88;  // panel_height's lines
   static constexpr int LIGHT_ROWS = ROWS_PER_SLOT;
   template <int EPI>
   static __device__ __forceinline__ void light(const StreamParams& p, const Slot& sl, int group, uint8_t* lds) {
@@ -1383,7 +1383,7 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   const bool dense = !e4m3 && panel_takes(m, ex->hidden) && panel_takes(pairs + shared_rows, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
                      (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && (pairs >= (ex->experts < named ? 48 : 32) * named || (pairs >= 16 * named && local * expert_blocks >= 650000) ||
                                                                                         (pairs >= 10 * named && local * expert_blocks >= 1400000))));
-  const int tiles = panel_height<TileW3<3>>(pairs, named, ex->experts, shared_rows), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
+  const int tiles = panel_height<TileW3<3>>(pairs, named, ex->experts, shared_rows, (ex->gated ? 2 : 1) * ex->inter / W3_BLOCK_ROWS), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
   // Under a budget the table ends behind the experts the selection can name: the launches' grids reach over all of it, and a
   // workgroup without rows is not free (40 rows of 10, a cap of 60 of 512 experts: 53.5 us before, 53.2 so). What a call of
   // these pairs is refused for, and how its launches split K, go by the whole table: the bits of the same ids without a budget.

@@ -88,6 +88,38 @@ def test_w3_calls_from_sixteen_rows_an_expert(m, panel):
     assert not torch.equal(by_panel, by_stream) and torch.equal(got, by_panel if panel else by_stream)
 
 
+def _most_rows(ex, m, x, topk=1):
+    """The rows of the highest slot of the plan that the last call left in its workspace."""
+    from hibana_amd import _lib
+    torch.cuda.synchronize()
+    head = _lib.workspace(x.cuda().device, 0).view(torch.int32)[:16 + 4 * (m * topk + 4096)].cpu()
+    return int(head[16:16 + 4 * int(head[0])].view(-1, 4)[:, 2].max())
+
+
+# rows an expert and the slots' height: 144 rows past the lines of the lower ones, however many, except where slots of 128 rows all
+# run at once (two workgroups on each of 256 compute units) and 144 hold no whole expert; the three-bit format's 80 rows serve up to 60
+# rows an expert at once and up to 72 past one round
+@pytest.mark.parametrize("fmt,experts,inter,rows,height", [
+    ("w3", 40, 512, 140, 144), ("w3", 40, 512, 150, 128), ("w3", 40, 1536, 150, 144), ("w3", 40, 1536, 250, 144), ("w3", 40, 1536, 260, 144),
+    ("w3", 40, 1536, 700, 144), ("w3", 32, 128, 300, 128), ("w3", 40, 2048, 71, 80), ("w3", 40, 2048, 73, 128), ("w3", 40, 512, 59, 80),
+    ("w3", 40, 512, 61, 128), ("nvfp4", 40, 512, 140, 144), ("nvfp4", 40, 512, 150, 128), ("nvfp4", 40, 1536, 150, 144),
+    ("nvfp4", 40, 1536, 260, 144), ("nvfp4", 40, 2048, 45, 80), ("nvfp4", 40, 2048, 47, 128)])
+def test_height_by_the_rows_an_expert(fmt, experts, inter, rows, height):
+    from hibana_amd import _lib, synthetic
+    from hibana_amd.kernels import w3_moe
+    ex = synthetic.w3_experts(experts, 128, inter, True, 3) if fmt == "w3" else synthetic.nvfp4_experts(experts, 128, 2 * inter, 3)
+    counts = [2 * rows] + [rows] * (experts - 2)
+    m, ids, g = _call(counts, rows)
+    x, ones = torch.randn(m, 128, generator=g).bfloat16().cuda(), torch.ones(m, 1, device="cuda")
+    key = b"w3_tile" if fmt == "w3" else b"nvfp4_tile"
+    assert _lib.lib().hb_tune(key, 1) == 0
+    try:
+        w3_moe.w3_moe(ex, x, ids.cuda(), ones) if fmt == "w3" else ex(x, ids.cuda(), ones)
+    finally:
+        _lib.lib().hb_tune(key, 0)
+    assert _most_rows(ex, m, x) == min(height, 2 * rows)
+
+
 @pytest.mark.parametrize("fmt", ["w3", "nvfp4"])
 def test_low_slots_refuse_nothing(fmt):
     """Ids that all lie in a small share of the experts: 3.3 million pairs are more slots of 48 rows than a call may have, and fewer

@@ -739,14 +739,20 @@ extern "C" int hb_nvfp4_dequant(const void* tiled, float global_scale, int64_t r
 }
 
 // The weight stream passes over the matrix once for every sixteen rows; the panel kernel expands it once for 128, and is the
-// faster one past sixteen rows except where K is long, the blocks are few and its cut gives no tile's K to several
-// workgroups: the stream splits K sixteen ways in a workgroup where the panel has eight, and its passes run side by side as
-// long as all of them fit the device at once. Measured, stream and panel, us: 2048 x 5120 17 rows 13.2 and 15.4, 64 rows 13.0
-// and 15.2; 5120 x 5120 (80 blocks) 48 rows (240 workgroups) 13.8 and 15.7, 64 rows (320) 22.3 and 13.6; 512 x 3072 (24 chunks)
-// 33 rows 10.0 and 10.9, 64 rows 11.2 and 10.8; 512 x 12800 17 rows 23.2 and, with K shared, 13.4, without 33.2.
-constexpr int STREAM_LONG_CHUNKS = 32, STREAM_PASSES_WORKGROUPS = 256;
+// faster one past sixteen rows except on few blocks. Measured, stream and panel, replayed graphs, us:
+// - Up to FP4_PARTS_BLOCKS blocks times passes, whose workgroups share each block's tiles (nvfp4_part_kernel), the stream is the faster
+//   one: 64 blocks x 8 chunks 32 rows 4.5 and 6.2, x 16 17 rows 5.8 and 8.7, x 40 10.0 and 16.0; 16 blocks x 24 128 rows 6.9 and 10.9; 8 blocks x
+//   64 256 rows 13.7 and 18.6. Past 64 chunks the panel's cut with K shared among workgroups takes over (8 blocks x 100 17 rows 15.8 and
+//   13.2, 64 blocks x 160 17 rows 33.1 and 26.1). Fewer than eight blocks leave compute dies idle, whose L2s would serve the rows of many passes: one
+//   block x 24 128 rows 6.2 and 10.6, 500 rows 18.4 and 10.8; x 48 128 rows 9.2 and 9.7, x 64 11.1 and 10.8.
+// - Up to 256, whole blocks a workgroup, where K is long and the cut shares no tile's K: the stream splits K sixteen ways in a workgroup
+//   where the panel has eight. 32 blocks x 32 chunks 128 rows 11.2 and 13.6, x 28 12.6 and 12.3, x 16 8.7 and 8.6, x 8 8.8 and 6.1; 80 blocks x 40
+//   48 rows (240 workgroups) 13.8 and 15.7, 64 rows (320) 22.3 and 13.6.
+constexpr int STREAM_LONG_CHUNKS = 32, STREAM_PASSES_WORKGROUPS = 256, DIES = 8;
 static bool stream_serves(int m, int n_blocks, int chunks, const PanelPlan& cut) {
-  return cut.kz == 1 && chunks >= STREAM_LONG_CHUNKS && (int64_t)n_blocks * ((m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT) <= STREAM_PASSES_WORKGROUPS;
+  const int64_t passes = (m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT;
+  if (n_blocks * passes <= FP4_PARTS_BLOCKS && (n_blocks >= DIES ? chunks <= 64 : chunks <= 48 && passes <= 8)) return true;
+  return cut.kz == 1 && chunks >= STREAM_LONG_CHUNKS && n_blocks * passes <= STREAM_PASSES_WORKGROUPS;
 }
 static PanelForce nvfp4_force() { return PanelForce{g_nvfp4_ksplit, g_nvfp4_nbw, g_nvfp4_tile_ks}; }
 
@@ -788,7 +794,9 @@ extern "C" size_t hb_nvfp4_gemm_workspace_bytes(int m, int n, int k) {
 
 extern "C" size_t hb_nvfp4_gemm_room_bytes(int m, int n, int k) {
   if (m <= ROWS_PER_SLOT || n <= 0 || k <= 0 || n % 64 || k % 128) return 0;
-  return panel_room(cut_panel<TileNvfp4>(m, n / 64, k / 128, PANEL_ANY_ROOM, nvfp4_force()));
+  const PanelForce force = nvfp4_force();
+  const PanelPlan cut = cut_panel<TileNvfp4>(m, n / 64, k / 128, PANEL_ANY_ROOM, force);
+  return g_nvfp4_tile == 0 && !force.ks && !force.kz && stream_serves(m, n / 64, k / 128, cut) ? 0 : panel_room(cut);
 }
 
 extern "C" int hb_nvfp4_gemm_ws(const void* x, int m, const void* tiled, float global_scale, int n, int k, int relu2, void* y, void* workspace,

@@ -39,3 +39,36 @@ def test_which_kernel_serves_a_call(n, k, m, room, relu2, stream):
     want = (x.float() @ lin.dequantize().T).bfloat16().float()
     mx, nr = errors(got, torch.relu(want) ** 2 if relu2 else want)
     assert mx < MAX_REL and nr < (2 * NORM_REL if relu2 else NORM_REL), (mx, nr)  # the square doubles a relative error
+
+
+@pytest.mark.parametrize("n,k,m,room,stream", [
+    (1024, 2048, 128, True, True), (1024, 3072, 129, True, False),                                      # 128 blocks x passes, shared tiles; past them
+    (4096, 3072, 32, True, True),
+    (512, 8192, 64, True, True), (512, 8192, 64, False, True), (512, 8320, 64, True, False),            # K up to 64 chunks, with room and without
+    (448, 6144, 128, True, True), (448, 6144, 129, True, False), (448, 6272, 64, True, False),          # fewer blocks than dies: eight passes, 48 chunks
+])
+def test_which_kernel_serves_a_call_of_few_blocks(n, k, m, room, stream):
+    test_which_kernel_serves_a_call(n, k, m, room, 0, stream)
+
+
+@pytest.mark.parametrize("n,k,m", [(4096, 1536, 17), (4096, 3072, 32), (2112, 3200, 48), (1024, 2048, 33), (576, 640, 40), (8192, 512, 9), (2048, 5120, 12),
+                                   (4160, 1152, 8), (1024, 4096, 3), (64, 128, 1)])
+def test_shared_tiles_add_as_one_workgroup_does(n, k, m):
+    """A block's tiles on two or four workgroups (one slot and several) against the same K split in one: the same bits."""
+    from hibana_amd import _lib, synthetic
+    from hibana_amd.kernels import ops
+    lib = _lib.lib()
+    lin = synthetic.nvfp4_linear(n, k, n + k, global_scale=0.02)
+    x = torch.randn(m, k, generator=torch.Generator().manual_seed(m)).bfloat16().cuda()
+    split, most = 1, 16 if m > 8 and k // 128 >= 24 else 8
+    while 2 * split <= min(most, k // 128):
+        split *= 2
+    assert lib.hb_tune(b"nvfp4_tile", 2) == 0
+    try:
+        got = ops.nvfp4_linear(x, lin)
+        assert lib.hb_tune(b"nvfp4_ksplit", split) == 0
+        want = ops.nvfp4_linear(x, lin)
+    finally:
+        lib.hb_tune(b"nvfp4_tile", 0)
+        lib.hb_tune(b"nvfp4_ksplit", 0)
+    assert torch.equal(got, want)

@@ -135,3 +135,14 @@ def test_routed_slots_around_whole_row_tiles(gated, mode, shift):
     mx, nr = errors(out[shift:shift + m * hidden].view(m, hidden), want)
     assert mx < MAX_REL and nr < NORM_REL, (mx, nr)
     assert bool((out[:shift] == 7).all()) and bool((out[shift + m * hidden:] == 7).all())
+
+
+@pytest.mark.parametrize("n,k", [(64, 128), (192, 640), (576, 1280), (320, 6400)])
+def test_nvfp4_rows_around_whole_tiles_on_the_panel(n, k):
+    """The same with the panel kernel for every size (few blocks are the weight stream's otherwise)."""
+    from hibana_amd import _lib
+    assert _lib.lib().hb_tune(b"nvfp4_tile", 1) == 0
+    try:
+        test_nvfp4_rows_around_whole_tiles(n, k)
+    finally:
+        _lib.lib().hb_tune(b"nvfp4_tile", 0)

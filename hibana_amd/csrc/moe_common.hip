@@ -810,12 +810,15 @@ __global__ __launch_bounds__(256) void moe_combine_wide_kernel(CombineParams p) 
   *reinterpret_cast<u32x4_t*>(p.out + (int64_t)r * p.h + c) = out;
 }
 
-constexpr int64_t COMBINE_ROW_VALUES = 1 << 20;
 // A row a workgroup, sixteen bytes of a pair a thread and load, the gate's dot product once a row: combine_span's chain and dot
 // product, operation for operation: the same bits. There every span of 512 columns makes the dot product again, whose loads (12 KB
-// at 2048 columns) are as many as the span's own. Measured alone, rows of ten
-// pairs, 2048 columns, in spans and so, us: BF16 1024 rows 17.4 and 11.2, 1543 rows 24.2 and 15.6, 2048 rows 30.6 and 19.1; FP32 256 rows 7.4 and 8.2,
-// 512 rows 12.2 and 10.8, 1000 rows 19.4 and 17.0; 500 rows of six, 1280 columns, 6.8 and 7.9.
+// at 2048 columns) are as many as the span's own. Bound by the pairs' traffic (3.7 TB/s at 1543 rows of 2048 columns). Measured alone, in spans
+// and so, us, BF16, rows x pairs x columns: 1543 x 10 x 2048 22.8 and 15.3, x 1152 17.9 and 12.1, x 2304 (a second pass by 32 of 256 threads) 29.0
+// and 22.5, x 2560 30.2 and 23.5; without a gate 21.1 and 13.9. Not below two spans of few pairs nor in one: 1543 x 6 x 1024 10.8 and 11.4, x 10
+// x 1024 13.4 and 11.9, x 10 x 512 8.6 and 11.2. FP32 pairs, twice the registers and passes of the spans, only where four and more dot products
+// are saved: 512 x 10 x 2048 10.9 and 10.4, 700 x 10 x 2560 18.0 and 16.3, 1000 x 12 x 2304 29.4 and 27.1, but 400 x 10 x 2048 9.3 and 9.6, 512 x 6 x
+// 2048 8.7 and 9.2, 1000 x 6 x 1536 10.8 and 12.2, 700 x 10 x 2560 without a gate 14.2 and 15.9.
+constexpr int COMBINE_ROW_FLOAT_ROWS = 512, COMBINE_ROW_FLOAT_COLUMNS = 4 * 512;
 template <int B, bool BF16>
 __global__ __launch_bounds__(256) void moe_combine_row_kernel(CombineParams p) {
   constexpr int V = BF16 ? 8 : 4;  // columns a load
@@ -1318,10 +1321,12 @@ void moe_launch_combine(const CombineParams& c, hipStream_t stream) {
     HB_LAUNCH(moe_combine_wide_kernel<12>, dim3((unsigned)c.m, (unsigned)((c.h / 8 + threads - 1) / threads)), dim3((unsigned)threads), 0, stream, c);
     return;
   }
-  // ... and with a shared expert a row a workgroup, FP32 pairs from the size where the dot products' loads, not one workgroup's
-  // trips to memory, are what takes time
-  if (c.shared && (c.pairs_bf16 ? c.m >= MOE_WIDE_ROWS : (int64_t)c.m * c.h >= COMBINE_ROW_VALUES) && c.h % 8 == 0 && c.shared_stride % 8 == 0 && (c.pairs_bf16 != 0) == (c.shared_f32 == 0) &&
-      aligned(c.pairs, 16) && aligned(c.shared, 16) && aligned(c.out, 16)) {
+  // ... and with a shared expert a row a workgroup, by the lines that its comment measures
+  const bool many = c.topk > 8;
+  const bool row = c.pairs_bf16 ? c.m >= MOE_WIDE_ROWS && (c.h > 2 * COMBINE_SPAN || (c.h > COMBINE_SPAN && many))
+                                : c.m >= COMBINE_ROW_FLOAT_ROWS && c.h >= COMBINE_ROW_FLOAT_COLUMNS && many && c.gate_vec;
+  if (c.shared && row && c.h % 8 == 0 && c.shared_stride % 8 == 0 && (c.pairs_bf16 != 0) == (c.shared_f32 == 0) && aligned(c.pairs, 16) && aligned(c.shared, 16) &&
+      aligned(c.out, 16)) {
     if (c.pairs_bf16) {
       HB_LAUNCH((moe_combine_row_kernel<12, true>), dim3((unsigned)c.m), dim3(256), 0, stream, c);
     } else {

@@ -28,14 +28,31 @@ def test_bf16_pairs(m, topk, h, gated):
     assert torch.equal(got, torch.cat(parts))
 
 
+@pytest.mark.parametrize("gated", [True, False])
+@pytest.mark.parametrize("m,topk,h", [(1024, 8, 1024), (1024, 9, 1024), (1024, 8, 1032), (1030, 9, 512), (1030, 9, 520), (1024, 12, 2304), (1024, 13, 2560)])
+def test_bf16_pairs_around_the_lines(m, topk, h, gated):
+    """Widths and selections on both sides of the lines between the two forms, and widths whose last pass few threads take."""
+    test_bf16_pairs(m, topk, h, gated)
+
+
+@pytest.mark.parametrize("m,topk,hidden", [(511, 9, 2048), (512, 8, 2048), (512, 9, 2048), (512, 9, 1920), (513, 12, 2304), (530, 13, 2560), (512, 9, 3200)])
+def test_fp32_pairs_of_a_layer_around_the_lines(m, topk, hidden):
+    """Passes of 1024 columns that are partly used, and both sides of the lines."""
+    _layer_of_fp32_pairs(m, topk, hidden)
+
+
 @pytest.mark.parametrize("m,topk", [(512, 2), (520, 13)])  # the first size, 2048 columns, and one more batch
 def test_fp32_pairs_of_a_layer(m, topk):
+    _layer_of_fp32_pairs(m, topk, 2048)
+
+
+def _layer_of_fp32_pairs(m, topk, hidden):
     from hibana_amd import _lib
     from hibana_amd.kernels import ops, w3_moe
-    (ex, _), (sh, _) = random_experts(16, 2048, 128, True, 5), random_experts(1, 2048, 128, True, 6)
+    (ex, _), (sh, _) = random_experts(16, hidden, 128, True, 5), random_experts(1, hidden, 128, True, 6)
     g = torch.Generator().manual_seed(m)
     ids = torch.stack([torch.randperm(17, generator=g)[:topk] for _ in range(m)]).to(torch.int32).cuda()  # 16: no expert
-    x, weights, gate = torch.randn(m, 2048, generator=g).bfloat16().cuda(), torch.rand(m, topk, generator=g).cuda(), (torch.randn(2048, generator=g) * 0.02).cuda()
+    x, weights, gate = torch.randn(m, hidden, generator=g).bfloat16().cuda(), torch.rand(m, topk, generator=g).cuda(), (torch.randn(hidden, generator=g) * 0.02).cuda()
     assert _lib.lib().hb_tune(b"w3_tile", 1) == 0
     try:
         got = w3_moe.moe_layer(ex, x, ids, weights, shared=sh, gate_vec=gate)

@@ -14,26 +14,37 @@ OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 REQUEST = re.compile(r"(buffer|global|flat)_(load|store|atomic)")  # (a spill is none: nothing may rest on one)
 
 
-def _kernels(folder):
-    """(name, [(address, instruction)]) of every three-bit stream kernel of the library."""
+def _kernels(folder, pattern=r"w3_(stream|part|fc\w+)_kernel"):
+    """(name, [(address, instruction)]) of every kernel of the library whose name matches: by default the three-bit streams'."""
     shutil.copy(_lib.LIBRARY, folder / "lib.so")
     subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=folder, check=True, capture_output=True)
     for part in sorted(p for p in os.listdir(folder) if "gfx950" in p):
         text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", part], cwd=folder, check=True, capture_output=True, text=True).stdout
         for name, code in re.findall(r"^[0-9a-f]+ <(\S+)>:\n((?:.+\n)*)", text, re.M):
-            if re.search(r"w3_(stream|part|fc\w+)_kernel", name):
+            if re.search(pattern, name):
                 yield name, [(int(at, 16), ins) for ins, at in re.findall(r"^\s+(\S.*?)\s*// ([0-9A-F]+):", code, re.M)]
 
 
-def _most_left_in_flight(code):
+def _skips_loads(code, i, to):
+    """Whether the branch at i leaves out a run of activation loads and nothing else (a block's next ones, on its last chunk)."""
+    left_out = [ins for _, ins in code[i + 1:to]]
+    requests = [ins for ins in left_out if REQUEST.match(ins)]
+    return bool(code[i][1].startswith("s_cbranch") and requests and len(left_out) < 40 and all("_load" in ins and not ins.endswith(" lds") for ins in requests)
+                and not any(ins.startswith(("s_branch", "s_cbranch", "ds_")) for ins in left_out))
+
+
+def _most_left_in_flight(code, loads_made=False):
     """For every wait of a ring's take: how many loads into LDS stand among the last requests that it leaves outstanding, over
-    all ways there, and how many loads a block has (as many as the take has reads)."""
+    all ways there, and how many loads a block has (as many as the take has reads). `loads_made`: not over the ways that leave out
+    the next chunk's activation loads, which a block takes on its last chunk only and no take follows."""
     place = {at: i for i, (at, _) in enumerate(code)}
     before = [[] for _ in code]
     for i, (at, ins) in enumerate(code):
         if ins.startswith(("s_branch", "s_cbranch")):
             words = int(ins.split()[1])
-            before[place[at + 4 + 4 * (words - 65536 if words >= 32768 else words)]].append(i)
+            to = place[at + 4 + 4 * (words - 65536 if words >= 32768 else words)]
+            if not (loads_made and _skips_loads(code, i, to)):
+                before[to].append(i)
         if not ins.startswith(("s_branch", "s_endpgm", "s_setpc")) and i + 1 < len(code):
             before[i + 1].append(i)
     for i, (_, ins) in enumerate(code[:-1]):
@@ -64,3 +75,25 @@ def test_a_wait_leaves_the_next_block_outstanding_and_no_more(tmp_path):
         assert takes and all(most <= reads for most, reads in takes), (name, takes)
         checked += 1
     assert checked >= 20, checked
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
+def test_light_slots_of_the_panel_kernel_wait_for_their_blocks(tmp_path):
+    """The same ring, of the slots that run on the weight stream's bodies inside the three-bit panel kernels."""
+    checked = 0
+    for name, code in _kernels(tmp_path, r"panel_tile_kernel.*TileW3"):
+        takes = list(_most_left_in_flight(code))
+        assert takes and all(most <= reads for most, reads in takes), (name, takes)
+        checked += 1
+    assert checked >= 12, checked
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
+def test_nvfp4_waits_leave_the_next_block_outstanding_and_no_more(tmp_path):
+    """The NVFP4 rings: a block's scales come in two loads and are read in one."""
+    checked = 0
+    for name, code in _kernels(tmp_path, r"nvfp4_(stream|part|twin)_kernel"):
+        takes = list(_most_left_in_flight(code, loads_made=True))
+        assert takes and all(most <= reads + 1 for most, reads in takes), (name, takes)
+        checked += 1
+    assert checked >= 12, checked

@@ -39,7 +39,7 @@ static void launch_route(const RouteParams& p, int m, hipStream_t stream) {
 constexpr int PLAN_THREADS = 1024;
 constexpr int PLAN_WAVES = PLAN_THREADS / 64;
 constexpr int PLAN_BATCH = 8;  // tiles of 64 pairs whose ids a wavefront requests at once
-constexpr int PLAN_WIDE_PAIRS = 8192;   // from this many pairs the plan is shared among workgroups (three launches)
+constexpr int PLAN_WIDE_PAIRS = 8192;   // from this many pairs they are counted by several workgroups in a launch of its own
 constexpr int PLAN_WIDE_GROUPS = 64;
 // Up to this many rows the plan workgroup routes them itself (one a wavefront): a row's selection is some 700 dependent
 // VALU instructions, so on ONE compute unit more than four rows take longer than a launch of their own over the device
@@ -426,10 +426,11 @@ __device__ __forceinline__ void plan_work(const int32_t* ids, int pairs, int e_l
 //
 // With `job.lanes` set the launch has further workgroups, which round the job's activations to E4M3 and plan nothing.
 //
-// Many pairs (a prefill chunk) are counted by `groups` workgroups into `wide` [groups, e_n] (phase 1; moe_place_kernel does the rest),
-// and very many, or ones with a rounding job, shared among them in three launches of this kernel, `wide` between them: phase 1, each group counts its share of the pairs per expert; phase 2, one workgroup adds the groups'
-// counts, writes the slot table and turns `wide` into the first sorted position of each group's run of each expert;
-// phase 3, each group places its share. Phase 0 is all of it in one workgroup.
+// Many pairs (a prefill chunk) are counted by `groups` workgroups into `wide` [groups, e_n] (phase 1), and moe_place_kernel does the rest.
+// Very many (more shares than PLAN_WIDE_GROUPS), or many with a rounding job, take three launches of this kernel, `wide` between them:
+// phase 1, each group counts its share of the pairs per expert; phase 2, one workgroup adds the groups' counts, writes the slot table and
+// turns `wide` into the first sorted position of each group's run of each expert; phase 3, each group places its share. Phase 0 is all of
+// it in one workgroup.
 template <bool WIDE>
 __global__ __launch_bounds__(PLAN_THREADS) void moe_plan_kernel(const int32_t* ids, int pairs, int e_lo, int e_n, int shared_rows,
                                                                 int32_t* __restrict__ plan, int32_t* __restrict__ order, RouteParams route,
@@ -462,6 +463,8 @@ __global__ __launch_bounds__(PLAN_THREADS) void moe_plan_kernel(const int32_t* i
 // routing launch and this one 5.4 + 5.9 and 6.2 + 7.2); alone 14.4 us at 5632 pairs; count, scan and place as three launches 19.2 us at
 // 15430 pairs, 19.8 at 45056 (count and this 12.2 and 14.7).
 constexpr int PLACE_SHARE = 256, PLACE_TABLE_SHARE = PLAN_THREADS;
+// Of at most PLACE_TABLE_SHARE pairs a counting workgroup, plan_work's segments are 64 pairs a wavefront: what it counts is that share.
+static_assert(PLACE_TABLE_SHARE == 64 * PLAN_WAVES, "the counting workgroups' shares are the placing ones'");
 template <bool TABLE>
 __global__ __launch_bounds__(PLAN_THREADS) void moe_place_kernel(const int32_t* __restrict__ ids, int pairs, int e_lo, int e_n, int shared_rows,
                                                                  int32_t* __restrict__ plan, int32_t* __restrict__ order, int slot_rows, int slot_cap,
@@ -630,7 +633,7 @@ __global__ __launch_bounds__(PLAN_THREADS) void moe_route_plan_kernel(const int3
 // wavefront), and the last of them to finish selects and plans, as in the routing launch above: candidates and ids go through
 // to memory, are waited for ahead of the ticket or the plan, and are read past the L2. (A rank launch of its own before it:
 // 5.0 + 13.0 us at 40 rows of 512 experts, the whole layer 50.4 us and 48.7 so.) `PLAN`: false leaves the plan to launches of
-// its own (a call of more pairs than one workgroup plans). `by_rows`: no row names an expert twice and they are at most
+// its own (more rows than plan_by_rows takes and PLACE_PAIRS pairs or more). `by_rows`: no row names an expert twice and they are at most
 // PLAN_ROWS_MAX; each group ranks one.
 template <int PER, bool PLAN>
 __global__ __launch_bounds__(PLAN_THREADS) void moe_budget_plan_kernel(BudgetParams q, int copies_n, int e_lo, int e_n, int shared_rows,
@@ -1125,7 +1128,9 @@ int moe_tune(const char* key, int value) {
 }
 
 // From this many pairs: the layer of 65 and 80 rows of ten took 66.5 and 71.8 us with one workgroup, 67.1 and 72.5 in shares, of 128
-// rows 80.8 and 77.9, of 256 rows 113.6 and 108.8; a latent block of 64 rows of 22 283 and 278.
+// rows 80.8 and 77.9, of 256 rows 113.6 and 108.8; a latent block of 64 rows of 22 283 and 278. Under a budget (the plan behind the selection in
+// its launch, and in shares): 96 rows of ten 74.7 and 75.0, 104 79.9 and 79.0, 128 83.3 and 82.4, 400 157.3 and 151.7; of 96 experts (1024, 256) 104
+// rows 50.2 and 50.5, 128 52.8 and 52.9, 256 74.0 and 72.3.
 constexpr int64_t PLACE_PAIRS = 1024;
 static unsigned plan_groups(const QuantJob* job) {
   if (!job) return 1u;
@@ -1169,8 +1174,9 @@ int moe_launch_plan(const int32_t* ids, int64_t pairs, int e_lo, int e_n, int sh
 int moe_check_route(int m, int e, int k) { return m <= 0 || e <= 0 || k <= 0 || k > e || k > 64 || e > 64 * ROUTE_PER_LANE ? HB_EINVAL : HB_OK; }
 
 // From more rows than compute units a workgroup routes several: each is a full one, of which a compute unit holds two, and all
-// draw tickets from one counter (800 rows of 512 experts, the whole layer 272.0 us with a row each, 263.7 with eight, 265.3 with
-// sixteen; 400 rows 169.7, 167.5, 168.9; at 200 rows and fewer no gain).
+// draw tickets from one counter. So many rows come here with E4M3 activations (whose rounding rides in the launch) or few selections: the
+// E4M3 layer of 512 experts, rows of ten, a row, eight and sixteen rows a workgroup, 300 rows 206.1, 201.5 and 202.4 us, 400 rows 223.0, 218.0
+// and 219.6, 800 rows 329.0, 317.9 and 318.1; weight-only, rows of three, 300 rows 138.9, 135.2 and 135.9.
 constexpr int ROUTE_GROUP_ROWS = 8, ROUTE_SPREAD_ROWS = 256;
 // Routing by `rp` (either rule) and the plan of its ids, in as few launches as the size allows.
 static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, int shared_rows, const MoeWorkspace& ws, hipStream_t stream, int slot_rows,

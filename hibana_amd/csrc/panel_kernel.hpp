@@ -30,8 +30,8 @@ constexpr int PANEL_LDS = 160 * 1024;
 constexpr int PANEL_MT = 8;          // row tiles of a dense call's slot, at most
 
 // The fewest blocks of a workgroup. A split's half chunk of activations is 2 mt pieces, brought by the split's wavefronts, one a
-// block, each of which holds its pieces' addresses in registers: eight at most, and four from seven row tiles on, where the
-// accumulators take most of them. (Whether a cut fits the LDS is panel_lds_bytes' to say.)
+// block, each of which holds its pieces' addresses in registers: eight at most, and four at seven and eight row tiles (five at a routed
+// slot's nine), where the accumulators take most of them. (Whether a cut fits the LDS is panel_lds_bytes' to say.)
 constexpr int panel_least_blocks(int mt) { return mt <= 4 ? 1 : mt <= 6 ? 2 : 4; }
 
 // A workgroup's part of the launch: its run of blocks, and where several workgroups share a tile's K (kz > 1), which
@@ -518,9 +518,9 @@ inline size_t panel_lds_bytes(int mt, int ks, int nbw) {
 }
 
 
-template <class Fmt, int EPI, int MT>  // as many row tiles as the slot's rows need, MT at most
+template <class Fmt, int EPI, int MT>  // as many row tiles as the slot's rows need, MT at most (light slots do not come here)
 __device__ __forceinline__ void panel_tiles(const StreamParams& p, const Slot& sl, uint8_t* lds, const PanelShare& part) {
-  if constexpr (MT > 1) {
+  if constexpr (MT > 1 + Fmt::LIGHT_ROWS / 16) {
     if ((sl.rows + 15) >> 4 < MT) return panel_tiles<Fmt, EPI, MT - 1>(p, sl, lds, part);
   }
   Panel<Fmt, EPI, MT> panel;

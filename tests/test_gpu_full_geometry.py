@@ -10,7 +10,7 @@
                  (tests/nemotron_reference.py:568-593 restated) is evaluated on a seeded sample of token rows; through
                  the panel kernel, the library's own choice and the weight stream.
 
-The 512-expert plan, the slot table at well over a hundred distinct experts, the three-launch plan of 45 056 pairs and
+The 512-expert plan, the slot table at well over a hundred distinct experts, the plan of 45 056 pairs in two launches and
 the stream / tile switch-over run here at the sizes they are built for.
 """
 import numpy as np

@@ -39,3 +39,19 @@ def test_shares_of_a_plan(experts, m, topk, base, count, shared):
     torch.cuda.synchronize()
     head, entries, slots, order = _read_plan(_lib.workspace(x.device, 0), w3_moe._struct(part), m, topk, shared)
     _check_plan(head, entries, slots, order, ids.numpy(), topk, base, count, m if shared else 0)
+
+
+@pytest.mark.parametrize("m,topk", [(1366, 6), (2731, 3), (5000, 4), (65537, 1), (1365, 6)])  # 8196, 8193, 20000, 65537 pairs; 8190, which one workgroup plans
+def test_three_launches_of_a_plan_beside_a_rounding_job(experts, m, topk):
+    """E4M3 activations are rounded by further workgroups: from 8192 pairs the plan is counted, scanned and placed in a launch each."""
+    from hibana_amd import _lib
+    from hibana_amd.kernels import w3_moe
+    ex, sh = experts
+    g = torch.Generator().manual_seed(m)
+    ids = torch.randint(0, E + 2, (m, topk), generator=g).to(torch.int32)
+    ids[m // 3:m // 2] = 20
+    x, weights = torch.randn(m, 128, generator=g).bfloat16().cuda(), torch.rand(m, topk, generator=g).cuda()
+    w3_moe.moe_layer(ex, x, ids.cuda(), weights, shared=sh, e4m3=True)
+    torch.cuda.synchronize()
+    head, entries, slots, order = _read_plan(_lib.workspace(x.device, 0), w3_moe._struct(ex), m, topk, True)
+    _check_plan(head, entries, slots, order, ids.numpy(), topk, 0, E, m)

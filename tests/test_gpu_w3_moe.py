@@ -343,8 +343,8 @@ def test_one_launch_for_fc1_and_fc2_gives_the_bits_of_two(gated, m):
 
 @pytest.mark.parametrize("m", [819, 820, 2000])
 def test_plan_orders_many_pairs_on_the_device(gated, m):
-    """8,190 pairs (the last count one workgroup plans alone), 8,200 and 20,000 (shared among 8 and 19 workgroups in
-    three launches), sorted by the planning kernel itself, against the oracle."""
+    """8,190 pairs (the last count that every placing workgroup makes for itself), 8,200 and 20,000 (counted by 9 and 20 workgroups
+    in a launch of its own), sorted by the planning kernels themselves, against the oracle."""
     _check(*gated, *_inputs(m, TOPK, 1234 + m))
 
 

@@ -119,7 +119,8 @@ def test_plan_of_given_ids_with_an_expert_range(small, base, count):
 
 
 def test_plan_of_a_prefill_sized_call_three_launches():
-    """45 056 pairs (2048 rows x 22): the plan shared among workgroups (count / scan / place), slots of 128 rows."""
+    """45 056 pairs (2048 rows x 22): the plan shared among workgroups (count, then place; three launches are those of more than
+    65 536 pairs and of rounding jobs: tests/test_gpu_plan_shares.py), slots of 128 rows."""
     from hibana_amd import _lib
     from hibana_amd.kernels import w3_moe
     ex, _ = random_experts(32, 128, 128, False, 23)

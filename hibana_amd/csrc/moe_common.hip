@@ -41,10 +41,15 @@ constexpr int PLAN_WAVES = PLAN_THREADS / 64;
 constexpr int PLAN_BATCH = 8;  // tiles of 64 pairs whose ids a wavefront requests at once
 constexpr int PLAN_WIDE_PAIRS = 8192;   // from this many pairs they are counted by several workgroups in a launch of its own
 constexpr int PLAN_WIDE_GROUPS = 64;
-// Up to this many rows the plan workgroup routes them itself (one a wavefront): a row's selection is some 700 dependent
-// VALU instructions, so on ONE compute unit more than four rows take longer than a launch of their own over the device
-// (measured, whole layer: 22.1 against 22.5 us at one row, even at four, 50.7 against 46.8 us at sixteen).
+// Up to this many rows the plan's workgroup routes them itself (one a wavefront): no ticket, no second workgroup to wait for, but the
+// rows share one compute unit. The three-bit layer, rows of 10 of 512 experts, even and skewed routing, us, routed there and in workgroups
+// of their own (moe_route_plan_kernel): two rows 28.4, 27.6 and 28.7, 28.0; three 29.1, 28.5 and 29.9, 28.8; four 31.6, 29.1 and 32.1, 29.6;
+// five 34.3, 32.8 and 34.2, 32.8; the latent block, 22 of 512, two rows 63.1 and 63.8, four 81.6 and 82.6, five 91.8 and 91.0.
 constexpr int ROUTE_FUSED_ROWS = 4;
+// Up to this many pairs of such rows one wavefront plans, above them plan_by_rows: its steps go by the pairs. In the same order, one
+// wavefront and by rows: two rows of ten 28.4 and 28.1, 27.8 and 27.7, of 22 65.8 and 63.1; three of ten 30.4 and 29.1, 29.2 and 28.4; four 33.8
+// and 31.6, 30.4 and 29.1; of eight of 256 experts two 26.5 and 26.7, three 27.5 and 27.3.
+constexpr int ROUTE_FEW_PAIRS = 24;
 
 struct Scan3 {
   int a, b, c;
@@ -1206,7 +1211,7 @@ static int launch_route_plan(const RouteParams& rp, int m, int e_lo, int e_n, in
   }
   static_assert(ROUTE_FUSED_ROWS <= PLAN_WAVES, "a wavefront a row");
   HB_LAUNCH(moe_plan_kernel<false>, dim3(plan_groups(job)), dim3(PLAN_THREADS), plan_lds, stream, rp.ids, (int)pairs, e_lo, e_n, shared_rows, ws.plan, ws.order,
-            rp, m, by_rows && pairs > 64 /* up to 64 pairs one wavefront plans */, slot_rows, (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows),
+            rp, m, by_rows && pairs > ROUTE_FEW_PAIRS, slot_rows, (int)moe_max_slots(pairs, e_n, shared_rows, slot_rows),
             ws.plan_wide, 1, 0, job ? *job : QuantJob{});
   return HB_OK;
 }

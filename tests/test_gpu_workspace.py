@@ -97,6 +97,11 @@ def test_plan_of_a_routed_call_is_the_oracles(small, m, topk, route_plan):
     _check_plan(head, entries, slots, order, ids.cpu().numpy(), topk, 0, 64, m)
 
 
+@pytest.mark.parametrize("m,topk", [(3, 8), (5, 5), (3, 9), (4, 7), (4, 16), (4, 17)])  # 24 pairs, 25, ... 64, 68: up to four rows by one wavefront or by rows
+def test_plan_of_few_routed_pairs(small, m, topk):
+    test_plan_of_a_routed_call_is_the_oracles(small, m, topk, 0)
+
+
 @pytest.mark.parametrize("base,count", [(0, 64), (16, 32)])
 def test_plan_of_given_ids_with_an_expert_range(small, base, count):
     """hb_w3_moe on caller's ids (the general form; an expert named twice by a row; experts outside the rank's range)."""

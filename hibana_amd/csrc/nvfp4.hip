@@ -477,7 +477,7 @@ __global__ __launch_bounds__(1024) void nvfp4_stream_kernel(StreamParams p) {
 }
 
 // A dense call of a few slots whose blocks are fewer than half the compute units: PARTS workgroups a 64-row block and slot, each
-// its 4 / PARTS 16-row tiles and only those tiles' codes. The sums and their order are those of the one workgroup. What bounds the
+// its 4 / PARTS 16-row tiles and only those tiles' codes. The sums and their order are those of one workgroup with the same K split. What bounds the
 // undivided launch is the expansion on a part of the device, and a small one the loads of a whole block ahead of the first product.
 // Traced, one workgroup a block and so, us: one row 1024 x 1024 4.5 and 3.4, 4096 x 2048 5.9 and 4.4, 2048 x 5120 8.1 and 5.5, 8192 x
 // 5120 9.0 and 7.0; eight rows 1024 x 4096 8.3 and 6.0, 8192 x 1024 5.5 and 4.4, 4096 x 5120 10.2 and 7.1; twelve rows, K split eight ways

@@ -57,6 +57,7 @@ SIGNATURES = {
     "hb_w3_quant_groups": (_I, [_P, _L, _I, _P, _P, _P]),
     "hb_w3_quant_rows": (_I, [_P, _L, _I, _P, _P, _P]),
     "hb_w3_gemm_e4m3": (_I, [_P, _P, _I, _P, _P, _L, _I, _I, _I, _P, _P]),
+    "hb_w3_mlp": (_I, [_P, _I, _P, _P, _L, _I, _I, _I, _I, _P, _P, _L, _I, _I, _P, _Z, _P, _P]),
     "hb_w3_moe_workspace_bytes": (_Z, [_I, _I, _EX, _I]),
     "hb_w3_moe": (_I, [_EX, _P, _P, _P, _I, _I, _I, _P, _P, _Z, _P]),
     "hb_w3_moe_among": (_I, [_EX, _I, _P, _P, _P, _I, _I, _I, _P, _P, _Z, _P]),

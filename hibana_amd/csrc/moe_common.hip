@@ -1454,8 +1454,7 @@ __global__ __launch_bounds__(256) void silu_mul_quant_groups_kernel(const uint16
   for (int j = 0; j < 8; j++) {
     const float g = __uint_as_float((j & 1) ? g4[j >> 1] & 0xffff0000u : g4[j >> 1] << 16);
     const float u = __uint_as_float((j & 1) ? u4[j >> 1] & 0xffff0000u : u4[j >> 1] << 16);
-    const float silu = g / (1.0f + expf(-g));
-    v[j] = round_bf16(torch_chain ? round_bf16(silu) * u : silu * u);
+    v[j] = torch_chain ? silu_chain(g, u) : round_bf16(g / (1.0f + expf(-g)) * u);
   }
   float amax = 0.f;
 #pragma unroll

@@ -114,6 +114,9 @@ __device__ __forceinline__ float pair_hi(uint32_t u) { return __uint_as_float(u 
 // silu with the fast exponential and division: the result is rounded to BF16 right after (8 significant bits).
 __device__ __forceinline__ float silu(float g) { return __fdividef(g, 1.0f + __expf(-g)); }
 
+// silu(g) * u as the BF16 tensor expression rounds it: silu in FP32 (the exponential and the division as they are), to BF16, the product to BF16.
+__device__ __forceinline__ float silu_chain(float g, float u) { return round_bf16(round_bf16(g / (1.0f + expf(-g))) * u); }
+
 // What a workgroup needs to know about its slot (up to 16 activation rows of one expert, or of the dense matrix).
 struct Slot {
   int index;           // which slot of the table (or of the dense call)

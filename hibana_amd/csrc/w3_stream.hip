@@ -845,6 +845,100 @@ __global__ __launch_bounds__(1024) void w3_part_kernel(StreamParams p) {
   }
 }
 
+// The gate | up projection of a dense SwiGLU block of at most sixteen rows together with what its 3-bit down projection takes: silu(gate) * up
+// as the BF16 tensor expression rounds it, then E4M3 codes and a scale a 32-group (p.oq, p.oq_scale [rows, p.out_stride]).
+// A workgroup holds the 64-row block of gate rows and the block of up rows of the same 64 columns of h (PARTS 2: half of either's
+// tiles, 32 columns), K split p.ks ways each, so that a pair of values meets in the exchange of the K splits through LDS
+// and neither leaves the compute unit. The sums are those of the dense kernels at the same K split, in their order.
+template <bool FEW, int T0, int T1>
+__device__ __forceinline__ void gate_up_block(const StreamParams& p, const Slot& sl, int gate, int up, int column0, int lane, int wave, uint8_t* rings) {
+  constexpr int GROUPS = (T1 - T0) / 2, STRIDE = RING_BYTES / 4;  // 32-column groups of h
+  const int q = lane >> 4, r16 = lane & 15;
+  const WaveShare share = wave_share(p, wave);
+  const int nb = share.nbi ? up : gate;
+  // the row scales of what this lane will add up, asked for ahead of the chunks: FEW: lanes 0 .. 31 a group's gate rows, 32 .. 63 its
+  // up rows; else both tiles of both
+  float scale[GROUPS][4];
+#pragma unroll
+  for (int g = 0; g < GROUPS; g++) {
+    const int t = T0 + 2 * g;
+    if constexpr (FEW) {
+      scale[g][0] = sl.rs[(lane < 32 ? gate : up) * 64 + 16 * t + (lane & 31)];
+    } else {
+#pragma unroll
+      for (int j = 0; j < 4; j++) scale[g][j] = sl.rs[(j < 2 ? gate : up) * 64 + 16 * (t + (j & 1)) + r16];
+    }
+  }
+  f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0, acc2 = acc0, acc3 = acc0;
+  uint8_t* ring = rings + wave * RING_BYTES;
+  if constexpr (T1 - T0 == 4) {
+    if constexpr (FEW) {
+      stream_block<EPI_DENSE, FewActs, W3Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+    } else {
+      stream_block<EPI_DENSE, FullActs, W3Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+    }
+  } else if constexpr (FEW) {
+    stream_block<EPI_DENSE, FewActsPart<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+  } else {
+    stream_block<EPI_DENSE, FullActsPart<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+  }
+  const f32x4_t all[4] = {acc0, acc1, acc2, acc3};
+  float* first = reinterpret_cast<float*>(rings);
+  float* mine = first + wave * STRIDE;
+#pragma unroll
+  for (int t = T0; t < T1; t++)
+#pragma unroll
+    for (int r = 0; r < 4; r++) mine[(t * 4 + r) * 64 + lane] = all[t][r];
+  __syncthreads();
+  const float* const second = first + p.ks * STRIDE;  // the up block's splits
+  // a unit of work: accumulator register r of a group's tiles (FEW: row r of the slot)
+  for (int unit = wave; unit < (FEW ? sl.rows : min(4, sl.rows)) * GROUPS; unit += 2 * p.ks) {  // uniform
+    const int r = GROUPS == 2 ? unit >> 1 : unit, g = GROUPS == 2 ? unit & 1 : 0, t = T0 + 2 * g;
+    if constexpr (FEW) {
+      const float* at = (lane < 32 ? first : second) + ((t + (q & 1)) * 4 + r) * 64 + r16;
+      float v = 0.f;
+      for (int s = 0; s < p.ks; s++, at += STRIDE) v += (at[0] + at[16]) + (at[32] + at[48]);
+      const float y = through_bf16(v * (GROUPS == 2 && g ? scale[GROUPS - 1][0] : scale[0][0])), other = __shfl_xor(y, 32);
+      const float h = silu_chain(lane < 32 ? y : other, lane < 32 ? other : y);
+      float amax = row16_max(fabsf(h));
+      amax = fmaxf(amax, __shfl_xor(amax, 16));
+      if (lane < 32) store_quantized(p, r, column0 + 32 * g + lane, h, amax, lane == 0);
+    } else {
+      const int i = 4 * q + r;
+      float v[4] = {0.f, 0.f, 0.f, 0.f};
+      for (int s = 0; s < p.ks; s++) {
+        const int at = s * STRIDE + (t * 4 + r) * 64 + lane;
+        v[0] += first[at], v[1] += first[at + 256], v[2] += second[at], v[3] += second[at + 256];
+      }
+      if (i >= sl.rows) continue;  // whole rows of lanes
+#pragma unroll
+      for (int j = 0; j < 4; j++) v[j] = through_bf16(v[j] * (GROUPS == 2 && g ? scale[GROUPS - 1][j] : scale[0][j]));
+      const float h0 = silu_chain(v[0], v[2]), h1 = silu_chain(v[1], v[3]);
+      const float amax = row16_max(fmaxf(fabsf(h0), fabsf(h1)));
+      store_quantized(p, i, column0 + 32 * g + r16, h0, amax, r16 == 0);
+      store_quantized(p, i, column0 + 32 * g + 16 + r16, h1, amax, false);
+    }
+  }
+}
+// h's 64-column block b: its gate rows are block b (of the first half; `pair_blocks` > 0: gate and up alternate in runs of that many
+// blocks), its up rows the block that many further on.
+template <bool FEW, int PARTS>
+__global__ __launch_bounds__(1024) void w3_fc_gate_up_kernel(StreamParams p, int half_blocks, int pair_blocks) {
+  extern __shared__ __align__(16) uint8_t rings[];
+  const int die = blockIdx.x & 7, local = blockIdx.x >> 3, part = local % PARTS, b = PARTS == 1 ? (int)blockIdx.x : local / PARTS * 8 + die;
+  if (b >= half_blocks) return;
+  const int gate = pair_blocks ? b / pair_blocks * 2 * pair_blocks + b % pair_blocks : b, up = gate + (pair_blocks ? pair_blocks : half_blocks);
+  const Slot sl = slot_of<EPI_DENSE>(p, 0);
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if constexpr (PARTS == 1) {
+    gate_up_block<FEW, 0, 4>(p, sl, gate, up, 64 * b, lane, wave, rings);
+  } else if (part == 0) {
+    gate_up_block<FEW, 0, 2>(p, sl, gate, up, 64 * b, lane, wave, rings);
+  } else {
+    gate_up_block<FEW, 2, 4>(p, sl, gate, up, 64 * b + 32, lane, wave, rings);
+  }
+}
+
 // One token from its router logits: fc1 with the routing inside it, so that the call has no launch for routing and plan.
 // Every wavefront of the launch routes the row for itself (about three microseconds in which it could not have known
 // its expert anyway; the logits are 2 KB): lane s then holds selection s, slot s is that expert with the token's one
@@ -1342,6 +1436,79 @@ extern "C" int hb_w3_gemm_e4m3(const void* xq, const float* x_scale, int m, cons
   if (slots > 65535) return HB_EINVAL;
   if (int e = launch_stream<EPI_DENSE>(p, slots, slots, Launch{g_tune.w3_ksplit, g_tune.w3_nbw}, as_stream(stream), bits)) return e;
   return launch_status();
+}
+
+// The dense SwiGLU block on its 3-bit copies. Gate | up, the SiLU product and its E4M3 rounding are one launch up to sixteen rows
+// (w3_fc_gate_up_kernel), which keeps gate | up out of memory and costs two launches' starts and ends less: the block (5120, 25600) of four rows
+// 51.4 -> 45.9 us, (4096, 8192) of one and sixteen 18.9 -> 15.4 and 28.0 -> 26.5, (1024, 1024) of four 10.6 -> 8.2 (replayed graphs on cycled weights).
+// Its shape, by h's 64-column blocks B and the chunks of K; swept over 16 to 512 blocks, 8 to 40 chunks, one to sixteen rows, times of the three
+// launches (1.0):
+// - up to 128 blocks half of them a workgroup, K split four ways: 0.75 to 0.99; eight ways the same or worse. The gate | up of up
+//   to 64 blocks alone is dealt out by quarters of a block, and where K is long that weighs more: from 32 chunks 1.02 to 1.14 past four rows, 0.99
+//   to 1.02 of 32 blocks below, from 24 chunks and twelve rows 1.0 to 1.04 of 32 blocks;
+// - up to 256 whole blocks, four ways: 0.82 to 0.95 (halves 0.83 to 1.10);
+// - up to 384 halves, two ways: 0.83 to 0.97 up to four rows or below 20 chunks (whole blocks 0.88 to 1.05: some compute units hold two);
+//   up to eight rows below 32 chunks 0.95 to 0.96; else 1.02 to 1.13;
+// - past them whole blocks, two ways: 0.87 to 0.99 (four ways 0.87 to 1.01, eight 0.94 to 1.04).
+struct GateUpShape {
+  int parts, ks;  // parts 0: three launches
+};
+static GateUpShape gate_up_shape(int m, int blocks, int chunks) {
+  const bool few = m <= FEW_ROWS;
+  GateUpShape s{1, 2};
+  if (blocks <= 128) {
+    s = GateUpShape{2, 4};
+    if ((chunks >= 32 && blocks <= (few ? 32 : 64)) || (chunks >= 24 && m >= 12 && blocks <= 32)) s.parts = 0;
+  } else if (blocks <= 256) {
+    s = GateUpShape{1, 4};
+  } else if (blocks <= 384) {
+    s = GateUpShape{few || chunks < 20 || (m <= 8 && chunks < 32) ? 2 : 0, 2};
+  }
+  while (s.ks > 1 && (few ? 2 : 1) * s.ks > chunks) s.ks /= 2;  // a wavefront's start costs about two chunks of the four-row body
+  return s;
+}
+
+extern "C" int hb_w3_mlp(const void* x, int m, const void* gate_up, const float* gate_up_rows, int64_t gate_up_lut, int inter, int hidden, int gate_up_bits,
+                         int pairs, const void* down, const float* down_rows, int64_t down_lut, int n, int down_bits, void* scratch, size_t scratch_bytes, void* y,
+                         void* stream) {
+  if (!x || !gate_up || !gate_up_rows || !down || !down_rows || !scratch || !y) return HB_ENULL;
+  if (m <= 0 || inter <= 0 || hidden <= 0 || inter % W3_CHUNK || hidden % W3_CHUNK || pairs < 0 || (pairs && (pairs % 32 || inter % pairs))) return HB_EINVAL;
+  if (!aligned(x, 16) || !aligned(gate_up, 16) || !aligned(gate_up_rows, 4) || !aligned(scratch, 16)) return HB_EINVAL;
+  if (scratch_bytes < HB_W3_MLP_SCRATCH_BYTES((size_t)m, (size_t)inter)) return HB_EWORKSPACE;
+  uint8_t* hq = static_cast<uint8_t*>(scratch);
+  float* h_scale = reinterpret_cast<float*>(hq + (size_t)m * inter);
+  const int blocks = inter / W3_BLOCK_ROWS;
+  const GateUpShape shape = gate_up_shape(m, blocks, hidden / W3_CHUNK);
+  if (m <= ROWS_PER_SLOT && gate_up_bits == 3 && pairs % W3_BLOCK_ROWS == 0 && shape.parts && blocks <= 0xffffff) {
+    StreamParams p{};
+    p.w = static_cast<const uint8_t*>(gate_up);
+    p.rows = gate_up_rows;
+    p.lut_lo = (uint32_t)((uint64_t)gate_up_lut & 0xffffffffu);
+    p.lut_hi = (uint32_t)((uint64_t)gate_up_lut >> 32);
+    p.n_blocks = 2 * blocks;
+    p.chunks = hidden / W3_CHUNK;
+    p.a = static_cast<const uint16_t*>(x);
+    p.a_stride = hidden;
+    p.m = m;
+    p.oq = hq;
+    p.oq_scale = h_scale;
+    p.out_stride = inter;
+    p.nbw = 2;
+    p.ks = shape.ks;
+    set_split(p);
+    const dim3 grid((unsigned)(shape.parts == 1 ? blocks : (blocks + 7) / 8 * 8 * 2)), block(64 * 2 * p.ks);
+    auto launch = [&](auto kernel) { HB_LAUNCH(kernel, grid, block, (size_t)2 * p.ks * RING_BYTES, as_stream(stream), p, blocks, pairs / W3_BLOCK_ROWS); };
+    if (m <= FEW_ROWS) {
+      shape.parts == 1 ? launch(w3_fc_gate_up_kernel<true, 1>) : launch(w3_fc_gate_up_kernel<true, 2>);
+    } else {
+      shape.parts == 1 ? launch(w3_fc_gate_up_kernel<false, 1>) : launch(w3_fc_gate_up_kernel<false, 2>);
+    }
+  } else {
+    uint16_t* both = reinterpret_cast<uint16_t*>(hq + (size_t)m * inter / 8 * 9);
+    if (int e = hb_w3_gemm(x, m, gate_up, gate_up_rows, gate_up_lut, 2 * inter, hidden, gate_up_bits, both, stream)) return e;
+    if (int e = hb_silu_mul_quant_groups(both, m, inter, pairs, 1, hq, h_scale, stream)) return e;
+  }
+  return hb_w3_gemm_e4m3(hq, h_scale, m, down, down_rows, down_lut, n, inter, down_bits, y, stream);
 }
 
 // ------------------------------------------------------------------------------------------------ routed experts

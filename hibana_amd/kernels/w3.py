@@ -365,6 +365,34 @@ def w3_linear(x: torch.Tensor, w3: W3Weight, x_scale: torch.Tensor | None = None
     return y
 
 
+def w3_mlp_takes(x: torch.Tensor, gate_up: W3Weight, down: W3Weight) -> bool:
+    """Whether `w3_mlp` serves a SwiGLU block's call on these copies."""
+    return (x.dtype == torch.bfloat16 and x.ndim == 2 and 0 < x.shape[0] <= MAX_ROWS and x.shape[1] == gate_up.in_features
+            and gate_up.out_features == 2 * down.in_features)
+
+
+def w3_mlp(x: torch.Tensor, gate_up: W3Weight, down: W3Weight, pairs: int = 0) -> torch.Tensor:
+    """`w3_linear(*silu_mul_quant_groups(w3_linear(x, gate_up), pairs, torch_chain=True), down)` in one call; up to sixteen rows the SiLU
+    product and its E4M3 rounding are the first launch's epilogue (hibana/model/mlp.py:36-42)."""
+    if not w3_mlp_takes(x, gate_up, down):
+        raise ValueError("w3_mlp: unsupported call")
+    _lib.need_gpu(x)
+    for w in (gate_up, down):
+        if w.tiled is None or w.tile_bits != w.bits:
+            tile(w)
+    m, inter = x.shape[0], down.in_features
+    x = x.contiguous()
+    y = x.new_empty((m, down.out_features))
+    need = m * inter // 8 * 41  # HB_W3_MLP_SCRATCH_BYTES
+    scratch = x.new_empty((need,), dtype=torch.uint8)
+    code = _lib.lib().hb_w3_mlp(x.data_ptr(), m, gate_up.tiled.data_ptr(), gate_up.row_scale.data_ptr(), gate_up.lut, inter, gate_up.in_features,
+                                gate_up.tile_bits, pairs, down.tiled.data_ptr(), down.row_scale.data_ptr(), down.lut, down.out_features, down.tile_bits,
+                                scratch.data_ptr(), need, y.data_ptr(), _lib.stream())
+    if code:
+        _lib.check(code, "w3_mlp")
+    return y
+
+
 def _missing(linears):
     return [(name, lin) for name, lin in linears if getattr(lin, "w3", None) is None]
 

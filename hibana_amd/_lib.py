@@ -93,6 +93,8 @@ SIGNATURES = {
     "hb_nvfp4_moe_among": (_I, [_EX4, _I, _P, _P, _P, _I, _I, _I, _P, _P, _Z, _P]),
     "hb_latent_workspace_bytes": (_Z, [_LW, _I, _I]),
     "hb_latent_router": (_I, [_LW, _P, _I, _I, _P, _I, _I, _I, _P, _P, _P, _P, _P, _Z, _P]),
+    "hb_latent_layer_workspace_bytes": (_Z, [_LW, _I, _I]),
+    "hb_latent_layer": (_I, [_LW, _P, _I, _I, _P, _I, _I, _P, _P, _Z, _P]),
     "hb_latent_block": (_I, [_LW, _P, _P, _P, _P, _I, _I, _I, _P, _P, _Z, _P]),
     "hb_latent_shared_up": (_I, [_LW, _P, _I, _I, _P, _Z, _P]),
     "hb_latent_out": (_I, [_LW, _P, _I, _I, _P, _P, _Z, _P]),

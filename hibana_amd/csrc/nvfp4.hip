@@ -12,8 +12,10 @@
 #include <string.h>
 
 #include <atomic>
+#include <cmath>
 
 #include "panel_kernel.hpp"
+#include "plan.hpp"
 #include "ring.hpp"
 #include "stream_common.hpp"
 
@@ -404,18 +406,24 @@ struct Fp4Full {
     }
   }
   // One loop body for every chunk: the ring's slot by its parity, what is still to come by uniform branches.
-  __device__ __forceinline__ void run(const StreamParams& p, const Slot& sl, int nb, int c0, int c1, int lane, uint8_t* ring) {
+  template <class Wait>
+  __device__ __forceinline__ void run(const StreamParams& p, const Slot& sl, int nb, int c0, int c1, int lane, uint8_t* ring, Wait& wait) {
     const int n = c1 - c0;
     RingSource src;
     src.row = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(sl.w + (int64_t)nb * p.chunks * NVFP4_BLOCK_BYTES), 0, p.chunks * NVFP4_BLOCK_BYTES, 0x00020000);
     const lds_ptr_t slot0 = (lds_ptr_t)ring;
     uint32_t codes, scales;
     Ring::lanes(src, lane, lane & 15, (uint32_t)(uintptr_t)slot0, codes, scales);
+    wait.look();
     Ring::request(src, c0, slot0);
     asm volatile("" ::: "memory");
+    if constexpr (Wait::WAITS) {  // (the second block ahead of the first pieces, here: they are on their way together)
+      if (n > 1) Ring::request(src, c0 + 1, slot0 + NVFP4_BLOCK_BYTES);
+      if (!wait.done()) return;
+    }
     start(p, sl, c0, lane);
     asm volatile("" ::: "memory");
-    if (n > 1) Ring::request(src, c0 + 1, slot0 + NVFP4_BLOCK_BYTES);
+    if (!Wait::WAITS && n > 1) Ring::request(src, c0 + 1, slot0 + NVFP4_BLOCK_BYTES);
     for (int i = 0; i < n; i++) {
       const uint32_t slot = (i & 1) * NVFP4_BLOCK_BYTES;
       Fp4Chunk ch;
@@ -432,8 +440,8 @@ struct Fp4Full {
 
 // y = x Wq^T, dense or grouped by the expert plan: one wavefront per (64-row block, K range, slot of 16 activation rows),
 // the same launch shape, slot table, weight ring, K-split exchange and epilogues as the W3 stream.
-template <int EPI>
-__device__ __forceinline__ void nvfp4_workgroup(const StreamParams& p, int slot, int bx, uint8_t* rings) {
+template <int EPI, class Wait>
+__device__ __forceinline__ void nvfp4_workgroup(const StreamParams& p, int slot, int bx, uint8_t* rings, Wait& wait) {
   const Slot sl = slot_of<EPI>(p, slot);
   if (sl.rows <= 0) return;  // a slot the plan did not fill: the whole workgroup leaves
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the same in every lane: kept in scalars
@@ -445,7 +453,7 @@ __device__ __forceinline__ void nvfp4_workgroup(const StreamParams& p, int slot,
   if (active) {  // at least one chunk: the launch keeps ks <= chunks
     uint8_t* ring = rings + wave * FP4_RING_BYTES;
     if (sl.rows <= FP4_FEWER_ROWS && !p.no_few) {  // uniform over the workgroup
-      stream_block<EPI, Fp4Few4Acts<>, Fp4RingOf<0>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+      stream_block_behind<EPI, Fp4Few4Acts<>, Fp4RingOf<0>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3, wait);
       for (int d = 16; d <= 32; d *= 2) {  // the four blocks' sums: lane q = 0 now holds the slot's rows as the epilogue expects them
         add_lanes(acc0, d);
         add_lanes(acc1, d);
@@ -453,21 +461,30 @@ __device__ __forceinline__ void nvfp4_workgroup(const StreamParams& p, int slot,
         add_lanes(acc3, d);
       }
     } else if (sl.rows <= FP4_FEW_ROWS && !p.no_few) {
-      stream_block<EPI, Fp4Few8Acts<>, Fp4Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+      stream_block_behind<EPI, Fp4Few8Acts<>, Fp4Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3, wait);
       add_lanes(acc0, 32);  // the two parities': lanes q = 0, 1 hold slot rows 0 .. 7
       add_lanes(acc1, 32);
       add_lanes(acc2, 32);
       add_lanes(acc3, 32);
     } else {
       Fp4Full<EPI> full;
-      full.run(p, sl, nb, share.c0, share.c1, lane, ring);
+      full.run(p, sl, nb, share.c0, share.c1, lane, ring, wait);
       acc0 = full.acc[0];
       acc1 = full.acc[1];
       acc2 = full.acc[2];
       acc3 = full.acc[3];
     }
+  } else if (Wait::WAITS) {
+    wait.done();
   }
+  if (!wait.there) return;
   finish_block<EPI, false, FP4_RING_BYTES / 4>(p, sl, RowScales{}, nb, active, ks, nbi, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3);
+}
+
+template <int EPI>
+__device__ __forceinline__ void nvfp4_workgroup(const StreamParams& p, int slot, int bx, uint8_t* rings) {
+  NoWait none;
+  nvfp4_workgroup<EPI>(p, slot, bx, rings, none);
 }
 
 template <int EPI>
@@ -500,7 +517,8 @@ __device__ __forceinline__ void nvfp4_part_block(const StreamParams& p, const Sl
     for (int t = T0; t < T1; t++) add_lanes(acc[t], 32);
   } else {
     Fp4Full<EPI, T0, T1, Fp4RingPart<1, T0, T1>> full;
-    full.run(p, sl, nb, share.c0, share.c1, lane, ring);
+    NoWait none;
+    full.run(p, sl, nb, share.c0, share.c1, lane, ring, none);
 #pragma unroll
     for (int t = T0; t < T1; t++) acc[t] = full.acc[t];
   }
@@ -557,8 +575,129 @@ __global__ __launch_bounds__(1024) void nvfp4_twin_kernel(StreamParams a, Stream
   }
 }
 
+// fc1 and fc2 of a routed call on the stream in one launch, as w3_fc12_kernel: the same order of the grid, the same counters and waits. `first`:
+// the workgroups of a dense matrix beside them (a shared expert's down projection), which come ahead of all others and wait for nothing.
+template <int EPI1>
+__global__ __launch_bounds__(1024) void nvfp4_fc12_kernel(StreamParams p1, StreamParams p2, StreamParams b, int groups1, int groups2, int slots, int lag, int first) {
+  extern __shared__ __align__(16) uint8_t rings[];
+  __shared__ int outcome;
+  const int id = blockIdx.x;
+  if (id < first) {
+    nvfp4_workgroup<EPI_DENSE>(b, 0, id, rings);
+    return;
+  }
+  const Fc12Place at = fc12_place(id - first, groups1, groups2, slots, lag);
+  if (p1.plan[PLAN_HEADER + 4 * at.slot + 2] <= 0) return;  // a slot without rows
+  if (at.is_fc1) {
+    nvfp4_workgroup<EPI1>(p1, at.slot, at.index, rings);
+    fc12_arrive(p1, at.slot);
+  } else {
+    SlotWait wait(p2, at.slot, &outcome, false);
+    nvfp4_workgroup<EPI_FC2>(p2, at.slot, at.index, rings, wait);
+  }
+}
+
+// The product of a small latent block's router: at most sixteen rows, fused[m, n] = x [router; fc1_latent]^T in
+// FP32, its latent columns also rounded to BF16 (hibana/kernels/csrc/nemotron_moe.cu:496-558 of the reference).
+// The product is bound by how fast a compute unit brings its columns in, so a workgroup has eight of them only: the sixteen columns of a product's
+// weight operand are eight weight rows over two parts of K. PACKED (up to eight rows): the sixteen activation rows are likewise eight
+// over both parts, and of the result the two quarters where the parts agree are kept; else a product each. With the plan's launch below, the
+// block of 512 experts (1024, 2688) and a shared one of 5376, router and block as six launches and so, us: one row 53.2 and 49.0, four 80.0 and
+// 77.4, eight 110.9 and 108.5, nine 126.9 and 119.0, sixteen 165.4 and 162.7.
+constexpr int FRONT_WAVES = 8, FRONT_COLUMNS = 8;
+struct FrontGemv {
+  const uint16_t* w;  // BF16 [n, k]
+  const uint16_t* x;  // BF16 [m, k]
+  float* fused;       // FP32 [m, n]
+  uint16_t* lat;      // BF16 [m, n - e]
+  int n, k, m, e;
+};
+template <bool PACKED>
+__global__ __launch_bounds__(64 * FRONT_WAVES) void latent_front_kernel(FrontGemv g) {
+  __shared__ float part[FRONT_WAVES * 256];
+  const int n0 = blockIdx.x * FRONT_COLUMNS;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), q = lane >> 4, r16 = lane & 15, half = r16 >> 3;
+  const int per_part = g.k / (2 * FRONT_WAVES), steps = per_part / 32, k0 = 2 * wave * per_part;  // k % 512 == 0
+  const uint16_t* wat = g.w + (int64_t)min(n0 + (r16 & 7), g.n - 1) * g.k + k0 + half * per_part + 8 * q;
+  const uint16_t* xat = g.x + (int64_t)min(PACKED ? r16 & 7 : r16, g.m - 1) * g.k + k0 + (PACKED ? half * per_part : 0) + 8 * q;
+  f32x4_t lower = {0.f, 0.f, 0.f, 0.f}, upper = lower;
+  constexpr int BATCH = 8;
+  for (int s0 = 0; s0 < steps; s0 += BATCH) {
+    u32x4_t b[BATCH], a[BATCH], a2[BATCH];
+#pragma unroll
+    for (int j = 0; j < BATCH; j++)
+      if (s0 + j < steps) {
+        b[j] = *reinterpret_cast<const u32x4_t*>(wat + 32 * (s0 + j));
+        a[j] = *reinterpret_cast<const u32x4_t*>(xat + 32 * (s0 + j));
+        if (!PACKED) a2[j] = *reinterpret_cast<const u32x4_t*>(xat + per_part + 32 * (s0 + j));
+      }
+#pragma unroll
+    for (int j = 0; j < BATCH; j++)
+      if (s0 + j < steps) {
+        lower = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a[j]), __builtin_bit_cast(bf16x8_t, b[j]), lower, 0, 0, 0);
+        if (!PACKED) upper = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, a2[j]), __builtin_bit_cast(bf16x8_t, b[j]), upper, 0, 0, 0);
+      }
+  }
+  // part[wave][register][lane]; lane (q, r16) of register i: activation row 4 q + i (PACKED: of part (4 q + i) / 8), column r16 & 7 of part r16 / 8
+  const f32x4_t mine = PACKED || half == 0 ? lower : upper;
+#pragma unroll
+  for (int i = 0; i < 4; i++) part[(wave * 4 + i) * 64 + lane] = mine[i];
+  __syncthreads();
+  if (threadIdx.x < 16 * FRONT_COLUMNS) {
+    const int row = threadIdx.x >> 3, c = threadIdx.x & 7, n = n0 + c;
+    if (row < g.m && n < g.n) {
+      float sum = 0.f;
+      for (int w = 0; w < FRONT_WAVES; w++) {  // in the order of K
+        const float* at = part + (w * 4 + (row & 3)) * 64;
+        sum += at[16 * (row >> 2) + c];
+        sum += at[16 * ((row >> 2) + (PACKED ? 2 : 0)) + 8 + c];
+      }
+      g.fused[(int64_t)row * g.n + n] = sum;
+      if (n >= g.e) g.lat[(int64_t)row * (g.n - g.e) + n - g.e] = bf16_of(sum);
+    }
+  }
+}
+// The second launch: routing and plan of those rows - up to ROUTE_FUSED_ROWS of them by one workgroup, else a workgroup a row of which the
+// last to arrive plans, as moe_plan_kernel and moe_route_plan_kernel do it - and beside them, in the workgroups past `groups`, the shared
+// expert's up projection, which needs nothing of the routing: the plan leaves the memory and all but a few compute units idle.
+template <bool MANY>
+__global__ __launch_bounds__(PLAN_THREADS) void latent_plan_kernel(RouteParams route, int rows, int by_rows, int e_lo, int e_n, int32_t* __restrict__ plan,
+                                                                   int32_t* __restrict__ order, int slot_cap, int groups, StreamParams up) {
+  extern __shared__ __align__(16) uint8_t rings[];
+  int* lds = reinterpret_cast<int*>(rings);
+  if ((int)blockIdx.x >= groups) {
+    nvfp4_workgroup<EPI_DENSE_RELU2>(up, 0, blockIdx.x - groups, rings);
+    return;
+  }
+  const int wave = threadIdx.x >> 6;
+  bool cleared = false;
+  if constexpr (MANY) {
+    __shared__ int last;
+    if (wave == 0) {
+      route_any(route, blockIdx.x, threadIdx.x);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this row's ids (write-through stores) have reached memory before the ticket is drawn
+    } else if (by_rows) {
+      constexpr int IDLE = PLAN_THREADS - 64;
+      clear_plan(plan, slot_cap, blockIdx.x * IDLE + (int)threadIdx.x - 64, groups * IDLE);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) last = last_to_arrive(plan, groups);
+    __syncthreads();
+    if (!last) return;
+    cleared = true;
+  } else {
+    if (wave < rows) route_any(route, wave, threadIdx.x & 63);
+    __syncthreads();
+  }
+  if (by_rows) {
+    plan_by_rows(route.ids, rows, route.k, e_lo, e_n, 0, plan, order, ROWS_PER_SLOT, slot_cap, lds, cleared);
+  } else {
+    plan_work<false>(route.ids, rows * route.k, e_lo, e_n, 0, plan, order, ROWS_PER_SLOT, slot_cap, nullptr, 1, 0, 0, lds);
+  }
+}
+
 // experiments (hb_tune): the stream's workgroup shape ("nvfp4_ksplit", "nvfp4_nbw"); "nvfp4_tile": 1 forces the panel kernel, 2 the stream
-static std::atomic<int> g_nvfp4_ksplit{0}, g_nvfp4_nbw{0}, g_nvfp4_tile{0}, g_nvfp4_few{0}, g_nvfp4_tile_ks{0};  // "nvfp4_few": 2 switches off the body for slots of at most eight rows; "nvfp4_tile_ks": the workgroups that share a tile's K
+static std::atomic<int> g_nvfp4_ksplit{0}, g_nvfp4_nbw{0}, g_nvfp4_tile{0}, g_nvfp4_few{0}, g_nvfp4_tile_ks{0}, g_nvfp4_lag{0}, g_nvfp4_fused{0};  // "nvfp4_fused": 1 runs fc1 and fc2 of a routed call on the stream in one launch, 2 in two; "nvfp4_lag": eighths of the slots fc2 is behind there; "nvfp4_few": 2 switches off the body for slots of at most eight rows; "nvfp4_tile_ks": the workgroups that share a tile's K
 
 static int shape_nvfp4(StreamParams& p, int64_t busy_slots) {
   pick_shape(p.n_blocks, p.chunks, busy_slots, 4096, &p.ks, &p.nbw);
@@ -642,6 +781,88 @@ static int launch_twin(StreamParams& a, int64_t slots_a, int64_t busy_a, StreamP
   if (all > 0x7fffffff) return HB_EINVAL;
   const int waves = std::max(a.ks * a.nbw, b.ks * b.nbw);
   HB_LAUNCH((nvfp4_twin_kernel<EPI_A, EPI_B>), dim3((unsigned)all), dim3(64 * waves), (size_t)waves * FP4_RING_BYTES, stream, a, b, groups_a, groups_b, (int)first);
+  return HB_OK;
+}
+
+// Whether the two layers share a launch. The one launch fills the compute units that a round of fc1's workgroups leaves idle when it
+// ends, and pays for it with a trip of h's arrival counters through memory, about a microsecond longer than the boundary between
+// two launches. So it needs about as many wavefronts as the device holds (4096), or a quarter of that where a wavefront has four chunks and more, and it
+// loses again over many rounds of slots of unequal length (the order of the grid then holds fc2 back). Measured, the two launches and the one, replayed
+// graphs of calls with changing routing, us, experts (latent, inter) and pairs:
+// - too few: 128 (512, 1024) 32 20.8 and 23.5, 320 31.4 and 34.9; 256 (768, 1536) 48 23.2 and 24.3; 160 (512, 1536) 192 35.1 and 37.5;
+// - 256 (768, 1536) 192 49.4 and 46.5; 512 (768, 1024) 256 51.4 and 47.1, 640 75.4 and 71.4; 512 (512, 2688) 176 61.7 and 58.2;
+// - eight chunks of K and more: 384 (1024, 2048) 16 38.5 and 37.8 (whole block), 64 48.0 and 43.5, 256 91.4 and 85.7; 512 (1024, 2688) 22 32.3 and 32.0, 88
+//   63.4 and 58.1, 352 152.4 and 147.7; 128 (1024, 1024) 320 43.3 and 38.9;
+// - too many: 384 (1024, 2048) 384 113.2 and 116.4; 512 (512, 2688) 880 131.3 and 136.5; 256 (768, 1536) 1440 86.8 and 90.6.
+constexpr int DEVICE_WAVES = 4096;
+// `local`: the experts held here, of the `experts` that the pairs name.
+static bool fc12_serves(int64_t pairs, int local, int64_t experts, int n_blocks, int chunks) {
+  if (g_nvfp4_fused) return g_nvfp4_fused == 1;
+  const bool deep = chunks >= 8;
+  const double distinct = local * (1.0 - std::exp(-(double)pairs / (double)experts));  // of a uniform routing
+  const double waves = distinct * n_blocks * (deep ? 2 : 1);
+  if (waves < (deep ? DEVICE_WAVES / 4 : DEVICE_WAVES * 3 / 4)) return false;
+  return pairs < experts || (waves <= 2 * DEVICE_WAVES && (deep || pairs <= 2 * experts));
+}
+
+// Both layers over a plan of `slots` entries (busy: the caller's estimate of those with rows), in one launch; `dense`: one slot of a dense matrix
+// beside them, or null.
+template <int EPI1>
+static int launch_fc12(StreamParams& p1, StreamParams& p2, int64_t slots, int64_t busy, StreamParams* dense, hipStream_t stream) {
+  if (int e = shape_nvfp4(p1, busy)) return e;
+  if (int e = shape_nvfp4(p2, busy)) return e;
+  const int waves = std::max(p1.ks * p1.nbw, p2.ks * p2.nbw);  // one workgroup size for both: all powers of two
+  p1.nbw = waves / p1.ks;
+  p2.nbw = waves / p2.ks;
+  int first = 0;
+  if (dense) {
+    if (int e = shape_nvfp4(*dense, 1)) return e;
+    dense->ks = std::min(dense->ks, waves);
+    dense->nbw = waves / dense->ks;
+    set_split(*dense);
+    first = (dense->n_blocks + dense->nbw - 1) / dense->nbw;
+  }
+  const int groups1 = (p1.n_blocks + p1.nbw - 1) / p1.nbw, groups2 = (p2.n_blocks + p2.nbw - 1) / p2.nbw;
+  const int64_t total = slots * (groups1 + groups2) + first;
+  if (total > 0x7fffffff) return HB_EINVAL;
+  p1.done = p2.done = plan_done(const_cast<int32_t*>(p1.plan), slots);
+  p2.done_need = groups1;
+  p2.wait_spins = WAIT_SPINS;
+  p2.fault = const_cast<int32_t*>(p1.plan) + PLAN_FAULT;
+  // about half the device's workgroups ahead (1024 (4 wavefronts) started at once, twice that: 512 (1024, 2688) at 176 pairs 32 slots 91.7 us, 48 89.2, 96 88.4)
+  const int lag = (int)std::min<int64_t>(slots, g_nvfp4_lag ? 8 * g_nvfp4_lag.load() : std::max(8, 2048 / groups1));
+  HB_LAUNCH(nvfp4_fc12_kernel<EPI1>, dim3((unsigned)total), dim3(64 * waves), (size_t)waves * FP4_RING_BYTES, stream, p1, p2, dense ? *dense : StreamParams{}, groups1,
+            groups2, (int)slots, lag, first);
+  return HB_OK;
+}
+
+static int launch_front(const LatentRouter& r, hipStream_t stream) {
+  const int n = r.experts + r.latent;
+  if (r.m <= 0 || r.m > LATENT_MAX_ROWS || r.hidden <= 0 || r.hidden % 512 || r.latent < 0 || r.steps <= 0) return HB_EINVAL;
+  const FrontGemv g{r.w, r.x, r.fused, r.lat, n, r.hidden, r.m, r.experts};
+  const dim3 grid((unsigned)((n + FRONT_COLUMNS - 1) / FRONT_COLUMNS));
+  auto launch = [&](auto kernel) { HB_LAUNCH(kernel, grid, dim3(64 * FRONT_WAVES), 0, stream, g); };
+  r.m <= 8 ? launch(latent_front_kernel<true>) : launch(latent_front_kernel<false>);
+  return HB_OK;
+}
+
+// Routing and plan beside `up` (latent_plan_kernel), or, where that form does not serve, apart.
+static int launch_latent_plan(const LatentRouter& r, StreamParams& up, hipStream_t stream) {
+  LatentPlan q;
+  if (!latent_plan_of(r, q)) {
+    if (int e = latent_launch_route(r, stream)) return e;
+    return launch_nvfp4<EPI_DENSE_RELU2>(up, 1, 1, stream);
+  }
+  if (int e = shape_nvfp4(up, 1)) return e;
+  up.nbw = 1;
+  while (up.ks < 8 && 2 * up.ks <= up.chunks) up.ks *= 2;
+  set_split(up);
+  const size_t lds = std::max(q.lds, (size_t)up.ks * FP4_RING_BYTES);
+  auto launch = [&](auto kernel) {
+    HB_LAUNCH(kernel, dim3((unsigned)(q.groups + up.n_blocks)), dim3(PLAN_THREADS), lds, stream, q.route, r.m, q.by_rows, r.e_lo, r.e_n, r.ws->plan, r.ws->order, q.slot_cap,
+              q.groups, up);
+  };
+  q.groups > 1 ? launch(latent_plan_kernel<true>) : launch(latent_plan_kernel<false>);
   return HB_OK;
 }
 
@@ -878,6 +1099,8 @@ int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, i
     if (int e = launch_panel_routed<TileNvfp4, EPI_FC2>(f2, tiles, slots, pairs, stream)) return e;
     return launch_status();
   }
+  if (fc12_serves(pairs, ex->experts, named, p.n_blocks, p.chunks) && (ex->gated ? launch_fc12<EPI_FC1_GATED>(p, f2, slots, est, nullptr, stream) : launch_fc12<EPI_FC1_RELU2>(p, f2, slots, est, nullptr, stream)) == HB_OK)
+    return launch_status();
   if (int e = ex->gated ? launch_nvfp4<EPI_FC1_GATED>(p, slots, est, stream) : launch_nvfp4<EPI_FC1_RELU2>(p, slots, est, stream)) return e;
   if (int e = launch_nvfp4<EPI_FC2>(f2, slots, est, stream)) return e;
   return launch_status();
@@ -931,7 +1154,8 @@ int check_latent(const hb_latent_weights* w, int m, int topk) {
 
 int hb::nvfp4_tune(const char* key, int value) {
   std::atomic<int>* slot = !strcmp(key, "nvfp4_tile") ? &g_nvfp4_tile : !strcmp(key, "nvfp4_ksplit") ? &g_nvfp4_ksplit : !strcmp(key, "nvfp4_nbw") ? &g_nvfp4_nbw
-              : !strcmp(key, "nvfp4_few") ? &g_nvfp4_few : !strcmp(key, "nvfp4_tile_ks") ? &g_nvfp4_tile_ks : nullptr;
+              : !strcmp(key, "nvfp4_few") ? &g_nvfp4_few : !strcmp(key, "nvfp4_tile_ks") ? &g_nvfp4_tile_ks
+              : !strcmp(key, "nvfp4_lag") ? &g_nvfp4_lag : !strcmp(key, "nvfp4_fused") ? &g_nvfp4_fused : nullptr;
   if (!slot || value < 0 || value > 16) return HB_EINVAL;
   *slot = value;
   return HB_OK;
@@ -983,15 +1207,8 @@ extern "C" size_t hb_latent_workspace_bytes(const hb_latent_weights* w, int m, i
   return latent_carve(w, nullptr, m, topk).bytes;
 }
 
-extern "C" int hb_latent_router(const hb_latent_weights* w, const void* x, int m, int topk, const int32_t* slots, int steps, int route, int pad_id,
-                                float* fused, int32_t* ids, float* weights, void* lat, void* workspace, size_t workspace_bytes, void* stream) {
-  if (int e = check_latent(w, m, topk)) return e;
-  if (!x || !fused || !lat || !workspace || (route && (!ids || !weights))) return HB_ENULL;
-  if (!aligned(x, 16) || !aligned(fused, 4) || !aligned(ids, 4) || !aligned(weights, 4) || !aligned(lat, 2) || !aligned(slots, 4) || !aligned(workspace, 16))
-    return HB_EINVAL;
-  if (pad_id > w->experts_total) return HB_EINVAL;
-  const LatentWorkspace l = latent_carve(w, workspace, m, topk);
-  if (workspace_bytes < l.bytes) return HB_EWORKSPACE;
+static LatentRouter latent_router_of(const hb_latent_weights* w, const void* x, int m, int topk, const int32_t* slots, int steps, int pad_id, float* fused,
+                                     int32_t* ids, float* weights, void* lat, const LatentWorkspace& l) {
   LatentRouter r{};
   r.w = static_cast<const uint16_t*>(w->gate_fc1);
   r.bias = w->bias;
@@ -1003,7 +1220,6 @@ extern "C" int hb_latent_router(const hb_latent_weights* w, const void* x, int m
   r.hidden = w->hidden;
   r.topk = topk;
   r.steps = steps;
-  r.route = route != 0;
   r.pad_id = pad_id;
   r.fused = fused;
   r.ids = ids;
@@ -1014,7 +1230,23 @@ extern "C" int hb_latent_router(const hb_latent_weights* w, const void* x, int m
     r.e_n = w->routed->experts;
     r.ws = &l.moe;
   }
-  if (int e = latent_launch_router(r, as_stream(stream))) return e;
+  return r;
+}
+
+extern "C" int hb_latent_router(const hb_latent_weights* w, const void* x, int m, int topk, const int32_t* slots, int steps, int route, int pad_id,
+                                float* fused, int32_t* ids, float* weights, void* lat, void* workspace, size_t workspace_bytes, void* stream) {
+  if (int e = check_latent(w, m, topk)) return e;
+  if (!x || !fused || !lat || !workspace || (route && (!ids || !weights))) return HB_ENULL;
+  if (!aligned(x, 16) || !aligned(fused, 4) || !aligned(ids, 4) || !aligned(weights, 4) || !aligned(lat, 2) || !aligned(slots, 4) || !aligned(workspace, 16))
+    return HB_EINVAL;
+  if (pad_id > w->experts_total || steps <= 0) return HB_EINVAL;
+  if (int e = moe_check_route(m, w->experts_total, topk)) return e;
+  const LatentWorkspace l = latent_carve(w, workspace, m, topk);
+  if (workspace_bytes < l.bytes) return HB_EWORKSPACE;
+  const LatentRouter r = latent_router_of(w, x, m, topk, slots, steps, pad_id, fused, ids, weights, lat, l);
+  if (int e = launch_front(r, as_stream(stream))) return e;
+  if (route)
+    if (int e = latent_launch_route(r, as_stream(stream))) return e;
   return launch_status();
 }
 
@@ -1046,6 +1278,25 @@ extern "C" int hb_latent_out(const hb_latent_weights* w, const void* routed, int
   return launch_status();
 }
 
+// The end of a latent block: the routed rows' sums, then out = bf16(shared + sum fc2^T).
+static int latent_finish(const hb_latent_weights* w, const int32_t* ids, const float* weights, int m, int topk, const LatentWorkspace& l, void* out, hipStream_t s) {
+  CombineParams c{};
+  c.pairs = l.moe.y;
+  c.ids = ids;
+  c.weights = weights;
+  c.e_lo = w->routed->base;
+  c.e_n = w->routed->experts;
+  c.m = m;
+  c.topk = topk;
+  c.h = w->latent;
+  c.out = l.routed;
+  moe_launch_combine(c, s);
+  if (int e = latent_launch_out(static_cast<const uint16_t*>(w->fc2), l.routed, w->shared_up ? l.shared_y : nullptr, static_cast<uint16_t*>(out), m, w->hidden,
+                                w->latent, s))
+    return e;
+  return launch_status();
+}
+
 extern "C" int hb_latent_block(const hb_latent_weights* w, const void* x, const void* lat, const int32_t* ids, const float* weights, int m, int topk,
                                int plan, void* out, void* workspace, size_t workspace_bytes, void* stream) {
   if (int e = check_latent(w, m, topk)) return e;
@@ -1071,19 +1322,69 @@ extern "C" int hb_latent_block(const hb_latent_weights* w, const void* x, const 
     if (int e = ex->gated ? launch_nvfp4<EPI_FC1_GATED>(fc1, slots, est, s) : launch_nvfp4<EPI_FC1_RELU2>(fc1, slots, est, s)) return e;
     if (int e = launch_nvfp4<EPI_FC2>(fc2, slots, est, s)) return e;
   }
-  CombineParams c{};
-  c.pairs = l.moe.y;
-  c.ids = ids;
-  c.weights = weights;
-  c.e_lo = ex->base;
-  c.e_n = ex->experts;
-  c.m = m;
-  c.topk = topk;
-  c.h = w->latent;
-  c.out = l.routed;
-  moe_launch_combine(c, s);
-  if (int e = latent_launch_out(static_cast<const uint16_t*>(w->fc2), l.routed, w->shared_up ? l.shared_y : nullptr, static_cast<uint16_t*>(out), m, w->hidden,
-                                w->latent, s))
-    return e;
-  return launch_status();
+  return latent_finish(w, ids, weights, m, topk, l, out, s);
+}
+
+// The block from its rows in one call: [workspace of the router and the block][latent rows][router product][ids][weights].
+namespace {
+struct LatentLayer {
+  LatentWorkspace l;
+  uint16_t* lat;
+  float* fused;
+  int32_t* ids;
+  float* weights;
+  size_t bytes;
+};
+LatentLayer latent_layer_carve(const hb_latent_weights* w, void* base, int m, int topk) {
+  LatentLayer c{latent_carve(w, base, m, topk), nullptr, nullptr, nullptr, nullptr, 0};
+  size_t off = c.l.bytes;
+  auto take = [&](size_t bytes) {
+    void* ptr = base ? static_cast<char*>(base) + off : nullptr;
+    off += (bytes + 255) & ~(size_t)255;
+    return ptr;
+  };
+  c.lat = static_cast<uint16_t*>(take((size_t)m * w->latent * 2));
+  c.fused = static_cast<float*>(take((size_t)m * (w->experts_total + w->latent) * 4));
+  c.ids = static_cast<int32_t*>(take((size_t)m * topk * 4));
+  c.weights = static_cast<float*>(take((size_t)m * topk * 4));
+  c.bytes = off;
+  return c;
+}
+}  // namespace
+
+extern "C" size_t hb_latent_layer_workspace_bytes(const hb_latent_weights* w, int m, int topk) {
+  if (check_latent(w, m, topk) != HB_OK || !w->routed) return 0;
+  return latent_layer_carve(w, nullptr, m, topk).bytes;
+}
+
+extern "C" int hb_latent_layer(const hb_latent_weights* w, const void* x, int m, int topk, const int32_t* slots, int steps, int pad_id, void* out,
+                               void* workspace, size_t workspace_bytes, void* stream) {
+  if (int e = check_latent(w, m, topk)) return e;
+  if (!w->routed || !x || !out || !workspace) return HB_ENULL;
+  if (!aligned(x, 16) || !aligned(slots, 4) || !aligned(out, 2) || !aligned(workspace, 16)) return HB_EINVAL;
+  if (pad_id > w->experts_total || steps <= 0) return HB_EINVAL;
+  if (int e = moe_check_route(m, w->experts_total, topk)) return e;
+  const LatentLayer c = latent_layer_carve(w, workspace, m, topk);
+  if (workspace_bytes < c.bytes) return HB_EWORKSPACE;
+  const LatentWorkspace& l = c.l;
+  const hb_nvfp4_experts* ex = w->routed;
+  hipStream_t s = as_stream(stream);
+  const LatentRouter r = latent_router_of(w, x, m, topk, slots, steps, pad_id, c.fused, c.ids, c.weights, c.lat, l);
+  StreamParams up, down, fc1, fc2;
+  if (w->shared_up) {
+    up = dense_params(w->shared_up, w->shared_up_scale, w->shared_inter, w->hidden, x, m, l.shared_h);
+    down = dense_params(w->shared_down, w->shared_down_scale, w->hidden, w->shared_inter, l.shared_h, m, l.shared_y);
+  }
+  if (int e = launch_front(r, s)) return e;
+  if (int e = w->shared_up ? launch_latent_plan(r, up, s) : latent_launch_route(r, s)) return e;
+  const int64_t pairs = (int64_t)m * topk, slot_cap = moe_max_slots(pairs, ex->experts, 0, ROWS_PER_SLOT), est = busy_slots(pairs, ex->experts, slot_cap);
+  expert_params(ex, c.lat, m, topk, l.moe, l.moe.y, 0, fc1, fc2);
+  StreamParams* dense = w->shared_up ? &down : nullptr;
+  const bool together = fc12_serves(pairs, ex->experts, experts_named(w->experts_total, ex->base, ex->experts), fc1.n_blocks, fc1.chunks) &&
+                        (ex->gated ? launch_fc12<EPI_FC1_GATED>(fc1, fc2, slot_cap, est, dense, s) : launch_fc12<EPI_FC1_RELU2>(fc1, fc2, slot_cap, est, dense, s)) == HB_OK;
+  if (!together) {
+    if (int e = ex->gated ? launch_nvfp4<EPI_FC1_GATED>(fc1, slot_cap, est, s) : launch_nvfp4<EPI_FC1_RELU2>(fc1, slot_cap, est, s)) return e;
+    if (int e = dense ? launch_twin<EPI_FC2, EPI_DENSE>(fc2, slot_cap, est, down, 1, s) : launch_nvfp4<EPI_FC2>(fc2, slot_cap, est, s)) return e;
+  }
+  return latent_finish(w, c.ids, c.weights, m, topk, l, out, s);
 }

@@ -42,9 +42,13 @@ struct RingSource {
 // Chunks c0 .. c1 - 1 (at least one) of block row `nb`, through the wavefront's ring, for the slot's rows from row0 (the
 // four-row bodies: row0 .. row0 + 3; the sixteen-row body: all, row0 = 0).
 // `acts`: the body's state (the caller's object when the body keeps results of its own beside the four accumulators).
-template <int EPI, class Acts, class Ring>
+// `wait`: what has to be there before the activations are read (SlotWait): both slots' blocks are asked for ahead of it, the activations behind it
+// (so at least as many requests as ever stand behind a block); if it gives up, nothing is computed. The routed latent block, weights asked for
+// behind the wait and ahead of it, us: 512 (1024, 2688) two rows 57.6 and 55.6, 256 (768, 1536) four 42.3 and 42.2, the three-bit layer of 40 rows
+// under a budget 51.0 and 50.7.
+template <int EPI, class Acts, class Ring, class Wait>
 __device__ __forceinline__ void stream_block(const StreamParams& p, const Slot& sl, int row0, int nb, int c0, int c1, int lane, uint8_t* ring,
-                                             f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, Acts& acts) {
+                                             f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, Acts& acts, Wait& wait) {
   constexpr int BEHIND = Ring::LOADS + Acts::LOADS;
   const int r16 = lane & 15, n = c1 - c0;
   RingSource src;
@@ -54,14 +58,19 @@ __device__ __forceinline__ void stream_block(const StreamParams& p, const Slot& 
   uint32_t codes, scales;  // LDS byte addresses of what the lane reads back from slot 0; the reads select the slot by their offset
   Ring::lanes(src, lane, r16, (uint32_t)(uintptr_t)slot0, codes, scales);
   typename Ring::Chunk ch;
+  wait.look();
   Ring::request(src, c0, slot0);
   asm volatile("" ::: "memory");  // whatever else the prologue asks for stands behind the first block
+  if constexpr (Wait::WAITS) {
+    if (n > 1) Ring::request(src, c0 + 1, slot1);
+    if (!wait.done()) return;
+  }
   acts.template start<EPI>(p, sl, row0, c0, n, lane);
   if (n == 1) {
     Ring::template take<0, 0>(ch, codes, scales);
     acts.template step<0, false, false>(ch, 0, acc0, acc1, acc2, acc3, sl);
   } else {
-    Ring::request(src, c0 + 1, slot1);
+    if constexpr (!Wait::WAITS) Ring::request(src, c0 + 1, slot1);
     int i = 0;
     for (; i + 3 < n; i += 2) {  // chunks i and i + 1, asking for the blocks of i + 2 and i + 3
       Ring::template take<BEHIND, 0>(ch, codes, scales);
@@ -90,9 +99,24 @@ __device__ __forceinline__ void stream_block(const StreamParams& p, const Slot& 
 
 template <int EPI, class Acts, class Ring>
 __device__ __forceinline__ void stream_block(const StreamParams& p, const Slot& sl, int row0, int nb, int c0, int c1, int lane, uint8_t* ring,
+                                             f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, Acts& acts) {
+  NoWait none;
+  stream_block<EPI, Acts, Ring>(p, sl, row0, nb, c0, c1, lane, ring, acc0, acc1, acc2, acc3, acts, none);
+}
+
+template <int EPI, class Acts, class Ring>
+__device__ __forceinline__ void stream_block(const StreamParams& p, const Slot& sl, int row0, int nb, int c0, int c1, int lane, uint8_t* ring,
                                              f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3) {
   Acts acts;
-  stream_block<EPI, Acts, Ring>(p, sl, row0, nb, c0, c1, lane, ring, acc0, acc1, acc2, acc3, acts);
+  NoWait none;
+  stream_block<EPI, Acts, Ring>(p, sl, row0, nb, c0, c1, lane, ring, acc0, acc1, acc2, acc3, acts, none);
+}
+
+template <int EPI, class Acts, class Ring, class Wait>
+__device__ __forceinline__ void stream_block_behind(const StreamParams& p, const Slot& sl, int row0, int nb, int c0, int c1, int lane, uint8_t* ring,
+                                                    f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, Wait& wait) {
+  Acts acts;
+  stream_block<EPI, Acts, Ring>(p, sl, row0, nb, c0, c1, lane, ring, acc0, acc1, acc2, acc3, acts, wait);
 }
 
 }  // namespace hb

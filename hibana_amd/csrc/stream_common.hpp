@@ -98,6 +98,83 @@ __device__ __forceinline__ bool await_count(const int32_t* at, int need, int spi
   return there;
 }
 
+// fc1 and fc2 of a routed call in one launch (w3_fc12_kernel says why, and why the waits end). Which workgroup of which layer and slot a
+// grid index is: slot-major, fc2 of a slot `lag` slots behind its fc1.
+struct Fc12Place {
+  int slot, index;  // `index`: the workgroup among its slot's of its layer
+  bool is_fc1;
+};
+__device__ __forceinline__ Fc12Place fc12_place(int id, int groups1, int groups2, int slots, int lag) {
+  Fc12Place at;
+  const int head = lag * groups1, both = groups1 + groups2, middle = (slots - lag) * both;
+  if (id < head) {  // the first slots' fc1
+    at.slot = id / groups1;
+    at.index = id - at.slot * groups1;
+    at.is_fc1 = true;
+  } else if (id < head + middle) {  // fc1(s) then fc2(s - lag)
+    id -= head;
+    const int step = id / both;
+    id -= step * both;
+    at.is_fc1 = id < groups1;
+    at.slot = at.is_fc1 ? lag + step : step;
+    at.index = at.is_fc1 ? id : id - groups1;
+  } else {  // the last slots' fc2
+    id -= head + middle;
+    const int step = id / groups2;
+    at.index = id - step * groups2;
+    at.slot = slots - lag + step;
+    at.is_fc1 = false;
+  }
+  return at;
+}
+// The end of an fc1 workgroup: its part of the slot's h is in memory (store_out's write-through stores), and counted.
+__device__ __forceinline__ void fc12_arrive(const StreamParams& p, int slot) {
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's part of h has reached memory
+  __syncthreads();
+  if (threadIdx.x == 0) atomicAdd(&p.done[slot * DONE_PITCH], 1);
+}
+// The start of an fc2 workgroup: a wait for all of the slot's h, with the first weights asked for ahead of it (stream_block calls the two
+// halves around those requests), so that the wait and the weights' way from memory lie side by side. One wavefront polls for the workgroup;
+// the others wait at the barrier and learn the outcome from a word of LDS of its own. The barrier and that word's accesses are written out: the
+// compiler would have the LDS-direct loads of the weights wait ahead of them.
+struct SlotWait {
+  static constexpr bool WAITS = true;
+  const int32_t* at;
+  int need, spins;
+  int32_t* fault;
+  uint32_t word;  // the LDS byte address of the outcome
+  bool timed, there;  // `timed`: measurement hook: `ended` takes the time of the wait's end
+  int64_t ended;
+  int seen;
+  __device__ __forceinline__ SlotWait(const StreamParams& p, int slot, int* outcome, bool timed)
+      : at(p.done + slot * DONE_PITCH), need(p.done_need), spins(p.wait_spins), fault(p.fault), word((uint32_t)(uintptr_t)(__attribute__((address_space(3))) int*)outcome),
+        timed(timed), there(false), ended(0), seen(0) {}
+  __device__ __forceinline__ void look() {  // a first poll, ahead of the weights' requests: its answer does not stand behind them
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0) seen = load_through(at);
+    asm volatile("" ::: "memory");
+  }
+  // false (the wait gave up): the workgroup must store nothing
+  __device__ __forceinline__ bool done() {
+    if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) == 0) {
+      const bool in = seen >= need || await_count(at, need, spins);
+      if (threadIdx.x == 0 && !in) atomicOr(fault, HB_FAULT_WAIT);  // the caller reads it with hb_workspace_status
+      asm volatile("ds_write_b32 %0, %1" ::"v"(word), "v"((int)in) : "memory");
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    int in;
+    asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(in) : "v"(word) : "memory");
+    there = __builtin_amdgcn_readfirstlane(in) != 0;
+    if (!there) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the weights on their way to LDS arrive before the workgroup leaves it
+    if (timed) ended = (int64_t)wall_clock64();
+    return there;
+  }
+};
+struct NoWait {
+  static constexpr bool WAITS = false, there = true;
+  __device__ __forceinline__ void look() {}
+  __device__ __forceinline__ bool done() { return true; }
+};
+
 // The epilogue's roundings use the hardware FP32 -> BF16 conversion (round to nearest even).
 __device__ __forceinline__ uint16_t bf16_of(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 __device__ __forceinline__ float through_bf16(float f) { return (float)(__bf16)f; }
@@ -612,8 +689,8 @@ struct CombineParams {
 void moe_launch_combine(const CombineParams& c, hipStream_t stream);
 
 // The dense ends of a latent block of at most LATENT_MAX_ROWS rows (hibana/kernels/csrc/nemotron_moe.cu of the reference).
-// Router: fused FP32 [m, experts + latent] = x [router; fc1_latent]^T and its latent columns as BF16 (one launch);
-// with `route`, a second launch: sigmoid + bias top-k routing of the rows (ids, weights; padded rows take `pad_id`, or
+// The router's product: fused FP32 [m, experts + latent] = x [router; fc1_latent]^T and its latent columns as BF16 (nvfp4.hip).
+// latent_launch_route: sigmoid + bias top-k routing of its rows (ids, weights; padded rows take `pad_id`, or
 // row 0's first choice when it is negative) and, given a workspace, the expert plan of experts e_lo .. e_lo + e_n - 1.
 constexpr int LATENT_MAX_ROWS = HB_LATENT_MAX_ROWS;
 struct LatentRouter {
@@ -621,7 +698,7 @@ struct LatentRouter {
   const float* bias;     // [experts]
   const uint16_t* x;     // BF16 [m, hidden]
   const int32_t* slots;  // or null
-  int m, experts, latent, hidden, topk, steps, route, pad_id;
+  int m, experts, latent, hidden, topk, steps, pad_id;
   float* fused;
   int32_t* ids;
   float* weights;
@@ -629,7 +706,7 @@ struct LatentRouter {
   int e_lo, e_n;
   const MoeWorkspace* ws;  // the plan's home, or null: routing only
 };
-int latent_launch_router(const LatentRouter& r, hipStream_t stream);
+int latent_launch_route(const LatentRouter& r, hipStream_t stream);
 // Out: out = bf16(shared + routed fc2^T), routed BF16 [m, latent].
 int latent_launch_out(const uint16_t* fc2, const uint16_t* routed, const uint16_t* shared, uint16_t* out, int m, int hidden, int latent, hipStream_t stream);
 

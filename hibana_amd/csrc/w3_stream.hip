@@ -720,14 +720,15 @@ __device__ __forceinline__ void finish_few(const StreamParams& p, const Slot& sl
 // scales (p.oq, p.oq_scale), the activation rounding done in its epilogue.
 // SPLIT: slots of at most two rows read the two-plane form of the activations (p.a2) and run on the FP8 matrix cores.
 // One workgroup's work: slot `sl` (with rows), the run `bx` of p.nbw 64-row blocks; `rings`: the launch's dynamic LDS.
-template <int EPI, bool A8, bool SPLIT, class Ring = W3Ring>
-__device__ __forceinline__ void stream_workgroup(const StreamParams& p, const Slot& sl, int bx, uint8_t* rings) {
+template <int EPI, bool A8, bool SPLIT, class Ring = W3Ring, class Wait>
+__device__ __forceinline__ void stream_workgroup(const StreamParams& p, const Slot& sl, int bx, uint8_t* rings, Wait& wait) {
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // the same in every lane: kept in scalars
   const WaveShare share = wave_share(p, wave);
   const int ks = share.ks, nbi = share.nbi, nb = bx * p.nbw + nbi;
   const bool active = nb < p.n_blocks;
   f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0, acc2 = acc0, acc3 = acc0;
   uint8_t* ring = rings + wave * RING_BYTES;
+  if (Wait::WAITS && !active) wait.done();
   constexpr bool QUANT = A8 && epi_gathers(EPI);  // fc1 on E4M3 activations hands fc2 E4M3 activations
   if (A8) {
     if (sl.rows <= FEW_ROWS) {  // uniform over the workgroup
@@ -736,15 +737,17 @@ __device__ __forceinline__ void stream_workgroup(const StreamParams& p, const Sl
       if (active) {
         scale = sl.rs[nb * 64 + lane];
         if (EPI == EPI_FC2) pairs.ask(p, sl, 0);
-        stream_block<EPI, FewActs8, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+        stream_block_behind<EPI, FewActs8, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3, wait);
       }
+      if (!wait.there) return;
       finish_few<EPI, QUANT>(p, sl, 0, scale, nb, active, wave, ks, nbi, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3, pairs);
     } else {
       RowScales rs{};
       if (active) {
-        stream_block<EPI, FullActs8, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+        stream_block_behind<EPI, FullActs8, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3, wait);
         rs = row_scales<true>(sl, nb, lane & 15);
       }
+      if (!wait.there) return;
       finish_block<EPI, true, RING_BYTES / 4, QUANT>(p, sl, rs, nb, active, ks, nbi, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3);
     }
   } else if (SPLIT && sl.rows <= PLANE_ROWS) {  // uniform over the workgroup
@@ -755,8 +758,9 @@ __device__ __forceinline__ void stream_workgroup(const StreamParams& p, const Sl
       scale = sl.rs[nb * 64 + lane];
       if (EPI == EPI_FC2) pairs.ask(p, sl, 0);
       xs.ask<EPI>(p, sl, 0);
-      stream_block<EPI, FewPlaneActs, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+      stream_block_behind<EPI, FewPlaneActs, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3, wait);
     }
+    if (!wait.there) return;
     finish_few<EPI, false, true, true>(p, sl, 0, scale, nb, active, wave, ks, nbi, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3, pairs, xs);
   } else if (sl.rows <= FEW_ROWS && !p.no_few) {  // uniform over the workgroup
     float scale = 0.f;
@@ -764,17 +768,24 @@ __device__ __forceinline__ void stream_workgroup(const StreamParams& p, const Sl
     if (active) {
       scale = sl.rs[nb * 64 + lane];  // row 16 q + r16 of the block: asked for ahead of the chunks, there when the epilogue wants it
       if (EPI == EPI_FC2) pairs.ask(p, sl, 0);
-      stream_block<EPI, FewActs, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);  // at least one chunk: ks <= chunks
+      stream_block_behind<EPI, FewActs, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3, wait);  // at least one chunk: ks <= chunks
     }
+    if (!wait.there) return;
     finish_few<EPI>(p, sl, 0, scale, nb, active, wave, ks, nbi, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3, pairs);
   } else {
     RowScales rs{};
     if (active) {
-      stream_block<EPI, FullActs, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+      stream_block_behind<EPI, FullActs, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3, wait);
       rs = row_scales<true>(sl, nb, lane & 15);
     }
+    if (!wait.there) return;
     finish_block<EPI, true, RING_BYTES / 4>(p, sl, rs, nb, active, ks, nbi, reinterpret_cast<float*>(rings), acc0, acc1, acc2, acc3);
   }
+}
+template <int EPI, bool A8, bool SPLIT, class Ring = W3Ring>
+__device__ __forceinline__ void stream_workgroup(const StreamParams& p, const Slot& sl, int bx, uint8_t* rings) {
+  NoWait none;
+  stream_workgroup<EPI, A8, SPLIT, Ring>(p, sl, bx, rings, none);
 }
 
 template <int EPI, bool A8, bool SPLIT = false, int BITS = 3>  // BITS: the tile layout's (two-bit matrices have their own)
@@ -984,8 +995,8 @@ __global__ __launch_bounds__(1024) void w3_fc1_route_one_kernel(StreamParams p, 
 // first every fc1 workgroup (slot-major, the slot table's order), then every fc2 workgroup. A slot's fc2 needs all of
 // the slot's h, that is all `groups1` fc1 workgroups of the slot: each of those, once its h is in memory (write-through
 // stores, waited for), adds one to the slot's arrival counter (plan_done: zero from the plan), and the slot's fc2
-// workgroups wait for the counter before they ask for anything (one wavefront polls with loads that bypass the L2, the
-// others stand at a barrier). What fc2 then reads of h it reads with ordinary loads: the lines were written through to
+// workgroups wait for the counter behind the requests of their first weights (one wavefront polls with loads that bypass the L2, the
+// others stand at a barrier: SlotWait). What fc2 then reads of h it reads with ordinary loads: the lines were written through to
 // memory before the count, and this compute die's L2 cannot hold an older copy of them, because every launch starts
 // with its L2 invalidated and no workgroup of this launch reads a slot's h before the slot's count is complete (h rows
 // are whole 256-byte multiples on 256-byte boundaries, so no line of h is shared with anything read earlier).
@@ -1004,64 +1015,33 @@ __global__ __launch_bounds__(1024) void w3_fc1_route_one_kernel(StreamParams p, 
 template <int EPI1, bool SPLIT>
 __global__ __launch_bounds__(1024) void w3_fc12_kernel(StreamParams p1, StreamParams p2, int groups1, int groups2, int slots, int lag) {
   extern __shared__ __align__(16) uint8_t rings[];
-  int id = blockIdx.x, slot;
-  bool is_fc1;
-  const int head = lag * groups1, both = groups1 + groups2, middle = (slots - lag) * both;
-  if (id < head) {  // the first slots' fc1
-    slot = id / groups1;
-    id -= slot * groups1;
-    is_fc1 = true;
-  } else if (id < head + middle) {  // fc1(s) then fc2(s - lag)
-    id -= head;
-    const int step = id / both;
-    id -= step * both;
-    is_fc1 = id < groups1;
-    slot = is_fc1 ? lag + step : step;
-    if (!is_fc1) id -= groups1;
-  } else {  // the last slots' fc2
-    id -= head + middle;
-    const int step = id / groups2;
-    id -= step * groups2;
-    slot = slots - lag + step;
-    is_fc1 = false;
-  }
+  __shared__ int outcome;
+  const Fc12Place at = fc12_place(blockIdx.x, groups1, groups2, slots, lag);
+  const int slot = at.slot;
   const int64_t t0 = p1.trace ? (int64_t)wall_clock64() : 0;
   int64_t t1 = 0;
   int rows = 0;
-  if (is_fc1) {
+  if (at.is_fc1) {
     const Slot sl = slot_of<EPI1>(p1, slot);
     if (sl.rows <= 0) return;
     rows = sl.rows;
-    stream_workgroup<EPI1, false, SPLIT>(p1, sl, id, rings);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's part of h has reached memory
-    __syncthreads();
-    if (threadIdx.x == 0) atomicAdd(&p1.done[slot * DONE_PITCH], 1);
+    stream_workgroup<EPI1, false, SPLIT>(p1, sl, at.index, rings);
+    fc12_arrive(p1, slot);
   } else {
     const Slot sl = slot_of<EPI_FC2>(p2, slot);
     if (sl.rows <= 0) return;
     rows = sl.rows;
-    // one wavefront polls for the workgroup; the others wait at the barrier and learn the outcome through LDS
-    int* outcome = reinterpret_cast<int*>(rings);
-    if (threadIdx.x < 64) {
-      const bool there = await_count(p2.done + slot * DONE_PITCH, p2.done_need, p2.wait_spins);
-      if (threadIdx.x == 0) {
-        *outcome = there;
-        if (!there) atomicOr(p2.fault, HB_FAULT_WAIT);  // the caller reads it with hb_workspace_status
-      }
-    }
-    __syncthreads();
-    const bool there = *outcome != 0;
-    __syncthreads();  // read by everyone before the rings take the memory
-    if (!there) return;  // h is not known to be complete: this workgroup's outputs stay as they were
-    if (p1.trace) t1 = (int64_t)wall_clock64();
-    stream_workgroup<EPI_FC2, false, false>(p2, sl, id, rings);
+    SlotWait wait(p2, slot, &outcome, p1.trace != nullptr);
+    stream_workgroup<EPI_FC2, false, false>(p2, sl, at.index, rings, wait);
+    if (!wait.there) return;  // h is not known to be complete: this workgroup's outputs stay as they were
+    t1 = wait.ended;
   }
   if (p1.trace && threadIdx.x == 0 && (int64_t)blockIdx.x < p1.trace_records) {  // measurement hook: start, end of the wait, end (100 MHz ticks), rows
     int64_t* rec = p1.trace + 4 * (int64_t)blockIdx.x;
     rec[0] = t0;
     rec[1] = t1;
     rec[2] = (int64_t)wall_clock64();
-    rec[3] = rows | (is_fc1 ? 1 << 16 : 0);
+    rec[3] = rows | (at.is_fc1 ? 1 << 16 : 0);
   }
 }
 

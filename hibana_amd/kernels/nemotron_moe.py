@@ -75,6 +75,12 @@ class SmallWeights:
             need = self._bytes[(m, k)] = _lib.lib().hb_latent_workspace_bytes(C.byref(self.struct()), m, k)
         return need
 
+    def layer_bytes(self, m: int, k: int) -> int:
+        need = self._bytes.get((m, k, "layer"))
+        if need is None:
+            need = self._bytes[(m, k, "layer")] = _lib.lib().hb_latent_layer_workspace_bytes(C.byref(self.struct()), m, k)
+        return need
+
     def _assemble(self) -> _lib.HbLatentWeights:
         up, down = self.shared_up, self.shared_down
         return _lib.HbLatentWeights(
@@ -130,6 +136,25 @@ def router(x: torch.Tensor, weights: SmallWeights, bias: torch.Tensor | None, k:
                                            _lib.ptr(wts), _lib.ptr(lat), _lib.ptr(buffer), need, _lib.stream()), "latent router")
     ws = Workspace(buffer, lat, m, k)
     return (fused, ids, wts, ws, lat) if latent else (fused, ids, wts, ws)
+
+
+def layer(x: torch.Tensor, weights: SmallWeights, k: int, slots: torch.Tensor | None = None, steps: int = 1, pad_id: int = -1) -> torch.Tensor:
+    """`router` (routing and planning) and `block` in one call -> BF16 [M, H], for a caller that wants nothing of what lies between."""
+    m = _rows(x, weights)
+    if weights.experts is None:
+        raise ValueError("layer: no NVFP4 routed experts (router and w3_block serve 3-bit ones)")
+    st = weights.struct()
+    need = weights.layer_bytes(m, k)
+    if need == 0:
+        raise ValueError("layer: the block's shapes are not ones the kernels take")
+    buffer = _lib.workspace(x.device, need, "latent")
+    out = x.new_empty((m, weights.hidden))
+    sl = None if slots is None else slots.to(torch.int32).contiguous()
+    xc = x.contiguous()
+    code = _lib.lib().hb_latent_layer(C.byref(st), xc.data_ptr(), m, k, _lib.ptr(sl), steps, pad_id, out.data_ptr(), buffer.data_ptr(), need, _lib.stream())
+    if code:
+        _lib.check(code, "latent layer")
+    return out
 
 
 def block(x: torch.Tensor, ws: Workspace, ids: torch.Tensor, wts: torch.Tensor, weights: SmallWeights, plan: bool = False,

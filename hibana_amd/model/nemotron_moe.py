@@ -185,8 +185,7 @@ class NemotronMoe:
         if self.w3 is not None:  # padded rows name no expert (id E), which w3_moe skips
             _, ids, weights, ws, lat = small_block.router(x, w, None, self.topk, slots, steps, pad_id=self.experts, latent=True)
             return small_block.w3_block(x, ws, lat, ids, weights, w, self.w3)
-        _, ids, weights, ws = small_block.router(x, w, None, self.topk, slots, steps)
-        return small_block.block(x, ws, ids, weights, w)
+        return small_block.layer(x, w, self.topk, slots, steps)
 
     def forward(self, x: torch.Tensor, ctx=None) -> torch.Tensor:
         """Post-norm rows x [M, H] BF16 -> the block's mixer output [M, H] BF16 (hibana/model/nemotron/moe.py:508-517)."""

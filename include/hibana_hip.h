@@ -535,6 +535,14 @@ int hb_latent_router(const hb_latent_weights* w, const void* x, int m, int topk,
                      int route, int pad_id, float* fused, int32_t* ids, float* weights, void* lat, void* workspace,
                      size_t workspace_bytes, void* stream);
 
+/* hb_latent_router (routing and planning) and hb_latent_block in one call, for a caller that wants the block's output alone: five launches, the
+ * shared expert's up projection beside the router's product, its down projection beside the routed experts' two layers.
+ * `workspace`: hb_latent_layer_workspace_bytes, under the rules of hb_latent_router's; NVFP4 routed experts only.
+ * ref: the block of at most 16 rows, NemotronMoe.small, hibana/model/nemotron/moe.py:484-502. */
+size_t hb_latent_layer_workspace_bytes(const hb_latent_weights* w, int m, int topk);
+int hb_latent_layer(const hb_latent_weights* w, const void* x, int m, int topk, const int32_t* slots, int steps, int pad_id, void* out,
+                    void* workspace, size_t workspace_bytes, void* stream);
+
 /* ref: `block`, hibana/kernels/nemotron_moe.py:58-60: the rest of the block after hb_latent_router -> out BF16
  * [m, hidden]. `plan` != 0 when ids are not the router's (the caller routed): the plan is then made here, one more
  * launch. Four launches otherwise: routed fc1 beside the shared expert's up, routed fc2 beside its down, the combine,

@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <type_traits>
 
 #include "panel_kernel.hpp"
 #include "ring.hpp"
@@ -535,6 +536,29 @@ struct FullActs {  // up to sixteen rows: lane (q, r16) feeds row r16, k 8 q .. 
   }
 };
 
+// The same of a routed slot, with two chunks' activations held and a chunk's asked for two chunks ahead, as its block is: asked for one chunk ahead
+// they stand behind a block asked for one chunk ago, and in a launch of few wavefronts a unit every chunk waits for memory: 40 rows
+// under a budget of 64 experts (2048, 512) 50.7 us, so 50.0. Dense calls, whose wavefronts have few chunks, lose by the second chunk's loads ahead of
+// the first product: 8192 x 2048 twelve rows 6.2 us, so 6.5; 51200 x 2048 17.3 and 16.7.
+struct FullActsAhead {
+  static constexpr int LOADS = 4;
+  Rows even, odd;
+  const uint16_t* at;
+  template <int EPI>
+  __device__ __forceinline__ void start(const StreamParams& p, const Slot& sl, int, int c0, int n, int lane) {
+    at = activation_row<EPI>(p, sl, lane & 15) + (int64_t)c0 * 128 + 8 * (lane >> 4);
+    load_rows(even, at);
+    if (n > 1) load_rows(odd, at + 128);
+  }
+  template <int ODD, bool MORE2, bool MORE1, class C>
+  __device__ __forceinline__ void step(const C& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot& sl) {
+    Rows& held = ODD ? odd : even;
+    compute_half_chunk<0>(ch, held.a0, held.a1, acc0, acc1, acc2, acc3, sl.lut_lo, sl.lut_hi);
+    compute_half_chunk<1>(ch, held.a2, held.a3, acc0, acc1, acc2, acc3, sl.lut_lo, sl.lut_hi);
+    if (MORE2) load_rows(held, at + (int64_t)(i + 2) * 128);
+  }
+};
+
 // The sixteen-row body on E4M3 activations: lane (q, r16) feeds row r16's eight codes of every group (the FP8 MFMA's A
 // operand) and folds, per group, the product of the weight scale and the activation scales of the four rows its
 // accumulator registers hold (rows 4 q .. 4 q + 3). Both are asked for again by halves, as FullActs does.
@@ -775,7 +799,8 @@ __device__ __forceinline__ void stream_workgroup(const StreamParams& p, const Sl
   } else {
     RowScales rs{};
     if (active) {
-      stream_block_behind<EPI, FullActs, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3, wait);
+      typedef typename std::conditional<epi_dense(EPI), FullActs, FullActsAhead>::type Acts;
+      stream_block_behind<EPI, Acts, Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3, wait);
       rs = row_scales<true>(sl, nb, lane & 15);
     }
     if (!wait.there) return;

@@ -697,7 +697,7 @@ __global__ __launch_bounds__(PLAN_THREADS) void latent_plan_kernel(RouteParams r
 }
 
 // experiments (hb_tune): the stream's workgroup shape ("nvfp4_ksplit", "nvfp4_nbw"); "nvfp4_tile": 1 forces the panel kernel, 2 the stream
-static std::atomic<int> g_nvfp4_ksplit{0}, g_nvfp4_nbw{0}, g_nvfp4_tile{0}, g_nvfp4_few{0}, g_nvfp4_tile_ks{0}, g_nvfp4_lag{0}, g_nvfp4_fused{0};  // "nvfp4_fused": 1 runs fc1 and fc2 of a routed call on the stream in one launch, 2 in two; "nvfp4_lag": eighths of the slots fc2 is behind there; "nvfp4_few": 2 switches off the body for slots of at most eight rows; "nvfp4_tile_ks": the workgroups that share a tile's K
+static std::atomic<int> g_nvfp4_ksplit{0}, g_nvfp4_nbw{0}, g_nvfp4_tile{0}, g_nvfp4_few{0}, g_nvfp4_tile_ks{0}, g_nvfp4_lag{0}, g_nvfp4_fused{0};  // "nvfp4_fused": 1 runs fc1 and fc2 of a routed call on the stream in one launch, 2 (of any) in two; "nvfp4_lag": eighths of the slots fc2 is behind in one; "nvfp4_few": 2 switches off the body for slots of at most eight rows; "nvfp4_tile_ks": the workgroups that share a tile's K
 
 static int shape_nvfp4(StreamParams& p, int64_t busy_slots) {
   pick_shape(p.n_blocks, p.chunks, busy_slots, 4096, &p.ks, &p.nbw);
@@ -908,8 +908,8 @@ struct TileNvfp4 {
   static constexpr int BESIDE_TILES = 0;
   static constexpr int LOW_ROWS = 24, MIDDLE_ROWS = 46, MIDDLE_ROWS_LARGE = 46, HIGH_ROWS = 70;  // panel_height's lines
   static constexpr int LIGHT_ROWS = 0;  // (an expansion takes the scale along at the price of the stream's)
-  template <int EPI>
-  static __device__ __forceinline__ void light(const StreamParams&, const Slot&, int, uint8_t*) {}
+  template <int EPI, class Wait>
+  static __device__ __forceinline__ void light(const StreamParams&, const Slot&, int, uint8_t*, Wait&) {}
 };
 
 static inline unsigned grid_for(int64_t threads) { return (unsigned)((threads + 255) / 256); }
@@ -1094,6 +1094,12 @@ int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, i
   const int64_t est = busy_slots(pairs, ex->experts, slots);
   StreamParams p, f2;
   expert_params(ex, x, m, topk, ws, out_pairs, pairs_bf16, p, f2);
+  if (dense && g_nvfp4_fused != 2) {
+    if (int e = ex->gated ? launch_panel_fc12<TileNvfp4, EPI_FC1_GATED>(p, f2, ws.plan, tiles, slots, m, pairs, g_nvfp4_lag, stream)
+                          : launch_panel_fc12<TileNvfp4, EPI_FC1_RELU2>(p, f2, ws.plan, tiles, slots, m, pairs, g_nvfp4_lag, stream))
+      return e;
+    return launch_status();
+  }
   if (dense) {
     if (int e = ex->gated ? launch_panel_routed<TileNvfp4, EPI_FC1_GATED>(p, tiles, slots, m, stream) : launch_panel_routed<TileNvfp4, EPI_FC1_RELU2>(p, tiles, slots, m, stream)) return e;
     if (int e = launch_panel_routed<TileNvfp4, EPI_FC2>(f2, tiles, slots, pairs, stream)) return e;

@@ -59,7 +59,8 @@ __device__ __forceinline__ PanelWave panel_wave(const StreamParams& p, const Pan
 // Sixteen bytes a lane past the caches. The wait state behind the store is its own: a vector instruction right after it may
 // overwrite the data registers before the last lanes are read, and the compiler, which guards its own stores, does not know
 // this statement for one.
-__device__ __forceinline__ void store_through16(f32x4_t* at, const f32x4_t& v) { asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(at), "v"(v) : "memory"); }
+template <class T>
+__device__ __forceinline__ void store_through16(T* at, const T& v) { asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(at), "v"(v) : "memory"); }
 template <int N>
 __device__ __forceinline__ void wait_vm(void) { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 __device__ __forceinline__ void wait_lds(void) { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
@@ -105,7 +106,8 @@ __device__ __forceinline__ void product_second(f32x4_t& acc, const u32x4_t& w, c
 }
 __device__ __forceinline__ void products_done(void) { asm volatile("s_nop 15\n\ts_nop 7" ::: "memory"); }
 
-template <class Fmt, int EPI, int MT>
+// THROUGH: the results are read by other workgroups of the same launch.
+template <class Fmt, int EPI, int MT, bool THROUGH = false>
 struct Panel {
   typedef typename Fmt::Ring Ring;
   typedef typename Fmt::Chunk Chunk;
@@ -194,6 +196,12 @@ struct Panel {
   }
 
   __device__ __forceinline__ void run(const StreamParams& p, const Slot& sl, uint8_t* lds, const PanelShare& part) {
+    NoWait none;
+    run(p, sl, lds, part, none);
+  }
+  // `wait`: for the activations, behind the requests of the first weights.
+  template <class Wait>
+  __device__ __forceinline__ void run(const StreamParams& p, const Slot& sl, uint8_t* lds, const PanelShare& part, Wait& wait) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), q = lane >> 4, r16 = lane & 15;
     const PanelWave share = panel_wave(p, part, wave);
     const int nb = part.group * p.nbw + share.nbi;
@@ -209,6 +217,7 @@ struct Panel {
     w.row = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(sl.w + (int64_t)(active ? nb : 0) * p.chunks * Fmt::BLOCK_BYTES), 0, p.chunks * Fmt::BLOCK_BYTES, 0x00020000);
     uint32_t codes, scales;
     Ring::lanes(w, lane, r16, (uint32_t)(uintptr_t)(lds_ptr_t)slot, codes, scales);
+    wait.look();
     Ring::request(w, share.c0, (lds_ptr_t)slot);
     // The split's pieces, dealt to its wavefronts in turn: piece j is rows 8 j .. 8 j + 7, lane l lands at its byte 16 l, the
     // 16-byte column (l & 7) of row 8 j + l / 8 - which holds the row's column (l & 7) ^ (row / 2 & 7), so that the sixteen
@@ -233,6 +242,7 @@ struct Panel {
       __builtin_amdgcn_sched_barrier(0);
     };
     const uint32_t at0 = (uint32_t)(uintptr_t)(lds_ptr_t)abuf + r16 * 128 + ((q ^ (r16 >> 1)) << 4), at1 = at0 ^ 64;
+    if (!wait.done()) return;  // nothing is computed or stored
     bring(0);
     bring(1);
     wait_vm<0>();
@@ -328,7 +338,9 @@ struct Panel {
     const f32x4_t s0 = column_scales(sl, nb, GATED ? 2 * nt : nt, q), s1 = GATED ? column_scales(sl, nb, 2 * nt + 1, q) : s0;
     const int64_t at = (EPI == EPI_FC2 ? (int64_t)p.order[pos] : pos) * p.out_stride + nb * (GATED ? 32 : 64) + 16 * nt + 4 * q;
     if (EPI != EPI_FC2 || p.out_bf16) {
-      *reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(p.out) + at) = rounded(v0, v1, s0, s1);
+      const u32x2_t v = rounded(v0, v1, s0, s1);
+      u32x2_t* to = reinterpret_cast<u32x2_t*>(reinterpret_cast<uint16_t*>(p.out) + at);
+      if constexpr (THROUGH) store_through(reinterpret_cast<uint64_t*>(to), __builtin_bit_cast(uint64_t, v)); else *to = v;
     } else {
       *reinterpret_cast<f32x4_t*>(reinterpret_cast<float*>(p.out) + at) = v0 * s0;
     }
@@ -364,7 +376,10 @@ struct Panel {
 #pragma unroll
       for (int u = 0; u < PASSES; u++) {
         const u32x4_t v = *reinterpret_cast<const u32x4_t*>(read + u * ROWS * LINE);
-        if (16 * t + ROWS * u + line < sl.rows) *reinterpret_cast<u32x4_t*>(out + row[PASSES * t + u] * pitch + offset) = v;
+        if (16 * t + ROWS * u + line < sl.rows) {
+          u32x4_t* to = reinterpret_cast<u32x4_t*>(out + row[PASSES * t + u] * pitch + offset);
+          if constexpr (THROUGH) store_through16(to, v); else *to = v;
+        }
       }
       asm volatile("" ::: "memory");
     };
@@ -518,13 +533,19 @@ inline size_t panel_lds_bytes(int mt, int ks, int nbw) {
 }
 
 
-template <class Fmt, int EPI, int MT>  // as many row tiles as the slot's rows need, MT at most (light slots do not come here)
-__device__ __forceinline__ void panel_tiles(const StreamParams& p, const Slot& sl, uint8_t* lds, const PanelShare& part) {
+template <class Fmt, int EPI, int MT, bool THROUGH, class Wait>  // as many row tiles as the slot's rows need, MT at most (light slots do not come here)
+__device__ __forceinline__ void panel_tiles(const StreamParams& p, const Slot& sl, uint8_t* lds, const PanelShare& part, Wait& wait) {
   if constexpr (MT > 1 + Fmt::LIGHT_ROWS / 16) {
-    if ((sl.rows + 15) >> 4 < MT) return panel_tiles<Fmt, EPI, MT - 1>(p, sl, lds, part);
+    if ((sl.rows + 15) >> 4 < MT) return panel_tiles<Fmt, EPI, MT - 1, THROUGH>(p, sl, lds, part, wait);
   }
-  Panel<Fmt, EPI, MT> panel;
-  panel.run(p, sl, lds, part);
+  Panel<Fmt, EPI, MT, THROUGH> panel;
+  panel.run(p, sl, lds, part, wait);
+}
+template <class Fmt, int EPI, int MOST, bool THROUGH, class Wait>
+__device__ __forceinline__ void panel_slot(const StreamParams& p, const Slot& sl, int group, uint8_t* lds, Wait& wait) {
+  const PanelShare part{group, 0, 1, 0};
+  if (sl.rows <= Fmt::LIGHT_ROWS) return Fmt::template light<EPI>(p, sl, group, lds, wait);
+  panel_tiles<Fmt, EPI, MOST, THROUGH>(p, sl, lds, part, wait);
 }
 
 // Routed calls: a plan's slots of up to 16 MOST rows. Workgroups go to the eight compute dies in turn: all of a slot's take
@@ -537,11 +558,39 @@ __global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void pane
   extern __shared__ __align__(16) uint8_t panel_lds[];
   const int die = blockIdx.x & 7, local = blockIdx.x >> 3, round = local / p.panel_groups, slot = 8 * round + die;
   if (slot >= p.panel_full) return;
-  const PanelShare part{local - round * p.panel_groups, 0, 1, 0};
   const Slot sl = slot_of<EPI>(p, slot);
   if (sl.rows <= 0) return;  // a slot the plan did not fill: the whole workgroup leaves
-  if (sl.rows <= Fmt::LIGHT_ROWS) return Fmt::template light<EPI>(p, sl, part.group, panel_lds);
-  panel_tiles<Fmt, EPI, MOST>(p, sl, panel_lds, part);
+  NoWait none;
+  panel_slot<Fmt, EPI, MOST, false>(p, sl, local - round * p.panel_groups, panel_lds, none);
+}
+
+// fc1 and fc2 of a routed call in one launch, as w3_fc12_kernel has them on the stream: fc2's workgroups fill the units that fc1's last
+// round leaves idle - where slots are few, a third of the time - and run beside its last ones instead of behind them. A die's workgroups are its slots'
+// in fc12_place's order, `lag` of its slots apart. h is written through to memory, and a slot's fc2 workgroups, which ask for their first weights
+// ahead of the wait, read it through their die's L2, which holds no older copy of it (a row of h is whole 256-byte pieces). The same sums
+// in the same order as the two launches: the same bits. Measured, two launches and one, the whole call, us: three-bit, skewed, 512 experts (2048, 512)
+// 1543 rows 231 and 217, 2048 rows 281 and 265, 256 (2560, 768) 1000 rows 247 and 227, 180 (1664, 384) 1000 rows 112 and 98, 64 (2048, 512) 2048 rows 196 and 168; even,
+// 128 (1024, 256) 1000 rows 84 and 73; NVFP4, 512 (1024, 2688) 2048 rows of 22 712 and 698, 200 rows 346 and 340, 256 (768, 1536) 500 rows of twelve 136
+// and 127, 16 (512, 1024) 40 rows of eight 48 and 46. No size of seventy gained by two.
+template <class Fmt, int EPI1, int MOST>
+__global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void panel_fc12_kernel(StreamParams p1, StreamParams p2, int rounds, int lag) {
+  extern __shared__ __align__(16) uint8_t panel_lds[];
+  __shared__ __align__(128) int outcome[32];  // (a whole 128 bytes: the panel's addresses of the halves of a row differ in one bit of its dynamic LDS)
+  const Fc12Place at = fc12_place(blockIdx.x >> 3, p1.panel_groups, p2.panel_groups, rounds, lag);
+  const int slot = 8 * at.slot + (blockIdx.x & 7);
+  if (slot >= p1.panel_full) return;
+  if (at.is_fc1) {
+    const Slot sl = slot_of<EPI1>(p1, slot);
+    if (sl.rows <= 0) return;
+    NoWait none;
+    panel_slot<Fmt, EPI1, MOST, true>(p1, sl, at.index, panel_lds, none);
+    fc12_arrive(p1, slot);
+  } else {
+    const Slot sl = slot_of<EPI_FC2>(p2, slot);
+    if (sl.rows <= 0) return;
+    SlotWait wait(p2, slot, outcome, false);
+    panel_slot<Fmt, EPI_FC2, MOST, false>(p2, sl, at.index, panel_lds, wait);
+  }
 }
 
 // How a dense call is cut: row tiles a slot, the shape of a workgroup, the tiles whose K is shared and among how many.
@@ -727,10 +776,9 @@ inline int panel_height(int64_t pairs, int64_t named, int experts, int shared_ro
   return tiles < 8 && moe_max_slots(pairs, experts, shared_rows, 16 * tiles) > PANEL_MAX_SLOTS ? 8 : tiles;
 }
 
-// Over a plan's slots of 16 `tiles` rows; `a_rows`: rows of the activation matrix. Four wavefronts a workgroup on four
+// What a routed call's launch needs of `p`; the workgroups of a slot. Four wavefronts a workgroup on four
 // blocks, two to four workgroups a compute unit: one's start and end lie beside the others' products.
-template <class Fmt, int EPI>
-static int launch_panel_routed(StreamParams& p, int tiles, int64_t slots, int64_t a_rows, hipStream_t stream) {
+inline int panel_routed(StreamParams& p, int tiles, int64_t slots, int64_t a_rows) {
   p.ks = 1;
   p.nbw = 4;
   set_split(p);
@@ -738,10 +786,39 @@ static int launch_panel_routed(StreamParams& p, int tiles, int64_t slots, int64_
   p.panel_groups = (p.n_blocks + p.nbw - 1) / p.nbw;
   p.a_bytes = (uint32_t)(a_rows * p.a_stride * 2);
   p.panel_full = (int)slots;
+  return panel_takes(a_rows, p.a_stride) ? HB_OK : HB_EINVAL;
+}
+
+// Over a plan's slots of 16 `tiles` rows; `a_rows`: rows of the activation matrix.
+template <class Fmt, int EPI>
+static int launch_panel_routed(StreamParams& p, int tiles, int64_t slots, int64_t a_rows, hipStream_t stream) {
+  if (int e = panel_routed(p, tiles, slots, a_rows)) return e;
   const int64_t grid = (slots + 7) / 8 * 8 * p.panel_groups;
-  if (!panel_takes(a_rows, p.a_stride) || grid > 0x7fffffff) return HB_EINVAL;
+  if (grid > 0x7fffffff) return HB_EINVAL;
   auto launch = [&](auto kernel) { HB_LAUNCH(kernel, dim3((unsigned)grid), dim3(64 * p.ks * p.nbw), panel_routed_lds<Fmt>(tiles, p.nbw), stream, p); };
   tiles == 3 ? launch(panel_tile_kernel<Fmt, EPI, 3>) : tiles == 5 ? launch(panel_tile_kernel<Fmt, EPI, 5>) : tiles == 8 ? launch(panel_tile_kernel<Fmt, EPI, 8>) : launch(panel_tile_kernel<Fmt, EPI, PANEL_SLOT_TILES>);
+  return HB_OK;
+}
+
+// Both layers of a call of `rows1` rows and `rows2` pairs (`plan`: the call's, whose counters the plan's launch has cleared). fc2 follows by the
+// slots whose fc1 workgroups fill the device twice: started sooner they stand waiting in fc1's places (three-bit, 512 experts (2048, 512) 1543
+// rows, of 85 slots a die 8 behind 247 us, 16 229, 24 217, 48 216; NVFP4, 512 (1024, 2688) 2048 rows, of 68, 4 704, 12 694 to 700, 32 702).
+template <class Fmt, int EPI1>
+static int launch_panel_fc12(StreamParams& p1, StreamParams& p2, int32_t* plan, int tiles, int64_t slots, int64_t rows1, int64_t rows2, int lag_forced, hipStream_t stream) {
+  if (int e = panel_routed(p1, tiles, slots, rows1)) return e;
+  if (int e = panel_routed(p2, tiles, slots, rows2)) return e;
+  const int rounds = (int)((slots + 7) / 8), both = p1.panel_groups + p2.panel_groups;
+  if ((int64_t)rounds * 8 * both > 0x7fffffff) return HB_EINVAL;
+  p1.done = p2.done = plan_done(plan, slots);
+  p2.done_need = p1.panel_groups;
+  p2.wait_spins = WAIT_SPINS;
+  p2.fault = plan + PLAN_FAULT;
+  const int resident = 256 * (tiles <= 3 ? 4 : tiles <= 5 ? 3 : 2);
+  const int lag = std::min(rounds, lag_forced ? lag_forced : std::max(1, 2 * resident / (8 * p1.panel_groups)));
+  auto launch = [&](auto kernel) {
+    HB_LAUNCH(kernel, dim3((unsigned)(8 * rounds * both)), dim3(64 * p1.nbw), panel_routed_lds<Fmt>(tiles, p1.nbw), stream, p1, p2, rounds, lag);
+  };
+  tiles == 3 ? launch(panel_fc12_kernel<Fmt, EPI1, 3>) : tiles == 5 ? launch(panel_fc12_kernel<Fmt, EPI1, 5>) : tiles == 8 ? launch(panel_fc12_kernel<Fmt, EPI1, 8>) : launch(panel_fc12_kernel<Fmt, EPI1, PANEL_SLOT_TILES>);
   return HB_OK;
 }
 

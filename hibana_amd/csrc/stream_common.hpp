@@ -75,6 +75,7 @@ __device__ __forceinline__ void store_through(float* at, float v) { __hip_atomic
 __device__ __forceinline__ float load_through(const float* at) { return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ uint16_t load_through(const uint16_t* at) { return __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
+__device__ __forceinline__ void store_through(uint64_t* at, uint64_t v) { __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 __device__ __forceinline__ void store_through(uint16_t* at, uint16_t v) { __hip_atomic_store(at, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
 
 // One arrival counter a slot, behind the plan's slot table (`slot_cap`: the table's entries, the launch's upper bound

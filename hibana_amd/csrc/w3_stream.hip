@@ -1190,10 +1190,10 @@ struct TileW3 {
   // ahead gave nothing: what the wavefronts wait for is each other's issue slots.
   static constexpr int LOW_ROWS = 22, MIDDLE_ROWS = 60, MIDDLE_ROWS_LARGE = 72, HIGH_ROWS = 88;  // panel_height's lines
   static constexpr int LIGHT_ROWS = ROWS_PER_SLOT;
-  template <int EPI>
-  static __device__ __forceinline__ void light(const StreamParams& p, const Slot& sl, int group, uint8_t* lds) {
+  template <int EPI, class Wait>
+  static __device__ __forceinline__ void light(const StreamParams& p, const Slot& sl, int group, uint8_t* lds, Wait& wait) {
     static_assert(BITS == 3 || epi_dense(EPI), "routed experts are three-bit");
-    if constexpr (BITS == 3) stream_workgroup<EPI, false, false, Ring>(p, sl, group, lds);
+    if constexpr (BITS == 3) stream_workgroup<EPI, false, false, Ring>(p, sl, group, lds, wait);
   }
   struct Part {
     uint32_t lo, hi;  // codebook bytes of weights 0 .. 3 and 4 .. 7
@@ -1635,6 +1635,13 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   f2.out = out_pairs;
   f2.out_stride = ex->hidden_out;
   f2.out_bf16 = pairs_bf16;
+  if (dense && g_tune.moe_fused != 2) {
+    if (int e = ex->gated ? launch_panel_fc12<TileW3<3>, EPI_FC1_GATED>(p, f2, ws.plan, tiles, slots, m, pairs + shared_rows, g_tune.moe_lag, stream)
+                          : launch_panel_fc12<TileW3<3>, EPI_FC1_RELU2>(p, f2, ws.plan, tiles, slots, m, pairs + shared_rows, g_tune.moe_lag, stream))
+      return e;
+    if (combine) moe_launch_combine(*combine, stream);
+    return launch_status();
+  }
   if (dense) {
     if (int e = ex->gated ? launch_panel_routed<TileW3<3>, EPI_FC1_GATED>(p, tiles, slots, m, stream) : launch_panel_routed<TileW3<3>, EPI_FC1_RELU2>(p, tiles, slots, m, stream)) return e;
     if (int e = launch_panel_routed<TileW3<3>, EPI_FC2>(f2, tiles, slots, pairs + shared_rows, stream)) return e;

@@ -1078,13 +1078,14 @@ int64_t busy_slots(int64_t pairs, int experts, int64_t slots) { return pairs < 2
 int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, int m, int topk, const MoeWorkspace& ws, void* out_pairs,
                 int pairs_bf16, hipStream_t stream, int experts_total) {
   const int64_t pairs = (int64_t)m * topk, named = experts_named(experts_total, ex->base, ex->experts);
-  // A dense contraction once an expert sees seven rows: the panel kernel; below that the 16-row slots of the weight stream. Measured,
-  // stream and panel, the two launches in us: 160 experts (512, 1536) 6 rows an expert 41.8 and 44.8, 8 rows 45.4 and 45.2, 14 rows 50.0
-  // and 46.6; 300 experts (640, 1280) 6 rows 67 and 66, 8 rows 75 and 68; 400 experts (896, 2048) 6 rows 170 and 177, 8 rows 190 and 178, 11 rows
-  // 224 and 194; the whole latent block of 512 experts (1024, 2688) 6 rows 344 and 326, 8 rows 380 and 341. A range of the experts sees its
-  // share of the pairs only, and its few slots fill the device a little later: 64 of 512 experts
-  // (1024, 2688), the summed experts alone, on slots of 128 rows 4 rows an expert 59 and 68, 8 rows 86 and 76.
-  const int64_t rows_min = ex->experts < named ? 8 : 7;
+  // A dense contraction once an expert sees three rows, or four of fewer than 768 columns: the panel kernel; below that the 16-row slots of the weight
+  // stream. Measured, stream and panel, the whole latent block in us: 128 experts (512, 1024) 3 rows an expert 52.5 and 53.3, 4 rows 55.2 and 54.1, 6 rows 60
+  // and 56; 300 (640, 1280) 3 rows 89 and 90, 4 rows 94 and 90; 256 (768, 1536) 3 rows 97 and 96, 5 rows 106 and 102; 400 (896, 2048) 3 rows 180
+  // and 175, 5 rows 202 and 190; 512 (1024, 2688) 3 rows 294 and 286, 5 rows 338 and 318, 7 rows 373 and 339. Few experts (`fill`: fc1's workgroups, a slot
+  // an expert) fill the device later, and a range of them sees its share of the pairs only: 64 of 512 experts
+  // (1024, 2688), the summed experts alone, two launches, on slots of 128 rows 4 rows an expert 59 and 68, 8 rows 86 and 76.
+  const int64_t fill = (int64_t)ex->experts * (((ex->gated ? 2 : 1) * ex->inter / 64 + 3) / 4);
+  const int64_t rows_min = ex->experts < named ? 8 : fill < 500 ? 7 : ex->hidden >= 768 ? 3 : 4;
   const bool dense = panel_takes(m, ex->hidden) && panel_takes(pairs, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
                      (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && pairs >= rows_min * named));
   const int tiles = panel_height<TileNvfp4>(pairs, named, ex->experts, 0, (ex->gated ? 2 : 1) * ex->inter / 64), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;

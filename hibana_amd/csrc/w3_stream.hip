@@ -1543,18 +1543,18 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
                 bool e4m3 = false, const CombineParams* combine = nullptr) {
   const int64_t pairs = (int64_t)m * topk, named = experts_named(experts_total, ex->base, ex->experts), local = pairs * ex->experts / named;
   const int shared_rows = shared ? m : 0;
-  // A dense contraction once an expert sees ten rows or more: the panel kernel's higher slots (E4M3 activations: the stream only).
-  // The stream pays for a pass a sixteen rows, the panel for two launches where the stream has one, which a call of few
-  // experts does not fill. The lines lie where neither even nor skewed routing loses. Measured, stream and panel (at its better
-  // height), the whole layer in us: 512 experts (2048, 512) 8 rows an expert 191 and 196 (skewed 152 and 131), 11 rows 215 and
-  // 211 (189 and 157), 14 rows 253 and 223 (225 and 176); 256 experts (2560, 768) 11 rows 210 and 192; 180 experts (1664, 384) 13 rows
-  // (0.55 M pairs x blocks) 88 and 88, 16 rows (0.67 M) 98 and 90; 300 experts (1280, 384) 13 rows 95 and 94, 16 rows 111 and 99; 96 experts (2560,
-  // 768) 13 rows (0.9 M) 100 and 107, 16 rows 128 and 119; 64 experts (2048, 512) 25 rows (0.6 M) 76 and 83; 128 experts (1024, 256)
-  // 24 rows 63 and 66, 32 rows 70 and 69, 40 rows 77 and 73. A range of the experts sees its share of the pairs only.
-  const int64_t expert_blocks = (int64_t)((ex->gated ? 2 : 1) * ex->inter / W3_BLOCK_ROWS) * (ex->hidden / W3_CHUNK) + (int64_t)(ex->hidden_out / W3_BLOCK_ROWS) * (ex->inter / W3_CHUNK);
+  // A dense contraction once an expert sees some rows: the panel kernel's higher slots (E4M3 activations: the stream only).
+  // The stream pays for a pass a sixteen rows, the panel for longer workgroups, which a call of few experts does not fill: `fill` is fc1's, a
+  // slot an expert. The lines lie where neither even nor skewed routing loses. Measured, even and (skewed) routing, stream and panel, the
+  // whole layer in us, experts (hidden, inter), fill: 512 (2048, 512), 2048, 5 rows an expert 175 and 166 (117 and 99), 9 rows 198 and 192 (167 and 125);
+  // 256 (2560, 768), 1536, 5 rows 164 and 155 (122 and 101); 300 (1280, 384), 900, 5 rows 72 and 72 (59 and 61), 7 rows 77 and 76 (69 and 64); 180 (1664, 384), 540,
+  // 5 rows 70 and 70 (61 and 62), 7 rows 72 and 71 (67 and 63); 96 (2560, 768), 576, 11 rows 93 and 96 (97 and 92), 18 rows 128 and 111 (125 and 106); 64
+  // (2048, 512), 256, 22 rows 74 and 78 (73 and 75), 27 rows 81 and 78 (81 and 78); 128 (1024, 256), 256, 18 rows 55 and 55 (54 and 54), 22 rows 61 and 59 (57 and 59),
+  // 27 rows 65 and 60 (64 and 61). A range of the experts sees its share of the pairs only.
+  const int64_t fill = (int64_t)ex->experts * (((ex->gated ? 2 : 1) * ex->inter / W3_BLOCK_ROWS + 3) / 4);
+  const int rows_min = fill >= 1500 ? 5 : fill >= 500 ? ex->experts >= 150 ? 7 : 16 : ex->experts < named ? 48 : 26;
   const bool dense = !e4m3 && panel_takes(m, ex->hidden) && panel_takes(pairs + shared_rows, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
-                     (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && (pairs >= (ex->experts < named ? 48 : 32) * named || (pairs >= 16 * named && local * expert_blocks >= 650000) ||
-                                                                                        (pairs >= 10 * named && local * expert_blocks >= 1400000))));
+                     (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && pairs >= rows_min * named));
   const int tiles = panel_height<TileW3<3>>(pairs, named, ex->experts, shared_rows, (ex->gated ? 2 : 1) * ex->inter / W3_BLOCK_ROWS), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;
   // Under a budget the table ends behind the experts the selection can name: the launches' grids reach over all of it, and a
   // workgroup without rows is not free (40 rows of 10, a cap of 60 of 512 experts: 53.5 us before, 53.2 so). What a call of

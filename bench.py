@@ -104,7 +104,7 @@ def latent_prefill(args) -> dict:
     """BASELINE config 4 (not the headline line; `--config 4`): the NVFP4 latent-MoE layer on a prefill chunk of 2048
     tokens - hidden 4096 projected to latent 1024, 512 ReLU^2 experts of intermediate 2688, top-22 by sigmoid scores.
     A step is the whole block (fused router|fc1_latent GEMM, routing, plan, the two expert GEMMs on the panel kernel,
-    combine, fc2_latent GEMM); the roofline entry is the fc1 expert GEMM against the dense BF16 MFMA peak."""
+    combine, fc2_latent GEMM); the roofline entry is the launch of the two expert GEMMs against the dense BF16 MFMA peak."""
     import torch
 
     from hibana_amd import _lib, synthetic
@@ -124,7 +124,7 @@ def latent_prefill(args) -> dict:
         block(x)
     torch.cuda.synchronize()
     hip = Hip()
-    names = ["route", "plan count", "plan place", "fc1", "fc2", "combine"]  # 45 056 pairs: the plan is two launches
+    names = ["route", "plan count", "plan place", "fc1 + fc2", "combine"]  # 45 056 pairs: the plan is two launches
     per_kernel = {n: [] for n in names}
     for rep in range(4):
         evs = hip.events(2 * len(names))
@@ -143,8 +143,8 @@ def latent_prefill(args) -> dict:
     times = replay_times(graph, steps)
     elapsed = median(times) * 1e-3 * steps
     del outs
-    gemm_flops = tokens * topk * 2 * inter * latent  # one expert GEMM (fc1 or fc2), useful flops
-    fc1_ms = mean(per_kernel["fc1"])
+    gemm_flops = 2 * tokens * topk * 2 * inter * latent  # both expert GEMMs, useful flops
+    gemm_ms = mean(per_kernel["fc1 + fc2"])
     mfma_tflops = mfma_rate_tflops(dev)
     cpu, check = None, None
     if not args.no_cpu:
@@ -159,10 +159,10 @@ def latent_prefill(args) -> dict:
         "config": {"workload": "BASELINE config 4: NVFP4 latent-MoE layer, 2048 tokens, hidden 4096 -> latent 1024, 512 experts x inter 2688, "
                                "ReLU^2, top-22 sigmoid routing of N(0,1) logits, no shared expert",
                    "timed_as": "replays of one HIP graph of all steps; value and ms_per_step are the median replay"},
-        "roofline": {"bound": "mfma", "kernel": "panel_tile_kernel<TileNvfp4, fc1 relu2>", "achieved": gemm_flops / (fc1_ms * 1e-3) / 1e12,
-                     "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": gemm_flops / (fc1_ms * 1e-3) / 1e12 / MFMA_BF16_PEAK_TFLOPS,
-                     "traffic": None, "launch_flops": gemm_flops, "launch_ms": fc1_ms, "peak_measured": mfma_tflops,
-                     "frac_of_measured": gemm_flops / (fc1_ms * 1e-3) / 1e12 / mfma_tflops,
+        "roofline": {"bound": "mfma", "kernel": "panel_fc12_tile_kernel<TileNvfp4, relu2>", "achieved": gemm_flops / (gemm_ms * 1e-3) / 1e12,
+                     "peak": MFMA_BF16_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": gemm_flops / (gemm_ms * 1e-3) / 1e12 / MFMA_BF16_PEAK_TFLOPS,
+                     "traffic": None, "launch_flops": gemm_flops, "launch_ms": gemm_ms, "peak_measured": mfma_tflops,
+                     "frac_of_measured": gemm_flops / (gemm_ms * 1e-3) / 1e12 / mfma_tflops,
                      "peak_measured_how": "BF16 16x16x32 MFMAs on registers alone in this run (hb_debug_mfma_rate)"},
         "layer_chain": {"kernel_ms": {n: mean(v) for n, v in per_kernel.items()}},
         "decode_calls": small,
@@ -174,7 +174,7 @@ def latent_prefill(args) -> dict:
 
 def latent_small_only(args) -> dict:
     """`--config 4 --small-rows M`: config 4's block with the shared expert at M rows through the small-call kernels
-    alone (a profiling mode: its kernel trace shows the six launches of a decode or verify call)."""
+    alone (a profiling mode: its kernel trace shows the five launches of a decode or verify call)."""
     import torch
 
     from hibana_amd import synthetic
@@ -204,7 +204,7 @@ def latent_small_only(args) -> dict:
 
 def latent_small_calls(block, ex, hidden: int, dev, g, shared_inter: int = 5376):
     """The same block with a shared expert of intermediate 5376 at 1, 4 and 16 rows (decode and verify calls):
-    microseconds a call through the small-call kernels (router, block: six launches) and through the operators a
+    microseconds a call through the small-call kernels (five launches) and through the operators a
     longer call uses (two GEMMs, routing, plan, two expert layers, combine, the shared expert's two linears: nine), each
     as replays of a graph of 32 calls over 8 inputs."""
     import torch

@@ -573,7 +573,7 @@ __global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void pane
 // 128 (1024, 256) 1000 rows 84 and 73; NVFP4, 512 (1024, 2688) 2048 rows of 22 712 and 698, 200 rows 346 and 340, 256 (768, 1536) 500 rows of twelve 136
 // and 127, 16 (512, 1024) 40 rows of eight 48 and 46. No size of seventy gained by two.
 template <class Fmt, int EPI1, int MOST>
-__global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void panel_fc12_kernel(StreamParams p1, StreamParams p2, int rounds, int lag) {
+__global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void panel_fc12_tile_kernel(StreamParams p1, StreamParams p2, int rounds, int lag) {
   extern __shared__ __align__(16) uint8_t panel_lds[];
   __shared__ __align__(128) int outcome[32];  // (a whole 128 bytes: the panel's addresses of the halves of a row differ in one bit of its dynamic LDS)
   const Fc12Place at = fc12_place(blockIdx.x >> 3, p1.panel_groups, p2.panel_groups, rounds, lag);
@@ -818,7 +818,7 @@ static int launch_panel_fc12(StreamParams& p1, StreamParams& p2, int32_t* plan, 
   auto launch = [&](auto kernel) {
     HB_LAUNCH(kernel, dim3((unsigned)(8 * rounds * both)), dim3(64 * p1.nbw), panel_routed_lds<Fmt>(tiles, p1.nbw), stream, p1, p2, rounds, lag);
   };
-  tiles == 3 ? launch(panel_fc12_kernel<Fmt, EPI1, 3>) : tiles == 5 ? launch(panel_fc12_kernel<Fmt, EPI1, 5>) : tiles == 8 ? launch(panel_fc12_kernel<Fmt, EPI1, 8>) : launch(panel_fc12_kernel<Fmt, EPI1, PANEL_SLOT_TILES>);
+  tiles == 3 ? launch(panel_fc12_tile_kernel<Fmt, EPI1, 3>) : tiles == 5 ? launch(panel_fc12_tile_kernel<Fmt, EPI1, 5>) : tiles == 8 ? launch(panel_fc12_tile_kernel<Fmt, EPI1, 8>) : launch(panel_fc12_tile_kernel<Fmt, EPI1, PANEL_SLOT_TILES>);
   return HB_OK;
 }
 

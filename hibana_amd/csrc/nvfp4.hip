@@ -809,6 +809,7 @@ static bool fc12_serves(int64_t pairs, int local, int64_t experts, int n_blocks,
 // beside them, or null.
 template <int EPI1>
 static int launch_fc12(StreamParams& p1, StreamParams& p2, int64_t slots, int64_t busy, StreamParams* dense, hipStream_t stream) {
+  if (!fc12_apart(p1)) return HB_EINVAL;  // (the caller then takes two)
   if (int e = shape_nvfp4(p1, busy)) return e;
   if (int e = shape_nvfp4(p2, busy)) return e;
   const int waves = std::max(p1.ks * p1.nbw, p2.ks * p2.nbw);  // one workgroup size for both: all powers of two
@@ -1095,7 +1096,7 @@ int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, i
   const int64_t est = busy_slots(pairs, ex->experts, slots);
   StreamParams p, f2;
   expert_params(ex, x, m, topk, ws, out_pairs, pairs_bf16, p, f2);
-  if (dense && g_nvfp4_fused != 2) {
+  if (dense && g_nvfp4_fused != 2 && fc12_apart(p)) {
     if (int e = ex->gated ? launch_panel_fc12<TileNvfp4, EPI_FC1_GATED>(p, f2, ws.plan, tiles, slots, m, pairs, g_nvfp4_lag, stream)
                           : launch_panel_fc12<TileNvfp4, EPI_FC1_RELU2>(p, f2, ws.plan, tiles, slots, m, pairs, g_nvfp4_lag, stream))
       return e;

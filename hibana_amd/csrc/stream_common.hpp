@@ -99,6 +99,10 @@ __device__ __forceinline__ bool await_count(const int32_t* at, int need, int spi
   return there;
 }
 
+// Whether one launch may hold fc1 (`p1`) and fc2: fc2 reads h through its die's L2, which must hold no older copy of a slot's rows, so no row
+// may share a cache line with a neighbour's that another slot read before (a caller's workspace need only lie on 16 bytes).
+inline bool fc12_apart(const StreamParams& p1) { return aligned(p1.out, 256) && p1.out_stride % 128 == 0; }
+
 // fc1 and fc2 of a routed call in one launch (w3_fc12_kernel says why, and why the waits end). Which workgroup of which layer and slot a
 // grid index is: slot-major, fc2 of a slot `lag` slots behind its fc1.
 struct Fc12Place {

@@ -1635,7 +1635,7 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   f2.out = out_pairs;
   f2.out_stride = ex->hidden_out;
   f2.out_bf16 = pairs_bf16;
-  if (dense && g_tune.moe_fused != 2) {
+  if (dense && g_tune.moe_fused != 2 && fc12_apart(p)) {
     if (int e = ex->gated ? launch_panel_fc12<TileW3<3>, EPI_FC1_GATED>(p, f2, ws.plan, tiles, slots, m, pairs + shared_rows, g_tune.moe_lag, stream)
                           : launch_panel_fc12<TileW3<3>, EPI_FC1_RELU2>(p, f2, ws.plan, tiles, slots, m, pairs + shared_rows, g_tune.moe_lag, stream))
       return e;
@@ -1676,7 +1676,7 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
     p.a2_scale = ws.x2s;
   }
   // more than one token, weight-only: fc1 and fc2 as one launch when their workgroups have the same shape
-  if (!e4m3 && m > 1 && g_tune.moe_fused != 2) {
+  if (!e4m3 && m > 1 && g_tune.moe_fused != 2 && fc12_apart(p)) {
     StreamParams q1 = p, q2 = f2;
     if (shape_stream(q1, est, l1) == HB_OK && shape_stream(q2, est, l2) == HB_OK && q1.ks * q1.nbw == q2.ks * q2.nbw) {
       const int groups1 = (q1.n_blocks + q1.nbw - 1) / q1.nbw, groups2 = (q2.n_blocks + q2.nbw - 1) / q2.nbw;

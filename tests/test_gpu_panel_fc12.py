@@ -51,3 +51,26 @@ def test_one_launch_has_the_bits_of_two(form, gated, hidden, inter, m, e):
         with _forced(**{fused: 2}):
             two = call().clone()
     assert torch.isfinite(two).all() and all(torch.equal(o, two) for o in one)
+
+
+# A caller's workspace need only lie on sixteen bytes: rows of h then share cache lines, and fc2 may not read them in the launch that writes them.
+@pytest.mark.parametrize("tile", [1, 2])
+@pytest.mark.parametrize("form", ["w3", "nvfp4"])
+def test_a_workspace_off_the_cache_lines_gives_the_same_bits(form, tile, monkeypatch):
+    from hibana_amd import _lib
+    m, e, hidden, inter = 40, 8, 1024, 384
+    x = torch.randn(m, hidden, generator=torch.Generator().manual_seed(m)).bfloat16().cuda()
+    ids, w = _routing(m, e, m + e)
+    if form == "w3":
+        from hibana_amd.kernels import w3_moe
+        ex, _ = random_experts(e, hidden, inter, True, 3)
+        call, keys = lambda: w3_moe.moe_layer(ex, x, ids, w), {"w3_tile": tile}
+    else:
+        ex, _ = _experts(e, hidden, inter, True, 5)
+        call, keys = lambda: ex(x, ids, w), {"nvfp4_tile": tile, "nvfp4_fused": 1}
+    with _forced(**keys):
+        want = call().clone()
+        asked = []
+        monkeypatch.setattr(_lib, "workspace", lambda device, need, kind="moe": asked.append(torch.zeros(need + 16, dtype=torch.uint8, device=device)[16:]) or asked[-1])
+        got = call().clone()
+    assert asked and all(a.data_ptr() % 256 == 16 for a in asked) and torch.equal(got, want)

@@ -881,97 +881,147 @@ __global__ __launch_bounds__(1024) void w3_part_kernel(StreamParams p) {
   }
 }
 
+// A body that hands over the sums of every K split of the dense launch (`Splits`) by itself: at a split's last chunk they go to the
+// workgroup's table in LDS and start again from zero, so that a wavefront may take several splits in a row and the table holds what as many
+// wavefronts would have left. A lane's part of a split, FEW: the four rows' sums over the four groups, (0 + 1) + (2 + 3) as finish_few adds them, of
+// one tile (two tiles: of two rows of one) - else what its accumulators hold. Written as statements of their own: the compiler would have the
+// LDS-direct loads of the weights wait ahead of its own LDS stores.
+template <bool FEW, int TILES>
+constexpr int split_bytes() { return (FEW ? 256 : 1024) * TILES; }
+template <class Acts, bool FEW, int T0, int T1>
+struct Splits : Acts {
+  uint32_t to;          // LDS byte address of the lane's part of the split under way
+  int left, base, more; // chunks it has left; chunks of the next ones, one more in the next `more` of them
+  __device__ __forceinline__ void hand_over(f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3) {
+    f32x4_t* const all[4] = {&acc0, &acc1, &acc2, &acc3};
+    if constexpr (!FEW) {
+#pragma unroll
+      for (int t = T0; t < T1; t++) asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(to), "v"(*all[t]), "n"(1024 * (t - T0)));
+    } else {
+      float pair[4][2];  // [row][pair of tiles]: lanes' quarters: groups 0 + 1 of the first and of the second tile, groups 2 + 3 of them
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+#pragma unroll
+        for (int t = T0; t < T1; t += 2) {
+          const auto x = __builtin_amdgcn_permlane16_swap(__float_as_uint((*all[t])[r]), __float_as_uint((*all[t + 1])[r]), false, false);
+          pair[r][(t - T0) / 2] = __uint_as_float(x[0]) + __uint_as_float(x[1]);
+        }
+      auto whole = [](float a, float b) {  // quarters: a's two tiles, b's two tiles
+        const auto x = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        return __uint_as_float(x[0]) + __uint_as_float(x[1]);
+      };
+      if constexpr (T1 - T0 == 4) {
+        const f32x4_t v = {whole(pair[0][0], pair[0][1]), whole(pair[1][0], pair[1][1]), whole(pair[2][0], pair[2][1]), whole(pair[3][0], pair[3][1])};
+        asm volatile("ds_write_b128 %0, %1" ::"v"(to), "v"(v));
+      } else {
+        typedef __attribute__((ext_vector_type(2))) float f32x2_t;
+        const f32x2_t v = {whole(pair[0][0], pair[1][0]), whole(pair[2][0], pair[3][0])};
+        asm volatile("ds_write_b64 %0, %1" ::"v"(to), "v"(v));
+      }
+    }
+    acc0 = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    acc1 = acc2 = acc3 = acc0;
+    to += split_bytes<FEW, T1 - T0>();
+    more--;
+    left = base + (more > 0 ? 1 : 0);
+  }
+  template <int ODD, bool MORE2, bool MORE1, class C>
+  __device__ __forceinline__ void step(const C& ch, int i, f32x4_t& acc0, f32x4_t& acc1, f32x4_t& acc2, f32x4_t& acc3, const Slot& sl) {
+    Acts::template step<ODD, MORE2, MORE1>(ch, i, acc0, acc1, acc2, acc3, sl);
+    if (--left == 0) hand_over(acc0, acc1, acc2, acc3);  // uniform
+  }
+};
+
 // The gate | up projection of a dense SwiGLU block of at most sixteen rows together with what its 3-bit down projection takes: silu(gate) * up
 // as the BF16 tensor expression rounds it, then E4M3 codes and a scale a 32-group (p.oq, p.oq_scale [rows, p.out_stride]).
 // A workgroup holds the 64-row block of gate rows and the block of up rows of the same 64 columns of h (PARTS 2: half of either's
-// tiles, 32 columns), K split p.ks ways each, so that a pair of values meets in the exchange of the K splits through LDS
-// and neither leaves the compute unit. The sums are those of the dense kernels at the same K split, in their order.
+// tiles, 32 columns), so that a pair of values meets in LDS and neither leaves the compute unit. K has the p.ks splits of the dense launch, `run` of
+// them one after the other a wavefront (Splits), and the sums are the dense launch's bit for bit.
+struct GateUp {
+  int half_blocks, pair_blocks;  // h's 64-column blocks; > 0: gate and up alternate in runs of that many blocks
+  int ways, run;                 // wavefronts a block; splits a wavefront: ways * run == p.ks
+};
 template <bool FEW, int T0, int T1>
-__device__ __forceinline__ void gate_up_block(const StreamParams& p, const Slot& sl, int gate, int up, int column0, int lane, int wave, uint8_t* rings) {
-  constexpr int GROUPS = (T1 - T0) / 2, STRIDE = RING_BYTES / 4;  // 32-column groups of h
+__device__ __forceinline__ void gate_up_block(const StreamParams& p, const GateUp& g, const Slot& sl, int gate, int up, int column0, int lane, int wave,
+                                              uint8_t* rings) {
+  constexpr int TILES = T1 - T0, GROUPS = TILES / 2, SPLIT = split_bytes<FEW, TILES>() / 4;  // 32-column groups of h; floats a split
   const int q = lane >> 4, r16 = lane & 15;
-  const WaveShare share = wave_share(p, wave);
-  const int nb = share.nbi ? up : gate;
+  const int second = wave >= g.ways ? 1 : 0, s0 = (wave - second * g.ways) * g.run, s1 = s0 + g.run;  // the wavefront's splits
+  const int nb = second ? up : gate, c0 = s0 * p.chunks_base + min(s0, p.chunks_rem), c1 = s1 * p.chunks_base + min(s1, p.chunks_rem);
   // the row scales of what this lane will add up, asked for ahead of the chunks: FEW: lanes 0 .. 31 a group's gate rows, 32 .. 63 its
   // up rows; else both tiles of both
-  float scale[GROUPS][4];
-#pragma unroll
-  for (int g = 0; g < GROUPS; g++) {
-    const int t = T0 + 2 * g;
+  f32x4_t scale0 = {0.f, 0.f, 0.f, 0.f}, scale1 = scale0;  // of the first and the second group (an array of both would be indexed, and so held in memory)
+  auto scales_of = [&](f32x4_t& to, int t) {
     if constexpr (FEW) {
-      scale[g][0] = sl.rs[(lane < 32 ? gate : up) * 64 + 16 * t + (lane & 31)];
+      to.x = sl.rs[(lane < 32 ? gate : up) * 64 + 16 * t + (lane & 31)];
     } else {
 #pragma unroll
-      for (int j = 0; j < 4; j++) scale[g][j] = sl.rs[(j < 2 ? gate : up) * 64 + 16 * (t + (j & 1)) + r16];
+      for (int j = 0; j < 4; j++) to[j] = sl.rs[(j < 2 ? gate : up) * 64 + 16 * (t + (j & 1)) + r16];
     }
-  }
-  f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0, acc2 = acc0, acc3 = acc0;
+  };
+  scales_of(scale0, T0);
+  if constexpr (GROUPS == 2) scales_of(scale1, T0 + 2);
   uint8_t* ring = rings + wave * RING_BYTES;
-  if constexpr (T1 - T0 == 4) {
-    if constexpr (FEW) {
-      stream_block<EPI_DENSE, FewActs, W3Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
-    } else {
-      stream_block<EPI_DENSE, FullActs, W3Ring>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
-    }
-  } else if constexpr (FEW) {
-    stream_block<EPI_DENSE, FewActsPart<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+  const float* const sums = reinterpret_cast<const float*>(rings + 2 * g.ways * RING_BYTES);  // [gate, up][split]
+  f32x4_t acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = acc0, acc2 = acc0, acc3 = acc0;
+  auto stream = [&](auto acts, auto ring_of) {
+    acts.to = (uint32_t)(uintptr_t)(lds_ptr_t)(rings + 2 * g.ways * RING_BYTES) + (second * p.ks + s0) * (4 * SPLIT) + lane * (FEW ? 4 * TILES : 16);
+    acts.base = p.chunks_base;
+    acts.more = p.chunks_rem - s0;
+    acts.left = acts.base + (acts.more > 0 ? 1 : 0);
+    stream_block<EPI_DENSE, decltype(acts), decltype(ring_of)>(p, sl, 0, nb, c0, c1, lane, ring, acc0, acc1, acc2, acc3, acts);
+  };
+  if constexpr (TILES == 4) {
+    stream(Splits<typename std::conditional<FEW, FewActs, FullActs>::type, FEW, T0, T1>{}, W3Ring{});
   } else {
-    stream_block<EPI_DENSE, FullActsPart<T0, T1>, W3RingPart<2, T0, T1>>(p, sl, 0, nb, share.c0, share.c1, lane, ring, acc0, acc1, acc2, acc3);
+    stream(Splits<typename std::conditional<FEW, FewActsPart<T0, T1>, FullActsPart<T0, T1>>::type, FEW, T0, T1>{}, W3RingPart<2, T0, T1>{});
   }
-  const f32x4_t all[4] = {acc0, acc1, acc2, acc3};
-  float* first = reinterpret_cast<float*>(rings);
-  float* mine = first + wave * STRIDE;
-#pragma unroll
-  for (int t = T0; t < T1; t++)
-#pragma unroll
-    for (int r = 0; r < 4; r++) mine[(t * 4 + r) * 64 + lane] = all[t][r];
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (hand_over's writes: the compiler does not count them)
   __syncthreads();
-  const float* const second = first + p.ks * STRIDE;  // the up block's splits
   // a unit of work: accumulator register r of a group's tiles (FEW: row r of the slot)
-  for (int unit = wave; unit < (FEW ? sl.rows : min(4, sl.rows)) * GROUPS; unit += 2 * p.ks) {  // uniform
-    const int r = GROUPS == 2 ? unit >> 1 : unit, g = GROUPS == 2 ? unit & 1 : 0, t = T0 + 2 * g;
+  for (int unit = wave; unit < (FEW ? sl.rows : min(4, sl.rows)) * GROUPS; unit += 2 * g.ways) {  // uniform
+    const int r = GROUPS == 2 ? unit >> 1 : unit, gr = GROUPS == 2 ? unit & 1 : 0, t = 2 * gr;
+    const f32x4_t scale = gr ? scale1 : scale0;
     if constexpr (FEW) {
-      const float* at = (lane < 32 ? first : second) + ((t + (q & 1)) * 4 + r) * 64 + r16;
+      const int tile = t + (q & 1);
+      const float* at = sums + (lane < 32 ? 0 : p.ks * SPLIT) + (TILES == 4 ? (tile * 16 + r16) * 4 + r : (((r & 1) * 2 + tile) * 16 + r16) * 2 + (r >> 1));
       float v = 0.f;
-      for (int s = 0; s < p.ks; s++, at += STRIDE) v += (at[0] + at[16]) + (at[32] + at[48]);
-      const float y = through_bf16(v * (GROUPS == 2 && g ? scale[GROUPS - 1][0] : scale[0][0])), other = __shfl_xor(y, 32);
+      for (int s = 0; s < p.ks; s++, at += SPLIT) v += *at;
+      const float y = through_bf16(v * scale.x), other = __shfl_xor(y, 32);
       const float h = silu_chain(lane < 32 ? y : other, lane < 32 ? other : y);
       float amax = row16_max(fabsf(h));
       amax = fmaxf(amax, __shfl_xor(amax, 16));
-      if (lane < 32) store_quantized(p, r, column0 + 32 * g + lane, h, amax, lane == 0);
+      if (lane < 32) store_quantized(p, r, column0 + 32 * gr + lane, h, amax, lane == 0);
     } else {
       const int i = 4 * q + r;
       float v[4] = {0.f, 0.f, 0.f, 0.f};
-      for (int s = 0; s < p.ks; s++) {
-        const int at = s * STRIDE + (t * 4 + r) * 64 + lane;
-        v[0] += first[at], v[1] += first[at + 256], v[2] += second[at], v[3] += second[at + 256];
-      }
+      const float *first = sums + (t * 64 + lane) * 4 + r, *other = first + p.ks * SPLIT;
+      for (int s = 0; s < p.ks; s++, first += SPLIT, other += SPLIT) v[0] += first[0], v[1] += first[256], v[2] += other[0], v[3] += other[256];
       if (i >= sl.rows) continue;  // whole rows of lanes
 #pragma unroll
-      for (int j = 0; j < 4; j++) v[j] = through_bf16(v[j] * (GROUPS == 2 && g ? scale[GROUPS - 1][j] : scale[0][j]));
+      for (int j = 0; j < 4; j++) v[j] = through_bf16(v[j] * scale[j]);
       const float h0 = silu_chain(v[0], v[2]), h1 = silu_chain(v[1], v[3]);
       const float amax = row16_max(fmaxf(fabsf(h0), fabsf(h1)));
-      store_quantized(p, i, column0 + 32 * g + r16, h0, amax, r16 == 0);
-      store_quantized(p, i, column0 + 32 * g + 16 + r16, h1, amax, false);
+      store_quantized(p, i, column0 + 32 * gr + r16, h0, amax, r16 == 0);
+      store_quantized(p, i, column0 + 32 * gr + 16 + r16, h1, amax, false);
     }
   }
 }
-// h's 64-column block b: its gate rows are block b (of the first half; `pair_blocks` > 0: gate and up alternate in runs of that many
-// blocks), its up rows the block that many further on.
+constexpr int GATE_UP_WAYS = 4;  // at most
 template <bool FEW, int PARTS>
-__global__ __launch_bounds__(1024) void w3_fc_gate_up_kernel(StreamParams p, int half_blocks, int pair_blocks) {
+__global__ __launch_bounds__(64 * 2 * GATE_UP_WAYS) void w3_fc_gate_up_kernel(StreamParams p, GateUp g) {
   extern __shared__ __align__(16) uint8_t rings[];
   const int die = blockIdx.x & 7, local = blockIdx.x >> 3, part = local % PARTS, b = PARTS == 1 ? (int)blockIdx.x : local / PARTS * 8 + die;
-  if (b >= half_blocks) return;
-  const int gate = pair_blocks ? b / pair_blocks * 2 * pair_blocks + b % pair_blocks : b, up = gate + (pair_blocks ? pair_blocks : half_blocks);
+  if (b >= g.half_blocks) return;
+  const int gate = g.pair_blocks ? b / g.pair_blocks * 2 * g.pair_blocks + b % g.pair_blocks : b, up = gate + (g.pair_blocks ? g.pair_blocks : g.half_blocks);
   const Slot sl = slot_of<EPI_DENSE>(p, 0);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if constexpr (PARTS == 1) {
-    gate_up_block<FEW, 0, 4>(p, sl, gate, up, 64 * b, lane, wave, rings);
+    gate_up_block<FEW, 0, 4>(p, g, sl, gate, up, 64 * b, lane, wave, rings);
   } else if (part == 0) {
-    gate_up_block<FEW, 0, 2>(p, sl, gate, up, 64 * b, lane, wave, rings);
+    gate_up_block<FEW, 0, 2>(p, g, sl, gate, up, 64 * b, lane, wave, rings);
   } else {
-    gate_up_block<FEW, 2, 4>(p, sl, gate, up, 64 * b + 32, lane, wave, rings);
+    gate_up_block<FEW, 2, 4>(p, g, sl, gate, up, 64 * b + 32, lane, wave, rings);
   }
 }
 
@@ -1300,14 +1350,18 @@ static void shape_dense(StreamParams& p) {
 // sixteen rows, replayed graphs, eight rows: 1024 x 4096 7.8 -> 5.5 us, 4096 x 5120 9.5 -> 6.6, 8192 x 5120 9.9 -> 7.5; the dense
 // block of ten rows (4096, 8192), whose down projection takes E4M3 activations, 31.2 -> 24.8.
 constexpr int PARTS_BLOCKS = 128;
+// The shape of a dense call of one slot whose shape nobody forces; whether it runs in parts.
+static bool shape_one_slot(StreamParams& p, int bits) {
+  const bool few = p.m <= FEW_ROWS, parted = bits == 3 && p.n_blocks <= PARTS_BLOCKS && !(few && p.no_few);
+  if (!p.aq && !(parted && few)) shape_dense(p);
+  return parted;
+}
 template <int EPI>
 static int launch_stream(StreamParams& p, int64_t slots, int64_t busy_slots, Launch want, hipStream_t stream, int bits = 3) {
   if (int e = shape_stream(p, busy_slots, want)) return e;
   if constexpr (EPI == EPI_DENSE) {
-    const bool chosen = slots == 1 && !want.ks && !want.nbw && !p.a2, few = p.m <= FEW_ROWS;
-    const bool parted = bits == 3 && p.n_blocks <= PARTS_BLOCKS && !(few && p.no_few);
-    if (chosen && !p.aq && !(parted && few)) shape_dense(p);
-    if (chosen && parted) {
+    const bool few = p.m <= FEW_ROWS;
+    if (slots == 1 && !want.ks && !want.nbw && !p.a2 && shape_one_slot(p, bits)) {
       p.nbw = 1;
       const int parts = p.n_blocks <= PARTS_BLOCKS / 2 ? 4 : 2;
       const dim3 blocks((unsigned)((p.n_blocks + 7) / 8 * 8 * parts));
@@ -1445,31 +1499,41 @@ extern "C" int hb_w3_gemm_e4m3(const void* xq, const float* x_scale, int m, cons
 
 // The dense SwiGLU block on its 3-bit copies. Gate | up, the SiLU product and its E4M3 rounding are one launch up to sixteen rows
 // (w3_fc_gate_up_kernel), which keeps gate | up out of memory and costs two launches' starts and ends less: the block (5120, 25600) of four rows
-// 51.4 -> 45.9 us, (4096, 8192) of one and sixteen 18.9 -> 15.4 and 28.0 -> 26.5, (1024, 1024) of four 10.6 -> 8.2 (replayed graphs on cycled weights).
-// Its shape, by h's 64-column blocks B and the chunks of K; swept over 16 to 512 blocks, 8 to 40 chunks, one to sixteen rows, times of the three
+// 52.7 -> 50.1 us, (4096, 8192) of one and sixteen 19.1 -> 15.5 and 28.6 -> 26.9, (1024, 1024) of four 10.5 -> 8.1 (replayed graphs on cycled weights).
+// Its splits of K are the dense launch's, so that its bits are; a wavefront takes `run` of them, and what it hands over between them costs 2 to
+// 4 % of the launch (a K split of its own, which a block of 400 x 40 had in two ways for eight, gave 41.8 us where this gives 42.8).
+// Its shape, by h's 64-column blocks B and the chunks of K; swept over 16 to 1024 blocks, 8 to 64 chunks, one to sixteen rows, times of the three
 // launches (1.0):
-// - up to 128 blocks half of them a workgroup, K split four ways: 0.75 to 0.99; eight ways the same or worse. The gate | up of up
-//   to 64 blocks alone is dealt out by quarters of a block, and where K is long that weighs more: from 32 chunks 1.02 to 1.14 past four rows, 0.99
-//   to 1.02 of 32 blocks below, from 24 chunks and twelve rows 1.0 to 1.04 of 32 blocks;
-// - up to 256 whole blocks, four ways: 0.82 to 0.95 (halves 0.83 to 1.10);
-// - up to 384 halves, two ways: 0.83 to 0.97 up to four rows or below 20 chunks (whole blocks 0.88 to 1.05: some compute units hold two);
-//   up to eight rows below 32 chunks 0.95 to 0.96; else 1.02 to 1.13;
-// - past them whole blocks, two ways: 0.87 to 0.99 (four ways 0.87 to 1.01, eight 0.94 to 1.04).
+// - up to 128 blocks half of them a workgroup, four wavefronts a block: 0.77 to 0.98. The gate | up of up to 64 blocks alone is dealt out
+//   by quarters of a block, and where K is long that weighs more: up to four rows 1.01 to 1.05 of 16 and 32 x 40 and 64 x 64 (48 x 40 0.96, 128 x 64
+//   0.90), above 1.0 to 1.17 of up to 64 x 40, from twelve rows 1.0 to 1.05 of up to 64 x 24 and 1.05 of 128 x 64;
+// - up to 256 whole blocks, four wavefronts: 0.81 to 0.93 (more than four rows past 40 chunks: the sums leave no room for the rings);
+// - up to 384 halves, two wavefronts: 0.86 to 0.98 up to four rows; above 0.96 to 0.99 of 8 chunks and 0.98 to 1.05 from 16;
+// - up to 512 whole blocks, two wavefronts: 0.88 to 0.97; more than four rows below 32 chunks, where a workgroup's sums leave room
+//   for a second one: 0.89 to 0.94, else 1.04 to 1.1;
+// - past them, up to four rows, by what their last round leaves idle: whole blocks 0.93 to 0.98 where it is nearly full (700, 1024), else halves 0.88
+//   to 0.98 (540, 600, 800; whole 0.9 to 1.05) below 32 chunks and 0.96 to 1.02 above; more rows whole blocks below 24 chunks 0.92 to
+//   1.0, else 0.97 to 1.2.
 struct GateUpShape {
-  int parts, ks;  // parts 0: three launches
+  int parts, ways;  // parts 0: three launches
 };
 static GateUpShape gate_up_shape(int m, int blocks, int chunks) {
   const bool few = m <= FEW_ROWS;
   GateUpShape s{1, 2};
   if (blocks <= 128) {
     s = GateUpShape{2, 4};
-    if ((chunks >= 32 && blocks <= (few ? 32 : 64)) || (chunks >= 24 && m >= 12 && blocks <= 32)) s.parts = 0;
+    if (few ? chunks >= 32 && blocks <= chunks : blocks <= 64 ? chunks >= (m >= 12 ? 24 : 32) : m >= 12 && chunks >= 48) s.parts = 0;
   } else if (blocks <= 256) {
     s = GateUpShape{1, 4};
   } else if (blocks <= 384) {
-    s = GateUpShape{few || chunks < 20 || (m <= 8 && chunks < 32) ? 2 : 0, 2};
+    s = GateUpShape{few || chunks < 16 ? 2 : 0, 2};
+  } else if (!few) {
+    if (chunks >= (blocks <= 512 ? 32 : 24)) s.parts = 0;
+  } else if (blocks > 512) {
+    const int last = blocks % COMPUTE_UNITS;  // workgroups of whole blocks in the last round
+    if (last && last < COMPUTE_UNITS * 5 / 8) s.parts = chunks < 32 ? 2 : 0;
   }
-  while (s.ks > 1 && (few ? 2 : 1) * s.ks > chunks) s.ks /= 2;  // a wavefront's start costs about two chunks of the four-row body
+  while (s.ways > 1 && (few ? 2 : 1) * s.ways > chunks) s.ways /= 2;  // a wavefront's start costs about two chunks of the four-row body
   return s;
 }
 
@@ -1483,27 +1547,36 @@ extern "C" int hb_w3_mlp(const void* x, int m, const void* gate_up, const float*
   uint8_t* hq = static_cast<uint8_t*>(scratch);
   float* h_scale = reinterpret_cast<float*>(hq + (size_t)m * inter);
   const int blocks = inter / W3_BLOCK_ROWS;
-  const GateUpShape shape = gate_up_shape(m, blocks, hidden / W3_CHUNK);
-  if (m <= ROWS_PER_SLOT && gate_up_bits == 3 && pairs % W3_BLOCK_ROWS == 0 && shape.parts && blocks <= 0xffffff) {
-    StreamParams p{};
-    p.w = static_cast<const uint8_t*>(gate_up);
-    p.rows = gate_up_rows;
-    p.lut_lo = (uint32_t)((uint64_t)gate_up_lut & 0xffffffffu);
-    p.lut_hi = (uint32_t)((uint64_t)gate_up_lut >> 32);
-    p.n_blocks = 2 * blocks;
-    p.chunks = hidden / W3_CHUNK;
-    p.a = static_cast<const uint16_t*>(x);
-    p.a_stride = hidden;
-    p.m = m;
-    p.oq = hq;
-    p.oq_scale = h_scale;
-    p.out_stride = inter;
-    p.nbw = 2;
-    p.ks = shape.ks;
-    set_split(p);
-    const dim3 grid((unsigned)(shape.parts == 1 ? blocks : (blocks + 7) / 8 * 8 * 2)), block(64 * 2 * p.ks);
-    auto launch = [&](auto kernel) { HB_LAUNCH(kernel, grid, block, (size_t)2 * p.ks * RING_BYTES, as_stream(stream), p, blocks, pairs / W3_BLOCK_ROWS); };
-    if (m <= FEW_ROWS) {
+  StreamParams p{};
+  p.w = static_cast<const uint8_t*>(gate_up);
+  p.rows = gate_up_rows;
+  p.lut_lo = (uint32_t)((uint64_t)gate_up_lut & 0xffffffffu);
+  p.lut_hi = (uint32_t)((uint64_t)gate_up_lut >> 32);
+  p.n_blocks = 2 * blocks;
+  p.chunks = hidden / W3_CHUNK;
+  p.a = static_cast<const uint16_t*>(x);
+  p.a_stride = hidden;
+  p.m = m;
+  p.oq = hq;
+  p.oq_scale = h_scale;
+  p.out_stride = inter;
+  const bool forced = g_tune.w3_tile || g_tune.w3_few || g_tune.w3_ksplit || g_tune.w3_nbw;  // (a shape of the dense launch's own)
+  const bool few = m <= FEW_ROWS, fits = m <= ROWS_PER_SLOT && gate_up_bits == 3 && pairs % W3_BLOCK_ROWS == 0 && blocks <= 0xffffff && !forced;
+  const GateUpShape shape = fits ? gate_up_shape(m, blocks, p.chunks) : GateUpShape{0, 1};
+  GateUp g{blocks, pairs / W3_BLOCK_ROWS, 1, 1};
+  size_t lds = 0;
+  if (shape.parts) {
+    if (int e = shape_stream(p, 1, Launch{0, 0})) return e;
+    shape_one_slot(p, 3);  // the dense launch's splits of K
+    g.ways = std::min(shape.ways, p.ks);
+    g.run = p.ks / g.ways;
+    const int split = few ? split_bytes<true, 4>() : split_bytes<false, 4>();
+    lds = (size_t)2 * g.ways * RING_BYTES + (size_t)2 * p.ks * split / shape.parts;
+  }
+  if (shape.parts && lds <= PANEL_LDS) {
+    const dim3 grid((unsigned)(shape.parts == 1 ? blocks : (blocks + 7) / 8 * 8 * 2)), block(64 * 2 * g.ways);
+    auto launch = [&](auto kernel) { HB_LAUNCH(kernel, grid, block, lds, as_stream(stream), p, g); };
+    if (few) {
       shape.parts == 1 ? launch(w3_fc_gate_up_kernel<true, 1>) : launch(w3_fc_gate_up_kernel<true, 2>);
     } else {
       shape.parts == 1 ? launch(w3_fc_gate_up_kernel<false, 1>) : launch(w3_fc_gate_up_kernel<false, 2>);

@@ -765,17 +765,22 @@ static int launch_nvfp4(StreamParams& p, int64_t slots, int64_t busy_slots, hipS
   return HB_OK;
 }
 
+// The shape of the dense `b` beside the shaped `a` in one launch: one workgroup size (and LDS a workgroup) for both, which the plan's matrix sets. A small
+// latent block's shared expert has these splits of K in every form, so that its bits do not depend on the form.
+static int shape_beside(StreamParams& b, int64_t slots_b, const StreamParams& a) {
+  if (int e = shape_nvfp4(b, slots_b)) return e;
+  const int waves = a.ks * a.nbw;
+  b.ks = std::min(b.ks, waves);
+  b.nbw = waves / b.ks;
+  set_split(b);
+  return HB_OK;
+}
+
 // `a` over its plan's slots beside the dense `b` in one launch (nvfp4_twin_kernel).
 template <int EPI_A, int EPI_B>
 static int launch_twin(StreamParams& a, int64_t slots_a, int64_t busy_a, StreamParams& b, int64_t slots_b, hipStream_t stream) {
   if (int e = shape_nvfp4(a, busy_a)) return e;
-  if (int e = shape_nvfp4(b, slots_b)) return e;
-  if (b.ks * b.nbw != a.ks * a.nbw) {  // one workgroup size (and LDS a workgroup) for both: the plan's matrix sets it
-    const int waves = a.ks * a.nbw;
-    b.ks = std::min(b.ks, waves);
-    b.nbw = waves / b.ks;
-    set_split(b);
-  }
+  if (int e = shape_beside(b, slots_b, a)) return e;
   const int groups_a = (a.n_blocks + a.nbw - 1) / a.nbw, groups_b = (b.n_blocks + b.nbw - 1) / b.nbw;
   const int64_t first = slots_b * groups_b, all = first + slots_a * groups_a;
   if (all > 0x7fffffff) return HB_EINVAL;
@@ -813,16 +818,14 @@ static int launch_fc12(StreamParams& p1, StreamParams& p2, int64_t slots, int64_
   if (int e = shape_nvfp4(p1, busy)) return e;
   if (int e = shape_nvfp4(p2, busy)) return e;
   const int waves = std::max(p1.ks * p1.nbw, p2.ks * p2.nbw);  // one workgroup size for both: all powers of two
-  p1.nbw = waves / p1.ks;
-  p2.nbw = waves / p2.ks;
   int first = 0;
   if (dense) {
-    if (int e = shape_nvfp4(*dense, 1)) return e;
-    dense->ks = std::min(dense->ks, waves);
+    if (int e = shape_beside(*dense, 1, p2)) return e;
     dense->nbw = waves / dense->ks;
-    set_split(*dense);
     first = (dense->n_blocks + dense->nbw - 1) / dense->nbw;
   }
+  p1.nbw = waves / p1.ks;
+  p2.nbw = waves / p2.ks;
   const int groups1 = (p1.n_blocks + p1.nbw - 1) / p1.nbw, groups2 = (p2.n_blocks + p2.nbw - 1) / p2.nbw;
   const int64_t total = slots * (groups1 + groups2) + first;
   if (total > 0x7fffffff) return HB_EINVAL;
@@ -847,17 +850,10 @@ static int launch_front(const LatentRouter& r, hipStream_t stream) {
   return HB_OK;
 }
 
-// Routing and plan beside `up` (latent_plan_kernel), or, where that form does not serve, apart.
-static int launch_latent_plan(const LatentRouter& r, StreamParams& up, hipStream_t stream) {
-  LatentPlan q;
-  if (!latent_plan_of(r, q)) {
-    if (int e = latent_launch_route(r, stream)) return e;
-    return launch_nvfp4<EPI_DENSE_RELU2>(up, 1, 1, stream);
-  }
-  if (int e = shape_nvfp4(up, 1)) return e;
+// Routing and plan beside `up` (latent_plan_kernel), whose splits of K are those of the launch beside `fc1`.
+static int launch_latent_plan(const LatentRouter& r, const LatentPlan& q, StreamParams& up, const StreamParams& fc1, hipStream_t stream) {
+  if (int e = shape_beside(up, 1, fc1)) return e;
   up.nbw = 1;
-  while (up.ks < 8 && 2 * up.ks <= up.chunks) up.ks *= 2;
-  set_split(up);
   const size_t lds = std::max(q.lds, (size_t)up.ks * FP4_RING_BYTES);
   auto launch = [&](auto kernel) {
     HB_LAUNCH(kernel, dim3((unsigned)(q.groups + up.n_blocks)), dim3(PLAN_THREADS), lds, stream, q.route, r.m, q.by_rows, r.e_lo, r.e_n, r.ws->plan, r.ws->order, q.slot_cap,
@@ -1383,15 +1379,23 @@ extern "C" int hb_latent_layer(const hb_latent_weights* w, const void* x, int m,
     up = dense_params(w->shared_up, w->shared_up_scale, w->shared_inter, w->hidden, x, m, l.shared_h);
     down = dense_params(w->shared_down, w->shared_down_scale, w->hidden, w->shared_inter, l.shared_h, m, l.shared_y);
   }
-  if (int e = launch_front(r, s)) return e;
-  if (int e = w->shared_up ? launch_latent_plan(r, up, s) : latent_launch_route(r, s)) return e;
   const int64_t pairs = (int64_t)m * topk, slot_cap = moe_max_slots(pairs, ex->experts, 0, ROWS_PER_SLOT), est = busy_slots(pairs, ex->experts, slot_cap);
   expert_params(ex, c.lat, m, topk, l.moe, l.moe.y, 0, fc1, fc2);
+  if (int e = shape_nvfp4(fc1, est)) return e;
+  if (int e = launch_front(r, s)) return e;
+  LatentPlan q;
+  const bool planned = w->shared_up && latent_plan_of(r, q);  // up beside routing and plan, else beside fc1
+  if (int e = planned ? launch_latent_plan(r, q, up, fc1, s) : latent_launch_route(r, s)) return e;
   StreamParams* dense = w->shared_up ? &down : nullptr;
-  const bool together = fc12_serves(pairs, ex->experts, experts_named(w->experts_total, ex->base, ex->experts), fc1.n_blocks, fc1.chunks) &&
+  const bool together = planned == (dense != nullptr) && fc12_serves(pairs, ex->experts, experts_named(w->experts_total, ex->base, ex->experts), fc1.n_blocks, fc1.chunks) &&
                         (ex->gated ? launch_fc12<EPI_FC1_GATED>(fc1, fc2, slot_cap, est, dense, s) : launch_fc12<EPI_FC1_RELU2>(fc1, fc2, slot_cap, est, dense, s)) == HB_OK;
   if (!together) {
-    if (int e = ex->gated ? launch_nvfp4<EPI_FC1_GATED>(fc1, slot_cap, est, s) : launch_nvfp4<EPI_FC1_RELU2>(fc1, slot_cap, est, s)) return e;
+    if (dense && !planned) {
+      if (int e = ex->gated ? launch_twin<EPI_FC1_GATED, EPI_DENSE_RELU2>(fc1, slot_cap, est, up, 1, s) : launch_twin<EPI_FC1_RELU2, EPI_DENSE_RELU2>(fc1, slot_cap, est, up, 1, s))
+        return e;
+    } else {
+      if (int e = ex->gated ? launch_nvfp4<EPI_FC1_GATED>(fc1, slot_cap, est, s) : launch_nvfp4<EPI_FC1_RELU2>(fc1, slot_cap, est, s)) return e;
+    }
     if (int e = dense ? launch_twin<EPI_FC2, EPI_DENSE>(fc2, slot_cap, est, down, 1, s) : launch_nvfp4<EPI_FC2>(fc2, slot_cap, est, s)) return e;
   }
   return latent_finish(w, c.ids, c.weights, m, topk, l, out, s);

@@ -690,10 +690,23 @@ void moe_launch_quant_groups(const QuantJob& job, hipStream_t stream) {
 }
 
 static std::atomic<int> g_route_plan_fused{0};  // hb_tune("route_plan", 2): routing and plan as two launches; 1: the general plan also where plan_by_rows serves
+static std::atomic<int> g_fault_inject{0};
 int moe_tune(const char* key, int value) {
+  if (!strcmp(key, "fault_inject") && (value == 0 || value == 1)) {
+    g_fault_inject.store(value, std::memory_order_relaxed);
+    return HB_OK;
+  }
   if (strcmp(key, "route_plan") || value < 0 || value > 2) return HB_EINVAL;
   g_route_plan_fused.store(value, std::memory_order_relaxed);
   return HB_OK;
+}
+
+void moe_await_slots(StreamParams& p1, StreamParams& p2, int32_t* plan, int64_t slots, int groups1) {
+  const bool inject = g_fault_inject.load(std::memory_order_relaxed) == 1;  // a test of the give-up path: a count one above what can arrive, a wait of a few polls
+  p1.done = p2.done = plan_done(plan, slots);
+  p1.done_need = p2.done_need = groups1 + (inject ? 1 : 0);
+  p2.wait_spins = inject ? 8 : WAIT_SPINS;
+  p2.fault = plan + PLAN_FAULT;
 }
 
 // From this many pairs: the layer of 65 and 80 rows of ten took 66.5 and 71.8 us with one workgroup, 67.1 and 72.5 in shares, of 128

@@ -829,10 +829,7 @@ static int launch_fc12(StreamParams& p1, StreamParams& p2, int64_t slots, int64_
   const int groups1 = (p1.n_blocks + p1.nbw - 1) / p1.nbw, groups2 = (p2.n_blocks + p2.nbw - 1) / p2.nbw;
   const int64_t total = slots * (groups1 + groups2) + first;
   if (total > 0x7fffffff) return HB_EINVAL;
-  p1.done = p2.done = plan_done(const_cast<int32_t*>(p1.plan), slots);
-  p2.done_need = groups1;
-  p2.wait_spins = WAIT_SPINS;
-  p2.fault = const_cast<int32_t*>(p1.plan) + PLAN_FAULT;
+  moe_await_slots(p1, p2, const_cast<int32_t*>(p1.plan), slots, groups1);
   // about half the device's workgroups ahead (1024 (4 wavefronts) started at once, twice that: 512 (1024, 2688) at 176 pairs 32 slots 91.7 us, 48 89.2, 96 88.4)
   const int lag = (int)std::min<int64_t>(slots, g_nvfp4_lag ? 8 * g_nvfp4_lag.load() : std::max(8, 2048 / groups1));
   HB_LAUNCH(nvfp4_fc12_kernel<EPI1>, dim3((unsigned)total), dim3(64 * waves), (size_t)waves * FP4_RING_BYTES, stream, p1, p2, dense ? *dense : StreamParams{}, groups1,

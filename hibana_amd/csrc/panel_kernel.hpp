@@ -809,10 +809,7 @@ static int launch_panel_fc12(StreamParams& p1, StreamParams& p2, int32_t* plan, 
   if (int e = panel_routed(p2, tiles, slots, rows2)) return e;
   const int rounds = (int)((slots + 7) / 8), both = p1.panel_groups + p2.panel_groups;
   if ((int64_t)rounds * 8 * both > 0x7fffffff) return HB_EINVAL;
-  p1.done = p2.done = plan_done(plan, slots);
-  p2.done_need = p1.panel_groups;
-  p2.wait_spins = WAIT_SPINS;
-  p2.fault = plan + PLAN_FAULT;
+  moe_await_slots(p1, p2, plan, slots, p1.panel_groups);
   const int resident = 256 * (tiles <= 3 ? 4 : tiles <= 5 ? 3 : 2);
   const int lag = std::min(rounds, lag_forced ? lag_forced : std::max(1, 2 * resident / (8 * p1.panel_groups)));
   auto launch = [&](auto kernel) {

@@ -99,6 +99,9 @@ __device__ __forceinline__ bool await_count(const int32_t* at, int need, int spi
   return there;
 }
 
+// What a launch that holds fc1 (`p1`, `groups1` workgroups a slot) and fc2 (`p2`) of a plan of `slots` entries needs to count and to wait.
+void moe_await_slots(StreamParams& p1, StreamParams& p2, int32_t* plan, int64_t slots, int groups1);
+
 // Whether one launch may hold fc1 (`p1`) and fc2: fc2 reads h through its die's L2, which must hold no older copy of a slot's rows, so no row
 // may share a cache line with a neighbour's that another slot read before (a caller's workspace need only lie on 16 bytes).
 inline bool fc12_apart(const StreamParams& p1) { return aligned(p1.out, 256) && p1.out_stride % 128 == 0; }
@@ -763,7 +766,7 @@ void pick_shape(int n_blocks, int chunks, int64_t slots, int want, int* ks, int*
 
 // hb_tune keys of the NVFP4 kernels ("nvfp4_tile": 1 forces the panel kernel, 2 the stream, 0 the built-in choice).
 int nvfp4_tune(const char* key, int value);
-// hb_tune keys of the kernels shared by the routed calls ("route_plan": 2 keeps routing and plan in separate launches).
+// hb_tune keys of the kernels shared by the routed calls ("route_plan": 2 keeps routing and plan in separate launches; "fault_inject": moe_await_slots).
 int moe_tune(const char* key, int value);
 
 }  // namespace hb

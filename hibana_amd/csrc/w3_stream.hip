@@ -1290,7 +1290,7 @@ constexpr int PANEL_W3_ROWS = 20, PANEL_W3_BLOCKS = 300;
 
 // ---------------------------------------------------------------------------------------------------- host side
 struct Tuning {  // hb_tune's knobs: relaxed atomics, so a knob set from one thread while another launches is a plain race-free read
-  std::atomic<int> w3_tile{0}, w3_few{0}, w3_ksplit{0}, w3_nbw{0}, moe_fc1_ksplit{0}, moe_fc1_nbw{0}, moe_fc2_ksplit{0}, moe_fc2_nbw{0}, moe_one{0}, moe_split{0}, moe_fused{0}, moe_lag{0}, fault_inject{0}, moe_one_parts{0};
+  std::atomic<int> w3_tile{0}, w3_few{0}, w3_ksplit{0}, w3_nbw{0}, moe_fc1_ksplit{0}, moe_fc1_nbw{0}, moe_fc2_ksplit{0}, moe_fc2_nbw{0}, moe_one{0}, moe_split{0}, moe_fused{0}, moe_lag{0}, moe_one_parts{0};
 };
 static Tuning g_tune;
 
@@ -1416,7 +1416,7 @@ extern "C" int hb_tune(const char* key, int value) {
     std::atomic<int>* slot;
   } table[] = {{"w3_tile", &g_tune.w3_tile}, {"w3_few", &g_tune.w3_few}, {"w3_ksplit", &g_tune.w3_ksplit},           {"w3_nbw", &g_tune.w3_nbw},
                {"moe_fc1_ksplit", &g_tune.moe_fc1_ksplit}, {"moe_fc1_nbw", &g_tune.moe_fc1_nbw},
-               {"moe_fc2_ksplit", &g_tune.moe_fc2_ksplit}, {"moe_fc2_nbw", &g_tune.moe_fc2_nbw}, {"moe_one", &g_tune.moe_one}, {"moe_split", &g_tune.moe_split}, {"moe_fused", &g_tune.moe_fused}, {"moe_lag", &g_tune.moe_lag}, {"fault_inject", &g_tune.fault_inject}, {"moe_one_parts", &g_tune.moe_one_parts}};
+               {"moe_fc2_ksplit", &g_tune.moe_fc2_ksplit}, {"moe_fc2_nbw", &g_tune.moe_fc2_nbw}, {"moe_one", &g_tune.moe_one}, {"moe_split", &g_tune.moe_split}, {"moe_fused", &g_tune.moe_fused}, {"moe_lag", &g_tune.moe_lag}, {"moe_one_parts", &g_tune.moe_one_parts}};
   for (auto& t : table)
     if (!strcmp(t.name, key)) {
       if (value < 0 || value > 16) return HB_EINVAL;
@@ -1755,15 +1755,8 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
       const int groups1 = (q1.n_blocks + q1.nbw - 1) / q1.nbw, groups2 = (q2.n_blocks + q2.nbw - 1) / q2.nbw;
       const int64_t total = slots * (groups1 + groups2);
       if (total <= 0x7fffffff) {
-        q1.done = q2.done = plan_done(ws.plan, slots);
+        moe_await_slots(q1, q2, ws.plan, slots, groups1);
         q1.trace = moe_trace_buffer(&q1.trace_records);
-        q1.done_need = q2.done_need = groups1;
-        q2.wait_spins = WAIT_SPINS;
-        q2.fault = ws.plan + PLAN_FAULT;
-        if (g_tune.fault_inject == 1) {  // a test of the give-up path: a count one above what can arrive, and a wait of a few polls
-          q2.done_need = groups1 + 1;
-          q2.wait_spins = 8;
-        }
         const int waves = q1.ks * q1.nbw;
         // about the slots whose workgroups fill the device once (four workgroups of four wavefronts a compute unit)
         const int lag_tuned = g_tune.moe_lag.load();

@@ -187,6 +187,67 @@ def test_a_wait_that_gives_up_is_reported_and_reset_restores_service(small):
     _lib.workspace_reset(None)
 
 
+def _routed_call(form, m):
+    """(call(x), two inputs that route alike, hb_tune keys) of a call whose fc1 and fc2 are one launch: every row names expert 0, so that it
+    has slots of every body: rows m, past 16 (a panel's height) another slot, the other experts' few."""
+    from tests.test_gpu_nvfp4_moe import _experts
+    from tests.test_gpu_panel_fc12 import _routing
+    g = torch.Generator().manual_seed(m)
+    if form.startswith("latent"):
+        from hibana_amd import synthetic
+        from hibana_amd.model.nemotron_moe import NemotronMoe
+        gate = torch.randn(16, 512, generator=g) / 512 ** 0.5
+        gate[:, 256:] = 0  # the router does not see what the two inputs differ in
+        fc1 = torch.randn(128, 512, generator=g) / 512 ** 0.5
+        shared = [synthetic.nvfp4_linear(128, 512, 1), synthetic.nvfp4_linear(512, 128, 2)] if form == "latent with a shared expert" else [None, None]
+        block = NemotronMoe(torch.cat([gate, fc1]).bfloat16().cuda(), torch.rand(16, generator=g).cuda(), (torch.randn(512, 128, generator=g) / 128 ** 0.5).bfloat16().cuda(),
+                            synthetic.nvfp4_experts(16, 128, 640, 3), 4, shared_up=shared[0], shared_down=shared[1])
+        x = torch.randn(m, 512, generator=g)
+        other = torch.cat([x[:, :256], torch.randn(m, 256, generator=g)], 1)
+        return lambda v: block(v, None).clone(), x.bfloat16().cuda(), other.bfloat16().cuda(), {"nvfp4_fused": 1}
+    ids, w = _routing(m, 8, m)
+    x, other = (torch.randn(m, 512, generator=g).bfloat16().cuda() for _ in range(2))
+    if form.startswith("w3"):
+        from hibana_amd.kernels import w3_moe
+        ex, _ = random_experts(8, 512, 384, True, 3)
+        sh, _ = random_experts(1, 512, 384, True, 4)
+        return lambda v: w3_moe.moe_layer(ex, v, ids, w, shared=sh).clone(), x, other, {"w3_tile": 1 if form == "w3 panel" else 2}
+    ex, _ = _experts(8, 512, 384, True, 5)
+    return lambda v: ex(v, ids, w).clone(), x, other, {"nvfp4_tile": 1} if form == "nvfp4 panel" else {"nvfp4_tile": 2, "nvfp4_fused": 1}
+
+
+@pytest.mark.parametrize("form,m", [(f, m) for f in ("w3 stream", "w3 panel", "nvfp4 stream", "nvfp4 panel") for m in (2, 4, 7, 12, 40, 150)] +
+                         [(f, m) for f in ("latent", "latent with a shared expert") for m in (1, 4, 7, 16)])
+def test_every_launch_of_both_layers_gives_up_without_storing(form, m, monkeypatch):
+    """Forced from the host as above, in every launch that holds fc1 and fc2 and every body that stands behind the wait: the fault word is set and the pair
+    outputs are those of the call before, so the sums are too; the next call is right."""
+    from hibana_amd import _lib
+    lib = _lib.lib()
+    call, x, other, keys = _routed_call(form, m)
+    asked, workspace = [], _lib.workspace
+    monkeypatch.setattr(_lib, "workspace", lambda *a: asked.append(workspace(*a)) or asked[-1])
+    for k, v in keys.items():
+        assert lib.hb_tune(k.encode(), v) == 0
+    try:
+        want = call(other)
+        before = call(x)
+        assert not torch.equal(want, before) and _lib.workspace_status(asked[-1]) == 0
+        assert lib.hb_tune(b"fault_inject", 1) == 0
+        try:
+            got = call(other)
+        finally:
+            lib.hb_tune(b"fault_inject", 0)
+        assert _lib.workspace_status(asked[-1]) == 1  # HB_FAULT_WAIT
+        if form != "latent with a shared expert":  # (whose own part is of this call)
+            assert torch.equal(got, before)
+        assert torch.equal(call(other), want)
+        _lib.workspace_reset(asked[-1])
+        assert _lib.workspace_status(asked[-1]) == 0 and torch.equal(call(other), want)
+    finally:
+        for k in keys:
+            lib.hb_tune(k.encode(), 0)
+
+
 def test_two_streams_with_workspaces_of_their_own_share_nothing(request):
     """Two verify-sized layer calls from logits (routing and plan in one launch: the arrival counter; fc1 and fc2 in one
     launch: the slots' counters) on two ordinary streams at once, and two NVFP4 products of 64 rows (tiles that share K:

@@ -1473,11 +1473,16 @@ extern "C" int hb_w3_quant_rows(const void* x, int64_t m, int k, void* q, float*
   return launch_status();
 }
 
-extern "C" int hb_w3_gemm_e4m3(const void* xq, const float* x_scale, int m, const void* tiled, const float* row_scale, int64_t lut, int n, int k,
-                               int bits, void* y, void* stream) {
+static int check_e4m3(const void* xq, const float* x_scale, int m, const void* tiled, const float* row_scale, int n, int k, int bits, const void* y) {
   if (!xq || !x_scale || !tiled || !row_scale || !y) return HB_ENULL;
   if (m <= 0 || n <= 0 || k <= 0 || n % W3_BLOCK_ROWS || k % W3_CHUNK || (int64_t)m * (k / 32) > 0xffffffffll || (bits != 2 && bits != 3)) return HB_EINVAL;
   if (!aligned(xq, 8) || !aligned(x_scale, 8) || !aligned(tiled, 16) || !aligned(row_scale, 4) || !aligned(y, 2)) return HB_EINVAL;
+  return ((int64_t)m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT > 65535 ? HB_EINVAL : HB_OK;
+}
+
+extern "C" int hb_w3_gemm_e4m3(const void* xq, const float* x_scale, int m, const void* tiled, const float* row_scale, int64_t lut, int n, int k,
+                               int bits, void* y, void* stream) {
+  if (int e = check_e4m3(xq, x_scale, m, tiled, row_scale, n, k, bits, y)) return e;
   StreamParams p{};
   p.w = static_cast<const uint8_t*>(tiled);
   p.rows = row_scale;
@@ -1491,8 +1496,7 @@ extern "C" int hb_w3_gemm_e4m3(const void* xq, const float* x_scale, int m, cons
   p.m = m;
   p.out = y;
   p.out_stride = n;
-  const int64_t slots = (m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT;
-  if (slots > 65535) return HB_EINVAL;
+  const int64_t slots = ((int64_t)m + ROWS_PER_SLOT - 1) / ROWS_PER_SLOT;
   if (int e = launch_stream<EPI_DENSE>(p, slots, slots, Launch{g_tune.w3_ksplit, g_tune.w3_nbw}, as_stream(stream), bits)) return e;
   return launch_status();
 }
@@ -1541,11 +1545,12 @@ extern "C" int hb_w3_mlp(const void* x, int m, const void* gate_up, const float*
                          int pairs, const void* down, const float* down_rows, int64_t down_lut, int n, int down_bits, void* scratch, size_t scratch_bytes, void* y,
                          void* stream) {
   if (!x || !gate_up || !gate_up_rows || !down || !down_rows || !scratch || !y) return HB_ENULL;
-  if (m <= 0 || inter <= 0 || hidden <= 0 || inter % W3_CHUNK || hidden % W3_CHUNK || pairs < 0 || (pairs && (pairs % 32 || inter % pairs))) return HB_EINVAL;
+  if (m <= 0 || inter <= 0 || inter > 0x3fffffff || hidden <= 0 || inter % W3_CHUNK || hidden % W3_CHUNK || pairs < 0 || (pairs && (pairs % 32 || inter % pairs)) || (gate_up_bits != 2 && gate_up_bits != 3)) return HB_EINVAL;
   if (!aligned(x, 16) || !aligned(gate_up, 16) || !aligned(gate_up_rows, 4) || !aligned(scratch, 16)) return HB_EINVAL;
   if (scratch_bytes < HB_W3_MLP_SCRATCH_BYTES((size_t)m, (size_t)inter)) return HB_EWORKSPACE;
   uint8_t* hq = static_cast<uint8_t*>(scratch);
   float* h_scale = reinterpret_cast<float*>(hq + (size_t)m * inter);
+  if (int e = check_e4m3(hq, h_scale, m, down, down_rows, n, inter, down_bits, y)) return e;  // ahead of the first launch
   const int blocks = inter / W3_BLOCK_ROWS;
   StreamParams p{};
   p.w = static_cast<const uint8_t*>(gate_up);

@@ -107,6 +107,15 @@ def test_validation_without_a_gpu():
         _lib.check(_lib.HB_ELAUNCH, "x")
 
 
+@pytest.mark.parametrize("change", [{"n": 96}, {"n": 0}, {"down_bits": 4}, {"down": 264}, {"down_rows": 258}, {"y": 257}, {"gate_up_bits": 1}, {"m": 1 << 21}])
+def test_a_dense_block_that_its_down_projection_refuses(change):
+    """hb_w3_mlp: what its last launch would refuse (that nothing is launched for it: tests/test_gpu_w3_mlp.py)."""
+    call = {"x": 256, "m": 4, "gate_up": 256, "gate_up_rows": 256, "gate_up_lut": 0, "inter": 128, "hidden": 128, "gate_up_bits": 3, "pairs": 0, "down": 256, "down_rows": 256,
+            "down_lut": 0, "n": 128, "down_bits": 3, "scratch": 256, "scratch_bytes": 1 << 40, "y": 256, "stream": None}
+    assert set(change) <= set(call)
+    assert _lib.lib().hb_w3_mlp(*{**call, **change}.values()) == _lib.HB_EINVAL
+
+
 @pytest.mark.parametrize("change", [dict(steps=0), dict(steps=-1), dict(steps=3), dict(per_request=-1), dict(min_cap=-1), dict(keep=21), dict(budget=-1), dict(topk=21),
                                     dict(experts_total=19)])
 def test_a_budget_that_is_refused_is_refused_before_anything_is_made_of_it(change):

@@ -65,3 +65,22 @@ def test_a_two_bit_copy_and_refused_calls():
         w3.w3_mlp(x, gate_up, down, pairs=40)
     with pytest.raises(RuntimeError):
         w3.w3_mlp(x.cpu(), gate_up, down)
+
+
+@pytest.mark.parametrize("m", [4, 17])
+@pytest.mark.parametrize("change", [{"n": 96}, {"down_bits": 4}, {"down": 8}, {"y": 1}])  # (pointers: bytes off their boundary)
+def test_what_the_down_projection_refuses_launches_nothing(change, m):
+    from hibana_amd import _lib
+    gate_up, down = _copies(256, 384)
+    x = torch.randn(m, 256, generator=torch.Generator().manual_seed(m)).bfloat16().cuda()
+    from hibana_amd.kernels import w3
+    w3.tile(gate_up), w3.tile(down)
+    scratch, y = torch.full((m * 384 // 8 * 41,), 0x7f, dtype=torch.uint8, device="cuda"), torch.zeros(m, 256, dtype=torch.bfloat16, device="cuda")
+    call = {"x": x.data_ptr(), "m": m, "gate_up": gate_up.tiled.data_ptr(), "gate_up_rows": gate_up.row_scale.data_ptr(), "gate_up_lut": gate_up.lut, "inter": 384, "hidden": 256,
+            "gate_up_bits": 3, "pairs": 0, "down": down.tiled.data_ptr(), "down_rows": down.row_scale.data_ptr(), "down_lut": down.lut, "n": 256, "down_bits": 3,
+            "scratch": scratch.data_ptr(), "scratch_bytes": scratch.numel(), "y": y.data_ptr(), "stream": _lib.stream()}
+    for k, v in change.items():
+        call[k] = call[k] + v if k in ("down", "y") else v
+    assert _lib.lib().hb_w3_mlp(*call.values()) == _lib.HB_EINVAL
+    torch.cuda.synchronize()
+    assert bool((scratch == 0x7f).all())

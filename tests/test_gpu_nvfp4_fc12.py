@@ -1,11 +1,13 @@
 """fc1 and fc2 of NVFP4 experts in one launch against the two launches, and the small latent block in one call against
-`router` and `block`: the same sums in the same order, so the same bits."""
+`router` and `block`: the same sums in the same order, so the same bits (of the block, behind a shared expert
+too: tests/test_gpu_latent_layer_bits.py)."""
 import contextlib
 
 import pytest
 import torch
 
 from tests.test_gpu_nvfp4_moe import _experts
+from tests.util import MAX_REL, NORM_REL, errors
 
 pytestmark = pytest.mark.gpu
 
@@ -38,7 +40,7 @@ def test_one_launch_has_the_bits_of_two(hidden, inter, gated, m):
     assert torch.isfinite(out[0]).all() and torch.equal(*out)
 
 
-@pytest.mark.parametrize("hidden,latent,inter,experts,topk,shared", [(512, 128, 640, 16, 4, 0), (1024, 512, 384, 200, 8, 640), (2048, 1024, 2688, 64, 22, 128), (4096, 1024, 2688, 64, 22, 5376)])
+@pytest.mark.parametrize("hidden,latent,inter,experts,topk,shared", [(512, 128, 640, 16, 4, 0), (1024, 512, 384, 200, 8, 640), (2048, 1024, 2688, 64, 22, 128)])
 @pytest.mark.parametrize("m", [1, 4, 5, 8, 9, 16])
 @pytest.mark.parametrize("form", [0, 1, 2])
 @pytest.mark.parametrize("padded", [False, True])
@@ -58,7 +60,11 @@ def test_layer_is_router_and_block(hidden, latent, inter, experts, topk, shared,
     want = small.block(x, ws, ids, w, weights).clone()
     with _forced(b"nvfp4_fused", form):
         got = small.layer(x, weights, topk, slots, 1)
-    assert torch.equal(got, want)
+    if shared:
+        mx, nr = errors(got, want)
+        assert mx < MAX_REL and nr < NORM_REL
+    else:
+        assert torch.equal(got, want)
 
 
 def test_layer_replays_in_a_graph():

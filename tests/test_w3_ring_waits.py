@@ -74,7 +74,7 @@ def test_a_wait_leaves_the_next_block_outstanding_and_no_more(tmp_path):
         takes = list(_most_left_in_flight(code))
         assert takes and all(most <= reads for most, reads in takes), (name, takes)
         checked += 1
-    assert checked >= 35, checked
+    assert checked >= 20, checked
 
 
 @pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
@@ -82,19 +82,36 @@ def test_light_slots_of_the_panel_kernel_wait_for_their_blocks(tmp_path):
     """The same ring, of the slots that run on the weight stream's bodies inside the three-bit panel kernels (a block is four reads;
     the panel's own waits stand ahead of single ones)."""
     checked = 0
-    for name, code in _kernels(tmp_path, r"panel_(fc12_)?tile_kernel.*TileW3"):
+    for name, code in _kernels(tmp_path, r"panel_tile_kernel.*TileW3"):
         takes = [(most, reads) for most, reads in _most_left_in_flight(code) if reads >= 4]
         assert len(takes) >= 10 and all(most <= 4 for most, _ in takes), (name, takes)
         checked += 1
-    assert checked >= 20, checked
+    assert checked >= 12, checked
 
 
 @pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
 def test_nvfp4_waits_leave_the_next_block_outstanding_and_no_more(tmp_path):
     """The NVFP4 rings: a block's scales come in two loads and are read in one."""
     checked = 0
-    for name, code in _kernels(tmp_path, r"nvfp4_(stream|part|twin|fc12)_kernel|latent_plan_kernel"):
+    for name, code in _kernels(tmp_path, r"nvfp4_(stream|part|twin)_kernel"):
         takes = list(_most_left_in_flight(code, loads_made=True))
         assert takes and all(most <= reads + 1 for most, reads in takes), (name, takes)
         checked += 1
-    assert checked >= 16, checked
+    assert checked >= 12, checked
+
+
+@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
+def test_kernels_of_two_layers_wait_for_their_blocks(tmp_path):
+    """The launches of fc1 and fc2, which ask for a second block ahead of the wait between them, and the small latent block's plan."""
+    for pattern, three_bit, least in ((r"w3_fc\w+_kernel", True, 5), (r"panel_fc12_tile_kernel.*TileW3", True, 8), (r"nvfp4_fc12_kernel|latent_plan_kernel", False, 4)):
+        checked = 0
+        folder = tmp_path / str(least)
+        folder.mkdir()
+        for name, code in _kernels(folder, pattern):
+            takes = list(_most_left_in_flight(code, loads_made=not three_bit))
+            if "panel" in name:
+                takes = [(most, reads) for most, reads in takes if reads >= 4]
+                assert len(takes) >= 10, name
+            assert takes and all(most <= (reads if three_bit else reads + 1) for most, reads in takes), (name, takes)
+            checked += 1
+        assert checked >= least, (pattern, checked)

@@ -1169,7 +1169,7 @@ extern "C" int hb_debug_events(void* const* events, int count) {
 // Minor: what was added since 1.0 (the small latent block, hb_nvfp4_gemm_ws, budgeted routing, the layer under a budget, the
 // ring skeleton hook, hb_workspace_reset / hb_workspace_status with the counters in the caller's workspace; 1.6: the layer from
 // its rows, hb_nvfp4_gemm_room_bytes, the calls on a range of the experts, and other bytes in an NVFP4 tile layout).
-extern "C" int hb_version(void) { return 1006; }
+extern "C" int hb_version(void) { return 1009; }
 
 extern "C" const char* hb_error_string(int code) {
   switch (code) {

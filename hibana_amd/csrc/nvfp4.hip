@@ -660,6 +660,7 @@ __global__ __launch_bounds__(64 * FRONT_WAVES) void latent_front_kernel(FrontGem
 // The second launch: routing and plan of those rows - up to ROUTE_FUSED_ROWS of them by one workgroup, else a workgroup a row of which the
 // last to arrive plans, as moe_plan_kernel and moe_route_plan_kernel do it - and beside them, in the workgroups past `groups`, the shared
 // expert's up projection, which needs nothing of the routing: the plan leaves the memory and all but a few compute units idle.
+// (18 and 9 registers a lane go to memory: the ranking's, as in moe_plan_kernel; the projection stays within the 128 of a workgroup of 1024.)
 template <bool MANY>
 __global__ __launch_bounds__(PLAN_THREADS) void latent_plan_kernel(RouteParams route, int rows, int by_rows, int e_lo, int e_n, int32_t* __restrict__ plan,
                                                                    int32_t* __restrict__ order, int slot_cap, int groups, StreamParams up) {
@@ -697,7 +698,7 @@ __global__ __launch_bounds__(PLAN_THREADS) void latent_plan_kernel(RouteParams r
 }
 
 // experiments (hb_tune): the stream's workgroup shape ("nvfp4_ksplit", "nvfp4_nbw"); "nvfp4_tile": 1 forces the panel kernel, 2 the stream
-static std::atomic<int> g_nvfp4_ksplit{0}, g_nvfp4_nbw{0}, g_nvfp4_tile{0}, g_nvfp4_few{0}, g_nvfp4_tile_ks{0}, g_nvfp4_lag{0}, g_nvfp4_fused{0};  // "nvfp4_fused": 1 runs fc1 and fc2 of a routed call on the stream in one launch, 2 (of any) in two; "nvfp4_lag": eighths of the slots fc2 is behind in one; "nvfp4_few": 2 switches off the body for slots of at most eight rows; "nvfp4_tile_ks": the workgroups that share a tile's K
+static std::atomic<int> g_nvfp4_ksplit{0}, g_nvfp4_nbw{0}, g_nvfp4_tile{0}, g_nvfp4_few{0}, g_nvfp4_tile_ks{0}, g_nvfp4_lag{0}, g_nvfp4_fused{0};  // "nvfp4_fused": 1 runs fc1 and fc2 of a routed call on the stream in one launch, 2 (of any) in two; "nvfp4_lag": how far fc2 is behind in one, in units of eight slots; "nvfp4_few": 2 switches off the body for slots of at most eight rows; "nvfp4_tile_ks": the workgroups that share a tile's K
 
 static int shape_nvfp4(StreamParams& p, int64_t busy_slots) {
   pick_shape(p.n_blocks, p.chunks, busy_slots, 4096, &p.ks, &p.nbw);

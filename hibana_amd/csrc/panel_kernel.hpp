@@ -504,7 +504,7 @@ struct Panel {
 // Dense calls: every slot has up to 16 MT rows. The tiles past p.panel_full have their K shared by p.panel_kz workgroups each.
 template <class Fmt, int EPI, int MT>
 __global__ __launch_bounds__(64 * PANEL_WAVES, 2) void panel_kernel(StreamParams p) {
-  extern __shared__ __align__(16) uint8_t panel_lds[];
+  extern __shared__ __align__(128) uint8_t panel_lds[];  // (the addresses of the halves of a row differ in one bit)
   int tile = blockIdx.x;
   PanelShare part{0, 0, 1, 0};
   if (tile >= p.panel_full) {
@@ -555,7 +555,7 @@ __device__ __forceinline__ void panel_slot(const StreamParams& p, const Slot& sl
 // with 80, two with 128 and 144 (the choice: panel_height).
 template <class Fmt, int EPI, int MOST>
 __global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void panel_tile_kernel(StreamParams p) {
-  extern __shared__ __align__(16) uint8_t panel_lds[];
+  extern __shared__ __align__(128) uint8_t panel_lds[];  // (the addresses of the halves of a row differ in one bit)
   const int die = blockIdx.x & 7, local = blockIdx.x >> 3, round = local / p.panel_groups, slot = 8 * round + die;
   if (slot >= p.panel_full) return;
   const Slot sl = slot_of<EPI>(p, slot);
@@ -574,8 +574,8 @@ __global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void pane
 // and 127, 16 (512, 1024) 40 rows of eight 48 and 46. No size of seventy gained by two.
 template <class Fmt, int EPI1, int MOST>
 __global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void panel_fc12_tile_kernel(StreamParams p1, StreamParams p2, int rounds, int lag) {
-  extern __shared__ __align__(16) uint8_t panel_lds[];
-  __shared__ __align__(128) int outcome[32];  // (a whole 128 bytes: the panel's addresses of the halves of a row differ in one bit of its dynamic LDS)
+  extern __shared__ __align__(128) uint8_t panel_lds[];  // (the addresses of the halves of a row differ in one bit)
+  __shared__ int outcome;
   const Fc12Place at = fc12_place(blockIdx.x >> 3, p1.panel_groups, p2.panel_groups, rounds, lag);
   const int slot = 8 * at.slot + (blockIdx.x & 7);
   if (slot >= p1.panel_full) return;
@@ -588,7 +588,7 @@ __global__ __launch_bounds__(256, (MOST <= 3 ? 4 : MOST <= 5 ? 3 : 2)) void pane
   } else {
     const Slot sl = slot_of<EPI_FC2>(p2, slot);
     if (sl.rows <= 0) return;
-    SlotWait wait(p2, slot, outcome, false);
+    SlotWait wait(p2, slot, &outcome, false);
     panel_slot<Fmt, EPI_FC2, MOST, false>(p2, sl, at.index, panel_lds, wait);
   }
 }

@@ -1619,7 +1619,7 @@ struct Routing {  // set: the chain routes the logits itself into the caller's i
 int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void* x, const int32_t* ids, int m, int topk,
                 const MoeWorkspace& ws, void* out_pairs, int pairs_bf16, hipStream_t stream, int experts_total, const Routing* route = nullptr,
                 bool e4m3 = false, const CombineParams* combine = nullptr) {
-  const int64_t pairs = (int64_t)m * topk, named = experts_named(experts_total, ex->base, ex->experts), local = pairs * ex->experts / named;
+  const int64_t pairs = (int64_t)m * topk, named = experts_named(experts_total, ex->base, ex->experts);
   const int shared_rows = shared ? m : 0;
   // A dense contraction once an expert sees some rows: the panel kernel's higher slots (E4M3 activations: the stream only).
   // The stream pays for a pass a sixteen rows, the panel for longer workgroups, which a call of few experts does not fill: `fill` is fc1's, a

@@ -77,10 +77,14 @@ int hb_workspace_status(const void* workspace, int32_t* status, int wait, void* 
  * "moe_fc1_ksplit" / "moe_fc1_nbw", "moe_fc2_ksplit" / "moe_fc2_nbw", "nvfp4_ksplit" / "nvfp4_nbw": K splits and 64-row
  * blocks per workgroup (their product at most 16); "w3_tile" / "nvfp4_tile": 1 forces the panel kernel, 2 the weight
  * stream; "w3_few" / "nvfp4_few": 2 switches off the stream's body for slots of few rows (W3: at most four, NVFP4: at
- * most eight); "moe_one": 2 switches off the single launch that does one token's fc2 and combine; "moe_fused": 2 runs a
- * routed call's fc1 and fc2 as two launches; "moe_lag": the slots fc2 lags fc1 by in their common launch; "moe_split":
- * 1 gives fc1's slots of at most two rows a two-plane E4M3 form of x (FP8 matrix cores; 4e-4 of the norm); "route_plan": 2 keeps
- * routing and plan in separate launches; "nvfp4_tile_ks": the workgroups that share a tile's K in hb_nvfp4_gemm_ws.
+ * most eight); "moe_one": 2 switches off the single launch that does one token's fc2 and combine; "moe_one_parts": the
+ * workgroups a block of one token's fc2 (1, 2 or 4); "moe_fused" / "nvfp4_fused": 2 runs a routed call's fc1 and fc2 as two
+ * launches, "nvfp4_fused" 1 as one on the stream whatever the size; "moe_lag" / "nvfp4_lag": how far fc2 lags fc1 in their
+ * common launch, in units of eight slots (the panel kernel's: one of each compute die); "moe_split": 1 gives fc1's slots
+ * of at most two rows a two-plane E4M3 form of x (FP8 matrix cores; 4e-4 of the norm); "route_plan": 1 plans by the general
+ * form, 2 keeps routing and plan in separate launches; "nvfp4_tile_ks": the workgroups that share a tile's K in
+ * hb_nvfp4_gemm_ws; "fault_inject": 1 has fc2 in a common launch wait for one arrival too many, for eight polls (the test of
+ * the fault word).
  * Returns HB_EINVAL for an unknown key or a value out of range. The knobs are process-wide relaxed atomics: setting one
  * while another thread launches is a race-free read of either value, not a per-call setting. */
 int hb_tune(const char* key, int value);
@@ -535,8 +539,10 @@ int hb_latent_router(const hb_latent_weights* w, const void* x, int m, int topk,
                      int route, int pad_id, float* fused, int32_t* ids, float* weights, void* lat, void* workspace,
                      size_t workspace_bytes, void* stream);
 
-/* hb_latent_router (routing and planning) and hb_latent_block in one call, for a caller that wants the block's output alone: five launches, the
- * shared expert's up projection beside the router's product, its down projection beside the routed experts' two layers.
+/* hb_latent_router (routing and planning) and hb_latent_block in one call, for a caller that wants the block's output alone, with the bits of the
+ * two. Five launches: the router's product; routing and plan, the shared expert's up projection beside them; both layers of the routed experts,
+ * its down projection beside them; the combine; the projection back. Six where the two layers are a launch each (few pairs, many of few
+ * experts, a workspace off 256-byte addresses).
  * `workspace`: hb_latent_layer_workspace_bytes, under the rules of hb_latent_router's; NVFP4 routed experts only.
  * ref: the block of at most 16 rows, NemotronMoe.small, hibana/model/nemotron/moe.py:484-502. */
 size_t hb_latent_layer_workspace_bytes(const hb_latent_weights* w, int m, int topk);

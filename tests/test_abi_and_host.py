@@ -107,6 +107,14 @@ def test_validation_without_a_gpu():
         _lib.check(_lib.HB_ELAUNCH, "x")
 
 
+def test_the_header_names_every_tuning_key():
+    text = "".join(open(os.path.join(ROOT, "hibana_amd", "csrc", f)).read() for f in ("w3_stream.hip", "nvfp4.hip", "moe_common.hip"))
+    keys = set(re.findall(r'\{"(\w+)", &g_tune\.', text)) | set(re.findall(r'strcmp\(key, "(\w+)"\)', text))
+    assert len(keys) >= 20
+    header = open(os.path.join(ROOT, "include", "hibana_hip.h")).read()
+    assert not [k for k in keys if f'"{k}"' not in header]
+
+
 @pytest.mark.parametrize("change", [{"n": 96}, {"n": 0}, {"down_bits": 4}, {"down": 264}, {"down_rows": 258}, {"y": 257}, {"gate_up_bits": 1}, {"m": 1 << 21}])
 def test_a_dense_block_that_its_down_projection_refuses(change):
     """hb_w3_mlp: what its last launch would refuse (that nothing is launched for it: tests/test_gpu_w3_mlp.py)."""

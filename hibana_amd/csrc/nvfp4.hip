@@ -1090,7 +1090,7 @@ int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, i
   const int64_t est = busy_slots(pairs, ex->experts, slots);
   StreamParams p, f2;
   expert_params(ex, x, m, topk, ws, out_pairs, pairs_bf16, p, f2);
-  if (dense && g_nvfp4_fused != 2 && fc12_apart(p)) {
+  if (dense && g_nvfp4_fused != 2 && fc12_apart(p) && (g_nvfp4_fused == 1 || panel_together(p, f2, ex->experts, tiles))) {
     if (int e = ex->gated ? launch_panel_fc12<TileNvfp4, EPI_FC1_GATED>(p, f2, ws.plan, tiles, slots, m, pairs, g_nvfp4_lag, stream)
                           : launch_panel_fc12<TileNvfp4, EPI_FC1_RELU2>(p, f2, ws.plan, tiles, slots, m, pairs, g_nvfp4_lag, stream))
       return e;

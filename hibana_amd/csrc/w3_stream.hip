@@ -1713,7 +1713,7 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   f2.out = out_pairs;
   f2.out_stride = ex->hidden_out;
   f2.out_bf16 = pairs_bf16;
-  if (dense && g_tune.moe_fused != 2 && fc12_apart(p)) {
+  if (dense && g_tune.moe_fused != 2 && fc12_apart(p) && (g_tune.moe_fused == 1 || panel_together(p, f2, ex->experts, tiles))) {
     if (int e = ex->gated ? launch_panel_fc12<TileW3<3>, EPI_FC1_GATED>(p, f2, ws.plan, tiles, slots, m, pairs + shared_rows, g_tune.moe_lag, stream)
                           : launch_panel_fc12<TileW3<3>, EPI_FC1_RELU2>(p, f2, ws.plan, tiles, slots, m, pairs + shared_rows, g_tune.moe_lag, stream))
       return e;

@@ -79,7 +79,7 @@ int hb_workspace_status(const void* workspace, int32_t* status, int wait, void* 
  * stream; "w3_few" / "nvfp4_few": 2 switches off the stream's body for slots of few rows (W3: at most four, NVFP4: at
  * most eight); "moe_one": 2 switches off the single launch that does one token's fc2 and combine; "moe_one_parts": the
  * workgroups a block of one token's fc2 (1, 2 or 4); "moe_fused" / "nvfp4_fused": 2 runs a routed call's fc1 and fc2 as two
- * launches, "nvfp4_fused" 1 as one on the stream whatever the size; "moe_lag" / "nvfp4_lag": how far fc2 lags fc1 in their
+ * launches, 1 as one where both forms serve ("moe_fused": on the panel kernel); "moe_lag" / "nvfp4_lag": how far fc2 lags fc1 in their
  * common launch, in units of eight slots (the panel kernel's: one of each compute die); "moe_split": 1 gives fc1's slots
  * of at most two rows a two-plane E4M3 form of x (FP8 matrix cores; 4e-4 of the norm); "route_plan": 1 plans by the general
  * form, 2 keeps routing and plan in separate launches; "nvfp4_tile_ks": the workgroups that share a tile's K in

@@ -1,0 +1,28 @@
+"""From how many rows an expert a routed call of few, wide experts takes the panel kernel: fc2's workgroups are then few and as long as its K, and the weight
+stream serves more rows. The two kernels add in different orders, so the bits say which one ran."""
+import pytest
+import torch
+
+from tests.test_gpu_expert_ranges import _by_kernel, _forced
+
+pytestmark = pytest.mark.gpu
+
+
+def _draw(m, e, k, hidden):
+    g = torch.Generator().manual_seed(m)
+    ids = torch.stack([torch.randperm(e, generator=g)[:k] for _ in range(m)]).int().cuda()
+    return torch.randn(m, hidden, generator=g).bfloat16().cuda(), ids, torch.rand(m, k, generator=g).cuda()
+
+
+# wider than long, all workgroups at once, and the long end that keeps its own launch: either way the same bits
+@pytest.mark.parametrize("experts,hidden,inter", [(64, 512, 4096), (24, 512, 4096), (32, 512, 6144)])
+@pytest.mark.parametrize("rows", [16, 40])
+def test_one_launch_and_two_have_the_same_bits(experts, hidden, inter, rows):
+    from hibana_amd import synthetic
+    ex = synthetic.nvfp4_experts(experts, hidden, inter, 1)
+    x, ids, w = _draw(rows * experts // 4, experts, 4, hidden)
+    out = [ex(x, ids, w).clone()]
+    for form in (1, 2):
+        with _forced(b"nvfp4_tile", 1), _forced(b"nvfp4_fused", form):
+            out.append(ex(x, ids, w).clone())
+    assert torch.isfinite(out[0]).all() and torch.equal(out[1], out[2])

@@ -1074,13 +1074,25 @@ int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, i
                 int pairs_bf16, hipStream_t stream, int experts_total) {
   const int64_t pairs = (int64_t)m * topk, named = experts_named(experts_total, ex->base, ex->experts);
   // A dense contraction once an expert sees three rows, or four of fewer than 768 columns: the panel kernel; below that the 16-row slots of the weight
-  // stream. Measured, stream and panel, the whole latent block in us: 128 experts (512, 1024) 3 rows an expert 52.5 and 53.3, 4 rows 55.2 and 54.1, 6 rows 60
-  // and 56; 300 (640, 1280) 3 rows 89 and 90, 4 rows 94 and 90; 256 (768, 1536) 3 rows 97 and 96, 5 rows 106 and 102; 400 (896, 2048) 3 rows 180
-  // and 175, 5 rows 202 and 190; 512 (1024, 2688) 3 rows 294 and 286, 5 rows 338 and 318, 7 rows 373 and 339. Few experts (`fill`: fc1's workgroups, a slot
-  // an expert) fill the device later, and a range of them sees its share of the pairs only: 64 of 512 experts
-  // (1024, 2688), the summed experts alone, two launches, on slots of 128 rows 4 rows an expert 59 and 68, 8 rows 86 and 76.
-  const int64_t fill = (int64_t)ex->experts * (((ex->gated ? 2 : 1) * ex->inter / 64 + 3) / 4);
-  const int64_t rows_min = ex->experts < named ? 8 : fill < 500 ? 7 : ex->hidden >= 768 ? 3 : 4;
+  // stream. Measured, stream and panel, the whole latent block in us: 300 (640, 1280) 3 rows an expert 89 and 90, 4 rows 94 and 90; 256 (768, 1536) 3 rows 97 and 96, 5 rows
+  // 106 and 102; 400 (896, 2048) 3 rows 180 and 175, 5 rows 202 and 190; 512 (1024, 2688) 3 rows 294 and 286, 5 rows 338 and 318, 7 rows 373 and 339.
+  // Few experts fill the device later: with fc1 (`fill`: its workgroups, a slot an expert), and with fc2, whose workgroups (`fill2`) are as long as their K. By fill2 a chunk of K,
+  // the routed call, even and (skewed) routing, us:
+  // - 32 to 50: 64 (2048, 2048) 4 rows 63 and 67 (66 and 68), 5 rows 71 and 68 (71 and 69); 128 (1024, 2048) 3 rows 65 and 73 (65 and 64), 5 rows 78 and 74 (76 and 73); 200 (896,
+  //   2048) 4 rows 93 and 93 (83 and 85), 6 rows 99 and 96 (98 and 93);
+  // - 12 to 26: 160 (512, 1536) 5 rows 48 and 51 (47 and 47), 7 rows 52 and 52 (52 and 54); 96 (1024, 4096) 5 rows 97 and 107 (90 and 108), 8 rows 114 and 110 (118 and 115);
+  // - 4 to 9: 48 (768, 2816) 8 rows 50 and 53 (51 and 55), 12 rows 56 and 54 (58 and 56); 32 (1024, 2688) 12 rows 47 and 51 (49 and 55), 20 rows 56 and 53 (56 and 58); 64 (1024, 8192) 10
+  //   rows 150 and 153 (159 and 175), 16 rows 203 and 155 (206 and 192);
+  // - 1: 16 (1024, 8192) 4 rows 42 and 100 (45 and 100), 40 rows 110 and 125 (109 and 131), 64 rows 159 and 136 (155 and 164).
+  // Too few workgroups for a round of both layers leave it to the stream: 8 (2048, 2048) 12 rows 28 and 51, 120 rows 78 and 87, 150 rows
+  // 103 and 88; 16 (512, 1024) 40 rows 27 and 32, 120 rows 39 and 44.
+  // A range of the experts sees its share of the pairs only: 64 of 512 experts (1024, 2688), the summed experts alone, two launches, on slots of 128 rows 4
+  // rows an expert 59 and 68, 8 rows 86 and 76.
+  const int64_t fill = (int64_t)ex->experts * (((ex->gated ? 2 : 1) * ex->inter / 64 + 3) / 4), fill2 = (int64_t)ex->experts * ((ex->hidden_out / 64 + 3) / 4), chunks2 = ex->inter / 128;
+  int64_t rows_min = fill2 >= 60 * chunks2 ? ex->hidden >= 768 ? 3 : 4 : fill2 >= 30 * chunks2 ? 5 : fill2 >= 10 * chunks2 ? 7 : fill2 >= 3 * chunks2 ? 14 : 60;
+  if (fill < 500) rows_min = std::max<int64_t>(rows_min, 7);
+  if (fill + fill2 < 256) rows_min = std::max<int64_t>(rows_min, 128);
+  if (ex->experts < named) rows_min = 8;
   const bool dense = panel_takes(m, ex->hidden) && panel_takes(pairs, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
                      (g_nvfp4_tile == 1 || (g_nvfp4_tile == 0 && pairs >= rows_min * named));
   const int tiles = panel_height<TileNvfp4>(pairs, named, ex->experts, 0, (ex->gated ? 2 : 1) * ex->inter / 64), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;

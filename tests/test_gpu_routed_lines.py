@@ -14,6 +14,17 @@ def _draw(m, e, k, hidden):
     return torch.randn(m, hidden, generator=g).bfloat16().cuda(), ids, torch.rand(m, k, generator=g).cuda()
 
 
+# fc2's workgroups a chunk of its K: 90, 64, 32, 26, 6, 0.5, 12 (fc1 of few workgroups)
+@pytest.mark.parametrize("experts,hidden,inter,rows", [(300, 640, 1280, 4), (256, 768, 1536, 3), (128, 512, 1024, 5), (160, 512, 1536, 7), (48, 768, 2816, 14), (16, 512, 8192, 60), (48, 512, 1024, 7)])
+def test_nvfp4(experts, hidden, inter, rows):
+    from hibana_amd import synthetic
+    ex = synthetic.nvfp4_experts(experts, hidden, inter, 1)
+    for m in (rows * experts // 4 - 1, rows * experts // 4):
+        x, ids, w = _draw(m, experts, 4, hidden)
+        by_panel, by_stream = _by_kernel(b"nvfp4_tile", lambda: ex(x, ids, w))
+        assert torch.equal(ex(x, ids, w), by_panel if 4 * m >= rows * experts else by_stream)
+
+
 # wider than long, all workgroups at once, and the long end that keeps its own launch: either way the same bits
 @pytest.mark.parametrize("experts,hidden,inter", [(64, 512, 4096), (24, 512, 4096), (32, 512, 6144)])
 @pytest.mark.parametrize("rows", [16, 40])

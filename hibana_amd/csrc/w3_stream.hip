@@ -1629,8 +1629,17 @@ int run_experts(const hb_w3_experts* ex, const hb_w3_experts* shared, const void
   // 5 rows 70 and 70 (61 and 62), 7 rows 72 and 71 (67 and 63); 96 (2560, 768), 576, 11 rows 93 and 96 (97 and 92), 18 rows 128 and 111 (125 and 106); 64
   // (2048, 512), 256, 22 rows 74 and 78 (73 and 75), 27 rows 81 and 78 (81 and 78); 128 (1024, 256), 256, 18 rows 55 and 55 (54 and 54), 22 rows 61 and 59 (57 and 59),
   // 27 rows 65 and 60 (64 and 61). A range of the experts sees its share of the pairs only.
-  const int64_t fill = (int64_t)ex->experts * (((ex->gated ? 2 : 1) * ex->inter / W3_BLOCK_ROWS + 3) / 4);
-  const int rows_min = fill >= 1500 ? 5 : fill >= 500 ? ex->experts >= 150 ? 7 : 16 : ex->experts < named ? 48 : 26;
+  // Few wide experts fill it with fc1 and not with fc2, whose workgroups (`fill2`) are then few and as long as their K: 96 (1024, 3072), fill2 a chunk of K 16, 9 rows
+  // 96 and 103 (103 and 111), 16 rows 130 and 129 (136 and 128); 64 (1536, 4096), 12, 7 rows 123 and 121 (126 and 130); 48 (2048, 8192), 6, 5 rows 204 and 212 (201 and 229),
+  // 9 rows 240 and 230 (270 and 253); 128 (2048, 4096), 32, 5 rows 263 and 267 (244 and 243); 32 (2048, 4096), 8, 15 rows 115 and 112 (115 and 121); 16 (2048, 8192),
+  // 2, 20 rows 150 and 155 (147 and 174), 40 rows 222 and 192 (223 and 215); 24 (2048, 6144), 4, 20 rows 162 and 156 (149 and 166), 30 rows 218 and 167 (219 and 196).
+  const int64_t fill = (int64_t)ex->experts * (((ex->gated ? 2 : 1) * ex->inter / W3_BLOCK_ROWS + 3) / 4), fill2 = (int64_t)ex->experts * ((ex->hidden_out / W3_BLOCK_ROWS + 3) / 4);
+  const int chunks2 = ex->inter / W3_CHUNK;
+  const int rows_min = fill >= 500 && ex->experts < 150 && fill2 < 5 * chunks2                   ? 24
+                       : fill >= 1500                                                            ? fill2 >= 30 * chunks2 ? 5 : ex->hidden >= 1536 ? 9 : 14
+                       : fill >= 500                                                             ? ex->experts >= 150 ? 7 : 16
+                       : ex->experts < named                                                     ? 48
+                                                                                                 : 26;
   const bool dense = !e4m3 && panel_takes(m, ex->hidden) && panel_takes(pairs + shared_rows, ex->inter) && panel_writes(out_pairs, !pairs_bf16) &&
                      (g_tune.w3_tile == 1 || (g_tune.w3_tile == 0 && pairs >= rows_min * named));
   const int tiles = panel_height<TileW3<3>>(pairs, named, ex->experts, shared_rows, (ex->gated ? 2 : 1) * ex->inter / W3_BLOCK_ROWS), slot_rows = dense ? 16 * tiles : ROWS_PER_SLOT;

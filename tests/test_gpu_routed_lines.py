@@ -25,6 +25,18 @@ def test_nvfp4(experts, hidden, inter, rows):
         assert torch.equal(ex(x, ids, w), by_panel if 4 * m >= rows * experts else by_stream)
 
 
+# 150 experts and more; fewer; fc2 of few workgroups a chunk of its K; fc1 of many workgroups
+@pytest.mark.parametrize("experts,hidden,inter,rows", [(180, 1664, 384, 7), (128, 512, 512, 16), (24, 512, 6144, 24), (96, 1024, 3072, 14), (64, 1536, 4096, 9)])
+def test_three_bit(experts, hidden, inter, rows):
+    from hibana_amd import synthetic
+    from hibana_amd.kernels import w3_moe
+    ex = w3_moe.tile(synthetic.w3_experts(experts, hidden, inter, True, 1), release=True)
+    for m in ((rows * experts - 1) // 4, (rows * experts + 3) // 4):
+        x, ids, w = _draw(m, experts, 4, hidden)
+        by_panel, by_stream = _by_kernel(b"w3_tile", lambda: w3_moe.w3_moe(ex, x, ids, w))
+        assert torch.equal(w3_moe.w3_moe(ex, x, ids, w), by_panel if 4 * m >= rows * experts else by_stream)
+
+
 # wider than long, all workgroups at once, and the long end that keeps its own launch: either way the same bits
 @pytest.mark.parametrize("experts,hidden,inter", [(64, 512, 4096), (24, 512, 4096), (32, 512, 6144)])
 @pytest.mark.parametrize("rows", [16, 40])

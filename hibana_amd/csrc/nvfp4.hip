@@ -799,16 +799,25 @@ static int launch_twin(StreamParams& a, int64_t slots_a, int64_t busy_a, StreamP
 // - 256 (768, 1536) 192 49.4 and 46.5; 512 (768, 1024) 256 51.4 and 47.1, 640 75.4 and 71.4; 512 (512, 2688) 176 61.7 and 58.2;
 // - eight chunks of K and more: 384 (1024, 2048) 16 38.5 and 37.8 (whole block), 64 48.0 and 43.5, 256 91.4 and 85.7; 512 (1024, 2688) 22 32.3 and 32.0, 88
 //   63.4 and 58.1, 352 152.4 and 147.7; 128 (1024, 1024) 320 43.3 and 38.9;
-// - too many: 384 (1024, 2048) 384 113.2 and 116.4; 512 (512, 2688) 880 131.3 and 136.5; 256 (768, 1536) 1440 86.8 and 90.6.
+// - too many: 384 (1024, 2048) 384 113.2 and 116.4; 512 (512, 2688) 880 131.3 and 136.5; 256 (768, 1536) 1440 86.8 and 90.6;
+// - more than two rows an expert, even and (skewed) routing: 128 (1024, 2048) 384 65.3 and 66.1 (60.7 and 64.4), 640 75.6 and 77.1 (70.8 and 74.8), but 128 (1024, 1024) 384
+//   42.7 and 38.2 (40.1 and 35.9), 64 (2048, 2048) 252 67.6 and 64.4 (66.4 and 66.8);
+// - a row an expert and K of fc1 below six chunks: 160 (512, 1536) 320 41.4 and 41.2 (38.7 and 42.4); 300 (640, 1280) 300 46.6 and 46.1 (42.4 and 44.6), 900 66.6 and
+//   66.4 (57.1 and 58.3); fewer pairs of few blocks: 512 (512, 1024) 256 40.0 and 38.9 (34.8 and 39.4), of many 512 (512, 2688) 176 61.1 and 57.5 (50.1 and 48.3);
+// - of six and seven chunks even routing, as this path's is, gains and skewed routing loses: 256 (768, 1536) 252 52.8 and 51.2 (47.4 and 50.1), 512 (768, 1024) 250 48.2
+//   and 43.7 (40.4 and 44.5);
+// - K of fc2 past 24 chunks, whose few long workgroups meet on one compute unit: 8 (2048, 5632) 16 28.5 and 34.2 (28.4 and 32.0), 32 31.6 and 37.1; 16 (1024, 8192) 8 25.8 and 28.3 (25.9 and
+//   29.0); 32 (2048, 4096) 64 60.9 and 57.5 (57.5 and 61.4), 96 62.7 and 58.5 (59.7 and 64.3).
 constexpr int DEVICE_WAVES = 4096;
-// `local`: the experts held here, of the `experts` that the pairs name.
-static bool fc12_serves(int64_t pairs, int local, int64_t experts, int n_blocks, int chunks) {
+// `local`: the experts held here, of the `experts` that the pairs name; p1, p2: the layers.
+static bool fc12_serves(int64_t pairs, int local, int64_t experts, const StreamParams& p1, const StreamParams& p2) {
   if (g_nvfp4_fused) return g_nvfp4_fused == 1;
-  const bool deep = chunks >= 8;
+  if (p2.chunks > 24) return false;
+  const bool deep = p1.chunks >= 8;
   const double distinct = local * (1.0 - std::exp(-(double)pairs / (double)experts));  // of a uniform routing
-  const double waves = distinct * n_blocks * (deep ? 2 : 1);
-  if (waves < (deep ? DEVICE_WAVES / 4 : DEVICE_WAVES * 3 / 4)) return false;
-  return pairs < experts || (waves <= 2 * DEVICE_WAVES && (deep || pairs <= 2 * experts));
+  const double waves = distinct * p1.n_blocks * (deep ? 2 : 1);
+  if (waves < (deep ? DEVICE_WAVES / 4 : p1.chunks >= 6 ? DEVICE_WAVES * 3 / 4 : DEVICE_WAVES)) return false;
+  return pairs < experts || (waves <= 2 * DEVICE_WAVES && pairs <= 2 * experts && p1.chunks >= 6) || (deep && waves <= DEVICE_WAVES);
 }
 
 // Both layers over a plan of `slots` entries (busy: the caller's estimate of those with rows), in one launch; `dense`: one slot of a dense matrix
@@ -1113,7 +1122,7 @@ int run_experts(const hb_nvfp4_experts* ex, const void* x, const int32_t* ids, i
     if (int e = launch_panel_routed<TileNvfp4, EPI_FC2>(f2, tiles, slots, pairs, stream)) return e;
     return launch_status();
   }
-  if (fc12_serves(pairs, ex->experts, named, p.n_blocks, p.chunks) && (ex->gated ? launch_fc12<EPI_FC1_GATED>(p, f2, slots, est, nullptr, stream) : launch_fc12<EPI_FC1_RELU2>(p, f2, slots, est, nullptr, stream)) == HB_OK)
+  if (fc12_serves(pairs, ex->experts, named, p, f2) && (ex->gated ? launch_fc12<EPI_FC1_GATED>(p, f2, slots, est, nullptr, stream) : launch_fc12<EPI_FC1_RELU2>(p, f2, slots, est, nullptr, stream)) == HB_OK)
     return launch_status();
   if (int e = ex->gated ? launch_nvfp4<EPI_FC1_GATED>(p, slots, est, stream) : launch_nvfp4<EPI_FC1_RELU2>(p, slots, est, stream)) return e;
   if (int e = launch_nvfp4<EPI_FC2>(f2, slots, est, stream)) return e;
@@ -1397,7 +1406,7 @@ extern "C" int hb_latent_layer(const hb_latent_weights* w, const void* x, int m,
   const bool planned = w->shared_up && latent_plan_of(r, q);  // up beside routing and plan, else beside fc1
   if (int e = planned ? launch_latent_plan(r, q, up, fc1, s) : latent_launch_route(r, s)) return e;
   StreamParams* dense = w->shared_up ? &down : nullptr;
-  const bool together = planned == (dense != nullptr) && fc12_serves(pairs, ex->experts, experts_named(w->experts_total, ex->base, ex->experts), fc1.n_blocks, fc1.chunks) &&
+  const bool together = planned == (dense != nullptr) && fc12_serves(pairs, ex->experts, experts_named(w->experts_total, ex->base, ex->experts), fc1, fc2) &&
                         (ex->gated ? launch_fc12<EPI_FC1_GATED>(fc1, fc2, slot_cap, est, dense, s) : launch_fc12<EPI_FC1_RELU2>(fc1, fc2, slot_cap, est, dense, s)) == HB_OK;
   if (!together) {
     if (dense && !planned) {

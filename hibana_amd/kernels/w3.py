@@ -372,8 +372,8 @@ def w3_mlp_takes(x: torch.Tensor, gate_up: W3Weight, down: W3Weight) -> bool:
 
 
 def w3_mlp(x: torch.Tensor, gate_up: W3Weight, down: W3Weight, pairs: int = 0) -> torch.Tensor:
-    """`w3_linear(*silu_mul_quant_groups(w3_linear(x, gate_up), pairs, torch_chain=True), down)` in one call; up to sixteen rows the SiLU
-    product and its E4M3 rounding are the first launch's epilogue (hibana/model/mlp.py:36-42)."""
+    """`w3_linear(*silu_mul_quant_groups(w3_linear(x, gate_up), pairs, torch_chain=True), down)` in one call, with its bits; up to
+    sixteen rows the SiLU product and its E4M3 rounding are the first launch's epilogue where that is the faster (hibana/model/mlp.py:36-42)."""
     if not w3_mlp_takes(x, gate_up, down):
         raise ValueError("w3_mlp: unsupported call")
     _lib.need_gpu(x)

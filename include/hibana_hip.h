@@ -205,7 +205,7 @@ int hb_w3_gemm_e4m3(const void* xq, const float* x_scale, int m, const void* til
 /* The dense SwiGLU block on its 3-bit copies: gate_up (`gate_up_bits` tiles [2 inter, hidden], rows [gate; up], or alternating in blocks of
  * `pairs` rows, pairs % 32 == 0) of x BF16 [m, hidden], what hb_silu_mul_quant_groups makes of its BF16 result (torch_chain), and
  * hb_w3_gemm_e4m3 of that with down (`down_bits` tiles [n, inter]) into y BF16 [m, n]. inter % 128 == 0, hidden % 128 == 0, n % 64 == 0.
- * Up to sixteen rows gate_up, product and rounding are one launch. scratch: HB_W3_MLP_SCRATCH_BYTES, of any contents.
+ * Up to sixteen rows gate_up, product and rounding are one launch, but for sizes where three are the faster: the same bits. scratch: HB_W3_MLP_SCRATCH_BYTES, of any contents.
  * ref: Mlp.__call__, hibana/model/mlp.py:26-48 (its 3-bit decode branch, :36-42). */
 #define HB_W3_MLP_SCRATCH_BYTES(m, inter) ((m) * (inter) / 8 * 41)
 int hb_w3_mlp(const void* x, int m, const void* gate_up, const float* gate_up_rows, int64_t gate_up_lut, int inter, int hidden, int gate_up_bits,

@@ -601,9 +601,9 @@ __global__ __launch_bounds__(1024) void nvfp4_fc12_kernel(StreamParams p1, Strea
 // FP32, its latent columns also rounded to BF16 (hibana/kernels/csrc/nemotron_moe.cu:496-558 of the reference).
 // The product is bound by how fast a compute unit brings its columns in, so a workgroup has eight of them only: the sixteen columns of a product's
 // weight operand are eight weight rows over two parts of K. PACKED (up to eight rows): the sixteen activation rows are likewise eight
-// over both parts, and of the result the two quarters where the parts agree are kept; else a product each. With the plan's launch below, the
-// block of 512 experts (1024, 2688) and a shared one of 5376, router and block as six launches and so, us: one row 53.2 and 49.0, four 80.0 and
-// 77.4, eight 110.9 and 108.5, nine 126.9 and 119.0, sixteen 165.4 and 162.7.
+// over both parts, and of the result the two quarters where the parts agree are kept; else a product each. With the launches below, the
+// block of 512 experts (1024, 2688) and a shared one of 5376, router and block in two calls of six launches and in one, us: one row 54.0 and 48.2, four 80.2
+// and 72.5, eight 113.7 and 104.8, nine 127.5 and 125.6, sixteen 166.6 and 164.8; this product alone 7.7 and 5.6 of eight rows, 9.2 and 7.8 of sixteen (traced).
 constexpr int FRONT_WAVES = 8, FRONT_COLUMNS = 8;
 struct FrontGemv {
   const uint16_t* w;  // BF16 [n, k]
@@ -1403,7 +1403,14 @@ extern "C" int hb_latent_layer(const hb_latent_weights* w, const void* x, int m,
   if (int e = shape_nvfp4(fc1, est)) return e;
   if (int e = launch_front(r, s)) return e;
   LatentPlan q;
-  const bool planned = w->shared_up && latent_plan_of(r, q);  // up beside routing and plan, else beside fc1
+  // Up beside routing and plan, else beside fc1, where more than eight rows take it longer than those two (its splits of K are fc1's launch's, of more than twelve
+  // chunks here): the block of 512 experts (1024, 2688) and a shared one of 5376, K split two ways, beside the plan (25.4 us) and so: nine rows 125 and 125, twelve
+  // 147 and 143, sixteen 172 and 165; eight rows, four ways, 104 and 110; 512 (512, 2688) and 2048, two ways, four rows 56.6 and 58.7, eight 75.1 and 76.0.
+  bool planned = w->shared_up != nullptr;
+  if (planned) {
+    if (int e = shape_beside(up, 1, fc1)) return e;
+    planned = (m <= FP4_FEW_ROWS || up.chunks <= 12 * up.ks) && latent_plan_of(r, q);
+  }
   if (int e = planned ? launch_latent_plan(r, q, up, fc1, s) : latent_launch_route(r, s)) return e;
   StreamParams* dense = w->shared_up ? &down : nullptr;
   const bool together = planned == (dense != nullptr) && fc12_serves(pairs, ex->experts, experts_named(w->experts_total, ex->base, ex->experts), fc1, fc2) &&

@@ -542,7 +542,7 @@ int hb_latent_router(const hb_latent_weights* w, const void* x, int m, int topk,
 /* hb_latent_router (routing and planning) and hb_latent_block in one call, for a caller that wants the block's output alone, with the bits of the
  * two. Five launches: the router's product; routing and plan, the shared expert's up projection beside them; both layers of the routed experts,
  * its down projection beside them; the combine; the projection back. Six where the two layers are a launch each (few pairs, many of few
- * experts, a workspace off 256-byte addresses).
+ * experts, a workspace off 256-byte addresses, an up projection of more than eight rows that is too long to stand beside the plan).
  * `workspace`: hb_latent_layer_workspace_bytes, under the rules of hb_latent_router's; NVFP4 routed experts only.
  * ref: the block of at most 16 rows, NemotronMoe.small, hibana/model/nemotron/moe.py:484-502. */
 size_t hb_latent_layer_workspace_bytes(const hb_latent_weights* w, int m, int topk);

@@ -790,15 +790,15 @@ inline int panel_routed(StreamParams& p, int tiles, int64_t slots, int64_t a_row
 }
 
 // Whether fc1 (`p1`) and fc2 (`p2`) of `experts` experts share a launch. One launch starts fc2's workgroups where fc1's leave room, several on one
-// compute unit, and where they are few and long (once over the device at most, K of twenty chunks and twice fc1's) and could not all stand
+// compute unit, and where they are few and long (once over the device at most, K of seventeen chunks and twice fc1's) and could not all stand
 // there from the start, their length is the call's end; a launch of their own spreads them out. Measured, two launches and one, the routed call,
 // even and (skewed) routing, us: NVFP4, 64 experts (1024, 8192), 8 rows an expert 148 and 160 (154 and 167), 28 rows 176 and 217 (220 and 246); 128 (1024, 4096) 8 rows 127
 // and 132 (135 and 138); 128 (896, 2688) 5 rows 86 and 91 (85 and 86); three-bit, 64 (2048, 6144) 16 rows 273 and 296 (278 and 280), 40 rows 368 and 383 (403 and 410); 24
-// (2048, 6144) 30 rows 167 and 184 (196 and 191); 32 (2048, 4096) 16 rows 112 and 118 (121 and 124), 40 rows 145 and 142 (170 and 165). On the other sides
-// of the line: 512 (1024, 2688) 8 rows 313 and 311 (308 and 304), 200 (896, 2048) 6 rows 101 and 96, 48 (768, 2816) 16 rows 58 and 55, three-bit 96 (2048, 2048) 7 rows 116 and 112.
+// (2048, 6144) 30 rows 167 and 184 (196 and 191); 32 (2048, 4096) 16 rows 112 and 118 (121 and 124), 40 rows 145 and 142 (170 and 165); NVFP4, 160 (640, 2304) 10 rows 78 and 81 (80 and 85), 60 rows 116 and 124 (146 and 134). On the other sides
+// of the line: 128 (768, 2048) 10 rows 67 and 63 (72 and 70), 512 (1024, 2688) 8 rows 313 and 311 (308 and 304), 200 (896, 2048) 6 rows 101 and 96, 48 (768, 2816) 16 rows 58 and 55, three-bit 96 (2048, 2048) 7 rows 116 and 112.
 inline bool panel_together(const StreamParams& p1, const StreamParams& p2, int64_t experts, int tiles) {
   const int64_t groups1 = (p1.n_blocks + 3) / 4, groups2 = (p2.n_blocks + 3) / 4;
-  const bool long_end = p2.chunks >= 20 && p2.chunks >= 2 * p1.chunks && experts * groups2 <= 1024;
+  const bool long_end = p2.chunks >= 17 && p2.chunks >= 2 * p1.chunks && experts * groups2 <= 1024;
   return !long_end || experts * (groups1 + groups2) <= (tiles <= 3 ? 1024 : 1280);
 }
 
